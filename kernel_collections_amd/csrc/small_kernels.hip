@@ -97,51 +97,57 @@ __global__ __launch_bounds__(256) void absorb_q_kernel(
   }
 }
 
-// Same product for head_dim 64 / 128 / 256 / 512 with coalesced reads: TPR = d / 8 consecutive lanes cover one row of B
-// (16 bytes each), 256 / TPR rows per pass; the per-row dot products are finished by a lane reduction.  A workgroup
-// takes ABS_ROWS rows of B and up to ABS_HEADS query heads of one kv head (their rows sit in LDS as fp32), so that
-// even a single sequence with one kv head spreads over tens of CUs.
-constexpr int ABS_ROWS = 16, ABS_HEADS = 8;
-template <typename T, int TPR>
-__global__ __launch_bounds__(256) void absorb_q_rows_kernel(
+// The same product for every head_dim that is a multiple of 32, on v_mfma_f32_16x16x32: both operands are rows whose 8
+// consecutive features are a lane's packet (A = 16 query heads, B = 16 rows of B), so they go from global memory straight into
+// the matrix pipe.  A wave owns 16 rows of B against all (up to 16 per workgroup) query heads of its kv head; with KSPLIT the
+// four waves of a workgroup share 16 rows and cut the features between them, so that a wave's loads are one round trip at
+// d 512 too.  The kernel is latency - a launch and a round trip - whatever the shape: by trace 3.5 us at 8 x 32 heads, d 128,
+// rank 512 (the LDS form it replaces: 4.4) and 4.6 us at 8 x 16 heads, d 512, rank 256 (15.5; 6.3 without KSPLIT).
+template <typename T, bool KSPLIT>
+__global__ __launch_bounds__(256) void absorb_q_mfma_kernel(
     const T* __restrict__ q, const T* __restrict__ B, T* __restrict__ qt_hi, T* __restrict__ qt_lo,
-    int hq, int hkv, int rank, int64_t sBb, int64_t sBh, int64_t sBr, int nhc) {
+    int hq, int hkv, int d, int rank, int64_t sBb, int64_t sBh, int64_t sBr) {
   typedef typename Elem<T>::vec8 vec8;
-  constexpr int D = TPR * 8, RPP = 256 / TPR;
-  __shared__ float qs[ABS_HEADS * D];
-  const int kh = blockIdx.x / nhc, g0 = (blockIdx.x % nhc) * ABS_HEADS, b = blockIdx.y, G = hq / hkv;
-  const int gn = G - g0 < ABS_HEADS ? G - g0 : ABS_HEADS;
-  const int sub = threadIdx.x % TPR, rr = threadIdx.x / TPR;
-  const T* Bh = B + b * sBb + kh * sBh;
-  const T* qb = q + ((int64_t)b * hq + (int64_t)kh * G + g0) * D;
-  for (int i = threadIdx.x; i < gn * D; i += 256) qs[i] = to_f32(qb[i]);
-  __syncthreads();
-  for (int r0 = 0; r0 < ABS_ROWS; r0 += RPP) {
-    const int rho = blockIdx.z * ABS_ROWS + r0 + rr;
-    const bool live = rho < rank && rr < ABS_ROWS;
-    float x[8];
-    {
-      vec8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (live) v = ld16<vec8>(Bh + (int64_t)rho * sBr + sub * 8);
+  constexpr int NK = KSPLIT ? 4 : 8;   // k-steps in flight
+  __shared__ f32x4 part[KSPLIT ? 3 : 1][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n16 = lane & 15, g4 = lane >> 4;
+  const int G = hq / hkv, nhb = (G + 15) / 16;
+  const int kh = blockIdx.x / nhb, g0 = (blockIdx.x % nhb) * 16, b = blockIdx.y;
+  const int rho = (KSPLIT ? blockIdx.z : blockIdx.z * 4 + wave) * 16 + n16;
+  const int gn = G - g0 < 16 ? G - g0 : 16;
+  // head rows past the group and rows past the rank repeat the last one: their products are never written
+  const T* qrow = q + ((int64_t)b * hq + (int64_t)kh * G + g0 + (n16 < gn ? n16 : gn - 1)) * d + 8 * g4;
+  const T* brow = B + b * sBb + kh * sBh + (int64_t)(rho < rank ? rho : rank - 1) * sBr + 8 * g4;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int c0 = KSPLIT ? 32 * NK * wave : 0; c0 < d; c0 += 32 * NK * (KSPLIT ? 4 : 1)) {
+    vec8 a[NK], w[NK];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = to_f32(v[e]);
-    }
-    for (int g = 0; g < gn; ++g) {
-      const f32x4 qa = *reinterpret_cast<const f32x4*>(qs + g * D + sub * 8);
-      const f32x4 qb4 = *reinterpret_cast<const f32x4*>(qs + g * D + sub * 8 + 4);
-      float a = x[0] * qa[0] + x[1] * qa[1] + x[2] * qa[2] + x[3] * qa[3] + x[4] * qb4[0] + x[5] * qb4[1] +
-                x[6] * qb4[2] + x[7] * qb4[3];
-      a = row_reduce<false, (TPR < 16 ? TPR : 16)>(a);
-      if (TPR >= 32) a += __shfl_xor(a, 16);
-      if (TPR >= 64) a += __shfl_xor(a, 32);
-      if (live && sub == (g % TPR)) {
-        const int64_t o = ((int64_t)b * hq + (int64_t)kh * G + g0 + g) * rank + rho;
-        const T hi = from_f32<T>(a);
-        qt_hi[o] = hi;
-        if (qt_lo) qt_lo[o] = from_f32<T>(a - to_f32(hi));
+    for (int k = 0; k < NK; ++k) {
+      a[k] = w[k] = vec8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (c0 + 32 * k < d) {
+        a[k] = ld16<vec8>(qrow + c0 + 32 * k);
+        w[k] = ld16<vec8>(brow + c0 + 32 * k);
       }
     }
+#pragma unroll
+    for (int k = 0; k < NK; ++k) acc = Elem<T>::mfma16(a[k], w[k], acc);
   }
+  if constexpr (KSPLIT) {
+    if (wave) part[wave - 1][lane] = acc;
+    __syncthreads();
+    if (wave) return;
+    acc += part[0][lane] + part[1][lane] + part[2][lane];
+  }
+  if (rho >= rank) return;
+  // lane (n16 = row of B, g4): heads g0 + 4 g4 + r
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (4 * g4 + r < gn) {
+      const int64_t o = ((int64_t)b * hq + (int64_t)kh * G + g0 + 4 * g4 + r) * rank + rho;
+      const T hi = from_f32<T>(acc[r]);
+      qt_hi[o] = hi;
+      if (qt_lo) qt_lo[o] = from_f32<T>(acc[r] - to_f32(hi));
+    }
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -589,21 +595,17 @@ extern "C" int xkv_absorb_q(const void* q, const void* B, void* qt_hi, void* qt_
   hipStream_t st = (hipStream_t)stream;
   if (dtype != XKV_BF16 && dtype != XKV_F16) return XKV_EDTYPE;
   const dim3 block(256);
-  const int nhc = (hq / hkv + ABS_HEADS - 1) / ABS_HEADS;   // head chunks per kv head
-#define XKV_ABSORB(T)                                                                                                         \
-  if (d == 128)                                                                                                               \
-    absorb_q_rows_kernel<T, 16><<<dim3(hkv * nhc, batch, (rank + ABS_ROWS - 1) / ABS_ROWS), block, 0, st>>>((const T*)q, (const T*)B, (T*)qt_hi,    \
-                                                                                        (T*)qt_lo, hq, hkv, rank, sBb, sBh, sBr, nhc); \
-  else if (d == 512)                                                                                                          \
-    absorb_q_rows_kernel<T, 64><<<dim3(hkv * nhc, batch, (rank + ABS_ROWS - 1) / ABS_ROWS), block, 0, st>>>((const T*)q, (const T*)B, (T*)qt_hi,    \
-                                                                                        (T*)qt_lo, hq, hkv, rank, sBb, sBh, sBr, nhc); \
-  else if (d == 256)                                                                                                          \
-    absorb_q_rows_kernel<T, 32><<<dim3(hkv * nhc, batch, (rank + ABS_ROWS - 1) / ABS_ROWS), block, 0, st>>>((const T*)q, (const T*)B, (T*)qt_hi,    \
-                                                                                        (T*)qt_lo, hq, hkv, rank, sBb, sBh, sBr, nhc); \
-  else if (d == 64)                                                                                                           \
-    absorb_q_rows_kernel<T, 8><<<dim3(hkv * nhc, batch, (rank + ABS_ROWS - 1) / ABS_ROWS), block, 0, st>>>((const T*)q, (const T*)B, (T*)qt_hi,     \
-                                                                                       (T*)qt_lo, hq, hkv, rank, sBb, sBh, sBr, nhc); \
-  else                                                                                                                        \
+  const int nhb = (hq / hkv + 15) / 16;   // blocks of 16 query heads per kv head
+  // the MFMA form reads 16-byte packets of q: a query buffer that is not aligned takes the scalar form, as does a head_dim
+  // that is not a whole number of 32-feature k-steps; beyond eight k-steps (d 256) the waves of a workgroup share them
+#define XKV_ABSORB(T)                                                                                                          \
+  if (d % 32 == 0 && ((uintptr_t)q & 15) == 0 && d > 256)                                                                      \
+    absorb_q_mfma_kernel<T, true><<<dim3(hkv * nhb, batch, (rank + 15) / 16), block, 0, st>>>((const T*)q, (const T*)B, (T*)qt_hi, \
+                                                                                 (T*)qt_lo, hq, hkv, d, rank, sBb, sBh, sBr);  \
+  else if (d % 32 == 0 && ((uintptr_t)q & 15) == 0)                                                                            \
+    absorb_q_mfma_kernel<T, false><<<dim3(hkv * nhb, batch, (rank + 63) / 64), block, 0, st>>>((const T*)q, (const T*)B, (T*)qt_hi, \
+                                                                                 (T*)qt_lo, hq, hkv, d, rank, sBb, sBh, sBr);  \
+  else                                                                                                                         \
     absorb_q_kernel<T><<<dim3(hkv, batch, (rank + 255) / 256), block, 0, st>>>((const T*)q, (const T*)B, (T*)qt_hi, (T*)qt_lo, \
                                                                                  hq, hkv, d, rank, sBb, sBh, sBr);
   if (dtype == XKV_BF16) { XKV_ABSORB(__bf16) } else { XKV_ABSORB(_Float16) }
