@@ -1,4 +1,6 @@
 // RoPE table, query absorption and the stage-2 merge: the small kernels around the scans.
+#include <type_traits>
+
 #include "xkv_common.h"
 
 namespace xkv {
@@ -172,205 +174,201 @@ __global__ __launch_bounds__(256) void blockdiag_q_kernel(const T* __restrict__ 
 }
 
 // ----------------------------------------------------------------------------------------------
-// Stage 2.  One workgroup per (kv head, batch), or per (query head, batch) when there are many splits: merges the live splits of its query heads
-// (reference order: increasing split id, running max of lse), then optionally multiplies the
-// merged rank-space rows by vB[b, kh] (read once for the G heads).
+// Stage 2: weights w_i = exp(lse_i - max lse) / sum over the live splits (a prefix of the split range: split i is live iff
+// per * i < L), weighted sum of the partial rows, optionally the up-projection by vB[b, kh].  Both kernels are chains of
+// dependent round trips, so each starts everything it can at once: the lse words and the partial rows of a thread's splits
+// are loaded together and folded with a running maximum, instead of weights first and rows after.
 // ----------------------------------------------------------------------------------------------
-constexpr int MERGE_RED_FLOATS = 32 * 4 * 64, MERGE_FIN_FLOATS = 4 * 512;   // the kernel's static LDS (the launcher counts it)
-template <typename O, typename TB>
-__global__ __launch_bounds__(256) void merge_stage2_kernel(
+__device__ __forceinline__ int merge_live_splits(int L, int ns, int max_splits) {
+  const int per = ns > 0 ? cdiv(cdiv(L, ns), MIN_BLOCK_KV) * MIN_BLOCK_KV : 0;
+  const int live = per > 0 ? cdiv(L, per) : 0;
+  return live < max_splits ? live : max_splits;
+}
+
+// A thread's share of one head's splits: i = first, first + step, ... < nlive, P consecutive features at pp.  Eight splits'
+// loads in flight; acc = sum exp(lse_i - m) * partial_i, l = sum exp(lse_i - m), m the running maximum (NEG_INF: no split).
+template <int P> struct MergeAcc { float m, l, acc[P]; };
+template <int P>
+__device__ __forceinline__ MergeAcc<P> merge_fold(const float* __restrict__ pl, const float* __restrict__ pp, int dv, int first,
+                                                  int step, int nlive) {
+  MergeAcc<P> r;
+  r.m = NEG_INF; r.l = 0.f;
+#pragma unroll
+  for (int e = 0; e < P; ++e) r.acc[e] = 0.f;
+  constexpr int NB = 8;
+  for (int i0 = first; i0 < nlive; i0 += NB * step) {
+    float w[NB], v[NB][P];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const int i = i0 + k * step;
+      w[k] = NEG_INF;
+#pragma unroll
+      for (int e = 0; e < P; ++e) v[k][e] = 0.f;
+      if (i < nlive) {
+        w[k] = pl[i];
+        const float* src = pp + (int64_t)i * dv;
+        if constexpr (P == 4) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(src);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[k][e] = x[e];
+        } else {
+          v[k][0] = src[0];
+        }
+      }
+    }
+    float mn = r.m;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) mn = fmaxf(mn, w[k]);
+    const float sc = r.m == NEG_INF ? 0.f : __expf(r.m - mn);
+    r.m = mn;
+    r.l *= sc;
+#pragma unroll
+    for (int e = 0; e < P; ++e) r.acc[e] *= sc;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const float x = w[k] == NEG_INF ? 0.f : __expf(w[k] - mn);
+      r.l += x;
+#pragma unroll
+      for (int e = 0; e < P; ++e) r.acc[e] += x * v[k][e];
+    }
+  }
+  return r;
+}
+
+// Without an up-projection: one workgroup per (head, block of `chunk` features), chunk / P lanes per group of threads; the
+// groups take the splits round-robin and meet in the LDS.  Short chunks when there are many splits, so that a single long
+// sequence is read by the whole chip: batch 1, 32 heads, 256 splits of 512 features (16.8 MB) in 6.0 us by trace, 64 x 16 heads
+// with 4 splits of 512 in 4.5 (with the weights of all splits first and the rows after them: 8.6).
+template <typename O, int P>
+__global__ __launch_bounds__(256) void merge_rows_kernel(
+    const float* __restrict__ partial, const float* __restrict__ lse, O* __restrict__ out,
+    const int32_t* __restrict__ num_kv_splits, const int32_t* __restrict__ kv_lens, int hq, int kv_len, int max_splits, int dv,
+    int chunk, int64_t sOb, int64_t sOh, float* __restrict__ lse_out, int64_t sLb, int64_t sLh, int split_cap,
+    const int32_t* __restrict__ split_plan) {
+  __shared__ float red[256 * P], ml[256][2];
+  const int h = blockIdx.x, b = blockIdx.y, c0 = blockIdx.z * chunk;
+  const int L = kv_lens ? kv_lens[b] : kv_len;
+  const int nlive = merge_live_splits(L, effective_splits(L, num_kv_splits[b], split_cap_in_force(split_cap, split_plan)), max_splits);
+  const int lanes = chunk / P, ngrp = 256 / lanes;          // lanes <= 256
+  const int sg = threadIdx.x / lanes, c = c0 + (threadIdx.x % lanes) * P;
+  const bool mine = sg < ngrp && c < dv;
+  const int64_t row = ((int64_t)b * hq + h) * max_splits;
+  MergeAcc<P> a;
+  if (mine) {
+    a = merge_fold<P>(lse + row, partial + row * dv + c, dv, sg, ngrp, nlive);
+#pragma unroll
+    for (int e = 0; e < P; ++e) red[threadIdx.x * P + e] = a.acc[e];
+    ml[threadIdx.x][0] = a.m;
+    ml[threadIdx.x][1] = a.l;
+  }
+  __syncthreads();
+  if (!mine || sg) return;
+  float M = a.m;
+  for (int g = 1; g < ngrp; ++g) M = fmaxf(M, ml[g * lanes + threadIdx.x][0]);
+  float l = 0.f, acc[P];
+#pragma unroll
+  for (int e = 0; e < P; ++e) acc[e] = 0.f;
+  for (int g = 0; g < ngrp; ++g) {
+    const int t = g * lanes + threadIdx.x;
+    const float w = ml[t][0] == NEG_INF ? 0.f : __expf(ml[t][0] - M);
+    l += w * ml[t][1];
+#pragma unroll
+    for (int e = 0; e < P; ++e) acc[e] += w * red[t * P + e];
+  }
+  const float inv = nlive > 0 ? 1.f / l : 0.f;
+  O* o = out + b * sOb + h * sOh + c;
+#pragma unroll
+  for (int e = 0; e < P; ++e) o[e] = (O)(acc[e] * inv);
+  if (lse_out && c == 0) lse_out[b * sLb + h * sLh] = M + __logf(l);   // log-sum-exp of the merged range
+}
+
+// With an up-projection: one workgroup per (hpw heads of one kv head, block of 64 output columns).  Thread (cb, grp): 8 columns
+// x the vB rows grp, grp + 64, ...; its vB packets are on the way before the split counts are known.  The heads' merged rows
+// meet in the LDS (every column block repeats that merge: a caller with many splits merges the rows first), then 8 FMAs per packet and head, and the 64 row groups are added by halving exchanges inside a 16-lane row (each step
+// a lane keeps half of its sums and hands the other half over) and four LDS words per total.  By trace, batch 1: one row per
+// head, dv 512, 6.4 us for 32 heads on 8 or 1 kv heads (rows + up-projection at 256 splits: 12.5 us, one kernel that did both
+// 20 - 21.7); 8 splits of 256, 4.7 us (7.0); 16 x 32 heads, 2 splits of 512, 8.6 us (11.6).
+constexpr int MERGE_CB = 64;       // columns per workgroup: whole 128-byte lines of a vB row
+constexpr int MERGE_UP_T = 512;
+template <typename O, typename TB, int RPT>
+__global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     const float* __restrict__ partial, const float* __restrict__ lse, O* __restrict__ out,
     const TB* __restrict__ vB, int64_t sVb, int64_t sVh, int64_t sVr, int d_out,
     const int32_t* __restrict__ num_kv_splits, const int32_t* __restrict__ kv_lens,
     int hq, int hkv, int kv_len, int max_splits, int dv, int64_t sOb, int64_t sOh, int hpw,
-    float* __restrict__ lse_out, int64_t sLb, int64_t sLh, int d_blk, int split_cap, const int32_t* __restrict__ split_plan) {
-  extern __shared__ float merged[];  // [G][dv], then the split weights [G][max_splits]
-  __shared__ float fin[MERGE_FIN_FLOATS];     // per-head-block totals of the up-projection
-  // this workgroup: heads hfirst .. hfirst + G - 1 of sequence b, all of kv head kh (G = hpw divides the GQA group size)
-  const int G = hpw, hfirst = blockIdx.x * hpw, kh = hfirst / (hq / hkv), b = blockIdx.y;
-  // blockIdx.z: a block of d_blk output columns of the up-projection (every block repeats the merge: when the grid is
-  // small the partial rows are read from more CUs at once, which is what bounds a single long sequence)
-  if (blockIdx.z > 0) {
-    const int cz = blockIdx.z * d_blk;
-    vB += cz;
-    out += cz;
-    d_out = d_out - cz < d_blk ? d_out - cz : d_blk;
-    lse_out = nullptr;
-  } else if (d_blk < d_out) {
-    d_out = d_blk;
+    float* __restrict__ lse_out, int64_t sLb, int64_t sLh, int split_cap, const int32_t* __restrict__ split_plan) {
+  typedef typename Elem<TB>::vec8 vec8;
+  extern __shared__ float merged[];               // [hpw][dv]
+  __shared__ float tot[4][4 * MERGE_CB];          // [quarter of the row groups][4 heads x 64 columns]
+  const int hfirst = blockIdx.x * hpw, kh = hfirst / (hq / hkv), b = blockIdx.y, c0 = blockIdx.z * MERGE_CB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // the 16 lanes of a row hold 16 row groups of one 8-column block; a wave covers four blocks, a pair of waves all eight
+  const int cb = (wave & 1) * 4 + (lane >> 4), grp = (wave >> 1) * 16 + (lane & 15);
+  const bool cols = c0 + cb * 8 < d_out;          // d_out is a multiple of 8
+  const TB* Bh = vB + b * sVb + kh * sVh + c0 + cb * 8;
+  vec8 w[RPT];
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    w[r] = vec8{0, 0, 0, 0, 0, 0, 0, 0};
+    if (cols && grp + 64 * r < dv) w[r] = ld16<vec8>(Bh + (int64_t)(grp + 64 * r) * sVr);
   }
   const int L = kv_lens ? kv_lens[b] : kv_len;
-  const int ns = effective_splits(L, num_kv_splits[b], split_cap_in_force(split_cap, split_plan));
-  float* wts = merged + G * dv;
-  int nlive = 0;
-  {
-    const int per = ns > 0 ? cdiv(cdiv(L, ns), MIN_BLOCK_KV) * MIN_BLOCK_KV : 0;
-    nlive = per > 0 ? cdiv(L, per) : 0;
-    nlive = nlive < max_splits ? nlive : max_splits;
-  }
-  // weights of the live splits, w_i = exp(lse_i - max lse) / sum: one wave per head, lanes stride over the splits
-  {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int gi = wave; gi < G; gi += 4) {
-      const float* pl = lse + ((int64_t)b * hq + hfirst + gi) * max_splits;
-      float mx = NEG_INF;
-      for (int i = lane; i < max_splits; i += 64) {
-        int s0, e0;
-        split_bounds(L, ns, i, s0, e0);
-        const float v = e0 > s0 ? pl[i] : NEG_INF;   // dead splits were never written
-        wts[gi * max_splits + i] = v;
-        mx = fmaxf(mx, v);
-      }
+  const int nlive = merge_live_splits(L, effective_splits(L, num_kv_splits[b], split_cap_in_force(split_cap, split_plan)), max_splits);
+  auto merge_packet = [&](int gi, int c, auto tag) {
+    constexpr int P = decltype(tag)::value;
+    const int64_t row = ((int64_t)b * hq + hfirst + gi) * max_splits;
+    const MergeAcc<P> a = merge_fold<P>(lse + row, partial + row * dv + c, dv, 0, 1, nlive);
+    const float inv = nlive > 0 ? 1.f / a.l : 0.f;
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-      float sum = 0.f;
-      for (int i = lane; i < max_splits; i += 64) {
-        const float v = wts[gi * max_splits + i];
-        const float w = v == NEG_INF ? 0.f : __expf(v - mx);
-        wts[gi * max_splits + i] = w;
-        sum += w;
-      }
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o);
-      const float inv = 1.f / sum;
-      for (int i = lane; i < max_splits; i += 64) wts[gi * max_splits + i] *= inv;
-      if (lse_out && lane == 0) lse_out[b * sLb + (hfirst + gi) * sLh] = mx + __logf(sum);   // log-sum-exp of the merged range
-    }
-  }
-  __syncthreads();
-  // weighted sum of the live splits (a prefix of the split range: split i is live iff per * i < L), 16 bytes per load.
-  // Work item = 4 consecutive features of one head; when there are fewer items than threads the threads form split
-  // groups (split i goes to group i % nsg) whose sums meet in LDS, so that a single long sequence still has 256 loads
-  // in flight per workgroup.
+    for (int e = 0; e < P; ++e) merged[gi * dv + c + e] = a.acc[e] * inv;
+    if (lse_out && c == 0 && blockIdx.z == 0) lse_out[b * sLb + (hfirst + gi) * sLh] = a.m + __logf(a.l);
+  };
   if ((dv & 3) == 0 && (reinterpret_cast<uintptr_t>(partial) & 15) == 0) {
-    const int items = G * dv / 4;
-    const int lanes_per = items < 256 ? items : 256;
-    const int nsg = 256 / lanes_per, sg = threadIdx.x / lanes_per;
-    for (int item = threadIdx.x % lanes_per; item < items && sg < nsg; item += lanes_per) {
-      const int gi = (item * 4) / dv, c = item * 4 - gi * dv;
-      const int h = hfirst + gi;
-      const float* pp = partial + ((int64_t)b * hq + h) * max_splits * (int64_t)dv + c;
-      const float* w = wts + gi * max_splits;
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-      for (int i = sg; i < nlive; i += nsg) acc += w[i] * *reinterpret_cast<const f32x4*>(pp + (int64_t)i * dv);
-      if (nsg == 1) {
-        if (vB) {
-          *reinterpret_cast<f32x4*>(merged + item * 4) = acc;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) out[b * sOb + h * sOh + c + e] = (O)acc[e];
-        }
-      } else {
-        *reinterpret_cast<f32x4*>(fin + (sg * items + item) * 4) = acc;   // nsg * items * 4 <= 1024 floats
-      }
-    }
-    if (nsg > 1) {
-      __syncthreads();
-      for (int idx = threadIdx.x; idx < G * dv; idx += blockDim.x) {
-        const int gi = idx / dv, c = idx - gi * dv;
-        float acc = 0.f;
-        for (int k = 0; k < nsg; ++k) acc += fin[k * items * 4 + idx];
-        if (vB)
-          merged[idx] = acc;
-        else
-          out[b * sOb + (hfirst + gi) * sOh + c] = (O)acc;
-      }
-      __syncthreads();   // fin is reused by the up-projection
-    }
+    const int ppr = dv >> 2;
+    for (int i = tid; i < hpw * ppr; i += MERGE_UP_T) merge_packet(i / ppr, (i % ppr) * 4, std::integral_constant<int, 4>());
   } else {
-    for (int idx = threadIdx.x; idx < G * dv; idx += blockDim.x) {
-      const int gi = idx / dv, c = idx - gi * dv;
-      const int h = hfirst + gi;
-      const float* pp = partial + ((int64_t)b * hq + h) * max_splits * (int64_t)dv + c;
-      const float* w = wts + gi * max_splits;
-      float acc = 0.f;
-#pragma unroll 8
-      for (int i = 0; i < nlive; ++i) acc += w[i] * pp[(int64_t)i * dv];
-      if (vB)
-        merged[idx] = acc;
-      else
-        out[b * sOb + h * sOh + c] = (O)acc;
-    }
+    for (int i = tid; i < hpw * dv; i += MERGE_UP_T) merge_packet(i / dv, i % dv, std::integral_constant<int, 1>());
   }
-  if (!vB) return;
   __syncthreads();
-  // out[g][c] = sum_rho merged[g][rho] * vB[rho][c].  Thread -> (8 output columns, one of 256/ncb rank groups): 16-byte
-  // loads of vB, several in flight, then a reduction over the rank groups through LDS.
-  typedef typename Elem<TB>::vec8 vec8;
-  const TB* Bh = vB + b * sVb + kh * sVh;
-  __shared__ float red[MERGE_RED_FLOATS];            // [rank group][4 heads][columns of the block]: 32 KiB
-  const int ncb = (d_out + 7) >> 3;                  // 8-column blocks (d_out <= 512 -> <= 64)
-  const int ngrp = 256 / ncb;                        // rank groups
-  const int cb = threadIdx.x % ncb, grp = threadIdx.x / ncb;
-  const bool active = grp < ngrp && cb * 8 + 8 <= d_out;
-  for (int g0 = 0; g0 < G; g0 += 4) {
-    float acc[4][8];
+  for (int g0 = 0; g0 < hpw; g0 += 4) {
+    float acc[32];                                // [4 heads][8 columns]
 #pragma unroll
-    for (int gi = 0; gi < 4; ++gi)
+    for (int i = 0; i < 32; ++i) acc[i] = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[gi][e] = 0.f;
-    if (active) {
-#pragma unroll 4
-      for (int rho = grp; rho < dv; rho += ngrp) {
-        const vec8 w = ld16<vec8>(Bh + rho * sVr + cb * 8);
+    for (int r = 0; r < RPT; ++r) {
+      const int rho = grp + 64 * r;
 #pragma unroll
-        for (int gi = 0; gi < 4; ++gi) {
-          const float m = g0 + gi < G ? merged[(g0 + gi) * dv + rho] : 0.f;
+      for (int gi = 0; gi < 4; ++gi) {
+        const float m = g0 + gi < hpw && rho < dv ? merged[(g0 + gi) * dv + rho] : 0.f;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) acc[gi][e] += m * to_f32(w[e]);
-        }
+        for (int e = 0; e < 8; ++e) acc[gi * 8 + e] += m * to_f32(w[r][e]);
       }
     }
-    // reduce over the rank groups through LDS, `chunk` groups per pass (as many as fit `red`)
-    const int cols = ncb * 8;                        // <= 512
-    const int gstride = 4 * cols;                    // a rank group's 4 x cols floats
-    const int chunk = MERGE_RED_FLOATS / gstride;    // groups per pass (>= 4): what fits `red`
-    for (int base = 0; base < ngrp; base += chunk) {
-      __syncthreads();
-      if (active && grp >= base && grp < base + chunk) {
-#pragma unroll
-        for (int gi = 0; gi < 4; ++gi)
-#pragma unroll
-          for (int e = 0; e < 8; ++e) red[(grp - base) * gstride + gi * cols + cb * 8 + e] = acc[gi][e];
-      }
-      __syncthreads();
-      const int n_here = (ngrp - base) < chunk ? (ngrp - base) : chunk;
-      const int nout = 4 * d_out;
-      if (nout <= 128 && ngrp <= chunk) {
-        // a narrow column block: fewer totals than threads and many rank groups (one pass).  256 / nout threads share a total's
-        // groups, so that nobody walks 64 LDS words one after the other; their sums meet in `fin`.
-        const int parts = 256 / nout, o = threadIdx.x % nout, part = threadIdx.x / nout;
-        const int gi = o / d_out, c = o - gi * d_out;
-        float sacc = 0.f;
-        if (part < parts) {
-#pragma unroll 8
-          for (int k = part; k < n_here; k += parts) sacc += red[k * gstride + gi * cols + c];
-          fin[part * nout + o] = sacc;
-        }
-        __syncthreads();
-        if (threadIdx.x < nout) {
-          float tot = fin[threadIdx.x];
-          for (int q = 1; q < parts; ++q) tot += fin[q * nout + threadIdx.x];
-          fin[threadIdx.x] = tot;
-        }
-      } else {
-        for (int idx = threadIdx.x; idx < nout; idx += blockDim.x) {
-          const int gi = idx / d_out, c = idx - gi * d_out;
-          if (g0 + gi < G) {
-            float sacc = 0.f;
-#pragma unroll 8
-            for (int k = 0; k < n_here; ++k) sacc += red[k * gstride + gi * cols + c];
-            fin[idx] = (base == 0 ? 0.f : fin[idx]) + sacc;
-          }
-        }
-      }
+    // halving exchanges over the 16 lanes that share a column block: partner 15 - l, then 7 - l, 3 - l, 1 - l of the shrinking
+    // group; the lane with the bit set keeps the upper half
+#define XKV_HALVE(N, BIT, CTRL)                                                                                               \
+    {                                                                                                                         \
+      const bool up = lane & BIT;                                                                                             \
+      _Pragma("unroll") for (int i = 0; i < N; ++i) {                                                                         \
+        const float give = up ? acc[i] : acc[N + i], keep = up ? acc[N + i] : acc[i];                                         \
+        acc[i] = keep + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give), CTRL, 0xf, 0xf, false)); \
+      }                                                                                                                       \
     }
+    XKV_HALVE(16, 8, 0x140)   // row_mirror
+    XKV_HALVE(8, 4, 0x141)    // row_half_mirror
+    XKV_HALVE(4, 2, 0x1B)     // quad_perm [3,2,1,0]
+    XKV_HALVE(2, 1, 0xB1)     // quad_perm [1,0,3,2]
+#undef XKV_HALVE
+    const int idx = (lane & 8 ? 16 : 0) + (lane & 4 ? 8 : 0) + (lane & 2 ? 4 : 0) + (lane & 1 ? 2 : 0);   // this lane's two sums
+#pragma unroll
+    for (int i = 0; i < 2; ++i) tot[wave >> 1][((idx + i) >> 3) * MERGE_CB + cb * 8 + ((idx + i) & 7)] = acc[i];
     __syncthreads();
-    for (int idx = threadIdx.x; idx < 4 * d_out; idx += blockDim.x) {
-      const int gi = idx / d_out, c = idx - gi * d_out;
-      if (g0 + gi < G) out[b * sOb + (hfirst + g0 + gi) * sOh + c] = (O)fin[idx];
+    if (tid < 4 * MERGE_CB) {
+      const int gi = tid / MERGE_CB, c = c0 + tid % MERGE_CB;
+      if (g0 + gi < hpw && c < d_out)
+        out[b * sOb + (hfirst + g0 + gi) * sOh + c] = (O)(tot[0][tid] + tot[1][tid] + tot[2][tid] + tot[3][tid]);
     }
+    __syncthreads();            // tot is reused by the next four heads
   }
 }
 
@@ -388,32 +386,36 @@ static int launch_merge(const float* partial, const float* lse, void* out, const
                         int64_t sVr, int d_out, const int32_t* ns, const int32_t* kl, int batch, int hq, int hkv,
                         int kv_len, int max_splits, int dv, int64_t sOb, int64_t sOh, float* lse_out, int64_t sLb, int64_t sLh,
                         int split_cap, const int32_t* split_plan, hipStream_t st) {
-  // few splits: one workgroup per kv head (vB read once for its heads); many splits: one per query head, so that the
-  // partial rows of a long sequence are spread over more CUs - unless the kv heads alone fill half the device and there
-  // is an up-projection, whose vB rows then weigh more than the partial rows
+  // what one head takes of the LDS was bounded when the weights of all its splits were held there; the bound stays part of the
+  // interface (a split count this large is refused before any launch)
+  if ((size_t)(dv + max_splits) * sizeof(float) > 24 * 1024) return XKV_EUNSUPPORTED;
+  if (!vB) {
+    // few splits: a head's whole row per workgroup; more: narrower feature blocks, so that a thread folds few splits
+    const bool vec = dv % 4 == 0 && (reinterpret_cast<uintptr_t>(partial) & 15) == 0;
+    int chunk = vec ? 1024 : 256;
+    while (chunk / 2 >= dv || (chunk > 64 && (int64_t)max_splits * chunk > (vec ? 8192 : 2048))) chunk /= 2;
+    const dim3 grid(hq, batch, cdiv(dv, chunk));
+    if (vec)
+      merge_rows_kernel<O, 4><<<grid, dim3(256), 0, st>>>(partial, lse, (O*)out, ns, kl, hq, kv_len, max_splits, dv, chunk, sOb, sOh,
+                                                          lse_out, sLb, sLh, split_cap, split_plan);
+    else
+      merge_rows_kernel<O, 1><<<grid, dim3(256), 0, st>>>(partial, lse, (O*)out, ns, kl, hq, kv_len, max_splits, dv, chunk, sOb, sOh,
+                                                          lse_out, sLb, sLh, split_cap, split_plan);
+    return launch_status();
+  }
+  // one workgroup for all heads of a kv head (vB is read once for them) as far as their merged rows fit 48 KiB of LDS
   const int g = hq / hkv;
-  const bool enough_wgs = vB && (int64_t)hkv * batch >= 128;   // vB costs more than the partial rows: keep it read once per kv head
-  int hpw = (g > 16 || (max_splits > 16 && !enough_wgs)) ? 1 : g;
-  if (!vB) hpw = 1;   // nothing is shared by the heads of a kv head without an up-projection: one workgroup per head
-  // dynamic LDS beside the kernel's static LDS (the up-projection's reduction buffers): the default limit of 64 KiB per
-  // workgroup must hold both; a group of heads that does not fit is merged one head per workgroup, and a single head that
-  // does not fit is refused
-  constexpr size_t LDS_LIMIT = 64 * 1024, STATIC_LDS = (MERGE_RED_FLOATS + MERGE_FIN_FLOATS) * sizeof(float);
-  auto dyn_lds = [&](int heads) { return (size_t)heads * (dv + max_splits) * sizeof(float); };
-  while (hpw > 1 && (g % hpw != 0 || dyn_lds(hpw) + STATIC_LDS > LDS_LIMIT)) --hpw;   // the largest group of heads that fits
-  const size_t shm = dyn_lds(hpw);
-  if (shm + STATIC_LDS > LDS_LIMIT) return XKV_EUNSUPPORTED;
-  // a small grid over many splits is bound by the latency of its partial-row loads: split the up-projection's columns
-  // over more workgroups
-  int zb = 1;
-  if (vB && (hq / hpw) * batch < 128 && max_splits >= 64 && d_out % 32 == 0) zb = d_out >= 512 ? 4 : d_out >= 256 ? 2 : 1;
-  // few splits: the merge itself is cheap to repeat, and what is left is the latency of the vB rows a thread reads one after
-  // the other - column blocks of >= 32 until the grid has 512 workgroups (a thread then reads dv / 64 rows instead of dv / 16)
-  if (vB && max_splits <= 16)
-    while ((int64_t)(hq / hpw) * batch * zb < 512 && d_out % (zb * 2 * 8) == 0 && d_out / (zb * 2) >= 32) zb *= 2;
-  merge_stage2_kernel<O, TB><<<dim3(hq / hpw, batch, zb), dim3(256), shm, st>>>(partial, lse, (O*)out, (const TB*)vB, sVb, sVh,
-                                                                               sVr, d_out, ns, kl, hq, hkv, kv_len, max_splits,
-                                                                               dv, sOb, sOh, hpw, lse_out, sLb, sLh, d_out / zb, split_cap, split_plan);
+  int hpw = g;
+  while (hpw > 1 && (g % hpw != 0 || (size_t)hpw * dv * sizeof(float) > 48 * 1024)) --hpw;
+  while (hpw > 4 && hpw % 2 == 0 && (int64_t)(hq / hpw) * batch * cdiv(d_out, MERGE_CB) < 256) hpw /= 2;
+  const dim3 grid(hq / hpw, batch, cdiv(d_out, MERGE_CB));
+  const size_t shm = (size_t)hpw * dv * sizeof(float);
+  if (dv <= 256)
+    merge_up_kernel<O, TB, 4><<<grid, dim3(MERGE_UP_T), shm, st>>>(partial, lse, (O*)out, (const TB*)vB, sVb, sVh, sVr, d_out, ns, kl, hq, hkv,
+                                                            kv_len, max_splits, dv, sOb, sOh, hpw, lse_out, sLb, sLh, split_cap, split_plan);
+  else
+    merge_up_kernel<O, TB, 8><<<grid, dim3(MERGE_UP_T), shm, st>>>(partial, lse, (O*)out, (const TB*)vB, sVb, sVh, sVr, d_out, ns, kl, hq, hkv,
+                                                            kv_len, max_splits, dv, sOb, sOh, hpw, lse_out, sLb, sLh, split_cap, split_plan);
   return launch_status();
 }
 

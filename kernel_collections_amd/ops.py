@@ -221,11 +221,25 @@ def recon_stage1(q3, kA, kB, vA, partial, lse, scores, num_kv_splits, kv_lens, b
         "xkv_recon_stage1")
 
 
+MERGE_ROWS_FLOATS = 16384   # partial values a workgroup of the up-projecting merge may fold (64 KiB: its share of one round of loads)
+
+
 def merge_stage2(partial, lse, out, vB, num_kv_splits, kv_lens, batch, hq, hkv, kv_len, max_splits, lse_out=None, split_cap=0,
                  split_plan=None):
     """out `[b,Hq,*]` (strides honoured on the first two axes).  `lse_out` `[b,Hq]` (any strides, fp32): log-sum-exp
     of the merged range.  Up-projections wider than 512 columns run as column blocks of 512."""
     dv = partial.shape[-1]
+    if vB is not None and max_splits > 1 and max_splits * (hq // hkv) * dv > MERGE_ROWS_FLOATS:
+        # many splits: merge the rows first, spread over the chip, then up-project one row per head.  The up-projecting kernel
+        # repeats the merge in every block of 64 columns, which costs more than a second launch once that is
+        # MERGE_ROWS_FLOATS partial values per workgroup.
+        mid, mid_lse = torch.empty((batch, hq, dv), dtype=torch.float32, device=partial.device), lse_out
+        if mid_lse is None:
+            mid_lse = torch.empty((batch, hq), dtype=torch.float32, device=partial.device)
+        merge_stage2(partial, lse, mid, None, num_kv_splits, kv_lens, batch, hq, hq, kv_len, max_splits, mid_lse, split_cap, split_plan)
+        one = uniform_splits(batch, 1, partial.device)
+        return merge_stage2(mid.unsqueeze(2), mid_lse if mid_lse.is_contiguous() else mid_lse.contiguous(), out, vB, one, None,
+                            batch, hq, hkv, 32, 1)
     assert out.stride(-1) == 1
     sl = (0, 0) if lse_out is None else (lse_out.stride(0), lse_out.stride(1))
 

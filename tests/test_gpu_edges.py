@@ -29,3 +29,38 @@ def test_absorb_q(dev, dtype, b, hq, hkv, d, r):
     got = hi.double().cpu() + lo.double().cpu()
     assert max_abs(got, ref) <= 2.0 ** -16 * ref.abs().max().item()
     assert max_abs(hi, ref) <= 2.0 ** (-8 if dtype == BF else -11) * ref.abs().max().item()
+
+
+@pytest.mark.parametrize("b,hq,hkv,S,live,dv,d_out", [
+    (2, 8, 2, 1, 1, 64, 0),          # rows only: one split, narrowest chunk
+    (1, 4, 4, 9, 9, 128, 0),         # one split past a round of eight
+    (1, 2, 2, 300, 270, 512, 0),     # many splits in 64-wide chunks, dead ones at the end
+    (2, 3, 1, 7, 5, 70, 0),          # rows that are not a multiple of 16 bytes
+    (1, 2, 1, 40, 33, 30, 0),
+    (2, 32, 8, 2, 2, 512, 128),      # up-projection: full rows, two column blocks
+    (1, 5, 1, 3, 2, 192, 40),        # five heads (a second group of one), a partial column block
+    (1, 24, 2, 4, 4, 256, 72),       # 12 heads per kv head, the last dv with four packets per thread
+    (1, 32, 1, 1, 1, 512, 512),      # 32 heads on one factor, more head groups than fit one workgroup's LDS
+    (1, 6, 2, 65, 60, 320, 128),     # many splits: rows first, then the up-projection
+    (2, 3, 1, 2, 2, 70, 24),         # odd dv in the up-projecting form
+])
+@pytest.mark.parametrize("dtype", [BF, FP])
+def test_merge(dev, dtype, b, hq, hkv, S, live, dv, d_out):
+    kv_len = 32 * live                                     # 32 tokens per split: `live` of S splits hold tokens
+    part = gen((b, hq, S, dv), dtype=torch.float32, seed=1)
+    lse = gen((b, hq, S), std=4.0, dtype=torch.float32, seed=2)
+    w = torch.softmax(lse[..., :live].double(), -1)
+    ref = (w.unsqueeze(-1) * part[:, :, :live].double()).sum(2)
+    part[:, :, live:], lse[..., live:] = float("nan"), float("nan")      # dead splits are never read
+    vB = None
+    if d_out:
+        vB = gen((b, hkv, dv, d_out), std=dv ** -0.5, dtype=dtype, seed=3)
+        ref = torch.einsum("bkgr,bkrd->bkgd", ref.reshape(b, hkv, hq // hkv, dv), vB.double()).reshape(b, hq, d_out)
+        vB = vB.to(dev)
+    out = torch.empty((b, hq, d_out or dv), dtype=torch.float32, device=dev)
+    lse_out = torch.empty((b, hq), dtype=torch.float32, device=dev)
+    ops.merge_stage2(part.to(dev), lse.to(dev), out, vB, ops.uniform_splits(b, S, dev), None, b, hq, hkv if d_out else hq, kv_len, S,
+                     lse_out=lse_out)
+    # fp32 sums of at most 300 splits and 512 ranks of unit terms, v_exp_f32 weights to 2^-21 of their value at |lse| <= 20
+    assert max_abs(out, ref) <= 2e-5 * max(1.0, ref.abs().max().item())
+    assert max_abs(lse_out, torch.logsumexp(lse[..., :live].double(), -1)) <= 1e-5
