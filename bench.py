@@ -552,7 +552,7 @@ def bench_c4(args, dev, vfact):
               for i in (order[0], order[B // 2], order[-1])}
     total_ms, step_q = time_loop(fn, args.steps, args.warmup)
     us = total_ms * 1e3 / args.steps
-    # the same call with the caller's splits taken as they are (split_cap_tokens = 0: the kernels add no splits)
+    # the same call with the caller's splits taken as they are (no plan)
     saved = gqa.MAX_SPLIT_TOKENS, gqa.MAX_SPLIT_TOKENS_WIDE
     gqa.MAX_SPLIT_TOKENS = gqa.MAX_SPLIT_TOKENS_WIDE = 0
     try:
@@ -562,8 +562,7 @@ def bench_c4(args, dev, vfact):
     algo_bytes = sum(lens) * per_tok
     gbs = algo_bytes / (us * 1e-6) / 1e9
     # the split length the wrappers planned on the device for this batch (read back here, outside every timed region)
-    plan_S = ops.capped_splits(Lmax, S, gqa.MAX_SPLIT_TOKENS_WIDE)
-    limit = int(ops.plan_splits(kl, ns, plan_S, gqa.MAX_SPLIT_TOKENS_WIDE, ops.num_cus())[0].item())
+    limit = int(ops.ragged_plan(kl, B, 1, Lmax, gqa.MAX_SPLIT_TOKENS_WIDE)[3][0].item())
     cpu = None
     if not args.no_cpu:
         # an eighth of every length (fp32): the scan is linear in the number of tokens, value = time x 8
@@ -589,8 +588,8 @@ def bench_c4(args, dev, vfact):
                                % (" V-factorised r512" if vfact else "", split), "sum_len": sum(lens), "max_len": Lmax,
                    "kv_splits_max_at_the_call": S,
                    "split_length_planned_on_the_device_tokens": limit,
-                   "kv_splits_max_in_the_kernel": max(max(s_, -(-n // limit)) for n, s_ in zip(lens, ns_l)),
-                   "workgroups_with_work": sum(max(s_, -(-n // limit)) for n, s_ in zip(lens, ns_l)),
+                   "kv_splits_max_in_the_kernel": max(-(-n // limit) for n in lens),
+                   "workgroups_with_work": sum(-(-n // limit) for n in lens),
                    "compute_units": ops.num_cus()},
         "roofline": {"bound": "hbm", "kernel": "latent_ring_kernel",
                      "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS,

@@ -18,6 +18,8 @@
  *   - split arithmetic (which tokens split i of a sequence covers, which splits are live) is
  *     the reference's, flash_decoding/gqa.py:95-99 and :273-281, bit for bit, with the
  *     sequence length taken from kv_lens[b] when kv_lens != NULL (ragged batch) else kv_len.
+ *   - num_kv_splits may be NULL (stage 1, merge, plan): every sequence then has max_splits splits, or - with split_cap_tokens or
+ *     a split plan - as many as the cap alone makes.  A kernel's first loads then do not wait for the array.
  *   - `split_cap_tokens` (xkv_latent_stage1, xkv_merge_stage2; 0 = off): no split longer than this many tokens.  Sequence b is
  *     then scanned with max(num_kv_splits[b], ceil(len_b / split_cap_tokens)) splits in that same arithmetic, evaluated on
  *     the device by stage 1 and by the merge alike, so a ragged batch whose caller asks for long splits is still spread over

@@ -99,6 +99,26 @@ def lib():
     return _lib
 
 
+_ctypes_lib, _native = lib, None
+NATIVE_PATH = os.path.join(_HERE, "_xkv_host.so")
+
+
+def native():
+    """The native host layer (csrc/host.cpp): whole calls - checks, split choice, scratch, every launch - in one.  None while the
+    ctypes binding is replaced by another object (an instrumenting proxy, say): launches then go through that, one by one."""
+    global _native
+    if lib is not _ctypes_lib:
+        return None
+    if _native is None:
+        _ctypes_lib()
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError(f"{NATIVE_PATH} is missing: build it with `python -m kernel_collections_amd.build`")
+        from . import _xkv_host
+        _xkv_host.init(LIB_PATH)
+        _native = _xkv_host
+    return _native
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = lib().xkv_error_string(rc).decode()

@@ -1,4 +1,5 @@
-"""Build libxkv_hip.so (gfx950 only) from csrc/*.hip with hipcc.  No torch / pybind headers involved."""
+"""Build libxkv_hip.so (gfx950 only) from csrc/*.hip with hipcc - no torch headers involved - and the native host layer
+_xkv_host.so from csrc/host.cpp with the host compiler."""
 from __future__ import annotations
 
 import concurrent.futures as cf
@@ -10,6 +11,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libxkv_hip.so")
+HOST = os.path.join(HERE, "_xkv_host.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -65,13 +67,31 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _compile_host() -> None:
+    """csrc/host.cpp, the native host layer: a plain CPython extension over the C++ tensor API (the libraries it names are
+    those `import torch` has loaded)."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+           "-isystem", os.path.join(root, "include"), "-isystem", sysconfig.get_paths()["include"], "-isystem", "/opt/rocm/include",
+           os.path.join(CSRC, "host.cpp"), "-o", HOST, "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10",
+           "-lc10_hip", "-ldl"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed on host.cpp:\n{r.stderr}")
+
+
 def build(verbose: bool = True) -> str:
-    """Compile every kernel source and link the shared library; always recompiles."""
+    """Compile every kernel source and link the shared library, and build the native host layer; always recompiles."""
     _check_compiler()
     os.makedirs(OBJ, exist_ok=True)
     srcs = sources()
-    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        host = ex.submit(_compile_host)
         objs = list(ex.map(_compile, srcs))
+        host.result()
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs]
     subprocess.check_call(cmd)
     if verbose:

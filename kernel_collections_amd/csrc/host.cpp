@@ -1,0 +1,559 @@
+// Native host layer of the decode and score calls: checks, split choice, scratch and every launch of one call behind a single
+// Python call.  A decode step of a short context is 10 - 20 us of kernels; marshalled through ctypes, launch by launch, the same
+// call cost 28 us (plain GQA, two launches) to 102 us (prefix + tail, six) of host time and was bound by it.
+//
+// Each function takes the operands as the public wrapper got them and returns its result, or None when an operand is not
+// what it serves as it is (a shape the wrapper asserts on, a layout that has to be copied first): the wrapper then goes through its
+// general path, which raises or copies.  No state but a per-thread table of split counts, which depend on sizes alone.
+//
+// The C ABI of libxkv_hip.so is called through the addresses of the library that the Python binding loaded (init).
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <dlfcn.h>
+#include <hip/hip_runtime_api.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <array>
+#include <atomic>
+#include <cstdint>
+#include <stdexcept>
+
+#include "../../include/xkv_hip.h"
+
+namespace {
+
+// ---- the kernels' library ------------------------------------------------------------------------------------------
+#define XKV_SYMBOLS(X)                                                                                              \
+  X(xkv_error_string) X(xkv_absorb_q) X(xkv_blockdiag_q) X(xkv_latent_stage1) X(xkv_softmax_pv_stage1) X(xkv_recon_stage1) \
+  X(xkv_recon_workspace_bytes) X(xkv_merge_stage2) X(xkv_plan_splits)
+#define XKV_DECLARE(name) decltype(&name) p_##name = nullptr;
+XKV_SYMBOLS(XKV_DECLARE)
+#undef XKV_DECLARE
+
+struct CallError : std::runtime_error { using std::runtime_error::runtime_error; };
+void check(int rc, const char* what) {
+  if (rc != XKV_OK)
+    throw CallError(std::string(what) + " failed: " + p_xkv_error_string(rc) + " (code " + std::to_string(rc) + ")");
+}
+
+struct Decline {};                       // an operand this layer does not serve as it is
+inline void need(bool ok) { if (!ok) throw Decline(); }
+
+inline int cdiv(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
+
+// ---- splits ----------------------------------------------------------------------------------------------------------
+int num_cus(int device) {
+  static std::array<std::atomic<int>, 64> cache{};
+  if (device < 0 || device >= 64) throw CallError("device index out of range");
+  int n = cache[device].load(std::memory_order_relaxed);
+  if (!n) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0)
+      throw CallError("cannot read the number of compute units");
+    cache[device].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+// Number of KV splits for a stage 1 that keeps `per_cu` workgroups on a CU: the count whose slowest CU is done first when every
+// workgroup costs its tiles plus a start of about four (launch, query and factor loads, first tile).  A count just past a
+// whole number of rounds would leave the chip idle behind a nearly empty last one (batch 3 x 8 kv heads: 11 splits are 264
+// workgroups, two rounds on 256 CUs; 10 are one), and 160 workgroups (batch 20) are one round of a chip that is two thirds full
+// where 480 are two full ones.
+int balanced_splits(int64_t batch, int groups, int64_t kv_len, int tile, int per_cu, int cus) {
+  struct Entry { int64_t batch = -1, kv_len = 0; int groups = 0, tile = 0, per_cu = 0, cus = 0, splits = 0; };
+  static thread_local std::array<Entry, 256> table;
+  size_t h = (size_t)(batch * 1000003 + kv_len) * 31 + groups * 7 + tile * 131 + per_cu;
+  Entry& e = table[(h ^ (h >> 8) ^ (h >> 17)) & 255];
+  if (e.batch == batch && e.kv_len == kv_len && e.groups == groups && e.tile == tile && e.per_cu == per_cu && e.cus == cus) return e.splits;
+  constexpr int XCDS = 8, START = 4;
+  const int64_t blocks = (kv_len + 31) / 32;   // split lengths are multiples of 32 tokens
+  int64_t best = 1, best_cost = INT64_MAX, seen = 0;
+  for (int64_t want = 1; want <= blocks && want <= 4LL * per_cu * cus; ++want) {
+    const int64_t per = (blocks + want - 1) / want, live = (blocks + per - 1) / per;   // splits that hold tokens
+    if (live == seen) continue;
+    seen = live;
+    // clusters of `groups` workgroups (one (sequence, split)) go round-robin over the XCDs, each with cus / XCDS CUs of its own
+    const int64_t slots = (int64_t)per_cu * (cus / XCDS);
+    const int64_t rounds = ((batch * live + XCDS - 1) / XCDS * groups + slots - 1) / slots;
+    const int64_t cost = rounds * ((32 * per + tile - 1) / tile + START);
+    if (cost < best_cost) { best = live; best_cost = cost; }
+    if (rounds > 2 && batch * live * groups > 8LL * per_cu * cus) break;   // finer only adds starts
+  }
+  e = Entry{batch, kv_len, groups, tile, per_cu, cus, (int)best};
+  return (int)best;
+}
+
+int head_groups(int64_t hq) {            // smallest number of equal head groups of at most 32
+  int g = cdiv(hq, 32);
+  while (hq % g) ++g;
+  return g;
+}
+
+// ---- operands --------------------------------------------------------------------------------------------------------
+typedef const at::Tensor& Ten;
+
+int code16(Ten t) {
+  const auto d = t.scalar_type();
+  need(d == at::kBFloat16 || d == at::kHalf);
+  return d == at::kBFloat16 ? XKV_BF16 : XKV_F16;
+}
+int code_any(Ten t) { return t.scalar_type() == at::kFloat ? XKV_F32 : code16(t); }
+
+// unit stride on the feature axis, every other stride a multiple of 8 elements, 16-byte base
+bool rows(Ten t) {
+  const auto st = t.strides();
+  const int64_t n = t.dim();
+  if (st[n - 1] != 1 || (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15)) return false;
+  for (int64_t i = 0; i + 1 < n; ++i)
+    if (st[i] & 7) return false;
+  return true;
+}
+bool packed_q(Ten t) { return t.is_contiguous() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+xkv_kv_operand kv(Ten t, int64_t sh, int64_t dim) { return {t.data_ptr(), t.stride(0), t.stride(1), sh, (int)dim}; }
+constexpr xkv_kv_operand NO_KV = {nullptr, 0, 0, 0, 0};
+constexpr xkv_q_operand NO_Q = {nullptr, 0};
+
+// One call: its device, stream, operand type, and one scratch buffer cut into 256-byte-aligned pieces.
+struct Call {
+  c10::DeviceGuard guard;
+  int device, cus, dt;
+  void* stream;
+  at::TensorOptions opts;
+  at::Tensor scratch;
+  int64_t used = 0;
+  Call(Ten q) : guard(q.device()), device(q.device().index()), cus(num_cus(device)), dt(code16(q)),
+                stream(c10::hip::getCurrentHIPStream(device).stream()), opts(q.options()) {}
+  int64_t plan(int64_t bytes) { const int64_t at = used; used += (bytes + 255) & ~(int64_t)255; return at; }
+  void alloc() { scratch = at::empty({used}, opts.dtype(at::kByte)); }
+  template <typename T> T* get(int64_t at) const { return reinterpret_cast<T*>(reinterpret_cast<char*>(scratch.data_ptr()) + at); }
+};
+inline void same(Ten q, std::initializer_list<const at::Tensor*> ts) {   // same 16-bit type, same device
+  need(q.is_cuda());
+  for (const at::Tensor* t : ts) need(t->is_cuda() && t->device() == q.device() && t->scalar_type() == q.scalar_type());
+}
+
+// Splits of one stage 1 + merge: a count for every sequence, or a plan on the device for a ragged batch.
+struct Splits { int S; int cap; const int32_t* lens; int32_t* plan; };
+
+// A ragged batch: planned on the device so that it is cut into at most one job per workgroup the chip holds, no job shorter than
+// `floor` tokens or a 256th of the longest sequence (which bounds the workspaces).
+struct Ragged { int cap, S, jobs; int64_t at; };
+Ragged ragged(Call& c, int64_t batch, int groups, int64_t kv_len, int floor, int per_cu) {
+  Ragged r;
+  r.cap = std::max<int64_t>(floor, (cdiv(kv_len, 256) + 31) / 32 * 32);
+  r.S = cdiv(kv_len, r.cap);
+  r.jobs = std::max(1, per_cu * c.cus / groups);
+  r.at = c.plan((2 + 2 * batch * (int64_t)r.S) * 4);
+  return r;
+}
+
+// ---- merge (with or without the up-projection by vB [b, hkv, dv, d_out]) ------------------------------------------------
+constexpr int64_t MERGE_ROWS_FLOATS = 16384;   // partial values a workgroup of the up-projecting merge may fold
+struct Up { const void* p; int64_t sb, sh, sr; int d_out, dtype, hkv; };
+bool rows_first(int S, int64_t hq, int hkv, int64_t dv) { return S > 1 && S * (hq / hkv) * dv > MERGE_ROWS_FLOATS; }
+int64_t rows_bytes(int64_t batch, int64_t hq, int64_t dv) { return batch * hq * (dv + 1) * 4; }
+
+void merge(const Call& c, const float* partial, const float* lse, void* out, int64_t sOb, int64_t sOh, int out_dtype, const Up* up,
+           int64_t rows_at, const Splits& s, int64_t batch, int64_t hq, int64_t kv_len, int64_t dv, float* lse_out = nullptr,
+           int64_t sLb = 0, int64_t sLh = 0) {
+  if (!up) {
+    check(p_xkv_merge_stage2(partial, lse, out, nullptr, 0, 0, 0, 0, XKV_BF16, nullptr, s.lens, batch, hq, hq, kv_len, s.S, s.cap,
+                             s.plan, dv, sOb, sOh, out_dtype, lse_out, sLb, sLh, c.stream), "xkv_merge_stage2");
+    return;
+  }
+  if (rows_first(s.S, hq, up->hkv, dv)) {   // many splits: merge the rows first, spread over the chip, then one row per head
+    float* mid = c.get<float>(rows_at);
+    float* mid_lse = lse_out ? lse_out : mid + batch * hq * dv;
+    if (!lse_out) { sLb = hq; sLh = 1; }
+    check(p_xkv_merge_stage2(partial, lse, mid, nullptr, 0, 0, 0, 0, XKV_BF16, nullptr, s.lens, batch, hq, hq, kv_len, s.S, s.cap,
+                             s.plan, dv, hq * dv, dv, XKV_F32, mid_lse, sLb, sLh, c.stream), "xkv_merge_stage2");
+    // a single row's log-sum-exp is not read
+    check(p_xkv_merge_stage2(mid, mid_lse, out, up->p, up->sb, up->sh, up->sr, up->d_out, up->dtype, nullptr, nullptr, batch, hq, up->hkv,
+                             32, 1, 0, nullptr, dv, sOb, sOh, out_dtype, nullptr, 0, 0, c.stream), "xkv_merge_stage2");
+    return;
+  }
+  check(p_xkv_merge_stage2(partial, lse, out, up->p, up->sb, up->sh, up->sr, up->d_out, up->dtype, nullptr, s.lens, batch, hq, up->hkv,
+                           kv_len, s.S, s.cap, s.plan, dv, sOb, sOh, out_dtype, lse_out, sLb, sLh, c.stream), "xkv_merge_stage2");
+}
+
+Up up_of(Ten vB, int64_t hq, int dt) {
+  need(rows(vB) && vB.size(3) <= 512 && vB.size(3) % 8 == 0);
+  Up u{vB.data_ptr(), vB.stride(0), vB.stride(1), vB.stride(2), (int)vB.size(3), dt, (int)vB.size(1)};
+  if (u.hkv == 1 && hq > 32) { u.hkv = head_groups(hq); u.sh = 0; }   // the kernel serves at most 32 query heads per kv head
+  need(hq / u.hkv <= 32);
+  return u;
+}
+
+// ---- arguments -------------------------------------------------------------------------------------------------------
+Ten T(PyObject* o) {
+  need(THPVariable_Check(o));
+  return THPVariable_Unpack(o);
+}
+float F(PyObject* o) {
+  const double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) { PyErr_Clear(); throw Decline(); }
+  return (float)v;
+}
+int64_t I(PyObject* o) {
+  const long long v = PyLong_AsLongLong(o);
+  if (v == -1 && PyErr_Occurred()) { PyErr_Clear(); throw Decline(); }
+  return v;
+}
+at::Tensor lens_of(PyObject* o, Ten q, int64_t batch) {   // undefined: one length
+  if (o == Py_None) return at::Tensor();
+  Ten l = T(o);
+  need(l.is_cuda() && l.device() == q.device() && l.scalar_type() == at::kInt && l.dim() == 1 && l.numel() == batch && l.is_contiguous());
+  return l;
+}
+
+template <typename Fn> PyObject* guarded(Py_ssize_t n, Py_ssize_t want, Fn fn) {
+  if (n != want) { PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", want, n); return nullptr; }
+  try {
+    return fn();
+  } catch (const Decline&) {
+    Py_RETURN_NONE;
+  } catch (const std::exception& e) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+inline PyObject* give(PyObject* o) { Py_INCREF(o); return o; }
+
+// ---- shared pieces of the factorised calls -----------------------------------------------------------------------------
+// Absorbed query q~ = q . B^T as a high + low pair [b, hq, rank]
+void absorb(const Call& c, const void* q, Ten B, void* hi, void* lo, int64_t batch, int64_t hq, int64_t d, int64_t rank) {
+  int64_t hkv = B.size(1), sh = B.stride(1);
+  if (hkv == 1 && hq > 32) { hkv = head_groups(hq); sh = 0; }
+  check(p_xkv_absorb_q(q, B.data_ptr(), hi, lo, batch, hq, hkv, d, rank, B.stride(0), sh, B.stride(2), c.dt, c.stream), "xkv_absorb_q");
+}
+bool ring_rank(int64_t r) { return r == 512 || r == 384 || r == 256; }
+// an absorbed scan over `rank`-wide rows: the LDS-ring kernel (one workgroup per CU) at ranks 256 .. 512, else the register-staged one
+int scan_splits(const Call& c, int64_t batch, int groups, int64_t kv_len, bool ring) {
+  return balanced_splits(batch, groups, kv_len, ring ? 32 : 64, ring ? 1 : 2, c.cus);
+}
+
+// nope_decode(q [b,hq,d], kA [b,L,r], kB [b,hkv,r,d], vA [b,L,rv], vB [b,hkv,rv,dv], o, sm_scale, lens | None) -> o | None
+PyObject* nope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 8, [&]() -> PyObject* {
+    Ten q = T(a[0]), kA = T(a[1]), kB = T(a[2]), vA = T(a[3]), vB = T(a[4]), o = T(a[5]);
+    const float scale = F(a[6]);
+    same(q, {&kA, &kB, &vA, &vB});
+    need(o.is_cuda() && o.device() == q.device());
+    need(q.dim() == 3 && kA.dim() == 3 && kB.dim() == 4 && vA.dim() == 3 && vB.dim() == 4 && o.dim() == 3);
+    const int64_t b = q.size(0), hq = q.size(1), d = q.size(2), L = kA.size(1), r = kA.size(2), hkv = kB.size(1), rv = vA.size(2);
+    need(b > 0 && L > 0 && hkv > 0 && kA.size(0) == b && kB.size(0) == b && vA.size(0) == b && vB.size(0) == b && vA.size(1) == L && vB.size(1) == hkv);
+    need(kB.size(2) == r && kB.size(3) == d && vB.size(2) == rv && hq % hkv == 0 && r % 32 == 0 && rv % 64 == 0 && rv <= 512 && d <= 512 && d % 8 == 0);
+    need(packed_q(q) && rows(kA) && rows(kB) && rows(vA) && o.stride(2) == 1 && o.size(0) == b && o.size(1) == hq && o.size(2) == vB.size(3));
+    need(hkv == 1 || hq / hkv <= 32);
+    Call c(q);
+    const Up up = up_of(vB, hq, c.dt);
+    const at::Tensor lens = lens_of(a[7], q, b);
+    const int groups = head_groups(hq), odt = code_any(o);
+    Ragged rg{};
+    Splits s{0, 0, nullptr, nullptr};
+    if (lens.defined()) { rg = ragged(c, b, groups, L, 128, ring_rank(r) ? 1 : 2); s.S = rg.S; s.cap = rg.cap; }
+    else s.S = scan_splits(c, b, groups, L, ring_rank(r));
+    const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part = c.plan(b * hq * s.S * rv * 4), lse = c.plan(b * hq * s.S * 4);
+    const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
+    c.alloc();
+    if (lens.defined()) {
+      s.lens = lens.data_ptr<int32_t>();
+      s.plan = c.get<int32_t>(rg.at);
+      check(p_xkv_plan_splits(s.lens, nullptr, b, s.S, s.cap, rg.jobs, s.plan, c.stream), "xkv_plan_splits");
+    }
+    absorb(c, q.data_ptr(), kB, c.get<void>(hi), c.get<void>(lo), b, hq, d, r);
+    check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(kA, 0, r), NO_KV, kv(vA, 0, rv), c.get<float>(part),
+                              c.get<float>(lse), nullptr, 0, nullptr, s.lens, b, hq, groups, L, s.S, s.cap, s.plan, scale, 0.f, c.dt,
+                              c.stream), "xkv_latent_stage1");
+    merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, L, rv);
+    return give(a[5]);
+  });
+}
+
+// nope_scores(q [b,hq,1,d], A [b,L,r], B [b,hkv,r,d], sm_scale, fp32_out) -> [b,hq,1,L] | None
+PyObject* nope_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 5, [&]() -> PyObject* {
+    Ten q = T(a[0]), A = T(a[1]), B = T(a[2]);
+    const float scale = F(a[3]);
+    const bool f32 = I(a[4]);
+    same(q, {&A, &B});
+    need(q.dim() == 4 && A.dim() == 3 && B.dim() == 4 && q.size(2) == 1);
+    const int64_t b = q.size(0), hq = q.size(1), d = q.size(3), L = A.size(1), r = A.size(2), hkv = B.size(1);
+    need(b > 0 && L > 0 && hkv > 0 && A.size(0) == b && B.size(0) == b && B.size(2) == r && B.size(3) == d && hq % hkv == 0 && r % 32 == 0);
+    need(d <= 512 && d % 8 == 0 && packed_q(q) && rows(A) && rows(B) && (hkv == 1 || hq / hkv <= 32));
+    Call c(q);
+    const int groups = head_groups(hq), S = scan_splits(c, b, groups, L, ring_rank(r));
+    const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2);
+    c.alloc();
+    at::Tensor out = at::empty({b, hq, 1, L}, f32 ? c.opts.dtype(at::kFloat) : c.opts);
+    absorb(c, q.data_ptr(), B, c.get<void>(hi), c.get<void>(lo), b, hq, d, r);
+    check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(A, 0, r), NO_KV, NO_KV, nullptr, nullptr, out.data_ptr(),
+                              f32 ? XKV_F32 : c.dt, nullptr, nullptr, b, hq, groups, L, S, 0, nullptr, scale, 0.f, c.dt, c.stream),
+          "xkv_latent_stage1");
+    return THPVariable_Wrap(out);
+  });
+}
+
+void recon(const Call& c, Ten q, Ten kA, Ten kB, const at::Tensor* vA, float* partial, float* lse, void* scores, int scores_dtype, int S,
+           int64_t b, int64_t hq, int64_t hkv, int64_t L, float scale, const float* inv, int64_t pos, void* ws, int64_t ws_bytes) {
+  check(p_xkv_recon_stage1(q.data_ptr(), kv(kA, 0, kA.size(2)), kB.data_ptr(), kB.stride(0), kB.stride(1), kB.stride(2),
+                           vA ? kv(*vA, 0, vA->size(2)) : NO_KV, partial, lse, scores, scores_dtype, nullptr, nullptr, b, hq, hkv, L, S,
+                           scale, 1, inv, pos, nullptr, 0, ws, ws_bytes, c.dt, c.stream), "xkv_recon_stage1");
+}
+void rope_operands(Ten q, int64_t hq, int64_t d, Ten kA, Ten kB, Ten inv) {
+  const int64_t b = q.size(0), hkv = kB.size(1), r = kA.size(2);
+  need(b > 0 && kA.size(1) > 0 && hkv > 0 && kA.size(0) == b && kB.size(0) == b && kB.size(2) == r && kB.size(3) == d && d == 128);
+  need(hq % hkv == 0 && hq / hkv <= 16 && r % 32 == 0 && r <= 512 && packed_q(q) && rows(kA) && kB.stride(3) == 1);
+  need(inv.is_cuda() && inv.device() == q.device() && inv.scalar_type() == at::kFloat && inv.numel() == 64 && inv.is_contiguous());
+}
+// the kernels that hold a kv head's factor in registers keep one workgroup per CU; two fit at rank 256 without P.A, the generic
+// kernel keeps two or three
+int recon_splits(const Call& c, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r, bool scores) {
+  const bool resident = ring_rank(r) && G <= 8;
+  const int per_cu = resident ? (scores && r == 256 ? 2 : 1) : r > 256 ? 1 : r > 128 ? 2 : 3;
+  return balanced_splits(b, hkv, L, 32, per_cu, c.cus);
+}
+
+// rope_decode(q [b,hq,128], kA, kB, vA, vB, o, sm_scale, inv_freq, pos_offset, two_pass) -> o | None
+PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 10, [&]() -> PyObject* {
+    Ten q = T(a[0]), kA = T(a[1]), kB = T(a[2]), vA = T(a[3]), vB = T(a[4]), o = T(a[5]), inv = T(a[7]);
+    const float scale = F(a[6]);
+    const int64_t pos = I(a[8]);
+    const bool may_two_pass = I(a[9]);
+    same(q, {&kA, &kB, &vA, &vB});
+    need(o.is_cuda() && o.device() == q.device());
+    need(q.dim() == 3 && kA.dim() == 3 && kB.dim() == 4 && vA.dim() == 3 && vB.dim() == 4 && o.dim() == 3);
+    const int64_t b = q.size(0), hq = q.size(1), L = kA.size(1), r = kA.size(2), hkv = kB.size(1), rv = vA.size(2);
+    rope_operands(q, hq, q.size(2), kA, kB, inv);
+    need(vA.size(0) == b && vA.size(1) == L && vB.size(0) == b && vB.size(1) == hkv && vB.size(2) == rv && rv % 64 == 0 && rv <= 512 && rows(vA));
+    need(o.stride(2) == 1 && o.size(0) == b && o.size(1) == hq && o.size(2) == vB.size(3));
+    Call c(q);
+    const Up up = up_of(vB, hq, c.dt);
+    const int odt = code_any(o);
+    const bool shared = vA.data_ptr() == kA.data_ptr() && vA.sizes() == kA.sizes() && vA.strides() == kA.strides();
+    const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, kB.stride(0)), ws = c.plan(ws_bytes);
+    const float* invp = inv.data_ptr<float>();
+    Splits s{0, 0, nullptr, nullptr};
+    if (may_two_pass && !shared && hq / hkv <= 8 && hq <= 32 && ring_rank(rv) && L % 4 == 0) {
+      // a value basis of its own: scores first, then softmax and P.v_A in one stream for all heads
+      s.S = scan_splits(c, b, 1, L, true);
+      const int64_t sc = c.plan(b * hq * L * 4), part = c.plan(b * hq * s.S * rv * 4), lse = c.plan(b * hq * s.S * 4);
+      const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
+      c.alloc();
+      recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, recon_splits(c, b, hkv, hq / hkv, L, r, true), b, hq, hkv, L,
+            scale, invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
+      check(p_xkv_softmax_pv_stage1(c.get<float>(sc), kv(vA, 0, rv), c.get<float>(part), c.get<float>(lse), nullptr, nullptr, b, hq, L, s.S,
+                                    0, nullptr, c.dt, c.stream), "xkv_softmax_pv_stage1");
+      merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, L, rv);
+      return give(a[5]);
+    }
+    s.S = recon_splits(c, b, hkv, hq / hkv, L, r, false);
+    const int64_t part = c.plan(b * hq * s.S * rv * 4), lse = c.plan(b * hq * s.S * 4);
+    const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
+    c.alloc();
+    recon(c, q, kA, kB, &vA, c.get<float>(part), c.get<float>(lse), nullptr, 0, s.S, b, hq, hkv, L, scale, invp, pos,
+          ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
+    merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, L, rv);
+    return give(a[5]);
+  });
+}
+
+// rope_scores(q [b,hq,1,128], A, B, sm_scale, inv_freq, pos_offset, fp32_out) -> [b,hq,1,L] | None
+PyObject* rope_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 7, [&]() -> PyObject* {
+    Ten q = T(a[0]), A = T(a[1]), B = T(a[2]), inv = T(a[4]);
+    const float scale = F(a[3]);
+    const int64_t pos = I(a[5]);
+    const bool f32 = I(a[6]);
+    same(q, {&A, &B});
+    need(q.dim() == 4 && A.dim() == 3 && B.dim() == 4 && q.size(2) == 1);
+    const int64_t b = q.size(0), hq = q.size(1), L = A.size(1), r = A.size(2), hkv = B.size(1);
+    rope_operands(q, hq, q.size(3), A, B, inv);
+    Call c(q);
+    const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, B.stride(0)), ws = c.plan(ws_bytes);
+    if (ws_bytes) c.alloc();
+    at::Tensor out = at::empty({b, hq, 1, L}, f32 ? c.opts.dtype(at::kFloat) : c.opts);
+    recon(c, q, A, B, nullptr, nullptr, nullptr, out.data_ptr(), f32 ? XKV_F32 : c.dt, recon_splits(c, b, hkv, hq / hkv, L, r, true), b, hq, hkv,
+          L, scale, inv.data_ptr<float>(), pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
+    return THPVariable_Wrap(out);
+  });
+}
+
+// gqa(q [b,hq,d], k [b,L,hkv,d], v | vA [b,L,rv], None | vB, o, sm_scale, lens | None, floor_wide, floor) -> o | None
+PyObject* gqa(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 9, [&]() -> PyObject* {
+    Ten q = T(a[0]), k = T(a[1]), v = T(a[2]), o = T(a[4]);
+    const bool fact = a[3] != Py_None;
+    const float scale = F(a[5]);
+    const int floor_wide = I(a[7]), floor_head = I(a[8]);
+    same(q, {&k, &v});
+    need(o.is_cuda() && o.device() == q.device());
+    need(q.dim() == 3 && k.dim() == 4 && v.dim() == (fact ? 3 : 4) && o.dim() == 3);
+    const int64_t b = q.size(0), hq = q.size(1), d = q.size(2), L = k.size(1), hkv = k.size(2), dv = v.size(-1);
+    need(b > 0 && L > 0 && hkv > 0 && k.size(0) == b && k.size(3) == d && v.size(0) == b && v.size(1) == L && hq % hkv == 0 && hq / hkv <= 32);
+    need(d % 32 == 0 && dv % 64 == 0 && dv <= 512 && packed_q(q) && rows(k) && rows(v) && o.stride(2) == 1 && o.size(0) == b && o.size(1) == hq);
+    if (!fact) need(v.size(2) == hkv && dv == d && o.size(2) == dv);
+    Call c(q);
+    const at::Tensor lens = lens_of(a[6], q, b);
+    const int odt = code_any(o);
+    Up up{};
+    if (fact) {
+      Ten vB = T(a[3]);
+      same(q, {&vB});
+      need(vB.dim() == 4 && vB.size(0) == b && vB.size(1) == hkv && vB.size(2) == dv && o.size(2) == vB.size(3));
+      up = up_of(vB, hq, c.dt);
+    }
+    // 8 kv heads of 128 side by side in a token row: stage 1 serves every head of a split from one workgroup, one per CU
+    const bool row8 = hkv == 8 && d == 128 && hq <= 32 && k.stride(2) == d && k.stride(1) >= 1024;
+    const bool wide8 = row8 && (fact ? ring_rank(dv) && v.stride(1) >= dv : v.stride(2) == d && v.stride(1) >= 1024);
+    // 512-wide token rows beside 512-wide value rows: the same form, against a block-diagonal query
+    const bool wide4 = fact && hkv * d == 512 && dv == 512 && hq <= 32 && k.stride(2) == d;
+    const bool wide = wide8 || wide4;
+    const int floor = wide ? floor_wide : floor_head, per_cu = wide ? 1 : 2, groups = wide ? 1 : (int)hkv;
+    need(floor > 0);
+    Ragged rg{};
+    Splits s{0, 0, nullptr, nullptr};
+    if (lens.defined()) { rg = ragged(c, b, groups, L, floor, per_cu); s.S = rg.S; s.cap = rg.cap; }
+    else s.S = std::min(balanced_splits(b, groups, L, 32, per_cu, c.cus), cdiv(L, floor));
+    const int64_t part = c.plan(b * hq * s.S * dv * 4), lse = c.plan(b * hq * s.S * 4), bd = c.plan(wide4 ? b * hq * 512 * 2 : 0);
+    const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, dv) ? rows_bytes(b, hq, dv) : 0);
+    c.alloc();
+    if (lens.defined()) {
+      s.lens = lens.data_ptr<int32_t>();
+      s.plan = c.get<int32_t>(rg.at);
+      check(p_xkv_plan_splits(s.lens, nullptr, b, s.S, s.cap, rg.jobs, s.plan, c.stream), "xkv_plan_splits");
+    }
+    const void* qp = q.data_ptr();
+    if (wide4) {
+      check(p_xkv_blockdiag_q(qp, c.get<void>(bd), b, hq, hkv, d, c.dt, c.stream), "xkv_blockdiag_q");
+      qp = c.get<void>(bd);
+    }
+    check(p_xkv_latent_stage1({qp, wide4 ? 512 : (int)d}, nullptr, NO_Q, wide4 ? kv(k, 0, 512) : kv(k, k.stride(2), d), NO_KV,
+                              kv(v, fact ? 0 : v.stride(2), dv), c.get<float>(part), c.get<float>(lse), nullptr, 0, nullptr, s.lens, b, hq,
+                              wide4 ? 1 : hkv, L, s.S, s.cap, s.plan, scale, 0.f, c.dt, c.stream), "xkv_latent_stage1");
+    merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, fact ? &up : nullptr, mid, s, b, hq, L, dv);
+    return give(a[4]);
+  });
+}
+
+// mla(q_nope [b,H,w], q_rope [b,H,e], kv [b,L,1,r], None | kv_B [b,1,r,w], k_rope [b,L,1,e], sm_scale) -> [b,H,w] | None
+PyObject* mla(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 6, [&]() -> PyObject* {
+    Ten qn = T(a[0]), qr = T(a[1]), C = T(a[2]), R = T(a[4]);
+    const bool fact = a[3] != Py_None;
+    const float scale = F(a[5]);
+    same(qn, {&qr, &C, &R});
+    need(qn.dim() == 3 && qr.dim() == 3 && C.dim() == 4 && R.dim() == 4 && C.size(2) == 1 && R.size(2) == 1);
+    const int64_t b = qn.size(0), hq = qn.size(1), w = qn.size(2), e = qr.size(2), L = C.size(1), r = C.size(3);
+    need(b > 0 && L > 0 && hq > 0 && C.size(0) == b && R.size(0) == b && R.size(1) == L && qr.size(0) == b && qr.size(1) == hq && R.size(3) == e);
+    need(r % 64 == 0 && r <= 512 && e % 32 == 0 && e > 0 && e <= 128 && packed_q(qn) && packed_q(qr) && rows(C) && rows(R));
+    Call c(qn);
+    Up up{};
+    if (fact) {
+      Ten B = T(a[3]);
+      same(qn, {&B});
+      need(B.dim() == 4 && B.size(0) == b && B.size(1) == 1 && B.size(2) == r && B.size(3) == w && w % 8 == 0 && w <= 512 && rows(B));
+      up = up_of(B, hq, c.dt);
+    } else {
+      need(w == r);
+    }
+    const int groups = head_groups(hq);
+    Splits s{scan_splits(c, b, groups, L, r == 512), 0, nullptr, nullptr};
+    const int64_t hi = c.plan(fact ? b * hq * r * 2 : 0), lo = c.plan(fact ? b * hq * r * 2 : 0);
+    const int64_t part = c.plan(b * hq * s.S * r * 4), lse = c.plan(b * hq * s.S * 4);
+    const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, r) ? rows_bytes(b, hq, r) : 0);
+    c.alloc();
+    at::Tensor o = at::empty({b, hq, w}, c.opts);
+    const void *q_hi = qn.data_ptr(), *q_lo = nullptr;
+    if (fact) {
+      absorb(c, q_hi, T(a[3]), c.get<void>(hi), c.get<void>(lo), b, hq, w, r);
+      q_hi = c.get<void>(hi);
+      q_lo = c.get<void>(lo);
+    }
+    check(p_xkv_latent_stage1({q_hi, (int)r}, q_lo, {qr.data_ptr(), (int)e}, kv(C, 0, r), kv(R, 0, e), kv(C, 0, r), c.get<float>(part),
+                              c.get<float>(lse), nullptr, 0, nullptr, nullptr, b, hq, groups, L, s.S, 0, nullptr, scale, 0.f, c.dt, c.stream),
+          "xkv_latent_stage1");
+    merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), hq * w, w, c.dt, fact ? &up : nullptr, mid, s, b, hq, L, r);
+    return THPVariable_Wrap(o);
+  });
+}
+
+// prefix_tail(q [b,H,w], kA, kB [b,1,r,w], vA, vB [b,1,rv,w], k_tail [b,Lt,1,w], v_tail, sm_scale, logit_cap) -> [b,H,w] | None
+PyObject* prefix_tail(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 9, [&]() -> PyObject* {
+    Ten q = T(a[0]), kA = T(a[1]), kB = T(a[2]), vA = T(a[3]), vB = T(a[4]), kT = T(a[5]), vT = T(a[6]);
+    const float scale = F(a[7]), logit_cap = F(a[8]);
+    same(q, {&kA, &kB, &vA, &vB, &kT, &vT});
+    need(q.dim() == 3 && kA.dim() == 3 && kB.dim() == 4 && vA.dim() == 3 && vB.dim() == 4 && kT.dim() == 4 && vT.dim() == 4);
+    const int64_t b = q.size(0), hq = q.size(1), w = q.size(2), L = kA.size(1), r = kA.size(2), rv = vA.size(2), Lt = kT.size(1);
+    need(b > 0 && L > 0 && Lt > 0 && kB.size(1) == 1 && vB.size(1) == 1 && kT.size(2) == 1 && vT.size(2) == 1);
+    need(kA.size(0) == b && kB.size(0) == b && vA.size(0) == b && vB.size(0) == b && kT.size(0) == b && vT.size(0) == b && vA.size(1) == L && vT.size(1) == Lt);
+    need(kB.size(2) == r && kB.size(3) == w && vB.size(2) == rv && kT.size(3) == w && w != 576 && w != 288 && vB.size(3) == vT.size(3));
+    const int64_t dv = vT.size(3);
+    need(r % 32 == 0 && rv % 64 == 0 && rv <= 512 && w % 32 == 0 && w <= 512 && dv % 64 == 0 && dv <= 512);
+    need(packed_q(q) && rows(kA) && rows(kB) && rows(vA) && rows(kT) && rows(vT));
+    Call c(q);
+    const Up up = up_of(vB, hq, c.dt);
+    const int groups = head_groups(hq);
+    const bool shared = vA.data_ptr() == kA.data_ptr() && vA.strides() == kA.strides() && rv == r;
+    Splits s1{scan_splits(c, b, groups, L, ring_rank(r)), 0, nullptr, nullptr};
+    // the tail in at most four splits of whole 32-token blocks, every one of them live; a cap states the count, because the rows
+    // of the shared workspace are one more: row 0 is the merged, up-projected prefix with its log-sum-exp
+    const int blocks = cdiv(Lt, 32), per = cdiv(blocks, 4), S2 = cdiv(blocks, per);
+    const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part1 = c.plan(b * hq * s1.S * rv * 4), lse1 = c.plan(b * hq * s1.S * 4);
+    const int64_t mid = c.plan(rows_first(s1.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
+    const int64_t part = c.plan(b * hq * (1 + S2) * dv * 4), lse = c.plan(b * hq * (1 + S2) * 4);
+    c.alloc();
+    at::Tensor o = at::empty({b, hq, dv}, c.opts);
+    absorb(c, q.data_ptr(), kB, c.get<void>(hi), c.get<void>(lo), b, hq, w, r);
+    check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(kA, 0, r), NO_KV, shared ? kv(kA, 0, r) : kv(vA, 0, rv),
+                              c.get<float>(part1), c.get<float>(lse1), nullptr, 0, nullptr, nullptr, b, hq, groups, L, s1.S, 0, nullptr, scale,
+                              logit_cap, c.dt, c.stream), "xkv_latent_stage1");
+    float *pf = c.get<float>(part), *lf = c.get<float>(lse);
+    merge(c, c.get<float>(part1), c.get<float>(lse1), pf, hq * (1 + S2) * dv, (1 + S2) * dv, XKV_F32, &up, mid, s1, b, hq, L, rv, lf,
+          hq * (1 + S2), 1 + S2);
+    check(p_xkv_latent_stage1({q.data_ptr(), (int)w}, nullptr, NO_Q, kv(kT, 0, w), NO_KV, kv(vT, 0, dv), pf + dv, lf + 1, nullptr, 0, nullptr,
+                              nullptr, b, hq, groups, Lt, 1 + S2, 32 * per, nullptr, scale, logit_cap, c.dt, c.stream), "xkv_latent_stage1");
+    const Splits s2{1 + S2, 0, nullptr, nullptr};
+    merge(c, pf, lf, o.data_ptr(), hq * dv, dv, c.dt, nullptr, 0, s2, b, hq, 32 * (1 + S2), dv);   // every row live
+    return THPVariable_Wrap(o);
+  });
+}
+
+// balanced_splits(batch, groups, kv_len, tile, per_cu, cus) -> int
+PyObject* py_balanced_splits(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 6, [&]() -> PyObject* {
+    return PyLong_FromLong(balanced_splits(I(a[0]), I(a[1]), I(a[2]), I(a[3]), I(a[4]), I(a[5])));
+  });
+}
+
+// init(path of libxkv_hip.so): the library is loaded already; take the addresses of its entry points
+PyObject* init(PyObject*, PyObject* path) {
+  const char* p = PyUnicode_AsUTF8(path);
+  if (!p) return nullptr;
+  void* h = dlopen(p, RTLD_NOW | RTLD_LOCAL);
+  if (!h) { PyErr_Format(PyExc_RuntimeError, "cannot load %s: %s", p, dlerror()); return nullptr; }
+#define XKV_RESOLVE(name)                                                                  \
+  p_##name = reinterpret_cast<decltype(p_##name)>(dlsym(h, #name));                        \
+  if (!p_##name) { PyErr_Format(PyExc_RuntimeError, "%s has no " #name, p); return nullptr; }
+  XKV_SYMBOLS(XKV_RESOLVE)
+#undef XKV_RESOLVE
+  Py_RETURN_NONE;
+}
+
+#define XKV_FAST(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fn)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {
+    {"init", init, METH_O, nullptr},       XKV_FAST("balanced_splits", py_balanced_splits), XKV_FAST("nope_decode", nope_decode),
+    XKV_FAST("nope_scores", nope_scores),  XKV_FAST("rope_decode", rope_decode),            XKV_FAST("rope_scores", rope_scores),
+    XKV_FAST("gqa", gqa),                  XKV_FAST("mla", mla),                            XKV_FAST("prefix_tail", prefix_tail),
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_xkv_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__xkv_host(void) { return PyModule_Create(&module); }

@@ -146,7 +146,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   }
   const int L = p.kv_lens ? p.kv_lens[b] : p.kv_len;
   int start, end;
-  split_bounds(L, effective_splits(L, p.num_splits[b], split_cap_in_force(p.split_cap, p.split_plan)), split, start, end);
+  split_bounds(L, effective_splits(L, asked_splits(p.num_splits, b, p.max_splits, p.split_cap), split_cap_in_force(p.split_cap, p.split_plan)), split, start, end);
   if (end <= start) return;
   const int hg = p.hq / p.groups, h0 = group * hg;
   const int ntiles = (end - start + TN - 1) / TN;

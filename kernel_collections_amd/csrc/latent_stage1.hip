@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
 
   const int L = p.kv_lens ? p.kv_lens[b] : p.kv_len;
   int start, end;
-  split_bounds(L, effective_splits(L, p.num_splits[b], split_cap_in_force(p.split_cap, p.split_plan)), split, start, end);
+  split_bounds(L, effective_splits(L, asked_splits(p.num_splits, b, p.max_splits, p.split_cap), split_cap_in_force(p.split_cap, p.split_plan)), split, start, end);
   if (end <= start) return;
 
   const int hg = p.hq / p.groups;  // heads of this kv group
@@ -367,7 +367,7 @@ extern "C" int xkv_latent_stage1(xkv_q_operand qn, const void* qn_lo, xkv_q_oper
                                  const int32_t* split_plan, float sm_scale,
                                  float logit_cap,
                                  int dtype, void* stream) {
-  if (!qn.ptr || !C.ptr || !num_kv_splits || batch <= 0 || hq <= 0 || n_kv_groups <= 0 || kv_len <= 0 ||
+  if (!qn.ptr || !C.ptr || batch <= 0 || hq <= 0 || n_kv_groups <= 0 || kv_len <= 0 ||
       max_splits <= 0)
     return XKV_EINVAL;
   // with a cap the longest sequence may need cdiv(kv_len, cap) splits: the workspace must have a row for each
@@ -434,7 +434,7 @@ extern "C" int xkv_latent_stage1(xkv_q_operand qn, const void* qn_lo, xkv_q_oper
 extern "C" int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, float* partial, float* lse,
                                      const int32_t* num_kv_splits, const int32_t* kv_lens, int batch, int hq, int kv_len,
                                      int max_splits, int split_cap_tokens, const int32_t* split_plan, int dtype, void* stream) {
-  if (!scores || !V.ptr || !partial || !lse || !num_kv_splits || batch <= 0 || hq <= 0 || kv_len <= 0 || max_splits <= 0)
+  if (!scores || !V.ptr || !partial || !lse || batch <= 0 || hq <= 0 || kv_len <= 0 || max_splits <= 0)
     return XKV_EINVAL;
   if (split_cap_tokens < 0 || (split_cap_tokens > 0 && max_splits < cdiv(kv_len, split_cap_tokens))) return XKV_EINVAL;
   if (split_plan && split_cap_tokens <= 0) return XKV_EINVAL;

@@ -190,7 +190,7 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
   const int b = wg / (p.hkv * p.max_splits);
   const int L = p.kv_lens ? p.kv_lens[b] : p.kv_len;
   int start, end;
-  split_bounds(L, p.num_splits[b], split, start, end);
+  split_bounds(L, asked_splits(p.num_splits, b, p.max_splits, 0), split, start, end);
   if (end <= start) return;
   const int G = p.hq / p.hkv, h0 = kh * G;
   const int ntiles = (end - start + FT - 1) / FT;

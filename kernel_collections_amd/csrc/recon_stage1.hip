@@ -66,7 +66,7 @@ __global__ __launch_bounds__(256) void recon_stage1_kernel(const ReconParams p) 
   const int b = wg / (p.hkv * p.max_splits);
   const int L = p.kv_lens ? p.kv_lens[b] : p.kv_len;
   int start, end;
-  split_bounds(L, p.num_splits[b], split, start, end);
+  split_bounds(L, asked_splits(p.num_splits, b, p.max_splits, 0), split, start, end);
   if (end <= start) return;
 
   const int G = p.hq / p.hkv, h0 = kh * G;
@@ -374,7 +374,7 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
                                 int hq, int hkv, int kv_len, int max_splits, float sm_scale, int rope,
                                 const float* inv_freq, int64_t pos_offset, const void* sin_cos, int64_t sc_stride_l,
                                 void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
-  if (!q_pe || !kA.ptr || !kB || !num_kv_splits || batch <= 0 || hq <= 0 || hkv <= 0 || kv_len <= 0 || max_splits <= 0)
+  if (!q_pe || !kA.ptr || !kB || batch <= 0 || hq <= 0 || hkv <= 0 || kv_len <= 0 || max_splits <= 0)
     return XKV_EINVAL;
   const bool so = scores_out != nullptr;
   if (!so && (!vA.ptr || !partial || !lse)) return XKV_EINVAL;

@@ -205,7 +205,7 @@ __device__ __forceinline__ MergeAcc<P> merge_fold(const float* __restrict__ pl, 
 #pragma unroll
       for (int e = 0; e < P; ++e) v[k][e] = 0.f;
       if (i < nlive) {
-        w[k] = pl[i];
+        w[k] = pl ? pl[i] : 0.f;
         const float* src = pp + (int64_t)i * dv;
         if constexpr (P == 4) {
           const f32x4 x = *reinterpret_cast<const f32x4*>(src);
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(
   __shared__ float red[256 * P], ml[256][2];
   const int h = blockIdx.x, b = blockIdx.y, c0 = blockIdx.z * chunk;
   const int L = kv_lens ? kv_lens[b] : kv_len;
-  const int nlive = merge_live_splits(L, effective_splits(L, num_kv_splits[b], split_cap_in_force(split_cap, split_plan)), max_splits);
+  const int nlive = merge_live_splits(L, effective_splits(L, asked_splits(num_kv_splits, b, max_splits, split_cap), split_cap_in_force(split_cap, split_plan)), max_splits);
   const int lanes = chunk / P, ngrp = 256 / lanes;          // lanes <= 256
   const int sg = threadIdx.x / lanes, c = c0 + (threadIdx.x % lanes) * P;
   const bool mine = sg < ngrp && c < dv;
@@ -313,11 +313,12 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     if (cols && grp + 64 * r < dv) w[r] = ld16<vec8>(Bh + (int64_t)(grp + 64 * r) * sVr);
   }
   const int L = kv_lens ? kv_lens[b] : kv_len;
-  const int nlive = merge_live_splits(L, effective_splits(L, num_kv_splits[b], split_cap_in_force(split_cap, split_plan)), max_splits);
+  const int nlive = merge_live_splits(L, effective_splits(L, asked_splits(num_kv_splits, b, max_splits, split_cap), split_cap_in_force(split_cap, split_plan)), max_splits);
   auto merge_packet = [&](int gi, int c, auto tag) {
     constexpr int P = decltype(tag)::value;
     const int64_t row = ((int64_t)b * hq + hfirst + gi) * max_splits;
-    const MergeAcc<P> a = merge_fold<P>(lse + row, partial + row * dv + c, dv, 0, 1, nlive);
+    // a single row's weight is 1 whatever its log-sum-exp
+    const MergeAcc<P> a = merge_fold<P>(max_splits == 1 && !lse_out ? nullptr : lse + row, partial + row * dv + c, dv, 0, 1, nlive);
     const float inv = nlive > 0 ? 1.f / a.l : 0.f;
 #pragma unroll
     for (int e = 0; e < P; ++e) merged[gi * dv + c + e] = a.acc[e] * inv;
@@ -483,7 +484,7 @@ __global__ __launch_bounds__(256) void plan_splits_kernel(const int32_t* __restr
   auto live_of = [&](int b) {
     const int L = kv_lens[b];
     if (L <= 0) return 0;
-    const int n = effective_splits(L, num_splits[b], cap);
+    const int n = effective_splits(L, asked_splits(num_splits, b, max_splits, cap), cap);
     const int per = cdiv(cdiv(L, n), MIN_BLOCK_KV) * MIN_BLOCK_KV;
     const int live = cdiv(L, per);
     return live < max_splits ? live : max_splits;
@@ -528,7 +529,7 @@ using namespace xkv;
 
 extern "C" int xkv_plan_splits(const int32_t* kv_lens, const int32_t* num_kv_splits, int batch, int max_splits, int floor_tokens,
                                int target_jobs, int32_t* plan, void* stream) {
-  if (!kv_lens || !num_kv_splits || !plan || batch <= 0 || max_splits <= 0 || floor_tokens <= 0 || target_jobs <= 0) return XKV_EINVAL;
+  if (!kv_lens || !plan || batch <= 0 || max_splits <= 0 || floor_tokens <= 0 || target_jobs <= 0) return XKV_EINVAL;
   plan_splits_kernel<<<dim3(1), dim3(256), 0, (hipStream_t)stream>>>(kv_lens, num_kv_splits, batch, max_splits, floor_tokens,
                                                                      target_jobs, plan);
   return launch_status();
@@ -633,7 +634,7 @@ extern "C" int xkv_merge_stage2(const float* partial, const float* lse, void* ou
                                 const int32_t* kl, int batch, int hq, int hkv, int kv_len, int max_splits,
                                 int split_cap_tokens, const int32_t* split_plan, int dv, int64_t sOb, int64_t sOh, int out_dtype, float* lse_out,
                                 int64_t sLb, int64_t sLh, void* stream) {
-  if (!partial || !lse || !out || !ns || batch <= 0 || hq <= 0 || hkv <= 0 || max_splits <= 0 || dv <= 0)
+  if (!partial || !lse || !out || batch <= 0 || hq <= 0 || hkv <= 0 || max_splits <= 0 || dv <= 0)
     return XKV_EINVAL;
   if (split_cap_tokens < 0 || (split_cap_tokens > 0 && (kv_len <= 0 || max_splits < cdiv(kv_len, split_cap_tokens)))) return XKV_EINVAL;
   if (split_plan && split_cap_tokens <= 0) return XKV_EINVAL;

@@ -86,6 +86,12 @@ __host__ __device__ __forceinline__ int effective_splits(int kv_len, int num_spl
   return num_splits;
 }
 
+// Split count a caller asks for: its device array's, or - with no array - one count for the whole batch: every row of the
+// workspace, or with a cap (or plan) as many as that alone makes.  Without the array a kernel's first loads do not wait for it.
+__host__ __device__ __forceinline__ int asked_splits(const int32_t* num_splits, int b, int max_splits, int cap_tokens) {
+  return num_splits ? num_splits[b] : cap_tokens > 0 ? 1 : max_splits;
+}
+
 // The cap in force: the host's value, raised by the one a planning kernel left in the first word of its plan (if any).
 __device__ __forceinline__ int split_cap_in_force(int cap_tokens, const int32_t* plan) {
   if (!plan) return cap_tokens;

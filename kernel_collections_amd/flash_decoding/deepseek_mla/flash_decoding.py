@@ -14,7 +14,7 @@ from __future__ import annotations
 
 import torch
 
-from kernel_collections_amd import ops
+from kernel_collections_amd import _lib, ops
 from kernel_collections_amd.flash_decoding.mla import stage1_operands
 
 
@@ -69,6 +69,11 @@ def mla_decode_attention_fwd_pd_sep(q, k_buffer, v_buffer, k_buffer_decoded, v_b
 
 def mla_decode_attention_fwd_pd_sep_xKV(q, k_A_buffer, k_B_buffer, v_A_buffer, v_B_buffer, k_buffer_decoded,
                                         v_buffer_decoded, sm_scale=1.0, logit_cap=0.0):
+    native = _lib.native()
+    out = native and native.prefix_tail(q, k_A_buffer, k_B_buffer, v_A_buffer, v_B_buffer, k_buffer_decoded, v_buffer_decoded,
+                                        sm_scale, logit_cap)
+    if out is not None:
+        return out
     batch, num_q_heads, head_dim = q.shape
     _, prefill_kv_len, rank = k_A_buffer.shape
     num_kv_heads = k_B_buffer.shape[1]

@@ -7,40 +7,36 @@ Call surface of the reference's flash_decoding/gqa.py:339-434 (``decode_attentio
     ``group_query_attention_factorized_v_only``, reference attention.py:202-274) as a split-K kernel
     that accumulates ``P @ v_A`` in rank space and multiplies by ``v_B`` after the merge.
 Split ranges follow gqa.py:95-99 exactly; ``sm_scale`` multiplies the scores (gqa.py:122).  The caller's split counts are a
-lower bound: a sequence is cut into more splits when that is what fills the device (split-K is exact under the merge), by a
-fixed cap in the per-head form and by a per-call plan computed on the device in the all-heads forms.
+hint: a sequence is cut into what fills the device (split-K is exact under the merge), chosen on the host for a batch of one
+length and per call on the device for a ragged one.
 """
 from __future__ import annotations
 
 import torch
 
-from kernel_collections_amd import ops
+from kernel_collections_amd import _lib, ops
 
 
-# Longest split, in tokens, that stage 1 scans as one workgroup (0: the caller's splits as they are).  The kernels raise a
-# sequence's split count to ceil(len / this) when the caller asked for fewer (`split_cap_tokens` of the C entry points):
-# split-K is exact under the merge, so the caller's count is a lower bound on the parallelism, not part of the result, and a
-# ragged batch scanned in 4096-token splits would otherwise leave most CUs idle behind its longest sequences.
-MAX_SPLIT_TOKENS = 1024
-# The all-heads ("wide") forms run one workgroup per CU and per (sequence, split), hkv times fewer workgroups than the
-# per-head form.  There the split length is planned per call: the shortest that still cuts the batch into at most one split
-# per CU, so that every CU gets one job and the jobs are as equal as the lengths allow - never below this floor, which is
-# also what sizes the workspaces (0: the caller's splits as they are).
-MAX_SPLIT_TOKENS_WIDE = 1024
+# Shortest split, in tokens, that the wrappers cut a sequence into (0: the caller's splits as they are).  Split-K is exact under
+# the merge, so the caller's count is a hint about parallelism and not part of the result: the wrappers choose the count that
+# fills the device - for one length on the host, for a ragged batch per call on the device (equal jobs, at most one per
+# workgroup the chip holds).  The caller's own counts miss it on both sides: 32 sequences of 1K .. 128K tokens in 4096-token
+# splits are 315 jobs on 256 CUs (1040 us, planned: 751), 8 of up to 16K are 20 (113 us
+# at no less than 1024 tokens each, planned: 57).
+# At 128 tokens a job's start (about 5 us) is a third of its time.  _WIDE: the all-heads forms, one workgroup per CU.
+MAX_SPLIT_TOKENS = 128
+MAX_SPLIT_TOKENS_WIDE = 128
 
 
-def _plan_wide(lens, splits, S, batch, kv_len):
-    """(cap that sizes the workspaces, their split dimension, split plan on the device or None) of an all-heads call."""
-    floor = MAX_SPLIT_TOKENS_WIDE
+def _plan(wide, lens, splits, S, batch, groups, kv_len):
+    """(num_kv_splits, cap, split dimension of the workspaces, split plan on the device or None) of a call."""
+    floor, per_cu = (MAX_SPLIT_TOKENS_WIDE, 1) if wide else (MAX_SPLIT_TOKENS, 2)
     if not floor:
-        return 0, S, None
-    jobs = ops.num_cus()
-    if lens is None:      # one length: plain host arithmetic
-        per_seq = max(1, jobs // batch)
-        cap = max(floor, -(-(-(-kv_len // per_seq)) // 32) * 32)
-        return cap, ops.capped_splits(kv_len, S, cap), None
-    S = ops.capped_splits(kv_len, S, floor)
-    return floor, S, ops.plan_splits(lens, splits, S, floor, jobs)
+        return splits, 0, S, None
+    if lens is not None:
+        return ops.ragged_plan(lens, batch, 1 if wide else groups, kv_len, floor, per_cu)
+    S = min(ops.occupancy_splits(batch, 1 if wide else groups, kv_len, tile=32, waves=per_cu), -(-kv_len // floor))
+    return ops.uniform_splits(batch, S, splits.device), 0, S, None
 
 
 def _prep(q, k_buffer, num_kv_splits, max_kv_splits, kv_lens):
@@ -60,6 +56,10 @@ def _prep(q, k_buffer, num_kv_splits, max_kv_splits, kv_lens):
 def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits, sm_scale=1.0, *, kv_lens=None):
     """q ``[batch, Hq, d]``; k_buffer / v_buffer ``[batch, kv_len, Hkv, d]``; o ``[batch, Hq, d]`` (filled,
     returned); num_kv_splits int32 ``[batch]`` on the device; max_kv_splits int."""
+    native = _lib.native()
+    done = native and native.gqa(q, k_buffer, v_buffer, None, o, sm_scale, kv_lens, MAX_SPLIT_TOKENS_WIDE, MAX_SPLIT_TOKENS)
+    if done is not None:
+        return done
     batch, hq, hkv, d, S, splits, lens = _prep(q, k_buffer, num_kv_splits, max_kv_splits, kv_lens)
     ops.check_16bit(q, k_buffer, v_buffer)
     assert k_buffer.shape[-1] == v_buffer.shape[-1], "head dim of K and V must be the same"
@@ -72,10 +72,7 @@ def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits,
     # rows through its LDS ring), so there are hkv times fewer workgroups and a split may be twice as long
     wide = (hkv * d == 1024 and d == 128 and hq <= 32 and k_buffer.stride(2) == d and v_buffer.stride(2) == d
             and k_buffer.stride(1) >= 1024 and v_buffer.stride(1) >= 1024)
-    if wide:
-        cap, S, plan = _plan_wide(lens, splits, S, batch, kv_len)
-    else:   # room in the workspaces for the splits the kernels may add (host arithmetic only)
-        cap, S, plan = MAX_SPLIT_TOKENS, ops.capped_splits(kv_len, S, MAX_SPLIT_TOKENS), None
+    splits, cap, S, plan = _plan(wide, lens, splits, S, batch, hkv, kv_len)
     partial, lse = ops.workspaces(batch, hq, S, dv, q.device)
     ops.latent_stage1(q3, None, None,
                       (k_buffer, k_buffer.stride(0), k_buffer.stride(1), k_buffer.stride(2), d), None,
@@ -88,6 +85,10 @@ def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits,
 def decode_attention_fwd_v_factorized(q, k_buffer, v_A_buffer, v_B_buffer, o, num_kv_splits, max_kv_splits,
                                       sm_scale=1.0, *, kv_lens=None):
     """K plain ``[batch, kv_len, Hkv, d]``; v_A ``[batch, kv_len, rv]``; v_B ``[batch, Hkv, rv, d]``."""
+    native = _lib.native()
+    done = native and native.gqa(q, k_buffer, v_A_buffer, v_B_buffer, o, sm_scale, kv_lens, MAX_SPLIT_TOKENS_WIDE, MAX_SPLIT_TOKENS)
+    if done is not None:
+        return done
     batch, hq, hkv, d, S, splits, lens = _prep(q, k_buffer, num_kv_splits, max_kv_splits, kv_lens)
     ops.check_16bit(q, k_buffer, v_A_buffer, v_B_buffer)
     rv = v_A_buffer.shape[-1]
@@ -101,7 +102,7 @@ def decode_attention_fwd_v_factorized(q, k_buffer, v_A_buffer, v_B_buffer, o, nu
     wide8 = hkv * d == 1024 and d == 128 and rv in (256, 384, 512) and hq <= 32 and k_buffer.stride(2) == d
     # 512-wide token rows (4 x 128, 2 x 256 ...): the same form, with the block-diagonal query built here
     wide4 = hkv * d == 512 and rv == 512 and hq <= 32 and k_buffer.stride(2) == d
-    cap, S, plan = _plan_wide(lens, splits, S, batch, kv_len) if (wide8 or wide4) else (0, S, None)
+    splits, cap, S, plan = _plan(wide8 or wide4, lens, splits, S, batch, hkv, kv_len)
     partial, lse = ops.workspaces(batch, hq, S, rv, q.device)
     if wide4:
         ops.latent_stage1(ops.blockdiag_q(q3, hkv), None, None,

@@ -8,7 +8,7 @@ from __future__ import annotations
 
 import torch
 
-from kernel_collections_amd import ops
+from kernel_collections_amd import _lib, ops
 from .stage1 import decoding_stage1
 from .stage2 import decoding_stage2
 
@@ -32,6 +32,10 @@ def _run(q_nope, q_rope, kv_nope, k_rope, sm_scale, q_nope_lo=None, up_proj=None
 def mla_decode_attention_fwd(q_nope, q_rope, kv_nope, k_rope, sm_scale=1.0):
     """q_nope ``[batch, H, lora]``, q_rope ``[batch, H, rope]``, kv_nope ``[batch, kv_len, 1, lora]``,
     k_rope ``[batch, kv_len, 1, rope]`` -> ``[batch, H, lora]``."""
+    native = _lib.native()
+    out = native and native.mla(q_nope, q_rope, kv_nope, None, k_rope, sm_scale)
+    if out is not None:
+        return out
     assert kv_nope.shape[2] == 1
     return _run(q_nope, q_rope, kv_nope, k_rope, sm_scale)
 
@@ -41,6 +45,10 @@ def mla_decode_attention_xKV(q_nope, q_rope, kv_A_nope, kv_B_nope, k_rope, sm_sc
     ``q_nope @ kv_B^T`` (reference :81-82) runs in ``xkv_absorb_q`` and is kept as a high + low 16-bit pair, so the scan over
     ``kv_A`` sees the query at ~16 mantissa bits; the un-absorb ``o @ kv_B`` (:128) is the up-projection of the merge
     kernel, applied to the fp32 merged latent."""
+    native = _lib.native()
+    out = native and native.mla(q_nope, q_rope, kv_A_nope, kv_B_nope, k_rope, sm_scale)
+    if out is not None:
+        return out
     assert kv_A_nope.shape[2] == 1
     assert kv_B_nope.shape[1] == 1
     assert kv_B_nope.shape[-1] <= 512 and kv_B_nope.shape[-1] % 8 == 0, "lora rank: a multiple of 8, at most 512"

@@ -5,7 +5,7 @@ from typing import Optional
 
 import torch
 
-from kernel_collections_amd import ops
+from kernel_collections_amd import _lib, ops
 
 
 def _common(q, k_A, k_B, num_kv_splits, max_kv_splits):
@@ -27,9 +27,22 @@ def _lens(kv_lens, batch, device):
     return None if kv_lens is None else ops.as_int32_dev(kv_lens, batch, device)
 
 
+def _plan(lens, batch, groups, kv_len, rank, device):
+    """(num_kv_splits, cap, split dimension, plan) that fill the device: the caller's count is a hint (split-K is exact under the
+    merge), and 128 splits of one long sequence - the reference scripts' count - would leave half the CUs idle."""
+    if lens is not None:
+        return ops.ragged_plan(lens, batch, groups, kv_len, 128, 1 if rank in (256, 384, 512) else 2)
+    S = ops.latent_splits(batch, groups, kv_len, rank, absorbed=True)
+    return ops.uniform_splits(batch, S, device), 0, S, None
+
+
 def decode_nope(q, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale, kv_lens=None):
     """K and V factorised, no positional encoding: absorb q into k_B, scan k_A / v_A once for
     all heads, merge in rank space, then multiply by v_B."""
+    native = _lib.native()
+    done = native and native.nope_decode(q, k_A, k_B, v_A, v_B, o, sm_scale, kv_lens)
+    if done is not None:
+        return done
     assert v_A.shape[1] == k_A.shape[1]
     assert v_B.shape[1] == k_B.shape[1]
     batch, hq, hkv, d, S, splits = _common(q, k_A, k_B, num_kv_splits, max_kv_splits)
@@ -42,12 +55,13 @@ def decode_nope(q, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale
     q3 = ops._q3(q)
     k_A, v_A = ops.as_rows(k_A), ops.as_rows(v_A)
     qt_hi, qt_lo = ops.absorb_q(q3, k_B, want_lo=True)
-    partial, lse = ops.workspaces(batch, hq, S, rank_v, q.device)
     groups = ops.head_groups(hq)
+    splits, cap, S, plan = _plan(lens, batch, groups, kv_len, k_A.shape[-1], q.device)
+    partial, lse = ops.workspaces(batch, hq, S, rank_v, q.device)
     ops.latent_stage1(qt_hi, qt_lo, None, (k_A, k_A.stride(0), k_A.stride(1), 0, k_A.shape[-1]), None,
                       (v_A, v_A.stride(0), v_A.stride(1), 0, rank_v), partial, lse, None, splits, lens,
-                      batch, hq, groups, kv_len, S, float(sm_scale))
-    return ops.merge_stage2(partial, lse, o, v_B, splits, lens, batch, hq, hkv, kv_len, S)
+                      batch, hq, groups, kv_len, S, float(sm_scale), split_cap=cap, split_plan=plan)
+    return ops.merge_stage2(partial, lse, o, v_B, splits, lens, batch, hq, hkv, kv_len, S, split_cap=cap, split_plan=plan)
 
 
 def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_scale, kv_lens=None):
@@ -62,11 +76,14 @@ def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_sca
     q3 = ops._q3(q)
     k_A, v_buffer = ops.as_rows(k_A), ops.as_rows(v_buffer)
     qt_hi, qt_lo = ops.absorb_q(q3, k_B, want_lo=True)
+    # 8 heads of 128 under ranks 256 / 384 / 512: one workgroup serves every kv head of a split
+    wide = hkv == 8 and dv == 128 and hq <= 32 and k_A.shape[-1] in (256, 384, 512) and v_buffer.stride(2) == dv
+    splits, cap, S, plan = _plan(lens, batch, 1 if wide else hkv, kv_len, 512 if wide else k_A.shape[-1], q.device)
     partial, lse = ops.workspaces(batch, hq, S, dv, q.device)
     ops.latent_stage1(qt_hi, qt_lo, None, (k_A, k_A.stride(0), k_A.stride(1), 0, k_A.shape[-1]), None,
                       (v_buffer, v_buffer.stride(0), v_buffer.stride(1), v_buffer.stride(2), dv),
-                      partial, lse, None, splits, lens, batch, hq, hkv, kv_len, S, float(sm_scale))
-    return ops.merge_stage2(partial, lse, o, None, splits, lens, batch, hq, hq, kv_len, S)
+                      partial, lse, None, splits, lens, batch, hq, hkv, kv_len, S, float(sm_scale), split_cap=cap, split_plan=plan)
+    return ops.merge_stage2(partial, lse, o, None, splits, lens, batch, hq, hq, kv_len, S, split_cap=cap, split_plan=plan)
 
 
 # key ranks at which fused RoPE decode with a value basis of its own runs as two passes (scores, then softmax + P.v_A)
@@ -80,6 +97,13 @@ TWO_PASS_MIN_TOKENS = 49152
 def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale, theta, sin_cos,
                 pos_offset=0, kv_lens=None):
     """K = RoPE(k_A @ k_B) rebuilt and rotated in registers, V factorised."""
+    if sin_cos is None and kv_lens is None and ops.USE_RECON_WORKSPACE:
+        native = _lib.native()
+        two_pass = k_A.shape[-1] in TWO_PASS_KEY_RANKS and k_A.shape[0] * k_A.shape[1] >= TWO_PASS_MIN_TOKENS
+        done = native and native.rope_decode(q_pe, k_A, k_B, v_A, v_B, o, sm_scale,
+                                             ops.rope_inv_freq(q_pe.shape[-1], theta, q_pe.device), pos_offset, two_pass)
+        if done is not None:
+            return done
     assert v_A.shape[1] == k_A.shape[1]
     assert v_B.shape[1] == k_B.shape[1]
     batch, hq, hkv, d, S, splits = _common(q_pe, k_A, k_B, num_kv_splits, max_kv_splits)

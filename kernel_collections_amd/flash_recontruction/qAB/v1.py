@@ -13,7 +13,7 @@ from typing import Optional
 
 import torch
 
-from kernel_collections_amd import ops
+from kernel_collections_amd import _lib, ops
 
 
 def _check(q, Ak, Bk):
@@ -36,6 +36,12 @@ def _check(q, Ak, Bk):
 
 
 def _scores(q, Ak, Bk, inv_freq, sin_cos, pos_offset, sm_scale, out_dtype):
+    if sin_cos is None and ops.USE_RECON_WORKSPACE and out_dtype in (None, q.dtype, torch.float32):
+        native = _lib.native()
+        out = native and native.rope_scores(q, Ak, Bk, 1.0 if sm_scale is None else sm_scale, inv_freq, pos_offset,
+                                            out_dtype is torch.float32)
+        if out is not None:
+            return out
     bsz, num_heads, num_kv_heads, head_dim, kv_len, rank = _check(q, Ak, Bk)
     out_dtype = out_dtype or q.dtype
     assert out_dtype in (q.dtype, torch.float32)

@@ -11,7 +11,7 @@ from typing import Optional
 
 import torch
 
-from kernel_collections_amd import ops
+from kernel_collections_amd import _lib, ops
 
 
 def qAB(q: torch.Tensor, Ak: torch.Tensor, Bk: torch.Tensor, *,
@@ -21,6 +21,11 @@ def qAB(q: torch.Tensor, Ak: torch.Tensor, Bk: torch.Tensor, *,
 
     ``sm_scale`` (default: none, like the reference) multiplies the scores; ``out_dtype``
     (default ``q.dtype``) may be ``torch.float32``."""
+    if out_dtype in (None, q.dtype, torch.float32):
+        native = _lib.native()
+        out = native and native.nope_scores(q, Ak, Bk, 1.0 if sm_scale is None else sm_scale, out_dtype is torch.float32)
+        if out is not None:
+            return out
     assert q.dim() == 4, f"Expected q to be 4D, got {q.dim()}D"
     assert Ak.dim() == 3, f"Expected Ak to be 3D, got {Ak.dim()}D"
     assert Bk.dim() == 4, f"Expected Bk to be 4D, got {Bk.dim()}D"

@@ -46,7 +46,7 @@ _splits_cache = {}
 def rope_inv_freq(dim: int, theta: float, device) -> torch.Tensor:
     """fp32 `theta**(-2j/dim)` evaluated exactly as the reference's eager RoPE does on the host
     (flash_recontruction/rope/rope_ref.py:4), cached per (dim, theta, device)."""
-    key = (int(dim), float(theta), str(device))
+    key = (dim, theta, device)
     t = _inv_freq_cache.get(key)
     if t is None:
         inv = 1.0 / (float(theta) ** (torch.arange(0, dim, 2, dtype=torch.int64).float() / dim))
@@ -58,7 +58,7 @@ def rope_inv_freq(dim: int, theta: float, device) -> torch.Tensor:
 def uniform_splits(batch: int, n: int, device) -> torch.Tensor:
     """int32 `[batch]` tensor filled with `n` (what the reference builds with torch.ones(...)*128,
     flash_decoding/mla2/mla_flash_decoding.py:20), cached."""
-    key = (int(batch), int(n), str(device))
+    key = (batch, n, device)
     t = _splits_cache.get(key)
     if t is None:
         t = torch.full((batch,), int(n), dtype=torch.int32, device=device)
@@ -67,11 +67,10 @@ def uniform_splits(batch: int, n: int, device) -> torch.Tensor:
 
 
 def occupancy_splits(batch: int, groups: int, kv_len: int, tile: int = 64, waves: int = 2) -> int:
-    """Number of KV splits that gives about `waves` workgroups per CU without making a split
-    shorter than 4 tiles."""
-    want = _cdiv(waves * num_cus(), max(1, batch * groups))
-    cap = max(1, kv_len // (4 * tile))
-    return max(1, min(want, cap))
+    """Number of KV splits for stage-1 kernels that keep `waves` workgroups on a CU: the count whose slowest CU is done
+    first (`balanced_splits` in csrc/host.cpp, which the native host layer uses itself)."""
+    from . import _xkv_host
+    return _xkv_host.balanced_splits(batch, groups, kv_len, tile, waves, num_cus())
 
 
 def settled_splits(kv_len: int, n: int) -> int:
@@ -237,9 +236,8 @@ def merge_stage2(partial, lse, out, vB, num_kv_splits, kv_lens, batch, hq, hkv, 
         if mid_lse is None:
             mid_lse = torch.empty((batch, hq), dtype=torch.float32, device=partial.device)
         merge_stage2(partial, lse, mid, None, num_kv_splits, kv_lens, batch, hq, hq, kv_len, max_splits, mid_lse, split_cap, split_plan)
-        one = uniform_splits(batch, 1, partial.device)
-        return merge_stage2(mid.unsqueeze(2), mid_lse if mid_lse.is_contiguous() else mid_lse.contiguous(), out, vB, one, None,
-                            batch, hq, hkv, 32, 1)
+        one = uniform_splits(batch, 1, partial.device)      # a single row's log-sum-exp is not read
+        return merge_stage2(mid.unsqueeze(2), mid_lse, out, vB, one, None, batch, hq, hkv, 32, 1)
     assert out.stride(-1) == 1
     sl = (0, 0) if lse_out is None else (lse_out.stride(0), lse_out.stride(1))
 
@@ -278,6 +276,17 @@ def plan_splits(kv_lens: torch.Tensor, num_kv_splits: torch.Tensor, max_splits: 
 def capped_splits(kv_len: int, max_kv_splits: int, cap_tokens: int) -> int:
     """Split dimension of the workspaces when no split may be longer than `cap_tokens` tokens (0: no cap)."""
     return max(int(max_kv_splits), _cdiv(kv_len, cap_tokens)) if cap_tokens else int(max_kv_splits)
+
+
+def ragged_plan(lens, batch: int, groups: int, kv_len: int, floor: int, per_cu: int = 1):
+    """Splits of a ragged batch: ``(num_kv_splits, cap, split dimension of the workspaces, split plan on the device)``.  The
+    split length is planned on the device so that the batch is cut into at most one job per workgroup the chip holds
+    (`per_cu` per CU, `groups` workgroups per job), no shorter than `floor` tokens or a 256th of the longest sequence
+    (which bounds the workspaces)."""
+    cap = max(floor, _cdiv(_cdiv(kv_len, 256), 32) * 32)
+    S = _cdiv(kv_len, cap)
+    one = uniform_splits(batch, 1, lens.device)
+    return one, cap, S, plan_splits(lens, one, S, cap, max(1, per_cu * num_cus() // groups))
 
 
 def workspaces(batch: int, hq: int, max_splits: int, dv: int, device):

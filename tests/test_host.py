@@ -1,0 +1,46 @@
+"""The native host layer: split counts, and that what it declines - operands that have to be copied first - still computes."""
+import pytest
+import torch
+
+import oracle
+from util import check_out, f32, gen
+
+from kernel_collections_amd import _lib, ops
+
+
+@pytest.mark.parametrize("batch,groups,kv_len,tile,per_cu", [
+    (1, 1, 1, 32, 1), (1, 8, 33, 32, 1), (3, 8, 5000, 32, 1), (20, 8, 32768, 32, 1), (1, 1, 262144, 32, 1), (300, 2, 777, 64, 2),
+    (64, 8, 131072, 32, 3), (7, 3, 4099, 64, 2)])
+def test_balanced_splits(batch, groups, kv_len, tile, per_cu):
+    """Every split of the chosen count holds tokens, and no other live count has a shorter slowest CU."""
+    from kernel_collections_amd import _xkv_host
+    cost = lambda S: -(-(-(-batch * S // 8) * groups) // (per_cu * 32)) * (-(-(32 * -(-(-(-kv_len // 32)) // S)) // tile) + 4)
+    S = _xkv_host.balanced_splits(batch, groups, kv_len, tile, per_cu, 256)
+    assert S >= 1 and ops.settled_splits(kv_len, S) == S
+    live = sorted({ops.settled_splits(kv_len, n) for n in range(1, min(-(-kv_len // 32), 1024 * per_cu) + 1)})
+    assert cost(S) <= min(cost(n) for n in live if batch * n * groups <= 8 * per_cu * 256 or n == 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("spoil", ["none", "key_rows", "query", "values", "lens"])
+def test_declined_operands_take_the_general_path(dev, spoil):
+    from kernel_collections_amd.flash_decoding import gqa
+    b, hq, hkv, d, L = 2, 8, 2, 128, 300
+    q, K, V = gen((b, hq, d), seed=1), gen((b, L, hkv, d), seed=2), gen((b, L, hkv, d), seed=3)
+    lens = [L, 77]
+    ref = oracle.ragged_apply(oracle.gqa_plain, lens, f32(q, K, V), (None, 1, 1), sm_scale=d ** -0.5)
+    qd, Kd, Vd, o = q.to(dev), K.to(dev), V.to(dev), torch.zeros(b, hq, d, dtype=q.dtype, device=dev)
+    kl = torch.tensor(lens, dtype=torch.int32, device=dev)
+    if spoil == "key_rows":      # features not unit-stride
+        Kd = torch.empty(b, L, hkv, d, 2, dtype=q.dtype, device=dev)[..., 0].copy_(Kd)
+    elif spoil == "query":       # rows of a wider buffer
+        qd = torch.empty(b, hq, d + 8, dtype=q.dtype, device=dev)[..., :d].copy_(qd)
+    elif spoil == "values":      # rows whose starts are not 16-byte aligned
+        Vd = torch.empty(b, L, hkv, d + 4, dtype=q.dtype, device=dev)[..., :d].copy_(Vd)
+    elif spoil == "lens":
+        kl = kl.to(torch.int64)
+    args = (qd, Kd, Vd, None, o, d ** -0.5, kl, gqa.MAX_SPLIT_TOKENS_WIDE, gqa.MAX_SPLIT_TOKENS)
+    assert (_lib.native().gqa(*args) is None) == (spoil != "none")
+    ns = torch.ones(b, dtype=torch.int32, device=dev)
+    assert gqa.decode_attention_fwd(qd, Kd, Vd, o.zero_(), ns, 1, d ** -0.5, kv_lens=kl) is o
+    check_out(o, ref, spoil)
