@@ -463,7 +463,7 @@ PyObject* mla(PyObject*, PyObject* const* a, Py_ssize_t n) {
       need(w == r);
     }
     const int groups = head_groups(hq);
-    Splits s{scan_splits(c, b, groups, L, r == 512), 0, nullptr, nullptr};
+    Splits s{scan_splits(c, b, groups, L, e == 64 && (r == 512 || (fact && ring_rank(r)))), 0, nullptr, nullptr};
     const int64_t hi = c.plan(fact ? b * hq * r * 2 : 0), lo = c.plan(fact ? b * hq * r * 2 : 0);
     const int64_t part = c.plan(b * hq * s.S * r * 4), lse = c.plan(b * hq * s.S * 4);
     const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, r) ? rows_bytes(b, hq, r) : 0);

@@ -21,7 +21,7 @@ struct LatentParams {
 typedef LatentParams RingParams;
 
 // True when the shape is one the ring kernel is built for: 512-wide latent rows (optionally + 64 RoPE features), or
-// 384 / 256 wide ones scanned with an absorbed query (hi + lo parts); V the latent itself, scores only, a second row
+// 384 / 256 wide ones scanned with an absorbed query (hi + lo parts; the RoPE features too); V the latent itself, scores only, a second row
 // stream 256 / 384 / 512 wide (keys then 256 .. 1024 wide), or plain per-kv-head values [token][8][128] under one shared
 // absorbed key basis or under plain per-head keys taken as one 1024-wide row.  Everything else runs the register-staged kernel.
 bool ring_eligible(const RingParams& p, bool vshared);

@@ -19,6 +19,8 @@
 // LDS tile layout: C (and V) rows are row-major with a 16-byte pad (conflict-free ds_read_b128 over 16 rows and
 // conflict-free transposed reads); the 128-byte RoPE-key rows are stored chunk-major ([8 chunks][TN rows][16 B]):
 // lane l of loader wave w fetches chunk 2w + l/32 of row l%32 and writes it at l * 16 of that wave's 1 KiB piece.
+#include <type_traits>
+
 #include "xkv_common.h"
 #include "latent_ring.h"
 
@@ -42,6 +44,12 @@ template <int OFF> __device__ __forceinline__ u32x4 ring_ldg_s(const void* sbase
   u32x4 v;
   asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3 nt" : "=v"(v) : "v"(voff), "s"(sbase), "n"(OFF));
   return v;
+}
+// a wave-uniform address, said so: the loads above take it in scalar registers
+__device__ __forceinline__ const unsigned char* ring_uniform(const unsigned char* p) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a), hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+  return reinterpret_cast<const unsigned char*>((uint64_t)hi << 32 | lo);
 }
 __device__ __forceinline__ void ring_landed(u32x4& v) { asm volatile("" : "+v"(v)); }
 template <int N> __device__ __forceinline__ void ring_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
@@ -77,13 +85,14 @@ struct RingShape {
   static constexpr int TAIL = KSPLIT * HB * SP * 4 + HB * LDP * 2 + HB * 4 + HB * 8;
   static constexpr int RSLOT = 2;                          // the tile being read and the tile being written
   static constexpr int SHM = RSLOT * SLOT + TAIL;
-  // staging area of the query rows (no-PE features | RoPE features | pad; a second set for the low-order part); used when
-  // it fits beside the ring
-  static constexpr int QSTRIDE = (DN + (HAS_R ? 64 : 0)) * 2 + 16;
-  static constexpr int qst_bytes(bool lo) { return HB * QSTRIDE * (lo ? 2 : 1); }
+  // staging area of the query rows (no-PE features | RoPE features | pad; a second set for the low-order part).  It lies over
+  // the second slot and the tail: neither is written before barrier A of tile 0, and by then the rows are in registers.
   // (not for the 1024-wide form: its query arrives as compact 128-wide rows and is expanded in registers)
-  static constexpr bool qst(bool lo) { return DN != 1024 && VMODE != RING_VGIVEN && SHM + qst_bytes(lo) <= 160 * 1024; }
-  static constexpr int shm(bool lo) { return SHM + (qst(lo) ? qst_bytes(lo) : 0); }
+  static constexpr int QSTRIDE = (DN + (HAS_R ? 64 : 0)) * 2 + 16;
+  static constexpr int QST = SLOT;
+  static constexpr int qst_bytes(bool lo) { return HB * QSTRIDE * (lo ? 2 : 1); }
+  static constexpr bool qst(bool lo) { return DN != 1024 && VMODE != RING_VGIVEN && QST + qst_bytes(lo) <= 160 * 1024; }
+  static constexpr int shm(bool lo) { return qst(lo) && QST + qst_bytes(lo) > SHM ? QST + qst_bytes(lo) : SHM; }
   static_assert(SHM <= 160 * 1024, "ring does not fit the LDS");
 };
 
@@ -112,12 +121,15 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   static_assert(NKS % KSPLIT == 0, "the k-ranges are equal");
   static_assert(!HAS_R || TN == 32, "RoPE-key rows need 32-token tiles");
   static_assert(DN <= 1024 && DVW <= 1024, "a row takes at most two load instructions");
-  constexpr int IPR = DN > 512 ? DN / 512 : 1;    // load instructions per C row (1 KiB each; rows under 1 KiB use DN/8 lanes)
-  constexpr bool CPART = DN < 512;               // a C row fills only part of a load instruction
+  constexpr int IPR = DN > 512 ? DN / 512 : 1;    // load instructions per C row (1 KiB each; 768-byte rows use 48 lanes)
+  constexpr bool CPART = DN == 384;               // a C row fills only part of a load instruction
+  constexpr int CRI = DN == 256 ? 2 : 1, VRI = DVW == 256 ? 2 : 1;   // rows per load instruction: two 512-byte rows share one
   // waves 4..7 move the tile rows; each brings TN/4 rows of C (and V) and two 16-byte chunks of every RoPE-key row
   constexpr int QD = RING_QD;
   constexpr int RPW = TN / 4;                     // rows per loader wave per tile
-  constexpr int LPT = RPW * IPR + ((HAS_R || GIVEN) ? 1 : 0) + (V2 ? RPW * VIPR : 0);   // loads per loader wave per tile
+  constexpr int NCL = RPW / CRI * IPR, NVL = V2 ? RPW / VRI * VIPR : 0;   // C and V load instructions per loader wave and tile
+  constexpr int LPT = NCL + ((HAS_R || GIVEN) ? 1 : 0) + NVL;
+  static_assert(RPW % CRI == 0 && RPW % VRI == 0, "whole row pairs");
   static_assert((QD - 1) * LPT <= 63, "vmcnt holds 6 bits");
   constexpr int DV = (VMODE == RING_VSHARED || GIVEN) ? DN : VHEADS ? RING_DVH : DVW;   // value features of an output row
   constexpr int NVB = VHEADS ? RING_DVH / 16 : DV / 64;   // 16-feature blocks per wave (per kv head under VHEADS)
@@ -169,28 +181,34 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   const int r_row = lane & 31;
   if (__builtin_expect(wave >= 4, 1)) {   // laid out first: the sooner the first loads are issued, the shorter the start
     u32x4 rq[QD][LPT];
+    const unsigned pair_off = (lane & 31) * 16;    // two rows per instruction: the upper lanes take the second one
     auto fetch = [&](int t, u32x4 (&q)[LPT]) {
       const int base = start + t * TN;
       int n = 0;
+      // rows of one stream: `ipr` instructions per row, or `ri` rows per instruction.  Rows past the split end are masked in the
+      // softmax; their reads repeat the last row.
+      auto stream = [&](const unsigned char* sbase, int64_t row_bytes, auto width, auto ipr, auto ri) {
+        constexpr int W = decltype(width)::value, NI = decltype(ipr)::value, RI = decltype(ri)::value;
 #pragma unroll
-      for (int r = 0; r < RPW; ++r) {
-        int tok = base + iw * RPW + r;
-        tok = tok < last ? tok : last;   // rows past the split end are masked in the softmax; keep the read in bounds
-        const unsigned char* row = Cb + (int64_t)tok * crow_bytes;   // wave-uniform
-        if (!CPART || lane < DN / 8) {
-          q[n] = ring_ldg_s<0>(row, lane_off);
-          if (IPR > 1) q[n + 1] = ring_ldg_s<1024>(row, lane_off);
-        }
-        n += IPR;
-        if (V2) {
-          const unsigned char* vrow = Vb + (int64_t)tok * vrow_bytes;
-          if (DVW >= 512 || lane < DVW / 8) {
-            q[n] = ring_ldg_s<0>(vrow, lane_off);
-            if (VIPR > 1) q[n + 1] = ring_ldg_s<1024>(vrow, lane_off);
+        for (int r = 0; r < RPW; r += RI) {
+          int tok = base + iw * RPW + r;
+          const unsigned step = RI == 2 && tok < last ? (unsigned)row_bytes : 0;
+          tok = tok < last ? tok : last;
+          const unsigned char* row = ring_uniform(sbase + (int64_t)tok * row_bytes);
+          if constexpr (RI == 2) {
+            q[n++] = ring_ldg_s<0>(row, pair_off + (lane >= 32 ? step : 0));
+          } else {
+            if (W >= 512 || lane < W / 8) {
+              q[n] = ring_ldg_s<0>(row, lane_off);
+              if (NI > 1) q[n + 1] = ring_ldg_s<1024>(row, lane_off);
+            }
+            n += NI;
           }
-          n += VIPR;
         }
-      }
+      };
+      stream(Cb, crow_bytes, std::integral_constant<int, DN>(), std::integral_constant<int, IPR>(), std::integral_constant<int, CRI>());
+      if constexpr (V2)
+        stream(Vb, vrow_bytes, std::integral_constant<int, DVW>(), std::integral_constant<int, VIPR>(), std::integral_constant<int, VRI>());
       if (HAS_R) {                       // this wave brings chunks 2 iw, 2 iw + 1 of every row
         int tok = base + r_row;
         tok = tok < last ? tok : last;
@@ -205,23 +223,29 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
       }
     };
     auto hand_on = [&](int t, u32x4 (&q)[LPT]) {   // the oldest tile of the queue: QD-1 younger ones stay in flight
-      unsigned char* slot = ring + (t % RSLOT) * SLOT + lane_off;
+      unsigned char* slot = ring + (t % RSLOT) * SLOT;
       ring_wait<(QD - 1) * LPT>();
 #pragma unroll
       for (int i = 0; i < LPT; ++i) ring_landed(q[i]);
       int n = 0;
+      auto stream = [&](unsigned char* dst, auto width, auto ipr, auto ri, auto pitch) {
+        constexpr int W = decltype(width)::value, NI = decltype(ipr)::value, RI = decltype(ri)::value, P = decltype(pitch)::value;
 #pragma unroll
-      for (int r = 0; r < RPW; ++r) {
+        for (int r = 0; r < RPW; r += RI) {
+          unsigned char* row = dst + (iw * RPW + r) * P;
+          if constexpr (RI == 2) {
+            st16(row + (lane >> 5) * P + pair_off, q[n++]);
+          } else {
 #pragma unroll
-        for (int c = 0; c < IPR; ++c, ++n)
-          if (!CPART || lane < DN / 8) st16(slot + (iw * RPW + r) * CROW + c * 1024, q[n]);
-        if (V2) {
-#pragma unroll
-          for (int c = 0; c < VIPR; ++c, ++n)
-            if (DVW >= 512 || lane < DVW / 8) st16(slot + CBYTES + S::RBYTES + (iw * RPW + r) * VROW + c * 1024, q[n]);
+            for (int c = 0; c < NI; ++c, ++n)
+              if (W >= 512 || lane < W / 8) st16(row + lane_off + c * 1024, q[n]);
+          }
         }
-      }
-      if (HAS_R || GIVEN) st16(slot + CBYTES + iw * 1024, q[n]);   // scores: [32 head rows][32 tokens] fp32, row-major
+      };
+      stream(slot, std::integral_constant<int, DN>(), std::integral_constant<int, IPR>(), std::integral_constant<int, CRI>(), std::integral_constant<int, CROW>());
+      if constexpr (V2)
+        stream(slot + CBYTES + S::RBYTES, std::integral_constant<int, DVW>(), std::integral_constant<int, VIPR>(), std::integral_constant<int, VRI>(), std::integral_constant<int, VROW>());
+      if (HAS_R || GIVEN) st16(slot + lane_off + CBYTES + iw * 1024, q[n]);   // scores: [32 head rows][32 tokens] fp32, row-major
     };
     // Iteration j: tile j - QD leaves the queue for the ring (its slot was released by barrier A of the tile before it) and
     // tile j enters the queue in its place, so the look-ahead lives in the queue and a tile is waited for only when the
@@ -263,7 +287,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
     // (Read straight into the operand layout, a load instruction touches 16 half-used cache lines and two waves fetch
     // the same rows: several microseconds at the start of a kernel that lasts tens.)
     constexpr int QSTRIDE = S::QSTRIDE, RQ = HB / 4;   // wave w stages head rows RQ w .. +RQ
-    unsigned char* qst = smem + S::SHM;
+    unsigned char* qst = smem + S::QST;
     u32x4 tmp[RQ * IPR * (LO ? 2 : 1) + (HAS_R ? 1 : 0)];
     int n = 0;
 #pragma unroll
@@ -273,7 +297,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
       const int64_t qoff = ((int64_t)b * p.hq + h0 + row) * (DN * 2) + lane_off;
 #pragma unroll
       for (int c = 0; c < IPR; ++c) {
-        if (!CPART || lane < DN / 8) {
+        if (DN >= 512 || lane < DN / 8) {
           tmp[n] = ld16<u32x4>(reinterpret_cast<const unsigned char*>(p.qn) + qoff + c * 1024);
           if (LO) tmp[n + 1] = ld16<u32x4>(reinterpret_cast<const unsigned char*>(p.qn_lo) + qoff + c * 1024);
         }
@@ -291,7 +315,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
       unsigned char* dst = qst + (wave * RQ + r) * QSTRIDE + lane_off;
 #pragma unroll
       for (int c = 0; c < IPR; ++c) {
-        if (!CPART || lane < DN / 8) {
+        if (DN >= 512 || lane < DN / 8) {
           st16(dst + c * 1024, tmp[n]);
           if (LO) st16(dst + HB * QSTRIDE + c * 1024, tmp[n + 1]);
         }
@@ -306,7 +330,10 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
 #pragma unroll
       for (int k = 0; k < KS_W; ++k) {
         qreg[k][hb] = ld16<vec8>(src + k * 64);
-        if (LO) qlo[k][hb] = ld16<vec8>(src + HB * QSTRIDE + k * 64);
+        if (LO) {
+          qlo[k][hb] = vec8{0, 0, 0, 0, 0, 0, 0, 0};   // the RoPE features have no low-order part
+          if (!HAS_R || ks0 + k < NKS_N) qlo[k][hb] = ld16<vec8>(src + HB * QSTRIDE + k * 64);
+        }
       }
     }
   } else if constexpr (DN == 1024) {
@@ -343,6 +370,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
           if (LO) qlo[k][hb] = ld16<vec8>(ql_l + k * 32);
         } else {
           qreg[k][hb] = ld16<vec8>(qr_l + k * 32);
+          if (LO) qlo[k][hb] = vec8{0, 0, 0, 0, 0, 0, 0, 0};
         }
       }
     }
@@ -620,10 +648,17 @@ static int launch_ring_dt(const RingParams& p, int batch, bool vshared, hipStrea
   XKV_RING_CASE(32, 1, false, 512, false, RING_VSHARED)  XKV_RING_CASE(32, 2, false, 512, false, RING_VSHARED)
   XKV_RING_CASE(32, 1, true, 512, false, RING_VSHARED)   XKV_RING_CASE(32, 2, true, 512, false, RING_VSHARED)
   XKV_RING_CASE(32, 1, false, 512, true, RING_VSHARED)   XKV_RING_CASE(32, 2, false, 512, true, RING_VSHARED)
-  // two row streams (keys 256 .. 1024 wide, values 256 .. 512 wide): 16-token tiles
+  // absorbed latent + RoPE keys (MLA over a factorised latent; batch 8 x 64K at rank 256: 58 us, 5.8 TB/s - the register-staged
+  // kernel: 203; a second workgroup per CU or a deeper queue: 56 - 60)
+  XKV_RING_CASE(32, 1, true, 512, true, RING_VSHARED)    XKV_RING_CASE(32, 2, true, 512, true, RING_VSHARED)
+  XKV_RING_CASE(32, 1, true, 384, true, RING_VSHARED)    XKV_RING_CASE(32, 2, true, 384, true, RING_VSHARED)
+  XKV_RING_CASE(32, 1, true, 256, true, RING_VSHARED)    XKV_RING_CASE(32, 2, true, 256, true, RING_VSHARED)
+  // two row streams (keys 256 .. 1024 wide, values 256 .. 512 wide): 32-token tiles while a token's two rows are below 2 KiB (what
+  // is in flight is two tiles: at 256 + 384 a 16-token tile leaves 42 KB of the 60 - 100 a CU needs - 262144 tokens, batch 1: 79.5
+  // us with 16-token tiles, 61 with 32), 16-token ones from there on (512 + 512: 85 us against 88.5)
 #define XKV_RING_V2(NHB, LO, DN, DVW) \
   if (nhb == NHB && lo == LO && p.dn == DN && !r && vm == RING_VDISTINCT && p.dv == DVW) \
-    return launch_ring_t<T, 16, NHB, LO, DN, false, RING_VDISTINCT, DVW>(p, batch, st);
+    return launch_ring_t<T, DN + DVW >= 1024 ? 16 : 32, NHB, LO, DN, false, RING_VDISTINCT, DVW>(p, batch, st);
 #define XKV_RING_V2_ALL(LO, DN) \
   XKV_RING_V2(1, LO, DN, 512) XKV_RING_V2(2, LO, DN, 512) XKV_RING_V2(1, LO, DN, 384) XKV_RING_V2(2, LO, DN, 384) \
   XKV_RING_V2(1, LO, DN, 256) XKV_RING_V2(2, LO, DN, 256)
@@ -647,8 +682,9 @@ bool ring_eligible(const RingParams& p, bool vshared) {
   if (vm == RING_VHEADS) return true;
   if (hg > 32 || vm < 0) return false;
   if ((p.dn == 1024) != (p.heads_in_row == 8)) return false;   // the 1024-wide form is only the eight-heads-in-a-row one
-  if (p.dn != 512 && !(p.dn == 1024 && vm == RING_VDISTINCT && !lo) && !((p.dn == 384 || p.dn == 256) && lo && !r)) return false;
-  if (r && (p.dr != 64 || lo || vm != RING_VSHARED)) return false;
+  if (p.dn != 512 && !(p.dn == 1024 && vm == RING_VDISTINCT && !lo) && !((p.dn == 384 || p.dn == 256) && lo)) return false;
+  if (r && (p.dr != 64 || vm != RING_VSHARED)) return false;
+  if (p.sCl >= (1 << 29) || (vm == RING_VDISTINCT && p.sVl >= (1 << 29))) return false;   // a row pair's 32-bit lane offset
   if (p.sCl < p.dn || (r && p.sRl < 64) || (vm == RING_VDISTINCT && p.sVl < p.dv)) return false;
   if (vm == RING_VDISTINCT && p.dn == 512 && !lo && p.dv != 512) return false;
   return true;

@@ -64,3 +64,25 @@ def test_merge(dev, dtype, b, hq, hkv, S, live, dv, d_out):
     # fp32 sums of at most 300 splits and 512 ranks of unit terms, v_exp_f32 weights to 2^-21 of their value at |lse| <= 20
     assert max_abs(out, ref) <= 2e-5 * max(1.0, ref.abs().max().item())
     assert max_abs(lse_out, torch.logsumexp(lse[..., :live].double(), -1)) <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", [BF, FP])
+@pytest.mark.parametrize("dn", [256, 384, 512])
+@pytest.mark.parametrize("lens,S", [
+    ([1], 1),            # one token: every row pair repeats it
+    ([33], 1),           # a tile and one token
+    ([640, 517], 2),     # each loader queue wraps several times; an odd end
+])
+def test_ring_absorbed_with_rope_features(dev, dtype, dn, lens, S):
+    """The ring kernel over an absorbed query (high + low part) with 64 RoPE features behind it, ranks 256 / 384 / 512."""
+    import test_gpu_ring_forms as forms
+    for hq in (8, 32):
+        forms.run_form(dev, dtype, hq=hq, dn=dn, lo=True, rope=True, mode="shared", dv=dn, lens=lens, S=S)
+
+
+@pytest.mark.parametrize("dn,dv", [(256, 256), (256, 512), (384, 256)])
+def test_ring_row_pairs_at_odd_ends(dev, dn, dv):
+    """Two 512-byte rows share a load instruction: ends one token past a pair, a tile, a split."""
+    import test_gpu_ring_forms as forms
+    for lens, S in (([1], 1), ([31], 1), ([65, 2], 2)):
+        forms.run_form(dev, BF, hq=16, dn=dn, lo=True, rope=False, mode="row", dv=dv, lens=lens, S=S)
