@@ -20,12 +20,12 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument", "-Wno-inline-asm",
 ]
-# Per-file additions.  the recon_fast_*.hip, recon_spec_*.hip and recon_duo_*.hip units: MFMA results must land in ordinary VGPRs (the RoPE / softmax VALU code reads
+# Per-file additions.  the recon_fast_*.hip, recon_scores.hip, recon_spec_*.hip and recon_duo_*.hip units: MFMA results must land in ordinary VGPRs (the RoPE / softmax VALU code reads
 # them; with accumulation-register results every value costs a v_accvgpr_read), while the stationary B operands are
 # pinned to accumulation registers by the source itself.
 _VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 EXTRA_FLAGS = {
-    "recon_fast_256.hip": _VGPR_FORM,
+    "recon_fast_256.hip": _VGPR_FORM, "recon_scores.hip": _VGPR_FORM,
     "recon_duo_b.hip": _VGPR_FORM, "recon_duo_c.hip": _VGPR_FORM, "recon_spec_512.hip": _VGPR_FORM, "recon_spec_384.hip": _VGPR_FORM, "recon_spec_256.hip": _VGPR_FORM,
 }
 

@@ -311,8 +311,9 @@ void rope_operands(Ten q, int64_t hq, int64_t d, Ten kA, Ten kB, Ten inv) {
   need(inv.is_cuda() && inv.device() == q.device() && inv.scalar_type() == at::kFloat && inv.numel() == 64 && inv.is_contiguous());
 }
 // the kernels that hold a kv head's factor in registers keep one workgroup per CU; two fit at rank 256 without P.A, the generic
-// kernel keeps two or three
-int recon_splits(const Call& c, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r, bool scores) {
+// kernel keeps two or three.  Scores at ranks up to 192: four independent waves of a 16-token tile each, one workgroup per CU.
+int recon_splits(const Call& c, Ten kB, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r, bool scores) {
+  if (scores && r <= 192 && rows(kB)) return balanced_splits(b, hkv, L, 64, 1, c.cus);
   const bool resident = ring_rank(r) && G <= 8;
   const int per_cu = resident ? (scores && r == 256 ? 2 : 1) : r > 256 ? 1 : r > 128 ? 2 : 3;
   return balanced_splits(b, hkv, L, 32, per_cu, c.cus);
@@ -345,14 +346,14 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int64_t sc = c.plan(b * hq * L * 4), part = c.plan(b * hq * s.S * rv * 4), lse = c.plan(b * hq * s.S * 4);
       const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
       c.alloc();
-      recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, recon_splits(c, b, hkv, hq / hkv, L, r, true), b, hq, hkv, L,
+      recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, recon_splits(c, kB, b, hkv, hq / hkv, L, r, true), b, hq, hkv, L,
             scale, invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
       check(p_xkv_softmax_pv_stage1(c.get<float>(sc), kv(vA, 0, rv), c.get<float>(part), c.get<float>(lse), nullptr, nullptr, b, hq, L, s.S,
                                     0, nullptr, c.dt, c.stream), "xkv_softmax_pv_stage1");
       merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, L, rv);
       return give(a[5]);
     }
-    s.S = recon_splits(c, b, hkv, hq / hkv, L, r, false);
+    s.S = recon_splits(c, kB, b, hkv, hq / hkv, L, r, false);
     const int64_t part = c.plan(b * hq * s.S * rv * 4), lse = c.plan(b * hq * s.S * 4);
     const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
     c.alloc();
@@ -378,7 +379,7 @@ PyObject* rope_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, B.stride(0)), ws = c.plan(ws_bytes);
     if (ws_bytes) c.alloc();
     at::Tensor out = at::empty({b, hq, 1, L}, f32 ? c.opts.dtype(at::kFloat) : c.opts);
-    recon(c, q, A, B, nullptr, nullptr, nullptr, out.data_ptr(), f32 ? XKV_F32 : c.dt, recon_splits(c, b, hkv, hq / hkv, L, r, true), b, hq, hkv,
+    recon(c, q, A, B, nullptr, nullptr, nullptr, out.data_ptr(), f32 ? XKV_F32 : c.dt, recon_splits(c, B, b, hkv, hq / hkv, L, r, true), b, hq, hkv,
           L, scale, inv.data_ptr<float>(), pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
     return THPVariable_Wrap(out);
   });

@@ -35,6 +35,11 @@ inline int launch_recon_spec(const FastParams& p, const void* kB, int64_t sBb, i
                        : launch_recon_spec_256(p, kB, sBb, sBh, sBr, batch, dtype, st);
 }
 
+// Scores only at ranks up to 192, up to 16 query heads per kv head (recon_scores.hip).  Reads kB as it is (16-byte packets of unit
+// stride; Bp of the parameters is not used).
+int launch_recon_scores(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype, int rank,
+                        hipStream_t st);
+
 // The 8-wave kernels (recon_duo_impl.h) for key ranks 256 / 384 / 512 with a separate value basis of rank rv (mode 2; the
 // kernel template also has a scores-only mode 0 and a shared-basis mode 1, which the 4-wave kernel above now serves).  Each
 // translation unit serves the shapes it instantiates and returns DUO_NOT_MINE for the others.

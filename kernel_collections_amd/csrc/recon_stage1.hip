@@ -434,6 +434,17 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
     if (rc == DUO_NOT_MINE) rc = launch_recon_duo_c(f, kB, sBb, sBh, sBr, batch, dtype, 2, rank, vA.dim, st);
     if (rc != DUO_NOT_MINE) return rc;
   }
+  // Scores at ranks whose factor fits one wave's registers (128K tokens, 8 kv heads, rank 192: 57 us, generic kernel 88); that
+  // kernel reads kB in 16-byte packets
+  if (so && rope && !sin_cos && rank <= 192 && !((sBb | sBh | sBr) & 7) && (reinterpret_cast<uintptr_t>(kB) & 15) == 0) {
+    FastParams f{};
+    f.q = q_pe; f.kA = kA.ptr; f.sAb = kA.stride_b; f.sAl = kA.stride_l;
+    f.scores = scores_out; f.scores_dtype = scores_dtype;
+    f.num_splits = num_kv_splits; f.kv_lens = kv_lens;
+    f.hq = hq; f.hkv = hkv; f.kv_len = kv_len; f.max_splits = max_splits; f.total_wg = batch * hkv * max_splits;
+    f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
+    return launch_recon_scores(f, kB, sBb, sBh, sBr, batch, dtype, rank, st);
+  }
   return dtype == XKV_BF16 ? dispatch_recon<__bf16>(p, batch, vshared, st) : dispatch_recon<_Float16>(p, batch, vshared, st);
 }
 

@@ -50,8 +50,12 @@ def _scores(q, Ak, Bk, inv_freq, sin_cos, pos_offset, sm_scale, out_dtype):
     Bk = Bk if Bk.stride(-1) == 1 else Bk.contiguous()
     out = torch.empty((bsz, num_heads, 1, kv_len), dtype=out_dtype, device=q.device)
     # ranks 384 / 512 run the wave-specialised MFMA kernel, one workgroup per CU; rank 256 the 4-wave kernel, whose scores-only
-    # form fits a CU twice (252 registers, 78 KB of LDS); below, the register-staged scores kernel keeps 2-3
-    n_splits = ops.occupancy_splits(bsz, num_kv_heads, kv_len, tile=32, waves=1 if rank > 256 else (2 if rank > 128 else 3))
+    # form fits a CU twice (252 registers, 78 KB of LDS); ranks to 192 a kernel of independent waves, one workgroup per CU and 64
+    # tokens per step, or - with a table, or a factor that is not 16-byte packets - the register-staged scores kernel, which keeps 2-3
+    if rank <= 192 and sin_cos is None and ops._row_ok(Bk):
+        n_splits = ops.occupancy_splits(bsz, num_kv_heads, kv_len, tile=64, waves=1)
+    else:
+        n_splits = ops.occupancy_splits(bsz, num_kv_heads, kv_len, tile=32, waves=1 if rank > 256 else (2 if rank > 128 else 3))
     splits = ops.uniform_splits(bsz, n_splits, q.device)
     ops.recon_stage1(q3, Ak, Bk, None, None, None, out, splits, None, bsz, num_heads, num_kv_heads, kv_len,
                      n_splits, 1.0 if sm_scale is None else float(sm_scale), True, inv_freq, int(pos_offset), sin_cos)

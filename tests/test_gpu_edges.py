@@ -3,7 +3,8 @@ remainders or ranges end, against float64 on the CPU."""
 import pytest
 import torch
 
-from util import gen, max_abs
+import oracle
+from util import check_scores, f32, gen, max_abs
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +87,33 @@ def test_ring_row_pairs_at_odd_ends(dev, dn, dv):
     import test_gpu_ring_forms as forms
     for lens, S in (([1], 1), ([31], 1), ([65, 2], 2)):
         forms.run_form(dev, BF, hq=16, dn=dn, lo=True, rope=False, mode="row", dv=dv, lens=lens, S=S)
+
+
+@pytest.mark.parametrize("dtype,out", [(BF, torch.float32), (FP, FP)])
+@pytest.mark.parametrize("b,hq,hkv,L,r,S,lens,off", [
+    (1, 4, 1, 1, 192, 1, None, 0),              # one token: one wave works, three have no tile
+    (2, 8, 2, 33, 32, 1, [33, 16], 0),          # smallest rank; a last tile of one token, a sequence of one tile
+    (1, 16, 1, 2212, 192, 1, None, 131072),     # 35 steps: every buffer, angles seeded three times; 16 heads per kv head
+    (1, 6, 2, 2049, 128, 3, None, 5),           # odd length (scalar stores), several splits
+    (2, 3, 3, 260, 160, 4, [260, 65], 0),       # one head per kv head, splits without tokens
+    (1, 8, 2, 448, 96, 1, None, 0), (1, 8, 2, 256, 64, 2, None, 0),   # whole steps only
+])
+def test_recon_scores_small_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, off):
+    q, A, B = gen((b, hq, 128), std=0.5, dtype=dtype, seed=1), gen((b, L, r), dtype=dtype, seed=2), \
+        gen((b, hkv, r, 128), std=r ** -0.5, dtype=dtype, seed=3)
+    cos, sin = oracle.rope_cos_sin(torch.arange(off, off + L), 128, 5e5)
+    ref = 0.25 * oracle.qab_rope(*f32(q.unsqueeze(2), A, B), cos, sin)
+    qd, Ad, Bd = q.to(dev), A.to(dev), B.to(dev)
+    kl = None if lens is None else torch.tensor(lens, dtype=torch.int32, device=dev)
+    got = {}
+    # the same factor at an odd 8-byte place: not 16-byte packets, so the register-staged kernel
+    shifted = torch.empty(B.numel() + 4, dtype=dtype, device=dev)[4:].view(B.shape).copy_(Bd)
+    for name, f in (("waves", Bd), ("staged", shifted)):
+        s = torch.full((b, hq, 1, L), float("nan"), dtype=out, device=dev)
+        ops.recon_stage1(qd, Ad, f, None, None, None, s, ops.uniform_splits(b, S, qd.device), kl, b, hq, hkv, L, S, 0.25, True,
+                         ops.rope_inv_freq(128, 5e5, qd.device), off, None)
+        got[name] = s
+        for i in range(b):
+            n = L if lens is None else lens[i]
+            check_scores(s[i, ..., :n], ref[i, ..., :n], name)
+            assert s[i, ..., n:].isnan().all()      # nothing is written past a sequence
