@@ -299,9 +299,10 @@ PyObject* nope_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 void recon(const Call& c, Ten q, Ten kA, Ten kB, const at::Tensor* vA, float* partial, float* lse, void* scores, int scores_dtype, int S,
-           int64_t b, int64_t hq, int64_t hkv, int64_t L, float scale, const float* inv, int64_t pos, void* ws, int64_t ws_bytes) {
+           int64_t b, int64_t hq, int64_t hkv, int64_t L, float scale, const float* inv, int64_t pos, void* ws, int64_t ws_bytes,
+           const int32_t* lens = nullptr) {
   check(p_xkv_recon_stage1(q.data_ptr(), kv(kA, 0, kA.size(2)), kB.data_ptr(), kB.stride(0), kB.stride(1), kB.stride(2),
-                           vA ? kv(*vA, 0, vA->size(2)) : NO_KV, partial, lse, scores, scores_dtype, nullptr, nullptr, b, hq, hkv, L, S,
+                           vA ? kv(*vA, 0, vA->size(2)) : NO_KV, partial, lse, scores, scores_dtype, nullptr, lens, b, hq, hkv, L, S,
                            scale, 1, inv, pos, nullptr, 0, ws, ws_bytes, c.dt, c.stream), "xkv_recon_stage1");
 }
 void rope_operands(Ten q, int64_t hq, int64_t d, Ten kA, Ten kB, Ten inv) {
@@ -340,17 +341,25 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, kB.stride(0)), ws = c.plan(ws_bytes);
     const float* invp = inv.data_ptr<float>();
     Splits s{0, 0, nullptr, nullptr};
-    if (may_two_pass && !shared && hq / hkv <= 8 && hq <= 32 && ring_rank(rv) && L % 4 == 0) {
-      // a value basis of its own: scores first, then softmax and P.v_A in one stream for all heads
+    if (may_two_pass && !shared && hq / hkv <= 8 && hq <= 32 && ring_rank(rv)) {
+      // a value basis of its own: scores first, then softmax and P.v_A in one stream for all heads.  The second pass reads the
+      // scores in 16-byte packets, so their rows are whole packets: at another length the kernels get the padded one as the row's
+      // and the true one as every sequence's (one fill, about 2 us).
+      const int64_t row = (L + 3) / 4 * 4;
+      at::Tensor lens;
+      if (row != L) {
+        lens = at::full({b}, L, c.opts.dtype(at::kInt));
+        s.lens = lens.data_ptr<int32_t>();
+      }
       s.S = scan_splits(c, b, 1, L, true);
-      const int64_t sc = c.plan(b * hq * L * 4), part = c.plan(b * hq * s.S * rv * 4), lse = c.plan(b * hq * s.S * 4);
+      const int64_t sc = c.plan(b * hq * row * 4), part = c.plan(b * hq * s.S * rv * 4), lse = c.plan(b * hq * s.S * 4);
       const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
       c.alloc();
-      recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, recon_splits(c, kB, b, hkv, hq / hkv, L, r, true), b, hq, hkv, L,
-            scale, invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
-      check(p_xkv_softmax_pv_stage1(c.get<float>(sc), kv(vA, 0, rv), c.get<float>(part), c.get<float>(lse), nullptr, nullptr, b, hq, L, s.S,
+      recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, recon_splits(c, kB, b, hkv, hq / hkv, L, r, true), b, hq, hkv, row,
+            scale, invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes, s.lens);
+      check(p_xkv_softmax_pv_stage1(c.get<float>(sc), kv(vA, 0, rv), c.get<float>(part), c.get<float>(lse), nullptr, s.lens, b, hq, row, s.S,
                                     0, nullptr, c.dt, c.stream), "xkv_softmax_pv_stage1");
-      merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, L, rv);
+      merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, row, rv);
       return give(a[5]);
     }
     s.S = recon_splits(c, kB, b, hkv, hq / hkv, L, r, false);

@@ -86,12 +86,21 @@ def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_sca
     return ops.merge_stage2(partial, lse, o, None, splits, lens, batch, hq, hq, kv_len, S, split_cap=cap, split_plan=plan)
 
 
-# key ranks at which fused RoPE decode with a value basis of its own runs as two passes (scores, then softmax + P.v_A)
 # A value basis of its own runs as two passes (scores, then softmax + P.v_A) at these key ranks once the call scans at
 # least TWO_PASS_MIN_TOKENS tokens (batch x kv_len); below, the extra launches cost more than the second row stream of
-# the fused 8-wave kernel (measured crossover: 32768 tokens at every rank).
+# the fused 8-wave kernel (measured crossover: 32768 tokens at every rank).  Key ranks up to 192 have no such fused kernel: two
+# passes from TWO_PASS_MIN_TOKENS_SMALL on (key rank 192, value rank 512, 32 heads, us fused / two passes: 4096 tokens
+# 37.5 / 32.2, 32768 107 / 52, 131072 356 / 109; at 2051 31.4 / 32.3, at 1024 21.3 / 26.7).
 TWO_PASS_KEY_RANKS = (512, 384, 256)
 TWO_PASS_MIN_TOKENS = 49152
+TWO_PASS_SMALL_RANK = 192
+TWO_PASS_MIN_TOKENS_SMALL = 4096
+
+
+def _two_pass(rank, tokens, k_B):
+    if rank in TWO_PASS_KEY_RANKS:
+        return tokens >= TWO_PASS_MIN_TOKENS
+    return rank <= TWO_PASS_SMALL_RANK and tokens >= TWO_PASS_MIN_TOKENS_SMALL and ops._row_ok(k_B)
 
 
 def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale, theta, sin_cos,
@@ -99,7 +108,7 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
     """K = RoPE(k_A @ k_B) rebuilt and rotated in registers, V factorised."""
     if sin_cos is None and kv_lens is None and ops.USE_RECON_WORKSPACE:
         native = _lib.native()
-        two_pass = k_A.shape[-1] in TWO_PASS_KEY_RANKS and k_A.shape[0] * k_A.shape[1] >= TWO_PASS_MIN_TOKENS
+        two_pass = _two_pass(k_A.shape[-1], k_A.shape[0] * k_A.shape[1], k_B)
         done = native and native.rope_decode(q_pe, k_A, k_B, v_A, v_B, o, sm_scale,
                                              ops.rope_inv_freq(q_pe.shape[-1], theta, q_pe.device), pos_offset, two_pass)
         if done is not None:
@@ -126,8 +135,7 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
         if sin_cos.dtype != q_pe.dtype or sin_cos.stride(-1) != 1:
             sin_cos = sin_cos.to(q_pe.dtype).contiguous()
     same_basis = (v_A.data_ptr() == k_A.data_ptr() and v_A.shape == k_A.shape and v_A.stride() == k_A.stride())
-    if (not same_basis and k_A.shape[-1] in TWO_PASS_KEY_RANKS and batch * kv_len >= TWO_PASS_MIN_TOKENS
-            and sin_cos is None and hq // hkv <= 8 and hq <= 32
+    if (not same_basis and _two_pass(k_A.shape[-1], batch * kv_len, k_B) and sin_cos is None and hq // hkv <= 8 and hq <= 32
             and rank_v in (256, 384, 512) and kv_len % 4 == 0 and ops.USE_RECON_WORKSPACE):
         # A value basis of its own: two passes.  The scores-only form of the reconstruction kernel runs at the rate of the
         # shared-basis fused kernel (one row stream, no P.A); softmax and P.v_A then stream v_A once for all heads at HBM
@@ -135,7 +143,8 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
         scores = torch.empty((batch, hq, kv_len), dtype=torch.float32, device=q_pe.device)
         # the scores do not depend on how pass 1 cuts the range: one round of workgroups per CU, two at key rank 256, whose
         # scores-only kernel is small enough for two workgroups to share a CU
-        S1 = ops.occupancy_splits(batch, hkv, kv_len, tile=32, waves=2 if k_A.shape[-1] == 256 else 1)
+        S1 = ops.occupancy_splits(batch, hkv, kv_len, tile=64 if k_A.shape[-1] <= TWO_PASS_SMALL_RANK else 32,
+                                  waves=2 if k_A.shape[-1] == 256 else 1)
         ops.recon_stage1(q3, k_A, k_B, None, None, None, scores, ops.uniform_splits(batch, S1, q_pe.device), lens, batch, hq,
                          hkv, kv_len, S1, float(sm_scale), True, inv, int(pos_offset), None)
         S2 = ops.latent_splits(batch, 1, kv_len, rank_v, absorbed=True)

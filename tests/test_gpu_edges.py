@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import oracle
-from util import check_scores, f32, gen, max_abs
+from util import check_out, check_scores, f32, gen, max_abs
 
 pytestmark = pytest.mark.gpu
 
@@ -117,3 +117,30 @@ def test_recon_scores_small_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, of
             n = L if lens is None else lens[i]
             check_scores(s[i, ..., :n], ref[i, ..., :n], name)
             assert s[i, ..., n:].isnan().all()      # nothing is written past a sequence
+
+
+@pytest.mark.parametrize("dtype", [BF, FP])
+@pytest.mark.parametrize("b,hq,hkv,L,rk,rv,off", [
+    (1, 8, 2, 2049, 192, 512, 0),        # a score row past whole packets by one
+    (2, 16, 2, 1027, 64, 256, 70000),    # ... by three, 8 heads per kv head
+    (3, 6, 3, 700, 128, 384, 0),         # whole packets
+    (1, 32, 8, 998, 384, 256, 5),        # the wide ranks' kernels, two past
+    (1, 4, 1, 5, 256, 256, 0),
+])
+def test_two_pass_rope_decode(dev, dtype, b, hq, hkv, L, rk, rv, off, monkeypatch):
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd.flash_recontruction.fused_attention import _fused
+    monkeypatch.setattr(_fused, "TWO_PASS_MIN_TOKENS", 0)
+    monkeypatch.setattr(_fused, "TWO_PASS_MIN_TOKENS_SMALL", 0)
+    q, kA, kB = gen((b, hq, 128), std=0.4, dtype=dtype, seed=1), gen((b, L, rk), dtype=dtype, seed=2), \
+        gen((b, hkv, rk, 128), std=rk ** -0.5, dtype=dtype, seed=3)
+    vA, vB = gen((b, L, rv), dtype=dtype, seed=4), gen((b, hkv, rv, 128), std=rv ** -0.5, dtype=dtype, seed=5)
+    cos, sin = oracle.rope_cos_sin(torch.arange(off, off + L), 128, 5e5)
+    ref = oracle.gqa_factorized_rope(*f32(q.unsqueeze(2), kA, kB, vA, vB), cos, sin, sm_scale=128 ** -0.5)[:, :, 0]
+    qd, kAd, kBd, vAd, vBd = (t.to(dev) for t in (q, kA, kB, vA, vB))
+    ns = torch.full((b,), 2, dtype=torch.int32, device=dev)
+    two = fr.gqa_xKV_rope(qd, kAd, kBd, vAd, vBd, torch.zeros_like(qd), ns, 2, 128 ** -0.5, 5e5, pos_offset=off)
+    check_out(two, ref, "two passes")
+    monkeypatch.setattr(_fused, "TWO_PASS_KEY_RANKS", ())
+    monkeypatch.setattr(_fused, "TWO_PASS_SMALL_RANK", 0)
+    check_out(fr.gqa_xKV_rope(qd, kAd, kBd, vAd, vBd, torch.zeros_like(qd), ns, 2, 128 ** -0.5, 5e5, pos_offset=off), ref, "one kernel")
