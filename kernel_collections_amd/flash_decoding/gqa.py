@@ -56,6 +56,7 @@ def _prep(q, k_buffer, num_kv_splits, max_kv_splits, kv_lens):
 def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits, sm_scale=1.0, *, kv_lens=None):
     """q ``[batch, Hq, d]``; k_buffer / v_buffer ``[batch, kv_len, Hkv, d]``; o ``[batch, Hq, d]`` (filled,
     returned); num_kv_splits int32 ``[batch]`` on the device; max_kv_splits int."""
+    ops.check_splits(num_kv_splits, max_kv_splits, q.shape[0])
     native = _lib.native()
     done = native and native.gqa(q, k_buffer, v_buffer, None, o, sm_scale, kv_lens, MAX_SPLIT_TOKENS_WIDE, MAX_SPLIT_TOKENS)
     if done is not None:
@@ -85,6 +86,7 @@ def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits,
 def decode_attention_fwd_v_factorized(q, k_buffer, v_A_buffer, v_B_buffer, o, num_kv_splits, max_kv_splits,
                                       sm_scale=1.0, *, kv_lens=None):
     """K plain ``[batch, kv_len, Hkv, d]``; v_A ``[batch, kv_len, rv]``; v_B ``[batch, Hkv, rv, d]``."""
+    ops.check_splits(num_kv_splits, max_kv_splits, q.shape[0])
     native = _lib.native()
     done = native and native.gqa(q, k_buffer, v_A_buffer, v_B_buffer, o, sm_scale, kv_lens, MAX_SPLIT_TOKENS_WIDE, MAX_SPLIT_TOKENS)
     if done is not None:

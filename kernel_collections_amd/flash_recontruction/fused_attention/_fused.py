@@ -39,6 +39,7 @@ def _plan(lens, batch, groups, kv_len, rank, device):
 def decode_nope(q, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale, kv_lens=None):
     """K and V factorised, no positional encoding: absorb q into k_B, scan k_A / v_A once for
     all heads, merge in rank space, then multiply by v_B."""
+    ops.check_splits(num_kv_splits, max_kv_splits, q.shape[0])
     native = _lib.native()
     done = native and native.nope_decode(q, k_A, k_B, v_A, v_B, o, sm_scale, kv_lens)
     if done is not None:
@@ -66,6 +67,7 @@ def decode_nope(q, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale
 
 def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_scale, kv_lens=None):
     """K factorised (absorbed), V plain ``[batch, kv_len, num_kv_heads, head_dim]``."""
+    ops.check_splits(num_kv_splits, max_kv_splits, q.shape[0])
     batch, hq, hkv, d, S, splits = _common(q, k_A, k_B, num_kv_splits, max_kv_splits)
     ops.check_16bit(q, k_A, k_B, v_buffer)
     assert v_buffer.shape[1] == k_A.shape[1] and v_buffer.shape[2] == hkv
@@ -106,6 +108,7 @@ def _two_pass(rank, tokens, k_B):
 def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale, theta, sin_cos,
                 pos_offset=0, kv_lens=None):
     """K = RoPE(k_A @ k_B) rebuilt and rotated in registers, V factorised."""
+    ops.check_splits(num_kv_splits, max_kv_splits, q_pe.shape[0])
     if sin_cos is None and kv_lens is None and ops.USE_RECON_WORKSPACE:
         native = _lib.native()
         two_pass = _two_pass(k_A.shape[-1], k_A.shape[0] * k_A.shape[1], k_B)

@@ -46,7 +46,7 @@ _splits_cache = {}
 def rope_inv_freq(dim: int, theta: float, device) -> torch.Tensor:
     """fp32 `theta**(-2j/dim)` evaluated exactly as the reference's eager RoPE does on the host
     (flash_recontruction/rope/rope_ref.py:4), cached per (dim, theta, device)."""
-    key = (dim, theta, device)
+    key = (int(dim), float(theta), device)
     t = _inv_freq_cache.get(key)
     if t is None:
         inv = 1.0 / (float(theta) ** (torch.arange(0, dim, 2, dtype=torch.int64).float() / dim))
@@ -310,6 +310,14 @@ def check_16bit(*ts):
         if t is not None:
             assert t.dtype == dt, f"operand dtypes differ: {t.dtype} vs {dt}"
             _lib.require_gpu(t)
+
+
+def check_splits(num_kv_splits, max_kv_splits, batch: int) -> None:
+    """What every call with split counts refuses, whatever count it then scans with."""
+    if torch.is_tensor(num_kv_splits):
+        assert num_kv_splits.numel() == batch, "num_kv_splits must hold one count per sequence"
+    if max_kv_splits < 1:
+        raise RuntimeError("max_kv_splits must be at least 1")
 
 
 def as_int32_dev(x, batch: int, device) -> torch.Tensor:

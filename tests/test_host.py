@@ -44,3 +44,25 @@ def test_declined_operands_take_the_general_path(dev, spoil):
     ns = torch.ones(b, dtype=torch.int32, device=dev)
     assert gqa.decode_attention_fwd(qd, Kd, Vd, o.zero_(), ns, 1, d ** -0.5, kv_lens=kl) is o
     check_out(o, ref, spoil)
+
+
+def test_split_hints_are_still_checked():
+    """The counts are hints, but a count that fits no call is refused before any path is chosen."""
+    from kernel_collections_amd.flash_decoding import gqa
+    import kernel_collections_amd.flash_recontruction as fr
+    z = lambda *s: torch.zeros(s, dtype=torch.bfloat16)
+    plain = lambda ns, n: gqa.decode_attention_fwd(z(2, 4, 128), z(2, 40, 2, 128), z(2, 40, 2, 128), z(2, 4, 128), ns, n)
+    fact = lambda ns, n: fr.gqa_xKV_no_pe(z(2, 4, 128), z(2, 40, 64), z(2, 2, 64, 128), z(2, 40, 64), z(2, 2, 64, 128), z(2, 4, 128), ns, n, 1.0)
+    for call in (plain, fact):
+        with pytest.raises(AssertionError):
+            call(torch.ones(3, dtype=torch.int32), 1)
+        with pytest.raises(RuntimeError):
+            call(torch.ones(2, dtype=torch.int32), 0)
+
+
+def test_inverse_frequencies_follow_the_base():
+    theta = torch.tensor(1e4)
+    a = ops.rope_inv_freq(128, theta, torch.device("cpu"))
+    theta.fill_(5e5)
+    b = ops.rope_inv_freq(128, theta, torch.device("cpu"))
+    assert not torch.equal(a, b) and torch.equal(b, ops.rope_inv_freq(128, 5e5, torch.device("cpu")))
