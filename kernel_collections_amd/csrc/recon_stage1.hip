@@ -434,7 +434,7 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
     if (rc == DUO_NOT_MINE) rc = launch_recon_duo_c(f, kB, sBb, sBh, sBr, batch, dtype, 2, rank, vA.dim, st);
     if (rc != DUO_NOT_MINE) return rc;
   }
-  // Scores at ranks whose factor fits one wave's registers (128K tokens, 8 kv heads, rank 192: 57 us, generic kernel 88); that
+  // Scores at ranks whose factor fits one wave's registers (128K tokens, 8 kv heads, rank 192: 61 us, generic kernel 88); that
   // kernel reads kB in 16-byte packets
   if (so && rope && !sin_cos && rank <= 192 && !((sBb | sBh | sBr) & 7) && (reinterpret_cast<uintptr_t>(kB) & 15) == 0) {
     FastParams f{};
