@@ -152,7 +152,10 @@ Ragged ragged(Call& c, int64_t batch, int groups, int64_t kv_len, int floor, int
 }
 
 // ---- merge (with or without the up-projection by vB [b, hkv, dv, d_out]) ------------------------------------------------
-constexpr int64_t MERGE_ROWS_FLOATS = 16384;   // partial values a workgroup of the up-projecting merge may fold
+// Partial values a workgroup of the up-projecting merge may fold; beyond, the rows are merged first.  us of one kernel / of rows and
+// up-projection, batches of 1 .. 32 of 16 .. 64 heads, dv 256 and 512: at 32768 5.0 - 14.4 / 7.8 - 17.7, one kernel ahead everywhere; at
+// 49152 even in the narrowest case (batch 4, 48 splits of 256: 8.6 / 8.6); at 65536 behind there (10.6 / 9.9).
+constexpr int64_t MERGE_ROWS_FLOATS = 49152;
 struct Up { const void* p; int64_t sb, sh, sr; int d_out, dtype, hkv; };
 bool rows_first(int S, int64_t hq, int hkv, int64_t dv) { return S > 1 && S * (hq / hkv) * dv > MERGE_ROWS_FLOATS; }
 int64_t rows_bytes(int64_t batch, int64_t hq, int64_t dv) { return batch * hq * (dv + 1) * 4; }

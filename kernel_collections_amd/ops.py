@@ -220,7 +220,7 @@ def recon_stage1(q3, kA, kB, vA, partial, lse, scores, num_kv_splits, kv_lens, b
         "xkv_recon_stage1")
 
 
-MERGE_ROWS_FLOATS = 16384   # partial values a workgroup of the up-projecting merge may fold (64 KiB: its share of one round of loads)
+MERGE_ROWS_FLOATS = 49152   # partial values a workgroup of the up-projecting merge may fold (measured beside the same constant of csrc/host.cpp)
 
 
 def merge_stage2(partial, lse, out, vB, num_kv_splits, kv_lens, batch, hq, hkv, kv_len, max_splits, lse_out=None, split_cap=0,
