@@ -30,6 +30,10 @@
  *     the device value, chosen from the lengths of the batch, which the host never reads, makes the splits as long as the
  *     batch allows while every CU still gets one.  Stage 1 also takes its (sequence, split) pairs from the plan's job
  *     list, so the workgroups that have work are the first ones of the grid and spread evenly over the XCDs.
+ *   - packed plan: with a split_plan and num_kv_splits == NULL (in xkv_plan_splits, stage 1 and the merge alike) the caps alone make
+ *     the jobs, at most max(target_jobs, batch) of them, and max_splits is that number.  partial and lse then hold max_splits rows
+ *     per head for the whole batch - sequence b's are [hq, live splits of b] from row hq * (its first job) on, which the plan
+ *     tells - instead of max_splits rows per head and sequence.
  */
 #ifndef XKV_HIP_H
 #define XKV_HIP_H
@@ -126,7 +130,7 @@ typedef struct {
  * If V.ptr == C.ptr with equal strides and dim the tile is loaded once.
  * If scores_out != NULL the kernel ONLY writes scores (scaled) as [batch, hq, kv_len] in
  * scores_dtype and skips softmax/PV (qAB no-PE form).
- * Dead splits write nothing.  partial is [batch, hq, max_splits, V.dim] fp32, lse [batch, hq, max_splits] fp32.
+ * Dead splits write nothing.  partial is [batch, hq, max_splits, V.dim] fp32, lse [batch, hq, max_splits] fp32 (packed plan: see above).
  * Envelope: heads per kv group <= 32; C.dim % 32 == 0, <= 1024; R.dim % 32 == 0, <= 128;
  *           V.dim % 64 == 0, <= 512.
  * Plain keys of 8 kv heads x 128 stored side by side in a token row (n_kv_groups == 8, C.dim == 128, C.stride_h == 128,
@@ -250,8 +254,9 @@ int xkv_merge_stage2(const float* partial, const float* lse, void* out,
  * split of job j (whole splits first, each sequence's last - shorter - split after them).  With target_jobs = the number
  * of CUs, a stage 1 that runs one workgroup per CU gives every CU exactly one job and the jobs are as equal as the lengths
  * allow; a batch scanned in fixed-length splits ends on whatever the last workgroups happen to hold.  plan holds
- * 2 + 2 * batch * max_splits int32 (max_splits as passed to stage 1, >= ceil(kv_len / floor_tokens)).  Pass plan as
- * split_plan, and floor_tokens as split_cap_tokens, to xkv_latent_stage1 and xkv_merge_stage2 on the same stream.  One
+ * 2 + 2 * batch * max_splits int32 (max_splits as passed to stage 1, >= ceil(kv_len / floor_tokens)); packed (num_kv_splits
+ * == NULL, max_splits >= max(target_jobs, batch), XKV_EINVAL otherwise) 2 + 2 * max_splits + batch: behind the pairs of
+ * max_splits jobs plan[2 + 2 * max_splits + b], the jobs of the sequences before b.  Pass plan as split_plan, and floor_tokens as split_cap_tokens, to xkv_latent_stage1 and xkv_merge_stage2 on the same stream.  One
  * small workgroup; no host synchronisation.  No counterpart in the reference, whose batches have one length
  * (flash_decoding/gqa.py:60,194). */
 int xkv_plan_splits(const int32_t* kv_lens, const int32_t* num_kv_splits, int batch, int max_splits, int floor_tokens,

@@ -136,19 +136,32 @@ inline void same(Ten q, std::initializer_list<const at::Tensor*> ts) {   // same
   for (const at::Tensor* t : ts) need(t->is_cuda() && t->device() == q.device() && t->scalar_type() == q.scalar_type());
 }
 
-// Splits of one stage 1 + merge: a count for every sequence, or a plan on the device for a ragged batch.
-struct Splits { int S; int cap; const int32_t* lens; int32_t* plan; };
+// Splits of one stage 1 + merge: a count for every sequence, or a packed plan on the device for a ragged batch.  S: splits that a
+// sequence may have; n: what the C entry points take as max_splits (S, or the jobs of the plan).
+struct Splits {
+  int S, cap;
+  const int32_t* lens;
+  int32_t* plan;
+  int jobs = 0;
+  int n() const { return jobs ? jobs : S; }
+  int64_t rows(int64_t batch, int64_t hq) const { return hq * (jobs ? jobs : batch * S); }   // partial rows of the whole call
+};
 
 // A ragged batch: planned on the device so that it is cut into at most one job per workgroup the chip holds, no job shorter than
-// `floor` tokens or a 256th of the longest sequence (which bounds the workspaces).
-struct Ragged { int cap, S, jobs; int64_t at; };
-Ragged ragged(Call& c, int64_t batch, int groups, int64_t kv_len, int floor, int per_cu) {
-  Ragged r;
-  r.cap = std::max<int64_t>(floor, (cdiv(kv_len, 256) + 31) / 32 * 32);
-  r.S = cdiv(kv_len, r.cap);
-  r.jobs = std::max(1, per_cu * c.cus / groups);
-  r.at = c.plan((2 + 2 * batch * (int64_t)r.S) * 4);
-  return r;
+// `floor` tokens or a 256th of the longest sequence.  Its partial rows are packed: as many as there are jobs, or sequences, whatever the
+// lengths (64 sequences of up to 32K tokens, 32 heads, value rank 512: 17 MB; one row per sequence and possible split would be 1.07 GB).
+struct Ragged { int target; int64_t at; };
+Ragged ragged(Call& c, Splits& s, int64_t batch, int groups, int64_t kv_len, int floor, int per_cu) {
+  s.cap = std::max<int64_t>(floor, (cdiv(kv_len, 256) + 31) / 32 * 32);
+  s.S = cdiv(kv_len, s.cap);
+  const int target = std::max(1, per_cu * c.cus / groups);
+  s.jobs = std::max<int64_t>(target, batch);
+  return {target, c.plan((2 + 2 * (int64_t)s.jobs + batch) * 4)};
+}
+void write_plan(const Call& c, Splits& s, const Ragged& r, const at::Tensor& lens, int64_t batch) {
+  s.lens = lens.data_ptr<int32_t>();
+  s.plan = c.get<int32_t>(r.at);
+  check(p_xkv_plan_splits(s.lens, nullptr, batch, s.jobs, s.cap, r.target, s.plan, c.stream), "xkv_plan_splits");
 }
 
 // ---- merge (with or without the up-projection by vB [b, hkv, dv, d_out]) ------------------------------------------------
@@ -164,7 +177,7 @@ void merge(const Call& c, const float* partial, const float* lse, void* out, int
            int64_t rows_at, const Splits& s, int64_t batch, int64_t hq, int64_t kv_len, int64_t dv, float* lse_out = nullptr,
            int64_t sLb = 0, int64_t sLh = 0) {
   if (!up) {
-    check(p_xkv_merge_stage2(partial, lse, out, nullptr, 0, 0, 0, 0, XKV_BF16, nullptr, s.lens, batch, hq, hq, kv_len, s.S, s.cap,
+    check(p_xkv_merge_stage2(partial, lse, out, nullptr, 0, 0, 0, 0, XKV_BF16, nullptr, s.lens, batch, hq, hq, kv_len, s.n(), s.cap,
                              s.plan, dv, sOb, sOh, out_dtype, lse_out, sLb, sLh, c.stream), "xkv_merge_stage2");
     return;
   }
@@ -172,7 +185,7 @@ void merge(const Call& c, const float* partial, const float* lse, void* out, int
     float* mid = c.get<float>(rows_at);
     float* mid_lse = lse_out ? lse_out : mid + batch * hq * dv;
     if (!lse_out) { sLb = hq; sLh = 1; }
-    check(p_xkv_merge_stage2(partial, lse, mid, nullptr, 0, 0, 0, 0, XKV_BF16, nullptr, s.lens, batch, hq, hq, kv_len, s.S, s.cap,
+    check(p_xkv_merge_stage2(partial, lse, mid, nullptr, 0, 0, 0, 0, XKV_BF16, nullptr, s.lens, batch, hq, hq, kv_len, s.n(), s.cap,
                              s.plan, dv, hq * dv, dv, XKV_F32, mid_lse, sLb, sLh, c.stream), "xkv_merge_stage2");
     // a single row's log-sum-exp is not read
     check(p_xkv_merge_stage2(mid, mid_lse, out, up->p, up->sb, up->sh, up->sr, up->d_out, up->dtype, nullptr, nullptr, batch, hq, up->hkv,
@@ -180,7 +193,7 @@ void merge(const Call& c, const float* partial, const float* lse, void* out, int
     return;
   }
   check(p_xkv_merge_stage2(partial, lse, out, up->p, up->sb, up->sh, up->sr, up->d_out, up->dtype, nullptr, s.lens, batch, hq, up->hkv,
-                           kv_len, s.S, s.cap, s.plan, dv, sOb, sOh, out_dtype, lse_out, sLb, sLh, c.stream), "xkv_merge_stage2");
+                           kv_len, s.n(), s.cap, s.plan, dv, sOb, sOh, out_dtype, lse_out, sLb, sLh, c.stream), "xkv_merge_stage2");
 }
 
 Up up_of(Ten vB, int64_t hq, int dt) {
@@ -258,19 +271,15 @@ PyObject* nope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int groups = head_groups(hq), odt = code_any(o);
     Ragged rg{};
     Splits s{0, 0, nullptr, nullptr};
-    if (lens.defined()) { rg = ragged(c, b, groups, L, 128, ring_rank(r) ? 1 : 2); s.S = rg.S; s.cap = rg.cap; }
+    if (lens.defined()) rg = ragged(c, s, b, groups, L, 128, ring_rank(r) ? 1 : 2);
     else s.S = scan_splits(c, b, groups, L, ring_rank(r));
-    const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part = c.plan(b * hq * s.S * rv * 4), lse = c.plan(b * hq * s.S * 4);
+    const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
     const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
     c.alloc();
-    if (lens.defined()) {
-      s.lens = lens.data_ptr<int32_t>();
-      s.plan = c.get<int32_t>(rg.at);
-      check(p_xkv_plan_splits(s.lens, nullptr, b, s.S, s.cap, rg.jobs, s.plan, c.stream), "xkv_plan_splits");
-    }
+    if (lens.defined()) write_plan(c, s, rg, lens, b);
     absorb(c, q.data_ptr(), kB, c.get<void>(hi), c.get<void>(lo), b, hq, d, r);
     check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(kA, 0, r), NO_KV, kv(vA, 0, rv), c.get<float>(part),
-                              c.get<float>(lse), nullptr, 0, nullptr, s.lens, b, hq, groups, L, s.S, s.cap, s.plan, scale, 0.f, c.dt,
+                              c.get<float>(lse), nullptr, 0, nullptr, s.lens, b, hq, groups, L, s.n(), s.cap, s.plan, scale, 0.f, c.dt,
                               c.stream), "xkv_latent_stage1");
     merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, L, rv);
     return give(a[5]);
@@ -355,7 +364,7 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         s.lens = lens.data_ptr<int32_t>();
       }
       s.S = scan_splits(c, b, 1, L, true);
-      const int64_t sc = c.plan(b * hq * row * 4), part = c.plan(b * hq * s.S * rv * 4), lse = c.plan(b * hq * s.S * 4);
+      const int64_t sc = c.plan(b * hq * row * 4), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
       const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
       c.alloc();
       recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, recon_splits(c, kB, b, hkv, hq / hkv, L, r, true), b, hq, hkv, row,
@@ -366,7 +375,7 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       return give(a[5]);
     }
     s.S = recon_splits(c, kB, b, hkv, hq / hkv, L, r, false);
-    const int64_t part = c.plan(b * hq * s.S * rv * 4), lse = c.plan(b * hq * s.S * 4);
+    const int64_t part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
     const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
     c.alloc();
     recon(c, q, kA, kB, &vA, c.get<float>(part), c.get<float>(lse), nullptr, 0, s.S, b, hq, hkv, L, scale, invp, pos,
@@ -431,16 +440,12 @@ PyObject* gqa(PyObject*, PyObject* const* a, Py_ssize_t n) {
     need(floor > 0);
     Ragged rg{};
     Splits s{0, 0, nullptr, nullptr};
-    if (lens.defined()) { rg = ragged(c, b, groups, L, floor, per_cu); s.S = rg.S; s.cap = rg.cap; }
+    if (lens.defined()) rg = ragged(c, s, b, groups, L, floor, per_cu);
     else s.S = std::min(balanced_splits(b, groups, L, 32, per_cu, c.cus), cdiv(L, floor));
-    const int64_t part = c.plan(b * hq * s.S * dv * 4), lse = c.plan(b * hq * s.S * 4), bd = c.plan(wide4 ? b * hq * 512 * 2 : 0);
+    const int64_t part = c.plan(s.rows(b, hq) * dv * 4), lse = c.plan(s.rows(b, hq) * 4), bd = c.plan(wide4 ? b * hq * 512 * 2 : 0);
     const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, dv) ? rows_bytes(b, hq, dv) : 0);
     c.alloc();
-    if (lens.defined()) {
-      s.lens = lens.data_ptr<int32_t>();
-      s.plan = c.get<int32_t>(rg.at);
-      check(p_xkv_plan_splits(s.lens, nullptr, b, s.S, s.cap, rg.jobs, s.plan, c.stream), "xkv_plan_splits");
-    }
+    if (lens.defined()) write_plan(c, s, rg, lens, b);
     const void* qp = q.data_ptr();
     if (wide4) {
       check(p_xkv_blockdiag_q(qp, c.get<void>(bd), b, hq, hkv, d, c.dt, c.stream), "xkv_blockdiag_q");
@@ -448,7 +453,7 @@ PyObject* gqa(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     check(p_xkv_latent_stage1({qp, wide4 ? 512 : (int)d}, nullptr, NO_Q, wide4 ? kv(k, 0, 512) : kv(k, k.stride(2), d), NO_KV,
                               kv(v, fact ? 0 : v.stride(2), dv), c.get<float>(part), c.get<float>(lse), nullptr, 0, nullptr, s.lens, b, hq,
-                              wide4 ? 1 : hkv, L, s.S, s.cap, s.plan, scale, 0.f, c.dt, c.stream), "xkv_latent_stage1");
+                              wide4 ? 1 : hkv, L, s.n(), s.cap, s.plan, scale, 0.f, c.dt, c.stream), "xkv_latent_stage1");
     merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, fact ? &up : nullptr, mid, s, b, hq, L, dv);
     return give(a[4]);
   });
@@ -478,7 +483,7 @@ PyObject* mla(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int groups = head_groups(hq);
     Splits s{scan_splits(c, b, groups, L, e == 64 && (r == 512 || (fact && ring_rank(r)))), 0, nullptr, nullptr};
     const int64_t hi = c.plan(fact ? b * hq * r * 2 : 0), lo = c.plan(fact ? b * hq * r * 2 : 0);
-    const int64_t part = c.plan(b * hq * s.S * r * 4), lse = c.plan(b * hq * s.S * 4);
+    const int64_t part = c.plan(s.rows(b, hq) * r * 4), lse = c.plan(s.rows(b, hq) * 4);
     const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, r) ? rows_bytes(b, hq, r) : 0);
     c.alloc();
     at::Tensor o = at::empty({b, hq, w}, c.opts);

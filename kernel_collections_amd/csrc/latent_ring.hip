@@ -157,8 +157,9 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
     split = p.split_plan[3 + 2 * job];
   }
   const int L = p.kv_lens ? p.kv_lens[b] : p.kv_len;
+  const int ns = effective_splits(L, asked_splits(p.num_splits, b, p.max_splits, p.split_cap), split_cap_in_force(p.split_cap, p.split_plan));
   int start, end;
-  split_bounds(L, effective_splits(L, asked_splits(p.num_splits, b, p.max_splits, p.split_cap), split_cap_in_force(p.split_cap, p.split_plan)), split, start, end);
+  split_bounds(L, ns, split, start, end);
   if (end <= start) return;
   const int hg = p.hq / p.groups, h0 = group * hg;
   const int ntiles = (end - start + TN - 1) / TN;
@@ -547,6 +548,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   if (SCORES) return;
 
   // ---- epilogue: normalise, write partial + lse --------------------------------------------------------------------
+  const PartialRows rows = partial_rows(b, p.hq, p.max_splits, [&] { return live_splits(L, ns, p.max_splits); }, p.num_splits, p.split_plan);
   if (ssub == 0) { ml_lds[2 * srow] = m_run; ml_lds[2 * srow + 1] = l_run; }
   __syncthreads();
   if (VHEADS) {
@@ -556,7 +558,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
       if (n16 < hpk) {
         const float m = ml_lds[2 * hrow], l = ml_lds[2 * hrow + 1];
         const float inv = 1.f / l;
-        const int64_t ph = ((int64_t)b * p.hq + hrow) * p.max_splits + split;
+        const int64_t ph = rows.base + (int64_t)hrow * rows.per_head + split;
         float* dst = p.partial + ph * RING_DVH + 4 * g4;
 #pragma unroll
         for (int mb = 0; mb < NVB; ++mb) *reinterpret_cast<f32x4*>(dst + mb * 16) = acc[mb][j] * inv;
@@ -571,7 +573,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
     if (hrow < hg) {
       const float m = ml_lds[2 * hrow], l = ml_lds[2 * hrow + 1];
       const float inv = 1.f / l;
-      const int64_t ph = ((int64_t)b * p.hq + h0 + hrow) * p.max_splits + split;
+      const int64_t ph = rows.base + (int64_t)(h0 + hrow) * rows.per_head + split;
       float* dst = p.partial + ph * DV + vcol0 + 4 * g4;
 #pragma unroll
       for (int mb = 0; mb < NVB; ++mb) *reinterpret_cast<f32x4*>(dst + mb * 16) = acc[mb][hb] * inv;
@@ -581,14 +583,13 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
 }
 
 template <typename T, int TN, int NHB, bool LO, int DN, bool HAS_R, int VMODE, int DVW = 512>
-static int launch_ring_t(const RingParams& p, int batch, hipStream_t st) {
+static int launch_ring_t(const RingParams& p, hipStream_t st) {
   constexpr int SHM = RingShape<TN, DN, HAS_R, VMODE, NHB, DVW>::shm(LO);
   auto kern = latent_ring_kernel<T, TN, NHB, LO, DN, HAS_R, VMODE, DVW>;
   static DynLds lds;
   const int e = ensure_dynamic_lds(lds, reinterpret_cast<const void*>(kern), SHM, true);
   if (e != XKV_OK) return e;
-  const int total = batch * p.groups * p.max_splits;
-  kern<<<dim3(xcd_grid(total, p.groups)), dim3(512), SHM, st>>>(p);
+  kern<<<dim3(xcd_grid(p.total_wg, p.groups)), dim3(512), SHM, st>>>(p);
   return launch_status();
 }
 
@@ -613,35 +614,35 @@ static int ring_vmode(const RingParams& p, bool vshared) {
 
 // softmax + P.V over given scores: the value rows are the C stream
 template <typename T>
-static int launch_ring_given_dt(const RingParams& p, int batch, hipStream_t st) {
+static int launch_ring_given_dt(const RingParams& p, hipStream_t st) {
   const int nhb = p.hq <= 16 ? 1 : 2;
 #define XKV_RING_GIVEN(NHB, DN) \
-  if (nhb == NHB && p.dn == DN) return launch_ring_t<T, 32, NHB, false, DN, false, RING_VGIVEN>(p, batch, st);
+  if (nhb == NHB && p.dn == DN) return launch_ring_t<T, 32, NHB, false, DN, false, RING_VGIVEN>(p, st);
   XKV_RING_GIVEN(1, 512) XKV_RING_GIVEN(2, 512) XKV_RING_GIVEN(1, 384) XKV_RING_GIVEN(2, 384) XKV_RING_GIVEN(1, 256) XKV_RING_GIVEN(2, 256)
 #undef XKV_RING_GIVEN
   return XKV_EUNSUPPORTED;
 }
 
 template <typename T>
-static int launch_ring_dt(const RingParams& p, int batch, bool vshared, hipStream_t st) {
+static int launch_ring_dt(const RingParams& p, bool vshared, hipStream_t st) {
   const int hg = p.hq / p.groups, vm = ring_vmode(p, vshared);
   const bool lo = p.qn_lo != nullptr, r = p.R != nullptr;
   if (vm == RING_VHEADS) {
     RingParams a = p;
     a.groups = 1;
-    a.total_wg = batch * p.max_splits;
+    a.total_wg = p.total_wg / p.groups;
 #define XKV_RING_VH(NHB, DN) \
-  if (lo && (p.hq <= 16 ? 1 : 2) == NHB && p.dn == DN) return launch_ring_t<T, 16, NHB, true, DN, false, RING_VHEADS, 1024>(a, batch, st);
+  if (lo && (p.hq <= 16 ? 1 : 2) == NHB && p.dn == DN) return launch_ring_t<T, 16, NHB, true, DN, false, RING_VHEADS, 1024>(a, st);
     XKV_RING_VH(1, 512) XKV_RING_VH(2, 512) XKV_RING_VH(1, 384) XKV_RING_VH(2, 384) XKV_RING_VH(1, 256) XKV_RING_VH(2, 256)
 #undef XKV_RING_VH
     if (p.dn == 1024 && !lo)
-      return p.hq <= 16 ? launch_ring_t<T, 16, 1, false, 1024, false, RING_VHEADS, 1024>(a, batch, st)
-                        : launch_ring_t<T, 16, 2, false, 1024, false, RING_VHEADS, 1024>(a, batch, st);
+      return p.hq <= 16 ? launch_ring_t<T, 16, 1, false, 1024, false, RING_VHEADS, 1024>(a, st)
+                        : launch_ring_t<T, 16, 2, false, 1024, false, RING_VHEADS, 1024>(a, st);
     return XKV_EUNSUPPORTED;
   }
   const int nhb = hg <= 16 ? 1 : 2;
 #define XKV_RING_CASE(TN, NHB, LO, DN, HAS_R, VM) \
-  if (nhb == NHB && lo == LO && p.dn == DN && r == HAS_R && vm == VM) return launch_ring_t<T, TN, NHB, LO, DN, HAS_R, VM>(p, batch, st);
+  if (nhb == NHB && lo == LO && p.dn == DN && r == HAS_R && vm == VM) return launch_ring_t<T, TN, NHB, LO, DN, HAS_R, VM>(p, st);
   // 512-wide rows, one stream: scores (absorbed q carries a low part or not), shared-tile decode (+ RoPE keys)
   XKV_RING_CASE(32, 1, true, 512, false, RING_SCORES)    XKV_RING_CASE(32, 2, true, 512, false, RING_SCORES)
   XKV_RING_CASE(32, 1, false, 512, false, RING_SCORES)   XKV_RING_CASE(32, 2, false, 512, false, RING_SCORES)
@@ -658,7 +659,7 @@ static int launch_ring_dt(const RingParams& p, int batch, bool vshared, hipStrea
   // us with 16-token tiles, 61 with 32), 16-token ones from there on (512 + 512: 85 us against 88.5)
 #define XKV_RING_V2(NHB, LO, DN, DVW) \
   if (nhb == NHB && lo == LO && p.dn == DN && !r && vm == RING_VDISTINCT && p.dv == DVW) \
-    return launch_ring_t<T, DN + DVW >= 1024 ? 16 : 32, NHB, LO, DN, false, RING_VDISTINCT, DVW>(p, batch, st);
+    return launch_ring_t<T, DN + DVW >= 1024 ? 16 : 32, NHB, LO, DN, false, RING_VDISTINCT, DVW>(p, st);
 #define XKV_RING_V2_ALL(LO, DN) \
   XKV_RING_V2(1, LO, DN, 512) XKV_RING_V2(2, LO, DN, 512) XKV_RING_V2(1, LO, DN, 384) XKV_RING_V2(2, LO, DN, 384) \
   XKV_RING_V2(1, LO, DN, 256) XKV_RING_V2(2, LO, DN, 256)
@@ -690,12 +691,12 @@ bool ring_eligible(const RingParams& p, bool vshared) {
   return true;
 }
 
-int launch_ring_given(const RingParams& p, int batch, int dtype, hipStream_t st) {
-  return dtype == XKV_BF16 ? launch_ring_given_dt<__bf16>(p, batch, st) : launch_ring_given_dt<_Float16>(p, batch, st);
+int launch_ring_given(const RingParams& p, int dtype, hipStream_t st) {
+  return dtype == XKV_BF16 ? launch_ring_given_dt<__bf16>(p, st) : launch_ring_given_dt<_Float16>(p, st);
 }
 
-int launch_ring(const RingParams& p, int batch, bool vshared, int dtype, hipStream_t st) {
-  return dtype == XKV_BF16 ? launch_ring_dt<__bf16>(p, batch, vshared, st) : launch_ring_dt<_Float16>(p, batch, vshared, st);
+int launch_ring(const RingParams& p, bool vshared, int dtype, hipStream_t st) {
+  return dtype == XKV_BF16 ? launch_ring_dt<__bf16>(p, vshared, st) : launch_ring_dt<_Float16>(p, vshared, st);
 }
 
 }  // namespace xkv

@@ -60,8 +60,9 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
   }
 
   const int L = p.kv_lens ? p.kv_lens[b] : p.kv_len;
+  const int ns = effective_splits(L, asked_splits(p.num_splits, b, p.max_splits, p.split_cap), split_cap_in_force(p.split_cap, p.split_plan));
   int start, end;
-  split_bounds(L, effective_splits(L, asked_splits(p.num_splits, b, p.max_splits, p.split_cap), split_cap_in_force(p.split_cap, p.split_plan)), split, start, end);
+  split_bounds(L, ns, split, start, end);
   if (end <= start) return;
 
   const int hg = p.hq / p.groups;  // heads of this kv group
@@ -299,6 +300,7 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
   if (SCORES_ONLY) return;
 
   // ---- epilogue: normalise, write partial + lse --------------------------------------------
+  const PartialRows rows = partial_rows(b, p.hq, p.max_splits, [&] { return live_splits(L, ns, p.max_splits); }, p.num_splits, p.split_plan);
   if (ssub == 0) { ml_lds[2 * srow] = m_run; ml_lds[2 * srow + 1] = l_run; }
   __syncthreads();
 #pragma unroll
@@ -307,7 +309,7 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
     if (hrow < hg) {
       const float m = ml_lds[2 * hrow], l = ml_lds[2 * hrow + 1];
       const float inv = 1.f / l;
-      const int64_t ph = ((int64_t)b * p.hq + h0 + hrow) * p.max_splits + split;
+      const int64_t ph = rows.base + (int64_t)(h0 + hrow) * rows.per_head + split;
       float* dst = p.partial + ph * p.dv + vcol0 + 4 * g4;
 #pragma unroll
       for (int mb = 0; mb < NVB_MAX; ++mb)
@@ -321,7 +323,7 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
 // host side
 // ------------------------------------------------------------------------------------------
 template <typename T, int NHB, int TN, int NVB_MAX, int NPK_C, int NPK_R, int NPK_V, bool VSHARED, bool SCORES_ONLY>
-static int launch_latent(const LatentParams& p, int batch, hipStream_t st) {
+static int launch_latent(const LatentParams& p, hipStream_t st) {
   constexpr int HB = 16 * NHB;
   const int dtot = p.dn + p.dr, ldc = dtot + 8, ldv = VSHARED ? ldc : p.dv + 8;
   // operands must fit the per-thread packet plan of this instantiation
@@ -338,19 +340,18 @@ static int launch_latent(const LatentParams& p, int batch, hipStream_t st) {
   static DynLds lds;
   const int e = ensure_dynamic_lds(lds, reinterpret_cast<const void*>(kern), (int)shm);
   if (e != XKV_OK) return e;
-  const int total = batch * p.groups * p.max_splits;
-  const int grid = xcd_grid(total, p.groups);
+  const int grid = xcd_grid(p.total_wg, p.groups);
   kern<<<dim3(grid), dim3(256), shm, st>>>(p);
   return launch_status();
 }
 
 template <typename T, int NHB>
-static int dispatch_latent(const LatentParams& p, int batch, bool vshared, hipStream_t st) {
-  if (p.scores) return launch_latent<T, NHB, 64, 1, 16, 4, 0, true, true>(p, batch, st);
-  if (vshared) return launch_latent<T, NHB, 64, 8, 16, 4, 0, true, false>(p, batch, st);
+static int dispatch_latent(const LatentParams& p, bool vshared, hipStream_t st) {
+  if (p.scores) return launch_latent<T, NHB, 64, 1, 16, 4, 0, true, true>(p, st);
+  if (vshared) return launch_latent<T, NHB, 64, 8, 16, 4, 0, true, false>(p, st);
   // distinct V: small operands (plain GQA heads) keep 64-token tiles, wide ones drop to 32
-  if (p.dn <= 256 && p.dr == 0 && p.dv <= 128) return launch_latent<T, NHB, 64, 2, 8, 0, 4, false, false>(p, batch, st);
-  return launch_latent<T, NHB, 32, 8, 16, 2, 8, false, false>(p, batch, st);
+  if (p.dn <= 256 && p.dr == 0 && p.dv <= 128) return launch_latent<T, NHB, 64, 2, 8, 0, 4, false, false>(p, st);
+  return launch_latent<T, NHB, 32, 8, 16, 2, 8, false, false>(p, st);
 }
 
 }  // namespace xkv
@@ -370,9 +371,7 @@ extern "C" int xkv_latent_stage1(xkv_q_operand qn, const void* qn_lo, xkv_q_oper
   if (!qn.ptr || !C.ptr || batch <= 0 || hq <= 0 || n_kv_groups <= 0 || kv_len <= 0 ||
       max_splits <= 0)
     return XKV_EINVAL;
-  // with a cap the longest sequence may need cdiv(kv_len, cap) splits: the workspace must have a row for each
-  if (split_cap_tokens < 0 || (split_cap_tokens > 0 && max_splits < cdiv(kv_len, split_cap_tokens))) return XKV_EINVAL;
-  if (split_plan && split_cap_tokens <= 0) return XKV_EINVAL;   // the host value is what bounds the workspaces
+  if (!cap_fits(num_kv_splits, batch, kv_len, max_splits, split_cap_tokens, split_plan)) return XKV_EINVAL;
   const bool scores_only = scores_out != nullptr;
   if (!scores_only && (!V.ptr || !partial || !lse)) return XKV_EINVAL;
   if (dtype != XKV_BF16 && dtype != XKV_F16) return XKV_EDTYPE;
@@ -404,7 +403,7 @@ extern "C" int xkv_latent_stage1(xkv_q_operand qn, const void* qn_lo, xkv_q_oper
   p.num_splits = num_kv_splits; p.kv_lens = kv_lens;
   p.hq = hq; p.groups = n_kv_groups; p.kv_len = kv_len; p.max_splits = max_splits; p.split_cap = split_cap_tokens;
   p.split_plan = split_plan;
-  p.total_wg = batch * n_kv_groups * max_splits;
+  p.total_wg = (packed_rows(num_kv_splits, split_plan) ? 1 : batch) * n_kv_groups * max_splits;
   p.sm_scale = sm_scale; p.logit_cap = logit_cap;
   p.heads_in_row = 0;
   const bool vshared = !scores_only && V.ptr == C.ptr && V.stride_b == C.stride_b && V.stride_l == C.stride_l &&
@@ -421,14 +420,14 @@ extern "C" int xkv_latent_stage1(xkv_q_operand qn, const void* qn_lo, xkv_q_oper
     if (v_heads || v_shared_row) {
       LatentParams w = p;
       w.dn = 1024; w.sCh = 0; w.heads_in_row = 8;
-      if (v_shared_row) { w.groups = 1; w.total_wg = batch * max_splits; }
-      if (ring_eligible(w, false)) return launch_ring(w, batch, false, dtype, st);
+      if (v_shared_row) { w.groups = 1; w.total_wg = p.total_wg / n_kv_groups; }
+      if (ring_eligible(w, false)) return launch_ring(w, false, dtype, st);
     }
   }
-  if (ring_eligible(p, vshared)) return launch_ring(p, batch, vshared, dtype, st);
+  if (ring_eligible(p, vshared)) return launch_ring(p, vshared, dtype, st);
   if (dtype == XKV_BF16)
-    return hg <= 16 ? dispatch_latent<__bf16, 1>(p, batch, vshared, st) : dispatch_latent<__bf16, 2>(p, batch, vshared, st);
-  return hg <= 16 ? dispatch_latent<_Float16, 1>(p, batch, vshared, st) : dispatch_latent<_Float16, 2>(p, batch, vshared, st);
+    return hg <= 16 ? dispatch_latent<__bf16, 1>(p, vshared, st) : dispatch_latent<__bf16, 2>(p, vshared, st);
+  return hg <= 16 ? dispatch_latent<_Float16, 1>(p, vshared, st) : dispatch_latent<_Float16, 2>(p, vshared, st);
 }
 
 extern "C" int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, float* partial, float* lse,
@@ -436,8 +435,7 @@ extern "C" int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, floa
                                      int max_splits, int split_cap_tokens, const int32_t* split_plan, int dtype, void* stream) {
   if (!scores || !V.ptr || !partial || !lse || batch <= 0 || hq <= 0 || kv_len <= 0 || max_splits <= 0)
     return XKV_EINVAL;
-  if (split_cap_tokens < 0 || (split_cap_tokens > 0 && max_splits < cdiv(kv_len, split_cap_tokens))) return XKV_EINVAL;
-  if (split_plan && split_cap_tokens <= 0) return XKV_EINVAL;
+  if (!cap_fits(num_kv_splits, batch, kv_len, max_splits, split_cap_tokens, split_plan)) return XKV_EINVAL;
   if (dtype != XKV_BF16 && dtype != XKV_F16) return XKV_EDTYPE;
   if (hq > 32 || (V.dim != 512 && V.dim != 384 && V.dim != 256) || V.stride_h != 0 || V.stride_l < V.dim || (kv_len & 3))
     return XKV_EUNSUPPORTED;
@@ -453,8 +451,8 @@ extern "C" int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, floa
   p.num_splits = num_kv_splits; p.kv_lens = kv_lens;
   p.hq = hq; p.groups = 1; p.kv_len = kv_len; p.max_splits = max_splits; p.split_cap = split_cap_tokens;
   p.split_plan = split_plan;
-  p.total_wg = batch * max_splits;
+  p.total_wg = packed_rows(num_kv_splits, split_plan) ? max_splits : batch * max_splits;
   p.sm_scale = 1.f; p.logit_cap = 0.f;
   p.heads_in_row = 0;
-  return launch_ring_given(p, batch, dtype, (hipStream_t)stream);
+  return launch_ring_given(p, dtype, (hipStream_t)stream);
 }

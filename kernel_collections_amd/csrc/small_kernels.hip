@@ -1,4 +1,5 @@
 // RoPE table, query absorption and the stage-2 merge: the small kernels around the scans.
+#include <algorithm>
 #include <type_traits>
 
 #include "xkv_common.h"
@@ -179,12 +180,6 @@ __global__ __launch_bounds__(256) void blockdiag_q_kernel(const T* __restrict__ 
 // dependent round trips, so each starts everything it can at once: the lse words and the partial rows of a thread's splits
 // are loaded together and folded with a running maximum, instead of weights first and rows after.
 // ----------------------------------------------------------------------------------------------
-__device__ __forceinline__ int merge_live_splits(int L, int ns, int max_splits) {
-  const int per = ns > 0 ? cdiv(cdiv(L, ns), MIN_BLOCK_KV) * MIN_BLOCK_KV : 0;
-  const int live = per > 0 ? cdiv(L, per) : 0;
-  return live < max_splits ? live : max_splits;
-}
-
 // A thread's share of one head's splits: i = first, first + step, ... < nlive, P consecutive features at pp.  Eight splits'
 // loads in flight; acc = sum exp(lse_i - m) * partial_i, l = sum exp(lse_i - m), m the running maximum (NEG_INF: no split).
 template <int P> struct MergeAcc { float m, l, acc[P]; };
@@ -248,11 +243,12 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(
   __shared__ float red[256 * P], ml[256][2];
   const int h = blockIdx.x, b = blockIdx.y, c0 = blockIdx.z * chunk;
   const int L = kv_lens ? kv_lens[b] : kv_len;
-  const int nlive = merge_live_splits(L, effective_splits(L, asked_splits(num_kv_splits, b, max_splits, split_cap), split_cap_in_force(split_cap, split_plan)), max_splits);
+  const int nlive = live_splits(L, effective_splits(L, asked_splits(num_kv_splits, b, max_splits, split_cap), split_cap_in_force(split_cap, split_plan)), max_splits);
   const int lanes = chunk / P, ngrp = 256 / lanes;          // lanes <= 256
   const int sg = threadIdx.x / lanes, c = c0 + (threadIdx.x % lanes) * P;
   const bool mine = sg < ngrp && c < dv;
-  const int64_t row = ((int64_t)b * hq + h) * max_splits;
+  const PartialRows rows = partial_rows(b, hq, max_splits, [&] { return nlive; }, num_kv_splits, split_plan);
+  const int64_t row = rows.base + (int64_t)h * rows.per_head;
   MergeAcc<P> a;
   if (mine) {
     a = merge_fold<P>(lse + row, partial + row * dv + c, dv, sg, ngrp, nlive);
@@ -313,10 +309,11 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     if (cols && grp + 64 * r < dv) w[r] = ld16<vec8>(Bh + (int64_t)(grp + 64 * r) * sVr);
   }
   const int L = kv_lens ? kv_lens[b] : kv_len;
-  const int nlive = merge_live_splits(L, effective_splits(L, asked_splits(num_kv_splits, b, max_splits, split_cap), split_cap_in_force(split_cap, split_plan)), max_splits);
+  const int nlive = live_splits(L, effective_splits(L, asked_splits(num_kv_splits, b, max_splits, split_cap), split_cap_in_force(split_cap, split_plan)), max_splits);
+  const PartialRows rows = partial_rows(b, hq, max_splits, [&] { return nlive; }, num_kv_splits, split_plan);
   auto merge_packet = [&](int gi, int c, auto tag) {
     constexpr int P = decltype(tag)::value;
-    const int64_t row = ((int64_t)b * hq + hfirst + gi) * max_splits;
+    const int64_t row = rows.base + (int64_t)(hfirst + gi) * rows.per_head;
     // a single row's weight is 1 whatever its log-sum-exp
     const MergeAcc<P> a = merge_fold<P>(max_splits == 1 && !lse_out ? nullptr : lse + row, partial + row * dv + c, dv, 0, 1, nlive);
     const float inv = nlive > 0 ? 1.f / a.l : 0.f;
@@ -387,15 +384,17 @@ static int launch_merge(const float* partial, const float* lse, void* out, const
                         int64_t sVr, int d_out, const int32_t* ns, const int32_t* kl, int batch, int hq, int hkv,
                         int kv_len, int max_splits, int dv, int64_t sOb, int64_t sOh, float* lse_out, int64_t sLb, int64_t sLh,
                         int split_cap, const int32_t* split_plan, hipStream_t st) {
+  // splits one sequence may have (a packed plan's max_splits counts the jobs of the whole batch)
+  const int seq_splits = packed_rows(ns, split_plan) ? std::min(max_splits, cdiv(kv_len, split_cap)) : max_splits;
   // what one head takes of the LDS was bounded when the weights of all its splits were held there; the bound stays part of the
   // interface (a split count this large is refused before any launch)
-  if ((size_t)(dv + max_splits) * sizeof(float) > 24 * 1024) return XKV_EUNSUPPORTED;
+  if ((size_t)(dv + seq_splits) * sizeof(float) > 24 * 1024) return XKV_EUNSUPPORTED;
   if (!vB) {
     // few splits: a head's whole row per workgroup; more: narrower feature blocks, so that a thread folds few splits, until the
     // grid fills the chip four times over
     const bool vec = dv % 4 == 0 && (reinterpret_cast<uintptr_t>(partial) & 15) == 0;
     int chunk = vec ? 1024 : 256;
-    while (chunk / 2 >= dv || (chunk > 64 && (int64_t)max_splits * chunk > (vec ? 8192 : 2048) &&
+    while (chunk / 2 >= dv || (chunk > 64 && (int64_t)seq_splits * chunk > (vec ? 8192 : 2048) &&
                                (int64_t)hq * batch * cdiv(dv, chunk) < 1024))
       chunk /= 2;
     const dim3 grid(hq, batch, cdiv(dv, chunk));
@@ -564,6 +563,8 @@ __global__ __launch_bounds__(PLAN_T) void plan_splits_kernel(const int32_t* __re
       plan[2 + 2 * (whole + last + i1 - 1)] = b;
       plan[3 + 2 * (whole + last + i1 - 1)] = live - 1;
     }
+    // a packed plan: the partial rows of the sequences lie behind each other
+    if (!num_splits && b < batch) plan[2 + 2 * (int64_t)max_splits + b] = done + last + (i0 - m0) + (i1 - m1);
     done += all0;
     last += all1;
   }
@@ -577,6 +578,8 @@ using namespace xkv;
 extern "C" int xkv_plan_splits(const int32_t* kv_lens, const int32_t* num_kv_splits, int batch, int max_splits, int floor_tokens,
                                int target_jobs, int32_t* plan, void* stream) {
   if (!kv_lens || !plan || batch <= 0 || max_splits <= 0 || floor_tokens <= 0 || target_jobs <= 0) return XKV_EINVAL;
+  // without an array of counts the caps alone make the jobs: at most target_jobs, or one a sequence
+  if (!num_kv_splits && max_splits < std::max(batch, target_jobs)) return XKV_EINVAL;
   plan_splits_kernel<<<dim3(1), dim3(PLAN_T), 0, (hipStream_t)stream>>>(kv_lens, num_kv_splits, batch, max_splits, floor_tokens,
                                                                      target_jobs, plan);
   return launch_status();
@@ -683,8 +686,7 @@ extern "C" int xkv_merge_stage2(const float* partial, const float* lse, void* ou
                                 int64_t sLb, int64_t sLh, void* stream) {
   if (!partial || !lse || !out || batch <= 0 || hq <= 0 || hkv <= 0 || max_splits <= 0 || dv <= 0)
     return XKV_EINVAL;
-  if (split_cap_tokens < 0 || (split_cap_tokens > 0 && (kv_len <= 0 || max_splits < cdiv(kv_len, split_cap_tokens)))) return XKV_EINVAL;
-  if (split_plan && split_cap_tokens <= 0) return XKV_EINVAL;
+  if (!cap_fits(ns, batch, kv_len, max_splits, split_cap_tokens, split_plan)) return XKV_EINVAL;
   if (hq % hkv || hq / hkv > 32 || dv > 512) return XKV_EUNSUPPORTED;
   if (vB && (d_out <= 0 || d_out > 512 || d_out % 8)) return XKV_EUNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;

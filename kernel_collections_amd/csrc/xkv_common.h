@@ -99,6 +99,32 @@ __device__ __forceinline__ int split_cap_in_force(int cap_tokens, const int32_t*
   return d > cap_tokens ? d : cap_tokens;
 }
 
+// Splits of a sequence that hold tokens when it is cut into ns: a prefix of the split range.
+__device__ __forceinline__ int live_splits(int L, int ns, int max_splits) {
+  const int per = ns > 0 ? cdiv(cdiv(L, ns), MIN_BLOCK_KV) * MIN_BLOCK_KV : 0;
+  const int live = per > 0 ? cdiv(L, per) : 0;
+  return live < max_splits ? live : max_splits;
+}
+
+// Where the partial rows of sequence b lie: row (h, split) is base + h * per_head + split.  [batch, hq, max_splits] as a rule.
+// With a plan and no array of counts (a packed plan) the sequences lie behind each other, hq * live rows each, max_splits counts
+// the jobs of the whole batch, and the plan holds every sequence's first job behind its job list: a ragged batch then needs
+// rows for the jobs it is cut into, not for as many splits of every sequence as the longest one might get.
+__host__ __device__ __forceinline__ bool packed_rows(const int32_t* num_splits, const int32_t* plan) { return plan && !num_splits; }
+// A call's cap and plan as stage 1 and the merge accept them: with a cap the longest sequence may need cdiv(kv_len, cap) splits, and the
+// workspace must have a row for each; a plan needs the host's cap, and a packed one a job for every sequence.
+inline bool cap_fits(const int32_t* num_splits, int batch, int kv_len, int max_splits, int cap, const int32_t* plan) {
+  if (cap < 0 || (plan && cap == 0)) return false;
+  if (packed_rows(num_splits, plan)) return kv_len > 0 && max_splits >= batch;
+  return cap == 0 || (kv_len > 0 && max_splits >= cdiv(kv_len, cap));
+}
+struct PartialRows { int64_t base; int per_head; };
+template <typename Live>   // live(): the sequence's live splits, evaluated only where rows are packed
+__device__ __forceinline__ PartialRows partial_rows(int b, int hq, int max_splits, Live live, const int32_t* num_splits, const int32_t* plan) {
+  if (__builtin_expect(packed_rows(num_splits, plan), 0)) return {(int64_t)plan[2 + 2 * (int64_t)max_splits + b] * hq, live()};
+  return {(int64_t)b * hq * max_splits, max_splits};
+}
+
 // Reductions over the 4 lane groups {n, n+16, n+32, n+48} that share a column
 // index in the 16x16 MFMA result layout.
 __device__ __forceinline__ float group4_max(float v) {

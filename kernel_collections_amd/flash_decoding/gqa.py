@@ -74,7 +74,7 @@ def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits,
     wide = (hkv * d == 1024 and d == 128 and hq <= 32 and k_buffer.stride(2) == d and v_buffer.stride(2) == d
             and k_buffer.stride(1) >= 1024 and v_buffer.stride(1) >= 1024)
     splits, cap, S, plan = _plan(wide, lens, splits, S, batch, hkv, kv_len)
-    partial, lse = ops.workspaces(batch, hq, S, dv, q.device)
+    partial, lse = ops.workspaces(batch, hq, S, dv, q.device, plan)
     ops.latent_stage1(q3, None, None,
                       (k_buffer, k_buffer.stride(0), k_buffer.stride(1), k_buffer.stride(2), d), None,
                       (v_buffer, v_buffer.stride(0), v_buffer.stride(1), v_buffer.stride(2), dv),
@@ -105,7 +105,7 @@ def decode_attention_fwd_v_factorized(q, k_buffer, v_A_buffer, v_B_buffer, o, nu
     # 512-wide token rows (4 x 128, 2 x 256 ...): the same form, with the block-diagonal query built here
     wide4 = hkv * d == 512 and rv == 512 and hq <= 32 and k_buffer.stride(2) == d
     splits, cap, S, plan = _plan(wide8 or wide4, lens, splits, S, batch, hkv, kv_len)
-    partial, lse = ops.workspaces(batch, hq, S, rv, q.device)
+    partial, lse = ops.workspaces(batch, hq, S, rv, q.device, plan)
     if wide4:
         ops.latent_stage1(ops.blockdiag_q(q3, hkv), None, None,
                           (k_buffer, k_buffer.stride(0), k_buffer.stride(1), 0, hkv * d), None,

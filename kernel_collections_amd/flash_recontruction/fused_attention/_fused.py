@@ -58,7 +58,7 @@ def decode_nope(q, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale
     qt_hi, qt_lo = ops.absorb_q(q3, k_B, want_lo=True)
     groups = ops.head_groups(hq)
     splits, cap, S, plan = _plan(lens, batch, groups, kv_len, k_A.shape[-1], q.device)
-    partial, lse = ops.workspaces(batch, hq, S, rank_v, q.device)
+    partial, lse = ops.workspaces(batch, hq, S, rank_v, q.device, plan)
     ops.latent_stage1(qt_hi, qt_lo, None, (k_A, k_A.stride(0), k_A.stride(1), 0, k_A.shape[-1]), None,
                       (v_A, v_A.stride(0), v_A.stride(1), 0, rank_v), partial, lse, None, splits, lens,
                       batch, hq, groups, kv_len, S, float(sm_scale), split_cap=cap, split_plan=plan)
@@ -81,7 +81,7 @@ def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_sca
     # 8 heads of 128 under ranks 256 / 384 / 512: one workgroup serves every kv head of a split
     wide = hkv == 8 and dv == 128 and hq <= 32 and k_A.shape[-1] in (256, 384, 512) and v_buffer.stride(2) == dv
     splits, cap, S, plan = _plan(lens, batch, 1 if wide else hkv, kv_len, 512 if wide else k_A.shape[-1], q.device)
-    partial, lse = ops.workspaces(batch, hq, S, dv, q.device)
+    partial, lse = ops.workspaces(batch, hq, S, dv, q.device, plan)
     ops.latent_stage1(qt_hi, qt_lo, None, (k_A, k_A.stride(0), k_A.stride(1), 0, k_A.shape[-1]), None,
                       (v_buffer, v_buffer.stride(0), v_buffer.stride(1), v_buffer.stride(2), dv),
                       partial, lse, None, splits, lens, batch, hq, hkv, kv_len, S, float(sm_scale), split_cap=cap, split_plan=plan)

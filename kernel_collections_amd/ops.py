@@ -228,7 +228,8 @@ def merge_stage2(partial, lse, out, vB, num_kv_splits, kv_lens, batch, hq, hkv, 
     """out `[b,Hq,*]` (strides honoured on the first two axes).  `lse_out` `[b,Hq]` (any strides, fp32): log-sum-exp
     of the merged range.  Up-projections wider than 512 columns run as column blocks of 512."""
     dv = partial.shape[-1]
-    if vB is not None and max_splits > 1 and max_splits * (hq // hkv) * dv > MERGE_ROWS_FLOATS:
+    seq_splits = max_splits if split_plan is None or num_kv_splits is not None else _cdiv(kv_len, split_cap)
+    if vB is not None and seq_splits > 1 and seq_splits * (hq // hkv) * dv > MERGE_ROWS_FLOATS:
         # many splits: merge the rows first, spread over the chip, then up-project one row per head.  The up-projecting kernel
         # repeats the merge in every block of 64 columns, which costs more than a second launch once that is
         # MERGE_ROWS_FLOATS partial values per workgroup.
@@ -262,12 +263,15 @@ def merge_stage2(partial, lse, out, vB, num_kv_splits, kv_lens, batch, hq, hkv, 
     return out
 
 
-def plan_splits(kv_lens: torch.Tensor, num_kv_splits: torch.Tensor, max_splits: int, floor_tokens: int, target_jobs: int):
+def plan_splits(kv_lens: torch.Tensor, num_kv_splits: Optional[torch.Tensor], max_splits: int, floor_tokens: int, target_jobs: int):
     """The int32 device array `xkv_plan_splits` fills: [0] the smallest multiple of 32, not below `floor_tokens`, that cuts the
     sequences of the batch into at most `target_jobs` splits; [1] the number of live (sequence, split) pairs; then the pairs.
-    Pass it as `split_plan` (with `split_cap=floor_tokens` and the same `max_splits`) to stage 1 and the merge."""
+    Pass it as `split_plan` (with `split_cap=floor_tokens` and the same `max_splits`) to stage 1 and the merge.  Without
+    `num_kv_splits` the plan is packed: `max_splits` counts the jobs of the batch (at least `target_jobs` and the batch), which is
+    how many partial rows per head the workspaces hold, and the first job of every sequence stands behind the pairs."""
     batch = kv_lens.numel()
-    plan = torch.empty(2 + 2 * batch * int(max_splits), dtype=torch.int32, device=kv_lens.device)
+    words = 2 + 2 * int(max_splits) * batch if num_kv_splits is not None else 2 + 2 * int(max_splits) + batch
+    plan = torch.empty(words, dtype=torch.int32, device=kv_lens.device)
     check(_lib.lib().xkv_plan_splits(ptr(kv_lens), ptr(num_kv_splits), batch, int(max_splits), int(floor_tokens),
                                      int(target_jobs), ptr(plan), stream_ptr(kv_lens)), "xkv_plan_splits")
     return plan
@@ -279,17 +283,19 @@ def capped_splits(kv_len: int, max_kv_splits: int, cap_tokens: int) -> int:
 
 
 def ragged_plan(lens, batch: int, groups: int, kv_len: int, floor: int, per_cu: int = 1):
-    """Splits of a ragged batch: ``(num_kv_splits, cap, split dimension of the workspaces, split plan on the device)``.  The
-    split length is planned on the device so that the batch is cut into at most one job per workgroup the chip holds
-    (`per_cu` per CU, `groups` workgroups per job), no shorter than `floor` tokens or a 256th of the longest sequence
-    (which bounds the workspaces)."""
+    """Splits of a ragged batch: ``(None, cap, jobs, split plan on the device)``, the plan packed.  The split length is planned on
+    the device so that the batch is cut into at most one job per workgroup the chip holds (`per_cu` per CU, `groups` workgroups
+    per job), no shorter than `floor` tokens or a 256th of the longest sequence; `jobs` is the most that can come of it."""
     cap = max(floor, _cdiv(_cdiv(kv_len, 256), 32) * 32)
-    S = _cdiv(kv_len, cap)
-    one = uniform_splits(batch, 1, lens.device)
-    return one, cap, S, plan_splits(lens, one, S, cap, max(1, per_cu * num_cus() // groups))
+    target = max(1, per_cu * num_cus() // groups)
+    jobs = max(target, batch)
+    return None, cap, jobs, plan_splits(lens, None, jobs, cap, target)
 
 
-def workspaces(batch: int, hq: int, max_splits: int, dv: int, device):
+def workspaces(batch: int, hq: int, max_splits: int, dv: int, device, split_plan=None):
+    """Partial rows and their log-sum-exps; under a packed plan `max_splits` jobs for the whole batch."""
+    if split_plan is not None:
+        batch = 1
     partial = torch.empty((batch, hq, max_splits, dv), dtype=torch.float32, device=device)
     lse = torch.empty((batch, hq, max_splits), dtype=torch.float32, device=device)
     return partial, lse

@@ -144,3 +144,67 @@ def test_two_pass_rope_decode(dev, dtype, b, hq, hkv, L, rk, rv, off, monkeypatc
     monkeypatch.setattr(_fused, "TWO_PASS_KEY_RANKS", ())
     monkeypatch.setattr(_fused, "TWO_PASS_SMALL_RANK", 0)
     check_out(fr.gqa_xKV_rope(qd, kAd, kBd, vAd, vBd, torch.zeros_like(qd), ns, 2, 128 ** -0.5, 5e5, pos_offset=off), ref, "one kernel")
+
+
+@pytest.mark.parametrize("lens,floor,target", [
+    ([1], 32, 1),                                   # one sequence, one job
+    ([0, 5, 0, 4000, 33, 0], 32, 7),                # sequences without tokens have no rows
+    ([300] * 40, 128, 8),                           # more sequences than jobs: one job each
+    ([7 + (613 * i) % 3000 for i in range(1100)], 128, 2048),   # several chunks of sequences
+])
+def test_packed_plan(dev, lens, floor, target):
+    """A plan without an array of counts: every job once, whole splits first, and each sequence's first partial row."""
+    b = len(lens)
+    n = max(b, target)
+    kl = torch.tensor(lens, dtype=torch.int32, device=dev)
+    plan = ops.plan_splits(kl, None, n, floor, target).cpu().tolist()
+    assert len(plan) == 2 + 2 * n + b
+    count = lambda cap: sum(-(-x // cap) for x in lens)
+    top = max(floor, -(-max(lens) // 32) * 32)
+    cap = next((c for c in range(floor, top, 32) if count(c) <= target), top)
+    live = [ops.settled_splits(x, -(-x // cap)) if x else 0 for x in lens]
+    assert plan[0] == cap and plan[1] == sum(live) <= n
+    assert plan[2 + 2 * n:] == [sum(live[:i]) for i in range(b)]
+    pairs = [(plan[2 + 2 * j], plan[3 + 2 * j]) for j in range(plan[1])]
+    assert sorted(pairs) == [(i, s) for i in range(b) for s in range(live[i])]
+    assert all(s == live[i] - 1 for i, s in pairs[sum(max(x - 1, 0) for x in live):])
+
+
+@pytest.mark.parametrize("hq,hkv,d,rv", [
+    (8, 2, 64, 0), (16, 4, 128, 0),     # register-staged kernel, several kv groups a job
+    (16, 8, 128, 0), (32, 8, 128, 0),   # all heads of a job in one workgroup, values per head
+    (8, 8, 128, 256), (32, 8, 128, 512),   # ... one value row for all heads, up-projected
+    (6, 2, 96, 192),                    # register-staged with a shared value row, up-projected
+])
+def test_packed_rows(dev, hq, hkv, d, rv):
+    """Stage 1 and merge over packed partial rows against the same sequences alone; sequences without tokens give zeros, as before."""
+    lens = [517, 0, 1, 2048, 33, 96, 1024]
+    b, L, dv, floor = len(lens), max(lens), rv or d, 64
+    kl = torch.tensor(lens, dtype=torch.int32, device=dev)
+    q, K = gen((b, hq, d), seed=1).to(dev), gen((b, L, hkv, d), seed=2).to(dev)
+    V = gen((b, L, rv) if rv else (b, L, hkv, d), seed=3).to(dev)
+    vB = gen((b, hkv, rv, 64), std=rv ** -0.5, seed=4).to(dev) if rv else None
+    kop = lambda K: (K, K.stride(0), K.stride(1), K.stride(2), d)
+    vop = lambda V: (V, V.stride(0), V.stride(1), 0 if rv else V.stride(2), dv)
+    for target in (9, 40):
+        n = max(b, target)
+        plan = ops.plan_splits(kl, None, n, floor, target)
+        partial, lse = (torch.full(s, float("nan"), device=dev) for s in ((hq * n, dv), (hq * n,)))
+        ops.latent_stage1(q, None, None, kop(K), None, vop(V), partial, lse, None, None, kl, b, hq, hkv, L, n, d ** -0.5, split_cap=floor,
+                          split_plan=plan)
+        o = torch.full((b, hq, 64 if rv else d), float("nan"), dtype=torch.float32, device=dev)
+        lo = torch.empty(b, hq, dtype=torch.float32, device=dev)
+        ops.merge_stage2(partial, lse, o, vB, None, kl, b, hq, hkv if rv else hq, L, n, lse_out=lo, split_cap=floor, split_plan=plan)
+        jobs = plan[1].item()
+        assert not lse[:hq * jobs].isnan().any() and lse[hq * jobs:].isnan().all()      # every row of a job, and no other
+        for i, x in enumerate(lens):
+            if x == 0:
+                assert (o[i] == 0).all()
+                continue
+            p1, l1 = ops.workspaces(1, hq, 1, dv, dev)
+            ops.latent_stage1(q[i:i + 1], None, None, kop(K[i:i + 1, :x]), None, vop(V[i:i + 1, :x]), p1, l1, None, None, None, 1, hq, hkv, x, 1, d ** -0.5)
+            ref = torch.empty_like(o[i:i + 1])
+            ops.merge_stage2(p1, l1, ref, vB[i:i + 1] if rv else None, None, None, 1, hq, hkv if rv else hq, x, 1)
+            # the softmax weights are rounded to bf16 against another running maximum: two roundings of 2^-9 of the weights' sum
+            assert max_abs(o[i], ref[0]) <= 2.0 ** -7 * max(1.0, ref.abs().max().item())
+            assert max_abs(lo[i], l1[0, :, 0]) <= 1e-5

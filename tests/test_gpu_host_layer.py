@@ -1,0 +1,53 @@
+"""The native host layer as a serving program meets it: scratch of a ragged batch, and what a call does besides computing."""
+import pytest
+import torch
+
+from util import check_out, gen
+
+pytestmark = pytest.mark.gpu
+
+BF, FP = torch.bfloat16, torch.float16
+
+
+def one_long(b, L):
+    return [L] + [1 + (37 * i) % 200 for i in range(1, b)]
+
+
+@pytest.mark.parametrize("path", ["native", "general"])
+@pytest.mark.parametrize("form", ["gqa", "v_factorized", "decode"])
+def test_scratch_of_a_ragged_batch_follows_its_jobs(dev, path, form):
+    """64 sequences, the longest of 32K tokens: partial rows for the jobs the batch is cut into, not for as many splits of every
+    sequence as the longest one gets (2.1 million rows of 128 or 512 floats, 268 MB and more)."""
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd.flash_decoding import gqa
+    b, L, hq, hkv, r = 64, 32768, 32, 8, 512
+    lens = one_long(b, L)
+    scale = 128 ** -0.5
+    one = lambda *s, seed: gen(s, seed=seed).to(dev).expand(b, *s[1:])   # one cache for all
+    q = gen((b, hq, 128), seed=1).to(dev)
+    if path == "general":       # rows of a wider buffer: the native layer declines, the wrapper copies q and launches by itself
+        q = torch.empty(b, hq, 136, dtype=BF, device=dev)[..., :128].copy_(q)
+    kl = torch.tensor(lens, dtype=torch.int32, device=dev)
+    ns = torch.full((b,), 4, dtype=torch.int32, device=dev)
+    o = torch.empty(b, hq, 128, dtype=BF, device=dev)
+    vB = gen((1, hkv, r, 128), std=r ** -0.5, seed=5).to(dev).expand(b, -1, -1, -1)
+    if form == "gqa":
+        K, V = one(1, L, hkv, 128, seed=2), one(1, L, hkv, 128, seed=3)
+        run = lambda i, j, n, lens: gqa.decode_attention_fwd(q[i:j], K[i:j, :n], V[i:j, :n], o[i:j], ns[i:j], 4, scale, kv_lens=lens)
+    elif form == "v_factorized":
+        K, V = one(1, L, hkv, 128, seed=2), one(1, L, r, seed=3)
+        run = lambda i, j, n, lens: gqa.decode_attention_fwd_v_factorized(q[i:j], K[i:j, :n], V[i:j, :n], vB[i:j], o[i:j], ns[i:j], 4, scale, kv_lens=lens)
+    else:
+        K, V = one(1, L, r, seed=2), one(1, L, r, seed=3)
+        run = lambda i, j, n, lens: fr.gqa_xKV_no_pe(q[i:j], K[i:j, :n], vB[i:j], V[i:j, :n], vB[i:j], o[i:j], ns[i:j], 4, scale, kv_lens=lens)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    run(0, b, L, kl)
+    used = torch.cuda.max_memory_allocated() - before
+    # 512 jobs at most (the per-head form on 256 CUs), 32 rows of 512 floats each, and their log-sum-exps, merged rows and queries
+    assert used <= 512 * hq * (r + 1) * 4 + (8 << 20), used
+    got = o.clone()
+    for i in (0, 1, 17, b - 1):
+        run(i, i + 1, lens[i], None)
+        check_out(got[i], o[i], f"sequence {i}")
