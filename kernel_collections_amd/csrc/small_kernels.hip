@@ -284,9 +284,13 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(
 // a lane keeps half of its sums and hands the other half over) and four LDS words per total.  By trace, batch 1: one row per
 // head, dv 512, 6.4 us for 32 heads on 8 or 1 kv heads (rows + up-projection at 256 splits: 12.5 us, one kernel that did both
 // 20 - 21.7); 8 splits of 256, 4.7 us (7.0); 16 x 32 heads, 2 splits of 512, 8.6 us (11.6).
+//
+// SPREAD: many splits on a chip that is not full (launch_merge): one head per workgroup, its splits dealt out among groups of threads
+// as in merge_rows_kernel.  256 splits of 512, 32 heads, d_out 128: 12.6 us (26.4 with a thread folding all splits of its packet).
 constexpr int MERGE_CB = 64;       // columns per workgroup: whole 128-byte lines of a vB row
 constexpr int MERGE_UP_T = 512;
-template <typename O, typename TB, int RPT>
+constexpr int MERGE_ROWS_FLOATS = 49152;   // partial values a workgroup folds in every column block at most; measured in host.cpp
+template <typename O, typename TB, int RPT, bool SPREAD>
 __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     const float* __restrict__ partial, const float* __restrict__ lse, O* __restrict__ out,
     const TB* __restrict__ vB, int64_t sVb, int64_t sVh, int64_t sVr, int d_out,
@@ -294,20 +298,24 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     int hq, int hkv, int kv_len, int max_splits, int dv, int64_t sOb, int64_t sOh, int hpw,
     float* __restrict__ lse_out, int64_t sLb, int64_t sLh, int split_cap, const int32_t* __restrict__ split_plan) {
   typedef typename Elem<TB>::vec8 vec8;
-  extern __shared__ float merged[];               // [hpw][dv]
+  extern __shared__ float merged[];               // [hpw][dv]; SPREAD: then a packet, a maximum and a sum of every thread
   __shared__ float tot[4][4 * MERGE_CB];          // [quarter of the row groups][4 heads x 64 columns]
-  const int hfirst = blockIdx.x * hpw, kh = hfirst / (hq / hkv), b = blockIdx.y, c0 = blockIdx.z * MERGE_CB;
+  const int hfirst = blockIdx.x * hpw, kh = hfirst / (hq / hkv), b = blockIdx.y;
+  int c0 = blockIdx.z * MERGE_CB;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // the 16 lanes of a row hold 16 row groups of one 8-column block; a wave covers four blocks, a pair of waves all eight
   const int cb = (wave & 1) * 4 + (lane >> 4), grp = (wave >> 1) * 16 + (lane & 15);
-  const bool cols = c0 + cb * 8 < d_out;          // d_out is a multiple of 8
-  const TB* Bh = vB + b * sVb + kh * sVh + c0 + cb * 8;
+  const TB* Bh = vB + b * sVb + kh * sVh + cb * 8;
   vec8 w[RPT];
+  auto load_w = [&]() {
+    const bool cols = c0 + cb * 8 < d_out;        // d_out is a multiple of 8
 #pragma unroll
-  for (int r = 0; r < RPT; ++r) {
-    w[r] = vec8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (cols && grp + 64 * r < dv) w[r] = ld16<vec8>(Bh + (int64_t)(grp + 64 * r) * sVr);
-  }
+    for (int r = 0; r < RPT; ++r) {
+      w[r] = vec8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (cols && grp + 64 * r < dv) w[r] = ld16<vec8>(Bh + c0 + (int64_t)(grp + 64 * r) * sVr);
+    }
+  };
+  load_w();
   const int L = kv_lens ? kv_lens[b] : kv_len;
   const int nlive = live_splits(L, effective_splits(L, asked_splits(num_kv_splits, b, max_splits, split_cap), split_cap_in_force(split_cap, split_plan)), max_splits);
   const PartialRows rows = partial_rows(b, hq, max_splits, [&] { return nlive; }, num_kv_splits, split_plan);
@@ -321,29 +329,66 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     for (int e = 0; e < P; ++e) merged[gi * dv + c + e] = a.acc[e] * inv;
     if (lse_out && c == 0 && blockIdx.z == 0) lse_out[b * sLb + (hfirst + gi) * sLh] = a.m + __logf(a.l);
   };
-  if ((dv & 3) == 0 && (reinterpret_cast<uintptr_t>(partial) & 15) == 0) {
+  auto merge_shared = [&](auto tag) {             // SPREAD: head hfirst, its splits dealt out among MERGE_UP_T / (dv / P) groups
+    constexpr int P = decltype(tag)::value;
+    float* red = merged + dv;
+    float* ml = red + MERGE_UP_T * P;
+    const int lanes = dv / P, ngrp = MERGE_UP_T / lanes, sg = tid / lanes, c = (tid % lanes) * P;
+    const int64_t row = rows.base + (int64_t)hfirst * rows.per_head;
+    if (sg < ngrp) {
+      const MergeAcc<P> a = merge_fold<P>(lse + row, partial + row * dv + c, dv, sg, ngrp, nlive);
+#pragma unroll
+      for (int e = 0; e < P; ++e) red[tid * P + e] = a.acc[e];
+      ml[2 * tid] = a.m;
+      ml[2 * tid + 1] = a.l;
+    }
+    __syncthreads();
+    if (sg) return;
+    float M = ml[2 * tid];
+    for (int g = 1; g < ngrp; ++g) M = fmaxf(M, ml[2 * (g * lanes + tid)]);
+    float l = 0.f, acc[P];
+#pragma unroll
+    for (int e = 0; e < P; ++e) acc[e] = 0.f;
+    for (int g = 0; g < ngrp; ++g) {
+      const int t = g * lanes + tid;
+      const float x = ml[2 * t] == NEG_INF ? 0.f : __expf(ml[2 * t] - M);
+      l += x * ml[2 * t + 1];
+#pragma unroll
+      for (int e = 0; e < P; ++e) acc[e] += x * red[t * P + e];
+    }
+    const float inv = nlive > 0 ? 1.f / l : 0.f;
+#pragma unroll
+    for (int e = 0; e < P; ++e) merged[c + e] = acc[e] * inv;
+    if (lse_out && c == 0 && blockIdx.z == 0) lse_out[b * sLb + hfirst * sLh] = M + __logf(l);
+  };
+  const bool vec = (dv & 3) == 0 && (reinterpret_cast<uintptr_t>(partial) & 15) == 0;
+  if constexpr (SPREAD) {
+    if (vec) merge_shared(std::integral_constant<int, 4>());
+    else merge_shared(std::integral_constant<int, 1>());
+  } else if (vec) {
     const int ppr = dv >> 2;
     for (int i = tid; i < hpw * ppr; i += MERGE_UP_T) merge_packet(i / ppr, (i % ppr) * 4, std::integral_constant<int, 4>());
   } else {
     for (int i = tid; i < hpw * dv; i += MERGE_UP_T) merge_packet(i / dv, i % dv, std::integral_constant<int, 1>());
   }
   __syncthreads();
-  for (int g0 = 0; g0 < hpw; g0 += 4) {
-    float acc[32];                                // [4 heads][8 columns]
+  for (;;) {                                      // this workgroup's column blocks
+    for (int g0 = 0; g0 < hpw; g0 += 4) {
+      float acc[32];                                // [4 heads][8 columns]
 #pragma unroll
-    for (int i = 0; i < 32; ++i) acc[i] = 0.f;
+      for (int i = 0; i < 32; ++i) acc[i] = 0.f;
 #pragma unroll
-    for (int r = 0; r < RPT; ++r) {
-      const int rho = grp + 64 * r;
+      for (int r = 0; r < RPT; ++r) {
+        const int rho = grp + 64 * r;
 #pragma unroll
-      for (int gi = 0; gi < 4; ++gi) {
-        const float m = g0 + gi < hpw && rho < dv ? merged[(g0 + gi) * dv + rho] : 0.f;
+        for (int gi = 0; gi < 4; ++gi) {
+          const float m = g0 + gi < hpw && rho < dv ? merged[(g0 + gi) * dv + rho] : 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[gi * 8 + e] += m * to_f32(w[r][e]);
+          for (int e = 0; e < 8; ++e) acc[gi * 8 + e] += m * to_f32(w[r][e]);
+        }
       }
-    }
-    // halving exchanges over the 16 lanes that share a column block: partner 15 - l, then 7 - l, 3 - l, 1 - l of the shrinking
-    // group; the lane with the bit set keeps the upper half
+      // halving exchanges over the 16 lanes that share a column block: partner 15 - l, then 7 - l, 3 - l, 1 - l of the shrinking
+      // group; the lane with the bit set keeps the upper half
 #define XKV_HALVE(N, BIT, CTRL)                                                                                               \
     {                                                                                                                         \
       const bool up = lane & BIT;                                                                                             \
@@ -351,22 +396,26 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
         const float give = up ? acc[i] : acc[N + i], keep = up ? acc[N + i] : acc[i];                                         \
         acc[i] = keep + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give), CTRL, 0xf, 0xf, false)); \
       }                                                                                                                       \
-    }
-    XKV_HALVE(16, 8, 0x140)   // row_mirror
-    XKV_HALVE(8, 4, 0x141)    // row_half_mirror
-    XKV_HALVE(4, 2, 0x1B)     // quad_perm [3,2,1,0]
-    XKV_HALVE(2, 1, 0xB1)     // quad_perm [1,0,3,2]
+      }
+      XKV_HALVE(16, 8, 0x140)   // row_mirror
+      XKV_HALVE(8, 4, 0x141)    // row_half_mirror
+      XKV_HALVE(4, 2, 0x1B)     // quad_perm [3,2,1,0]
+      XKV_HALVE(2, 1, 0xB1)     // quad_perm [1,0,3,2]
 #undef XKV_HALVE
-    const int idx = (lane & 8 ? 16 : 0) + (lane & 4 ? 8 : 0) + (lane & 2 ? 4 : 0) + (lane & 1 ? 2 : 0);   // this lane's two sums
+      const int idx = (lane & 8 ? 16 : 0) + (lane & 4 ? 8 : 0) + (lane & 2 ? 4 : 0) + (lane & 1 ? 2 : 0);   // this lane's two sums
 #pragma unroll
-    for (int i = 0; i < 2; ++i) tot[wave >> 1][((idx + i) >> 3) * MERGE_CB + cb * 8 + ((idx + i) & 7)] = acc[i];
-    __syncthreads();
-    if (tid < 4 * MERGE_CB) {
-      const int gi = tid / MERGE_CB, c = c0 + tid % MERGE_CB;
-      if (g0 + gi < hpw && c < d_out)
-        out[b * sOb + (hfirst + g0 + gi) * sOh + c] = (O)(tot[0][tid] + tot[1][tid] + tot[2][tid] + tot[3][tid]);
+      for (int i = 0; i < 2; ++i) tot[wave >> 1][((idx + i) >> 3) * MERGE_CB + cb * 8 + ((idx + i) & 7)] = acc[i];
+      __syncthreads();
+      if (tid < 4 * MERGE_CB) {
+        const int gi = tid / MERGE_CB, c = c0 + tid % MERGE_CB;
+        if (g0 + gi < hpw && c < d_out)
+          out[b * sOb + (hfirst + g0 + gi) * sOh + c] = (O)(tot[0][tid] + tot[1][tid] + tot[2][tid] + tot[3][tid]);
+      }
+      __syncthreads();            // tot is reused by the next four heads, or the next columns
     }
-    __syncthreads();            // tot is reused by the next four heads
+    c0 += gridDim.z * MERGE_CB;
+    if (c0 >= d_out) return;
+    load_w();
   }
 }
 
@@ -411,14 +460,22 @@ static int launch_merge(const float* partial, const float* lse, void* out, const
   int hpw = g;
   while (hpw > 1 && (g % hpw != 0 || (size_t)hpw * dv * sizeof(float) > 48 * 1024)) --hpw;
   while (hpw > 4 && hpw % 2 == 0 && (int64_t)(hq / hpw) * batch * cdiv(d_out, MERGE_CB) < 256) hpw /= 2;
-  const dim3 grid(hq / hpw, batch, cdiv(d_out, MERGE_CB));
-  const size_t shm = (size_t)hpw * dv * sizeof(float);
-  if (dv <= 256)
-    merge_up_kernel<O, TB, 4><<<grid, dim3(MERGE_UP_T), shm, st>>>(partial, lse, (O*)out, (const TB*)vB, sVb, sVh, sVr, d_out, ns, kl, hq, hkv,
-                                                            kv_len, max_splits, dv, sOb, sOh, hpw, lse_out, sLb, sLh, split_cap, split_plan);
-  else
-    merge_up_kernel<O, TB, 8><<<grid, dim3(MERGE_UP_T), shm, st>>>(partial, lse, (O*)out, (const TB*)vB, sVb, sVh, sVr, d_out, ns, kl, hq, hkv,
-                                                            kv_len, max_splits, dv, sOb, sOh, hpw, lse_out, sLb, sLh, split_cap, split_plan);
+  // Many splits (a caller with scratch to spare merges the rows first, as the wrappers do): where the heads fill the chip a workgroup
+  // folds once for several column blocks; where they do not even with a workgroup per block, a workgroup takes one head and deals
+  // its splits out among groups of threads.
+  int z = cdiv(d_out, MERGE_CB);
+  const bool many = seq_splits > 1 && (int64_t)seq_splits * g * dv > MERGE_ROWS_FLOATS;
+  const bool spread = many && (int64_t)(hq / hpw) * batch * z < 256;
+  if (spread) hpw = 1;
+  if (many) z = (int)std::min<int64_t>(z, cdiv(256, std::min<int64_t>(256, (int64_t)(hq / hpw) * batch)));
+  const dim3 grid(hq / hpw, batch, z);
+  const size_t shm = ((size_t)hpw * dv + (spread ? MERGE_UP_T * 6 : 0)) * sizeof(float);
+#define XKV_MERGE_UP(RPT, SPREAD)                                                                                                      \
+  merge_up_kernel<O, TB, RPT, SPREAD><<<grid, dim3(MERGE_UP_T), shm, st>>>(partial, lse, (O*)out, (const TB*)vB, sVb, sVh, sVr, d_out, ns, kl, \
+                                                         hq, hkv, kv_len, max_splits, dv, sOb, sOh, hpw, lse_out, sLb, sLh, split_cap, split_plan)
+  if (dv <= 256) { if (spread) XKV_MERGE_UP(4, true); else XKV_MERGE_UP(4, false); }
+  else { if (spread) XKV_MERGE_UP(8, true); else XKV_MERGE_UP(8, false); }
+#undef XKV_MERGE_UP
   return launch_status();
 }
 

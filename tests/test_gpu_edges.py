@@ -208,3 +208,70 @@ def test_packed_rows(dev, hq, hkv, d, rv):
             # the softmax weights are rounded to bf16 against another running maximum: two roundings of 2^-9 of the weights' sum
             assert max_abs(o[i], ref[0]) <= 2.0 ** -7 * max(1.0, ref.abs().max().item())
             assert max_abs(lo[i], l1[0, :, 0]) <= 1e-5
+
+
+def merge_c(part, lse, out, vB, S, kv_len, lse_out=None):
+    """xkv_merge_stage2 itself: one launch, whatever the number of splits (ops.merge_stage2 merges the rows of many splits first)."""
+    from ctypes import c_int64 as i64
+
+    from kernel_collections_amd import _lib
+    b, hq, dv = lse.shape[0], lse.shape[1], part.shape[-1]
+    sv = vB.stride() if vB is not None else (0, 0, 0)
+    rc = _lib.lib().xkv_merge_stage2(
+        _lib.ptr(part), _lib.ptr(lse), _lib.ptr(out), _lib.ptr(vB), i64(sv[0]), i64(sv[1]), i64(sv[2]), vB.shape[-1] if vB is not None else dv,
+        _lib.dtype_code(vB.dtype) if vB is not None else _lib.XKV_BF16, _lib.ptr(None), _lib.ptr(None), b, hq,
+        vB.shape[1] if vB is not None else hq, kv_len, S, 0, _lib.ptr(None), dv, i64(out.stride(0)), i64(out.stride(1)),
+        _lib.dtype_code(out.dtype), _lib.ptr(lse_out), i64(hq), i64(1), _lib.stream_ptr(part))
+    _lib.check(rc, "xkv_merge_stage2")
+
+
+@pytest.mark.parametrize("b,hq,hkv,S,live,dv,d_out,shift", [
+    (1, 8, 2, 128, 128, 512, 128, 0),     # two column blocks, four groups of threads
+    (1, 32, 1, 33, 29, 256, 512, 0),      # the last dv with four packets per thread, dead splits, eight column blocks
+    (5, 40, 4, 97, 97, 192, 72, 0),       # ten groups and idle threads; a partial second block
+    (33, 32, 8, 40, 40, 320, 200, 0),     # heads fill the chip: one workgroup for all four column blocks
+    (1, 3, 1, 300, 299, 70, 24, 0),       # rows that are not a multiple of 16 bytes
+    (2, 4, 1, 64, 64, 256, 64, 1),        # ... whose base is not 16-byte aligned
+])
+@pytest.mark.parametrize("dtype", [BF, FP])
+def test_merge_of_many_splits_in_one_launch(dev, dtype, b, hq, hkv, S, live, dv, d_out, shift):
+    part, lse = gen((b, hq, S, dv), dtype=torch.float32, seed=1), gen((b, hq, S), std=4.0, dtype=torch.float32, seed=2)
+    w = torch.softmax(lse[..., :live].double(), -1)
+    vB = gen((b, hkv, dv, d_out), std=dv ** -0.5, dtype=dtype, seed=3)
+    ref = torch.einsum("bkgr,bkrd->bkgd", (w.unsqueeze(-1) * part[:, :, :live].double()).sum(2).reshape(b, hkv, hq // hkv, dv), vB.double())
+    part[:, :, live:], lse[..., live:] = float("nan"), float("nan")      # dead splits are never read
+    pd = torch.empty(part.numel() + shift, dtype=torch.float32, device=dev)[shift:].view(part.shape).copy_(part)
+    out, lo = torch.empty((b, hq, d_out), dtype=torch.float32, device=dev), torch.empty((b, hq), dtype=torch.float32, device=dev)
+    merge_c(pd, lse.to(dev), out, vB.to(dev), S, 32 * live, lo)
+    # fp32 sums of at most 300 splits and 512 ranks of unit terms, v_exp_f32 weights to 2^-21 of their value at |lse| <= 20
+    ref = ref.reshape(b, hq, d_out)
+    assert max_abs(out, ref) <= 2e-5 * max(1.0, ref.abs().max().item())
+    assert max_abs(lo, torch.logsumexp(lse[..., :live].double(), -1)) <= 1e-5
+
+
+def test_merge_of_many_splits_keeps_the_chip_busy(dev):
+    """256 splits, up-projected: one launch that folds the splits in every column block took twice as long as merging the rows first."""
+    b, hq, hkv, S, dv, d_out = 1, 32, 8, 256, 512, 128
+    part, lse, mid, lo = (torch.randn(s, device=dev) for s in ((b, hq, S, dv), (b, hq, S), (b, hq, 1, dv), (b, hq)))
+    vB, out = torch.randn(b, hkv, dv, d_out, device=dev).to(BF), torch.empty(b, hq, d_out, dtype=BF, device=dev)
+
+    def us(call):          # device time: 20 calls in a graph
+        call()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            for _ in range(20):
+                call()
+        ev, best = [torch.cuda.Event(enable_timing=True) for _ in range(2)], 1e9
+        for _ in range(10):
+            ev[0].record()
+            g.replay()
+            ev[1].record()
+            torch.cuda.synchronize()
+            best = min(best, ev[0].elapsed_time(ev[1]) * 50)
+        return best
+
+    def rows_first():
+        merge_c(part, lse, mid, None, S, 32 * S, lo)
+        merge_c(mid, lo, out, vB, 1, 32)
+    one, two = us(lambda: merge_c(part, lse, out, vB, S, 32 * S)), us(rows_first)
+    assert one <= 1.5 * two, (one, two)
