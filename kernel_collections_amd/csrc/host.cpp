@@ -88,6 +88,7 @@ int balanced_splits(int64_t batch, int groups, int64_t kv_len, int tile, int per
 }
 
 int head_groups(int64_t hq) {            // smallest number of equal head groups of at most 32
+  need(hq > 0);
   int g = cdiv(hq, 32);
   while (hq % g) ++g;
   return g;

@@ -51,3 +51,21 @@ def test_scratch_of_a_ragged_batch_follows_its_jobs(dev, path, form):
     for i in (0, 1, 17, b - 1):
         run(i, i + 1, lens[i], None)
         check_out(got[i], o[i], f"sequence {i}")
+
+
+def test_no_query_heads_are_refused(dev):
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd.flash_decoding import deepseek_mla, mla2
+    z = lambda *s: torch.zeros(s, dtype=BF, device=dev)
+    ns = torch.ones(1, dtype=torch.int32, device=dev)
+    calls = [
+        lambda: fr.qAB_no_pe_v1(z(1, 0, 1, 128), z(1, 40, 64), z(1, 2, 64, 128)),
+        lambda: fr.qAB_rope_v1(z(1, 0, 1, 128), z(1, 40, 64), z(1, 2, 64, 128)),
+        lambda: fr.gqa_xKV_no_pe(z(1, 0, 128), z(1, 40, 64), z(1, 2, 64, 128), z(1, 40, 64), z(1, 2, 64, 128), z(1, 0, 128), ns, 1, 1.0),
+        lambda: deepseek_mla.mla_decode_attention_fwd_pd_sep_xKV(z(1, 0, 128), z(1, 40, 64), z(1, 1, 64, 128), z(1, 40, 64), z(1, 1, 64, 128),
+                                                                 z(1, 3, 1, 128), z(1, 3, 1, 128)),
+        lambda: mla2.mla_decode_attention_fwd(z(1, 0, 512), z(1, 0, 64), z(1, 40, 1, 512), z(1, 40, 1, 64)),
+    ]
+    for call in calls:
+        with pytest.raises((AssertionError, RuntimeError, ZeroDivisionError)):
+            call()
