@@ -15,6 +15,7 @@
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <array>
@@ -233,8 +234,8 @@ template <typename Fn> PyObject* guarded(Py_ssize_t n, Py_ssize_t want, Fn fn) {
     return fn();
   } catch (const Decline&) {
     Py_RETURN_NONE;
-  } catch (const std::exception& e) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+  } catch (...) {   // as torch's own bindings raise it: an allocator that ran out of memory as torch.OutOfMemoryError
+    if (!PyErr_Occurred()) torch::translate_exception_to_python(std::current_exception());
     return nullptr;
   }
 }

@@ -69,3 +69,31 @@ def test_no_query_heads_are_refused(dev):
     for call in calls:
         with pytest.raises((AssertionError, RuntimeError, ZeroDivisionError)):
             call()
+
+
+def test_out_of_memory_is_torchs_own_error(dev):
+    """What a server catches to evict and try again - and the same call computes once there is room."""
+    import kernel_collections_amd.flash_recontruction as fr
+    L = 1 << 20
+    b = 32
+    q, A, B = gen((b, 32, 1, 128), seed=1).to(dev), torch.ones(1, L, 32, dtype=BF, device=dev).expand(b, -1, -1), gen((b, 8, 32, 128), seed=2).to(dev)
+    call = lambda: fr.qAB_rope_v1(q, A, B, out_dtype=torch.float32)      # 4 GiB of scores
+    call()
+    torch.cuda.empty_cache()
+    room = torch.cuda.memory_reserved() + (32 << 20)
+    try:
+        torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(dev).total_memory)
+        with pytest.raises(torch.OutOfMemoryError):
+            call()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert call().shape == (b, 32, 1, L)
+
+
+def test_a_kernels_refusal_is_a_runtime_error(dev):
+    """An error code of the C entry points keeps its text: rows wider than stage 1 serves."""
+    import kernel_collections_amd.flash_recontruction as fr
+    z = lambda *s: torch.zeros(s, dtype=BF, device=dev)
+    with pytest.raises(RuntimeError, match="xkv_latent_stage1 failed: shape outside the built envelope .code -2") as e:
+        fr.qAB_no_pe_v1(z(1, 4, 1, 128), z(1, 40, 1056), z(1, 2, 1056, 128))
+    assert type(e.value) is RuntimeError
