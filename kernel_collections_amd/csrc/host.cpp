@@ -240,6 +240,15 @@ template <typename Fn> PyObject* guarded(Py_ssize_t n, Py_ssize_t want, Fn fn) {
   }
 }
 inline PyObject* give(PyObject* o) { Py_INCREF(o); return o; }
+// What a call does once its arguments are C++ values.  Other Python threads run meanwhile: an allocator that has to free its cache
+// waits for the device, and a host function that Python put on a stream needs the interpreter to finish.
+template <typename Fn> void without_gil(Fn fn) {
+  struct Released {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(state); }
+  } released;
+  fn();
+}
 
 // ---- shared pieces of the factorised calls -----------------------------------------------------------------------------
 // Absorbed query q~ = q . B^T as a high + low pair [b, hq, rank]
@@ -267,23 +276,25 @@ PyObject* nope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     need(kB.size(2) == r && kB.size(3) == d && vB.size(2) == rv && hq % hkv == 0 && r % 32 == 0 && rv % 64 == 0 && rv <= 512 && d <= 512 && d % 8 == 0);
     need(packed_q(q) && rows(kA) && rows(kB) && rows(vA) && o.stride(2) == 1 && o.size(0) == b && o.size(1) == hq && o.size(2) == vB.size(3));
     need(hkv == 1 || hq / hkv <= 32);
-    Call c(q);
-    const Up up = up_of(vB, hq, c.dt);
     const at::Tensor lens = lens_of(a[7], q, b);
-    const int groups = head_groups(hq), odt = code_any(o);
-    Ragged rg{};
-    Splits s{0, 0, nullptr, nullptr};
-    if (lens.defined()) rg = ragged(c, s, b, groups, L, 128, ring_rank(r) ? 1 : 2);
-    else s.S = scan_splits(c, b, groups, L, ring_rank(r));
-    const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
-    const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
-    c.alloc();
-    if (lens.defined()) write_plan(c, s, rg, lens, b);
-    absorb(c, q.data_ptr(), kB, c.get<void>(hi), c.get<void>(lo), b, hq, d, r);
-    check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(kA, 0, r), NO_KV, kv(vA, 0, rv), c.get<float>(part),
-                              c.get<float>(lse), nullptr, 0, nullptr, s.lens, b, hq, groups, L, s.n(), s.cap, s.plan, scale, 0.f, c.dt,
-                              c.stream), "xkv_latent_stage1");
-    merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, L, rv);
+    without_gil([&] {
+      Call c(q);
+      const Up up = up_of(vB, hq, c.dt);
+      const int groups = head_groups(hq), odt = code_any(o);
+      Ragged rg{};
+      Splits s{0, 0, nullptr, nullptr};
+      if (lens.defined()) rg = ragged(c, s, b, groups, L, 128, ring_rank(r) ? 1 : 2);
+      else s.S = scan_splits(c, b, groups, L, ring_rank(r));
+      const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
+      const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
+      c.alloc();
+      if (lens.defined()) write_plan(c, s, rg, lens, b);
+      absorb(c, q.data_ptr(), kB, c.get<void>(hi), c.get<void>(lo), b, hq, d, r);
+      check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(kA, 0, r), NO_KV, kv(vA, 0, rv), c.get<float>(part),
+                                c.get<float>(lse), nullptr, 0, nullptr, s.lens, b, hq, groups, L, s.n(), s.cap, s.plan, scale, 0.f, c.dt,
+                                c.stream), "xkv_latent_stage1");
+      merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, L, rv);
+    });
     return give(a[5]);
   });
 }
@@ -299,15 +310,18 @@ PyObject* nope_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t b = q.size(0), hq = q.size(1), d = q.size(3), L = A.size(1), r = A.size(2), hkv = B.size(1);
     need(b > 0 && L > 0 && hkv > 0 && A.size(0) == b && B.size(0) == b && B.size(2) == r && B.size(3) == d && hq % hkv == 0 && r % 32 == 0);
     need(d <= 512 && d % 8 == 0 && packed_q(q) && rows(A) && rows(B) && (hkv == 1 || hq / hkv <= 32));
-    Call c(q);
-    const int groups = head_groups(hq), S = scan_splits(c, b, groups, L, ring_rank(r));
-    const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2);
-    c.alloc();
-    at::Tensor out = at::empty({b, hq, 1, L}, f32 ? c.opts.dtype(at::kFloat) : c.opts);
-    absorb(c, q.data_ptr(), B, c.get<void>(hi), c.get<void>(lo), b, hq, d, r);
-    check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(A, 0, r), NO_KV, NO_KV, nullptr, nullptr, out.data_ptr(),
-                              f32 ? XKV_F32 : c.dt, nullptr, nullptr, b, hq, groups, L, S, 0, nullptr, scale, 0.f, c.dt, c.stream),
-          "xkv_latent_stage1");
+    at::Tensor out;
+    without_gil([&] {
+      Call c(q);
+      const int groups = head_groups(hq), S = scan_splits(c, b, groups, L, ring_rank(r));
+      const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2);
+      c.alloc();
+      out = at::empty({b, hq, 1, L}, f32 ? c.opts.dtype(at::kFloat) : c.opts);
+      absorb(c, q.data_ptr(), B, c.get<void>(hi), c.get<void>(lo), b, hq, d, r);
+      check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(A, 0, r), NO_KV, NO_KV, nullptr, nullptr, out.data_ptr(),
+                                f32 ? XKV_F32 : c.dt, nullptr, nullptr, b, hq, groups, L, S, 0, nullptr, scale, 0.f, c.dt, c.stream),
+            "xkv_latent_stage1");
+    });
     return THPVariable_Wrap(out);
   });
 }
@@ -348,41 +362,43 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     rope_operands(q, hq, q.size(2), kA, kB, inv);
     need(vA.size(0) == b && vA.size(1) == L && vB.size(0) == b && vB.size(1) == hkv && vB.size(2) == rv && rv % 64 == 0 && rv <= 512 && rows(vA));
     need(o.stride(2) == 1 && o.size(0) == b && o.size(1) == hq && o.size(2) == vB.size(3));
-    Call c(q);
-    const Up up = up_of(vB, hq, c.dt);
-    const int odt = code_any(o);
-    const bool shared = vA.data_ptr() == kA.data_ptr() && vA.sizes() == kA.sizes() && vA.strides() == kA.strides();
-    const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, kB.stride(0)), ws = c.plan(ws_bytes);
-    const float* invp = inv.data_ptr<float>();
-    Splits s{0, 0, nullptr, nullptr};
-    if (may_two_pass && !shared && hq / hkv <= 8 && hq <= 32 && ring_rank(rv)) {
-      // a value basis of its own: scores first, then softmax and P.v_A in one stream for all heads.  The second pass reads the
-      // scores in 16-byte packets, so their rows are whole packets: at another length the kernels get the padded one as the row's
-      // and the true one as every sequence's (one fill, about 2 us).
-      const int64_t row = (L + 3) / 4 * 4;
-      at::Tensor lens;
-      if (row != L) {
-        lens = at::full({b}, L, c.opts.dtype(at::kInt));
-        s.lens = lens.data_ptr<int32_t>();
+    without_gil([&] {
+      Call c(q);
+      const Up up = up_of(vB, hq, c.dt);
+      const int odt = code_any(o);
+      const bool shared = vA.data_ptr() == kA.data_ptr() && vA.sizes() == kA.sizes() && vA.strides() == kA.strides();
+      const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, kB.stride(0)), ws = c.plan(ws_bytes);
+      const float* invp = inv.data_ptr<float>();
+      Splits s{0, 0, nullptr, nullptr};
+      if (may_two_pass && !shared && hq / hkv <= 8 && hq <= 32 && ring_rank(rv)) {
+        // a value basis of its own: scores first, then softmax and P.v_A in one stream for all heads.  The second pass reads the
+        // scores in 16-byte packets, so their rows are whole packets: at another length the kernels get the padded one as the row's
+        // and the true one as every sequence's (one fill, about 2 us).
+        const int64_t row = (L + 3) / 4 * 4;
+        at::Tensor lens;
+        if (row != L) {
+          lens = at::full({b}, L, c.opts.dtype(at::kInt));
+          s.lens = lens.data_ptr<int32_t>();
+        }
+        s.S = scan_splits(c, b, 1, L, true);
+        const int64_t sc = c.plan(b * hq * row * 4), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
+        const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
+        c.alloc();
+        recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, recon_splits(c, kB, b, hkv, hq / hkv, L, r, true), b, hq, hkv, row,
+              scale, invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes, s.lens);
+        check(p_xkv_softmax_pv_stage1(c.get<float>(sc), kv(vA, 0, rv), c.get<float>(part), c.get<float>(lse), nullptr, s.lens, b, hq, row, s.S,
+                                      0, nullptr, c.dt, c.stream), "xkv_softmax_pv_stage1");
+        merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, row, rv);
+        return;
       }
-      s.S = scan_splits(c, b, 1, L, true);
-      const int64_t sc = c.plan(b * hq * row * 4), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
+      s.S = recon_splits(c, kB, b, hkv, hq / hkv, L, r, false);
+      const int64_t part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
       const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
       c.alloc();
-      recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, recon_splits(c, kB, b, hkv, hq / hkv, L, r, true), b, hq, hkv, row,
-            scale, invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes, s.lens);
-      check(p_xkv_softmax_pv_stage1(c.get<float>(sc), kv(vA, 0, rv), c.get<float>(part), c.get<float>(lse), nullptr, s.lens, b, hq, row, s.S,
-                                    0, nullptr, c.dt, c.stream), "xkv_softmax_pv_stage1");
-      merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, row, rv);
-      return give(a[5]);
-    }
-    s.S = recon_splits(c, kB, b, hkv, hq / hkv, L, r, false);
-    const int64_t part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
-    const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
-    c.alloc();
-    recon(c, q, kA, kB, &vA, c.get<float>(part), c.get<float>(lse), nullptr, 0, s.S, b, hq, hkv, L, scale, invp, pos,
-          ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
-    merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, L, rv);
+      recon(c, q, kA, kB, &vA, c.get<float>(part), c.get<float>(lse), nullptr, 0, s.S, b, hq, hkv, L, scale, invp, pos,
+            ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
+      merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, L, rv);
+    });
     return give(a[5]);
   });
 }
@@ -398,12 +414,15 @@ PyObject* rope_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
     need(q.dim() == 4 && A.dim() == 3 && B.dim() == 4 && q.size(2) == 1);
     const int64_t b = q.size(0), hq = q.size(1), L = A.size(1), r = A.size(2), hkv = B.size(1);
     rope_operands(q, hq, q.size(3), A, B, inv);
-    Call c(q);
-    const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, B.stride(0)), ws = c.plan(ws_bytes);
-    if (ws_bytes) c.alloc();
-    at::Tensor out = at::empty({b, hq, 1, L}, f32 ? c.opts.dtype(at::kFloat) : c.opts);
-    recon(c, q, A, B, nullptr, nullptr, nullptr, out.data_ptr(), f32 ? XKV_F32 : c.dt, recon_splits(c, B, b, hkv, hq / hkv, L, r, true), b, hq, hkv,
-          L, scale, inv.data_ptr<float>(), pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
+    at::Tensor out;
+    without_gil([&] {
+      Call c(q);
+      const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, B.stride(0)), ws = c.plan(ws_bytes);
+      if (ws_bytes) c.alloc();
+      out = at::empty({b, hq, 1, L}, f32 ? c.opts.dtype(at::kFloat) : c.opts);
+      recon(c, q, A, B, nullptr, nullptr, nullptr, out.data_ptr(), f32 ? XKV_F32 : c.dt, recon_splits(c, B, b, hkv, hq / hkv, L, r, true), b, hq, hkv,
+            L, scale, inv.data_ptr<float>(), pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
+    });
     return THPVariable_Wrap(out);
   });
 }
@@ -422,41 +441,43 @@ PyObject* gqa(PyObject*, PyObject* const* a, Py_ssize_t n) {
     need(b > 0 && L > 0 && hkv > 0 && k.size(0) == b && k.size(3) == d && v.size(0) == b && v.size(1) == L && hq % hkv == 0 && hq / hkv <= 32);
     need(d % 32 == 0 && dv % 64 == 0 && dv <= 512 && packed_q(q) && rows(k) && rows(v) && o.stride(2) == 1 && o.size(0) == b && o.size(1) == hq);
     if (!fact) need(v.size(2) == hkv && dv == d && o.size(2) == dv);
-    Call c(q);
     const at::Tensor lens = lens_of(a[6], q, b);
-    const int odt = code_any(o);
-    Up up{};
-    if (fact) {
-      Ten vB = T(a[3]);
-      same(q, {&vB});
-      need(vB.dim() == 4 && vB.size(0) == b && vB.size(1) == hkv && vB.size(2) == dv && o.size(2) == vB.size(3));
-      up = up_of(vB, hq, c.dt);
-    }
-    // 8 kv heads of 128 side by side in a token row: stage 1 serves every head of a split from one workgroup, one per CU
-    const bool row8 = hkv == 8 && d == 128 && hq <= 32 && k.stride(2) == d && k.stride(1) >= 1024;
-    const bool wide8 = row8 && (fact ? ring_rank(dv) && v.stride(1) >= dv : v.stride(2) == d && v.stride(1) >= 1024);
-    // 512-wide token rows beside 512-wide value rows: the same form, against a block-diagonal query
-    const bool wide4 = fact && hkv * d == 512 && dv == 512 && hq <= 32 && k.stride(2) == d;
-    const bool wide = wide8 || wide4;
-    const int floor = wide ? floor_wide : floor_head, per_cu = wide ? 1 : 2, groups = wide ? 1 : (int)hkv;
-    need(floor > 0);
-    Ragged rg{};
-    Splits s{0, 0, nullptr, nullptr};
-    if (lens.defined()) rg = ragged(c, s, b, groups, L, floor, per_cu);
-    else s.S = std::min(balanced_splits(b, groups, L, 32, per_cu, c.cus), cdiv(L, floor));
-    const int64_t part = c.plan(s.rows(b, hq) * dv * 4), lse = c.plan(s.rows(b, hq) * 4), bd = c.plan(wide4 ? b * hq * 512 * 2 : 0);
-    const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, dv) ? rows_bytes(b, hq, dv) : 0);
-    c.alloc();
-    if (lens.defined()) write_plan(c, s, rg, lens, b);
-    const void* qp = q.data_ptr();
-    if (wide4) {
-      check(p_xkv_blockdiag_q(qp, c.get<void>(bd), b, hq, hkv, d, c.dt, c.stream), "xkv_blockdiag_q");
-      qp = c.get<void>(bd);
-    }
-    check(p_xkv_latent_stage1({qp, wide4 ? 512 : (int)d}, nullptr, NO_Q, wide4 ? kv(k, 0, 512) : kv(k, k.stride(2), d), NO_KV,
-                              kv(v, fact ? 0 : v.stride(2), dv), c.get<float>(part), c.get<float>(lse), nullptr, 0, nullptr, s.lens, b, hq,
-                              wide4 ? 1 : hkv, L, s.n(), s.cap, s.plan, scale, 0.f, c.dt, c.stream), "xkv_latent_stage1");
-    merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, fact ? &up : nullptr, mid, s, b, hq, L, dv);
+    Ten vB = fact ? T(a[3]) : v;
+    without_gil([&] {
+      Call c(q);
+      const int odt = code_any(o);
+      Up up{};
+      if (fact) {
+        same(q, {&vB});
+        need(vB.dim() == 4 && vB.size(0) == b && vB.size(1) == hkv && vB.size(2) == dv && o.size(2) == vB.size(3));
+        up = up_of(vB, hq, c.dt);
+      }
+      // 8 kv heads of 128 side by side in a token row: stage 1 serves every head of a split from one workgroup, one per CU
+      const bool row8 = hkv == 8 && d == 128 && hq <= 32 && k.stride(2) == d && k.stride(1) >= 1024;
+      const bool wide8 = row8 && (fact ? ring_rank(dv) && v.stride(1) >= dv : v.stride(2) == d && v.stride(1) >= 1024);
+      // 512-wide token rows beside 512-wide value rows: the same form, against a block-diagonal query
+      const bool wide4 = fact && hkv * d == 512 && dv == 512 && hq <= 32 && k.stride(2) == d;
+      const bool wide = wide8 || wide4;
+      const int floor = wide ? floor_wide : floor_head, per_cu = wide ? 1 : 2, groups = wide ? 1 : (int)hkv;
+      need(floor > 0);
+      Ragged rg{};
+      Splits s{0, 0, nullptr, nullptr};
+      if (lens.defined()) rg = ragged(c, s, b, groups, L, floor, per_cu);
+      else s.S = std::min(balanced_splits(b, groups, L, 32, per_cu, c.cus), cdiv(L, floor));
+      const int64_t part = c.plan(s.rows(b, hq) * dv * 4), lse = c.plan(s.rows(b, hq) * 4), bd = c.plan(wide4 ? b * hq * 512 * 2 : 0);
+      const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, dv) ? rows_bytes(b, hq, dv) : 0);
+      c.alloc();
+      if (lens.defined()) write_plan(c, s, rg, lens, b);
+      const void* qp = q.data_ptr();
+      if (wide4) {
+        check(p_xkv_blockdiag_q(qp, c.get<void>(bd), b, hq, hkv, d, c.dt, c.stream), "xkv_blockdiag_q");
+        qp = c.get<void>(bd);
+      }
+      check(p_xkv_latent_stage1({qp, wide4 ? 512 : (int)d}, nullptr, NO_Q, wide4 ? kv(k, 0, 512) : kv(k, k.stride(2), d), NO_KV,
+                                kv(v, fact ? 0 : v.stride(2), dv), c.get<float>(part), c.get<float>(lse), nullptr, 0, nullptr, s.lens, b, hq,
+                                wide4 ? 1 : hkv, L, s.n(), s.cap, s.plan, scale, 0.f, c.dt, c.stream), "xkv_latent_stage1");
+      merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, fact ? &up : nullptr, mid, s, b, hq, L, dv);
+    });
     return give(a[4]);
   });
 }
@@ -472,33 +493,36 @@ PyObject* mla(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t b = qn.size(0), hq = qn.size(1), w = qn.size(2), e = qr.size(2), L = C.size(1), r = C.size(3);
     need(b > 0 && L > 0 && hq > 0 && C.size(0) == b && R.size(0) == b && R.size(1) == L && qr.size(0) == b && qr.size(1) == hq && R.size(3) == e);
     need(r % 64 == 0 && r <= 512 && e % 32 == 0 && e > 0 && e <= 128 && packed_q(qn) && packed_q(qr) && rows(C) && rows(R));
-    Call c(qn);
-    Up up{};
-    if (fact) {
-      Ten B = T(a[3]);
-      same(qn, {&B});
-      need(B.dim() == 4 && B.size(0) == b && B.size(1) == 1 && B.size(2) == r && B.size(3) == w && w % 8 == 0 && w <= 512 && rows(B));
-      up = up_of(B, hq, c.dt);
-    } else {
-      need(w == r);
-    }
-    const int groups = head_groups(hq);
-    Splits s{scan_splits(c, b, groups, L, e == 64 && (r == 512 || (fact && ring_rank(r)))), 0, nullptr, nullptr};
-    const int64_t hi = c.plan(fact ? b * hq * r * 2 : 0), lo = c.plan(fact ? b * hq * r * 2 : 0);
-    const int64_t part = c.plan(s.rows(b, hq) * r * 4), lse = c.plan(s.rows(b, hq) * 4);
-    const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, r) ? rows_bytes(b, hq, r) : 0);
-    c.alloc();
-    at::Tensor o = at::empty({b, hq, w}, c.opts);
-    const void *q_hi = qn.data_ptr(), *q_lo = nullptr;
-    if (fact) {
-      absorb(c, q_hi, T(a[3]), c.get<void>(hi), c.get<void>(lo), b, hq, w, r);
-      q_hi = c.get<void>(hi);
-      q_lo = c.get<void>(lo);
-    }
-    check(p_xkv_latent_stage1({q_hi, (int)r}, q_lo, {qr.data_ptr(), (int)e}, kv(C, 0, r), kv(R, 0, e), kv(C, 0, r), c.get<float>(part),
-                              c.get<float>(lse), nullptr, 0, nullptr, nullptr, b, hq, groups, L, s.S, 0, nullptr, scale, 0.f, c.dt, c.stream),
-          "xkv_latent_stage1");
-    merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), hq * w, w, c.dt, fact ? &up : nullptr, mid, s, b, hq, L, r);
+    Ten B = fact ? T(a[3]) : C;
+    at::Tensor o;
+    without_gil([&] {
+      Call c(qn);
+      Up up{};
+      if (fact) {
+        same(qn, {&B});
+        need(B.dim() == 4 && B.size(0) == b && B.size(1) == 1 && B.size(2) == r && B.size(3) == w && w % 8 == 0 && w <= 512 && rows(B));
+        up = up_of(B, hq, c.dt);
+      } else {
+        need(w == r);
+      }
+      const int groups = head_groups(hq);
+      Splits s{scan_splits(c, b, groups, L, e == 64 && (r == 512 || (fact && ring_rank(r)))), 0, nullptr, nullptr};
+      const int64_t hi = c.plan(fact ? b * hq * r * 2 : 0), lo = c.plan(fact ? b * hq * r * 2 : 0);
+      const int64_t part = c.plan(s.rows(b, hq) * r * 4), lse = c.plan(s.rows(b, hq) * 4);
+      const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, r) ? rows_bytes(b, hq, r) : 0);
+      c.alloc();
+      o = at::empty({b, hq, w}, c.opts);
+      const void *q_hi = qn.data_ptr(), *q_lo = nullptr;
+      if (fact) {
+        absorb(c, q_hi, B, c.get<void>(hi), c.get<void>(lo), b, hq, w, r);
+        q_hi = c.get<void>(hi);
+        q_lo = c.get<void>(lo);
+      }
+      check(p_xkv_latent_stage1({q_hi, (int)r}, q_lo, {qr.data_ptr(), (int)e}, kv(C, 0, r), kv(R, 0, e), kv(C, 0, r), c.get<float>(part),
+                                c.get<float>(lse), nullptr, 0, nullptr, nullptr, b, hq, groups, L, s.S, 0, nullptr, scale, 0.f, c.dt, c.stream),
+            "xkv_latent_stage1");
+      merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), hq * w, w, c.dt, fact ? &up : nullptr, mid, s, b, hq, L, r);
+    });
     return THPVariable_Wrap(o);
   });
 }
@@ -517,30 +541,33 @@ PyObject* prefix_tail(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t dv = vT.size(3);
     need(r % 32 == 0 && rv % 64 == 0 && rv <= 512 && w % 32 == 0 && w <= 512 && dv % 64 == 0 && dv <= 512);
     need(packed_q(q) && rows(kA) && rows(kB) && rows(vA) && rows(kT) && rows(vT));
-    Call c(q);
-    const Up up = up_of(vB, hq, c.dt);
-    const int groups = head_groups(hq);
-    const bool shared = vA.data_ptr() == kA.data_ptr() && vA.strides() == kA.strides() && rv == r;
-    Splits s1{scan_splits(c, b, groups, L, ring_rank(r)), 0, nullptr, nullptr};
-    // the tail in at most four splits of whole 32-token blocks, every one of them live; a cap states the count, because the rows
-    // of the shared workspace are one more: row 0 is the merged, up-projected prefix with its log-sum-exp
-    const int blocks = cdiv(Lt, 32), per = cdiv(blocks, 4), S2 = cdiv(blocks, per);
-    const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part1 = c.plan(b * hq * s1.S * rv * 4), lse1 = c.plan(b * hq * s1.S * 4);
-    const int64_t mid = c.plan(rows_first(s1.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
-    const int64_t part = c.plan(b * hq * (1 + S2) * dv * 4), lse = c.plan(b * hq * (1 + S2) * 4);
-    c.alloc();
-    at::Tensor o = at::empty({b, hq, dv}, c.opts);
-    absorb(c, q.data_ptr(), kB, c.get<void>(hi), c.get<void>(lo), b, hq, w, r);
-    check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(kA, 0, r), NO_KV, shared ? kv(kA, 0, r) : kv(vA, 0, rv),
-                              c.get<float>(part1), c.get<float>(lse1), nullptr, 0, nullptr, nullptr, b, hq, groups, L, s1.S, 0, nullptr, scale,
-                              logit_cap, c.dt, c.stream), "xkv_latent_stage1");
-    float *pf = c.get<float>(part), *lf = c.get<float>(lse);
-    merge(c, c.get<float>(part1), c.get<float>(lse1), pf, hq * (1 + S2) * dv, (1 + S2) * dv, XKV_F32, &up, mid, s1, b, hq, L, rv, lf,
-          hq * (1 + S2), 1 + S2);
-    check(p_xkv_latent_stage1({q.data_ptr(), (int)w}, nullptr, NO_Q, kv(kT, 0, w), NO_KV, kv(vT, 0, dv), pf + dv, lf + 1, nullptr, 0, nullptr,
-                              nullptr, b, hq, groups, Lt, 1 + S2, 32 * per, nullptr, scale, logit_cap, c.dt, c.stream), "xkv_latent_stage1");
-    const Splits s2{1 + S2, 0, nullptr, nullptr};
-    merge(c, pf, lf, o.data_ptr(), hq * dv, dv, c.dt, nullptr, 0, s2, b, hq, 32 * (1 + S2), dv);   // every row live
+    at::Tensor o;
+    without_gil([&] {
+      Call c(q);
+      const Up up = up_of(vB, hq, c.dt);
+      const int groups = head_groups(hq);
+      const bool shared = vA.data_ptr() == kA.data_ptr() && vA.strides() == kA.strides() && rv == r;
+      Splits s1{scan_splits(c, b, groups, L, ring_rank(r)), 0, nullptr, nullptr};
+      // the tail in at most four splits of whole 32-token blocks, every one of them live; a cap states the count, because the rows
+      // of the shared workspace are one more: row 0 is the merged, up-projected prefix with its log-sum-exp
+      const int blocks = cdiv(Lt, 32), per = cdiv(blocks, 4), S2 = cdiv(blocks, per);
+      const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part1 = c.plan(b * hq * s1.S * rv * 4), lse1 = c.plan(b * hq * s1.S * 4);
+      const int64_t mid = c.plan(rows_first(s1.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
+      const int64_t part = c.plan(b * hq * (1 + S2) * dv * 4), lse = c.plan(b * hq * (1 + S2) * 4);
+      c.alloc();
+      o = at::empty({b, hq, dv}, c.opts);
+      absorb(c, q.data_ptr(), kB, c.get<void>(hi), c.get<void>(lo), b, hq, w, r);
+      check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(kA, 0, r), NO_KV, shared ? kv(kA, 0, r) : kv(vA, 0, rv),
+                                c.get<float>(part1), c.get<float>(lse1), nullptr, 0, nullptr, nullptr, b, hq, groups, L, s1.S, 0, nullptr, scale,
+                                logit_cap, c.dt, c.stream), "xkv_latent_stage1");
+      float *pf = c.get<float>(part), *lf = c.get<float>(lse);
+      merge(c, c.get<float>(part1), c.get<float>(lse1), pf, hq * (1 + S2) * dv, (1 + S2) * dv, XKV_F32, &up, mid, s1, b, hq, L, rv, lf,
+            hq * (1 + S2), 1 + S2);
+      check(p_xkv_latent_stage1({q.data_ptr(), (int)w}, nullptr, NO_Q, kv(kT, 0, w), NO_KV, kv(vT, 0, dv), pf + dv, lf + 1, nullptr, 0, nullptr,
+                                nullptr, b, hq, groups, Lt, 1 + S2, 32 * per, nullptr, scale, logit_cap, c.dt, c.stream), "xkv_latent_stage1");
+      const Splits s2{1 + S2, 0, nullptr, nullptr};
+      merge(c, pf, lf, o.data_ptr(), hq * dv, dv, c.dt, nullptr, 0, s2, b, hq, 32 * (1 + S2), dv);   // every row live
+    });
     return THPVariable_Wrap(o);
   });
 }

@@ -32,3 +32,34 @@ def pytest_collection_modifyitems(config, items):
 @pytest.fixture(scope="session")
 def dev():
     return torch.device("cuda:0")
+
+
+@pytest.fixture(scope="session")
+def shim_lib(tmp_path_factory):
+    import ctypes
+    import subprocess
+
+    from kernel_collections_amd import _lib
+    so = str(tmp_path_factory.mktemp("shim") / "liblaunch_shim.so")
+    subprocess.check_call(["g++", "-O1", "-shared", "-fPIC", "-o", so, os.path.join(ROOT, "tests", "launch_shim.cpp"), "-ldl"])
+    lib = ctypes.CDLL(so)
+    assert lib.shim_init(_lib.LIB_PATH.encode()) == 0
+    return so, lib
+
+
+@pytest.fixture
+def shim(shim_lib):
+    """The native host layer over launch_shim.cpp: yields the shim, whose counters tell what a call did."""
+    import ctypes
+
+    from kernel_collections_amd import _lib
+    so, lib = shim_lib
+    lib.count = lambda name: ctypes.c_int.in_dll(lib, name).value
+    native = _lib.native()
+    for name in ("shim_launches", "shim_locked_calls", "shim_poison", "shim_poisoned"):
+        ctypes.c_int.in_dll(lib, name).value = 0
+    native.init(so)
+    try:
+        yield lib
+    finally:
+        native.init(_lib.LIB_PATH)

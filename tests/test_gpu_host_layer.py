@@ -97,3 +97,46 @@ def test_a_kernels_refusal_is_a_runtime_error(dev):
     with pytest.raises(RuntimeError, match="xkv_latent_stage1 failed: shape outside the built envelope .code -2") as e:
         fr.qAB_no_pe_v1(z(1, 4, 1, 128), z(1, 40, 1056), z(1, 2, 1056, 128))
     assert type(e.value) is RuntimeError
+
+
+def every_call(dev, b=2, L=700, hq=8, hkv=2, r=256, seed=0):
+    """name -> (call, its tensors) for each entry point of the native layer, every operand as it serves it."""
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd.flash_decoding import deepseek_mla, gqa, mla2
+    t = lambda *s, std=1.0, n=0: gen(s, std=std, seed=seed + n).to(dev)
+    q, A, Av = t(b, hq, 128, n=1), t(b, L, r, n=2), t(b, L, r, n=3)
+    B, Bv = t(b, hkv, r, 128, std=r ** -0.5, n=4), t(b, hkv, r, 128, std=r ** -0.5, n=5)
+    K, V = t(b, L, hkv, 128, n=6), t(b, L, hkv, 128, n=7)
+    c, pe, qn, qr, B1 = t(b, L, 1, r, n=8), t(b, L, 1, 64, n=9), t(b, hq, 128, n=10), t(b, hq, 64, n=11), t(b, 1, r, 128, std=r ** -0.5, n=12)
+    kt, vt = t(b, 33, 1, 128, n=13), t(b, 33, 1, 128, n=14)
+    ns, lens = torch.full((b,), 2, dtype=torch.int32, device=dev), torch.tensor([L] + [L // 3] * (b - 1), dtype=torch.int32, device=dev)
+    s = 128 ** -0.5
+    new = lambda: torch.empty_like(q)
+    return {
+        "scores": lambda: fr.qAB_no_pe_v1(q.unsqueeze(2), A, B, sm_scale=s, out_dtype=torch.float32),
+        "rope_scores": lambda: fr.qAB_rope_v1(q.unsqueeze(2), A, B, sm_scale=s, out_dtype=torch.float32),
+        "decode": lambda: fr.gqa_xKV_no_pe(q, A, B, Av, Bv, new(), ns, 2, s),
+        "decode_ragged": lambda: fr.gqa_xKV_no_pe(q, A, B, Av, Bv, new(), ns, 2, s, kv_lens=lens),
+        "rope_decode": lambda: fr.gqa_xKV_rope(q, A, B, A, Bv, new(), ns, 2, s, 5e5),
+        "rope_decode_own_values": lambda: fr.gqa_xKV_rope(q, A, B, Av, Bv, new(), ns, 2, s, 5e5),
+        "gqa": lambda: gqa.decode_attention_fwd(q, K, V, new(), ns, 2, s),
+        "gqa_ragged": lambda: gqa.decode_attention_fwd(q, K, V, new(), ns, 2, s, kv_lens=lens),
+        "v_factorized": lambda: gqa.decode_attention_fwd_v_factorized(q, K, Av, Bv, new(), ns, 2, s),
+        "mla": lambda: mla2.mla_decode_attention_fwd(q_nope(c, q), qr, c, pe, s),
+        "mla_xkv": lambda: mla2.mla_decode_attention_xKV(qn, qr, c, B1, pe, s),
+        "prefix_tail": lambda: deepseek_mla.mla_decode_attention_fwd_pd_sep_xKV(q, A, B1, Av, B1, kt, vt, s),
+    }
+
+
+def q_nope(c, q):
+    return torch.cat([q, q], -1)[..., :c.shape[-1]].contiguous()
+
+
+def test_launches_let_other_threads_run(dev, shim):
+    """No launch of any call is made with the interpreter locked (and every call goes through the native layer)."""
+    for name, call in every_call(dev).items():
+        n = shim.count("shim_launches")
+        call()
+        assert shim.count("shim_launches") > n, name
+        assert shim.count("shim_locked_calls") == 0, name
+    torch.cuda.synchronize()
