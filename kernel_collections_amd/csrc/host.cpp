@@ -18,6 +18,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <array>
 #include <atomic>
 #include <cstdint>
@@ -65,16 +66,20 @@ int num_cus(int device) {
 // workgroups, two rounds on 256 CUs; 10 are one), and 160 workgroups (batch 20) are one round of a chip that is two thirds full
 // where 480 are two full ones.
 int balanced_splits(int64_t batch, int groups, int64_t kv_len, int tile, int per_cu, int cus) {
-  struct Entry { int64_t batch = -1, kv_len = 0; int groups = 0, tile = 0, per_cu = 0, cus = 0, splits = 0; };
+  const int64_t blocks = (kv_len + 31) / 32;   // split lengths are multiples of 32 tokens, and the length counts in those alone
+  // a decode loop has another length at every token: it finds its count here for 32 steps, and the search for the next (a few
+  // microseconds) looks at every length of a split once, not at every number of splits
+  struct Entry { int64_t batch = -1, blocks = 0; int groups = 0, tile = 0, per_cu = 0, cus = 0, splits = 0; };
   static thread_local std::array<Entry, 256> table;
-  size_t h = (size_t)(batch * 1000003 + kv_len) * 31 + groups * 7 + tile * 131 + per_cu;
+  size_t h = (size_t)(batch * 1000003 + blocks) * 31 + groups * 7 + tile * 131 + per_cu;
   Entry& e = table[(h ^ (h >> 8) ^ (h >> 17)) & 255];
-  if (e.batch == batch && e.kv_len == kv_len && e.groups == groups && e.tile == tile && e.per_cu == per_cu && e.cus == cus) return e.splits;
+  if (e.batch == batch && e.blocks == blocks && e.groups == groups && e.tile == tile && e.per_cu == per_cu && e.cus == cus) return e.splits;
   constexpr int XCDS = 8, START = 4;
-  const int64_t blocks = (kv_len + 31) / 32;   // split lengths are multiples of 32 tokens
+  const int64_t most = std::min<int64_t>(blocks, 4LL * per_cu * cus);
   int64_t best = 1, best_cost = INT64_MAX, seen = 0;
-  for (int64_t want = 1; want <= blocks && want <= 4LL * per_cu * cus; ++want) {
-    const int64_t per = (blocks + want - 1) / want, live = (blocks + per - 1) / per;   // splits that hold tokens
+  for (int64_t want = 1, per; want <= most; want = per > 1 ? (blocks + per - 2) / (per - 1) : most + 1) {
+    per = (blocks + want - 1) / want;
+    const int64_t live = (blocks + per - 1) / per;   // splits that hold tokens
     if (live == seen) continue;
     seen = live;
     // clusters of `groups` workgroups (one (sequence, split)) go round-robin over the XCDs, each with cus / XCDS CUs of its own
@@ -84,7 +89,7 @@ int balanced_splits(int64_t batch, int groups, int64_t kv_len, int tile, int per
     if (cost < best_cost) { best = live; best_cost = cost; }
     if (rounds > 2 && batch * live * groups > 8LL * per_cu * cus) break;   // finer only adds starts
   }
-  e = Entry{batch, kv_len, groups, tile, per_cu, cus, (int)best};
+  e = Entry{batch, blocks, groups, tile, per_cu, cus, (int)best};
   return (int)best;
 }
 

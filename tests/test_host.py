@@ -66,3 +66,43 @@ def test_inverse_frequencies_follow_the_base():
     theta.fill_(5e5)
     b = ops.rope_inv_freq(128, theta, torch.device("cpu"))
     assert not torch.equal(a, b) and torch.equal(b, ops.rope_inv_freq(128, 5e5, torch.device("cpu")))
+
+
+def exhaustive_splits(batch, groups, kv_len, tile, per_cu, cus):
+    """The search of balanced_splits over every number of splits."""
+    blocks = -(-kv_len // 32)
+    best, best_cost, seen = 1, 1 << 62, 0
+    for want in range(1, min(blocks, 4 * per_cu * cus) + 1):
+        per = -(-blocks // want)
+        live = -(-blocks // per)
+        if live == seen:
+            continue
+        seen = live
+        rounds = -(-(-(-batch * live // 8) * groups) // (per_cu * (cus // 8)))
+        cost = rounds * (-(-32 * per // tile) + 4)
+        if cost < best_cost:
+            best, best_cost = live, cost
+        if rounds > 2 and batch * live * groups > 8 * per_cu * cus:
+            break
+    return best
+
+
+def test_split_counts_of_a_growing_sequence():
+    """One look-up a step in 31 of 32 steps of a decode loop, and the same counts as the search over every number of splits."""
+    import random
+    import time
+    from kernel_collections_amd import _xkv_host
+    rng = random.Random(3)
+    for _ in range(300):
+        args = (rng.choice([1, 2, 3, 5, 20, 64]), rng.choice([1, 2, 3, 8]), int(2 ** rng.uniform(0, 18)), rng.choice([16, 32, 64]), rng.choice([1, 2, 3]), 256)
+        first = -(-args[2] // 32) * 32 - 31
+        want = exhaustive_splits(*args)
+        for kv_len in (args[2], first, first + 31):      # every length of a 32-token block
+            assert _xkv_host.balanced_splits(args[0], args[1], kv_len, *args[3:]) == want, args
+    best = 1e9
+    for rep in range(5):
+        t0 = time.perf_counter()
+        for i in range(2048):
+            _xkv_host.balanced_splits(1, 1, 131072 + 4096 * rep + i, 64, 2, 256)
+        best = min(best, (time.perf_counter() - t0) / 2048)
+    assert best < 4e-6, best      # 0.26 us; 15.8 with a search at every step
