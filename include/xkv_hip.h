@@ -44,7 +44,7 @@
 extern "C" {
 #endif
 
-#define XKV_ABI_VERSION 6
+#define XKV_ABI_VERSION 7
 
 enum { XKV_F16 = 0, XKV_BF16 = 1, XKV_F32 = 2 };
 

@@ -590,6 +590,11 @@ PyObject* init(PyObject*, PyObject* path) {
   if (!p) return nullptr;
   void* h = dlopen(p, RTLD_NOW | RTLD_LOCAL);
   if (!h) { PyErr_Format(PyExc_RuntimeError, "cannot load %s: %s", p, dlerror()); return nullptr; }
+  const auto version = reinterpret_cast<decltype(&xkv_abi_version)>(dlsym(h, "xkv_abi_version"));
+  if (!version || version() != XKV_ABI_VERSION) {
+    PyErr_Format(PyExc_RuntimeError, "%s has ABI %d, the native host layer is built for %d; rebuild", p, version ? version() : 0, XKV_ABI_VERSION);
+    return nullptr;
+  }
 #define XKV_RESOLVE(name)                                                                  \
   p_##name = reinterpret_cast<decltype(p_##name)>(dlsym(h, #name));                        \
   if (!p_##name) { PyErr_Format(PyExc_RuntimeError, "%s has no " #name, p); return nullptr; }

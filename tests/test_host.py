@@ -106,3 +106,16 @@ def test_split_counts_of_a_growing_sequence():
             _xkv_host.balanced_splits(1, 1, 131072 + 4096 * rep + i, 64, 2, 256)
         best = min(best, (time.perf_counter() - t0) / 2048)
     assert best < 4e-6, best      # 0.26 us; 15.8 with a search at every step
+
+
+def test_a_library_of_another_abi_is_refused(tmp_path):
+    import ctypes
+    import subprocess
+    from kernel_collections_amd import _xkv_host
+    src, so = tmp_path / "old.c", tmp_path / "libold.so"
+    src.write_text("int xkv_abi_version(void) { return 6; }\n")     # without the optional split counts and packed plans of version 7
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)])
+    assert _lib.ABI_VERSION == _lib.lib().xkv_abi_version() == 7
+    assert ctypes.CDLL(str(so)).xkv_abi_version() != _lib.ABI_VERSION
+    with pytest.raises(RuntimeError, match="has ABI 6, the native host layer is built for 7"):
+        _xkv_host.init(str(so))
