@@ -69,6 +69,8 @@ __device__ __forceinline__ f32x4 mfma16k16(_Float16, s16x4r a, s16x4r b, f32x4 c
 constexpr int RING_QD = 2;      // tiles per loader wave in flight in registers (deeper queues only lengthen the start); >= 2
 enum { RING_SCORES = 0, RING_VSHARED = 1, RING_VDISTINCT = 2, RING_VHEADS = 3, RING_VGIVEN = 4 };
 constexpr int RING_DVH = 128;   // head width of the per-head value rows (RING_VHEADS)
+// token stride, in elements, from which a row pair's second row may be out of reach of a 32-bit lane offset
+constexpr int64_t RING_FAR_STRIDE = 1 << 29;
 
 template <int TN, int DN, bool HAS_R, int VMODE, int NHB, int DVW>
 struct RingShape {
@@ -104,7 +106,8 @@ struct RingShape {
 // RING_VGIVEN: no query at all - the scaled scores [b, hq, kv_len] (fp32) are an input, the C rows are the values: softmax
 // and P.V over a value basis of its own, behind a kernel that produced the scores (two-pass fused decode).
 // DN 1024 means eight plain kv heads of 128 side by side in a token row, against compact query rows [b, hq, 128].
-template <typename T, int TN, int NHB, bool LO, int DN, bool HAS_R, int VMODE, int DVW>
+// PAIRS: two 256-wide rows share a load instruction, whose 32-bit lane offset then spans a token stride (RING_FAR_STRIDE).
+template <typename T, int TN, int NHB, bool LO, int DN, bool HAS_R, int VMODE, int DVW, bool PAIRS>
 __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   static_assert(DN != 1024 || (!LO && !HAS_R), "the 1024-wide form is plain per-head keys");
   typedef typename Elem<T>::vec8 vec8;
@@ -123,7 +126,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   static_assert(DN <= 1024 && DVW <= 1024, "a row takes at most two load instructions");
   constexpr int IPR = DN > 512 ? DN / 512 : 1;    // load instructions per C row (1 KiB each; 768-byte rows use 48 lanes)
   constexpr bool CPART = DN == 384;               // a C row fills only part of a load instruction
-  constexpr int CRI = DN == 256 ? 2 : 1, VRI = DVW == 256 ? 2 : 1;   // rows per load instruction: two 512-byte rows share one
+  constexpr int CRI = PAIRS && DN == 256 ? 2 : 1, VRI = PAIRS && DVW == 256 ? 2 : 1;   // rows per load instruction: two 512-byte rows share one
   // waves 4..7 move the tile rows; each brings TN/4 rows of C (and V) and two 16-byte chunks of every RoPE-key row
   constexpr int QD = RING_QD;
   constexpr int RPW = TN / 4;                     // rows per loader wave per tile
@@ -582,10 +585,10 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   }
 }
 
-template <typename T, int TN, int NHB, bool LO, int DN, bool HAS_R, int VMODE, int DVW = 512>
+template <typename T, int TN, int NHB, bool LO, int DN, bool HAS_R, int VMODE, int DVW = 512, bool PAIRS = true>
 static int launch_ring_t(const RingParams& p, hipStream_t st) {
   constexpr int SHM = RingShape<TN, DN, HAS_R, VMODE, NHB, DVW>::shm(LO);
-  auto kern = latent_ring_kernel<T, TN, NHB, LO, DN, HAS_R, VMODE, DVW>;
+  auto kern = latent_ring_kernel<T, TN, NHB, LO, DN, HAS_R, VMODE, DVW, PAIRS>;
   static DynLds lds;
   const int e = ensure_dynamic_lds(lds, reinterpret_cast<const void*>(kern), SHM, true);
   if (e != XKV_OK) return e;
@@ -616,6 +619,10 @@ static int ring_vmode(const RingParams& p, bool vshared) {
 template <typename T>
 static int launch_ring_given_dt(const RingParams& p, hipStream_t st) {
   const int nhb = p.hq <= 16 ? 1 : 2;
+  const bool far = p.sCl >= RING_FAR_STRIDE;   // no other kernel serves given scores: a row an instruction there
+  if (far && p.dn == 256)
+    return nhb == 1 ? launch_ring_t<T, 32, 1, false, 256, false, RING_VGIVEN, 512, false>(p, st)
+                    : launch_ring_t<T, 32, 2, false, 256, false, RING_VGIVEN, 512, false>(p, st);
 #define XKV_RING_GIVEN(NHB, DN) \
   if (nhb == NHB && p.dn == DN) return launch_ring_t<T, 32, NHB, false, DN, false, RING_VGIVEN>(p, st);
   XKV_RING_GIVEN(1, 512) XKV_RING_GIVEN(2, 512) XKV_RING_GIVEN(1, 384) XKV_RING_GIVEN(2, 384) XKV_RING_GIVEN(1, 256) XKV_RING_GIVEN(2, 256)
@@ -680,12 +687,12 @@ static int launch_ring_dt(const RingParams& p, bool vshared, hipStream_t st) {
 bool ring_eligible(const RingParams& p, bool vshared) {
   const int hg = p.hq / p.groups, vm = ring_vmode(p, vshared);
   const bool lo = p.qn_lo != nullptr, r = p.R != nullptr;
+  if (p.sCl >= RING_FAR_STRIDE || (vm == RING_VDISTINCT && p.sVl >= RING_FAR_STRIDE)) return false;
   if (vm == RING_VHEADS) return true;
   if (hg > 32 || vm < 0) return false;
   if ((p.dn == 1024) != (p.heads_in_row == 8)) return false;   // the 1024-wide form is only the eight-heads-in-a-row one
   if (p.dn != 512 && !(p.dn == 1024 && vm == RING_VDISTINCT && !lo) && !((p.dn == 384 || p.dn == 256) && lo)) return false;
   if (r && (p.dr != 64 || vm != RING_VSHARED)) return false;
-  if (p.sCl >= (1 << 29) || (vm == RING_VDISTINCT && p.sVl >= (1 << 29))) return false;   // a row pair's 32-bit lane offset
   if (p.sCl < p.dn || (r && p.sRl < 64) || (vm == RING_VDISTINCT && p.sVl < p.dv)) return false;
   if (vm == RING_VDISTINCT && p.dn == 512 && !lo && p.dv != 512) return false;
   return true;

@@ -275,3 +275,38 @@ def test_merge_of_many_splits_keeps_the_chip_busy(dev):
         merge_c(mid, lo, out, vB, 1, 32)
     one, two = us(lambda: merge_c(part, lse, out, vB, S, 32 * S)), us(rows_first)
     assert one <= 1.5 * two, (one, two)
+
+
+@pytest.mark.parametrize("form", ["heads", "given"])
+@pytest.mark.parametrize("stride,L", [
+    (1 << 31, 5),          # 2^32 bytes: a 32-bit offset between two rows is zero
+    ((1 << 29) - 8, 37),   # the last stride at which two rows share a load instruction
+    (1 << 29, 70),         # one past it: three tiles
+])
+def test_rows_far_apart(dev, form, stride, L):
+    """256-wide rows of a cache whose tokens lie 1 GiB and more apart, against the same rows side by side."""
+    b, hq, hkv, r = 1, 16, 8, 256
+    rows = gen((b, L, r), seed=1)
+    far = torch.empty(stride * (L - 1) + r, dtype=BF, device=dev).as_strided((b, L, r), (8, stride, 1))
+    far.copy_(rows)
+    S, ns = 2, None
+    if form == "heads":        # absorbed keys under plain per-head values
+        q, V = gen((b, hq, r), std=0.1, seed=2), gen((b, L, hkv, 128), seed=3)
+        s = torch.einsum("bhr,blr->bhl", q.double(), rows.double())
+        ref = torch.einsum("bkgl,blkd->bkgd", torch.softmax(s, -1).reshape(b, hkv, -1, L), V.double()).reshape(b, hq, 128)
+        qd, lo, Vd = q.to(dev), torch.zeros_like(q).to(dev), V.to(dev)
+        part, lse = ops.workspaces(b, hq, S, 128, dev)
+        ops.latent_stage1(qd, lo, None, (far, 0, stride, 0, r), None, (Vd, Vd.stride(0), Vd.stride(1), 128, 128), part, lse, None, ns, None,
+                          b, hq, hkv, L, S, 1.0)
+    else:                      # softmax and P.V over given scores
+        n = (L + 3) // 4 * 4
+        s = gen((b, hq, n), std=1.0, dtype=torch.float32, seed=2)
+        ref = torch.softmax(s[..., :L].double(), -1) @ rows.double()
+        kl = torch.tensor([L], dtype=torch.int32, device=dev)
+        part, lse = ops.workspaces(b, hq, S, r, dev)
+        ops.softmax_pv_stage1(s.to(dev), far, part, lse, ns, kl, b, hq, n, S, BF)
+    out = torch.empty(b, hq, ref.shape[-1], dtype=torch.float32, device=dev)
+    kl = torch.tensor([L], dtype=torch.int32, device=dev)
+    ops.merge_stage2(part, lse, out, None, ns, kl, b, hq, hq, n if form == "given" else L, S)
+    # weights rounded to bf16: 2^-9 of values up to 4.5 each, a few of them carry the sum
+    assert max_abs(out, ref) <= 2.0 ** -9 * 8
