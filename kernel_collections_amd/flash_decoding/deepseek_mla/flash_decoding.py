@@ -18,19 +18,20 @@ from kernel_collections_amd import _lib, ops
 from kernel_collections_amd.flash_decoding.mla import stage1_operands
 
 
-def _all_live(n_splits: int, batch: int, device):
-    """(kv_len, num_kv_splits) under which every one of `n_splits` workspace rows counts as live in the merge."""
-    return 32 * n_splits, ops.uniform_splits(batch, n_splits, device)
+def _all_live(n_splits: int) -> int:
+    """The kv_len under which every one of `n_splits` workspace rows counts as live in the merge."""
+    return 32 * n_splits
 
 
 def _stage1_into(q, k_buffer, v_buffer, partial, lse, first_split, n_splits, sm_scale, logit_cap):
-    """Stage 1 of one buffer into rows first_split .. first_split + n_splits - 1 of a shared workspace."""
+    """Stage 1 of one buffer into rows first_split .. first_split + n_splits - 1 of a shared workspace, every one of them live: the
+    workspace has more, so a cap - the length of a split - states their number."""
     batch, num_q_heads, _ = q.shape
     kv_len = k_buffer.shape[1]
     qn, qr, C, R, V, groups, dn, dv = stage1_operands(q, k_buffer, v_buffer)
-    splits = ops.uniform_splits(batch, n_splits, q.device)
-    ops.latent_stage1(qn, None, qr, C, R, V, partial[:, :, first_split:], lse[:, :, first_split:], None, splits, None,
-                      batch, num_q_heads, groups, kv_len, partial.shape[2], float(sm_scale), float(logit_cap))
+    cap = -(-kv_len // (32 * n_splits)) * 32
+    ops.latent_stage1(qn, None, qr, C, R, V, partial[:, :, first_split:], lse[:, :, first_split:], None, None, None,
+                      batch, num_q_heads, groups, kv_len, partial.shape[2], float(sm_scale), float(logit_cap), split_cap=cap)
 
 
 def _tail_splits(decode_kv_len: int, want: int) -> int:
@@ -45,8 +46,7 @@ def mla_decode_attention_fwd(q, k_buffer, v_buffer, sm_scale=1.0, logit_cap=0.0)
     partial, lse = ops.workspaces(batch, num_q_heads, S, dv, q.device)
     _stage1_into(q, k_buffer, v_buffer, partial, lse, 0, S, sm_scale, logit_cap)
     o = torch.empty((batch, num_q_heads, dv), dtype=q.dtype, device=q.device)
-    ops.merge_stage2(partial, lse, o, None, ops.uniform_splits(batch, S, q.device), None, batch, num_q_heads, num_q_heads,
-                     kv_len, S)
+    ops.merge_stage2(partial, lse, o, None, None, None, batch, num_q_heads, num_q_heads, kv_len, S)
     return o
 
 
@@ -62,8 +62,7 @@ def mla_decode_attention_fwd_pd_sep(q, k_buffer, v_buffer, k_buffer_decoded, v_b
     _stage1_into(q, k_buffer, v_buffer, partial, lse, 0, S1, sm_scale, logit_cap)
     _stage1_into(q, k_buffer_decoded, v_buffer_decoded, partial, lse, S1, S2, sm_scale, logit_cap)
     o = torch.empty((batch, num_q_heads, dv), dtype=q.dtype, device=q.device)
-    live_len, live_splits = _all_live(S1 + S2, batch, q.device)
-    ops.merge_stage2(partial, lse, o, None, live_splits, None, batch, num_q_heads, num_q_heads, live_len, S1 + S2)
+    ops.merge_stage2(partial, lse, o, None, None, None, batch, num_q_heads, num_q_heads, _all_live(S1 + S2), S1 + S2)
     return o
 
 
@@ -90,21 +89,19 @@ def mla_decode_attention_fwd_pd_sep_xKV(q, k_A_buffer, k_B_buffer, v_A_buffer, v
     # prefix: q absorbed into k_B (the reference's torch.matmul at :178), scan over k_A / v_A, partials in rank space
     qt_hi, qt_lo = ops.absorb_q(q3, k_B_buffer, want_lo=True)
     S1 = ops.latent_splits(batch, groups, prefill_kv_len, rank, absorbed=True)
-    splits1 = ops.uniform_splits(batch, S1, q.device)
     part1, lse1 = ops.workspaces(batch, num_q_heads, S1, rank_v, q.device)
     shared = v_A.data_ptr() == k_A.data_ptr() and v_A.stride() == k_A.stride() and rank_v == rank
     Cop = (k_A, k_A.stride(0), k_A.stride(1), 0, rank)
     Vop = Cop if shared else (v_A, v_A.stride(0), v_A.stride(1), 0, rank_v)
-    ops.latent_stage1(qt_hi, qt_lo, None, Cop, None, Vop, part1, lse1, None, splits1, None, batch, num_q_heads, groups,
+    ops.latent_stage1(qt_hi, qt_lo, None, Cop, None, Vop, part1, lse1, None, None, None, batch, num_q_heads, groups,
                       prefill_kv_len, S1, float(sm_scale), float(logit_cap))
 
     # final workspace: row 0 = the merged, up-projected prefix with its log-sum-exp; rows 1.. = the tail's splits
     S2 = _tail_splits(decode_kv_len, 4)                      # the reference uses 4 (:189)
     partial, lse = ops.workspaces(batch, num_q_heads, 1 + S2, v_dim, q.device)
-    ops.merge_stage2(part1, lse1, partial[:, :, 0], v_B_buffer, splits1, None, batch, num_q_heads, num_kv_heads,
+    ops.merge_stage2(part1, lse1, partial[:, :, 0], v_B_buffer, None, None, batch, num_q_heads, num_kv_heads,
                      prefill_kv_len, S1, lse_out=lse[:, :, 0])
     _stage1_into(q, k_buffer_decoded, v_buffer_decoded, partial, lse, 1, S2, sm_scale, logit_cap)
     o = torch.empty((batch, num_q_heads, v_dim), dtype=q.dtype, device=q.device)
-    live_len, live_splits = _all_live(1 + S2, batch, q.device)
-    ops.merge_stage2(partial, lse, o, None, live_splits, None, batch, num_q_heads, num_q_heads, live_len, 1 + S2)
+    ops.merge_stage2(partial, lse, o, None, None, None, batch, num_q_heads, num_q_heads, _all_live(1 + S2), 1 + S2)
     return o

@@ -28,18 +28,18 @@ MAX_SPLIT_TOKENS = 128
 MAX_SPLIT_TOKENS_WIDE = 128
 
 
-def _plan(wide, lens, splits, S, batch, groups, kv_len):
+def _plan(wide, lens, splits, S, batch, groups, kv_len, device):
     """(num_kv_splits, cap, split dimension of the workspaces, split plan on the device or None) of a call."""
     floor, per_cu = (MAX_SPLIT_TOKENS_WIDE, 1) if wide else (MAX_SPLIT_TOKENS, 2)
     if not floor:
-        return splits, 0, S, None
+        return ops.as_int32_dev(splits, batch, device), 0, S, None
     if lens is not None:
         return ops.ragged_plan(lens, batch, 1 if wide else groups, kv_len, floor, per_cu)
     S = min(ops.occupancy_splits(batch, 1 if wide else groups, kv_len, tile=32, waves=per_cu), -(-kv_len // floor))
-    return ops.uniform_splits(batch, S, splits.device), 0, S, None
+    return None, 0, S, None
 
 
-def _prep(q, k_buffer, num_kv_splits, max_kv_splits, kv_lens):
+def _prep(q, k_buffer, max_kv_splits, kv_lens):
     assert q.dim() == 3 and k_buffer.dim() == 4
     batch, num_q_heads, head_dim = q.shape
     num_kv_heads = k_buffer.shape[2]
@@ -48,9 +48,8 @@ def _prep(q, k_buffer, num_kv_splits, max_kv_splits, kv_lens):
     assert kv_group_num >= 1 and num_q_heads % num_kv_heads == 0
     assert kv_group_num <= 32, "at most 32 query heads per kv head"
     assert head_dim % 32 == 0, "head_dim must be a multiple of 32"
-    splits = ops.as_int32_dev(num_kv_splits, batch, q.device)
     lens = None if kv_lens is None else ops.as_int32_dev(kv_lens, batch, q.device)
-    return batch, num_q_heads, num_kv_heads, head_dim, int(max_kv_splits), splits, lens
+    return batch, num_q_heads, num_kv_heads, head_dim, int(max_kv_splits), lens
 
 
 def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits, sm_scale=1.0, *, kv_lens=None):
@@ -61,7 +60,7 @@ def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits,
     done = native and native.gqa(q, k_buffer, v_buffer, None, o, sm_scale, kv_lens, MAX_SPLIT_TOKENS_WIDE, MAX_SPLIT_TOKENS)
     if done is not None:
         return done
-    batch, hq, hkv, d, S, splits, lens = _prep(q, k_buffer, num_kv_splits, max_kv_splits, kv_lens)
+    batch, hq, hkv, d, S, lens = _prep(q, k_buffer, max_kv_splits, kv_lens)
     ops.check_16bit(q, k_buffer, v_buffer)
     assert k_buffer.shape[-1] == v_buffer.shape[-1], "head dim of K and V must be the same"
     dv = v_buffer.shape[-1]
@@ -73,7 +72,7 @@ def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits,
     # rows through its LDS ring), so there are hkv times fewer workgroups and a split may be twice as long
     wide = (hkv * d == 1024 and d == 128 and hq <= 32 and k_buffer.stride(2) == d and v_buffer.stride(2) == d
             and k_buffer.stride(1) >= 1024 and v_buffer.stride(1) >= 1024)
-    splits, cap, S, plan = _plan(wide, lens, splits, S, batch, hkv, kv_len)
+    splits, cap, S, plan = _plan(wide, lens, num_kv_splits, S, batch, hkv, kv_len, q.device)
     partial, lse = ops.workspaces(batch, hq, S, dv, q.device, plan)
     ops.latent_stage1(q3, None, None,
                       (k_buffer, k_buffer.stride(0), k_buffer.stride(1), k_buffer.stride(2), d), None,
@@ -91,7 +90,7 @@ def decode_attention_fwd_v_factorized(q, k_buffer, v_A_buffer, v_B_buffer, o, nu
     done = native and native.gqa(q, k_buffer, v_A_buffer, v_B_buffer, o, sm_scale, kv_lens, MAX_SPLIT_TOKENS_WIDE, MAX_SPLIT_TOKENS)
     if done is not None:
         return done
-    batch, hq, hkv, d, S, splits, lens = _prep(q, k_buffer, num_kv_splits, max_kv_splits, kv_lens)
+    batch, hq, hkv, d, S, lens = _prep(q, k_buffer, max_kv_splits, kv_lens)
     ops.check_16bit(q, k_buffer, v_A_buffer, v_B_buffer)
     rv = v_A_buffer.shape[-1]
     assert v_A_buffer.shape[1] == k_buffer.shape[1] and v_B_buffer.shape[1] == hkv and v_B_buffer.shape[2] == rv
@@ -104,7 +103,7 @@ def decode_attention_fwd_v_factorized(q, k_buffer, v_A_buffer, v_B_buffer, o, nu
     wide8 = hkv * d == 1024 and d == 128 and rv in (256, 384, 512) and hq <= 32 and k_buffer.stride(2) == d
     # 512-wide token rows (4 x 128, 2 x 256 ...): the same form, with the block-diagonal query built here
     wide4 = hkv * d == 512 and rv == 512 and hq <= 32 and k_buffer.stride(2) == d
-    splits, cap, S, plan = _plan(wide8 or wide4, lens, splits, S, batch, hkv, kv_len)
+    splits, cap, S, plan = _plan(wide8 or wide4, lens, num_kv_splits, S, batch, hkv, kv_len, q.device)
     partial, lse = ops.workspaces(batch, hq, S, rv, q.device, plan)
     if wide4:
         ops.latent_stage1(ops.blockdiag_q(q3, hkv), None, None,

@@ -55,11 +55,10 @@ def decode_attention_fwd(q, k_buffer, v_buffer, o, sm_scale=1.0, logit_cap=0.0):
     kv_len = k_buffer.shape[1]
     qn, qr, C, R, V, groups, dn, dv = stage1_operands(q, k_buffer, v_buffer)
     S = ops.latent_splits(batch, groups, kv_len, dn)
-    splits = ops.uniform_splits(batch, S, q.device)
     partial, lse = ops.workspaces(batch, num_q_heads, S, dv, q.device)
-    ops.latent_stage1(qn, None, qr, C, R, V, partial, lse, None, splits, None, batch, num_q_heads, groups,
+    ops.latent_stage1(qn, None, qr, C, R, V, partial, lse, None, None, None, batch, num_q_heads, groups,
                       kv_len, S, float(sm_scale), float(logit_cap))
-    ops.merge_stage2(partial, lse, o, None, splits, None, batch, num_q_heads, num_q_heads, kv_len, S)
+    ops.merge_stage2(partial, lse, o, None, None, None, batch, num_q_heads, num_q_heads, kv_len, S)
     return None
 
 

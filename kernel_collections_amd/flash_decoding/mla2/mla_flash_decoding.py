@@ -18,15 +18,14 @@ def _run(q_nope, q_rope, kv_nope, k_rope, sm_scale, q_nope_lo=None, up_proj=None
     kv_len = kv_nope.shape[1]
     groups = ops.head_groups(num_q_heads)
     S = ops.latent_splits(batch, groups, kv_len, width)
-    splits = ops.uniform_splits(batch, S, q_nope.device)
     attn_logits, attn_lse = ops.workspaces(batch, num_q_heads, S, width, q_nope.device)
-    decoding_stage1(q_nope, q_rope, kv_nope, k_rope, attn_logits, attn_lse, splits, S, sm_scale, q_nope_lo=q_nope_lo)
+    decoding_stage1(q_nope, q_rope, kv_nope, k_rope, attn_logits, attn_lse, None, S, sm_scale, q_nope_lo=q_nope_lo)
     if up_proj is None:
         o = torch.empty_like(q_nope)
-        decoding_stage2(attn_logits, attn_lse, o, kv_seq_len=kv_len, num_kv_splits=splits, max_kv_splits=S)
+        decoding_stage2(attn_logits, attn_lse, o, kv_seq_len=kv_len, num_kv_splits=None, max_kv_splits=S)
         return o
     o = torch.empty((batch, num_q_heads, up_proj.shape[-1]), dtype=q_nope.dtype, device=q_nope.device)
-    return ops.merge_stage2(attn_logits, attn_lse, o, up_proj, splits, None, batch, num_q_heads, 1, kv_len, S)
+    return ops.merge_stage2(attn_logits, attn_lse, o, up_proj, None, None, batch, num_q_heads, 1, kv_len, S)
 
 
 def mla_decode_attention_fwd(q_nope, q_rope, kv_nope, k_rope, sm_scale=1.0):

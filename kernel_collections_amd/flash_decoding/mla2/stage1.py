@@ -22,7 +22,7 @@ def decoding_stage1(q_nope, q_rope, kv_nope, k_rope, attn_out, attn_lse, num_kv_
     groups = n_kv * per_kv_groups
     sh_c = kv_nope.stride(2) if per_kv_groups == 1 else 0
     sh_r = k_rope.stride(2) if per_kv_groups == 1 else 0
-    splits = ops.as_int32_dev(num_kv_splits, batch, q_nope.device)
+    splits = None if num_kv_splits is None else ops.as_int32_dev(num_kv_splits, batch, q_nope.device)
     C = (kv_nope, kv_nope.stride(0), kv_nope.stride(1), sh_c, dmodel)
     R = (k_rope, k_rope.stride(0), k_rope.stride(1), sh_r, k_rope.shape[-1])
     ops.latent_stage1(ops._q3(q_nope), None if q_nope_lo is None else ops._q3(q_nope_lo), ops._q3(q_rope), C, R, C, attn_out, attn_lse, None, splits, None,

@@ -8,7 +8,7 @@ import torch
 from kernel_collections_amd import _lib, ops
 
 
-def _common(q, k_A, k_B, num_kv_splits, max_kv_splits):
+def _common(q, k_A, k_B):
     assert q.dim() == 3, "q must be [batch, num_q_heads, head_dim]"
     batch, num_q_heads, head_dim = q.shape
     num_kv_heads = k_B.shape[1]
@@ -19,21 +19,20 @@ def _common(q, k_A, k_B, num_kv_splits, max_kv_splits):
     kv_group_num = num_q_heads // num_kv_heads
     assert kv_group_num >= 1
     assert k_A.shape[-1] % 32 == 0, "rank must be a multiple of 32"
-    splits = ops.as_int32_dev(num_kv_splits, batch, q.device)
-    return batch, num_q_heads, num_kv_heads, head_dim, int(max_kv_splits), splits
+    return batch, num_q_heads, num_kv_heads, head_dim
 
 
 def _lens(kv_lens, batch, device):
     return None if kv_lens is None else ops.as_int32_dev(kv_lens, batch, device)
 
 
-def _plan(lens, batch, groups, kv_len, rank, device):
+def _plan(lens, batch, groups, kv_len, rank):
     """(num_kv_splits, cap, split dimension, plan) that fill the device: the caller's count is a hint (split-K is exact under the
     merge), and 128 splits of one long sequence - the reference scripts' count - would leave half the CUs idle."""
     if lens is not None:
         return ops.ragged_plan(lens, batch, groups, kv_len, 128, 1 if rank in (256, 384, 512) else 2)
     S = ops.latent_splits(batch, groups, kv_len, rank, absorbed=True)
-    return ops.uniform_splits(batch, S, device), 0, S, None
+    return None, 0, S, None
 
 
 def decode_nope(q, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale, kv_lens=None):
@@ -46,7 +45,7 @@ def decode_nope(q, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale
         return done
     assert v_A.shape[1] == k_A.shape[1]
     assert v_B.shape[1] == k_B.shape[1]
-    batch, hq, hkv, d, S, splits = _common(q, k_A, k_B, num_kv_splits, max_kv_splits)
+    batch, hq, hkv, d = _common(q, k_A, k_B)
     ops.check_16bit(q, k_A, k_B, v_A, v_B)
     rank_v = v_A.shape[-1]
     assert rank_v == v_B.shape[2], "Rank mismatch between v_A and v_B"
@@ -57,7 +56,7 @@ def decode_nope(q, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale
     k_A, v_A = ops.as_rows(k_A), ops.as_rows(v_A)
     qt_hi, qt_lo = ops.absorb_q(q3, k_B, want_lo=True)
     groups = ops.head_groups(hq)
-    splits, cap, S, plan = _plan(lens, batch, groups, kv_len, k_A.shape[-1], q.device)
+    splits, cap, S, plan = _plan(lens, batch, groups, kv_len, k_A.shape[-1])
     partial, lse = ops.workspaces(batch, hq, S, rank_v, q.device, plan)
     ops.latent_stage1(qt_hi, qt_lo, None, (k_A, k_A.stride(0), k_A.stride(1), 0, k_A.shape[-1]), None,
                       (v_A, v_A.stride(0), v_A.stride(1), 0, rank_v), partial, lse, None, splits, lens,
@@ -68,7 +67,7 @@ def decode_nope(q, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale
 def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_scale, kv_lens=None):
     """K factorised (absorbed), V plain ``[batch, kv_len, num_kv_heads, head_dim]``."""
     ops.check_splits(num_kv_splits, max_kv_splits, q.shape[0])
-    batch, hq, hkv, d, S, splits = _common(q, k_A, k_B, num_kv_splits, max_kv_splits)
+    batch, hq, hkv, d = _common(q, k_A, k_B)
     ops.check_16bit(q, k_A, k_B, v_buffer)
     assert v_buffer.shape[1] == k_A.shape[1] and v_buffer.shape[2] == hkv
     dv = v_buffer.shape[-1]
@@ -80,7 +79,7 @@ def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_sca
     qt_hi, qt_lo = ops.absorb_q(q3, k_B, want_lo=True)
     # 8 heads of 128 under ranks 256 / 384 / 512: one workgroup serves every kv head of a split
     wide = hkv == 8 and dv == 128 and hq <= 32 and k_A.shape[-1] in (256, 384, 512) and v_buffer.stride(2) == dv
-    splits, cap, S, plan = _plan(lens, batch, 1 if wide else hkv, kv_len, 512 if wide else k_A.shape[-1], q.device)
+    splits, cap, S, plan = _plan(lens, batch, 1 if wide else hkv, kv_len, 512 if wide else k_A.shape[-1])
     partial, lse = ops.workspaces(batch, hq, S, dv, q.device, plan)
     ops.latent_stage1(qt_hi, qt_lo, None, (k_A, k_A.stride(0), k_A.stride(1), 0, k_A.shape[-1]), None,
                       (v_buffer, v_buffer.stride(0), v_buffer.stride(1), v_buffer.stride(2), dv),
@@ -118,7 +117,7 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
             return done
     assert v_A.shape[1] == k_A.shape[1]
     assert v_B.shape[1] == k_B.shape[1]
-    batch, hq, hkv, d, S, splits = _common(q_pe, k_A, k_B, num_kv_splits, max_kv_splits)
+    batch, hq, hkv, d = _common(q_pe, k_A, k_B)
     ops.check_16bit(q_pe, k_A, k_B, v_A, v_B)
     assert d == 128, "the RoPE reconstruction kernels are built for head_dim 128"
     assert hq // hkv <= 16 and k_A.shape[-1] <= 512
@@ -148,13 +147,13 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
         # scores-only kernel is small enough for two workgroups to share a CU
         S1 = ops.occupancy_splits(batch, hkv, kv_len, tile=64 if k_A.shape[-1] <= TWO_PASS_SMALL_RANK else 32,
                                   waves=2 if k_A.shape[-1] == 256 else 1)
-        ops.recon_stage1(q3, k_A, k_B, None, None, None, scores, ops.uniform_splits(batch, S1, q_pe.device), lens, batch, hq,
+        ops.recon_stage1(q3, k_A, k_B, None, None, None, scores, None, lens, batch, hq,
                          hkv, kv_len, S1, float(sm_scale), True, inv, int(pos_offset), None)
         S2 = ops.latent_splits(batch, 1, kv_len, rank_v, absorbed=True)
-        splits2 = ops.uniform_splits(batch, S2, q_pe.device)
         partial, lse = ops.workspaces(batch, hq, S2, rank_v, q_pe.device)
-        ops.softmax_pv_stage1(scores, v_A, partial, lse, splits2, lens, batch, hq, kv_len, S2, q_pe.dtype)
-        return ops.merge_stage2(partial, lse, o, v_B, splits2, lens, batch, hq, hkv, kv_len, S2)
+        ops.softmax_pv_stage1(scores, v_A, partial, lse, None, lens, batch, hq, kv_len, S2, q_pe.dtype)
+        return ops.merge_stage2(partial, lse, o, v_B, None, lens, batch, hq, hkv, kv_len, S2)
+    S, splits = int(max_kv_splits), ops.as_int32_dev(num_kv_splits, batch, q_pe.device)
     partial, lse = ops.workspaces(batch, hq, S, rank_v, q_pe.device)
     ops.recon_stage1(q3, k_A, k_B, v_A, partial, lse, None, splits, lens, batch, hq, hkv, kv_len, S,
                      float(sm_scale), True, inv, int(pos_offset), sin_cos)

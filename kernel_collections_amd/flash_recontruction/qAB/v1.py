@@ -56,8 +56,7 @@ def _scores(q, Ak, Bk, inv_freq, sin_cos, pos_offset, sm_scale, out_dtype):
         n_splits = ops.occupancy_splits(bsz, num_kv_heads, kv_len, tile=64, waves=1)
     else:
         n_splits = ops.occupancy_splits(bsz, num_kv_heads, kv_len, tile=32, waves=1 if rank > 256 else (2 if rank > 128 else 3))
-    splits = ops.uniform_splits(bsz, n_splits, q.device)
-    ops.recon_stage1(q3, Ak, Bk, None, None, None, out, splits, None, bsz, num_heads, num_kv_heads, kv_len,
+    ops.recon_stage1(q3, Ak, Bk, None, None, None, out, None, None, bsz, num_heads, num_kv_heads, kv_len,
                      n_splits, 1.0 if sm_scale is None else float(sm_scale), True, inv_freq, int(pos_offset), sin_cos)
     return out
 

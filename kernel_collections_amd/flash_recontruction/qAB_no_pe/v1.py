@@ -48,9 +48,8 @@ def qAB(q: torch.Tensor, Ak: torch.Tensor, Bk: torch.Tensor, *,
     out = torch.empty((bsz, num_heads, 1, kv_len), dtype=out_dtype, device=q.device)
     groups = ops.head_groups(num_heads)
     n_splits = ops.latent_splits(bsz, groups, kv_len, rank, absorbed=True)
-    splits = ops.uniform_splits(bsz, n_splits, q.device)
     ops.latent_stage1(qt_hi, qt_lo, None, (Ak, Ak.stride(0), Ak.stride(1), 0, rank), None, None,
-                      None, None, out, splits, None, bsz, num_heads, groups, kv_len, n_splits,
+                      None, None, out, None, None, bsz, num_heads, groups, kv_len, n_splits,
                       1.0 if sm_scale is None else float(sm_scale))
     return out
 

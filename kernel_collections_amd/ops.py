@@ -40,7 +40,6 @@ def _cdiv(a: int, b: int) -> int:
 # small cached device constants (no per-call host->device traffic on the hot path)
 # ------------------------------------------------------------------------------------------------
 _inv_freq_cache = {}
-_splits_cache = {}
 
 
 def rope_inv_freq(dim: int, theta: float, device) -> torch.Tensor:
@@ -57,13 +56,10 @@ def rope_inv_freq(dim: int, theta: float, device) -> torch.Tensor:
 
 def uniform_splits(batch: int, n: int, device) -> torch.Tensor:
     """int32 `[batch]` tensor filled with `n` (what the reference builds with torch.ones(...)*128,
-    flash_decoding/mla2/mla_flash_decoding.py:20), cached."""
-    key = (batch, n, device)
-    t = _splits_cache.get(key)
-    if t is None:
-        t = torch.full((batch,), int(n), dtype=torch.int32, device=device)
-        _splits_cache[key] = t
-    return t
+    flash_decoding/mla2/mla_flash_decoding.py:20).  A new one for every caller: one that is kept would be filled on the stream
+    of its first call and read on others that do not wait for it.  The wrappers pass no counts at all (None) where every sequence
+    has the workspaces' number of splits."""
+    return torch.full((batch,), int(n), dtype=torch.int32, device=device)
 
 
 def occupancy_splits(batch: int, groups: int, kv_len: int, tile: int = 64, waves: int = 2) -> int:
@@ -237,8 +233,8 @@ def merge_stage2(partial, lse, out, vB, num_kv_splits, kv_lens, batch, hq, hkv, 
         if mid_lse is None:
             mid_lse = torch.empty((batch, hq), dtype=torch.float32, device=partial.device)
         merge_stage2(partial, lse, mid, None, num_kv_splits, kv_lens, batch, hq, hq, kv_len, max_splits, mid_lse, split_cap, split_plan)
-        one = uniform_splits(batch, 1, partial.device)      # a single row's log-sum-exp is not read
-        return merge_stage2(mid.unsqueeze(2), mid_lse, out, vB, one, None, batch, hq, hkv, 32, 1)
+        # a single row's log-sum-exp is not read
+        return merge_stage2(mid.unsqueeze(2), mid_lse, out, vB, None, None, batch, hq, hkv, 32, 1)
     assert out.stride(-1) == 1
     sl = (0, 0) if lse_out is None else (lse_out.stride(0), lse_out.stride(1))
 

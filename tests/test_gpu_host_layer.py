@@ -140,3 +140,77 @@ def test_launches_let_other_threads_run(dev, shim):
         assert shim.count("shim_launches") > n, name
         assert shim.count("shim_locked_calls") == 0, name
     torch.cuda.synchronize()
+
+
+def general_calls(dev, L):
+    """name -> a call of the wrappers' general path (operands that the native layer declines, or calls that it does not hold)."""
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd.flash_decoding import deepseek_mla, gqa, mla, mla2
+    b, hq, hkv, r = 3, 8, 8, 256
+    t = lambda *s, std=1.0, n=0: gen(s, std=std, seed=n).to(dev)
+    wide = lambda x: torch.empty(*x.shape[:-1], x.shape[-1] + 8, dtype=BF, device=dev)[..., :x.shape[-1]].copy_(x)   # copied by the wrapper
+    q, A, Av, B = wide(t(b, hq, 128, n=1)), t(b, L, r, n=2), t(b, L, r, n=3), t(b, hkv, r, 128, std=r ** -0.5, n=4)
+    K, V, ns = t(b, L, hkv, 128, n=6), t(b, L, hkv, 128, n=7), torch.full((b,), 2, dtype=torch.int32, device=dev)
+    kc, vc, qc, c, pe = t(b, L, 1, 576, n=8), t(b, L, 1, 512, n=9), t(b, hq, 576, std=0.1, n=10), t(b, L, 1, r, n=11), t(b, L, 1, 64, n=12)
+    kt, vt, B1 = t(b, 40, 1, 576, n=13), t(b, 40, 1, 512, n=14), t(b, 1, r, 128, std=r ** -0.5, n=15)
+    qr, k1, v1 = wide(t(b, hq, 64, n=16)), t(b, 70, 1, 128, n=17), t(b, 70, 1, 128, n=18)
+    s, new = 128 ** -0.5, lambda w=128: torch.empty(b, hq, w, dtype=BF, device=dev)
+
+    def cat():
+        o = new(512)
+        mla.decode_attention_fwd(qc, kc, vc, o)
+        return o
+    return {
+        "scores": lambda: fr.qAB_no_pe_v1(q.unsqueeze(2), A, B, sm_scale=s),
+        "rope_scores": lambda: fr.qAB_rope_v1(q.unsqueeze(2), A, B, sm_scale=s),
+        "decode": lambda: fr.gqa_xKV_no_pe(q, A, B, Av, B, new(), ns, 2, s),
+        "k_only": lambda: fr.gqa_xKV_no_pe_k_only(q, A, B, V, new(), ns, 2, s),
+        "rope_decode_own_values": lambda: fr.gqa_xKV_rope(q, A, B, Av, B, new(), ns, 2, s, 5e5),
+        "gqa": lambda: gqa.decode_attention_fwd(q, K, V, new(), ns, 2, s),
+        "mla_concatenated": cat,
+        "one_buffer": lambda: deepseek_mla.mla_decode_attention_fwd(qc, kc, vc),
+        "prefix_tail": lambda: deepseek_mla.mla_decode_attention_fwd_pd_sep(qc, kc, vc, kt, vt),
+        "prefix_tail_xkv": lambda: deepseek_mla.mla_decode_attention_fwd_pd_sep_xKV(q, A, B1, Av, B1, k1, v1, s),
+        "mla": lambda: mla2.mla_decode_attention_fwd(q_nope(c, q), qr, c, pe, s),
+        "mla_xkv": lambda: mla2.mla_decode_attention_xKV(q, qr, c, B1, pe, s),
+    }
+
+
+def test_general_calls_share_nothing_across_streams(dev, monkeypatch):
+    """The first call of a size waits behind other work on its stream; the same call on another stream does not wait for it."""
+    from kernel_collections_amd.flash_recontruction.fused_attention import _fused
+    monkeypatch.setattr(_fused, "TWO_PASS_MIN_TOKENS", 0)
+    for name, call in general_calls(dev, 900).items():
+        ref = call()                     # kernels loaded; a split count of another size
+        torch.cuda.synchronize()
+        one, two = torch.cuda.Stream(), torch.cuda.Stream()
+        calls = general_calls(dev, 3300)[name]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(one):
+            torch.cuda._sleep(20_000_000)        # about 10 ms
+            first = calls()
+        with torch.cuda.stream(two):
+            second = calls()
+        two.synchronize()
+        got = second.clone()
+        torch.cuda.synchronize()
+        assert ref.isfinite().all() and got.isfinite().all(), name
+        assert torch.equal(got, first) and torch.equal(got, calls()), name
+
+
+def test_captured_calls_leave_nothing_behind(dev):
+    """A call of a new size recorded into a graph does not change what the same call computes outside of it, before the graph runs."""
+    for name, call in general_calls(dev, 900).items():
+        call()
+        big = general_calls(dev, 2500)[name]
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            captured = big()
+        eager = big().clone()
+        torch.cuda.synchronize()
+        for _ in range(3):
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(captured, eager), name
+            assert torch.equal(big(), eager), name
