@@ -318,6 +318,8 @@ def check_splits(num_kv_splits, max_kv_splits, batch: int) -> None:
     """What every call with split counts refuses, whatever count it then scans with."""
     if torch.is_tensor(num_kv_splits):
         assert num_kv_splits.numel() == batch, "num_kv_splits must hold one count per sequence"
+    else:
+        int(num_kv_splits)
     if max_kv_splits < 1:
         raise RuntimeError("max_kv_splits must be at least 1")
 

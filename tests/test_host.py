@@ -119,3 +119,14 @@ def test_a_library_of_another_abi_is_refused(tmp_path):
     assert ctypes.CDLL(str(so)).xkv_abi_version() != _lib.ABI_VERSION
     with pytest.raises(RuntimeError, match="has ABI 6, the native host layer is built for 7"):
         _xkv_host.init(str(so))
+
+
+def test_split_hints_of_no_number_are_refused():
+    from kernel_collections_amd.flash_decoding import gqa
+    import kernel_collections_amd.flash_recontruction as fr
+    z = lambda *s: torch.zeros(s, dtype=torch.bfloat16)
+    for ns in (None, [1, 1]):
+        with pytest.raises(TypeError):
+            gqa.decode_attention_fwd(z(2, 4, 128), z(2, 40, 2, 128), z(2, 40, 2, 128), z(2, 4, 128), ns, 1)
+        with pytest.raises(TypeError):
+            fr.gqa_xKV_no_pe(z(2, 4, 128), z(2, 40, 64), z(2, 2, 64, 128), z(2, 40, 64), z(2, 2, 64, 128), z(2, 4, 128), ns, 1, 1.0)
