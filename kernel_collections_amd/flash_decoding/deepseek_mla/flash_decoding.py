@@ -15,7 +15,7 @@ from __future__ import annotations
 import torch
 
 from kernel_collections_amd import _lib, ops
-from kernel_collections_amd.flash_decoding.mla import stage1_operands
+from kernel_collections_amd.flash_decoding.mla import stage1_operands, stage1_splits
 
 
 def _all_live(n_splits: int) -> int:
@@ -41,8 +41,7 @@ def _tail_splits(decode_kv_len: int, want: int) -> int:
 def mla_decode_attention_fwd(q, k_buffer, v_buffer, sm_scale=1.0, logit_cap=0.0):
     batch, num_q_heads, _ = q.shape
     kv_len, dv = k_buffer.shape[1], v_buffer.shape[-1]
-    groups = stage1_operands(q, k_buffer, v_buffer)[5]
-    S = ops.latent_splits(batch, groups, kv_len, k_buffer.shape[-1])
+    S = stage1_splits(batch, kv_len, stage1_operands(q, k_buffer, v_buffer))
     partial, lse = ops.workspaces(batch, num_q_heads, S, dv, q.device)
     _stage1_into(q, k_buffer, v_buffer, partial, lse, 0, S, sm_scale, logit_cap)
     o = torch.empty((batch, num_q_heads, dv), dtype=q.dtype, device=q.device)
@@ -55,8 +54,7 @@ def mla_decode_attention_fwd_pd_sep(q, k_buffer, v_buffer, k_buffer_decoded, v_b
     prefill_kv_len, decode_kv_len = k_buffer.shape[1], k_buffer_decoded.shape[1]
     dv = v_buffer.shape[-1]
     assert v_buffer_decoded.shape[-1] == dv
-    groups = stage1_operands(q, k_buffer, v_buffer)[5]
-    S1 = ops.settled_splits(prefill_kv_len, ops.latent_splits(batch, groups, prefill_kv_len, k_buffer.shape[-1]))
+    S1 = ops.settled_splits(prefill_kv_len, stage1_splits(batch, prefill_kv_len, stage1_operands(q, k_buffer, v_buffer)))
     S2 = _tail_splits(decode_kv_len, 2)                      # the reference uses 2 (:89)
     partial, lse = ops.workspaces(batch, num_q_heads, S1 + S2, dv, q.device)
     _stage1_into(q, k_buffer, v_buffer, partial, lse, 0, S1, sm_scale, logit_cap)

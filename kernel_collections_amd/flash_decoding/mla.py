@@ -50,11 +50,18 @@ def stage1_operands(q, k_buffer, v_buffer):
     return qn, qr, C, R, V, groups, dn, dv
 
 
+def stage1_splits(batch, kv_len, operands) -> int:
+    """The split count for what `stage1_operands` returned."""
+    _, _, _, R, _, groups, dn, _ = operands
+    return ops.latent_splits(batch, groups, kv_len, dn, rope=R[4] if R else 0)
+
+
 def decode_attention_fwd(q, k_buffer, v_buffer, o, sm_scale=1.0, logit_cap=0.0):
     batch, num_q_heads, _ = q.shape
     kv_len = k_buffer.shape[1]
-    qn, qr, C, R, V, groups, dn, dv = stage1_operands(q, k_buffer, v_buffer)
-    S = ops.latent_splits(batch, groups, kv_len, dn)
+    operands = stage1_operands(q, k_buffer, v_buffer)
+    qn, qr, C, R, V, groups, dn, dv = operands
+    S = stage1_splits(batch, kv_len, operands)
     partial, lse = ops.workspaces(batch, num_q_heads, S, dv, q.device)
     ops.latent_stage1(qn, None, qr, C, R, V, partial, lse, None, None, None, batch, num_q_heads, groups,
                       kv_len, S, float(sm_scale), float(logit_cap))

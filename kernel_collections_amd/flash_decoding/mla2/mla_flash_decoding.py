@@ -17,7 +17,7 @@ def _run(q_nope, q_rope, kv_nope, k_rope, sm_scale, q_nope_lo=None, up_proj=None
     batch, num_q_heads, width = q_nope.shape
     kv_len = kv_nope.shape[1]
     groups = ops.head_groups(num_q_heads)
-    S = ops.latent_splits(batch, groups, kv_len, width)
+    S = ops.latent_splits(batch, groups, kv_len, width, absorbed=q_nope_lo is not None, rope=q_rope.shape[-1])
     attn_logits, attn_lse = ops.workspaces(batch, num_q_heads, S, width, q_nope.device)
     decoding_stage1(q_nope, q_rope, kv_nope, k_rope, attn_logits, attn_lse, None, S, sm_scale, q_nope_lo=q_nope_lo)
     if up_proj is None:

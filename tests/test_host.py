@@ -130,3 +130,41 @@ def test_split_hints_of_no_number_are_refused():
             gqa.decode_attention_fwd(z(2, 4, 128), z(2, 40, 2, 128), z(2, 40, 2, 128), z(2, 4, 128), ns, 1)
         with pytest.raises(TypeError):
             fr.gqa_xKV_no_pe(z(2, 4, 128), z(2, 40, 64), z(2, 2, 64, 128), z(2, 40, 64), z(2, 2, 64, 128), z(2, 4, 128), ns, 1, 1.0)
+
+
+@pytest.mark.parametrize("form,ring", [
+    ("mla", True), ("mla_xkv_256", True), ("mla_xkv_384", True), ("mla_xkv_512", True), ("mla_xkv_192", False),
+    ("cat", True), ("cat_288", False), ("one_buffer", True), ("prefix", True)])
+def test_general_path_plans_for_the_kernel_that_runs(form, ring, monkeypatch):
+    """One workgroup a CU and 32-token tiles where the ring kernel serves the call, two and 64 where the register-staged one does."""
+    from kernel_collections_amd import _xkv_host
+    from kernel_collections_amd.flash_decoding import deepseek_mla, mla, mla2
+
+    class Planned(Exception):
+        pass
+
+    def stop(*shape_and_device):
+        raise Planned(shape_and_device[2])
+    monkeypatch.setattr(ops, "workspaces", stop)
+    monkeypatch.setattr(_lib, "require_gpu", lambda t: None)
+    b, hq, L = 8, 16, 65536
+    z = lambda *s: torch.zeros(s, dtype=torch.bfloat16)
+    one = lambda *s: torch.zeros((1,) + s[1:], dtype=torch.bfloat16).expand(*s)
+    k = one(b, L, 1, 288 if form == "cat_288" else 576)
+    if form == "mla":
+        call = lambda: mla2.mla_decode_attention_fwd(z(b, hq, 512), z(b, hq, 64), one(b, L, 1, 512), one(b, L, 1, 64))
+    elif form.startswith("mla_xkv"):
+        r = int(form[-3:])
+        monkeypatch.setattr(ops, "absorb_q", lambda q, B, want_lo: (z(b, hq, r), z(b, hq, r)))
+        call = lambda: mla2.mla_decode_attention_xKV(z(b, hq, 128), z(b, hq, 64), one(b, L, 1, r), z(b, 1, r, 128), one(b, L, 1, 64))
+    elif form.startswith("cat"):
+        w = k.shape[-1] // 9 * 8
+        call = lambda: mla.decode_attention_fwd(z(b, hq, k.shape[-1]), k, k[..., :w], z(b, hq, w))
+    elif form == "one_buffer":
+        call = lambda: deepseek_mla.mla_decode_attention_fwd(z(b, hq, 576), k, k[..., :512])
+    else:
+        call = lambda: deepseek_mla.mla_decode_attention_fwd_pd_sep(z(b, hq, 576), k, k[..., :512], z(b, 32, 1, 576), z(b, 32, 1, 512))
+    want = _xkv_host.balanced_splits(b, 1, L, 32 if ring else 64, 1 if ring else 2, ops.num_cus())
+    with pytest.raises(Planned) as e:
+        call()
+    assert e.value.args[0] == want + (1 if form == "prefix" else 0)
