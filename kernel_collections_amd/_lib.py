@@ -99,18 +99,15 @@ def lib():
     return _lib
 
 
-_ctypes_lib, _native = lib, None
+_native = None
 NATIVE_PATH = os.path.join(_HERE, "_xkv_host.so")
 
 
 def native():
-    """The native host layer (csrc/host.cpp): whole calls - checks, split choice, scratch, every launch - in one.  None while the
-    ctypes binding is replaced by another object (an instrumenting proxy, say): launches then go through that, one by one."""
+    """The native host layer (csrc/host.cpp): whole calls - checks, split choice, scratch, every launch - in one."""
     global _native
-    if lib is not _ctypes_lib:
-        return None
     if _native is None:
-        _ctypes_lib()
+        lib()
         if not os.path.exists(NATIVE_PATH):
             raise RuntimeError(f"{NATIVE_PATH} is missing: build it with `python -m kernel_collections_amd.build`")
         from . import _xkv_host

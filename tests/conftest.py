@@ -56,7 +56,7 @@ def shim(shim_lib):
     so, lib = shim_lib
     lib.count = lambda name: ctypes.c_int.in_dll(lib, name).value
     native = _lib.native()
-    for name in ("shim_launches", "shim_locked_calls", "shim_poison", "shim_poisoned"):
+    for name in ("shim_launches", "shim_stage1", "shim_locked_calls", "shim_poison", "shim_poisoned"):
         ctypes.c_int.in_dll(lib, name).value = 0
     native.init(so)
     try:

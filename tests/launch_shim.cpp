@@ -8,7 +8,7 @@
 static void* real_lib;
 static int (*gil_held)();
 extern "C" {
-int shim_launches, shim_locked_calls, shim_poison, shim_poisoned;
+int shim_launches, shim_stage1, shim_locked_calls, shim_poison, shim_poisoned;
 int shim_init(const char* path) {
   real_lib = dlopen(path, RTLD_NOW | RTLD_LOCAL);
   gil_held = (int (*)())dlsym(RTLD_DEFAULT, "PyGILState_Check");
@@ -20,9 +20,10 @@ template <typename F> static F* real(const char* name) { return (F*)dlsym(real_l
 static void before(bool stage1, void* stream) {
   ++shim_launches;
   if (gil_held()) ++shim_locked_calls;
-  if (!stage1 || !shim_poison) return;
-  real<decltype(xkv_poison_lds)>("xkv_poison_lds")(0x7FFF7FFF, nullptr, stream);   // a NaN as fp16, bf16 and fp32
-  ++shim_poisoned;
+  if (!stage1) return;
+  ++shim_stage1;
+  if (shim_poison && real<decltype(xkv_poison_lds)>("xkv_poison_lds")(0x7FFF7FFF, nullptr, stream) == 0)   // a NaN as fp16, bf16 and fp32
+    ++shim_poisoned;
 }
 #define FORWARD(name, stage1, params, args) \
   extern "C" int name params { before(stage1, stream); return real<decltype(name)>(#name) args; }

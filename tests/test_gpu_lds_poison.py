@@ -2,9 +2,12 @@
 tile has landed there (a wrong wait count, a barrier too few, a register handed on before its load has returned) can still
 pass a parity test when the previous launch left the same rows in the same place.  Here every stage-1 launch is preceded, on
 the same stream, by `xkv_poison_lds`, which leaves a NaN pattern in all 160 KiB of every CU: stale reads then show up as NaNs in
-the output.  The cases are the parity tests of test_gpu_parity.py themselves, one or two per kernel family that tracks its own
-loads (latent_ring, recon_spec, recon_fast, recon_duo) plus the generic kernels, called again under the poisoning binding.
+the output.  Both host layers: the native one over launch_shim.cpp, which poisons before every stage-1 launch of a call, and the
+general one, launch by launch, under a poisoning binding.  The cases are the parity tests of test_gpu_parity.py themselves, one or two per kernel family that tracks its own
+loads (latent_ring, recon_spec, recon_fast, recon_duo) plus the generic kernels, called again.
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -37,12 +40,18 @@ class _Poisoning:
         return call
 
 
-@pytest.fixture
-def poisoned(monkeypatch):
+@pytest.fixture(params=["native", "general"])
+def poisoned(request, monkeypatch):
+    shim = request.getfixturevalue("shim")      # the native layer's launches; calls that it does not hold still go through the binding
+    ctypes.c_int.in_dll(shim, "shim_poison").value = 1
     proxy = _Poisoning(_lib.lib())
     monkeypatch.setattr(_lib, "lib", lambda: proxy)
+    if request.param == "general":
+        monkeypatch.setattr(_lib, "native", lambda: None)
     yield proxy
-    assert proxy.poisoned > 0, "the case launched no stage-1 kernel through the binding"
+    assert proxy.poisoned + shim.count("shim_poisoned") > 0, "the case launched no stage-1 kernel"
+    assert shim.count("shim_poisoned") == shim.count("shim_stage1")
+    assert request.param == "native" or shim.count("shim_launches") == 0
 
 
 def test_poison_is_still_there_for_the_next_kernel(dev):
