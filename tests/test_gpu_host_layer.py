@@ -214,3 +214,57 @@ def test_captured_calls_leave_nothing_behind(dev):
             torch.cuda.synchronize()
             assert torch.equal(captured, eager), name
             assert torch.equal(big(), eager), name
+
+
+def test_calls_on_other_streams_and_threads(dev):
+    """The same calls on a side stream behind other work, and from several threads with a stream each: the eager results, bit for bit."""
+    import threading
+    calls = [every_call(dev, seed=100 * i, L=700 + 333 * i) for i in range(4)]
+    want = [{name: call() for name, call in c.items()} for c in calls]
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(2_000_000)
+        got = {name: call() for name, call in calls[0].items()}
+    side.synchronize()
+    for name, x in got.items():
+        assert torch.equal(x, want[0][name]), name
+    wrong = []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(5):
+                    out = {name: call() for name, call in calls[i].items()}
+                    torch.cuda.current_stream().synchronize()
+                    wrong.extend((i, name) for name, x in out.items() if not torch.equal(x, want[i][name]))
+        except Exception as e:      # noqa: BLE001 - reported by the assertion below
+            wrong.append((i, e))
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong[:5]
+
+
+def test_calls_under_graph_capture(dev):
+    """Each call recorded after one warm-up, replayed three times with new keys in the captured buffers' place."""
+    for name in every_call(dev):
+        q_sets = [every_call(dev, seed=s)[name] for s in (0, 7, 8, 9)]
+        eager = [c() for c in q_sets]
+        live = q_sets[0]
+        tensors = lambda c: [x.cell_contents for x in c.__closure__ if isinstance(x.cell_contents, torch.Tensor) and x.cell_contents.is_floating_point()]
+        static = tensors(live)
+        keep = [[t.clone() for t in tensors(c)] for c in q_sets]
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            out = live()
+        for i in (1, 2, 3):
+            for dst, src in zip(static, keep[i]):
+                dst.copy_(src)
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, eager[i]), (name, i)
+            assert torch.equal(live(), eager[i]), (name, i)      # eager work between the replays
