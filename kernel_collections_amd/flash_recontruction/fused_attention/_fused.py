@@ -89,19 +89,24 @@ def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_sca
 
 # A value basis of its own runs as two passes (scores, then softmax + P.v_A) at these key ranks once the call scans at
 # least TWO_PASS_MIN_TOKENS tokens (batch x kv_len); below, the extra launches cost more than the second row stream of
-# the fused 8-wave kernel (measured crossover: 32768 tokens at every rank).  Key ranks up to 192 have no such fused kernel: two
-# passes from TWO_PASS_MIN_TOKENS_SMALL on (key rank 192, value rank 512, 32 heads, us fused / two passes: 4096 tokens
-# 37.5 / 32.2, 32768 107 / 52, 131072 356 / 109; at 2051 31.4 / 32.3, at 1024 21.3 / 26.7).
+# the fused 8-wave kernel.  Where the two cross depends on the kv heads, each of which rebuilds every token; the line holds the
+# crossings of all but the fewest heads (us fused / two passes, batch 1, key rank 384, value rank 512: 32 heads on 8 kv heads, 16384
+# tokens 44.9 / 46.7, 24576 58.2 / 53.5, 49152 94.4 / 76.0; 16 on 4, 16384 33.9 / 38.2, 49152 62.1 / 55.8; 16 on 2, 49152 45.6 / 47.5,
+# 98304 68.7 / 67.4), and those of the rank pairs without an 8-wave kernel lie lower (512 / 384, 32 on 8: 4096 32.9 / 33.1, 8192 46.4 / 38.8).
 TWO_PASS_KEY_RANKS = (512, 384, 256)
 TWO_PASS_MIN_TOKENS = 49152
+# Key ranks up to 192 have no 8-wave kernel: two passes from this many tokens on, counted for every kv head - the generic kernel fills
+# the device once at 8192 of them, and from there takes a second round (us fused / two passes, key rank 192, value rank 512: 32 heads on
+# 8 kv heads, 1024 tokens 20.8 / 26.1, 2048 29.8 / 28.3, 16384 66.2 / 44.1; 12 on 3, 2048 21.0 / 25.8, 3072 29.4 / 26.6; 16 on 2, 4096
+# 22.6 / 27.9, 5461 31.8 / 31.4; 8 on 1, 8192 24.3 / 29.1, 12288 35.0 / 29.5).
 TWO_PASS_SMALL_RANK = 192
-TWO_PASS_MIN_TOKENS_SMALL = 4096
+TWO_PASS_MIN_TOKENS_SMALL = 9216
 
 
 def _two_pass(rank, tokens, k_B):
     if rank in TWO_PASS_KEY_RANKS:
         return tokens >= TWO_PASS_MIN_TOKENS
-    return rank <= TWO_PASS_SMALL_RANK and tokens >= TWO_PASS_MIN_TOKENS_SMALL and ops._row_ok(k_B)
+    return rank <= TWO_PASS_SMALL_RANK and tokens * k_B.shape[1] >= TWO_PASS_MIN_TOKENS_SMALL and ops._row_ok(k_B)
 
 
 def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale, theta, sin_cos,

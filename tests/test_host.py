@@ -168,3 +168,12 @@ def test_general_path_plans_for_the_kernel_that_runs(form, ring, monkeypatch):
     with pytest.raises(Planned) as e:
         call()
     assert e.value.args[0] == want + (1 if form == "prefix" else 0)
+
+
+@pytest.mark.parametrize("hkv,tokens,two", [
+    (2, 4096, False), (2, 5461, True), (1, 8192, False), (1, 12288, True), (3, 2048, False), (3, 3072, True), (8, 1024, False), (8, 2048, True)])
+def test_two_passes_at_small_key_ranks_where_they_are_faster(hkv, tokens, two):
+    """Both sides as measured: a model of few kv heads fills the device later."""
+    from kernel_collections_amd.flash_recontruction.fused_attention import _fused
+    for rank in (64, 128, 192):
+        assert _fused._two_pass(rank, tokens, torch.zeros(1, hkv, rank, 128, dtype=torch.bfloat16)) == two
