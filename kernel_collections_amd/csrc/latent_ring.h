@@ -12,7 +12,8 @@ struct LatentParams {
   int dn, dr, dv;
   float* partial; float* lse; void* scores; int scores_dtype;
   const int32_t* num_splits; const int32_t* kv_lens;
-  int hq, groups, kv_len, max_splits, total_wg;   // total_wg = groups * (sequence, split) pairs, or * max_splits jobs of a packed plan
+  int hq, groups, kv_len, max_splits;
+  int grid_splits, total_wg;   // total_wg = groups * batch * grid_splits, or groups * max_splits jobs of a packed plan
   int split_cap;   // > 0: no split longer than this many tokens (effective_splits)
   const int32_t* split_plan;   // not null: [0] cap (the cap in force is max(split_cap, it)), [1] jobs, then (sequence, split) pairs
   int heads_in_row;   // 8: C rows are 8 plain kv heads of 128 side by side and qn holds compact rows [b, hq, 128]; else 0

@@ -151,8 +151,8 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   const int wg = xcd_cluster_remap(blockIdx.x, p.groups);   // the kv groups of one (sequence, split) share an L2
   if (wg >= p.total_wg) return;
   const int group = wg % p.groups;
-  int split = (wg / p.groups) % p.max_splits;
-  int b = wg / (p.groups * p.max_splits);
+  int split = (wg / p.groups) % p.grid_splits;
+  int b = wg / (p.groups * p.grid_splits);
   if (p.split_plan) {   // job list: the live (sequence, split) pairs come first in the grid
     const int job = wg / p.groups;
     if (job >= p.split_plan[1]) return;

@@ -13,6 +13,8 @@
 //          ds_read_b64_tr_b16 (4 tokens x 16 features transposed per 16 lanes).
 // When V is the same tensor as C (MLA latent, xKV with a basis shared by K and V) the tile is
 // loaded once and used for both products.
+#include <algorithm>
+
 #include "xkv_common.h"
 #include "latent_ring.h"
 
@@ -50,8 +52,8 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
   const int wg = xcd_cluster_remap(blockIdx.x, p.groups);   // the kv groups of one (sequence, split) share an L2
   if (wg >= p.total_wg) return;
   const int group = wg % p.groups;
-  int split = (wg / p.groups) % p.max_splits;
-  int b = wg / (p.groups * p.max_splits);
+  int split = (wg / p.groups) % p.grid_splits;
+  int b = wg / (p.groups * p.grid_splits);
   if (p.split_plan) {   // job list: the live (sequence, split) pairs come first in the grid
     const int job = wg / p.groups;
     if (job >= p.split_plan[1]) return;
@@ -358,6 +360,13 @@ static int dispatch_latent(const LatentParams& p, bool vshared, hipStream_t st) 
 
 using namespace xkv;
 
+// Splits a sequence gets workgroups for.  Where a cap alone makes the splits of one length, the host knows their number: a workspace
+// with more rows (a prefix scan beside the rows of a tail) then costs no workgroups without tokens.  Such workgroups end at once, but they
+// deal the others out unevenly - 18 rows for 16 splits of 16 sequences left an XCD of 32 CUs with more than 32 jobs, a second round
+// (24 heads, 17377 tokens, 576-wide rows, prefix + tail: 134 us, 94 without them).
+static int grid_splits(const int32_t* num_splits, const int32_t* kv_lens, int kv_len, int max_splits, int cap, const int32_t* plan) {
+  return !num_splits && !kv_lens && !plan && cap > 0 ? std::min(max_splits, cdiv(kv_len, cap)) : max_splits;
+}
 static bool aligned8(int64_t s) { return (s & 7) == 0; }
 static bool ptr16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -403,7 +412,8 @@ extern "C" int xkv_latent_stage1(xkv_q_operand qn, const void* qn_lo, xkv_q_oper
   p.num_splits = num_kv_splits; p.kv_lens = kv_lens;
   p.hq = hq; p.groups = n_kv_groups; p.kv_len = kv_len; p.max_splits = max_splits; p.split_cap = split_cap_tokens;
   p.split_plan = split_plan;
-  p.total_wg = (packed_rows(num_kv_splits, split_plan) ? 1 : batch) * n_kv_groups * max_splits;
+  p.grid_splits = grid_splits(num_kv_splits, kv_lens, kv_len, max_splits, split_cap_tokens, split_plan);
+  p.total_wg = (packed_rows(num_kv_splits, split_plan) ? 1 : batch) * n_kv_groups * p.grid_splits;
   p.sm_scale = sm_scale; p.logit_cap = logit_cap;
   p.heads_in_row = 0;
   const bool vshared = !scores_only && V.ptr == C.ptr && V.stride_b == C.stride_b && V.stride_l == C.stride_l &&
@@ -451,7 +461,8 @@ extern "C" int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, floa
   p.num_splits = num_kv_splits; p.kv_lens = kv_lens;
   p.hq = hq; p.groups = 1; p.kv_len = kv_len; p.max_splits = max_splits; p.split_cap = split_cap_tokens;
   p.split_plan = split_plan;
-  p.total_wg = packed_rows(num_kv_splits, split_plan) ? max_splits : batch * max_splits;
+  p.grid_splits = grid_splits(num_kv_splits, kv_lens, kv_len, max_splits, split_cap_tokens, split_plan);
+  p.total_wg = (packed_rows(num_kv_splits, split_plan) ? 1 : batch) * p.grid_splits;
   p.sm_scale = 1.f; p.logit_cap = 0.f;
   p.heads_in_row = 0;
   return launch_ring_given(p, dtype, (hipStream_t)stream);

@@ -249,26 +249,27 @@ def test_merge_of_many_splits_in_one_launch(dev, dtype, b, hq, hkv, S, live, dv,
     assert max_abs(lo, torch.logsumexp(lse[..., :live].double(), -1)) <= 1e-5
 
 
+def us(call):          # device time: 20 calls in a graph
+    call()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        for _ in range(20):
+            call()
+    ev, best = [torch.cuda.Event(enable_timing=True) for _ in range(2)], 1e9
+    for _ in range(10):
+        ev[0].record()
+        g.replay()
+        ev[1].record()
+        torch.cuda.synchronize()
+        best = min(best, ev[0].elapsed_time(ev[1]) * 50)
+    return best
+
+
 def test_merge_of_many_splits_keeps_the_chip_busy(dev):
     """256 splits, up-projected: one launch that folds the splits in every column block took twice as long as merging the rows first."""
     b, hq, hkv, S, dv, d_out = 1, 32, 8, 256, 512, 128
     part, lse, mid, lo = (torch.randn(s, device=dev) for s in ((b, hq, S, dv), (b, hq, S), (b, hq, 1, dv), (b, hq)))
     vB, out = torch.randn(b, hkv, dv, d_out, device=dev).to(BF), torch.empty(b, hq, d_out, dtype=BF, device=dev)
-
-    def us(call):          # device time: 20 calls in a graph
-        call()
-        g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g):
-            for _ in range(20):
-                call()
-        ev, best = [torch.cuda.Event(enable_timing=True) for _ in range(2)], 1e9
-        for _ in range(10):
-            ev[0].record()
-            g.replay()
-            ev[1].record()
-            torch.cuda.synchronize()
-            best = min(best, ev[0].elapsed_time(ev[1]) * 50)
-        return best
 
     def rows_first():
         merge_c(part, lse, mid, None, S, 32 * S, lo)
@@ -310,3 +311,20 @@ def test_rows_far_apart(dev, form, stride, L):
     ops.merge_stage2(part, lse, out, None, ns, kl, b, hq, hq, n if form == "given" else L, S)
     # weights rounded to bf16: 2^-9 of values up to 4.5 each, a few of them carry the sum
     assert max_abs(out, ref) <= 2.0 ** -9 * 8
+
+
+def test_rows_of_a_tail_cost_the_prefix_scan_nothing(dev):
+    """A prefix scan into a workspace with rows for a tail: workgroups without tokens would deal the others out unevenly."""
+    b, hq, L, S = 16, 24, 17377, 16
+    k, qn, qr = torch.randn(b, L, 1, 576, device=dev).to(BF), torch.randn(b, hq, 512, device=dev).to(BF), torch.randn(b, hq, 64, device=dev).to(BF)
+    C, R = (k, k.stride(0), k.stride(1), 0, 512), (k[..., 512:], k.stride(0), k.stride(1), 0, 64)
+
+    def scan(rows):
+        part, lse = ops.workspaces(b, hq, rows, 512, dev)
+        cap = -(-L // (32 * S)) * 32
+        call = lambda: ops.latent_stage1(qn, None, qr, C, R, C, part, lse, None, None, None, b, hq, 1, L, rows, 0.05, split_cap=cap)
+        t = us(call)
+        return t, part[:, :, :S], lse[:, :, :S]
+    (alone, p0, l0), (beside, p1, l1) = scan(S), scan(S + 2)
+    assert torch.equal(p0, p1) and torch.equal(l0, l1)
+    assert beside <= 1.2 * alone, (beside, alone)      # prefix + tail: 134 us with 18 workgroups a sequence, 94 with 16
