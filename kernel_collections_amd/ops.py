@@ -281,9 +281,11 @@ def capped_splits(kv_len: int, max_kv_splits: int, cap_tokens: int) -> int:
 def ragged_plan(lens, batch: int, groups: int, kv_len: int, floor: int, per_cu: int = 1):
     """Splits of a ragged batch: ``(None, cap, jobs, split plan on the device)``, the plan packed.  The split length is planned on
     the device so that the batch is cut into at most one job per workgroup the chip holds (`per_cu` per CU, `groups` workgroups
-    per job), no shorter than `floor` tokens or a 256th of the longest sequence; `jobs` is the most that can come of it."""
+    per job; in whole rounds up to two jobs a sequence, `ragged_target` in csrc/host.cpp), no shorter than `floor` tokens or a 256th
+    of the longest sequence; `jobs` is the most that can come of it."""
+    from . import _xkv_host
     cap = max(floor, _cdiv(_cdiv(kv_len, 256), 32) * 32)
-    target = max(1, per_cu * num_cus() // groups)
+    target = _xkv_host.ragged_target(batch, groups, per_cu, num_cus())
     jobs = max(target, batch)
     return None, cap, jobs, plan_splits(lens, None, jobs, cap, target)
 

@@ -328,3 +328,17 @@ def test_rows_of_a_tail_cost_the_prefix_scan_nothing(dev):
     (alone, p0, l0), (beside, p1, l1) = scan(S), scan(S + 2)
     assert torch.equal(p0, p1) and torch.equal(l0, l1)
     assert beside <= 1.2 * alone, (beside, alone)      # prefix + tail: 134 us with 18 workgroups a sequence, 94 with 16
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(64, 8, 128), (8, 8, 64), (32, 8, 128)])
+def test_a_long_sequence_among_many_short_ones_is_cut(dev, hq, hkv, d):
+    """As many sequences as a round of workgroups holds jobs: the longest one is not left to one workgroup per kv head."""
+    from kernel_collections_amd.flash_decoding import gqa
+    for b in (64, 256):
+        L = 8192
+        kl = torch.tensor([L] + [64] * (b - 1), dtype=torch.int32, device=dev)
+        q, K = torch.randn(b, hq, d, device=dev).to(BF), torch.randn(1, L, hkv, d, device=dev).to(BF).expand(b, -1, -1, -1)
+        o, ns = torch.empty_like(q), torch.ones(b, dtype=torch.int32, device=dev)
+        many = us(lambda: gqa.decode_attention_fwd(q, K, K, o, ns, 1, 0.1, kv_lens=kl))
+        alone = us(lambda: gqa.decode_attention_fwd(q[:1], K[:1], K[:1], o[:1], ns[:1], 1, 0.1, kv_lens=kl[:1]))
+        assert many <= 4 * alone, (b, many, alone)

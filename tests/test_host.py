@@ -177,3 +177,10 @@ def test_two_passes_at_small_key_ranks_where_they_are_faster(hkv, tokens, two):
     from kernel_collections_amd.flash_recontruction.fused_attention import _fused
     for rank in (64, 128, 192):
         assert _fused._two_pass(rank, tokens, torch.zeros(1, hkv, rank, 128, dtype=torch.bfloat16)) == two
+
+
+@pytest.mark.parametrize("batch,groups,per_cu,jobs", [(1, 1, 1, 256), (32, 1, 1, 256), (128, 1, 1, 256), (129, 1, 1, 512), (64, 8, 2, 128),
+                                                     (65, 8, 2, 192), (3, 300, 1, 6), (5, 512, 2, 10)])
+def test_ragged_batches_get_two_jobs_a_sequence(batch, groups, per_cu, jobs):
+    from kernel_collections_amd import _xkv_host
+    assert _xkv_host.ragged_target(batch, groups, per_cu, 256) == jobs >= 2 * batch
