@@ -26,12 +26,12 @@ def _lens(kv_lens, batch, device):
     return None if kv_lens is None else ops.as_int32_dev(kv_lens, batch, device)
 
 
-def _plan(lens, batch, groups, kv_len, rank):
+def _plan(lens, batch, groups, kv_len, rank, absorbed=True):
     """(num_kv_splits, cap, split dimension, plan) that fill the device: the caller's count is a hint (split-K is exact under the
     merge), and 128 splits of one long sequence - the reference scripts' count - would leave half the CUs idle."""
     if lens is not None:
-        return ops.ragged_plan(lens, batch, groups, kv_len, 128, 1 if rank in (256, 384, 512) else 2)
-    S = ops.latent_splits(batch, groups, kv_len, rank, absorbed=True)
+        return ops.ragged_plan(lens, batch, groups, kv_len, 128, 1 if absorbed and rank in (256, 384, 512) else 2)
+    S = ops.latent_splits(batch, groups, kv_len, rank, absorbed=absorbed)
     return None, 0, S, None
 
 
@@ -79,7 +79,9 @@ def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_sca
     qt_hi, qt_lo = ops.absorb_q(q3, k_B, want_lo=True)
     # 8 heads of 128 under ranks 256 / 384 / 512: one workgroup serves every kv head of a split
     wide = hkv == 8 and dv == 128 and hq <= 32 and k_A.shape[-1] in (256, 384, 512) and v_buffer.stride(2) == dv
-    splits, cap, S, plan = _plan(lens, batch, 1 if wide else hkv, kv_len, 512 if wide else k_A.shape[-1])
+    # Everything else is register-staged: two workgroups per CU and 64-token tiles up to rank 256, one and 32 beyond (us with a plan
+    # for one and 32 / for two and 64: rank 256, 64 heads on 8, batch 32 x 4000 171 / 109, batch 8 x 7001 80 / 54; rank 512 466 / 472, 210 / 218)
+    splits, cap, S, plan = _plan(lens, batch, 1 if wide else hkv, kv_len, 512 if wide else k_A.shape[-1], absorbed=wide or k_A.shape[-1] > 256)
     partial, lse = ops.workspaces(batch, hq, S, dv, q.device, plan)
     ops.latent_stage1(qt_hi, qt_lo, None, (k_A, k_A.stride(0), k_A.stride(1), 0, k_A.shape[-1]), None,
                       (v_buffer, v_buffer.stride(0), v_buffer.stride(1), v_buffer.stride(2), dv),

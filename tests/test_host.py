@@ -184,3 +184,31 @@ def test_two_passes_at_small_key_ranks_where_they_are_faster(hkv, tokens, two):
 def test_ragged_batches_get_two_jobs_a_sequence(batch, groups, per_cu, jobs):
     from kernel_collections_amd import _xkv_host
     assert _xkv_host.ragged_target(batch, groups, per_cu, 256) == jobs >= 2 * batch
+
+
+@pytest.mark.parametrize("hq,hkv,r,tile,per_cu,groups", [
+    (64, 8, 256, 64, 2, 8), (16, 2, 256, 64, 2, 2), (16, 2, 512, 32, 1, 2), (32, 8, 256, 32, 1, 1), (32, 8, 512, 32, 1, 1), (32, 8, 192, 64, 2, 8)])
+def test_k_only_plans_for_the_kernel_that_runs(hq, hkv, r, tile, per_cu, groups, monkeypatch):
+    from kernel_collections_amd import _xkv_host
+    import kernel_collections_amd.flash_recontruction as fr
+
+    class Planned(Exception):
+        pass
+
+    def stop(batch, hq, S, dv, device, plan=None):
+        raise Planned(S)
+    monkeypatch.setattr(ops, "workspaces", stop)
+    monkeypatch.setattr(_lib, "require_gpu", lambda t: None)
+    z = lambda *s: torch.zeros(s, dtype=torch.bfloat16)
+    monkeypatch.setattr(ops, "absorb_q", lambda q, B, want_lo: (z(8, hq, r), z(8, hq, r)))
+    one = lambda *s: torch.zeros((1,) + s[1:], dtype=torch.bfloat16).expand(*s)
+    args = (z(8, hq, 128), one(8, 7001, r), one(8, hkv, r, 128), one(8, 7001, hkv, 128), z(8, hq, 128), torch.ones(8, dtype=torch.int32), 1, 0.1)
+    with pytest.raises(Planned) as e:
+        fr.gqa_xKV_no_pe_k_only(*args)
+    assert e.value.args[0] == _xkv_host.balanced_splits(8, groups, 7001, tile, per_cu, ops.num_cus())
+    plans = []
+    monkeypatch.setattr(ops, "plan_splits", lambda lens, counts, S, floor, target: plans.append((S, target)) or lens)
+    with pytest.raises(Planned) as e:
+        fr.gqa_xKV_no_pe_k_only(*args, kv_lens=torch.full((8,), 7001, dtype=torch.int32))
+    target = _xkv_host.ragged_target(8, groups, per_cu, ops.num_cus())
+    assert plans == [(target, target)] and e.value.args[0] == target
