@@ -154,6 +154,14 @@ struct Splits {
   int64_t rows(int64_t batch, int64_t hq) const { return hq * (jobs ? jobs : batch * S); }   // partial rows of the whole call
 };
 
+// Shortest split, in tokens: 128, where a job's start (about 5 us) is a third of its time, or less for a batch too short to fill the
+// device at that.  u: the split at which it is filled once, or half of it where the merged rows are up-projected (every split adds a
+// partial row to that merge).  The register-staged kernel goes down to its tile of 64.
+int split_floor(int64_t batch, int groups, int64_t kv_len, int per_cu, int cus, bool up) {
+  const int64_t slots = (int64_t)per_cu * cus / (up ? 2 : 1), u = (batch * kv_len * groups + slots - 1) / slots;
+  if (per_cu > 1) return u <= 64 ? 64 : 128;
+  return (int)std::clamp<int64_t>((u + 31) / 32 * 32, up ? 64 : 32, 128);
+}
 // Jobs that a ragged batch is cut into at most: one per workgroup the chip holds, or as many whole rounds as make two a sequence.  With
 // no more jobs than sequences none is cut, and the longest one is the call: 64 sequences, one of 8000 tokens among short ones, 64 heads
 // on 8 kv heads (64 jobs a round) 250 us, with two rounds 40; all of 1000 .. 8000 tokens 299 and 269.  Three or more jobs a sequence
@@ -170,12 +178,14 @@ struct Ragged { int target; int64_t at; };
 Ragged ragged(Call& c, Splits& s, int64_t batch, int groups, int64_t kv_len, int floor, int per_cu) {
   s.cap = std::max<int64_t>(floor, (cdiv(kv_len, 256) + 31) / 32 * 32);
   s.S = cdiv(kv_len, s.cap);
+  // a workgroup per CU even if all are as long: the floor is the plan, without the 4 us of the planning kernel in front of the scan
+  if (batch * s.S * groups <= c.cus) return {0, 0};
   const int target = ragged_target(batch, groups, per_cu, c.cus);
   s.jobs = std::max<int64_t>(target, batch);
   return {target, c.plan((2 + 2 * (int64_t)s.jobs + batch) * 4)};
 }
-void write_plan(const Call& c, Splits& s, const Ragged& r, const at::Tensor& lens, int64_t batch) {
-  s.lens = lens.data_ptr<int32_t>();
+void write_plan(const Call& c, Splits& s, const Ragged& r, int64_t batch) {
+  if (!s.jobs) return;
   s.plan = c.get<int32_t>(r.at);
   check(p_xkv_plan_splits(s.lens, nullptr, batch, s.jobs, s.cap, r.target, s.plan, c.stream), "xkv_plan_splits");
 }
@@ -297,12 +307,15 @@ PyObject* nope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int groups = head_groups(hq), odt = code_any(o);
       Ragged rg{};
       Splits s{0, 0, nullptr, nullptr};
-      if (lens.defined()) rg = ragged(c, s, b, groups, L, 128, ring_rank(r) ? 1 : 2);
+      const int per_cu = ring_rank(r) ? 1 : 2;
+      const bool planned = lens.defined() && b > 1;   // one sequence is cut into the splits of the longest it may be
+      if (planned) rg = ragged(c, s, b, groups, L, split_floor(b, groups, L, per_cu, c.cus, true), per_cu);
       else s.S = scan_splits(c, b, groups, L, ring_rank(r));
+      if (lens.defined()) s.lens = lens.data_ptr<int32_t>();
       const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
       const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
       c.alloc();
-      if (lens.defined()) write_plan(c, s, rg, lens, b);
+      if (planned) write_plan(c, s, rg, b);
       absorb(c, q.data_ptr(), kB, c.get<void>(hi), c.get<void>(lo), b, hq, d, r);
       check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(kA, 0, r), NO_KV, kv(vA, 0, rv), c.get<float>(part),
                                 c.get<float>(lse), nullptr, 0, nullptr, s.lens, b, hq, groups, L, s.n(), s.cap, s.plan, scale, 0.f, c.dt,
@@ -472,16 +485,19 @@ PyObject* gqa(PyObject*, PyObject* const* a, Py_ssize_t n) {
       // 512-wide token rows beside 512-wide value rows: the same form, against a block-diagonal query
       const bool wide4 = fact && hkv * d == 512 && dv == 512 && hq <= 32 && k.stride(2) == d;
       const bool wide = wide8 || wide4;
-      const int floor = wide ? floor_wide : floor_head, per_cu = wide ? 1 : 2, groups = wide ? 1 : (int)hkv;
-      need(floor > 0);
+      const int per_cu = wide ? 1 : 2, groups = wide ? 1 : (int)hkv, longest_floor = wide ? floor_wide : floor_head;
+      need(longest_floor > 0);
+      const int floor = std::min(longest_floor, split_floor(b, groups, L, per_cu, c.cus, fact));
       Ragged rg{};
       Splits s{0, 0, nullptr, nullptr};
-      if (lens.defined()) rg = ragged(c, s, b, groups, L, floor, per_cu);
+      const bool planned = lens.defined() && b > 1;   // one sequence is cut into the splits of the longest it may be
+      if (planned) rg = ragged(c, s, b, groups, L, floor, per_cu);
       else s.S = std::min(balanced_splits(b, groups, L, 32, per_cu, c.cus), cdiv(L, floor));
+      if (lens.defined()) s.lens = lens.data_ptr<int32_t>();
       const int64_t part = c.plan(s.rows(b, hq) * dv * 4), lse = c.plan(s.rows(b, hq) * 4), bd = c.plan(wide4 ? b * hq * 512 * 2 : 0);
       const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, dv) ? rows_bytes(b, hq, dv) : 0);
       c.alloc();
-      if (lens.defined()) write_plan(c, s, rg, lens, b);
+      if (planned) write_plan(c, s, rg, b);
       const void* qp = q.data_ptr();
       if (wide4) {
         check(p_xkv_blockdiag_q(qp, c.get<void>(bd), b, hq, hkv, d, c.dt, c.stream), "xkv_blockdiag_q");
@@ -586,6 +602,11 @@ PyObject* prefix_tail(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// split_floor(batch, groups, kv_len, per_cu, cus, up) -> int
+PyObject* py_split_floor(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 6, [&]() -> PyObject* { return PyLong_FromLong(split_floor(I(a[0]), I(a[1]), I(a[2]), I(a[3]), I(a[4]), I(a[5]))); });
+}
+
 // ragged_target(batch, groups, per_cu, cus) -> int
 PyObject* py_ragged_target(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 4, [&]() -> PyObject* { return PyLong_FromLong(ragged_target(I(a[0]), I(a[1]), I(a[2]), I(a[3]))); });
@@ -620,6 +641,7 @@ PyObject* init(PyObject*, PyObject* path) {
 #define XKV_FAST(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fn)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"init", init, METH_O, nullptr},       XKV_FAST("balanced_splits", py_balanced_splits), XKV_FAST("nope_decode", nope_decode), XKV_FAST("ragged_target", py_ragged_target),
+    XKV_FAST("split_floor", py_split_floor),
     XKV_FAST("nope_scores", nope_scores),  XKV_FAST("rope_decode", rope_decode),            XKV_FAST("rope_scores", rope_scores),
     XKV_FAST("gqa", gqa),                  XKV_FAST("mla", mla),                            XKV_FAST("prefix_tail", prefix_tail),
     {nullptr, nullptr, 0, nullptr}};

@@ -23,19 +23,22 @@ from kernel_collections_amd import _lib, ops
 # workgroup the chip holds).  The caller's own counts miss it on both sides: 32 sequences of 1K .. 128K tokens in 4096-token
 # splits are 315 jobs on 256 CUs (1040 us, planned: 751), 8 of up to 16K are 20 (113 us
 # at no less than 1024 tokens each, planned: 57).
-# At 128 tokens a job's start (about 5 us) is a third of its time.  _WIDE: the all-heads forms, one workgroup per CU.
+# At 128 tokens a job's start (about 5 us) is a third of its time; a batch too short to fill the device at that takes shorter ones
+# (`split_floor` in csrc/host.cpp).  _WIDE: the all-heads forms, one workgroup per CU.
 MAX_SPLIT_TOKENS = 128
 MAX_SPLIT_TOKENS_WIDE = 128
 
 
-def _plan(wide, lens, splits, S, batch, groups, kv_len, device):
+def _plan(wide, lens, splits, S, batch, groups, kv_len, device, up):
     """(num_kv_splits, cap, split dimension of the workspaces, split plan on the device or None) of a call."""
     floor, per_cu = (MAX_SPLIT_TOKENS_WIDE, 1) if wide else (MAX_SPLIT_TOKENS, 2)
     if not floor:
         return ops.as_int32_dev(splits, batch, device), 0, S, None
-    if lens is not None:
-        return ops.ragged_plan(lens, batch, 1 if wide else groups, kv_len, floor, per_cu)
-    S = min(ops.occupancy_splits(batch, 1 if wide else groups, kv_len, tile=32, waves=per_cu), -(-kv_len // floor))
+    groups = 1 if wide else groups
+    floor = min(floor, ops.split_floor(batch, groups, kv_len, per_cu, up))
+    if lens is not None and batch > 1:
+        return ops.ragged_plan(lens, batch, groups, kv_len, floor, per_cu)
+    S = min(ops.occupancy_splits(batch, groups, kv_len, tile=32, waves=per_cu), -(-kv_len // floor))
     return None, 0, S, None
 
 
@@ -72,7 +75,7 @@ def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits,
     # rows through its LDS ring), so there are hkv times fewer workgroups and a split may be twice as long
     wide = (hkv * d == 1024 and d == 128 and hq <= 32 and k_buffer.stride(2) == d and v_buffer.stride(2) == d
             and k_buffer.stride(1) >= 1024 and v_buffer.stride(1) >= 1024)
-    splits, cap, S, plan = _plan(wide, lens, num_kv_splits, S, batch, hkv, kv_len, q.device)
+    splits, cap, S, plan = _plan(wide, lens, num_kv_splits, S, batch, hkv, kv_len, q.device, False)
     partial, lse = ops.workspaces(batch, hq, S, dv, q.device, plan)
     ops.latent_stage1(q3, None, None,
                       (k_buffer, k_buffer.stride(0), k_buffer.stride(1), k_buffer.stride(2), d), None,
@@ -103,7 +106,7 @@ def decode_attention_fwd_v_factorized(q, k_buffer, v_A_buffer, v_B_buffer, o, nu
     wide8 = hkv * d == 1024 and d == 128 and rv in (256, 384, 512) and hq <= 32 and k_buffer.stride(2) == d
     # 512-wide token rows (4 x 128, 2 x 256 ...): the same form, with the block-diagonal query built here
     wide4 = hkv * d == 512 and rv == 512 and hq <= 32 and k_buffer.stride(2) == d
-    splits, cap, S, plan = _plan(wide8 or wide4, lens, num_kv_splits, S, batch, hkv, kv_len, q.device)
+    splits, cap, S, plan = _plan(wide8 or wide4, lens, num_kv_splits, S, batch, hkv, kv_len, q.device, True)
     partial, lse = ops.workspaces(batch, hq, S, rv, q.device, plan)
     if wide4:
         ops.latent_stage1(ops.blockdiag_q(q3, hkv), None, None,

@@ -26,11 +26,12 @@ def _lens(kv_lens, batch, device):
     return None if kv_lens is None else ops.as_int32_dev(kv_lens, batch, device)
 
 
-def _plan(lens, batch, groups, kv_len, rank, absorbed=True):
+def _plan(lens, batch, groups, kv_len, rank, absorbed=True, up=False):
     """(num_kv_splits, cap, split dimension, plan) that fill the device: the caller's count is a hint (split-K is exact under the
     merge), and 128 splits of one long sequence - the reference scripts' count - would leave half the CUs idle."""
-    if lens is not None:
-        return ops.ragged_plan(lens, batch, groups, kv_len, 128, 1 if absorbed and rank in (256, 384, 512) else 2)
+    if lens is not None and batch > 1:
+        per_cu = 1 if absorbed and rank in (256, 384, 512) else 2
+        return ops.ragged_plan(lens, batch, groups, kv_len, ops.split_floor(batch, groups, kv_len, per_cu, up), per_cu)
     S = ops.latent_splits(batch, groups, kv_len, rank, absorbed=absorbed)
     return None, 0, S, None
 
@@ -56,7 +57,7 @@ def decode_nope(q, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale
     k_A, v_A = ops.as_rows(k_A), ops.as_rows(v_A)
     qt_hi, qt_lo = ops.absorb_q(q3, k_B, want_lo=True)
     groups = ops.head_groups(hq)
-    splits, cap, S, plan = _plan(lens, batch, groups, kv_len, k_A.shape[-1])
+    splits, cap, S, plan = _plan(lens, batch, groups, kv_len, k_A.shape[-1], up=True)
     partial, lse = ops.workspaces(batch, hq, S, rank_v, q.device, plan)
     ops.latent_stage1(qt_hi, qt_lo, None, (k_A, k_A.stride(0), k_A.stride(1), 0, k_A.shape[-1]), None,
                       (v_A, v_A.stride(0), v_A.stride(1), 0, rank_v), partial, lse, None, splits, lens,

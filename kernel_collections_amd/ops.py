@@ -278,13 +278,23 @@ def capped_splits(kv_len: int, max_kv_splits: int, cap_tokens: int) -> int:
     return max(int(max_kv_splits), _cdiv(kv_len, cap_tokens)) if cap_tokens else int(max_kv_splits)
 
 
+def split_floor(batch: int, groups: int, kv_len: int, per_cu: int, up: bool) -> int:
+    """Shortest split in tokens (`split_floor` in csrc/host.cpp); `up`: the merged rows are up-projected."""
+    from . import _xkv_host
+    return _xkv_host.split_floor(batch, groups, kv_len, per_cu, num_cus(), up)
+
+
 def ragged_plan(lens, batch: int, groups: int, kv_len: int, floor: int, per_cu: int = 1):
-    """Splits of a ragged batch: ``(None, cap, jobs, split plan on the device)``, the plan packed.  The split length is planned on
+    """Splits of a ragged batch: ``(None, cap, jobs, split plan on the device)``, the plan packed - or ``(None, cap, splits, None)`` for
+    a batch that fits the device at the shortest splits.  The split length is planned on
     the device so that the batch is cut into at most one job per workgroup the chip holds (`per_cu` per CU, `groups` workgroups
     per job; in whole rounds up to two jobs a sequence, `ragged_target` in csrc/host.cpp), no shorter than `floor` tokens or a 256th
     of the longest sequence; `jobs` is the most that can come of it."""
     from . import _xkv_host
     cap = max(floor, _cdiv(_cdiv(kv_len, 256), 32) * 32)
+    S = _cdiv(kv_len, cap)
+    if batch * S * groups <= num_cus():      # a workgroup per CU even if all are as long: the floor is the plan
+        return None, cap, S, None
     target = _xkv_host.ragged_target(batch, groups, per_cu, num_cus())
     jobs = max(target, batch)
     return None, cap, jobs, plan_splits(lens, None, jobs, cap, target)

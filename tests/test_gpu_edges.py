@@ -339,6 +339,9 @@ def test_a_long_sequence_among_many_short_ones_is_cut(dev, hq, hkv, d):
         kl = torch.tensor([L] + [64] * (b - 1), dtype=torch.int32, device=dev)
         q, K = torch.randn(b, hq, d, device=dev).to(BF), torch.randn(1, L, hkv, d, device=dev).to(BF).expand(b, -1, -1, -1)
         o, ns = torch.empty_like(q), torch.ones(b, dtype=torch.int32, device=dev)
+        kl64 = torch.full_like(kl, 64)
         many = us(lambda: gqa.decode_attention_fwd(q, K, K, o, ns, 1, 0.1, kv_lens=kl))
         alone = us(lambda: gqa.decode_attention_fwd(q[:1], K[:1], K[:1], o[:1], ns[:1], 1, 0.1, kv_lens=kl[:1]))
-        assert many <= 4 * alone, (b, many, alone)
+        short = us(lambda: gqa.decode_attention_fwd(q, K, K, o, ns, 1, 0.1, kv_lens=kl64))
+        # one call for both costs no more than twice the two calls; left whole, the long one took 250 us beside 40 + 30
+        assert many <= 2 * (alone + short), (b, many, alone, short)

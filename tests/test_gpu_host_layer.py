@@ -268,3 +268,33 @@ def test_calls_under_graph_capture(dev):
             torch.cuda.synchronize()
             assert torch.equal(out, eager[i]), (name, i)
             assert torch.equal(live(), eager[i]), (name, i)      # eager work between the replays
+
+
+@pytest.mark.parametrize("path", ["native", "general"])
+@pytest.mark.parametrize("L,lens", [(900, [0]), (900, [1]), (900, [777]), (70000, [69999]), (900, [0, 900, 31]), (9000, [33, 8999, 0, 4096])])
+def test_ragged_batches_with_and_without_a_plan(dev, path, L, lens):
+    """One sequence, a batch that fits the device at the shortest splits, a planned one - each sequence as alone, none as zeros."""
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd.flash_decoding import gqa
+    b, hq, r = len(lens), 16, 256
+    kl = torch.tensor(lens, dtype=torch.int32, device=dev)
+    t = lambda *s, std=1.0, n=0: gen(s, std=std, seed=n).to(dev)
+    q = t(b, hq, 128, n=1)
+    if path == "general":
+        q = torch.empty(b, hq, 136, dtype=BF, device=dev)[..., :128].copy_(q)
+    ns, new = torch.ones(b, dtype=torch.int32, device=dev), lambda n: torch.full((n, hq, 128), float("nan"), dtype=BF, device=dev)
+    for hkv in (8, 2):
+        K, V, A, vA = t(b, L, hkv, 128, n=2), t(b, L, hkv, 128, n=3), t(b, L, r, n=4), t(b, L, r, n=5)
+        B, vB = t(b, hkv, r, 128, std=r ** -0.5, n=6), t(b, hkv, r, 128, std=r ** -0.5, n=7)
+        for name, call in {
+            "gqa": lambda s, n, l: gqa.decode_attention_fwd(q[s], K[s, :n], V[s, :n], new(len(l) if l is not None else 1), ns[s], 1, 0.1, kv_lens=l),
+            "v_factorized": lambda s, n, l: gqa.decode_attention_fwd_v_factorized(q[s], K[s, :n], vA[s, :n], vB[s], new(len(l) if l is not None else 1), ns[s], 1, 0.1, kv_lens=l),
+            "decode": lambda s, n, l: fr.gqa_xKV_no_pe(q[s], A[s, :n], B[s], vA[s, :n], vB[s], new(len(l) if l is not None else 1), ns[s], 1, 0.1, kv_lens=l),
+            "k_only": lambda s, n, l: fr.gqa_xKV_no_pe_k_only(q[s], A[s, :n], B[s], V[s, :n], new(len(l) if l is not None else 1), ns[s], 1, 0.1, kv_lens=l),
+        }.items():
+            got = call(slice(0, b), L, kl)
+            for i, n in enumerate(lens):
+                if n == 0:
+                    assert (got[i] == 0).all(), (name, hkv)
+                else:
+                    check_out(got[i], call(slice(i, i + 1), n, None)[0], f"{name} {hkv} sequence {i}")

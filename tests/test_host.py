@@ -212,3 +212,13 @@ def test_k_only_plans_for_the_kernel_that_runs(hq, hkv, r, tile, per_cu, groups,
         fr.gqa_xKV_no_pe_k_only(*args, kv_lens=torch.full((8,), 7001, dtype=torch.int32))
     target = _xkv_host.ragged_target(8, groups, per_cu, ops.num_cus())
     assert plans == [(target, target)] and e.value.args[0] == target
+
+
+@pytest.mark.parametrize("batch,groups,kv_len,per_cu,up,floor", [
+    (1, 1, 599, 1, False, 32), (8, 1, 1295, 1, False, 64), (8, 1, 2500, 1, False, 96), (32, 1, 1295, 1, False, 128),    # all heads a workgroup
+    (1, 1, 5000, 1, True, 64), (8, 1, 1295, 1, True, 96), (3, 1, 5000, 1, True, 128),                                   # ... and up-projected
+    (1, 2, 5000, 2, False, 64), (8, 2, 2500, 2, False, 128), (3, 2, 1295, 2, True, 64), (1, 2, 12000, 2, True, 128)])    # register-staged
+def test_short_batches_are_cut_shorter(batch, groups, kv_len, per_cu, up, floor):
+    """The fastest of 32, 64, 96, 128 and 256 tokens as measured, within 3 %."""
+    from kernel_collections_amd import _xkv_host
+    assert _xkv_host.split_floor(batch, groups, kv_len, per_cu, 256, up) == floor == ops.split_floor(batch, groups, kv_len, per_cu, up)
