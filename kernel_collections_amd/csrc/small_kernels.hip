@@ -285,12 +285,13 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(
 // head, dv 512, 6.4 us for 32 heads on 8 or 1 kv heads (rows + up-projection at 256 splits: 12.5 us, one kernel that did both
 // 20 - 21.7); 8 splits of 256, 4.7 us (7.0); 16 x 32 heads, 2 splits of 512, 8.6 us (11.6).
 //
-// SPREAD: many splits on a chip that is not full (launch_merge): one head per workgroup, its splits dealt out among groups of threads
-// as in merge_rows_kernel.  256 splits of 512, 32 heads, d_out 128: 12.6 us (26.4 with a thread folding all splits of its packet).
+// MANY_LOOP: many splits on a chip that the heads fill (launch_merge): a workgroup folds once for several column blocks.  MANY_SPREAD: on
+// one that is not full: one head per workgroup, its splits dealt out among groups of threads as in merge_rows_kernel.  256 splits of 512, 32 heads, d_out 128: 12.6 us (26.4 with a thread folding all splits of its packet).
 constexpr int MERGE_CB = 64;       // columns per workgroup: whole 128-byte lines of a vB row
 constexpr int MERGE_UP_T = 512;
+enum { MANY_LOOP = 1, MANY_SPREAD = 2 };
 constexpr int MERGE_ROWS_FLOATS = 49152;   // partial values a workgroup folds in every column block at most; measured in host.cpp
-template <typename O, typename TB, int RPT, bool SPREAD>
+template <typename O, typename TB, int RPT, int MANY>
 __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     const float* __restrict__ partial, const float* __restrict__ lse, O* __restrict__ out,
     const TB* __restrict__ vB, int64_t sVb, int64_t sVh, int64_t sVr, int d_out,
@@ -298,7 +299,7 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     int hq, int hkv, int kv_len, int max_splits, int dv, int64_t sOb, int64_t sOh, int hpw,
     float* __restrict__ lse_out, int64_t sLb, int64_t sLh, int split_cap, const int32_t* __restrict__ split_plan) {
   typedef typename Elem<TB>::vec8 vec8;
-  extern __shared__ float merged[];               // [hpw][dv]; SPREAD: then a packet, a maximum and a sum of every thread
+  extern __shared__ float merged[];               // [hpw][dv]; MANY_SPREAD: then a packet, a maximum and a sum of every thread
   __shared__ float tot[4][4 * MERGE_CB];          // [quarter of the row groups][4 heads x 64 columns]
   const int hfirst = blockIdx.x * hpw, kh = hfirst / (hq / hkv), b = blockIdx.y;
   int c0 = blockIdx.z * MERGE_CB;
@@ -329,7 +330,7 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     for (int e = 0; e < P; ++e) merged[gi * dv + c + e] = a.acc[e] * inv;
     if (lse_out && c == 0 && blockIdx.z == 0) lse_out[b * sLb + (hfirst + gi) * sLh] = a.m + __logf(a.l);
   };
-  auto merge_shared = [&](auto tag) {             // SPREAD: head hfirst, its splits dealt out among MERGE_UP_T / (dv / P) groups
+  auto merge_shared = [&](auto tag) {             // MANY_SPREAD: head hfirst, its splits dealt out among MERGE_UP_T / (dv / P) groups
     constexpr int P = decltype(tag)::value;
     float* red = merged + dv;
     float* ml = red + MERGE_UP_T * P;
@@ -362,7 +363,7 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     if (lse_out && c == 0 && blockIdx.z == 0) lse_out[b * sLb + hfirst * sLh] = M + __logf(l);
   };
   const bool vec = (dv & 3) == 0 && (reinterpret_cast<uintptr_t>(partial) & 15) == 0;
-  if constexpr (SPREAD) {
+  if constexpr (MANY == MANY_SPREAD) {
     if (vec) merge_shared(std::integral_constant<int, 4>());
     else merge_shared(std::integral_constant<int, 1>());
   } else if (vec) {
@@ -413,6 +414,7 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
       }
       __syncthreads();            // tot is reused by the next four heads, or the next columns
     }
+    if constexpr (!MANY) return;
     c0 += gridDim.z * MERGE_CB;
     if (c0 >= d_out) return;
     load_w();
@@ -470,11 +472,11 @@ static int launch_merge(const float* partial, const float* lse, void* out, const
   if (many) z = (int)std::min<int64_t>(z, cdiv(256, std::min<int64_t>(256, (int64_t)(hq / hpw) * batch)));
   const dim3 grid(hq / hpw, batch, z);
   const size_t shm = ((size_t)hpw * dv + (spread ? MERGE_UP_T * 6 : 0)) * sizeof(float);
-#define XKV_MERGE_UP(RPT, SPREAD)                                                                                                      \
-  merge_up_kernel<O, TB, RPT, SPREAD><<<grid, dim3(MERGE_UP_T), shm, st>>>(partial, lse, (O*)out, (const TB*)vB, sVb, sVh, sVr, d_out, ns, kl, \
+#define XKV_MERGE_UP(RPT, MANY)                                                                                                      \
+  merge_up_kernel<O, TB, RPT, MANY><<<grid, dim3(MERGE_UP_T), shm, st>>>(partial, lse, (O*)out, (const TB*)vB, sVb, sVh, sVr, d_out, ns, kl, \
                                                          hq, hkv, kv_len, max_splits, dv, sOb, sOh, hpw, lse_out, sLb, sLh, split_cap, split_plan)
-  if (dv <= 256) { if (spread) XKV_MERGE_UP(4, true); else XKV_MERGE_UP(4, false); }
-  else { if (spread) XKV_MERGE_UP(8, true); else XKV_MERGE_UP(8, false); }
+  if (dv <= 256) { if (spread) XKV_MERGE_UP(4, MANY_SPREAD); else if (many) XKV_MERGE_UP(4, MANY_LOOP); else XKV_MERGE_UP(4, 0); }
+  else { if (spread) XKV_MERGE_UP(8, MANY_SPREAD); else if (many) XKV_MERGE_UP(8, MANY_LOOP); else XKV_MERGE_UP(8, 0); }
 #undef XKV_MERGE_UP
   return launch_status();
 }
