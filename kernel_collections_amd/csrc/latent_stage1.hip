@@ -33,7 +33,39 @@ __device__ __forceinline__ V8 tr_operand(const void* p0, const void* p1) {
   return __builtin_bit_cast(V8, r);
 }
 
-template <typename T, int NHB, int TN, int NVB_MAX, int NPK_C, int NPK_R, int NPK_V, bool VSHARED, bool SCORES_ONLY>
+// Where a workgroup's results go: the partial row of its first head, and the rows from head to head.  Calls with a plan or fewer workgroups
+// than workspace rows work all of it out once more, from parameters read again (1155 us at the shape below with the workgroup's place held
+// through the scan, 1149 without).
+struct SplitRows { int64_t row; int per_head, dv; float* partial; float* lse; };
+template <bool PLAIN> __device__ __forceinline__ SplitRows split_rows(const LatentParams& p, int b, int split, int h0) {
+  if constexpr (PLAIN) {
+    return {((int64_t)b * p.hq + h0) * p.max_splits + split, p.max_splits, p.dv, p.partial, p.lse};
+  } else {
+    typedef const __attribute__((address_space(4))) LatentParams* Params;
+    Params q = (Params)__builtin_amdgcn_kernarg_segment_ptr();
+    int id = blockIdx.x;
+    asm volatile("" : "+s"(q), "+s"(id));
+    const int32_t* lens = q->kv_lens;
+    const int32_t* counts = q->num_splits;
+    const int32_t* plan = q->split_plan;
+    const int groups = q->groups, grid_splits = q->grid_splits, hq = q->hq, max_splits = q->max_splits, cap = q->split_cap;
+    const int wg = xcd_cluster_remap(id, groups), first = wg % groups * (hq / groups);
+    int at = (wg / groups) % grid_splits, seq = wg / (groups * grid_splits);
+    if (plan) {
+      seq = plan[2 + 2 * (wg / groups)];
+      at = plan[3 + 2 * (wg / groups)];
+    }
+    const PartialRows rows = partial_rows(seq, hq, max_splits, [&] {
+      const int L = lens ? lens[seq] : q->kv_len;
+      return live_splits(L, effective_splits(L, asked_splits(counts, seq, max_splits, cap), split_cap_in_force(cap, plan)), max_splits);
+    }, counts, plan);
+    return {rows.base + (int64_t)first * rows.per_head + at, rows.per_head, q->dv, q->partial, q->lse};
+  }
+}
+
+// PLAIN: no plan, and a workgroup for every workspace row.  The scan has no scalar registers to spare: what only the other calls need
+// slows it down (32 x 15558 tokens, 8 heads, values of rank 192: 1165 us for one kernel, 1137 for PLAIN), so those have a kernel of their own.
+template <typename T, int NHB, int TN, int NVB_MAX, int NPK_C, int NPK_R, int NPK_V, bool VSHARED, bool SCORES_ONLY, bool PLAIN>
 __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p) {
   typedef typename Elem<T>::vec8 vec8;
   constexpr int HB = 16 * NHB;       // head rows held (zero padded)
@@ -52,9 +84,9 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
   const int wg = xcd_cluster_remap(blockIdx.x, p.groups);   // the kv groups of one (sequence, split) share an L2
   if (wg >= p.total_wg) return;
   const int group = wg % p.groups;
-  int split = (wg / p.groups) % p.grid_splits;
-  int b = wg / (p.groups * p.grid_splits);
-  if (p.split_plan) {   // job list: the live (sequence, split) pairs come first in the grid
+  int split = (wg / p.groups) % (PLAIN ? p.max_splits : p.grid_splits);
+  int b = wg / (p.groups * (PLAIN ? p.max_splits : p.grid_splits));
+  if (!PLAIN && p.split_plan) {   // job list: the live (sequence, split) pairs come first in the grid
     const int job = wg / p.groups;
     if (job >= p.split_plan[1]) return;
     b = p.split_plan[2 + 2 * job];
@@ -62,7 +94,8 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
   }
 
   const int L = p.kv_lens ? p.kv_lens[b] : p.kv_len;
-  const int ns = effective_splits(L, asked_splits(p.num_splits, b, p.max_splits, p.split_cap), split_cap_in_force(p.split_cap, p.split_plan));
+  const int ns = effective_splits(L, asked_splits(p.num_splits, b, p.max_splits, p.split_cap),
+                                  PLAIN ? p.split_cap : split_cap_in_force(p.split_cap, p.split_plan));
   int start, end;
   split_bounds(L, ns, split, start, end);
   if (end <= start) return;
@@ -83,14 +116,6 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
   T* p_lds = reinterpret_cast<T*>(s_lds + HB * LDS_S);
   float* alpha_lds = reinterpret_cast<float*>(p_lds + HB * LDP);
   float* ml_lds = alpha_lds + HB;
-  // [0] partial row of head h0, [1] rows from head to head: found here and kept in the LDS, since the scan has no scalar registers to
-  // spare for what the epilogue needs (held there: 2.3 % of 580 us, 32 ragged sequences of up to 14K tokens, 8 heads, values of rank 192)
-  int64_t* row_lds = reinterpret_cast<int64_t*>(ml_lds + 2 * HB);
-  if (!SCORES_ONLY && tid == 0) {
-    const PartialRows rows = partial_rows(b, p.hq, p.max_splits, [&] { return live_splits(L, ns, p.max_splits); }, p.num_splits, p.split_plan);
-    row_lds[0] = rows.base + (int64_t)h0 * rows.per_head + split;
-    row_lds[1] = rows.per_head;
-  }
 
   // ---- query rows -> LDS ([qn | qr], zero rows above hg) -----------------------------------
   {
@@ -310,6 +335,7 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
   if (SCORES_ONLY) return;
 
   // ---- epilogue: normalise, write partial + lse --------------------------------------------
+  const SplitRows out = split_rows<PLAIN>(p, b, split, h0);
   if (ssub == 0) { ml_lds[2 * srow] = m_run; ml_lds[2 * srow + 1] = l_run; }
   __syncthreads();
 #pragma unroll
@@ -318,12 +344,12 @@ __global__ __launch_bounds__(256) void latent_stage1_kernel(const LatentParams p
     if (hrow < hg) {
       const float m = ml_lds[2 * hrow], l = ml_lds[2 * hrow + 1];
       const float inv = 1.f / l;
-      const int64_t ph = row_lds[0] + hrow * row_lds[1];
-      float* dst = p.partial + ph * p.dv + vcol0 + 4 * g4;
+      const int64_t ph = out.row + (int64_t)hrow * out.per_head;
+      float* dst = out.partial + ph * out.dv + vcol0 + 4 * g4;
 #pragma unroll
       for (int mb = 0; mb < NVB_MAX; ++mb)
         if (mb < nvb) *reinterpret_cast<f32x4*>(dst + mb * 16) = acc[mb][hb] * inv;
-      if (wave == 0 && g4 == 0) p.lse[ph] = m + __logf(l);
+      if (wave == 0 && g4 == 0) out.lse[ph] = m + __logf(l);
     }
   }
 }
@@ -343,11 +369,13 @@ static int launch_latent(const LatentParams& p, hipStream_t st) {
   size_t shm = (size_t)TN * ldc * 2;
   if (!VSHARED && !SCORES_ONLY) shm += (size_t)TN * ldv * 2;
   shm += (size_t)HB * ldc * 2 * (p.qn_lo ? 2 : 1);
-  shm += (size_t)HB * (TN + 4) * 4 + (size_t)HB * (TN + 8) * 2 + HB * 4 + HB * 8 + 16;
+  shm += (size_t)HB * (TN + 4) * 4 + (size_t)HB * (TN + 8) * 2 + HB * 4 + HB * 8;
   if (shm > 160 * 1024) return XKV_EUNSUPPORTED;
-  auto kern = latent_stage1_kernel<T, NHB, TN, NVB_MAX, NPK_C, NPK_R, NPK_V, VSHARED, SCORES_ONLY>;
-  static DynLds lds;
-  const int e = ensure_dynamic_lds(lds, reinterpret_cast<const void*>(kern), (int)shm);
+  const bool plain = !p.split_plan && p.grid_splits == p.max_splits;
+  auto kern = plain ? latent_stage1_kernel<T, NHB, TN, NVB_MAX, NPK_C, NPK_R, NPK_V, VSHARED, SCORES_ONLY, true>
+                    : latent_stage1_kernel<T, NHB, TN, NVB_MAX, NPK_C, NPK_R, NPK_V, VSHARED, SCORES_ONLY, false>;
+  static DynLds lds[2];
+  const int e = ensure_dynamic_lds(lds[plain], reinterpret_cast<const void*>(kern), (int)shm);
   if (e != XKV_OK) return e;
   const int grid = xcd_grid(p.total_wg, p.groups);
   kern<<<dim3(grid), dim3(256), shm, st>>>(p);
