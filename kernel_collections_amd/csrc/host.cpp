@@ -368,11 +368,16 @@ void rope_operands(Ten q, int64_t hq, int64_t d, Ten kA, Ten kB, Ten inv) {
 }
 // the kernels that hold a kv head's factor in registers keep one workgroup per CU; two fit at rank 256 without P.A, the generic
 // kernel keeps two or three.  Scores at ranks up to 192: four independent waves of a 16-token tile each, one workgroup per CU.
-int recon_splits(const Call& c, Ten kB, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r, bool scores) {
-  if (scores && r <= 192 && rows(kB)) return balanced_splits(b, hkv, L, 64, 1, c.cus);
+int score_splits(const Call& c, Ten kB, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r) {
+  if (r <= 192 && rows(kB)) return balanced_splits(b, hkv, L, 64, 1, c.cus);
   const bool resident = ring_rank(r) && G <= 8;
-  const int per_cu = resident ? (scores && r == 256 ? 2 : 1) : r > 256 ? 1 : r > 128 ? 2 : 3;
-  return balanced_splits(b, hkv, L, 32, per_cu, c.cus);
+  return balanced_splits(b, hkv, L, 32, resident ? (r == 256 ? 2 : 1) : r > 256 ? 1 : r > 128 ? 2 : 3, c.cus);
+}
+// Scores and P.A in one kernel: one workgroup per CU; two only where the generic kernel, instantiated for the rank, does without a value
+// tile of its own (us at one / two / three workgroups a CU, batch 1, 32 heads on 8, 9000 tokens: rank 64 32 / 42 / 50, rank 128 28 / 26 / 34,
+// rank 192 31 / 29 / 33, rank 192 with values of its own 34 / 45 / 47).
+int decode_splits(const Call& c, int64_t b, int64_t hkv, int64_t L, int64_t r, bool shared) {
+  return balanced_splits(b, hkv, L, 32, shared && (r == 128 || r == 192) ? 2 : 1, c.cus);
 }
 
 // rope_decode(q [b,hq,128], kA, kB, vA, vB, o, sm_scale, inv_freq, pos_offset, two_pass) -> o | None
@@ -411,14 +416,14 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t sc = c.plan(b * hq * row * 4), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
         const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
         c.alloc();
-        recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, recon_splits(c, kB, b, hkv, hq / hkv, L, r, true), b, hq, hkv, row,
+        recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, score_splits(c, kB, b, hkv, hq / hkv, L, r), b, hq, hkv, row,
               scale, invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes, s.lens);
         check(p_xkv_softmax_pv_stage1(c.get<float>(sc), kv(vA, 0, rv), c.get<float>(part), c.get<float>(lse), nullptr, s.lens, b, hq, row, s.S,
                                       0, nullptr, c.dt, c.stream), "xkv_softmax_pv_stage1");
         merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, row, rv);
         return;
       }
-      s.S = recon_splits(c, kB, b, hkv, hq / hkv, L, r, false);
+      s.S = decode_splits(c, b, hkv, L, r, shared);
       const int64_t part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
       const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
       c.alloc();
@@ -447,7 +452,7 @@ PyObject* rope_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, B.stride(0)), ws = c.plan(ws_bytes);
       if (ws_bytes) c.alloc();
       out = at::empty({b, hq, 1, L}, f32 ? c.opts.dtype(at::kFloat) : c.opts);
-      recon(c, q, A, B, nullptr, nullptr, nullptr, out.data_ptr(), f32 ? XKV_F32 : c.dt, recon_splits(c, B, b, hkv, hq / hkv, L, r, true), b, hq, hkv,
+      recon(c, q, A, B, nullptr, nullptr, nullptr, out.data_ptr(), f32 ? XKV_F32 : c.dt, score_splits(c, B, b, hkv, hq / hkv, L, r), b, hq, hkv,
             L, scale, inv.data_ptr<float>(), pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
     });
     return THPVariable_Wrap(out);

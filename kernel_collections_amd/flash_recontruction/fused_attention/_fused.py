@@ -98,18 +98,21 @@ def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_sca
 # 98304 68.7 / 67.4), and those of the rank pairs without an 8-wave kernel lie lower (512 / 384, 32 on 8: 4096 32.9 / 33.1, 8192 46.4 / 38.8).
 TWO_PASS_KEY_RANKS = (512, 384, 256)
 TWO_PASS_MIN_TOKENS = 49152
-# Key ranks up to 192 have no 8-wave kernel: two passes from this many tokens on, counted for every kv head - the generic kernel fills
-# the device once at 8192 of them, and from there takes a second round (us fused / two passes, key rank 192, value rank 512: 32 heads on
-# 8 kv heads, 1024 tokens 20.8 / 26.1, 2048 29.8 / 28.3, 16384 66.2 / 44.1; 12 on 3, 2048 21.0 / 25.8, 3072 29.4 / 26.6; 16 on 2, 4096
-# 22.6 / 27.9, 5461 31.8 / 31.4; 8 on 1, 8192 24.3 / 29.1, 12288 35.0 / 29.5).
+# Key ranks up to 192 have no 8-wave kernel: two passes from this many tokens on, counted for every kv head, and from five times as many
+# at the ranks that the generic kernel is instantiated for (us fused / two passes: key rank 64, value rank 256, 32 heads on 8 kv heads, 1024
+# tokens 17.6 / 18.9, 4096 27.8 / 24.7; 16 on 4, 2048 19.7 / 20.6, 3072 22.9 / 21.7; 8 on 1, 8192 21.5 / 23.1, 12288 24.1 / 23.4; key rank
+# 192, value rank 512, 32 on 8, 4096 29.1 / 32.7, 8192 39.1 / 40.7, 16384 60.8 / 43.8; batch 16 x 512 35.7 / 33.4; 16 on 2, 16384 30.9 /
+# 34.7; key rank 128, value rank 384, 32 on 8, 8192 34.6 / 35.0).
 TWO_PASS_SMALL_RANK = 192
-TWO_PASS_MIN_TOKENS_SMALL = 9216
+TWO_PASS_MIN_TOKENS_SMALL = 12288
+GENERIC_RANKS = (128, 192)
 
 
 def _two_pass(rank, tokens, k_B):
     if rank in TWO_PASS_KEY_RANKS:
         return tokens >= TWO_PASS_MIN_TOKENS
-    return rank <= TWO_PASS_SMALL_RANK and tokens * k_B.shape[1] >= TWO_PASS_MIN_TOKENS_SMALL and ops._row_ok(k_B)
+    least = TWO_PASS_MIN_TOKENS_SMALL * (5 if rank in GENERIC_RANKS else 1)
+    return rank <= TWO_PASS_SMALL_RANK and tokens * k_B.shape[1] >= least and ops._row_ok(k_B)
 
 
 def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale, theta, sin_cos,

@@ -1,6 +1,6 @@
 // The entry points that the native host layer calls, in front of libxkv_hip.so (tests load this in the library's place): each one
 // counts the calls made with the Python interpreter locked and, when poisoning is on, fills the LDS of the whole device before a
-// stage-1 launch.
+// stage-1 launch.  shim_recon_splits: the splits that the last reconstructing launch was given.
 #include <dlfcn.h>
 
 #include "../include/xkv_hip.h"
@@ -8,7 +8,7 @@
 static void* real_lib;
 static int (*gil_held)();
 extern "C" {
-int shim_launches, shim_stage1, shim_locked_calls, shim_poison, shim_poisoned;
+int shim_launches, shim_stage1, shim_locked_calls, shim_poison, shim_poisoned, shim_recon_splits;
 int shim_init(const char* path) {
   real_lib = dlopen(path, RTLD_NOW | RTLD_LOCAL);
   gil_held = (int (*)())dlsym(RTLD_DEFAULT, "PyGILState_Check");
@@ -49,7 +49,7 @@ FORWARD(xkv_recon_stage1, true, (const void* q, xkv_kv_operand A, const void* B,
                                  float* lse, void* sc, int sdt, const int32_t* ns, const int32_t* kl, int b, int hq, int hkv, int L, int S,
                                  float scale, int rope, const float* inv, int64_t pos, const void* tab, int64_t st, void* ws, int64_t wb, int dt,
                                  void* stream),
-        (q, A, B, s0, s1, s2, V, part, lse, sc, sdt, ns, kl, b, hq, hkv, L, S, scale, rope, inv, pos, tab, st, ws, wb, dt, stream))
+        (q, A, B, s0, s1, s2, V, part, lse, sc, sdt, ns, kl, b, hq, hkv, L, shim_recon_splits = S, scale, rope, inv, pos, tab, st, ws, wb, dt, stream))
 FORWARD(xkv_merge_stage2, false, (const float* part, const float* lse, void* out, const void* vB, int64_t v0, int64_t v1, int64_t v2, int d, int vdt,
                                   const int32_t* ns, const int32_t* kl, int b, int hq, int hkv, int L, int S, int cap, const int32_t* plan, int dv,
                                   int64_t o0, int64_t o1, int odt, float* lo, int64_t l0, int64_t l1, void* stream),

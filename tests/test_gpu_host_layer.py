@@ -298,3 +298,17 @@ def test_ragged_batches_with_and_without_a_plan(dev, path, L, lens):
                     assert (got[i] == 0).all(), (name, hkv)
                 else:
                     check_out(got[i], call(slice(i, i + 1), n, None)[0], f"{name} {hkv} sequence {i}")
+
+
+@pytest.mark.parametrize("hq,hkv,r,rv,per_cu", [(32, 8, 64, 0, 1), (32, 8, 128, 0, 2), (32, 8, 192, 0, 2), (32, 8, 192, 192, 1), (32, 8, 128, 64, 1),
+                                                (16, 1, 256, 0, 1), (32, 8, 512, 0, 1)])
+def test_one_kernel_rope_decode_is_planned_for_its_occupancy(dev, shim, hq, hkv, r, rv, per_cu):
+    """Workgroups per CU of the kernel that takes scores and P.A in one, as measured beside decode_splits in csrc/host.cpp."""
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd import ops
+    L = 9000
+    t = lambda *s, n=0: gen(s, seed=n).to(dev)
+    q, A, B = t(1, hq, 128, n=1), t(1, L, r, n=2), t(1, hkv, r, 128, n=3)
+    V, vB = (t(1, L, rv, n=4), t(1, hkv, rv, 128, n=5)) if rv else (A, B)
+    fr.gqa_xKV_rope(q, A, B, V, vB, torch.empty_like(q), torch.ones(1, dtype=torch.int32, device=dev), 1, 0.1, 5e5)
+    assert shim.count("shim_recon_splits") == ops.occupancy_splits(1, hkv, L, tile=32, waves=per_cu)
