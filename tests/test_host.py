@@ -222,3 +222,10 @@ def test_short_batches_are_cut_shorter(batch, groups, kv_len, per_cu, up, floor)
     """The fastest of 32, 64, 96, 128 and 256 tokens as measured, within 3 %."""
     from kernel_collections_amd import _xkv_host
     assert _xkv_host.split_floor(batch, groups, kv_len, per_cu, 256, up) == floor == ops.split_floor(batch, groups, kv_len, per_cu, up)
+
+
+def test_short_sequences_under_many_heads_are_not_cut_below_64_tokens(monkeypatch):
+    from kernel_collections_amd.flash_decoding import mla
+    monkeypatch.setattr(_lib, "require_gpu", lambda t: None)
+    k = torch.zeros(3, 1227, 1, 576, dtype=torch.bfloat16)
+    assert mla.stage1_splits(3, 1227, mla.stage1_operands(torch.zeros(3, 64, 576, dtype=torch.bfloat16), k, k[..., :512])) == 20
