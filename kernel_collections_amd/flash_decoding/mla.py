@@ -51,10 +51,12 @@ def stage1_operands(q, k_buffer, v_buffer):
 
 
 def stage1_splits(batch, kv_len, operands) -> int:
-    """The split count for what `stage1_operands` returned.  No split below 64 tokens: the partial rows of a short one (2 KiB a head)
-    outweigh its keys (3 sequences of 1227 tokens, 64 heads, 576 wide: 31.6 us in 32-token splits, 26.2 in 64)."""
-    _, _, _, R, _, groups, dn, _ = operands
-    return min(ops.latent_splits(batch, groups, kv_len, dn, rope=R[4] if R else 0), -(-kv_len // 64))
+    """The split count for what `stage1_operands` returned.  No split below 64 tokens once they are
+    more than 1024 partial rows (2 KiB each): those of short splits then outweigh the keys (us in 32- / 64-token splits, 576 wide: 3 x 1227
+    tokens, 64 heads 31.6 / 26.2; 1 x 5469, 24 heads 20.6 / 19.4; 2 x 832, 16 heads 14.9 / 15.7)."""
+    qn, _, _, R, _, groups, dn, _ = operands
+    floor = 32 if batch * qn.shape[1] * -(-kv_len // 32) <= 1024 else 64
+    return min(ops.latent_splits(batch, groups, kv_len, dn, rope=R[4] if R else 0), -(-kv_len // floor))
 
 
 def decode_attention_fwd(q, k_buffer, v_buffer, o, sm_scale=1.0, logit_cap=0.0):

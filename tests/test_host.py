@@ -229,3 +229,10 @@ def test_short_sequences_under_many_heads_are_not_cut_below_64_tokens(monkeypatc
     monkeypatch.setattr(_lib, "require_gpu", lambda t: None)
     k = torch.zeros(3, 1227, 1, 576, dtype=torch.bfloat16)
     assert mla.stage1_splits(3, 1227, mla.stage1_operands(torch.zeros(3, 64, 576, dtype=torch.bfloat16), k, k[..., :512])) == 20
+
+
+def test_few_partial_rows_are_cut_to_32_tokens(monkeypatch):
+    from kernel_collections_amd.flash_decoding import mla
+    monkeypatch.setattr(_lib, "require_gpu", lambda t: None)
+    k = torch.zeros(2, 832, 1, 576, dtype=torch.bfloat16)
+    assert mla.stage1_splits(2, 832, mla.stage1_operands(torch.zeros(2, 16, 576, dtype=torch.bfloat16), k, k[..., :512])) == 26
