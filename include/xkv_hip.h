@@ -235,7 +235,8 @@ int xkv_recon_stage1_static(const void* q_pe, xkv_kv_operand kA, const void* kB,
  * (stride_o_b, stride_o_h), written as out_dtype.
  * Replaces _fwd_kernel_stage2[grid] at flash_decoding/gqa.py:322-337 (mla.py, mla2/stage2.py:117-135,
  * fused_attention/no_pe/v1.py:345-362 twins) and the torch.matmul with v_B_buffer at
- * fused_attention/no_pe/v2.py:468-471 / v1.py:458-460.   dv <= 512; d_out <= 512.
+ * fused_attention/no_pe/v2.py:468-471 / v1.py:458-460.   dv <= 512; d_out <= 512; dv plus the splits a sequence may have <= 6144
+ * (XKV_EUNSUPPORTED; a limit of the interface from the time when a head's split weights were held in the LDS).
  * lse_out (may be NULL): the log-sum-exp of the merged range, lse_out[b * stride_lse_b + h * stride_lse_h] =
  * log sum_i exp(lse_i), which lets the merged row take part in a further merge as one split (prefix + tail decode,
  * flash_decoding/deepseek_mla/flash_decoding.py:137-155 concatenates the workspaces instead). */
@@ -255,8 +256,8 @@ int xkv_merge_stage2(const float* partial, const float* lse, void* out,
  * of CUs, a stage 1 that runs one workgroup per CU gives every CU exactly one job and the jobs are as equal as the lengths
  * allow; a batch scanned in fixed-length splits ends on whatever the last workgroups happen to hold.  plan holds
  * 2 + 2 * batch * max_splits int32 (max_splits as passed to stage 1, >= ceil(kv_len / floor_tokens)); packed (num_kv_splits
- * == NULL, max_splits >= max(target_jobs, batch), XKV_EINVAL otherwise) 2 + 2 * max_splits + batch: behind the pairs of
- * max_splits jobs plan[2 + 2 * max_splits + b], the jobs of the sequences before b.  Pass plan as split_plan, and floor_tokens as split_cap_tokens, to xkv_latent_stage1 and xkv_merge_stage2 on the same stream.  One
+ * == NULL, max_splits >= max(target_jobs, batch), XKV_EINVAL otherwise) 3 + 2 * max_splits + batch: behind the pairs of
+ * max_splits jobs plan[2 + 2 * max_splits + b], the jobs of the sequences before b (b == batch: of all).  Pass plan as split_plan, and floor_tokens as split_cap_tokens, to xkv_latent_stage1 and xkv_merge_stage2 on the same stream.  One
  * small workgroup; no host synchronisation.  No counterpart in the reference, whose batches have one length
  * (flash_decoding/gqa.py:60,194). */
 int xkv_plan_splits(const int32_t* kv_lens, const int32_t* num_kv_splits, int batch, int max_splits, int floor_tokens,

@@ -182,7 +182,7 @@ Ragged ragged(Call& c, Splits& s, int64_t batch, int groups, int64_t kv_len, int
   if (batch * s.S * groups <= c.cus) return {0, 0};
   const int target = ragged_target(batch, groups, per_cu, c.cus);
   s.jobs = std::max<int64_t>(target, batch);
-  return {target, c.plan((2 + 2 * (int64_t)s.jobs + batch) * 4)};
+  return {target, c.plan((3 + 2 * (int64_t)s.jobs + batch) * 4)};
 }
 void write_plan(const Call& c, Splits& s, const Ragged& r, int64_t batch) {
   if (!s.jobs) return;

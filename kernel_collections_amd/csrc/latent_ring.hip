@@ -551,7 +551,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   if (SCORES) return;
 
   // ---- epilogue: normalise, write partial + lse --------------------------------------------------------------------
-  const PartialRows rows = partial_rows(b, p.hq, p.max_splits, [&] { return live_splits(L, ns, p.max_splits); }, p.num_splits, p.split_plan);
+  const PartialRows rows = partial_rows(b, p.hq, p.max_splits, p.num_splits, p.split_plan);
   if (ssub == 0) { ml_lds[2 * srow] = m_run; ml_lds[2 * srow + 1] = l_run; }
   __syncthreads();
   if (VHEADS) {

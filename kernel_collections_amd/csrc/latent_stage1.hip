@@ -33,9 +33,9 @@ __device__ __forceinline__ V8 tr_operand(const void* p0, const void* p1) {
   return __builtin_bit_cast(V8, r);
 }
 
-// Where a workgroup's results go: the partial row of its first head, and the rows from head to head.  Calls with a plan or fewer workgroups
-// than workspace rows work all of it out once more, from parameters read again (1155 us at the shape below with the workgroup's place held
-// through the scan, 1149 without).
+// Where a workgroup's results go: the partial row of its first head, and the rows from head to head.  For calls with a plan or fewer workgroups
+// than workspace rows from parameters read again, which the scan then does not hold (32 ragged sequences of up to 14000 tokens, 8 heads, values
+// of rank 192: 892 us; 871 before rows were packed).
 struct SplitRows { int64_t row; int per_head, dv; float* partial; float* lse; };
 template <bool PLAIN> __device__ __forceinline__ SplitRows split_rows(const LatentParams& p, int b, int split, int h0) {
   if constexpr (PLAIN) {
@@ -43,23 +43,9 @@ template <bool PLAIN> __device__ __forceinline__ SplitRows split_rows(const Late
   } else {
     typedef const __attribute__((address_space(4))) LatentParams* Params;
     Params q = (Params)__builtin_amdgcn_kernarg_segment_ptr();
-    int id = blockIdx.x;
-    asm volatile("" : "+s"(q), "+s"(id));
-    const int32_t* lens = q->kv_lens;
-    const int32_t* counts = q->num_splits;
-    const int32_t* plan = q->split_plan;
-    const int groups = q->groups, grid_splits = q->grid_splits, hq = q->hq, max_splits = q->max_splits, cap = q->split_cap;
-    const int wg = xcd_cluster_remap(id, groups), first = wg % groups * (hq / groups);
-    int at = (wg / groups) % grid_splits, seq = wg / (groups * grid_splits);
-    if (plan) {
-      seq = plan[2 + 2 * (wg / groups)];
-      at = plan[3 + 2 * (wg / groups)];
-    }
-    const PartialRows rows = partial_rows(seq, hq, max_splits, [&] {
-      const int L = lens ? lens[seq] : q->kv_len;
-      return live_splits(L, effective_splits(L, asked_splits(counts, seq, max_splits, cap), split_cap_in_force(cap, plan)), max_splits);
-    }, counts, plan);
-    return {rows.base + (int64_t)first * rows.per_head + at, rows.per_head, q->dv, q->partial, q->lse};
+    asm volatile("" : "+s"(q));
+    const PartialRows rows = partial_rows(b, q->hq, q->max_splits, q->num_splits, q->split_plan);
+    return {rows.base + (int64_t)h0 * rows.per_head + split, rows.per_head, q->dv, q->partial, q->lse};
   }
 }
 

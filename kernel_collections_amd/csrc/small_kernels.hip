@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(
   const int lanes = chunk / P, ngrp = 256 / lanes;          // lanes <= 256
   const int sg = threadIdx.x / lanes, c = c0 + (threadIdx.x % lanes) * P;
   const bool mine = sg < ngrp && c < dv;
-  const PartialRows rows = partial_rows(b, hq, max_splits, [&] { return nlive; }, num_kv_splits, split_plan);
+  const PartialRows rows = partial_rows(b, hq, max_splits, num_kv_splits, split_plan);
   const int64_t row = rows.base + (int64_t)h * rows.per_head;
   MergeAcc<P> a;
   if (mine) {
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
   load_w();
   const int L = kv_lens ? kv_lens[b] : kv_len;
   const int nlive = live_splits(L, effective_splits(L, asked_splits(num_kv_splits, b, max_splits, split_cap), split_cap_in_force(split_cap, split_plan)), max_splits);
-  const PartialRows rows = partial_rows(b, hq, max_splits, [&] { return nlive; }, num_kv_splits, split_plan);
+  const PartialRows rows = partial_rows(b, hq, max_splits, num_kv_splits, split_plan);
   auto merge_packet = [&](int gi, int c, auto tag) {
     constexpr int P = decltype(tag)::value;
     const int64_t row = rows.base + (int64_t)(hfirst + gi) * rows.per_head;
@@ -627,7 +627,11 @@ __global__ __launch_bounds__(PLAN_T) void plan_splits_kernel(const int32_t* __re
     done += all0;
     last += all1;
   }
-  if (tid == 0) { plan[0] = cap; plan[1] = done + last; }
+  if (tid == 0) {
+    plan[0] = cap;
+    plan[1] = done + last;
+    if (!num_splits) plan[2 + 2 * (int64_t)max_splits + batch] = done + last;
+  }
 }
 
 }  // namespace xkv

@@ -119,9 +119,11 @@ inline bool cap_fits(const int32_t* num_splits, int batch, int kv_len, int max_s
   return cap == 0 || (kv_len > 0 && max_splits >= cdiv(kv_len, cap));
 }
 struct PartialRows { int64_t base; int per_head; };
-template <typename Live>   // live(): the sequence's live splits, evaluated only where rows are packed
-__device__ __forceinline__ PartialRows partial_rows(int b, int hq, int max_splits, Live live, const int32_t* num_splits, const int32_t* plan) {
-  if (__builtin_expect(packed_rows(num_splits, plan), 0)) return {(int64_t)plan[2 + 2 * (int64_t)max_splits + b] * hq, live()};
+__device__ __forceinline__ PartialRows partial_rows(int b, int hq, int max_splits, const int32_t* num_splits, const int32_t* plan) {
+  if (__builtin_expect(packed_rows(num_splits, plan), 0)) {
+    const int32_t* first = plan + 2 + 2 * (int64_t)max_splits + b;
+    return {(int64_t)first[0] * hq, first[1] - first[0]};
+  }
   return {(int64_t)b * hq * max_splits, max_splits};
 }
 

@@ -21,8 +21,8 @@ from kernel_collections_amd import _lib, ops
 # the merge, so the caller's count is a hint about parallelism and not part of the result: the wrappers choose the count that
 # fills the device - for one length on the host, for a ragged batch per call on the device (equal jobs, at most one per
 # workgroup the chip holds).  The caller's own counts miss it on both sides: 32 sequences of 1K .. 128K tokens in 4096-token
-# splits are 315 jobs on 256 CUs (1040 us, planned: 751), 8 of up to 16K are 20 (113 us
-# at no less than 1024 tokens each, planned: 57).
+# splits are 315 jobs on 256 CUs (1040 us, planned: 748), 8 of up to 16K are 20 (113 us
+# at no less than 1024 tokens each, planned: 52).
 # At 128 tokens a job's start (about 5 us) is a third of its time; a batch too short to fill the device at that takes shorter ones
 # (`split_floor` in csrc/host.cpp).  _WIDE: the all-heads forms, one workgroup per CU.
 MAX_SPLIT_TOKENS = 128

@@ -264,9 +264,9 @@ def plan_splits(kv_lens: torch.Tensor, num_kv_splits: Optional[torch.Tensor], ma
     sequences of the batch into at most `target_jobs` splits; [1] the number of live (sequence, split) pairs; then the pairs.
     Pass it as `split_plan` (with `split_cap=floor_tokens` and the same `max_splits`) to stage 1 and the merge.  Without
     `num_kv_splits` the plan is packed: `max_splits` counts the jobs of the batch (at least `target_jobs` and the batch), which is
-    how many partial rows per head the workspaces hold, and the first job of every sequence stands behind the pairs."""
+    how many partial rows per head the workspaces hold, and the first job of every sequence, then their number, stand behind the pairs."""
     batch = kv_lens.numel()
-    words = 2 + 2 * int(max_splits) * batch if num_kv_splits is not None else 2 + 2 * int(max_splits) + batch
+    words = 2 + 2 * int(max_splits) * batch if num_kv_splits is not None else 3 + 2 * int(max_splits) + batch
     plan = torch.empty(words, dtype=torch.int32, device=kv_lens.device)
     check(_lib.lib().xkv_plan_splits(ptr(kv_lens), ptr(num_kv_splits), batch, int(max_splits), int(floor_tokens),
                                      int(target_jobs), ptr(plan), stream_ptr(kv_lens)), "xkv_plan_splits")

@@ -158,13 +158,13 @@ def test_packed_plan(dev, lens, floor, target):
     n = max(b, target)
     kl = torch.tensor(lens, dtype=torch.int32, device=dev)
     plan = ops.plan_splits(kl, None, n, floor, target).cpu().tolist()
-    assert len(plan) == 2 + 2 * n + b
+    assert len(plan) == 3 + 2 * n + b
     count = lambda cap: sum(-(-x // cap) for x in lens)
     top = max(floor, -(-max(lens) // 32) * 32)
     cap = next((c for c in range(floor, top, 32) if count(c) <= target), top)
     live = [ops.settled_splits(x, -(-x // cap)) if x else 0 for x in lens]
     assert plan[0] == cap and plan[1] == sum(live) <= n
-    assert plan[2 + 2 * n:] == [sum(live[:i]) for i in range(b)]
+    assert plan[2 + 2 * n:] == [sum(live[:i]) for i in range(b + 1)]
     pairs = [(plan[2 + 2 * j], plan[3 + 2 * j]) for j in range(plan[1])]
     assert sorted(pairs) == [(i, s) for i in range(b) for s in range(live[i])]
     assert all(s == live[i] - 1 for i, s in pairs[sum(max(x - 1, 0) for x in live):])
