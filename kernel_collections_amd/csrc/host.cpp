@@ -376,8 +376,8 @@ int score_splits(const Call& c, Ten kB, int64_t b, int64_t hkv, int64_t G, int64
 // Scores and P.A in one kernel: one workgroup per CU; two only where the generic kernel, instantiated for the rank, does without a value
 // tile of its own (us at one / two / three workgroups a CU, batch 1, 32 heads on 8, 9000 tokens: rank 64 32 / 42 / 50, rank 128 28 / 26 / 34,
 // rank 192 31 / 29 / 33, rank 192 with values of its own 34 / 45 / 47).
-int decode_splits(const Call& c, int64_t b, int64_t hkv, int64_t L, int64_t r, bool shared) {
-  return balanced_splits(b, hkv, L, 32, shared && (r == 128 || r == 192) ? 2 : 1, c.cus);
+int decode_splits(int64_t b, int64_t hkv, int64_t L, int64_t r, bool shared, int cus) {
+  return balanced_splits(b, hkv, L, 32, shared && (r == 128 || r == 192) ? 2 : 1, cus);
 }
 
 // rope_decode(q [b,hq,128], kA, kB, vA, vB, o, sm_scale, inv_freq, pos_offset, two_pass) -> o | None
@@ -423,7 +423,7 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, row, rv);
         return;
       }
-      s.S = decode_splits(c, b, hkv, L, r, shared);
+      s.S = decode_splits(b, hkv, L, r, shared, c.cus);
       const int64_t part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
       const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
       c.alloc();
@@ -607,6 +607,11 @@ PyObject* prefix_tail(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// decode_splits(batch, kv heads, kv_len, rank, shared, cus) -> int
+PyObject* py_decode_splits(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 6, [&]() -> PyObject* { return PyLong_FromLong(decode_splits(I(a[0]), I(a[1]), I(a[2]), I(a[3]), I(a[4]), I(a[5]))); });
+}
+
 // split_floor(batch, groups, kv_len, per_cu, cus, up) -> int
 PyObject* py_split_floor(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 6, [&]() -> PyObject* { return PyLong_FromLong(split_floor(I(a[0]), I(a[1]), I(a[2]), I(a[3]), I(a[4]), I(a[5]))); });
@@ -646,7 +651,7 @@ PyObject* init(PyObject*, PyObject* path) {
 #define XKV_FAST(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fn)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"init", init, METH_O, nullptr},       XKV_FAST("balanced_splits", py_balanced_splits), XKV_FAST("nope_decode", nope_decode), XKV_FAST("ragged_target", py_ragged_target),
-    XKV_FAST("split_floor", py_split_floor),
+    XKV_FAST("split_floor", py_split_floor), XKV_FAST("decode_splits", py_decode_splits),
     XKV_FAST("nope_scores", nope_scores),  XKV_FAST("rope_decode", rope_decode),            XKV_FAST("rope_scores", rope_scores),
     XKV_FAST("gqa", gqa),                  XKV_FAST("mla", mla),                            XKV_FAST("prefix_tail", prefix_tail),
     {nullptr, nullptr, 0, nullptr}};

@@ -106,13 +106,19 @@ TWO_PASS_MIN_TOKENS = 49152
 TWO_PASS_SMALL_RANK = 192
 TWO_PASS_MIN_TOKENS_SMALL = 12288
 GENERIC_RANKS = (128, 192)
+# A ragged batch in one kernel is scanned with the caller's counts, which may leave most of the device idle (16 heads on 2 kv heads, 8 splits
+# of 7368 tokens: 84 us, two passes 29): two passes from here on, whatever the heads.
+TWO_PASS_MIN_TOKENS_ASKED = 4096
 
 
-def _two_pass(rank, tokens, k_B):
+def _two_pass(rank, tokens, k_B, asked=False):
     if rank in TWO_PASS_KEY_RANKS:
         return tokens >= TWO_PASS_MIN_TOKENS
-    least = TWO_PASS_MIN_TOKENS_SMALL * (5 if rank in GENERIC_RANKS else 1)
-    return rank <= TWO_PASS_SMALL_RANK and tokens * k_B.shape[1] >= least and ops._row_ok(k_B)
+    if rank > TWO_PASS_SMALL_RANK or not ops._row_ok(k_B):
+        return False
+    if asked:
+        return tokens >= TWO_PASS_MIN_TOKENS_ASKED
+    return tokens * k_B.shape[1] >= TWO_PASS_MIN_TOKENS_SMALL * (5 if rank in GENERIC_RANKS else 1)
 
 
 def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale, theta, sin_cos,
@@ -148,7 +154,8 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
         if sin_cos.dtype != q_pe.dtype or sin_cos.stride(-1) != 1:
             sin_cos = sin_cos.to(q_pe.dtype).contiguous()
     same_basis = (v_A.data_ptr() == k_A.data_ptr() and v_A.shape == k_A.shape and v_A.stride() == k_A.stride())
-    if (not same_basis and _two_pass(k_A.shape[-1], batch * kv_len, k_B) and sin_cos is None and hq // hkv <= 8 and hq <= 32
+    asked = (lens is not None and batch > 1) or sin_cos is not None       # the caller's counts are taken
+    if (not same_basis and _two_pass(k_A.shape[-1], batch * kv_len, k_B, asked) and sin_cos is None and hq // hkv <= 8 and hq <= 32
             and rank_v in (256, 384, 512) and kv_len % 4 == 0 and ops.USE_RECON_WORKSPACE):
         # A value basis of its own: two passes.  The scores-only form of the reconstruction kernel runs at the rate of the
         # shared-basis fused kernel (one row stream, no P.A); softmax and P.v_A then stream v_A once for all heads at HBM
@@ -164,7 +171,10 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
         partial, lse = ops.workspaces(batch, hq, S2, rank_v, q_pe.device)
         ops.softmax_pv_stage1(scores, v_A, partial, lse, None, lens, batch, hq, kv_len, S2, q_pe.dtype)
         return ops.merge_stage2(partial, lse, o, v_B, None, lens, batch, hq, hkv, kv_len, S2)
-    S, splits = int(max_kv_splits), ops.as_int32_dev(num_kv_splits, batch, q_pe.device)
+    if asked:
+        S, splits = int(max_kv_splits), ops.as_int32_dev(num_kv_splits, batch, q_pe.device)
+    else:
+        S, splits = ops.decode_splits(batch, hkv, kv_len, k_A.shape[-1], same_basis), None
     partial, lse = ops.workspaces(batch, hq, S, rank_v, q_pe.device)
     ops.recon_stage1(q3, k_A, k_B, v_A, partial, lse, None, splits, lens, batch, hq, hkv, kv_len, S,
                      float(sm_scale), True, inv, int(pos_offset), sin_cos)

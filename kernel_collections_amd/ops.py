@@ -278,6 +278,12 @@ def capped_splits(kv_len: int, max_kv_splits: int, cap_tokens: int) -> int:
     return max(int(max_kv_splits), _cdiv(kv_len, cap_tokens)) if cap_tokens else int(max_kv_splits)
 
 
+def decode_splits(batch: int, hkv: int, kv_len: int, rank: int, shared: bool) -> int:
+    """Splits of a RoPE decode in one kernel (`decode_splits` in csrc/host.cpp)."""
+    from . import _xkv_host
+    return _xkv_host.decode_splits(batch, hkv, kv_len, rank, shared, num_cus())
+
+
 def split_floor(batch: int, groups: int, kv_len: int, per_cu: int, up: bool) -> int:
     """Shortest split in tokens (`split_floor` in csrc/host.cpp); `up`: the merged rows are up-projected."""
     from . import _xkv_host

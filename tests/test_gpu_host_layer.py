@@ -312,3 +312,26 @@ def test_one_kernel_rope_decode_is_planned_for_its_occupancy(dev, shim, hq, hkv,
     V, vB = (t(1, L, rv, n=4), t(1, hkv, rv, 128, n=5)) if rv else (A, B)
     fr.gqa_xKV_rope(q, A, B, V, vB, torch.empty_like(q), torch.ones(1, dtype=torch.int32, device=dev), 1, 0.1, 5e5)
     assert shim.count("shim_recon_splits") == ops.occupancy_splits(1, hkv, L, tile=32, waves=per_cu)
+
+
+@pytest.mark.parametrize("form", ["copied", "one_sequence"])
+def test_general_rope_decode_fills_the_device(dev, form, monkeypatch):
+    """The caller's two splits are a hint here too - operands to be copied first, one sequence of a given length."""
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd import ops
+    L, r = 5000, 192
+    t = lambda *s, std=1.0, n=0: gen(s, std=std, seed=n).to(dev)
+    q, A, B = t(1, 16, 128, std=0.4, n=1), t(1, L, r, n=2), t(1, 2, r, 128, std=r ** -0.5, n=3)
+    ns = torch.full((1,), 2, dtype=torch.int32, device=dev)
+    want = fr.gqa_xKV_rope(q, A, B, A, B, torch.empty_like(q), ns, 2, 128 ** -0.5, 5e5)
+    seen = []
+    real = ops.recon_stage1
+    monkeypatch.setattr(ops, "recon_stage1", lambda *a: seen.append(a[13]) or real(*a))
+    kw = {}
+    if form == "copied":
+        q = torch.empty(1, 16, 136, dtype=BF, device=dev)[..., :128].copy_(q)
+    else:
+        kw = dict(kv_lens=torch.full((1,), L, dtype=torch.int32, device=dev))
+    got = fr.gqa_xKV_rope(q, A, B, A, B, torch.empty(1, 16, 128, dtype=BF, device=dev), ns, 2, 128 ** -0.5, 5e5, **kw)
+    assert seen == [ops.decode_splits(1, 2, L, r, True)] and seen[0] > 64
+    check_out(got, want, form)

@@ -236,3 +236,9 @@ def test_few_partial_rows_are_cut_to_32_tokens(monkeypatch):
     monkeypatch.setattr(_lib, "require_gpu", lambda t: None)
     k = torch.zeros(2, 832, 1, 576, dtype=torch.bfloat16)
     assert mla.stage1_splits(2, 832, mla.stage1_operands(torch.zeros(2, 16, 576, dtype=torch.bfloat16), k, k[..., :512])) == 26
+
+
+def test_two_passes_where_the_callers_counts_are_taken():
+    from kernel_collections_amd.flash_recontruction.fused_attention import _fused
+    B = torch.zeros(1, 2, 192, 128, dtype=torch.bfloat16)
+    assert _fused._two_pass(192, 7368, B, asked=True) and not _fused._two_pass(192, 7368, B) and not _fused._two_pass(192, 4095, B, asked=True)
