@@ -366,12 +366,12 @@ void rope_operands(Ten q, int64_t hq, int64_t d, Ten kA, Ten kB, Ten inv) {
   need(hq % hkv == 0 && hq / hkv <= 16 && r % 32 == 0 && r <= 512 && packed_q(q) && rows(kA) && kB.stride(3) == 1);
   need(inv.is_cuda() && inv.device() == q.device() && inv.scalar_type() == at::kFloat && inv.numel() == 64 && inv.is_contiguous());
 }
-// the kernels that hold a kv head's factor in registers keep one workgroup per CU; two fit at rank 256 without P.A, the generic
-// kernel keeps two or three.  Scores at ranks up to 192: four independent waves of a 16-token tile each, one workgroup per CU.
+// recon_scores_kernel: four tiles of 16 tokens a step (two beyond rank 256), one workgroup per CU; otherwise the kernels that hold a kv
+// head's factor in registers keep one, the generic kernel two or three.
 int score_splits(const Call& c, Ten kB, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r) {
-  if (r <= 192 && rows(kB)) return balanced_splits(b, hkv, L, 64, 1, c.cus);
+  if (rows(kB) && (r <= 256 || r % 64 == 0)) return balanced_splits(b, hkv, L, r <= 256 ? 64 : 32, 1, c.cus);
   const bool resident = ring_rank(r) && G <= 8;
-  return balanced_splits(b, hkv, L, 32, resident ? (r == 256 ? 2 : 1) : r > 256 ? 1 : r > 128 ? 2 : 3, c.cus);
+  return balanced_splits(b, hkv, L, 32, resident || r > 256 ? 1 : r > 128 ? 2 : 3, c.cus);
 }
 // Scores and P.A in one kernel: one workgroup per CU; two only where the generic kernel, instantiated for the rank, does without a value
 // tile of its own (us at one / two / three workgroups a CU, batch 1, 32 heads on 8, 9000 tokens: rank 64 32 / 42 / 50, rank 128 28 / 26 / 34,

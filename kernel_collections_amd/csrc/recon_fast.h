@@ -1,4 +1,4 @@
-// Interface between the recon stage-1 dispatcher and its MFMA-bound fast paths (recon_fast_*.hip, recon_duo_*.hip).
+// Interface between the recon stage-1 dispatcher and its MFMA-bound paths (recon_scores.hip, recon_spec_*.hip, recon_duo_*.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -17,11 +17,8 @@ struct FastParams {
   const void* vA; int64_t sVb, sVl;             // separate value basis (recon_duo kernels only)
 };
 
-// The 4-wave kernel (recon_fast_impl.h): scores only, or the key basis reused as the value basis.  Instantiated at rank 256,
-// where its scores-only form fits a CU twice.
-int launch_recon_fast_256(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                          hipStream_t st);
-// The wave-specialised 8-wave kernel (recon_spec_impl.h), one translation unit per key rank: the same shapes and arguments.
+// The wave-specialised 8-wave kernel (recon_spec_impl.h), one translation unit per key rank: the key basis reused as
+// the value basis, and scores only where a factor is not made of 16-byte packets.
 int launch_recon_spec_512(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
                           hipStream_t st);
 int launch_recon_spec_384(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
@@ -35,13 +32,14 @@ inline int launch_recon_spec(const FastParams& p, const void* kB, int64_t sBb, i
                        : launch_recon_spec_256(p, kB, sBb, sBh, sBr, batch, dtype, st);
 }
 
-// Scores only at ranks up to 192, up to 16 query heads per kv head (recon_scores.hip).  Reads kB as it is (16-byte packets of unit
-// stride; Bp of the parameters is not used).
+// Scores only, up to 16 query heads per kv head (recon_scores.hip): ranks up to 256, multiples of 64 up to 512.  Reads kB as it is
+// (16-byte packets of unit stride; Bp of the parameters is not used).
+bool recon_scores_serves(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int rank);
 int launch_recon_scores(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype, int rank,
                         hipStream_t st);
 
 // The 8-wave kernels (recon_duo_impl.h) for key ranks 256 / 384 / 512 with a separate value basis of rank rv (mode 2; the
-// kernel template also has a scores-only mode 0 and a shared-basis mode 1, which the 4-wave kernel above now serves).  Each
+// kernel template also has a scores-only mode 0 and a shared-basis mode 1, which the kernels above now serve).  Each
 // translation unit serves the shapes it instantiates and returns DUO_NOT_MINE for the others.
 constexpr int DUO_NOT_MINE = -1000;
 int launch_recon_duo_b(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,

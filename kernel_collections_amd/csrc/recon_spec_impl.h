@@ -1,7 +1,7 @@
 // Wave-specialised form of the fused reconstruct + RoPE + softmax + P.A stage 1 (rank RK = 512 / 384 / 256, head_dim 128,
 // the token basis shared by K and V): 8 wavefronts per workgroup, two per SIMD, with different jobs.
 //
-// Reconstruction waves (0..3) form the 2 x 2 grid over (rank half kq, feature half dq) of recon_fast_impl.h: wave (kq, dq)
+// Reconstruction waves (0..3) form the 2 x 2 grid over (rank half kq, feature half dq): wave (kq, dq)
 // keeps its quarter of B_h stationary in RK / 4 accumulation registers and issues nothing but the v_mfma_f32_32x32x16 of the
 // 32-token tile, the LDS reads of its operands, and the hand-over of the finished partial key tile - rounded to fp16, 16 KB
 // per tile - to the consumer waves through a double-buffered LDS area.  Their instruction stream is 32 MFMAs against ~40

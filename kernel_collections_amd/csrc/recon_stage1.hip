@@ -401,7 +401,18 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
   const bool vshared = !so && vA.ptr == kA.ptr && vA.stride_b == kA.stride_b && vA.stride_l == kA.stride_l &&
                        vA.dim == kA.dim;
   hipStream_t st = (hipStream_t)stream;
-  // MFMA-bound fast path: rank 512 / 384 / 256, scores only or a basis shared by K and V, computed RoPE angles, at most 8 query heads
+  if (so && rope && !sin_cos) {
+    FastParams f{};
+    f.q = q_pe; f.kA = kA.ptr; f.sAb = kA.stride_b; f.sAl = kA.stride_l;
+    f.scores = scores_out; f.scores_dtype = scores_dtype;
+    f.num_splits = num_kv_splits; f.kv_lens = kv_lens;
+    f.hq = hq; f.hkv = hkv; f.kv_len = kv_len; f.max_splits = max_splits; f.total_wg = batch * hkv * max_splits;
+    f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
+    // Every scores-only shape that it takes (us a call, this kernel / the one it replaces, 32 heads on 8 kv heads: rank 128, 5 x 7488 tokens 17.9 / 21.6; rank
+    // 192, 7 x 39246 124 / 153; rank 256, 2 x 28611 30.9 / 41.8; rank 384, 5 x 2903 19.8 / 21.4, 2 x 81976 135 / 146)
+    if (recon_scores_serves(f, kB, sBb, sBh, sBr, rank)) return launch_recon_scores(f, kB, sBb, sBh, sBr, batch, dtype, rank, st);
+  }
+  // The wave-specialised kernel: rank 512 / 384 / 256, a basis shared by K and V (or scores of a factor that is not 16-byte packets), computed RoPE angles, at most 8 query heads
   // per kv head
   const int64_t need = xkv_recon_workspace_bytes(batch, hkv, rank, sBb);
   if ((so || vshared) && rope && !sin_cos && (rank == 512 || rank == 384 || rank == 256) && hq / hkv <= 8 && workspace && need > 0 &&
@@ -413,10 +424,7 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
     f.num_splits = num_kv_splits; f.kv_lens = kv_lens;
     f.hq = hq; f.hkv = hkv; f.kv_len = kv_len; f.max_splits = max_splits; f.total_wg = batch * hkv * max_splits;
     f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
-    // Scores only at rank 256: the 4-wave kernel, the one instantiation small enough for two workgroups per CU (measured
-    // 10 - 15 % ahead there).  Everything else: the wave-specialised kernel (8 - 13 % ahead of the 4-wave kernel).
-    if (!(so && rank == 256)) return launch_recon_spec(f, kB, sBb, sBh, sBr, batch, dtype, rank, st);
-    return launch_recon_fast_256(f, kB, sBb, sBh, sBr, batch, dtype, st);
+    return launch_recon_spec(f, kB, sBb, sBh, sBr, batch, dtype, rank, st);
   }
   // 8-wave kernels: a value basis of its own beside key ranks 256 / 384 / 512
   if (!so && !vshared && rope && !sin_cos && hq / hkv <= 8 && workspace && need > 0 && workspace_bytes >= need &&
@@ -433,17 +441,6 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
     int rc = launch_recon_duo_b(f, kB, sBb, sBh, sBr, batch, dtype, 2, rank, vA.dim, st);
     if (rc == DUO_NOT_MINE) rc = launch_recon_duo_c(f, kB, sBb, sBh, sBr, batch, dtype, 2, rank, vA.dim, st);
     if (rc != DUO_NOT_MINE) return rc;
-  }
-  // Scores at ranks whose factor fits one wave's registers (128K tokens, 8 kv heads, rank 192: 61 us, generic kernel 88); that
-  // kernel reads kB in 16-byte packets
-  if (so && rope && !sin_cos && rank <= 192 && !((sBb | sBh | sBr) & 7) && (reinterpret_cast<uintptr_t>(kB) & 15) == 0) {
-    FastParams f{};
-    f.q = q_pe; f.kA = kA.ptr; f.sAb = kA.stride_b; f.sAl = kA.stride_l;
-    f.scores = scores_out; f.scores_dtype = scores_dtype;
-    f.num_splits = num_kv_splits; f.kv_lens = kv_lens;
-    f.hq = hq; f.hkv = hkv; f.kv_len = kv_len; f.max_splits = max_splits; f.total_wg = batch * hkv * max_splits;
-    f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
-    return launch_recon_scores(f, kB, sBb, sBh, sBr, batch, dtype, rank, st);
   }
   return dtype == XKV_BF16 ? dispatch_recon<__bf16>(p, batch, vshared, st) : dispatch_recon<_Float16>(p, batch, vshared, st);
 }

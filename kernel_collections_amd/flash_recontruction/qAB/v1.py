@@ -49,11 +49,10 @@ def _scores(q, Ak, Bk, inv_freq, sin_cos, pos_offset, sm_scale, out_dtype):
     Ak = ops.as_rows(Ak)
     Bk = Bk if Bk.stride(-1) == 1 else Bk.contiguous()
     out = torch.empty((bsz, num_heads, 1, kv_len), dtype=out_dtype, device=q.device)
-    # ranks 384 / 512 run the wave-specialised MFMA kernel, one workgroup per CU; rank 256 the 4-wave kernel, whose scores-only
-    # form fits a CU twice (252 registers, 78 KB of LDS); ranks to 192 a kernel of independent waves, one workgroup per CU and 64
-    # tokens per step, or - with a table, or a factor that is not 16-byte packets - the register-staged scores kernel, which keeps 2-3
-    if rank <= 192 and sin_cos is None and ops._row_ok(Bk):
-        n_splits = ops.occupancy_splits(bsz, num_kv_heads, kv_len, tile=64, waves=1)
+    # one workgroup per CU that takes 64 tokens a step, 32 beyond rank 256; with a table, or a factor that is not 16-byte packets,
+    # the register-staged scores kernel, which keeps 2-3 up to rank 256
+    if (rank <= 256 or rank % 64 == 0) and sin_cos is None and ops._row_ok(Bk):
+        n_splits = ops.occupancy_splits(bsz, num_kv_heads, kv_len, tile=64 if rank <= 256 else 32, waves=1)
     else:
         n_splits = ops.occupancy_splits(bsz, num_kv_heads, kv_len, tile=32, waves=1 if rank > 256 else (2 if rank > 128 else 3))
     ops.recon_stage1(q3, Ak, Bk, None, None, None, out, None, None, bsz, num_heads, num_kv_heads, kv_len,

@@ -119,6 +119,22 @@ def test_recon_scores_small_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, of
             assert s[i, ..., n:].isnan().all()      # nothing is written past a sequence
 
 
+@pytest.mark.parametrize("dtype,out", [(BF, torch.float32), (FP, FP), (BF, BF)])
+@pytest.mark.parametrize("b,hq,hkv,L,r,S,lens,off", [
+    (1, 4, 1, 1, 256, 1, None, 0),              # one token
+    (2, 8, 1, 97, 224, 1, [97, 15], 0),         # an odd number of k-steps; two steps, the last of one token; less than a tile
+    (1, 5, 1, 131, 256, 1, None, 7),            # three steps: a tail of every length ...
+    (1, 7, 1, 259, 256, 1, None, 0),            # ... and five: one group of groups and a tail of one
+    (1, 16, 1, 1123, 224, 1, None, 131072),     # 18 steps, angles seeded twice, 16 heads per kv head
+    (1, 6, 2, 2049, 384, 3, None, 5),           # two waves a tile: odd length, several splits
+    (2, 3, 3, 260, 320, 4, [260, 65], 0),       # splits without tokens
+    (1, 16, 2, 33, 512, 1, None, 0), (1, 8, 2, 66, 512, 1, None, 0), (1, 8, 2, 98, 448, 1, None, 0),   # two, three, four steps
+    (1, 8, 2, 640, 512, 1, None, 99999),        # whole steps only, angles seeded twice
+])
+def test_recon_scores_large_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, off):
+    test_recon_scores_small_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, off)
+
+
 @pytest.mark.parametrize("dtype", [BF, FP])
 @pytest.mark.parametrize("b,hq,hkv,L,rk,rv,off", [
     (1, 8, 2, 2049, 192, 512, 0),        # a score row past whole packets by one
