@@ -28,7 +28,7 @@ typedef LatentParams RingParams;
 bool ring_eligible(const RingParams& p, bool vshared);
 int launch_ring(const RingParams& p, bool vshared, int dtype, hipStream_t st);
 // Softmax + P.V over scores that are an input (p.scores: fp32 [batch, hq, kv_len], already scaled); p.C = the value rows
-// (256 / 384 / 512 wide, one row per token for every head), p.groups == 1, hq <= 32, kv_len % 4 == 0.
+// (128 .. 512 wide, one row per token for every head), hq / groups <= 32, kv_len % 4 == 0.
 int launch_ring_given(const RingParams& p, int dtype, hipStream_t st);
 
 }  // namespace xkv

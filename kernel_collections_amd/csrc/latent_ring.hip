@@ -72,6 +72,9 @@ constexpr int RING_DVH = 128;   // head width of the per-head value rows (RING_V
 // token stride, in elements, from which a row pair's second row may be out of reach of a 32-bit lane offset
 constexpr int64_t RING_FAR_STRIDE = 1 << 29;
 
+// rows of `width` features that share a load instruction (16 bytes a lane): two of 192 or 256, four of 128
+__host__ __device__ constexpr int ring_rows_per_load(int width, bool pairs) { return !pairs || width > 256 ? 1 : width > 128 ? 2 : 4; }
+
 template <int TN, int DN, bool HAS_R, int VMODE, int NHB, int DVW>
 struct RingShape {
   static constexpr int HB = 16 * NHB;
@@ -126,7 +129,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   static_assert(DN <= 1024 && DVW <= 1024, "a row takes at most two load instructions");
   constexpr int IPR = DN > 512 ? DN / 512 : 1;    // load instructions per C row (1 KiB each; 768-byte rows use 48 lanes)
   constexpr bool CPART = DN == 384;               // a C row fills only part of a load instruction
-  constexpr int CRI = PAIRS && DN == 256 ? 2 : 1, VRI = PAIRS && DVW == 256 ? 2 : 1;   // rows per load instruction: two 512-byte rows share one
+  constexpr int CRI = ring_rows_per_load(DN, PAIRS), VRI = ring_rows_per_load(DVW, PAIRS);
   // waves 4..7 move the tile rows; each brings TN/4 rows of C (and V) and two 16-byte chunks of every RoPE-key row
   constexpr int QD = RING_QD;
   constexpr int RPW = TN / 4;                     // rows per loader wave per tile
@@ -185,7 +188,6 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   const int r_row = lane & 31;
   if (__builtin_expect(wave >= 4, 1)) {   // laid out first: the sooner the first loads are issued, the shorter the start
     u32x4 rq[QD][LPT];
-    const unsigned pair_off = (lane & 31) * 16;    // two rows per instruction: the upper lanes take the second one
     auto fetch = [&](int t, u32x4 (&q)[LPT]) {
       const int base = start + t * TN;
       int n = 0;
@@ -199,8 +201,13 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
           const unsigned step = RI == 2 && tok < last ? (unsigned)row_bytes : 0;
           tok = tok < last ? tok : last;
           const unsigned char* row = ring_uniform(sbase + (int64_t)tok * row_bytes);
-          if constexpr (RI == 2) {
-            q[n++] = ring_ldg_s<0>(row, pair_off + (lane >= 32 ? step : 0));
+          constexpr int LPR = W / 8;               // lanes of a row
+          if constexpr (RI == 2) {                 // the upper lanes take the second row
+            if (2 * LPR == 64 || lane < 2 * LPR) q[n] = ring_ldg_s<0>(row, (lane < LPR ? lane : lane - LPR) * 16u + (lane >= LPR ? step : 0));
+            ++n;
+          } else if constexpr (RI == 4) {
+            const int sub = lane / LPR, left = last - tok;
+            q[n++] = ring_ldg_s<0>(row, (lane % LPR) * 16u + (unsigned)(sub < left ? sub : left) * (unsigned)row_bytes);
           } else {
             if (W >= 512 || lane < W / 8) {
               q[n] = ring_ldg_s<0>(row, lane_off);
@@ -237,8 +244,10 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
 #pragma unroll
         for (int r = 0; r < RPW; r += RI) {
           unsigned char* row = dst + (iw * RPW + r) * P;
-          if constexpr (RI == 2) {
-            st16(row + (lane >> 5) * P + pair_off, q[n++]);
+          constexpr int LPR = W / 8;
+          if constexpr (RI > 1) {
+            if (RI * LPR == 64 || lane < RI * LPR) st16(row + (lane / LPR) * P + (lane % LPR) * 16, q[n]);
+            ++n;
           } else {
 #pragma unroll
             for (int c = 0; c < NI; ++c, ++n)
@@ -618,14 +627,16 @@ static int ring_vmode(const RingParams& p, bool vshared) {
 // softmax + P.V over given scores: the value rows are the C stream
 template <typename T>
 static int launch_ring_given_dt(const RingParams& p, hipStream_t st) {
-  const int nhb = p.hq <= 16 ? 1 : 2;
+  const int nhb = p.hq / p.groups <= 16 ? 1 : 2;
   const bool far = p.sCl >= RING_FAR_STRIDE;   // no other kernel serves given scores: a row an instruction there
-  if (far && p.dn == 256)
-    return nhb == 1 ? launch_ring_t<T, 32, 1, false, 256, false, RING_VGIVEN, 512, false>(p, st)
-                    : launch_ring_t<T, 32, 2, false, 256, false, RING_VGIVEN, 512, false>(p, st);
+#define XKV_RING_GIVEN(NHB, DN) \
+  if (far && nhb == NHB && p.dn == DN) return launch_ring_t<T, 32, NHB, false, DN, false, RING_VGIVEN, 512, false>(p, st);
+  XKV_RING_GIVEN(1, 256) XKV_RING_GIVEN(2, 256) XKV_RING_GIVEN(1, 192) XKV_RING_GIVEN(2, 192) XKV_RING_GIVEN(1, 128) XKV_RING_GIVEN(2, 128)
+#undef XKV_RING_GIVEN
 #define XKV_RING_GIVEN(NHB, DN) \
   if (nhb == NHB && p.dn == DN) return launch_ring_t<T, 32, NHB, false, DN, false, RING_VGIVEN>(p, st);
   XKV_RING_GIVEN(1, 512) XKV_RING_GIVEN(2, 512) XKV_RING_GIVEN(1, 384) XKV_RING_GIVEN(2, 384) XKV_RING_GIVEN(1, 256) XKV_RING_GIVEN(2, 256)
+  XKV_RING_GIVEN(1, 192) XKV_RING_GIVEN(2, 192) XKV_RING_GIVEN(1, 128) XKV_RING_GIVEN(2, 128)
 #undef XKV_RING_GIVEN
   return XKV_EUNSUPPORTED;
 }

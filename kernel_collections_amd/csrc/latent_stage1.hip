@@ -468,7 +468,7 @@ extern "C" int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, floa
     return XKV_EINVAL;
   if (!cap_fits(num_kv_splits, batch, kv_len, max_splits, split_cap_tokens, split_plan)) return XKV_EINVAL;
   if (dtype != XKV_BF16 && dtype != XKV_F16) return XKV_EDTYPE;
-  if (hq > 32 || (V.dim != 512 && V.dim != 384 && V.dim != 256) || V.stride_h != 0 || V.stride_l < V.dim || (kv_len & 3))
+  if ((V.dim != 512 && V.dim != 384 && V.dim != 256 && V.dim != 192 && V.dim != 128) || V.stride_h != 0 || V.stride_l < V.dim || (kv_len & 3))
     return XKV_EUNSUPPORTED;
   if (!aligned8(V.stride_b) || !aligned8(V.stride_l) || !ptr16(V.ptr) || !ptr16(scores)) return XKV_EALIGN;
   LatentParams p;
@@ -480,10 +480,12 @@ extern "C" int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, floa
   p.dn = V.dim; p.dr = 0; p.dv = V.dim;
   p.partial = partial; p.lse = lse; p.scores = const_cast<float*>(scores); p.scores_dtype = XKV_F32;
   p.num_splits = num_kv_splits; p.kv_lens = kv_lens;
-  p.hq = hq; p.groups = 1; p.kv_len = kv_len; p.max_splits = max_splits; p.split_cap = split_cap_tokens;
+  int groups = cdiv(hq, 32);          // equal groups of at most 32 heads, one workgroup each
+  while (hq % groups) ++groups;
+  p.hq = hq; p.groups = groups; p.kv_len = kv_len; p.max_splits = max_splits; p.split_cap = split_cap_tokens;
   p.split_plan = split_plan;
   p.grid_splits = grid_splits(num_kv_splits, kv_lens, kv_len, max_splits, split_cap_tokens, split_plan);
-  p.total_wg = (packed_rows(num_kv_splits, split_plan) ? 1 : batch) * p.grid_splits;
+  p.total_wg = groups * (packed_rows(num_kv_splits, split_plan) ? 1 : batch) * p.grid_splits;
   p.sm_scale = 1.f; p.logit_cap = 0.f;
   p.heads_in_row = 0;
   return launch_ring_given(p, dtype, (hipStream_t)stream);

@@ -90,19 +90,23 @@ def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_sca
     return ops.merge_stage2(partial, lse, o, None, splits, lens, batch, hq, hq, kv_len, S, split_cap=cap, split_plan=plan)
 
 
-# A value basis of its own runs as two passes (scores, then softmax + P.v_A) at these key ranks once the call scans at
-# least TWO_PASS_MIN_TOKENS tokens (batch x kv_len); below, the extra launches cost more than the second row stream of
-# the fused 8-wave kernel.  Where the two cross depends on the kv heads, each of which rebuilds every token; the line holds the
-# crossings of all but the fewest heads (us fused / two passes, batch 1, key rank 384, value rank 512: 32 heads on 8 kv heads, 16384
-# tokens 44.9 / 46.7, 24576 58.2 / 53.5, 49152 94.4 / 76.0; 16 on 4, 16384 33.9 / 38.2, 49152 62.1 / 55.8; 16 on 2, 49152 45.6 / 47.5,
-# 98304 68.7 / 67.4), and those of the rank pairs without an 8-wave kernel lie lower (512 / 384, 32 on 8: 4096 32.9 / 33.1, 8192 46.4 / 38.8).
+# Two passes (scores, then softmax + P.v_A) or one kernel: scores and values each run at the rate of a kernel made for them, but a third launch and
+# the scores' way through memory cost 5 - 8 us.  Where the two cross is a matter of the tokens scanned (batch x kv_len) times the kv heads, each of
+# which rebuilds them.  us of one kernel / two passes, 32 heads on 8 kv heads unless said:
+#   values of their own: rank 256 / 256, 8192 tokens 25.6 / 29.8, 16384 35.4 / 32.6 (16 on 4: 16384 27.4 / 28.2, 32768 34.3 / 31.1; 16 on 2: 32768 28.1 / 29.7,
+#   65536 39.1 / 37.3); 384 / 512, 16384 41.7 / 44.4, 32768 59.9 / 57.0 (16 on 4: 65536 63.8 / 59.8; 16 on 2: 65536 44.7 / 50.7); 512 / 512, 16384 43.3 / 47.4,
+#   32768 64.1 / 62.3; rank pairs without an 8-wave kernel, 512 / 384: 4096 31.5 / 32.0, 8192 45.6 / 37.3 (16 on 2: 16384 34.9 / 33.8)
+#   one basis: rank 192, 8192 26.4 / 28.4, 16384 34.1 / 31.8, 131072 143 / 78.7 (16 on 2: 65536 34.9 / 34.8); rank 256, 32768 36.1 / 40.0, 65536 60.0 / 56.3 (16 on 4:
+#   65536 40.3 / 42.0, 131072 59.1 / 58.0; 16 on 2: 131072 39.6 / 48.5); rank 384 and 512 one kernel up to 131072 tokens (122 / 130, 142 / 161)
 TWO_PASS_KEY_RANKS = (512, 384, 256)
-TWO_PASS_MIN_TOKENS = 49152
-# Key ranks up to 192 have no 8-wave kernel: two passes from this many tokens on, counted for every kv head, and from five times as many
-# at the ranks that the generic kernel is instantiated for (us fused / two passes: key rank 64, value rank 256, 32 heads on 8 kv heads, 1024
-# tokens 17.6 / 18.9, 4096 27.8 / 24.7; 16 on 4, 2048 19.7 / 20.6, 3072 22.9 / 21.7; 8 on 1, 8192 21.5 / 23.1, 12288 24.1 / 23.4; key rank
-# 192, value rank 512, 32 on 8, 4096 29.1 / 32.7, 8192 39.1 / 40.7, 16384 60.8 / 43.8; batch 16 x 512 35.7 / 33.4; 16 on 2, 16384 30.9 /
-# 34.7; key rank 128, value rank 384, 32 on 8, 8192 34.6 / 35.0).
+TWO_PASS_MIN_TOKENS = 49152         # from here on at 8 kv heads whatever the ranks, and where a caller's counts are taken
+TWO_PASS_WORK = {(256, 256): 98304, (256, 512): 98304, (384, 384): 229376, (384, 512): 229376, (512, 512): 245760}   # pairs with an 8-wave kernel
+TWO_PASS_WORK_OTHER = 32768
+TWO_PASS_WORK_SHARED = {128: (1, 114688), 192: (1, 114688), 256: (4, 409600)}    # least kv heads, tokens x kv heads
+# Key ranks up to 192 have no 8-wave kernel: two passes from this many tokens x kv heads on, and from four times as many at the ranks
+# that the generic kernel is instantiated for (key rank 64, value rank 256, 1024 tokens 17.6 / 18.9, 4096 27.8 / 24.7; 16 on 4, 2048 19.7 / 20.6, 3072 22.9 / 21.7;
+# 8 on 1, 8192 21.5 / 23.1, 12288 24.1 / 23.4; key rank 192, value rank 512, 4096 27.8 / 30.3, 8192 38.3 / 37.4, 16384 59.4 / 40.1; 16 on 4, 8192 28.5 / 30.2, 16384
+# 38.9 / 33.7; 16 on 2, 16384 29.2 / 31.8, 32768 38.7 / 34.5).
 TWO_PASS_SMALL_RANK = 192
 TWO_PASS_MIN_TOKENS_SMALL = 12288
 GENERIC_RANKS = (128, 192)
@@ -111,14 +115,19 @@ GENERIC_RANKS = (128, 192)
 TWO_PASS_MIN_TOKENS_ASKED = 4096
 
 
-def _two_pass(rank, tokens, k_B, asked=False):
+def _two_pass(rank, tokens, k_B, asked=False, v_rank=512, shared=False):
+    hkv = k_B.shape[1]
+    if shared:
+        least, work = TWO_PASS_WORK_SHARED.get(rank, (1, float("inf")))
+        return hkv >= least and tokens * hkv >= work
     if rank in TWO_PASS_KEY_RANKS:
-        return tokens >= TWO_PASS_MIN_TOKENS
+        work = min(TWO_PASS_WORK.get((rank, v_rank), TWO_PASS_WORK_OTHER), 8 * TWO_PASS_MIN_TOKENS)
+        return tokens * hkv >= work or (asked and tokens >= TWO_PASS_MIN_TOKENS)
     if rank > TWO_PASS_SMALL_RANK or not ops._row_ok(k_B):
         return False
     if asked:
         return tokens >= TWO_PASS_MIN_TOKENS_ASKED
-    return tokens * k_B.shape[1] >= TWO_PASS_MIN_TOKENS_SMALL * (5 if rank in GENERIC_RANKS else 1)
+    return tokens * hkv >= TWO_PASS_MIN_TOKENS_SMALL * (4 if rank in GENERIC_RANKS else 1)
 
 
 def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_scale, theta, sin_cos,
@@ -127,7 +136,8 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
     ops.check_splits(num_kv_splits, max_kv_splits, q_pe.shape[0])
     if sin_cos is None and kv_lens is None and ops.USE_RECON_WORKSPACE:
         native = _lib.native()
-        two_pass = _two_pass(k_A.shape[-1], k_A.shape[0] * k_A.shape[1], k_B)
+        shared = v_A is k_A or (v_A.data_ptr() == k_A.data_ptr() and v_A.shape == k_A.shape and v_A.stride() == k_A.stride())
+        two_pass = _two_pass(k_A.shape[-1], k_A.shape[0] * k_A.shape[1], k_B, v_rank=v_A.shape[-1], shared=shared)
         done = native and native.rope_decode(q_pe, k_A, k_B, v_A, v_B, o, sm_scale,
                                              ops.rope_inv_freq(q_pe.shape[-1], theta, q_pe.device), pos_offset, two_pass)
         if done is not None:
@@ -155,7 +165,7 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
             sin_cos = sin_cos.to(q_pe.dtype).contiguous()
     same_basis = (v_A.data_ptr() == k_A.data_ptr() and v_A.shape == k_A.shape and v_A.stride() == k_A.stride())
     asked = (lens is not None and batch > 1) or sin_cos is not None       # the caller's counts are taken
-    if (not same_basis and _two_pass(k_A.shape[-1], batch * kv_len, k_B, asked) and sin_cos is None and hq // hkv <= 8 and hq <= 32
+    if (not same_basis and _two_pass(k_A.shape[-1], batch * kv_len, k_B, asked, rank_v) and sin_cos is None and hq // hkv <= 8 and hq <= 32
             and rank_v in (256, 384, 512) and kv_len % 4 == 0 and ops.USE_RECON_WORKSPACE):
         # A value basis of its own: two passes.  The scores-only form of the reconstruction kernel runs at the rate of the
         # shared-basis fused kernel (one row stream, no P.A); softmax and P.v_A then stream v_A once for all heads at HBM

@@ -162,6 +162,33 @@ def test_two_pass_rope_decode(dev, dtype, b, hq, hkv, L, rk, rv, off, monkeypatc
     check_out(fr.gqa_xKV_rope(qd, kAd, kBd, vAd, vBd, torch.zeros_like(qd), ns, 2, 128 ** -0.5, 5e5, pos_offset=off), ref, "one kernel")
 
 
+@pytest.mark.parametrize("dtype", [BF, FP])
+@pytest.mark.parametrize("b,hq,hkv,L,r,shared", [
+    (1, 8, 2, 2049, 192, True),          # rows of 24 lanes, two an instruction; a score row past whole packets by one
+    (2, 16, 4, 1027, 128, True),         # four rows an instruction; by three
+    (1, 64, 8, 998, 256, True), (1, 64, 8, 700, 256, False),   # two groups of 32 heads over the same values
+    (3, 48, 4, 100, 192, True),          # 12 heads per kv head, groups of 24
+    (1, 4, 1, 5, 128, True), (1, 8, 8, 33, 192, True),
+])
+def test_two_pass_rope_decode_of_one_basis(dev, dtype, b, hq, hkv, L, r, shared, monkeypatch):
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd.flash_recontruction.fused_attention import _fused
+    monkeypatch.setattr(_fused, "TWO_PASS_MIN_TOKENS", 0)
+    q, kA, kB = gen((b, hq, 128), std=0.4, dtype=dtype, seed=1), gen((b, L, r), dtype=dtype, seed=2), \
+        gen((b, hkv, r, 128), std=r ** -0.5, dtype=dtype, seed=3)
+    vA = kA if shared else gen((b, L, r), dtype=dtype, seed=4)
+    vB = gen((b, hkv, r, 128), std=r ** -0.5, dtype=dtype, seed=5)
+    cos, sin = oracle.rope_cos_sin(torch.arange(L), 128, 5e5)
+    ref = oracle.gqa_factorized_rope(*f32(q.unsqueeze(2), kA, kB, vA, vB), cos, sin, sm_scale=128 ** -0.5)[:, :, 0]
+    qd, kAd, kBd, vBd = (t.to(dev) for t in (q, kA, kB, vB))
+    vAd = kAd if shared else vA.to(dev)
+    ns = torch.full((b,), 2, dtype=torch.int32, device=dev)
+    call = lambda: fr.gqa_xKV_rope(qd, kAd, kBd, vAd, vBd, torch.zeros_like(qd), ns, 2, 128 ** -0.5, 5e5)
+    for name, work in (("two passes", 0), ("one kernel", 1 << 40)):
+        monkeypatch.setattr(_fused, "TWO_PASS_WORK_SHARED", {x: (1, work) for x in (128, 192, 256)})
+        check_out(call(), ref, name)
+
+
 @pytest.mark.parametrize("lens,floor,target", [
     ([1], 32, 1),                                   # one sequence, one job
     ([0, 5, 0, 4000, 33, 0], 32, 7),                # sequences without tokens have no rows
