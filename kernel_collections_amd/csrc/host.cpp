@@ -282,6 +282,8 @@ void absorb(const Call& c, const void* q, Ten B, void* hi, void* lo, int64_t bat
   check(p_xkv_absorb_q(q, B.data_ptr(), hi, lo, batch, hq, hkv, d, rank, B.stride(0), sh, B.stride(2), c.dt, c.stream), "xkv_absorb_q");
 }
 bool ring_rank(int64_t r) { return r == 512 || r == 384 || r == 256; }
+// absorbed scans that the LDS-ring kernel serves: key rank 192 only beside values of a ring rank of their own, or for scores (rv 0)
+bool ring_scan(int64_t r, int64_t rv) { return ring_rank(r) || (r == 192 && (rv == 0 || ring_rank(rv))); }
 // an absorbed scan over `rank`-wide rows: the LDS-ring kernel (one workgroup per CU) at ranks 256 .. 512, else the register-staged one
 int scan_splits(const Call& c, int64_t batch, int groups, int64_t kv_len, bool ring) {
   return balanced_splits(batch, groups, kv_len, ring ? 32 : 64, ring ? 1 : 2, c.cus);
@@ -307,10 +309,10 @@ PyObject* nope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int groups = head_groups(hq), odt = code_any(o);
       Ragged rg{};
       Splits s{0, 0, nullptr, nullptr};
-      const int per_cu = ring_rank(r) ? 1 : 2;
+      const int per_cu = ring_scan(r, rv) ? 1 : 2;
       const bool planned = lens.defined() && b > 1;   // one sequence is cut into the splits of the longest it may be
       if (planned) rg = ragged(c, s, b, groups, L, split_floor(b, groups, L, per_cu, c.cus, true), per_cu);
-      else s.S = scan_splits(c, b, groups, L, ring_rank(r));
+      else s.S = scan_splits(c, b, groups, L, ring_scan(r, rv));
       if (lens.defined()) s.lens = lens.data_ptr<int32_t>();
       const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
       const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
@@ -340,7 +342,7 @@ PyObject* nope_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
     at::Tensor out;
     without_gil([&] {
       Call c(q);
-      const int groups = head_groups(hq), S = scan_splits(c, b, groups, L, ring_rank(r));
+      const int groups = head_groups(hq), S = scan_splits(c, b, groups, L, ring_scan(r, 0));
       const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2);
       c.alloc();
       out = at::empty({b, hq, 1, L}, f32 ? c.opts.dtype(at::kFloat) : c.opts);
@@ -486,12 +488,12 @@ PyObject* gqa(PyObject*, PyObject* const* a, Py_ssize_t n) {
         need(vB.dim() == 4 && vB.size(0) == b && vB.size(1) == hkv && vB.size(2) == dv && o.size(2) == vB.size(3));
         up = up_of(vB, hq, c.dt);
       }
-      // 8 kv heads of 128 side by side in a token row: stage 1 serves every head of a split from one workgroup, one per CU
-      const bool row8 = hkv == 8 && d == 128 && hq <= 32 && k.stride(2) == d && k.stride(1) >= 1024;
-      const bool wide8 = row8 && (fact ? ring_rank(dv) && v.stride(1) >= dv : v.stride(2) == d && v.stride(1) >= 1024);
-      // 512-wide token rows beside 512-wide value rows: the same form, against a block-diagonal query
-      const bool wide4 = fact && hkv * d == 512 && dv == 512 && hq <= 32 && k.stride(2) == d;
-      const bool wide = wide8 || wide4;
+      // 2, 4 or 8 kv heads of 128 side by side in a token row: stage 1 serves every head of a split from one workgroup, one per CU
+      const bool rows128 = (hkv == 8 || hkv == 4 || hkv == 2) && d == 128 && hq <= 32 && k.stride(2) == d && k.stride(1) >= hkv * d;
+      const bool in_row = rows128 && (fact ? ring_rank(dv) && v.stride(1) >= dv : v.stride(2) == d && v.stride(1) >= hkv * d);
+      // 512-wide token rows of other heads beside 512-wide value rows: the same form, against a block-diagonal query
+      const bool wide4 = !in_row && fact && hkv * d == 512 && dv == 512 && hq <= 32 && k.stride(2) == d;
+      const bool wide = in_row || wide4;
       const int per_cu = wide ? 1 : 2, groups = wide ? 1 : (int)hkv, longest_floor = wide ? floor_wide : floor_head;
       need(longest_floor > 0);
       const int floor = std::min(longest_floor, split_floor(b, groups, L, per_cu, c.cus, fact));

@@ -16,15 +16,15 @@ struct LatentParams {
   int grid_splits, total_wg;   // total_wg = groups * batch * grid_splits, or groups * max_splits jobs of a packed plan
   int split_cap;   // > 0: no split longer than this many tokens (effective_splits)
   const int32_t* split_plan;   // not null: [0] cap (the cap in force is max(split_cap, it)), [1] jobs, then (sequence, split) pairs
-  int heads_in_row;   // 8: C rows are 8 plain kv heads of 128 side by side and qn holds compact rows [b, hq, 128]; else 0
+  int heads_in_row;   // 2, 4 or 8: C rows are that many plain kv heads of 128 side by side and qn holds compact rows [b, hq, 128]; else 0
   float sm_scale, logit_cap;
 };
 typedef LatentParams RingParams;
 
 // True when the shape is one the ring kernel is built for: 512-wide latent rows (optionally + 64 RoPE features), or
 // 384 / 256 wide ones scanned with an absorbed query (hi + lo parts; the RoPE features too); V the latent itself, scores only, a second row
-// stream 256 / 384 / 512 wide (keys then 256 .. 1024 wide), or plain per-kv-head values [token][8][128] under one shared
-// absorbed key basis or under plain per-head keys taken as one 1024-wide row.  Everything else runs the register-staged kernel.
+// stream 256 / 384 / 512 wide (keys then 192 .. 1024 wide), or plain per-kv-head values [token][heads][128] under one shared
+// absorbed key basis (8 heads) or under plain per-head keys taken as one row (2, 4 or 8).  Everything else runs the register-staged kernel.
 bool ring_eligible(const RingParams& p, bool vshared);
 int launch_ring(const RingParams& p, bool vshared, int dtype, hipStream_t st);
 // Softmax + P.V over scores that are an input (p.scores: fp32 [batch, hq, kv_len], already scaled); p.C = the value rows

@@ -75,7 +75,15 @@ constexpr int64_t RING_FAR_STRIDE = 1 << 29;
 // rows of `width` features that share a load instruction (16 bytes a lane): two of 192 or 256, four of 128
 __host__ __device__ constexpr int ring_rows_per_load(int width, bool pairs) { return !pairs || width > 256 ? 1 : width > 128 ? 2 : 4; }
 
-template <int TN, int DN, bool HAS_R, int VMODE, int NHB, int DVW>
+// A lane's place among the lanes of a load.  Where the rows of an instruction leave lanes over (48 of 64 at 384 and 192 features) those repeat the last
+// ones, load and store alike: under a mask the compiler joins the loaded registers with what they held before, by copies that
+// read values that have not landed (seen at width 192: rows 4 .. 7 of a wave's first tile).
+template <int W, int RI> __device__ __forceinline__ int ring_lane(int lane) {
+  constexpr int USED = W >= 512 ? 64 : RI * W / 8;
+  return USED == 64 || lane < USED ? lane : lane - (64 - USED);
+}
+
+template <int TN, int DN, bool HAS_R, int VMODE, int NHB, int DVW, int HR>
 struct RingShape {
   static constexpr int HB = 16 * NHB;
   static constexpr int CROW = DN * 2 + 16;                 // padded C row (bytes)
@@ -92,11 +100,11 @@ struct RingShape {
   static constexpr int SHM = RSLOT * SLOT + TAIL;
   // staging area of the query rows (no-PE features | RoPE features | pad; a second set for the low-order part).  It lies over
   // the second slot and the tail: neither is written before barrier A of tile 0, and by then the rows are in registers.
-  // (not for the 1024-wide form: its query arrives as compact 128-wide rows and is expanded in registers)
+  // (not where the query arrives as compact 128-wide rows and is expanded in registers)
   static constexpr int QSTRIDE = (DN + (HAS_R ? 64 : 0)) * 2 + 16;
   static constexpr int QST = SLOT;
   static constexpr int qst_bytes(bool lo) { return HB * QSTRIDE * (lo ? 2 : 1); }
-  static constexpr bool qst(bool lo) { return DN != 1024 && VMODE != RING_VGIVEN && QST + qst_bytes(lo) <= 160 * 1024; }
+  static constexpr bool qst(bool lo) { return !HR && VMODE != RING_VGIVEN && QST + qst_bytes(lo) <= 160 * 1024; }
   static constexpr int shm(bool lo) { return qst(lo) && QST + qst_bytes(lo) > SHM ? QST + qst_bytes(lo) : SHM; }
   static_assert(SHM <= 160 * 1024, "ring does not fit the LDS");
 };
@@ -108,18 +116,19 @@ struct RingShape {
 // accumulates kv heads 2w, 2w+1, and query head h multiplies the values of kv head h / (heads per kv head).
 // RING_VGIVEN: no query at all - the scaled scores [b, hq, kv_len] (fp32) are an input, the C rows are the values: softmax
 // and P.V over a value basis of its own, behind a kernel that produced the scores (two-pass fused decode).
-// DN 1024 means eight plain kv heads of 128 side by side in a token row, against compact query rows [b, hq, 128].
+// HR > 0: a row is HR plain kv heads of 128 side by side, against compact query rows [b, hq, 128].
 // PAIRS: two 256-wide rows share a load instruction, whose 32-bit lane offset then spans a token stride (RING_FAR_STRIDE).
-template <typename T, int TN, int NHB, bool LO, int DN, bool HAS_R, int VMODE, int DVW, bool PAIRS>
+template <typename T, int TN, int NHB, bool LO, int DN, bool HAS_R, int VMODE, int DVW, bool PAIRS, int HR>
 __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
-  static_assert(DN != 1024 || (!LO && !HAS_R), "the 1024-wide form is plain per-head keys");
+  static_assert(HR ? DN == HR * 128 && !LO && !HAS_R : DN != 1024, "plain per-head keys side by side");
   typedef typename Elem<T>::vec8 vec8;
-  typedef RingShape<TN, DN, HAS_R, VMODE, NHB, DVW> S;
+  typedef RingShape<TN, DN, HAS_R, VMODE, NHB, DVW, HR> S;
   constexpr bool SCORES = VMODE == RING_SCORES, V2 = VMODE == RING_VDISTINCT || VMODE == RING_VHEADS, VHEADS = VMODE == RING_VHEADS;
   constexpr bool GIVEN = VMODE == RING_VGIVEN;
   static_assert(!GIVEN || (!LO && !HAS_R && TN == 32), "given scores: plain 32-token tiles of value rows");
   constexpr int VIPR = DVW > 512 ? DVW / 512 : 1;   // load instructions per V row
-  constexpr int KVH = DVW / RING_DVH, KVW = VHEADS ? KVH / 4 : 1;   // kv heads of a value row, per wave
+  constexpr int KVH = DVW / RING_DVH, KVW = VHEADS && KVH > 4 ? KVH / 4 : 1;   // kv heads of a value row, per wave
+  constexpr int WPH = VHEADS && KVH < 4 ? 4 / KVH : 1;                          // waves that share a kv head's features
   constexpr int HB = S::HB, CROW = S::CROW, CBYTES = S::CBYTES, VROW = S::VROW, SLOT = S::SLOT, RSLOT = S::RSLOT;
   constexpr int NTB = TN / 16, KSPLIT = S::KSPLIT, SP = S::SP, LDP = S::LDP;
   constexpr int NKS_N = DN / 32, NKS = NKS_N + (HAS_R ? 2 : 0);
@@ -128,7 +137,6 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   static_assert(!HAS_R || TN == 32, "RoPE-key rows need 32-token tiles");
   static_assert(DN <= 1024 && DVW <= 1024, "a row takes at most two load instructions");
   constexpr int IPR = DN > 512 ? DN / 512 : 1;    // load instructions per C row (1 KiB each; 768-byte rows use 48 lanes)
-  constexpr bool CPART = DN == 384;               // a C row fills only part of a load instruction
   constexpr int CRI = ring_rows_per_load(DN, PAIRS), VRI = ring_rows_per_load(DVW, PAIRS);
   // waves 4..7 move the tile rows; each brings TN/4 rows of C (and V) and two 16-byte chunks of every RoPE-key row
   constexpr int QD = RING_QD;
@@ -138,9 +146,9 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   static_assert(RPW % CRI == 0 && RPW % VRI == 0, "whole row pairs");
   static_assert((QD - 1) * LPT <= 63, "vmcnt holds 6 bits");
   constexpr int DV = (VMODE == RING_VSHARED || GIVEN) ? DN : VHEADS ? RING_DVH : DVW;   // value features of an output row
-  constexpr int NVB = VHEADS ? RING_DVH / 16 : DV / 64;   // 16-feature blocks per wave (per kv head under VHEADS)
+  constexpr int NVB = VHEADS ? RING_DVH / 16 / WPH : DV / 64;   // 16-feature blocks per wave (per kv head under VHEADS)
   constexpr int NA2 = VHEADS ? KVW : NHB;
-  static_assert(!VHEADS || (TN == 16 && KVH % 4 == 0), "per-head values: 16-token tiles, kv heads split over 4 waves");
+  static_assert(!VHEADS || KVH % 4 == 0 || 4 % KVH == 0, "per-head values: kv heads split over 4 waves, or waves over kv heads");
   constexpr int TPH = 256 / HB, TPT = TN / TPH;   // softmax threads per head row, tokens per thread
   static_assert(TPT >= 1, "tile too short for the softmax thread map");
 
@@ -202,17 +210,15 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
           tok = tok < last ? tok : last;
           const unsigned char* row = ring_uniform(sbase + (int64_t)tok * row_bytes);
           constexpr int LPR = W / 8;               // lanes of a row
+          const int l = ring_lane<W, RI>(lane);
           if constexpr (RI == 2) {                 // the upper lanes take the second row
-            if (2 * LPR == 64 || lane < 2 * LPR) q[n] = ring_ldg_s<0>(row, (lane < LPR ? lane : lane - LPR) * 16u + (lane >= LPR ? step : 0));
-            ++n;
+            q[n++] = ring_ldg_s<0>(row, (l < LPR ? l : l - LPR) * 16u + (l >= LPR ? step : 0));
           } else if constexpr (RI == 4) {
-            const int sub = lane / LPR, left = last - tok;
-            q[n++] = ring_ldg_s<0>(row, (lane % LPR) * 16u + (unsigned)(sub < left ? sub : left) * (unsigned)row_bytes);
+            const int sub = l / LPR, left = last - tok;
+            q[n++] = ring_ldg_s<0>(row, (l % LPR) * 16u + (unsigned)(sub < left ? sub : left) * (unsigned)row_bytes);
           } else {
-            if (W >= 512 || lane < W / 8) {
-              q[n] = ring_ldg_s<0>(row, lane_off);
-              if (NI > 1) q[n + 1] = ring_ldg_s<1024>(row, lane_off);
-            }
+            q[n] = ring_ldg_s<0>(row, l * 16u);
+            if (NI > 1) q[n + 1] = ring_ldg_s<1024>(row, l * 16u);
             n += NI;
           }
         }
@@ -245,13 +251,12 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
         for (int r = 0; r < RPW; r += RI) {
           unsigned char* row = dst + (iw * RPW + r) * P;
           constexpr int LPR = W / 8;
+          const int l = ring_lane<W, RI>(lane);
           if constexpr (RI > 1) {
-            if (RI * LPR == 64 || lane < RI * LPR) st16(row + (lane / LPR) * P + (lane % LPR) * 16, q[n]);
-            ++n;
+            st16(row + (l / LPR) * P + (l % LPR) * 16, q[n++]);
           } else {
 #pragma unroll
-            for (int c = 0; c < NI; ++c, ++n)
-              if (W >= 512 || lane < W / 8) st16(row + lane_off + c * 1024, q[n]);
+            for (int c = 0; c < NI; ++c, ++n) st16(row + l * 16 + c * 1024, q[n]);
           }
         }
       };
@@ -349,10 +354,10 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
         }
       }
     }
-  } else if constexpr (DN == 1024) {
-    // Eight kv heads of 128 side by side in a token row: the query is block-diagonal and comes as its compact rows
+  } else if constexpr (HR > 0) {
+    // HR kv heads of 128 side by side in a token row: the query is block-diagonal and comes as its compact rows
     // [b, hq, 128]; head row r multiplies only k-steps 4 kvh .. 4 kvh + 3 of its kv head kvh = r / (heads per kv head).
-    const int hpq = hg / 8;
+    const int hpq = hg / HR;
 #pragma unroll
     for (int hb = 0; hb < NHB; ++hb) {
       int row = hb * 16 + n16;
@@ -409,6 +414,7 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
     for (int hb = 0; hb < NA2; ++hb) acc[mb][hb] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int hpk = VHEADS ? hg / KVH : 0;   // query heads per kv head
   const int vcol0 = wave * (DV / 4);
+  const int kvh0 = VHEADS ? (WPH > 1 ? wave / WPH : wave * KVW) : 0, vf0 = WPH > 1 ? wave % WPH * (RING_DVH / WPH) : 0;   // VHEADS: this wave's heads, its features
 
   for (int t = 0; t < ntiles; ++t) {
     __syncthreads();                  // A: tile t is in its slot; every wave is past PV / score write of tile t-1
@@ -516,14 +522,24 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
       const unsigned char* vbase = slot + CBYTES + S::RBYTES;
 #pragma unroll
       for (int j = 0; j < KVW; ++j) {
-        const int kvh = wave * KVW + j;
+        const int kvh = kvh0 + j;
         int prow = hpk * kvh + n16;
         prow = prow < HB - 1 ? prow : HB - 1;
         const float al = alpha_lds[prow];
-        const s16x4r pb = *reinterpret_cast<const s16x4r*>(p_lds + prow * LDP + 4 * g4);
-        const unsigned char* vrow = vbase + (4 * g4 + (n16 >> 2)) * VROW + (kvh * RING_DVH + 4 * (n16 & 3)) * 2;
+        if constexpr (TN == 16) {
+          const s16x4r pb = *reinterpret_cast<const s16x4r*>(p_lds + prow * LDP + 4 * g4);
+          const unsigned char* vrow = vbase + (4 * g4 + (n16 >> 2)) * VROW + (kvh * RING_DVH + vf0 + 4 * (n16 & 3)) * 2;
 #pragma unroll
-        for (int mb = 0; mb < NVB; ++mb) acc[mb][j] = mfma16k16(T(), ring_tr4(vrow + mb * 32), pb, acc[mb][j] * al);
+          for (int mb = 0; mb < NVB; ++mb) acc[mb][j] = mfma16k16(T(), ring_tr4(vrow + mb * 32), pb, acc[mb][j] * al);
+        } else {
+          const vec8 pb = ld16<vec8>(p_lds + prow * LDP + 8 * g4);
+          const unsigned char* vrow = vbase + (8 * g4 + (n16 >> 2)) * VROW + (kvh * RING_DVH + vf0 + 4 * (n16 & 3)) * 2;
+#pragma unroll
+          for (int mb = 0; mb < NVB; ++mb) {
+            const s16x8r a8 = __builtin_shufflevector(ring_tr4(vrow + mb * 32), ring_tr4(vrow + mb * 32 + 4 * VROW), 0, 1, 2, 3, 4, 5, 6, 7);
+            acc[mb][j] = Elem<T>::mfma16(__builtin_bit_cast(vec8, a8), pb, acc[mb][j] * al);
+          }
+        }
       }
     } else {
       constexpr int VR = VMODE == RING_VDISTINCT ? VROW : CROW;
@@ -566,15 +582,15 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   if (VHEADS) {
 #pragma unroll
     for (int j = 0; j < KVW; ++j) {
-      const int hrow = hpk * (wave * KVW + j) + n16;
+      const int hrow = hpk * (kvh0 + j) + n16;
       if (n16 < hpk) {
         const float m = ml_lds[2 * hrow], l = ml_lds[2 * hrow + 1];
         const float inv = 1.f / l;
         const int64_t ph = rows.base + (int64_t)hrow * rows.per_head + split;
-        float* dst = p.partial + ph * RING_DVH + 4 * g4;
+        float* dst = p.partial + ph * RING_DVH + vf0 + 4 * g4;
 #pragma unroll
         for (int mb = 0; mb < NVB; ++mb) *reinterpret_cast<f32x4*>(dst + mb * 16) = acc[mb][j] * inv;
-        if (g4 == 0) p.lse[ph] = m + __logf(l);
+        if (g4 == 0 && vf0 == 0) p.lse[ph] = m + __logf(l);
       }
     }
     return;
@@ -594,10 +610,10 @@ __global__ __launch_bounds__(512) void latent_ring_kernel(const RingParams p) {
   }
 }
 
-template <typename T, int TN, int NHB, bool LO, int DN, bool HAS_R, int VMODE, int DVW = 512, bool PAIRS = true>
+template <typename T, int TN, int NHB, bool LO, int DN, bool HAS_R, int VMODE, int DVW = 512, bool PAIRS = true, int HR = 0>
 static int launch_ring_t(const RingParams& p, hipStream_t st) {
-  constexpr int SHM = RingShape<TN, DN, HAS_R, VMODE, NHB, DVW>::shm(LO);
-  auto kern = latent_ring_kernel<T, TN, NHB, LO, DN, HAS_R, VMODE, DVW, PAIRS>;
+  constexpr int SHM = RingShape<TN, DN, HAS_R, VMODE, NHB, DVW, HR>::shm(LO);
+  auto kern = latent_ring_kernel<T, TN, NHB, LO, DN, HAS_R, VMODE, DVW, PAIRS, HR>;
   static DynLds lds;
   const int e = ensure_dynamic_lds(lds, reinterpret_cast<const void*>(kern), SHM, true);
   if (e != XKV_OK) return e;
@@ -611,9 +627,9 @@ static int launch_ring_t(const RingParams& p, hipStream_t st) {
 // - or plain per-head keys too, viewed as one 1024-wide row against a block-diagonal query (no low-order part)
 static bool ring_vheads(const RingParams& p, bool vshared) {
   const bool absorbed = p.qn_lo && (p.dn == 512 || p.dn == 384 || p.dn == 256);
-  const bool plain_keys = !p.qn_lo && p.dn == 1024 && p.heads_in_row == 8;
-  return !p.scores && !vshared && p.groups * RING_DVH == 1024 && p.dv == RING_DVH && p.sVh == RING_DVH && p.sCh == 0 &&
-         (absorbed || plain_keys) && !p.R && p.hq <= 32 && p.hq % p.groups == 0 && p.sCl >= p.dn && p.sVl >= 1024;
+  const bool plain_keys = !p.qn_lo && p.heads_in_row && p.dn == p.heads_in_row * RING_DVH && p.groups == p.heads_in_row;
+  return !p.scores && !vshared && p.dv == RING_DVH && p.sVh == RING_DVH && p.sCh == 0 && ((absorbed && p.groups == 8) || plain_keys) &&
+         !p.R && p.hq <= 32 && p.hq % p.groups == 0 && p.sCl >= p.dn && p.sVl >= p.groups * RING_DVH;
 }
 
 static int ring_vmode(const RingParams& p, bool vshared) {
@@ -653,9 +669,12 @@ static int launch_ring_dt(const RingParams& p, bool vshared, hipStream_t st) {
   if (lo && (p.hq <= 16 ? 1 : 2) == NHB && p.dn == DN) return launch_ring_t<T, 16, NHB, true, DN, false, RING_VHEADS, 1024>(a, st);
     XKV_RING_VH(1, 512) XKV_RING_VH(2, 512) XKV_RING_VH(1, 384) XKV_RING_VH(2, 384) XKV_RING_VH(1, 256) XKV_RING_VH(2, 256)
 #undef XKV_RING_VH
-    if (p.dn == 1024 && !lo)
-      return p.hq <= 16 ? launch_ring_t<T, 16, 1, false, 1024, false, RING_VHEADS, 1024>(a, st)
-                        : launch_ring_t<T, 16, 2, false, 1024, false, RING_VHEADS, 1024>(a, st);
+    // keys and values of HR heads, one row each: 32-token tiles while the two rows are below 2 KiB
+#define XKV_RING_HR(NHB, HR) \
+  if (!lo && (p.hq <= 16 ? 1 : 2) == NHB && p.heads_in_row == HR) \
+    return launch_ring_t<T, HR < 4 ? 32 : 16, NHB, false, HR * 128, false, RING_VHEADS, HR * 128, true, HR>(a, st);
+    XKV_RING_HR(1, 8) XKV_RING_HR(2, 8) XKV_RING_HR(1, 4) XKV_RING_HR(2, 4) XKV_RING_HR(1, 2) XKV_RING_HR(2, 2)
+#undef XKV_RING_HR
     return XKV_EUNSUPPORTED;
   }
   const int nhb = hg <= 16 ? 1 : 2;
@@ -676,17 +695,26 @@ static int launch_ring_dt(const RingParams& p, bool vshared, hipStream_t st) {
   // is in flight is two tiles: at 256 + 384 a 16-token tile leaves 42 KB of the 60 - 100 a CU needs - 262144 tokens, batch 1: 79.5
   // us with 16-token tiles, 61 with 32), 16-token ones from there on (512 + 512: 85 us against 88.5)
 #define XKV_RING_V2(NHB, LO, DN, DVW) \
-  if (nhb == NHB && lo == LO && p.dn == DN && !r && vm == RING_VDISTINCT && p.dv == DVW) \
+  if (nhb == NHB && lo == LO && p.dn == DN && !p.heads_in_row && !r && vm == RING_VDISTINCT && p.dv == DVW) \
     return launch_ring_t<T, DN + DVW >= 1024 ? 16 : 32, NHB, LO, DN, false, RING_VDISTINCT, DVW>(p, st);
 #define XKV_RING_V2_ALL(LO, DN) \
   XKV_RING_V2(1, LO, DN, 512) XKV_RING_V2(2, LO, DN, 512) XKV_RING_V2(1, LO, DN, 384) XKV_RING_V2(2, LO, DN, 384) \
   XKV_RING_V2(1, LO, DN, 256) XKV_RING_V2(2, LO, DN, 256)
-  XKV_RING_V2_ALL(true, 512) XKV_RING_V2_ALL(true, 384) XKV_RING_V2_ALL(true, 256)   // absorbed query, both factorised
-  XKV_RING_V2_ALL(false, 1024)                                                       // per-head keys as one row, V factorised
+  XKV_RING_V2_ALL(true, 512) XKV_RING_V2_ALL(true, 384) XKV_RING_V2_ALL(true, 256) XKV_RING_V2_ALL(true, 192)   // absorbed query, both factorised
+  // per-head keys as one row, V factorised (16 heads on 2 kv heads, 4 x 32326 tokens, values of rank 256: 97 us register-staged per head)
+#define XKV_RING_HR(NHB, HR, DVW) \
+  if (nhb == NHB && !lo && p.heads_in_row == HR && p.dv == DVW) \
+    return launch_ring_t<T, HR * 128 + DVW >= 1024 ? 16 : 32, NHB, false, HR * 128, false, RING_VDISTINCT, DVW, true, HR>(p, st);
+#define XKV_RING_HR_ALL(HR) \
+  XKV_RING_HR(1, HR, 512) XKV_RING_HR(2, HR, 512) XKV_RING_HR(1, HR, 384) XKV_RING_HR(2, HR, 384) XKV_RING_HR(1, HR, 256) XKV_RING_HR(2, HR, 256)
+  XKV_RING_HR_ALL(8) XKV_RING_HR_ALL(4) XKV_RING_HR_ALL(2)
+#undef XKV_RING_HR_ALL
+#undef XKV_RING_HR
   XKV_RING_V2(1, false, 512, 512) XKV_RING_V2(2, false, 512, 512)                    // plain 512-wide keys and values
 #undef XKV_RING_V2_ALL
 #undef XKV_RING_V2
-  // ranks 384 and 256, one stream (absorbed queries always carry a low part)
+  // ranks 384, 256 and 192, one stream (absorbed queries always carry a low part)
+  XKV_RING_CASE(32, 1, true, 192, false, RING_SCORES)    XKV_RING_CASE(32, 2, true, 192, false, RING_SCORES)
   XKV_RING_CASE(32, 1, true, 384, false, RING_SCORES)    XKV_RING_CASE(32, 2, true, 384, false, RING_SCORES)
   XKV_RING_CASE(32, 1, true, 384, false, RING_VSHARED)   XKV_RING_CASE(32, 2, true, 384, false, RING_VSHARED)
   XKV_RING_CASE(32, 1, true, 256, false, RING_SCORES)    XKV_RING_CASE(32, 2, true, 256, false, RING_SCORES)
@@ -701,8 +729,8 @@ bool ring_eligible(const RingParams& p, bool vshared) {
   if (p.sCl >= RING_FAR_STRIDE || (vm == RING_VDISTINCT && p.sVl >= RING_FAR_STRIDE)) return false;
   if (vm == RING_VHEADS) return true;
   if (hg > 32 || vm < 0) return false;
-  if ((p.dn == 1024) != (p.heads_in_row == 8)) return false;   // the 1024-wide form is only the eight-heads-in-a-row one
-  if (p.dn != 512 && !(p.dn == 1024 && vm == RING_VDISTINCT && !lo) && !((p.dn == 384 || p.dn == 256) && lo)) return false;
+  if (p.heads_in_row) return vm == RING_VDISTINCT && !lo && !r && p.dn == p.heads_in_row * RING_DVH && p.sCl >= p.dn && p.sVl >= p.dv;
+  if (p.dn == 192 ? !lo || r || (vm != RING_SCORES && vm != RING_VDISTINCT) : p.dn != 512 && !((p.dn == 384 || p.dn == 256) && lo)) return false;
   if (r && (p.dr != 64 || vm != RING_VSHARED)) return false;
   if (p.sCl < p.dn || (r && p.sRl < 64) || (vm == RING_VDISTINCT && p.sVl < p.dv)) return false;
   if (vm == RING_VDISTINCT && p.dn == 512 && !lo && p.dv != 512) return false;

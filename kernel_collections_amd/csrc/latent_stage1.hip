@@ -440,17 +440,18 @@ extern "C" int xkv_latent_stage1(xkv_q_operand qn, const void* qn_lo, xkv_q_oper
   const bool vshared = !scores_only && V.ptr == C.ptr && V.stride_b == C.stride_b && V.stride_l == C.stride_l &&
                        V.stride_h == C.stride_h && V.dim == C.dim;
   hipStream_t st = (hipStream_t)stream;
-  // Plain keys of 8 kv heads x 128 side by side in a token row, values either laid out the same way or one shared
-  // 256 .. 512-wide row (V = v_A): one workgroup serves every head of a split.  A token's keys are then one 1024-wide row
-  // against a block-diagonal query (which the kernel builds from the compact rows), so whole 2 KiB rows stream through
+  // Plain keys of 2, 4 or 8 kv heads x 128 side by side in a token row, values either laid out the same way or one shared
+  // 256 .. 512-wide row (V = v_A): one workgroup serves every head of a split.  A token's keys are then one row
+  // against a block-diagonal query (which the kernel builds from the compact rows), so whole rows stream through
   // the LDS ring and the shared value row is read once per token instead of once per kv head.
-  if (!scores_only && !qn_lo && !dr && C.dim == 128 && n_kv_groups == 8 && C.stride_h == 128 && C.stride_l >= 1024 &&
+  const int row_heads = n_kv_groups == 8 || n_kv_groups == 4 || n_kv_groups == 2 ? n_kv_groups : 0;
+  if (!scores_only && !qn_lo && !dr && C.dim == 128 && row_heads && C.stride_h == 128 && C.stride_l >= row_heads * 128 &&
       hq <= 32) {
-    const bool v_heads = V.dim == 128 && V.stride_h == 128 && V.stride_l >= 1024;
+    const bool v_heads = V.dim == 128 && V.stride_h == 128 && V.stride_l >= row_heads * 128;
     const bool v_shared_row = V.stride_h == 0 && (V.dim == 256 || V.dim == 384 || V.dim == 512) && V.stride_l >= V.dim;
     if (v_heads || v_shared_row) {
       LatentParams w = p;
-      w.dn = 1024; w.sCh = 0; w.heads_in_row = 8;
+      w.dn = row_heads * 128; w.sCh = 0; w.heads_in_row = row_heads;
       if (v_shared_row) { w.groups = 1; w.total_wg = p.total_wg / n_kv_groups; }
       if (ring_eligible(w, false)) return launch_ring(w, false, dtype, st);
     }

@@ -71,10 +71,10 @@ def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits,
     kv_len = k_buffer.shape[1]
     q3 = ops._q3(q)
     k_buffer, v_buffer = ops.as_rows(k_buffer), ops.as_rows(v_buffer)
-    # 8 kv heads of 128 side by side in a token row: stage 1 serves every head of a split from one workgroup (whole 2 KiB
+    # 2, 4 or 8 kv heads of 128 side by side in a token row: stage 1 serves every head of a split from one workgroup (whole
     # rows through its LDS ring), so there are hkv times fewer workgroups and a split may be twice as long
-    wide = (hkv * d == 1024 and d == 128 and hq <= 32 and k_buffer.stride(2) == d and v_buffer.stride(2) == d
-            and k_buffer.stride(1) >= 1024 and v_buffer.stride(1) >= 1024)
+    wide = (hkv in (2, 4, 8) and d == 128 and hq <= 32 and k_buffer.stride(2) == d and v_buffer.stride(2) == d
+            and k_buffer.stride(1) >= hkv * d and v_buffer.stride(1) >= hkv * d)
     splits, cap, S, plan = _plan(wide, lens, num_kv_splits, S, batch, hkv, kv_len, q.device, False)
     partial, lse = ops.workspaces(batch, hq, S, dv, q.device, plan)
     ops.latent_stage1(q3, None, None,
@@ -101,12 +101,13 @@ def decode_attention_fwd_v_factorized(q, k_buffer, v_A_buffer, v_B_buffer, o, nu
     kv_len = k_buffer.shape[1]
     q3 = ops._q3(q)
     k_buffer, v_A_buffer = ops.as_rows(k_buffer), ops.as_rows(v_A_buffer)
-    # 8 kv heads of 128 side by side in a token row: stage 1 serves every head of a split from one workgroup, and the value
+    # 2, 4 or 8 kv heads of 128 side by side in a token row: stage 1 serves every head of a split from one workgroup, and the value
     # basis (shared by the heads) is read once per token instead of once per kv head
-    wide8 = hkv * d == 1024 and d == 128 and rv in (256, 384, 512) and hq <= 32 and k_buffer.stride(2) == d
-    # 512-wide token rows (4 x 128, 2 x 256 ...): the same form, with the block-diagonal query built here
-    wide4 = hkv * d == 512 and rv == 512 and hq <= 32 and k_buffer.stride(2) == d
-    splits, cap, S, plan = _plan(wide8 or wide4, lens, num_kv_splits, S, batch, hkv, kv_len, q.device, True)
+    in_row = (hkv in (2, 4, 8) and d == 128 and rv in (256, 384, 512) and hq <= 32 and k_buffer.stride(2) == d
+              and k_buffer.stride(1) >= hkv * d and v_A_buffer.stride(1) >= rv)
+    # 512-wide token rows of other heads (2 x 256, 8 x 64 ...): the same form, with the block-diagonal query built here
+    wide4 = not in_row and hkv * d == 512 and rv == 512 and hq <= 32 and k_buffer.stride(2) == d
+    splits, cap, S, plan = _plan(in_row or wide4, lens, num_kv_splits, S, batch, hkv, kv_len, q.device, True)
     partial, lse = ops.workspaces(batch, hq, S, rv, q.device, plan)
     if wide4:
         ops.latent_stage1(ops.blockdiag_q(q3, hkv), None, None,

@@ -137,3 +137,34 @@ def test_softmax_pv_over_given_scores(dev, dtype, hq):
             ref = p @ V[i, :n].float()
             err = max_abs(o[i].float().cpu(), ref.cpu())
             assert err <= OUT_ATOL, f"given scores hq{hq} dv{dv} {dtype}: sequence {i}: max abs err {err:.3e}"
+
+
+@pytest.mark.parametrize("dtype", [BF, FP], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("hq", [8, 32], ids=["one_head_block", "two_head_blocks"])
+def test_key_rank_192_forms(dev, dtype, hq):
+    lens = [700, 333]
+    run_form(dev, dtype, hq=hq, dn=192, lo=True, rope=False, mode="scores", dv=0, lens=lens, S=2)
+    for dv in (512, 384, 256):
+        run_form(dev, dtype, hq=hq, dn=192, lo=True, rope=False, mode="row", dv=dv, lens=lens, S=2)
+
+
+@pytest.mark.parametrize("dtype", [BF, FP], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("heads,hq", [(2, 2), (2, 16), (2, 32), (4, 12), (4, 32)])
+@pytest.mark.parametrize("dv", [0, 256, 384, 512])
+def test_few_heads_in_a_row(dev, dtype, heads, hq, dv):
+    """Keys of 2 or 4 kv heads of 128 as one row; values laid out the same way (dv 0) or one shared row of dv."""
+    scale, lens, S = 0.5, [1, 33, 500, 777], 2
+    b, L, w = len(lens), max(lens), dv or 128
+    K, q = draw((b, L, heads, 128), 1.0, dtype, dev, 1), draw((b, hq, 128), 128 ** -0.5, dtype, dev, 2)
+    V = draw((b, L, dv) if dv else (b, L, heads, 128), 1.0, dtype, dev, 3)
+    kl, splits = torch.tensor(lens, dtype=torch.int32, device=dev), torch.full((b,), S, dtype=torch.int32, device=dev)
+    partial, lse = ops.workspaces(b, hq, S, w, dev)
+    ops.latent_stage1(q, None, None, (K, K.stride(0), K.stride(1), K.stride(2), 128), None,
+                      (V, V.stride(0), V.stride(1), 0 if dv else V.stride(2), w), partial, lse, None, splits, kl, b, hq, heads, L, S, scale)
+    o = torch.empty(b, hq, w, dtype=torch.float32, device=dev)
+    ops.merge_stage2(partial, lse, o, None, splits, kl, b, hq, hq, L, S)
+    s = torch.einsum("bhd,blhd->bhl", q.float(), K.float().repeat_interleave(hq // heads, dim=2)) * scale
+    vals = V.float().unsqueeze(2).expand(b, L, hq, dv) if dv else V.float().repeat_interleave(hq // heads, dim=2)
+    for i, n in enumerate(lens):
+        ref = torch.einsum("hl,lhd->hd", s[i, :, :n].softmax(-1), vals[i, :n])
+        assert max_abs(o[i].cpu(), ref.cpu()) <= OUT_ATOL, (heads, hq, dv, n)
