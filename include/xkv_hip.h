@@ -249,6 +249,23 @@ int xkv_merge_stage2(const float* partial, const float* lse, void* out,
                      int64_t stride_o_b, int64_t stride_o_h, int out_dtype,
                      float* lse_out, int64_t stride_lse_b, int64_t stride_lse_h, void* stream);
 
+/* Prefix + tail decode (flash_decoding/deepseek_mla/flash_decoding.py:159-255), first launch: xkv_absorb_q for the factorised prefix, and the
+ * attention over the plain tail, one shared key / value row per token ([batch, tail_len, d] / [batch, tail_len, dv], operands as elsewhere):
+ * tail_partial [batch, hq, tail_splits, dv] (normalised) and tail_lse [batch, hq, tail_splits].  A split holds whole 32-token blocks, all
+ * but the last the same number, and every split must hold tokens.  d % 32 == 0, dv % 64 == 0, both <= 512. */
+int xkv_absorb_q_tail(const void* q, const void* B, void* qt_hi, void* qt_lo, int batch, int hq, int hkv, int d, int rank,
+                      int64_t stride_B_b, int64_t stride_B_h, int64_t stride_B_r, xkv_kv_operand k_tail, xkv_kv_operand v_tail,
+                      int tail_len, int tail_splits, float* tail_partial, float* tail_lse, float sm_scale, float logit_cap, int dtype,
+                      void* stream);
+
+/* Last launch: the up-projecting merge of xkv_merge_stage2 (one length, max_splits the splits of every sequence) whose rows are then merged
+ * with the tail's by their log-sum-exps; out and vB of type `dtype`, d_out the tail's dv.  XKV_EUNSUPPORTED for as many splits as
+ * would be folded in every column block: merge the rows first (max_splits 1). */
+int xkv_merge_stage2_tail(const float* partial, const float* lse, void* out, const void* vB, int64_t stride_vB_b, int64_t stride_vB_h,
+                          int64_t stride_vB_r, int d_out, int dtype, int batch, int hq, int hkv, int kv_len, int max_splits, int dv,
+                          const float* tail_partial, const float* tail_lse, int tail_splits, int64_t stride_o_b, int64_t stride_o_h,
+                          void* stream);
+
 /* Split plan for a ragged batch: plan[0] = cap, the smallest multiple of 32, not below floor_tokens, such that
  * sum_b ceil(kv_lens[b] / cap) <= target_jobs; plan[1] = the number of jobs, i.e. live (sequence, split) pairs when
  * sequence b is cut into max(num_kv_splits[b], ceil(kv_lens[b] / cap)) splits; plan[2 + 2 j], plan[3 + 2 j] = sequence and

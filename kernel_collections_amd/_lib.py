@@ -16,7 +16,7 @@ ABI_VERSION = 7
 
 EXPORTS = (
     "xkv_abi_version", "xkv_error_string", "xkv_rope_table", "xkv_absorb_q",
-    "xkv_blockdiag_q", "xkv_latent_stage1", "xkv_recon_stage1", "xkv_recon_workspace_bytes", "xkv_merge_stage2",
+    "xkv_blockdiag_q", "xkv_latent_stage1", "xkv_recon_stage1", "xkv_recon_workspace_bytes", "xkv_merge_stage2", "xkv_merge_stage2_tail", "xkv_absorb_q_tail",
     "xkv_recon_stage1_static", "xkv_rope_apply", "xkv_ceiling_mfma", "xkv_ceiling_stream", "xkv_plan_splits", "xkv_softmax_pv_stage1",
     "xkv_poison_lds",
 )
@@ -73,6 +73,12 @@ def _declare(lib):
     lib.xkv_merge_stage2.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int,
                                      c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int,
                                      c_int64, c_int64, c_int, c_void_p, c_int64, c_int64, c_void_p]
+    lib.xkv_absorb_q_tail.restype = c_int
+    lib.xkv_absorb_q_tail.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int64, c_int64, c_int64,
+                                      KVOperand, KVOperand, c_int, c_int, c_void_p, c_void_p, c_float, c_float, c_int, c_void_p]
+    lib.xkv_merge_stage2_tail.restype = c_int
+    lib.xkv_merge_stage2_tail.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int, c_int,
+                                          c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int64, c_int64, c_void_p]
     lib.xkv_softmax_pv_stage1.restype = c_int
     lib.xkv_softmax_pv_stage1.argtypes = [c_void_p, KVOperand, c_void_p, c_void_p, c_void_p, c_void_p,
                                           c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p]

@@ -32,8 +32,11 @@ namespace {
 #define XKV_SYMBOLS(X)                                                                                              \
   X(xkv_error_string) X(xkv_absorb_q) X(xkv_blockdiag_q) X(xkv_latent_stage1) X(xkv_softmax_pv_stage1) X(xkv_recon_stage1) \
   X(xkv_recon_workspace_bytes) X(xkv_merge_stage2) X(xkv_plan_splits)
+// newer than the version they are in: a library without them has prefix + tail decode declined
+#define XKV_OPTIONAL_SYMBOLS(X) X(xkv_absorb_q_tail) X(xkv_merge_stage2_tail)
 #define XKV_DECLARE(name) decltype(&name) p_##name = nullptr;
 XKV_SYMBOLS(XKV_DECLARE)
+XKV_OPTIONAL_SYMBOLS(XKV_DECLARE)
 #undef XKV_DECLARE
 
 struct CallError : std::runtime_error { using std::runtime_error::runtime_error; };
@@ -571,6 +574,7 @@ PyObject* prefix_tail(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 9, [&]() -> PyObject* {
     Ten q = T(a[0]), kA = T(a[1]), kB = T(a[2]), vA = T(a[3]), vB = T(a[4]), kT = T(a[5]), vT = T(a[6]);
     const float scale = F(a[7]), logit_cap = F(a[8]);
+    need(p_xkv_absorb_q_tail && p_xkv_merge_stage2_tail);
     same(q, {&kA, &kB, &vA, &vB, &kT, &vT});
     need(q.dim() == 3 && kA.dim() == 3 && kB.dim() == 4 && vA.dim() == 3 && vB.dim() == 4 && kT.dim() == 4 && vT.dim() == 4);
     const int64_t b = q.size(0), hq = q.size(1), w = q.size(2), L = kA.size(1), r = kA.size(2), rv = vA.size(2), Lt = kT.size(1);
@@ -587,25 +591,30 @@ PyObject* prefix_tail(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int groups = head_groups(hq);
       const bool shared = vA.data_ptr() == kA.data_ptr() && vA.strides() == kA.strides() && rv == r;
       Splits s1{scan_splits(c, b, groups, L, ring_rank(r)), 0, nullptr, nullptr};
-      // the tail in at most four splits of whole 32-token blocks, every one of them live; a cap states the count, because the rows
-      // of the shared workspace are one more: row 0 is the merged, up-projected prefix with its log-sum-exp
-      const int blocks = cdiv(Lt, 32), per = cdiv(blocks, 4), S2 = cdiv(blocks, per);
+      // the tail: as many splits as it has 32-token blocks, up to 16 of equal numbers of them
+      const int blocks = cdiv(Lt, 32), per = cdiv(blocks, 16), S2 = cdiv(blocks, per);
+      const bool first = rows_first(s1.S, hq, up.hkv, rv);
       const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part1 = c.plan(b * hq * s1.S * rv * 4), lse1 = c.plan(b * hq * s1.S * 4);
-      const int64_t mid = c.plan(rows_first(s1.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
-      const int64_t part = c.plan(b * hq * (1 + S2) * dv * 4), lse = c.plan(b * hq * (1 + S2) * 4);
+      const int64_t mid = c.plan(first ? rows_bytes(b, hq, rv) : 0), part2 = c.plan(b * hq * S2 * dv * 4), lse2 = c.plan(b * hq * S2 * 4);
       c.alloc();
       o = at::empty({b, hq, dv}, c.opts);
-      absorb(c, q.data_ptr(), kB, c.get<void>(hi), c.get<void>(lo), b, hq, w, r);
+      // the query absorbed and the tail attended to in one launch: neither depends on the other
+      check(p_xkv_absorb_q_tail(q.data_ptr(), kB.data_ptr(), c.get<void>(hi), c.get<void>(lo), b, hq, groups, w, r, kB.stride(0), 0, kB.stride(2),
+                                kv(kT, 0, w), kv(vT, 0, dv), Lt, S2, c.get<float>(part2), c.get<float>(lse2), scale, logit_cap, c.dt, c.stream),
+            "xkv_absorb_q_tail");
       check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(kA, 0, r), NO_KV, shared ? kv(kA, 0, r) : kv(vA, 0, rv),
                                 c.get<float>(part1), c.get<float>(lse1), nullptr, 0, nullptr, nullptr, b, hq, groups, L, s1.S, 0, nullptr, scale,
                                 logit_cap, c.dt, c.stream), "xkv_latent_stage1");
-      float *pf = c.get<float>(part), *lf = c.get<float>(lse);
-      merge(c, c.get<float>(part1), c.get<float>(lse1), pf, hq * (1 + S2) * dv, (1 + S2) * dv, XKV_F32, &up, mid, s1, b, hq, L, rv, lf,
-            hq * (1 + S2), 1 + S2);
-      check(p_xkv_latent_stage1({q.data_ptr(), (int)w}, nullptr, NO_Q, kv(kT, 0, w), NO_KV, kv(vT, 0, dv), pf + dv, lf + 1, nullptr, 0, nullptr,
-                                nullptr, b, hq, groups, Lt, 1 + S2, 32 * per, nullptr, scale, logit_cap, c.dt, c.stream), "xkv_latent_stage1");
-      const Splits s2{1 + S2, 0, nullptr, nullptr};
-      merge(c, pf, lf, o.data_ptr(), hq * dv, dv, c.dt, nullptr, 0, s2, b, hq, 32 * (1 + S2), dv);   // every row live
+      const float *rows = c.get<float>(part1), *rows_lse = c.get<float>(lse1);
+      int n_rows = s1.S, len = L;
+      if (first) {   // many splits: merged by the whole chip, then one row per head
+        float* m = c.get<float>(mid);
+        check(p_xkv_merge_stage2(rows, rows_lse, m, nullptr, 0, 0, 0, 0, XKV_BF16, nullptr, nullptr, b, hq, hq, L, s1.S, 0, nullptr, rv, hq * rv, rv,
+                                 XKV_F32, m + b * hq * rv, hq, 1, c.stream), "xkv_merge_stage2");
+        rows = m; rows_lse = m + b * hq * rv; n_rows = 1; len = 32;
+      }
+      check(p_xkv_merge_stage2_tail(rows, rows_lse, o.data_ptr(), up.p, up.sb, up.sh, up.sr, up.d_out, c.dt, b, hq, up.hkv, len, n_rows, rv,
+                                    c.get<float>(part2), c.get<float>(lse2), S2, hq * dv, dv, c.stream), "xkv_merge_stage2_tail");
     });
     return THPVariable_Wrap(o);
   });
@@ -648,6 +657,9 @@ PyObject* init(PyObject*, PyObject* path) {
   p_##name = reinterpret_cast<decltype(p_##name)>(dlsym(h, #name));                        \
   if (!p_##name) { PyErr_Format(PyExc_RuntimeError, "%s has no " #name, p); return nullptr; }
   XKV_SYMBOLS(XKV_RESOLVE)
+#undef XKV_RESOLVE
+#define XKV_RESOLVE(name) p_##name = reinterpret_cast<decltype(p_##name)>(dlsym(h, #name));
+  XKV_OPTIONAL_SYMBOLS(XKV_RESOLVE)
 #undef XKV_RESOLVE
   Py_RETURN_NONE;
 }

@@ -326,7 +326,7 @@ __global__ __launch_bounds__(256, 1) void recon_scores_kernel(const FastParams p
   };
   auto dot = [&](auto pb_c, auto part_c, f32x4 s) {   // lane (head n16, g4): tokens 4 g4 + r
     const sc_vec8 kop = {kw[0][0], kw[0][1], kw[1][0], kw[1][1], kw[2][0], kw[2][1], kw[3][0], kw[3][1]};
-    return Elem<sc_t>::mfma16(kop, qb[decltype(pb_c)::value & 1][decltype(part_c)::value], s);
+    return Elem<sc_t>::mfma16(kop, qb[decltype(pb_c)::value & 1][decltype(part_c)::value % (LO ? 2 : 1)], s);
   };
   // Block PB of the tile in use: its matrix instructions, one by one, with the rotation of the block before dealt out among
   // them, and the q-dot of the one before that in front.  A wave that issues in order has both pipes wait for each other if either's

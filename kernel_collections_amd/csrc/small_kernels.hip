@@ -6,6 +6,9 @@
 
 namespace xkv {
 
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+
 // ----------------------------------------------------------------------------------------------
 // RoPE table.  angle = float(pos) * inv_freq[j] in fp32 (one rounding), then sincosf with full
 // range reduction - the eager closed form of the reference (rope/rope_ref.py:3-9), not the
@@ -107,16 +110,16 @@ __global__ __launch_bounds__(256) void absorb_q_kernel(
 // d 512 too.  The kernel is latency - a launch and a round trip - whatever the shape: by trace 3.5 us at 8 x 32 heads, d 128,
 // rank 512 (the LDS form it replaces: 4.4) and 4.6 us at 8 x 16 heads, d 512, rank 256 (15.5; 6.3 without KSPLIT).
 template <typename T, bool KSPLIT>
-__global__ __launch_bounds__(256) void absorb_q_mfma_kernel(
+__device__ __forceinline__ void absorb_q_mfma(
     const T* __restrict__ q, const T* __restrict__ B, T* __restrict__ qt_hi, T* __restrict__ qt_lo,
-    int hq, int hkv, int d, int rank, int64_t sBb, int64_t sBh, int64_t sBr) {
+    int hq, int hkv, int d, int rank, int64_t sBb, int64_t sBh, int64_t sBr, int head_block, int b, int rank_block) {
   typedef typename Elem<T>::vec8 vec8;
   constexpr int NK = KSPLIT ? 4 : 8;   // k-steps in flight
   __shared__ f32x4 part[KSPLIT ? 3 : 1][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n16 = lane & 15, g4 = lane >> 4;
   const int G = hq / hkv, nhb = (G + 15) / 16;
-  const int kh = blockIdx.x / nhb, g0 = (blockIdx.x % nhb) * 16, b = blockIdx.y;
-  const int rho = (KSPLIT ? blockIdx.z : blockIdx.z * 4 + wave) * 16 + n16;
+  const int kh = head_block / nhb, g0 = (head_block % nhb) * 16;
+  const int rho = (KSPLIT ? rank_block : rank_block * 4 + wave) * 16 + n16;
   const int gn = G - g0 < 16 ? G - g0 : 16;
   // head rows past the group and rows past the rank repeat the last one: their products are never written
   const T* qrow = q + ((int64_t)b * hq + (int64_t)kh * G + g0 + (n16 < gn ? n16 : gn - 1)) * d + 8 * g4;
@@ -151,6 +154,141 @@ __global__ __launch_bounds__(256) void absorb_q_mfma_kernel(
       qt_hi[o] = hi;
       if (qt_lo) qt_lo[o] = from_f32<T>(acc[r] - to_f32(hi));
     }
+}
+
+template <typename T, bool KSPLIT>
+__global__ __launch_bounds__(256) void absorb_q_mfma_kernel(
+    const T* __restrict__ q, const T* __restrict__ B, T* __restrict__ qt_hi, T* __restrict__ qt_lo,
+    int hq, int hkv, int d, int rank, int64_t sBb, int64_t sBh, int64_t sBr) {
+  absorb_q_mfma<T, KSPLIT>(q, B, qt_hi, qt_lo, hq, hkv, d, rank, sBb, sBh, sBr, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// ----------------------------------------------------------------------------------------------
+// Prefix + tail decode starts with two things that do not depend on each other and leave most of the device idle: the query's absorption
+// for the prefix, and the attention over the plain tail of recently decoded tokens.  One launch does both: the first
+// `absorbing` workgroups absorb, the others take a split of the tail each, all heads of a group of at most 32.
+// A tail workgroup: `tiles` tiles of 32 tokens with a running maximum.  Scores on v_mfma_f32_16x16x32, a wave for 16 tokens x 16 heads, operands
+// straight from memory; the value tile goes through the LDS and is read transposed.  A launch saved is 5 - 9 us of prefix + tail calls that
+// take 29 (3033 + 97 tokens, 8 heads) to 115 us (262144 + 128); the splits of the tail, four before, are as many as the tail has tiles up to
+// TAIL_SPLITS: 4 x (20780 + 1822) tokens spent 35 us in four workgroups per sequence.
+// ----------------------------------------------------------------------------------------------
+constexpr int TAIL_SPLITS = 16;
+struct TailParams {
+  const void* k; const void* v;
+  int64_t sKb, sKl, sVb, sVl;
+  float* partial; float* lse;        // [batch, hq, splits, dv], [batch, hq, splits]
+  int len, splits, tiles, groups, dv, absorbing, head_blocks, rank_blocks;
+  float sm_scale, logit_cap;
+};
+__device__ __forceinline__ s16x4 tail_tr4(const unsigned char* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+}
+template <typename T, bool KSPLIT>
+__global__ __launch_bounds__(256) void absorb_tail_kernel(
+    const T* __restrict__ q, const T* __restrict__ B, T* __restrict__ qt_hi, T* __restrict__ qt_lo,
+    int hq, int hkv, int d, int rank, int64_t sBb, int64_t sBh, int64_t sBr, const TailParams t) {
+  typedef typename Elem<T>::vec8 vec8;
+  if ((int)blockIdx.x < t.absorbing) {
+    const int i = blockIdx.x, hb = i % t.head_blocks, b = i / t.head_blocks / t.rank_blocks;
+    absorb_q_mfma<T, KSPLIT>(q, B, qt_hi, qt_lo, hq, hkv, d, rank, sBb, sBh, sBr, hb, b, i / t.head_blocks % t.rank_blocks);
+    return;
+  }
+  constexpr int SP = 32 + 4, LDP = 32 + 8, NVB = 8;
+  __shared__ float s_lds[32][SP];
+  __shared__ T p_lds[32][LDP];
+  __shared__ float a_lds[32], l_lds[32];
+  extern __shared__ __attribute__((aligned(16))) unsigned char vtile[];   // [32 tokens][dv + 8]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n16 = lane & 15, g4 = lane >> 4;
+  const int j = blockIdx.x - t.absorbing, split = j % t.splits, group = j / t.splits % t.groups, b = j / t.splits / t.groups;
+  const int hg = hq / t.groups, h0 = group * hg;
+  const int start = split * t.tiles * 32, end = min(t.len, start + t.tiles * 32), last = end - 1;
+  const int tb = wave & 1, hb = wave >> 1, head = hb * 16 + n16;
+  // head rows past the group and tokens past the end repeat the last ones: never written, or weighted by zero
+  const T* qrow = q + ((int64_t)b * hq + h0 + (head < hg ? head : hg - 1)) * d + 8 * g4;
+  const T* kb = reinterpret_cast<const T*>(t.k) + b * t.sKb + 8 * g4;
+  const T* vb = reinterpret_cast<const T*>(t.v) + b * t.sVb;
+  const int vrow_bytes = t.dv * 2 + 16, ppr = t.dv / 8, nvb = t.dv / 64;
+  const int srow = tid >> 3, ssub = tid & 7;
+  float m_run = NEG_INF, l_run = 0.f;
+  f32x4 acc[NVB][2];
+#pragma unroll
+  for (int mb = 0; mb < NVB; ++mb) acc[mb][0] = acc[mb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int base = start; base < end; base += 32) {
+    if (base > start) __syncthreads();               // the tile before has been read
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    if (hb * 16 < hg) {
+      const int tok = base + tb * 16 + n16;
+      const T* krow = kb + (int64_t)(tok < last ? tok : last) * t.sKl;
+      for (int c0 = 0; c0 < d; c0 += 256) {
+        vec8 a[8], w[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          a[k] = w[k] = vec8{0, 0, 0, 0, 0, 0, 0, 0};
+          if (c0 + 32 * k < d) { a[k] = ld16<vec8>(krow + c0 + 32 * k); w[k] = ld16<vec8>(qrow + c0 + 32 * k); }
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s = Elem<T>::mfma16(a[k], w[k], s);
+      }
+    }
+    for (int i = tid; i < 32 * ppr; i += 256) {
+      const int r = i / ppr, c = i - r * ppr, tok = base + r;
+      st16(vtile + r * vrow_bytes + c * 16, ld16<vec8>(vb + (int64_t)(tok < last ? tok : last) * t.sVl + c * 8));
+    }
+    if (hb * 16 < hg) *reinterpret_cast<f32x4*>(&s_lds[head][tb * 16 + 4 * g4]) = s;   // lane (head n16, g4): tokens 4 g4 + r
+    __syncthreads();
+    if (srow < hg) {                                  // 8 threads a head, 4 tokens each
+      float sv[4], mx = NEG_INF, sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x = s_lds[srow][ssub * 4 + i] * t.sm_scale;
+        if (t.logit_cap > 0.f) x = t.logit_cap * tanhf(x / t.logit_cap);
+        sv[i] = base + ssub * 4 + i < end ? x : NEG_INF;
+        mx = fmaxf(mx, sv[i]);
+      }
+      const float m_new = fmaxf(m_run, row_reduce<true, 8>(mx)), alpha = __expf(m_run - m_new);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float e = __expf(sv[i] - m_new);
+        sum += e;
+        p_lds[srow][ssub * 4 + i] = from_f32<T>(e);
+      }
+      l_run = l_run * alpha + row_reduce<false, 8>(sum);
+      m_run = m_new;
+      if (ssub == 0) a_lds[srow] = alpha;
+    }
+    __syncthreads();
+    // every wave a quarter of the features
+#pragma unroll
+    for (int hb2 = 0; hb2 < 2; ++hb2)
+      if (hb2 * 16 < hg) {
+        const int row = hb2 * 16 + n16 < hg ? hb2 * 16 + n16 : hg - 1;
+        const float al = a_lds[row];
+        const vec8 pb = ld16<vec8>(&p_lds[row][8 * g4]);
+        const unsigned char* vrow = vtile + (8 * g4 + (n16 >> 2)) * vrow_bytes + (wave * (t.dv / 4) + 4 * (n16 & 3)) * 2;
+#pragma unroll
+        for (int mb = 0; mb < NVB; ++mb)
+          if (mb < nvb) {
+            const s16x8 a = __builtin_shufflevector(tail_tr4(vrow + mb * 32), tail_tr4(vrow + mb * 32 + 4 * vrow_bytes), 0, 1, 2, 3, 4, 5, 6, 7);
+            acc[mb][hb2] = Elem<T>::mfma16(__builtin_bit_cast(vec8, a), pb, acc[mb][hb2] * al);
+          }
+      }
+  }
+  if (srow < hg && ssub == 0) {
+    l_lds[srow] = l_run;
+    t.lse[((int64_t)b * hq + h0 + srow) * t.splits + split] = m_run + __logf(l_run);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int hb2 = 0; hb2 < 2; ++hb2) {
+    const int h = hb2 * 16 + n16;
+    if (h < hg) {
+      const float inv = 1.f / l_lds[h];
+      float* dst = t.partial + (((int64_t)b * hq + h0 + h) * t.splits + split) * t.dv + wave * (t.dv / 4) + 4 * g4;
+#pragma unroll
+      for (int mb = 0; mb < NVB; ++mb)
+        if (mb < nvb) *reinterpret_cast<f32x4*>(dst + mb * 16) = acc[mb][hb2] * inv;
+    }
+  }
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -291,13 +429,17 @@ constexpr int MERGE_CB = 64;       // columns per workgroup: whole 128-byte line
 constexpr int MERGE_UP_T = 512;
 enum { MANY_LOOP = 1, MANY_SPREAD = 2 };
 constexpr int MERGE_ROWS_FLOATS = 49152;   // partial values a workgroup folds in every column block at most; measured in host.cpp
-template <typename O, typename TB, int RPT, int MANY>
+//
+// TAIL: the up-projected row is merged with rows that are in output space already (the plain tail beside a factorised prefix), by their
+// log-sum-exps.  Their packets are folded while the merged rows are; a kernel of its own for it was 4 - 5 us more.
+struct MergeTail { const float* partial; const float* lse; int splits; };   // [batch, hq, splits, d_out], [batch, hq, splits]
+template <typename O, typename TB, int RPT, int MANY, bool TAIL>
 __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     const float* __restrict__ partial, const float* __restrict__ lse, O* __restrict__ out,
     const TB* __restrict__ vB, int64_t sVb, int64_t sVh, int64_t sVr, int d_out,
     const int32_t* __restrict__ num_kv_splits, const int32_t* __restrict__ kv_lens,
     int hq, int hkv, int kv_len, int max_splits, int dv, int64_t sOb, int64_t sOh, int hpw,
-    float* __restrict__ lse_out, int64_t sLb, int64_t sLh, int split_cap, const int32_t* __restrict__ split_plan) {
+    float* __restrict__ lse_out, int64_t sLb, int64_t sLh, int split_cap, const int32_t* __restrict__ split_plan, const MergeTail tail) {
   typedef typename Elem<TB>::vec8 vec8;
   extern __shared__ float merged[];               // [hpw][dv]; MANY_SPREAD: then a packet, a maximum and a sum of every thread
   __shared__ float tot[4][4 * MERGE_CB];          // [quarter of the row groups][4 heads x 64 columns]
@@ -320,11 +462,25 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
   const int L = kv_lens ? kv_lens[b] : kv_len;
   const int nlive = live_splits(L, effective_splits(L, asked_splits(num_kv_splits, b, max_splits, split_cap), split_cap_in_force(split_cap, split_plan)), max_splits);
   const PartialRows rows = partial_rows(b, hq, max_splits, num_kv_splits, split_plan);
+  float* head_lse = merged + hpw * dv;            // TAIL: [hpw][3] prefix log-sum-exp, the tail's maximum and sum; then [hpw][MERGE_CB] its rows
+  if constexpr (TAIL) {
+    float* rows_t = head_lse + 3 * hpw;
+    for (int i = tid; i < hpw * MERGE_CB; i += MERGE_UP_T) {
+      const int gi = i / MERGE_CB, c = c0 + i % MERGE_CB;
+      if (c < d_out) {
+        const int64_t row = ((int64_t)b * hq + hfirst + gi) * tail.splits;
+        const MergeAcc<1> a = merge_fold<1>(tail.lse + row, tail.partial + row * d_out + c, d_out, 0, 1, tail.splits);
+        rows_t[i] = a.acc[0];
+        if (c == c0) { head_lse[3 * gi + 1] = a.m; head_lse[3 * gi + 2] = a.l; }
+      }
+    }
+  }
   auto merge_packet = [&](int gi, int c, auto tag) {
     constexpr int P = decltype(tag)::value;
     const int64_t row = rows.base + (int64_t)(hfirst + gi) * rows.per_head;
     // a single row's weight is 1 whatever its log-sum-exp
-    const MergeAcc<P> a = merge_fold<P>(max_splits == 1 && !lse_out ? nullptr : lse + row, partial + row * dv + c, dv, 0, 1, nlive);
+    const MergeAcc<P> a = merge_fold<P>(max_splits == 1 && !lse_out && !TAIL ? nullptr : lse + row, partial + row * dv + c, dv, 0, 1, nlive);
+    if (TAIL && c == 0) head_lse[3 * gi] = a.m + __logf(a.l);
     const float inv = nlive > 0 ? 1.f / a.l : 0.f;
 #pragma unroll
     for (int e = 0; e < P; ++e) merged[gi * dv + c + e] = a.acc[e] * inv;
@@ -409,8 +565,14 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
       __syncthreads();
       if (tid < 4 * MERGE_CB) {
         const int gi = tid / MERGE_CB, c = c0 + tid % MERGE_CB;
-        if (g0 + gi < hpw && c < d_out)
-          out[b * sOb + (hfirst + g0 + gi) * sOh + c] = (O)(tot[0][tid] + tot[1][tid] + tot[2][tid] + tot[3][tid]);
+        if (g0 + gi < hpw && c < d_out) {
+          float v = tot[0][tid] + tot[1][tid] + tot[2][tid] + tot[3][tid];
+          if constexpr (TAIL) {
+            const float *h = head_lse + 3 * (g0 + gi), M = fmaxf(h[0], h[1]), wp = __expf(h[0] - M), wt = __expf(h[1] - M);
+            v = (v * wp + head_lse[3 * hpw + (g0 + gi) * MERGE_CB + c - c0] * wt) / (wp + h[2] * wt);
+          }
+          out[b * sOb + (hfirst + g0 + gi) * sOh + c] = (O)v;
+        }
       }
       __syncthreads();            // tot is reused by the next four heads, or the next columns
     }
@@ -434,7 +596,7 @@ template <typename O, typename TB>
 static int launch_merge(const float* partial, const float* lse, void* out, const void* vB, int64_t sVb, int64_t sVh,
                         int64_t sVr, int d_out, const int32_t* ns, const int32_t* kl, int batch, int hq, int hkv,
                         int kv_len, int max_splits, int dv, int64_t sOb, int64_t sOh, float* lse_out, int64_t sLb, int64_t sLh,
-                        int split_cap, const int32_t* split_plan, hipStream_t st) {
+                        int split_cap, const int32_t* split_plan, const MergeTail& tail, hipStream_t st) {
   // splits one sequence may have (a packed plan's max_splits counts the jobs of the whole batch)
   const int seq_splits = packed_rows(ns, split_plan) ? std::min(max_splits, cdiv(kv_len, split_cap)) : max_splits;
   // what one head takes of the LDS was bounded when the weights of all its splits were held there; the bound stays part of the
@@ -471,13 +633,23 @@ static int launch_merge(const float* partial, const float* lse, void* out, const
   if (spread) hpw = 1;
   if (many) z = (int)std::min<int64_t>(z, cdiv(256, std::min<int64_t>(256, (int64_t)(hq / hpw) * batch)));
   const dim3 grid(hq / hpw, batch, z);
-  const size_t shm = ((size_t)hpw * dv + (spread ? MERGE_UP_T * 6 : 0)) * sizeof(float);
-#define XKV_MERGE_UP(RPT, MANY)                                                                                                      \
-  merge_up_kernel<O, TB, RPT, MANY><<<grid, dim3(MERGE_UP_T), shm, st>>>(partial, lse, (O*)out, (const TB*)vB, sVb, sVh, sVr, d_out, ns, kl, \
-                                                         hq, hkv, kv_len, max_splits, dv, sOb, sOh, hpw, lse_out, sLb, sLh, split_cap, split_plan)
+  const size_t shm = ((size_t)hpw * dv + (spread ? MERGE_UP_T * 6 : 0) + (tail.splits ? hpw * (MERGE_CB + 3) : 0)) * sizeof(float);
+#define XKV_MERGE_UP_TAIL(RPT, MANY, TAIL)                                                                                           \
+  merge_up_kernel<O, TB, RPT, MANY, TAIL><<<grid, dim3(MERGE_UP_T), shm, st>>>(partial, lse, (O*)out, (const TB*)vB, sVb, sVh, sVr, d_out, ns, kl, \
+                                                         hq, hkv, kv_len, max_splits, dv, sOb, sOh, hpw, lse_out, sLb, sLh, split_cap, split_plan, tail)
+#define XKV_MERGE_UP(RPT, MANY) XKV_MERGE_UP_TAIL(RPT, MANY, false)
+  if (tail.splits) {
+    if (many) return XKV_EUNSUPPORTED;   // the caller merges the rows first
+    if constexpr (std::is_same<O, TB>::value) {
+      if (dv <= 256) XKV_MERGE_UP_TAIL(4, 0, true); else XKV_MERGE_UP_TAIL(8, 0, true);
+      return launch_status();
+    }
+    return XKV_EDTYPE;
+  }
   if (dv <= 256) { if (spread) XKV_MERGE_UP(4, MANY_SPREAD); else if (many) XKV_MERGE_UP(4, MANY_LOOP); else XKV_MERGE_UP(4, 0); }
   else { if (spread) XKV_MERGE_UP(8, MANY_SPREAD); else if (many) XKV_MERGE_UP(8, MANY_LOOP); else XKV_MERGE_UP(8, 0); }
 #undef XKV_MERGE_UP
+#undef XKV_MERGE_UP_TAIL
   return launch_status();
 }
 
@@ -754,7 +926,7 @@ extern "C" int xkv_merge_stage2(const float* partial, const float* lse, void* ou
   if (vB && (d_out <= 0 || d_out > 512 || d_out % 8)) return XKV_EUNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
 #define XKV_MERGE(O, TB) \
-  return launch_merge<O, TB>(partial, lse, out, vB, sVb, sVh, sVr, d_out, ns, kl, batch, hq, hkv, kv_len, max_splits, dv, sOb, sOh, lse_out, sLb, sLh, split_cap_tokens, split_plan, st)
+  return launch_merge<O, TB>(partial, lse, out, vB, sVb, sVh, sVr, d_out, ns, kl, batch, hq, hkv, kv_len, max_splits, dv, sOb, sOh, lse_out, sLb, sLh, split_cap_tokens, split_plan, MergeTail{nullptr, nullptr, 0}, st)
   const int bt = vB ? vB_dtype : XKV_BF16;
   if (bt != XKV_BF16 && bt != XKV_F16) return XKV_EDTYPE;
   switch (out_dtype) {
@@ -764,4 +936,62 @@ extern "C" int xkv_merge_stage2(const float* partial, const float* lse, void* ou
     default: return XKV_EDTYPE;
   }
 #undef XKV_MERGE
+}
+
+extern "C" int xkv_absorb_q_tail(const void* q, const void* B, void* qt_hi, void* qt_lo, int batch, int hq, int hkv, int d, int rank,
+                                 int64_t sBb, int64_t sBh, int64_t sBr, xkv_kv_operand k_tail, xkv_kv_operand v_tail, int tail_len,
+                                 int tail_splits, float* tail_partial, float* tail_lse, float sm_scale, float logit_cap, int dtype,
+                                 void* stream) {
+  if (!q || !B || !qt_hi || !k_tail.ptr || !v_tail.ptr || !tail_partial || !tail_lse || batch <= 0 || hq <= 0 || hkv <= 0 || d <= 0 ||
+      rank <= 0 || tail_len <= 0 || tail_splits <= 0)
+    return XKV_EINVAL;
+  if (hq % hkv || hq / hkv > 32 || d > 512 || d % 32 || k_tail.dim != d || v_tail.dim <= 0 || v_tail.dim % 64 || v_tail.dim > 512)
+    return XKV_EUNSUPPORTED;
+  const int blocks = cdiv(tail_len, 32), tiles = cdiv(blocks, tail_splits);
+  if (cdiv(blocks, tiles) != tail_splits) return XKV_EINVAL;   // every split of the tail holds tokens
+  if ((sBr | sBh | sBb | k_tail.stride_b | k_tail.stride_l | v_tail.stride_b | v_tail.stride_l) & 7 ||
+      ((uintptr_t)B | (uintptr_t)q | (uintptr_t)k_tail.ptr | (uintptr_t)v_tail.ptr | (uintptr_t)tail_partial) & 15)
+    return XKV_EALIGN;
+  if (dtype != XKV_BF16 && dtype != XKV_F16) return XKV_EDTYPE;
+  TailParams t;
+  t.k = k_tail.ptr; t.v = v_tail.ptr;
+  t.sKb = k_tail.stride_b; t.sKl = k_tail.stride_l; t.sVb = v_tail.stride_b; t.sVl = v_tail.stride_l;
+  t.partial = tail_partial; t.lse = tail_lse;
+  t.len = tail_len; t.splits = tail_splits; t.tiles = tiles; t.dv = v_tail.dim;
+  t.groups = cdiv(hq, 32);
+  while (hq % t.groups) ++t.groups;
+  t.sm_scale = sm_scale; t.logit_cap = logit_cap;
+  const bool ksplit = d > 256;
+  t.head_blocks = hkv * ((hq / hkv + 15) / 16);
+  t.rank_blocks = ksplit ? cdiv(rank, 16) : cdiv(rank, 64);
+  const int64_t absorbing = (int64_t)t.head_blocks * t.rank_blocks * batch, grid = absorbing + (int64_t)batch * t.groups * tail_splits;
+  if (grid > 0x7fffffff) return XKV_EUNSUPPORTED;
+  t.absorbing = (int)absorbing;
+  const size_t shm = (size_t)32 * (t.dv + 8) * 2;
+  hipStream_t st = (hipStream_t)stream;
+#define XKV_ABSORB_TAIL(T, KS) \
+  absorb_tail_kernel<T, KS><<<dim3((unsigned)grid), dim3(256), shm, st>>>((const T*)q, (const T*)B, (T*)qt_hi, (T*)qt_lo, hq, hkv, d, rank, sBb, sBh, sBr, t)
+  if (dtype == XKV_BF16) { if (ksplit) XKV_ABSORB_TAIL(__bf16, true); else XKV_ABSORB_TAIL(__bf16, false); }
+  else { if (ksplit) XKV_ABSORB_TAIL(_Float16, true); else XKV_ABSORB_TAIL(_Float16, false); }
+#undef XKV_ABSORB_TAIL
+  return launch_status();
+}
+
+extern "C" int xkv_merge_stage2_tail(const float* partial, const float* lse, void* out, const void* vB, int64_t sVb, int64_t sVh,
+                                     int64_t sVr, int d_out, int dtype, int batch, int hq, int hkv, int kv_len, int max_splits, int dv,
+                                     const float* tail_partial, const float* tail_lse, int tail_splits, int64_t sOb, int64_t sOh,
+                                     void* stream) {
+  if (!partial || !lse || !out || !vB || !tail_partial || !tail_lse || batch <= 0 || hq <= 0 || hkv <= 0 || max_splits <= 0 || dv <= 0 ||
+      kv_len <= 0 || tail_splits <= 0)
+    return XKV_EINVAL;
+  if (hq % hkv || hq / hkv > 32 || dv > 512 || d_out <= 0 || d_out > 512 || d_out % 8) return XKV_EUNSUPPORTED;
+  const MergeTail tail{tail_partial, tail_lse, tail_splits};
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == XKV_BF16)
+    return launch_merge<__bf16, __bf16>(partial, lse, out, vB, sVb, sVh, sVr, d_out, nullptr, nullptr, batch, hq, hkv, kv_len, max_splits, dv,
+                                        sOb, sOh, nullptr, 0, 0, 0, nullptr, tail, st);
+  if (dtype == XKV_F16)
+    return launch_merge<_Float16, _Float16>(partial, lse, out, vB, sVb, sVh, sVr, d_out, nullptr, nullptr, batch, hq, hkv, kv_len, max_splits,
+                                            dv, sOb, sOh, nullptr, 0, 0, 0, nullptr, tail, st);
+  return XKV_EDTYPE;
 }

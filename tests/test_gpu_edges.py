@@ -388,3 +388,31 @@ def test_a_long_sequence_among_many_short_ones_is_cut(dev, hq, hkv, d):
         short = us(lambda: gqa.decode_attention_fwd(q, K, K, o, ns, 1, 0.1, kv_lens=kl64))
         # one call for both costs no more than twice the two calls; left whole, the long one took 250 us beside 40 + 30
         assert many <= 2 * (alone + short), (b, many, alone, short)
+
+
+@pytest.mark.parametrize("dtype", [BF, FP])
+@pytest.mark.parametrize("b,hq,L,Lt,r,rv,w,dv,cap", [
+    (1, 8, 40, 1, 256, 256, 128, 128, 0.0),       # one token in the tail
+    (2, 16, 300, 31, 512, 512, 512, 512, 0.0),    # less than a tile
+    (1, 32, 700, 33, 384, 384, 512, 512, 30.0),   # two splits, the last of one token; two head blocks
+    (1, 3, 64, 512, 64, 192, 32, 64, 0.0),        # 16 splits of a tile; few heads, narrow rows
+    (2, 40, 900, 545, 256, 384, 256, 320, 5.0),   # 18 tiles: 9 splits of two; two groups of 20 heads
+    (1, 16, 33000, 1500, 512, 512, 512, 512, 0.0),   # many prefix splits: their rows are merged first
+])
+def test_prefix_tail_in_one_merge(dev, dtype, b, hq, L, Lt, r, rv, w, dv, cap):
+    """Absorption and tail in one launch, prefix and tail in one merge, against attention over the concatenation in float64."""
+    from kernel_collections_amd import _lib
+    scale = w ** -0.5
+    q, kA, kB = gen((b, hq, w), dtype=dtype, seed=1).to(dev), gen((b, L, r), dtype=dtype, seed=2).to(dev), gen((b, 1, r, w), std=r ** -0.5, dtype=dtype, seed=3).to(dev)
+    vA, vB = gen((b, L, rv), dtype=dtype, seed=4).to(dev), gen((b, 1, rv, dv), std=rv ** -0.5, dtype=dtype, seed=5).to(dev)
+    kT, vT = gen((b, Lt, 1, w), dtype=dtype, seed=6).to(dev), gen((b, Lt, 1, dv), dtype=dtype, seed=7).to(dev)
+    kT[:, -1, 0] = q[:, 0] * 2                    # the tail's last token has the largest weight of a head
+    got = _lib.native().prefix_tail(q, kA, kB, vA, vB, kT, vT, scale, cap)
+    assert got is not None and got.dtype == dtype
+    q, kA, kB, vA, vB, kT, vT = (t.cpu().double() for t in (q, kA, kB, vA, vB, kT, vT))
+    k, v = torch.cat((kA @ kB[:, 0], kT[:, :, 0]), 1), torch.cat((vA @ vB[:, 0], vT[:, :, 0]), 1)
+    s = torch.einsum("bhd,bld->bhl", q, k) * scale
+    if cap:
+        s = cap * torch.tanh(s / cap)
+    ref = torch.einsum("bhl,bld->bhd", s.softmax(-1), v)
+    check_out(got, ref.float(), "prefix + tail")
