@@ -591,8 +591,8 @@ PyObject* prefix_tail(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int groups = head_groups(hq);
       const bool shared = vA.data_ptr() == kA.data_ptr() && vA.strides() == kA.strides() && rv == r;
       Splits s1{scan_splits(c, b, groups, L, ring_rank(r)), 0, nullptr, nullptr};
-      // the tail: as many splits as it has 32-token blocks, up to 16 of equal numbers of them
-      const int blocks = cdiv(Lt, 32), per = cdiv(blocks, 16), S2 = cdiv(blocks, per);
+      // the tail: as many splits as it has 32-token blocks, up to 32 of equal numbers of them
+      const int blocks = cdiv(Lt, 32), per = cdiv(blocks, 32), S2 = cdiv(blocks, per);
       const bool first = rows_first(s1.S, hq, up.hkv, rv);
       const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part1 = c.plan(b * hq * s1.S * rv * 4), lse1 = c.plan(b * hq * s1.S * 4);
       const int64_t mid = c.plan(first ? rows_bytes(b, hq, rv) : 0), part2 = c.plan(b * hq * S2 * dv * 4), lse2 = c.plan(b * hq * S2 * 4);

@@ -169,10 +169,9 @@ __global__ __launch_bounds__(256) void absorb_q_mfma_kernel(
 // `absorbing` workgroups absorb, the others take a split of the tail each, all heads of a group of at most 32.
 // A tail workgroup: `tiles` tiles of 32 tokens with a running maximum.  Scores on v_mfma_f32_16x16x32, a wave for 16 tokens x 16 heads, operands
 // straight from memory; the value tile goes through the LDS and is read transposed.  A launch saved is 5 - 9 us of prefix + tail calls that
-// take 29 (3033 + 97 tokens, 8 heads) to 115 us (262144 + 128); the splits of the tail, four before, are as many as the tail has tiles up to
-// TAIL_SPLITS: 4 x (20780 + 1822) tokens spent 35 us in four workgroups per sequence.
+// take 29 (3033 + 97 tokens, 8 heads; 22 with both launches saved) to 115 us (262144 + 128; 111); the splits of the tail, four before, are as many as the tail has tiles, up to
+// 32: 4 x (20780 + 1822) tokens spent 35 us in four workgroups per sequence (88 us a call, now 68).
 // ----------------------------------------------------------------------------------------------
-constexpr int TAIL_SPLITS = 16;
 struct TailParams {
   const void* k; const void* v;
   int64_t sKb, sKl, sVb, sVl;
@@ -193,7 +192,7 @@ __global__ __launch_bounds__(256) void absorb_tail_kernel(
     absorb_q_mfma<T, KSPLIT>(q, B, qt_hi, qt_lo, hq, hkv, d, rank, sBb, sBh, sBr, hb, b, i / t.head_blocks % t.rank_blocks);
     return;
   }
-  constexpr int SP = 32 + 4, LDP = 32 + 8, NVB = 8;
+  constexpr int SP = 32 + 4, LDP = 32 + 8, NVB = 8, NK = KSPLIT ? 16 : 8;
   __shared__ float s_lds[32][SP];
   __shared__ T p_lds[32][LDP];
   __shared__ float a_lds[32], l_lds[32];
@@ -205,9 +204,15 @@ __global__ __launch_bounds__(256) void absorb_tail_kernel(
   const int tb = wave & 1, hb = wave >> 1, head = hb * 16 + n16;
   // head rows past the group and tokens past the end repeat the last ones: never written, or weighted by zero
   const T* qrow = q + ((int64_t)b * hq + h0 + (head < hg ? head : hg - 1)) * d + 8 * g4;
+  vec8 w[NK];                                        // k-steps past the width multiply zeros
+#pragma unroll
+  for (int k = 0; k < NK; ++k) {
+    w[k] = ld16<vec8>(qrow + min(32 * k, d - 32));
+    if (32 * k >= d) w[k] = vec8{0, 0, 0, 0, 0, 0, 0, 0};
+  }
   const T* kb = reinterpret_cast<const T*>(t.k) + b * t.sKb + 8 * g4;
   const T* vb = reinterpret_cast<const T*>(t.v) + b * t.sVb;
-  const int vrow_bytes = t.dv * 2 + 16, ppr = t.dv / 8, nvb = t.dv / 64;
+  const int vrow_bytes = t.dv * 2 + 16, nvb = t.dv / 64;
   const int srow = tid >> 3, ssub = tid & 7;
   float m_run = NEG_INF, l_run = 0.f;
   f32x4 acc[NVB][2];
@@ -215,25 +220,21 @@ __global__ __launch_bounds__(256) void absorb_tail_kernel(
   for (int mb = 0; mb < NVB; ++mb) acc[mb][0] = acc[mb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int base = start; base < end; base += 32) {
     if (base > start) __syncthreads();               // the tile before has been read
+    // every load of the tile under way before the first is waited for: a tile is one round trip
+    vec8 vreg[8], a[NK];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)                      // eight threads a row
+      vreg[i] = ld16<vec8>(vb + (int64_t)min(base + srow, last) * t.sVl + (ssub + 8 * min(i, nvb - 1)) * 8);
+    const int tok = base + tb * 16 + n16;
+    const T* krow = kb + (int64_t)(tok < last ? tok : last) * t.sKl;
+#pragma unroll
+    for (int k = 0; k < NK; ++k) a[k] = ld16<vec8>(krow + min(32 * k, d - 32));
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
-    if (hb * 16 < hg) {
-      const int tok = base + tb * 16 + n16;
-      const T* krow = kb + (int64_t)(tok < last ? tok : last) * t.sKl;
-      for (int c0 = 0; c0 < d; c0 += 256) {
-        vec8 a[8], w[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          a[k] = w[k] = vec8{0, 0, 0, 0, 0, 0, 0, 0};
-          if (c0 + 32 * k < d) { a[k] = ld16<vec8>(krow + c0 + 32 * k); w[k] = ld16<vec8>(qrow + c0 + 32 * k); }
-        }
+    for (int k = 0; k < NK; ++k) s = Elem<T>::mfma16(a[k], w[k], s);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) s = Elem<T>::mfma16(a[k], w[k], s);
-      }
-    }
-    for (int i = tid; i < 32 * ppr; i += 256) {
-      const int r = i / ppr, c = i - r * ppr, tok = base + r;
-      st16(vtile + r * vrow_bytes + c * 16, ld16<vec8>(vb + (int64_t)(tok < last ? tok : last) * t.sVl + c * 8));
-    }
+    for (int i = 0; i < 8; ++i)
+      if (i < nvb) st16(vtile + srow * vrow_bytes + (ssub + 8 * i) * 16, vreg[i]);
     if (hb * 16 < hg) *reinterpret_cast<f32x4*>(&s_lds[head][tb * 16 + 4 * g4]) = s;   // lane (head n16, g4): tokens 4 g4 + r
     __syncthreads();
     if (srow < hg) {                                  // 8 threads a head, 4 tokens each

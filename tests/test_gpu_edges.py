@@ -395,8 +395,8 @@ def test_a_long_sequence_among_many_short_ones_is_cut(dev, hq, hkv, d):
     (1, 8, 40, 1, 256, 256, 128, 128, 0.0),       # one token in the tail
     (2, 16, 300, 31, 512, 512, 512, 512, 0.0),    # less than a tile
     (1, 32, 700, 33, 384, 384, 512, 512, 30.0),   # two splits, the last of one token; two head blocks
-    (1, 3, 64, 512, 64, 192, 32, 64, 0.0),        # 16 splits of a tile; few heads, narrow rows
-    (2, 40, 900, 545, 256, 384, 256, 320, 5.0),   # 18 tiles: 9 splits of two; two groups of 20 heads
+    (1, 3, 64, 1024, 64, 192, 32, 64, 0.0),       # 32 splits of a tile; few heads, narrow rows
+    (2, 40, 900, 1057, 256, 384, 256, 320, 5.0),  # 34 tiles: 17 splits of two; two groups of 20 heads
     (1, 16, 33000, 1500, 512, 512, 512, 512, 0.0),   # many prefix splits: their rows are merged first
 ])
 def test_prefix_tail_in_one_merge(dev, dtype, b, hq, L, Lt, r, rv, w, dv, cap):
