@@ -292,7 +292,7 @@ def bench_c3(args, dev):
         parity["distinct_value_basis"] = require_close(o2[:1], ref_d, "c3 with its own value basis, sequence 0")
         d_ms, d_q = time_loop(lambda i: fr.gqa_xKV_rope(q[i % layers], A, kB[i % layers], Av, vB[i % layers], o2, ns, S, scale, theta),
                               args.steps, args.warmup)
-        distinct = {"us": round(d_ms * 1e3 / args.steps, 2), "step_us": d_q, "kernel": "recon_spec_kernel (scores) + latent_ring_kernel (given scores), two passes",
+        distinct = {"us": round(d_ms * 1e3 / args.steps, 2), "step_us": d_q, "kernel": "recon_scores_kernel + latent_ring_kernel (given scores), two passes",
                     "hbm_bytes": 2 * B * L * r * 2}
         del Av
 
@@ -705,7 +705,7 @@ def bench_ropedecode(args, dev):
         "ms_per_step": total_ms / args.steps, "step_us": step_q,
         "config": {"workload": "fused RoPE xKV decode, separate bases: batch 1, 32q/8kv, d128, kv_len %d, K rank %d, V rank %d, bf16"
                                % (L, rk, rv), "kv_splits": S},
-        "roofline": {"bound": "mfma", "kernel": "recon_spec_kernel (scores) + latent_ring_kernel (given scores), two passes", "achieved": round(tf, 1), "peak": PEAK_BF16_TFLOPS,
+        "roofline": {"bound": "mfma", "kernel": "recon_scores_kernel + latent_ring_kernel (given scores), two passes", "achieved": round(tf, 1), "peak": PEAK_BF16_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(tf / PEAK_BF16_TFLOPS, 4), "traffic": None,
                      "note": "whole call (pack, stage 1, merge) over algorithmic FLOP", "algorithmic_flop": flops,
                      "hbm_side_GBps": round(B * L * (rk + rv) * 2 / (us * 1e-6) / 1e9, 1)},
