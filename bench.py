@@ -292,7 +292,7 @@ def bench_c3(args, dev):
         parity["distinct_value_basis"] = require_close(o2[:1], ref_d, "c3 with its own value basis, sequence 0")
         d_ms, d_q = time_loop(lambda i: fr.gqa_xKV_rope(q[i % layers], A, kB[i % layers], Av, vB[i % layers], o2, ns, S, scale, theta),
                               args.steps, args.warmup)
-        distinct = {"us": round(d_ms * 1e3 / args.steps, 2), "step_us": d_q, "kernel": "recon_scores_kernel + latent_ring_kernel (given scores), two passes",
+        distinct = {"us": round(d_ms * 1e3 / args.steps, 2), "step_us": d_q, "kernel": "recon_spec_kernel (scores) + latent_ring_kernel (given scores), two passes",
                     "hbm_bytes": 2 * B * L * r * 2}
         del Av
 

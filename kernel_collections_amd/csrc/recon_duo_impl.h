@@ -1,7 +1,7 @@
 // Fused reconstruct + RoPE + softmax + P.A stage 1 with a SEPARATE value basis (a second row stream), which the
 // wave-specialised kernel (recon_spec_impl.h) is not built for: key rank 256 / 384 / 512, value rank 256 / 384 / 512, head_dim 128, computed
 // RoPE angles.  (The template also has a scores-only and a shared-basis mode; recon_scores.hip and
-// recon_spec_impl.h are faster there and the dispatcher sends those shapes to them.)  Included by the recon_duo_*.hip translation units, which instantiate the shapes.
+// recon_spec_impl.h are the faster ones there and the dispatcher sends those shapes to them.)  Included by the recon_duo_*.hip translation units, which instantiate the shapes.
 //
 // Work split.  One workgroup = one (batch, kv head, split), 8 wavefronts = two per SIMD.  The waves form a 2 x 4 grid
 // over (rank half kq, feature quarter dq): wave (kq, dq) keeps B[kh][RK/2 kq .. +RK/2][{16 dq .. +16} u {64 + 16 dq .. +16}]
