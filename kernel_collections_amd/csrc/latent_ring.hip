@@ -624,7 +624,7 @@ static int launch_ring_t(const RingParams& p, hipStream_t st) {
 // which instantiation serves a call; -1: none (the register-staged kernel runs instead)
 // plain per-kv-head values [token][8 heads][128] under one shared, absorbed key basis: the call's kv groups all scan the
 // same C rows, so one workgroup per (sequence, split) serves every head
-// - or plain per-head keys too, viewed as one 1024-wide row against a block-diagonal query (no low-order part)
+// - or plain keys of 2, 4 or 8 heads too, viewed as one row against a block-diagonal query (no low-order part)
 static bool ring_vheads(const RingParams& p, bool vshared) {
   const bool absorbed = p.qn_lo && (p.dn == 512 || p.dn == 384 || p.dn == 256);
   const bool plain_keys = !p.qn_lo && p.heads_in_row && p.dn == p.heads_in_row * RING_DVH && p.groups == p.heads_in_row;
@@ -726,7 +726,9 @@ static int launch_ring_dt(const RingParams& p, bool vshared, hipStream_t st) {
 bool ring_eligible(const RingParams& p, bool vshared) {
   const int hg = p.hq / p.groups, vm = ring_vmode(p, vshared);
   const bool lo = p.qn_lo != nullptr, r = p.R != nullptr;
-  if (p.sCl >= RING_FAR_STRIDE || (vm == RING_VDISTINCT && p.sVl >= RING_FAR_STRIDE)) return false;
+  // the register-staged kernel's addresses are 64 bits wide
+  const bool v_pairs = vm == RING_VDISTINCT || (vm == RING_VHEADS && ring_rows_per_load(p.groups * RING_DVH, true) > 1);
+  if (p.sCl >= RING_FAR_STRIDE || (v_pairs && p.sVl >= RING_FAR_STRIDE)) return false;
   if (vm == RING_VHEADS) return true;
   if (hg > 32 || vm < 0) return false;
   if (p.heads_in_row) return vm == RING_VDISTINCT && !lo && !r && p.dn == p.heads_in_row * RING_DVH && p.sCl >= p.dn && p.sVl >= p.dv;

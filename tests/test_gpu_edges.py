@@ -359,6 +359,24 @@ def test_rows_far_apart(dev, form, stride, L):
     assert max_abs(out, ref) <= 2.0 ** -9 * 8
 
 
+@pytest.mark.parametrize("stride,L", [(1 << 31, 5), ((1 << 29) - 8, 37), (1 << 29, 70)])
+def test_value_rows_of_few_heads_far_apart(dev, stride, L):
+    """Plain values of two kv heads, a 256-wide row a token, whose tokens lie 1 GiB and more apart (keys side by side)."""
+    b, hq, hkv, S = 1, 16, 2, 2
+    q, K, V = gen((b, hq, 128), std=0.1, seed=1), gen((b, L, hkv, 128), seed=2), gen((b, L, hkv, 128), seed=3)
+    far = torch.empty(stride * (L - 1) + hkv * 128, dtype=BF, device=dev).as_strided((b, L, hkv, 128), (8, stride, 128, 1))
+    far.copy_(V)
+    s = torch.einsum("bkgd,blkd->bkgl", q.double().reshape(b, hkv, -1, 128), K.double())
+    ref = torch.einsum("bkgl,blkd->bkgd", torch.softmax(s, -1), V.double()).reshape(b, hq, 128)
+    Kd, ns = K.to(dev), None
+    part, lse = ops.workspaces(b, hq, S, 128, dev)
+    ops.latent_stage1(q.to(dev), None, None, (Kd, Kd.stride(0), Kd.stride(1), 128, 128), None, (far, 0, stride, 128, 128), part, lse, None, ns, None,
+                      b, hq, hkv, L, S, 1.0)
+    out = torch.empty(b, hq, 128, dtype=torch.float32, device=dev)
+    ops.merge_stage2(part, lse, out, None, ns, None, b, hq, hq, L, S)
+    assert max_abs(out, ref) <= 2.0 ** -9 * 8      # as above
+
+
 def test_rows_of_a_tail_cost_the_prefix_scan_nothing(dev):
     """A prefix scan into a workspace with rows for a tail: workgroups without tokens would deal the others out unevenly."""
     b, hq, L, S = 16, 24, 17377, 16
