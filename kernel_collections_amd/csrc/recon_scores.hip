@@ -426,6 +426,8 @@ __global__ __launch_bounds__(256, 1) void recon_scores_kernel(const FastParams p
     if (i < n - 1) store_last(i, s_done[0]);
     store_last(n - 1, s_cur);
   } else {
+    // the last tile may lie where the last group's start has read tile i - 3, with no barrier since (n even, from 6 on)
+    __syncthreads();
     *part(n - 1, wave) = s_cur;
     __syncthreads();
     for (int t = (i > 0 ? i - 1 : 0) + half; t < n; t += 2) store_last(t, *part(t, 2 * tw) + *part(t, 2 * tw + 1));

@@ -138,6 +138,15 @@ def test_recon_scores_large_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, of
     test_recon_scores_small_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, off)
 
 
+@pytest.mark.parametrize("hkv,r", [(4, 384), (1, 320), (4, 448)])
+def test_recon_scores_ends_of_two_wave_tiles(dev, hkv, r):
+    """The last tile's scores meet in the LDS place of the tile four before: every number of steps from one on, each in many workgroups."""
+    b, S = 1, 32
+    for n in range(1, 13):        # steps of 32 tokens of a split, the last one whole or of one token
+        for L in (32 * n * S, 32 * n * S - 31):
+            test_recon_scores_small_ranks(dev, BF, torch.float32, b, 4 * hkv, hkv, L, r, S, None, 3)
+
+
 @pytest.mark.parametrize("dtype", [BF, FP])
 @pytest.mark.parametrize("b,hq,hkv,L,rk,rv,off", [
     (1, 8, 2, 2049, 192, 512, 0),        # a score row past whole packets by one
