@@ -182,6 +182,7 @@ int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, float* partial,
  * accumulate P.A), with scores_out at rank 512 and, where G > 4, 384; at those ranks with a separate vA of rank 256 / 384 / 512 the 8-wave
  * kernel (2 x 4 split, second row stream for vA).  Other scores of computed angles and a 16-byte aligned factor need no workspace: independent
  * waves, one to 16 tokens at ranks up to 256, two at 320 / 384 / 448 / 512 (G <= 8).  Otherwise the generic one.
+ * Computed angles rotate the query in most of these kernels: one that holds an infinity or a NaN gives scores that are no numbers.
  * Replaces _qAB_fwd[grid] at flash_recontruction/qAB/v1.py:135-145 (v3.py / v4.py / ref.py twins) and
  * _qAB_fwd_precomp[grid] at qAB/v2.py:170-186 in scores_out mode; the fused form has no single
  * reference launch - it composes that reconstruction with the stage 1 of

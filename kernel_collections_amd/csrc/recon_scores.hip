@@ -60,10 +60,12 @@ template <int NKS, int WPT> struct ScoresShape {
   // the start's: angles of the waves' tiles, then the factor, RK ranks at a time, over all but the first two slots
   static constexpr int START = 2 * 4 * TILE, TABLE = 4 * 16 * 64 * 2 * 4, FACTOR = RK * BLD * 2;
   static constexpr int qheads(int G) { return G <= 4 ? 4 : (G + 1) & ~1; }   // two waves turn two heads each whatever the number
-  static constexpr int shm(int G) {
+  // what the scores of even and of odd heads are multiplied by, behind all
+  static constexpr int unscale(int G) {
     const int loop = RING + PART + 2 * GROUP * (LO ? 2 : 1) * qheads(G) * QROW * 4, start = START + (TABLE > FACTOR ? TABLE : FACTOR);
     return loop > start ? loop : start;
   }
+  static constexpr int shm(int G) { return unscale(G) + 16; }
 };
 
 // N 1 KB pieces of a tile, to consecutive places in the LDS: an instruction's offset moves both addresses, so voff[i] is 1024 i less than what
@@ -140,6 +142,16 @@ __global__ __launch_bounds__(256, 1) void recon_scores_kernel(const FastParams p
   fetch_tile(IC<0>());
   fetch_tile(IC<1>());
 
+  // ---- queries, a pair per lane ------------
+  constexpr int HEADS = 8;   // of 16 at most: this wave turns heads wave / 2, + 2, ...
+  vec2 qp[HEADS];
+#pragma unroll
+  for (int j = 0; j < HEADS; ++j) {
+    const int h = (wave >> 1) + 2 * j;
+    const T* src = reinterpret_cast<const T*>(p.q) + ((int64_t)b * p.hq + h0 + (h < G ? h : 0)) * 128 + lane;
+    qp[j] = vec2{src[0], src[64]};
+  }
+
   // ---- the factor, through the LDS into accumulation registers: lane (feature n16, g4) holds 8 consecutive ranks ------------
   vec8 rows[2 * NKS * WPT];   // on the way while the angles are computed
   {
@@ -176,6 +188,35 @@ __global__ __launch_bounds__(256, 1) void recon_scores_kernel(const FastParams p
     ci[pb] = f32x4{a[0], a[2], c[0], c[2]};
     si[pb] = f32x4{a[1], a[3], c[1], c[3]};
   }
+  // This wave's queries are multiplied by the power of two that brings their largest feature to 2^14 .. 2^15, and the scores by the inverse.  fp16
+  // then holds every rotated pair, which may be 1.41 times as long as its larger feature, and the parts of small queries are no subnormals there.
+  // A feature that is no finite number leaves the others as they are.
+  float* unscale = reinterpret_cast<float*>(smem + S::unscale(G));   // of even heads, of odd heads
+  {
+    float m = 0.f;
+    auto largest = [&](auto j_c) {
+      constexpr int J = decltype(j_c)::value;
+      m = fmaxf(m, fmaxf(fabsf(to_f32(qp[J][0])), fabsf(to_f32(qp[J][1]))));
+    };
+    largest(IC<0>());
+    largest(IC<1>());
+    if (G > 4) unrolled<HEADS - 2>([&](auto j_c) { largest(IC<decltype(j_c)::value + 2>()); });
+    const int bits = __builtin_bit_cast(int, row_reduce<true, 16>(m));
+    const int top = max(max(__builtin_amdgcn_readlane(bits, 0), __builtin_amdgcn_readlane(bits, 16)),
+                        max(__builtin_amdgcn_readlane(bits, 32), __builtin_amdgcn_readlane(bits, 48)));
+    const int up = max(-1, min(14 + 127 - (top >> 23), 100));
+    const float f = __builtin_bit_cast(float, (127 + up) << 23);
+    auto lift = [&](auto j_c) {
+      constexpr int J = decltype(j_c)::value;
+      qp[J] = vec2{from_f32<T>(to_f32(qp[J][0]) * f), from_f32<T>(to_f32(qp[J][1]) * f)};
+    };
+    lift(IC<0>());
+    lift(IC<1>());
+    if (G > 4) unrolled<HEADS - 2>([&](auto j_c) { lift(IC<decltype(j_c)::value + 2>()); });
+    if (lane == 0) unscale[wave >> 1] = __builtin_bit_cast(float, (127 - up) << 23);
+  }
+#pragma unroll
+  for (int j = 0; j < HEADS; ++j) asm volatile("" : "+v"(qp[j]));   // waited for here: in the loop it would be a wait for rows
   vec8 breg[NKS][8];
   T* factor = reinterpret_cast<T*>(smem + S::START);
 #pragma unroll
@@ -203,16 +244,6 @@ __global__ __launch_bounds__(256, 1) void recon_scores_kernel(const FastParams p
   // ---- q^ of the steps i0 + wave, lane = pair: words of (low feature, partner), 16 bytes for a lane's four pairs of a block ----------
   unsigned* qhat = reinterpret_cast<unsigned*>(smem + S::RING + S::PART);
   const int qpart = S::qheads(G) * QROW, qstep = (LO ? 2 : 1) * qpart;
-  constexpr int HEADS = 8;   // of 16 at most: this wave turns heads wave / 2, + 2, ...
-  vec2 qp[HEADS];
-#pragma unroll
-  for (int j = 0; j < HEADS; ++j) {
-    const int h = (wave >> 1) + 2 * j;
-    const T* src = reinterpret_cast<const T*>(p.q) + ((int64_t)b * p.hq + h0 + (h < G ? h : 0)) * 128 + lane;
-    qp[j] = vec2{src[0], src[64]};
-  }
-#pragma unroll
-  for (int j = 0; j < HEADS; ++j) asm volatile("" : "+v"(qp[j]));   // waited for here: in the loop it would be a wait for rows
   float cb = 1.f, sb = 0.f;
   unsigned* qdst = qhat + (wave & 1) * qstep + (wave >> 1) * QROW + lane;
   auto seed = [&](int i0) { sincosf((float)(p.pos_offset + start + (int64_t)(i0 + (wave & 1)) * STEP) * inv, &sb, &cb); };
@@ -276,8 +307,9 @@ __global__ __launch_bounds__(256, 1) void recon_scores_kernel(const FastParams p
   unsigned char* out = reinterpret_cast<unsigned char*>(p.scores) + (((int64_t)b * p.hq + h0) * p.kv_len + tok0) * es;
   const int out_step = STEP * es;
   const int olane = n16 < G ? (n16 * p.kv_len + 4 * g4) * es : OUT;
+  const float scale = p.sm_scale * unscale[n16 & 1];
   auto store_full = [&](int i, int at_lane, f32x4 s) {   // a tile that ends before the split does
-    s *= p.sm_scale;
+    s *= scale;
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(out + (int64_t)i * out_step, 0, 0x7fffffff, 0x00020000);
     if constexpr (MODE == TO_F32) {
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, s), r, at_lane, 0, 0);
@@ -294,7 +326,7 @@ __global__ __launch_bounds__(256, 1) void recon_scores_kernel(const FastParams p
   auto store_last = [&](int i, f32x4 s) {
     const int t = tok0 + i * STEP + 4 * g4;
     if (n16 >= G || t >= end) return;
-    s *= p.sm_scale;
+    s *= scale;
     const int64_t o = ((int64_t)b * p.hq + h0 + n16) * p.kv_len + t;
 #pragma unroll
     for (int r = 0; r < 4; ++r)

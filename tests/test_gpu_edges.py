@@ -147,6 +147,31 @@ def test_recon_scores_ends_of_two_wave_tiles(dev, hkv, r):
             test_recon_scores_small_ranks(dev, BF, torch.float32, b, 4 * hkv, hkv, L, r, S, None, 3)
 
 
+@pytest.mark.parametrize("r", [64, 192, 256])
+@pytest.mark.parametrize("G", [1, 4, 5, 16])
+def test_recon_scores_of_large_and_small_queries(dev, r, G):
+    """A rotated pair is up to 1.41 times as long as its larger feature, past fp16's largest number; the parts of a query below 6e-5 are subnormals there."""
+    L, hkv = 300, 2
+    A, B = gen((1, L, r), std=0.02, dtype=FP, seed=2), gen((1, hkv, r, 128), std=r ** -0.5, dtype=FP, seed=3)
+    cos, sin = oracle.rope_cos_sin(torch.arange(L), 128, 5e5)
+    unit = gen((1, hkv * G, 1, 128), dtype=FP, seed=1)
+    huge, tiny = unit.sign() * 65504, unit * 2.0 ** -12
+    none, nan, inf = torch.zeros_like(unit), unit.clone(), unit.clone()
+    nan[0, 0, 0, 3], inf[0, 0, 0, 3] = float("nan"), float("inf")
+    for name, q in (("huge", huge), ("tiny", tiny), ("none", none), ("one head of a NaN", nan), ("one head of an infinity", inf)):
+        ref = oracle.qab_rope(*(t.double() for t in (q, A, B)), cos.double(), sin.double())
+        s = torch.empty(1, hkv * G, 1, L, dtype=torch.float32, device=dev)
+        Bd = B.to(dev)
+        ops.recon_stage1(q.to(dev), A.to(dev), Bd, None, None, None, s, None, None, 1, hkv * G, hkv, L, 2, 1.0, True,
+                         ops.rope_inv_freq(128, 5e5, Bd.device), 0, None)
+        s = s.cpu().double()
+        if name.startswith("one"):
+            assert not s[0, 0].isfinite().any()
+            s, ref = s[:, 1:], ref[:, 1:]
+        # a key rounded to fp16 (2^-11 / sqrt 12 x 2 of its size, 2.8e-4 at most), at rank 256 the query too (1.41 times that), fp32 angles
+        assert (s - ref).norm() <= 4e-4 * ref.norm(), (name, ((s - ref).norm() / ref.norm()).item())
+
+
 @pytest.mark.parametrize("dtype", [BF, FP])
 @pytest.mark.parametrize("b,hq,hkv,L,rk,rv,off", [
     (1, 8, 2, 2049, 192, 512, 0),        # a score row past whole packets by one
