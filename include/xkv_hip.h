@@ -180,8 +180,10 @@ int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, float* partial,
  * rings): at ranks 256 / 384 / 512 with vA the same tensor as kA the wave-specialised kernel (four
  * reconstruction waves in a 2 x 2 rank/feature split hand fp16 key tiles to four waves that rotate, score, soften and
  * accumulate P.A), with scores_out at rank 512 and, where G > 4, 384; at those ranks with a separate vA of rank 256 / 384 / 512 the 8-wave
- * kernel (2 x 4 split, second row stream for vA).  Other scores of computed angles and a 16-byte aligned factor need no workspace: independent
- * waves, one to 16 tokens at ranks up to 256, two at 320 / 384 / 448 / 512 (G <= 8).  Otherwise the generic one.
+ * kernel (2 x 4 split, second row stream for vA); other scores_out at ranks 256 and 384 with a factor of 16-byte packets independent waves, one or two
+ * to 16 tokens, which read kB as it is.  These hold the rotated query as one fp16 value, beside the keys' rounding to fp16 (scores within 2.9e-4 .. 4.4e-4 of
+ * float64 against 2.1e-4).  Without a workspace: independent waves with a query of two parts for scores_out at ranks up to 224 (G <= 16), 320 and 448
+ * (G <= 8); otherwise the generic kernel, whose query is not rotated.
  * Computed angles rotate the query in most of these kernels: one that holds an infinity or a NaN gives scores that are no numbers.
  * Replaces _qAB_fwd[grid] at flash_recontruction/qAB/v1.py:135-145 (v3.py / v4.py / ref.py twins) and
  * _qAB_fwd_precomp[grid] at qAB/v2.py:170-186 in scores_out mode; the fused form has no single

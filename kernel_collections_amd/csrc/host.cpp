@@ -373,8 +373,10 @@ void rope_operands(Ten q, int64_t hq, int64_t d, Ten kA, Ten kB, Ten inv) {
 }
 // recon_scores_kernel: four tiles of 16 tokens a step (two beyond rank 256), one workgroup per CU; otherwise the kernels that hold a kv
 // head's factor in registers keep one, the generic kernel two or three.
-// what recon_scores_kernel serves, of the operands that this layer takes
-bool scores_alone(Ten kB, int64_t r, int64_t G) { return rows(kB) && (r <= 256 || r % 64 == 0) && G <= (r > 224 ? 8 : 16); }
+// what recon_scores_kernel runs, of the operands that this layer takes
+bool scores_alone(Ten kB, int64_t r, int64_t G) {
+  return rows(kB) && (r <= 224 ? G <= 16 : r == 384 ? G <= 4 : (r == 256 || r == 320 || r == 448) && G <= 8);
+}
 int score_splits(const Call& c, Ten kB, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r) {
   if (scores_alone(kB, r, G)) return balanced_splits(b, hkv, L, r <= 256 ? 64 : 32, 1, c.cus);
   const bool resident = ring_rank(r) && G <= 8;
@@ -409,7 +411,7 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, kB.stride(0)), ws = c.plan(ws_bytes);
       const float* invp = inv.data_ptr<float>();
       Splits s{0, 0, nullptr, nullptr};
-      if (may_two_pass && scores_alone(kB, r, hq / hkv) && (ring_rank(rv) || (shared && (rv == 192 || rv == 128)))) {
+      if (may_two_pass && (scores_alone(kB, r, hq / hkv) || (rows(kB) && ring_rank(r) && hq / hkv <= 8)) && (ring_rank(rv) || (shared && (rv == 192 || rv == 128)))) {
         // scores first, then softmax and P.v_A in one stream for all heads.  The second pass reads the
         // scores in 16-byte packets, so their rows are whole packets: at another length the kernels get the padded one as the row's
         // and the true one as every sequence's (one fill, about 2 us).

@@ -14,8 +14,9 @@
 //
 // RoPE by angle addition: R(position) = R(first token of the step) R(place in the step).  The second factor is per-lane constants; the
 // first is moved to the query, q^ = R(step)^T q, which the workgroup needs once for all its tokens: in every group of two steps the waves
-// make the q^ of the next group (a pair per lane) and leave it in the LDS, as a high and a low fp16 part up to 192 ranks, beyond
-// as one fp16 value beside keys that are as coarse.
+// make the q^ of the next group (a pair per lane) and leave it in the LDS, as a high and a low fp16 part: the scores are then as exact as those
+// of an unrotated query (2.1e-4 of their size against float64, all of it the keys' rounding to fp16).  At ranks 256 and 384 it is one fp16 value
+// (2.9e-4), for callers that give a workspace and with it had the wave-specialised kernels' one value (3.8e-4 and 4.4e-4): a low part costs 4 - 8 % there.
 //
 // What bounds it: one wave per SIMD that issues everything in order, an instruction in 5 cycles at best, and the LDS.  At 256 ranks the 68 matrix
 // instructions of a tile are 1088 cycles, a block of 16 pairs takes 400 with everything else, and a group's start (barrier, q^)
@@ -53,7 +54,7 @@ struct FactorOperand { const void* p; int64_t sb, sh, sr; };
 template <int NKS, int WPT> struct ScoresShape {
   static constexpr int RK = 32 * NKS, RANK = RK * WPT;           // ranks of a wave
   static constexpr int STEP = 64 / WPT;                          // tokens
-  static constexpr bool LO = RANK <= 192;                        // q^ has a low part
+  static constexpr bool LO = RANK != 256 && RANK != 384;         // q^ has a low part
   static constexpr int ROW = RK * 2, TILE = 16 * ROW, RING = SLOTS * 4 * TILE;   // [slot][wave][16 rows]
   // behind the ring: scores that wait for the other wave's [2 GROUP steps][wave][lane], q^ [2 groups][GROUP steps][parts][head][QROW words]
   static constexpr int PART = WPT == 1 ? 0 : 2 * GROUP * 4 * 64 * 16, QROW = 64 + 4;
@@ -487,7 +488,7 @@ int launch_mode(const FastParams& p, const FactorOperand& kB, int batch, int ran
     XKV_SCORES_RANK(8)
 #undef XKV_SCORES_RANK
 #define XKV_SCORES_RANK(N) case 64 * N: return launch_t<T, N, 2, MODE>(p, kB, batch, st);
-    XKV_SCORES_RANK(5) XKV_SCORES_RANK(6) XKV_SCORES_RANK(7) XKV_SCORES_RANK(8)
+    XKV_SCORES_RANK(5) XKV_SCORES_RANK(6) XKV_SCORES_RANK(7)
 #undef XKV_SCORES_RANK
     default: return XKV_EUNSUPPORTED;
   }
@@ -504,7 +505,8 @@ int launch(const FastParams& p, const FactorOperand& kB, int batch, int rank, hi
 
 bool recon_scores_serves(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int rank) {
   if (((sBb | sBh | sBr) & 7) || (reinterpret_cast<uintptr_t>(kB) & 15)) return false;
-  if (rank > 256 && (rank % 64 || p.hq / p.hkv > 8)) return false;   // two equal halves; the LDS
+  if (rank > 224 && p.hq / p.hkv > 8) return false;                  // the LDS
+  if (rank > 256 && (rank % 64 || rank == 512)) return false;        // two equal halves; 512 is faster elsewhere
   // 32-bit lane offsets: 16 token rows, the score rows of 16 heads.  Rows that overlap would make offsets negative
   return p.sAl >= rank && p.sAl < (1 << 25) && (int64_t)(p.hq / p.hkv) * p.kv_len < (1 << 28);
 }

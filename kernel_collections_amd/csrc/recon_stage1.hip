@@ -411,13 +411,13 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
     f.num_splits = num_kv_splits; f.kv_lens = kv_lens;
     f.hq = hq; f.hkv = hkv; f.kv_len = kv_len; f.max_splits = max_splits; f.total_wg = batch * hkv * max_splits;
     f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
-    // Every scores-only shape that it takes (us a call, this kernel / the one it replaces, 32 heads on 8 kv heads: rank 128, 5 x 7488 tokens 17.9 / 21.6; rank
-    // 192, 7 x 39246 124 / 153; rank 256, 2 x 28611 30.9 / 41.8; rank 384, 5 x 2903 19.8 / 21.4, 2 x 81976 135 / 146).  Where the wave-specialised
-    // kernel can run, not rank 512, nor 384 beyond four heads per kv head: two waves' halves of the q-dot cost more there than its pack launch (rank 512, 32 on 8,
-    // 9001 17.8 / 18.1, 8 x 200001 1673 / 1604; 64 on 8, 2500 13.0 / 11.9, 40000 47.4 / 47.7, 3 x 130001 426 / 397; 16 on 2, 9000 13.1 / 10.9; rank 384,
-    // 32 on 8, 2100 10.5 / 10.6, 8 x 200001 1320 / 1342; 48 on 8, 3 x 130001 344 / 342; 64 on 8, 2500 11.3 / 10.8; 16 on 2, 9000 11.6 / 10.2)
-    const bool spec_scores = spec && (rank == 512 || (rank == 384 && hq / hkv > 4));
-    if (!spec_scores && recon_scores_serves(f, kB, sBb, sBh, sBr, rank))
+    // Scores-only shapes (us a call, this kernel / the one it replaces, 32 heads on 8 kv heads: rank 128, 5 x 7488 tokens 17.9 / 21.6; rank
+    // 192, 7 x 39246 124 / 153; rank 224, 131072 64.5 / 241; rank 256, 2 x 28611 30.9 / 41.8; rank 320, 131072 99.8 / 269; rank 384, 5 x 2903 19.8 / 21.4, 2 x
+    // 81976 135 / 146; rank 448, 131072 127 / 313).  At ranks 256 and 384 its rotated query is one fp16 value, so only where the caller's workspace asks for kernels that have
+    // that.  At rank 384 not beyond four heads per kv head: two waves' halves of the q-dot cost more there than the wave-specialised kernel's pack launch
+    // (32 on 8, 2100 10.5 / 10.6, 8 x 200001 1320 / 1342; 48 on 8, 3 x 130001 344 / 342; 64 on 8, 2500 11.3 / 10.8; 16 on 2, 9000 11.6 / 10.2)
+    const bool here = rank == 256 ? spec : rank == 384 ? spec && hq / hkv <= 4 : true;
+    if (here && recon_scores_serves(f, kB, sBb, sBh, sBr, rank))
       return launch_recon_scores(f, kB, sBb, sBh, sBr, batch, dtype, rank, st);
   }
   // The wave-specialised kernel: rank 512 / 384 / 256, a basis shared by K and V (or scores that stay with it, or of a factor that is not 16-byte packets), computed

@@ -132,7 +132,7 @@ def test_recon_scores_small_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, of
     (1, 8, 2, 640, 512, 1, None, 99999),        # whole steps only, angles seeded twice
 ])
 def test_recon_scores_large_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, off, monkeypatch):
-    if r in (384, 512):    # with a workspace the wave-specialised kernel, at rank 384 beyond four heads per kv head
+    if r in (384, 512):    # with a workspace the wave-specialised kernel (at rank 384 beyond four heads per kv head), without one the generic one
         test_recon_scores_small_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, off)
         monkeypatch.setattr(ops, "USE_RECON_WORKSPACE", False)
     test_recon_scores_small_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, off)
@@ -145,6 +145,22 @@ def test_recon_scores_ends_of_two_wave_tiles(dev, hkv, r):
     for n in range(1, 13):        # steps of 32 tokens of a split, the last one whole or of one token
         for L in (32 * n * S, 32 * n * S - 31):
             test_recon_scores_small_ranks(dev, BF, torch.float32, b, 4 * hkv, hkv, L, r, S, None, 3)
+
+
+@pytest.mark.parametrize("r,G,workspace", [(64, 16, True), (192, 4, True), (224, 1, True), (224, 16, True), (256, 9, True), (256, 16, True), (320, 4, True), (320, 8, True),
+                                           (448, 5, True), (256, 4, False), (256, 8, False), (384, 4, False), (512, 8, False)])
+def test_scores_of_an_exact_query(dev, r, G, workspace, monkeypatch):
+    """Every rank, and calls without a workspace: no rounding but the keys' to fp16 (ranks 256, 384 and 512 with a workspace and up to 8 heads have the query's too)."""
+    monkeypatch.setattr(ops, "USE_RECON_WORKSPACE", workspace)
+    import kernel_collections_amd.flash_recontruction as fr
+    L, hkv = 1500, 2
+    for dtype in (BF, FP):
+        q, A, B = gen((1, hkv * G, 1, 128), dtype=dtype, seed=1), gen((1, L, r), dtype=dtype, seed=2), gen((1, hkv, r, 128), std=r ** -0.5, dtype=dtype, seed=3)
+        ang = (torch.arange(L).float()[:, None] * ops.rope_inv_freq(128, 5e5, torch.device("cpu"))).double()
+        ref = oracle.qab_rope(*(t.double() for t in (q, A, B)), torch.cat((ang, ang), -1).cos(), torch.cat((ang, ang), -1).sin())
+        s = fr.qAB_rope_v1(q.to(dev), A.to(dev), B.to(dev), 5e5, out_dtype=torch.float32).cpu().double()
+        # rounding to 11 bits: 2^-11 / sqrt(3) of a mantissa's lowest value, 0.73 of that over all mantissas: 2.06e-4; twice the rounding is 2.9e-4
+        assert (s - ref).norm() <= 2.4e-4 * ref.norm(), (dtype, ((s - ref).norm() / ref.norm()).item())
 
 
 @pytest.mark.parametrize("r", [64, 192, 256])
