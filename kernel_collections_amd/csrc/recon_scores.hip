@@ -474,7 +474,7 @@ int launch_t(const FastParams& p, const FactorOperand& kB, int batch, hipStream_
   auto kern = recon_scores_kernel<T, NKS, WPT, MODE>;
   const int shm = S::shm(p.hq / p.hkv);
   static DynLds lds;
-  const int e = ensure_dynamic_lds(lds, reinterpret_cast<const void*>(kern), shm);
+  const int e = ensure_dynamic_lds(lds, reinterpret_cast<const void*>(kern), shm, true);
   if (e != XKV_OK) return e;
   kern<<<dim3(xcd_grid(batch * p.hkv * p.max_splits, p.hkv)), dim3(256), shm, st>>>(p, kB);
   return launch_status();

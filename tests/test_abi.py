@@ -252,3 +252,18 @@ def test_ctypes_stub_of_the_notes_computes_qab_rope(monkeypatch, dtype):
     assert out.shape == (b, hq, 1, L) and out.dtype == dtype
     err = (out.float().cpu() - ref).abs().max().item() / ref.abs().max().item()
     assert err <= 1e-2, err
+
+
+def test_kernels_that_count_their_own_loads_are_refused_if_they_spill():
+    """Every unit with a wait by count launches through the check of ensure_dynamic_lds."""
+    from kernel_collections_amd import build
+    units = 0
+    for name in os.listdir(build.CSRC):
+        if not name.startswith(("latent_", "recon_")):      # ceilings.hip measures the card
+            continue
+        text = open(os.path.join(build.CSRC, name)).read()
+        launches = re.findall(r"ensure_dynamic_lds\((?:lds|st)\b.*\);", text)
+        if launches and re.search(r"s_waitcnt vmcnt\(|wait_vmcnt", text):
+            units += 1
+            assert all(c.endswith(", true);") for c in launches), (name, launches)
+    assert units == 4      # latent_ring, recon_scores, recon_spec, recon_duo
