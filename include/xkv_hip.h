@@ -256,7 +256,9 @@ int xkv_merge_stage2(const float* partial, const float* lse, void* out,
 /* Prefix + tail decode (flash_decoding/deepseek_mla/flash_decoding.py:159-255), first launch: xkv_absorb_q for the factorised prefix, and the
  * attention over the plain tail, one shared key / value row per token ([batch, tail_len, d] / [batch, tail_len, dv], operands as elsewhere):
  * tail_partial [batch, hq, tail_splits, dv] (normalised) and tail_lse [batch, hq, tail_splits].  A split holds whole 32-token blocks, all
- * but the last the same number, and every split must hold tokens.  d % 32 == 0, dv % 64 == 0, both <= 512. */
+ * but the last the same number, and every split must hold tokens.  d % 32 == 0, dv % 64 == 0, both <= 512.
+ * This and the next entry point are newer than ABI version 7: a library of that version may lack them, and with them xkv_softmax_pv_stage1 over
+ * V.dim 128 / 192 and more than 32 heads. */
 int xkv_absorb_q_tail(const void* q, const void* B, void* qt_hi, void* qt_lo, int batch, int hq, int hkv, int d, int rank,
                       int64_t stride_B_b, int64_t stride_B_h, int64_t stride_B_r, xkv_kv_operand k_tail, xkv_kv_operand v_tail,
                       int tail_len, int tail_splits, float* tail_partial, float* tail_lse, float sm_scale, float logit_cap, int dtype,

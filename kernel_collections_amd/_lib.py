@@ -73,12 +73,13 @@ def _declare(lib):
     lib.xkv_merge_stage2.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int,
                                      c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int,
                                      c_int64, c_int64, c_int, c_void_p, c_int64, c_int64, c_void_p]
-    lib.xkv_absorb_q_tail.restype = c_int
-    lib.xkv_absorb_q_tail.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int64, c_int64, c_int64,
-                                      KVOperand, KVOperand, c_int, c_int, c_void_p, c_void_p, c_float, c_float, c_int, c_void_p]
-    lib.xkv_merge_stage2_tail.restype = c_int
-    lib.xkv_merge_stage2_tail.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int, c_int,
-                                          c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int64, c_int64, c_void_p]
+    if hasattr(lib, "xkv_absorb_q_tail"):      # newer than the version they are in; called by the native host layer alone, which knows
+        lib.xkv_absorb_q_tail.restype = c_int
+        lib.xkv_absorb_q_tail.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int64, c_int64, c_int64,
+                                          KVOperand, KVOperand, c_int, c_int, c_void_p, c_void_p, c_float, c_float, c_int, c_void_p]
+        lib.xkv_merge_stage2_tail.restype = c_int
+        lib.xkv_merge_stage2_tail.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int, c_int,
+                                              c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int64, c_int64, c_void_p]
     lib.xkv_softmax_pv_stage1.restype = c_int
     lib.xkv_softmax_pv_stage1.argtypes = [c_void_p, KVOperand, c_void_p, c_void_p, c_void_p, c_void_p,
                                           c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p]

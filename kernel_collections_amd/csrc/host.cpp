@@ -32,12 +32,15 @@ namespace {
 #define XKV_SYMBOLS(X)                                                                                              \
   X(xkv_error_string) X(xkv_absorb_q) X(xkv_blockdiag_q) X(xkv_latent_stage1) X(xkv_softmax_pv_stage1) X(xkv_recon_stage1) \
   X(xkv_recon_workspace_bytes) X(xkv_merge_stage2) X(xkv_plan_splits)
-// newer than the version they are in: a library without them has prefix + tail decode declined
+// newer than the version they are in, with xkv_softmax_pv_stage1 over value rows of 128 and 192 and more than 32 heads: over a library
+// without them (joined() false) a call takes the launches that it has
 #define XKV_OPTIONAL_SYMBOLS(X) X(xkv_absorb_q_tail) X(xkv_merge_stage2_tail)
 #define XKV_DECLARE(name) decltype(&name) p_##name = nullptr;
 XKV_SYMBOLS(XKV_DECLARE)
 XKV_OPTIONAL_SYMBOLS(XKV_DECLARE)
 #undef XKV_DECLARE
+
+bool joined() { return p_xkv_absorb_q_tail && p_xkv_merge_stage2_tail; }
 
 struct CallError : std::runtime_error { using std::runtime_error::runtime_error; };
 void check(int rc, const char* what) {
@@ -411,7 +414,8 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, kB.stride(0)), ws = c.plan(ws_bytes);
       const float* invp = inv.data_ptr<float>();
       Splits s{0, 0, nullptr, nullptr};
-      if (may_two_pass && (scores_alone(kB, r, hq / hkv) || (rows(kB) && ring_rank(r) && hq / hkv <= 8)) && (ring_rank(rv) || (shared && (rv == 192 || rv == 128)))) {
+      if (may_two_pass && (scores_alone(kB, r, hq / hkv) || (rows(kB) && ring_rank(r) && hq / hkv <= 8)) && (joined() || hq <= 32) &&
+          (ring_rank(rv) || (joined() && shared && (rv == 192 || rv == 128)))) {
         // scores first, then softmax and P.v_A in one stream for all heads.  The second pass reads the
         // scores in 16-byte packets, so their rows are whole packets: at another length the kernels get the padded one as the row's
         // and the true one as every sequence's (one fill, about 2 us).
@@ -576,7 +580,6 @@ PyObject* prefix_tail(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 9, [&]() -> PyObject* {
     Ten q = T(a[0]), kA = T(a[1]), kB = T(a[2]), vA = T(a[3]), vB = T(a[4]), kT = T(a[5]), vT = T(a[6]);
     const float scale = F(a[7]), logit_cap = F(a[8]);
-    need(p_xkv_absorb_q_tail && p_xkv_merge_stage2_tail);
     same(q, {&kA, &kB, &vA, &vB, &kT, &vT});
     need(q.dim() == 3 && kA.dim() == 3 && kB.dim() == 4 && vA.dim() == 3 && vB.dim() == 4 && kT.dim() == 4 && vT.dim() == 4);
     const int64_t b = q.size(0), hq = q.size(1), w = q.size(2), L = kA.size(1), r = kA.size(2), rv = vA.size(2), Lt = kT.size(1);
@@ -593,20 +596,31 @@ PyObject* prefix_tail(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int groups = head_groups(hq);
       const bool shared = vA.data_ptr() == kA.data_ptr() && vA.strides() == kA.strides() && rv == r;
       Splits s1{scan_splits(c, b, groups, L, ring_rank(r)), 0, nullptr, nullptr};
-      // the tail: as many splits as it has 32-token blocks, up to 32 of equal numbers of them
-      const int blocks = cdiv(Lt, 32), per = cdiv(blocks, 32), S2 = cdiv(blocks, per);
+      // the tail: as many splits as it has 32-token blocks, up to 32 of equal numbers of them.  In launches of its own at most four, every one of
+      // them live; a cap states the count, because the rows are one more: row 0 is the merged, up-projected prefix with its log-sum-exp
+      const bool join = joined();
+      const int blocks = cdiv(Lt, 32), per = cdiv(blocks, join ? 32 : 4), S2 = cdiv(blocks, per), rows2 = S2 + (join ? 0 : 1);
       const bool first = rows_first(s1.S, hq, up.hkv, rv);
       const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part1 = c.plan(b * hq * s1.S * rv * 4), lse1 = c.plan(b * hq * s1.S * 4);
-      const int64_t mid = c.plan(first ? rows_bytes(b, hq, rv) : 0), part2 = c.plan(b * hq * S2 * dv * 4), lse2 = c.plan(b * hq * S2 * 4);
+      const int64_t mid = c.plan(first ? rows_bytes(b, hq, rv) : 0), part2 = c.plan(b * hq * rows2 * dv * 4), lse2 = c.plan(b * hq * rows2 * 4);
       c.alloc();
       o = at::empty({b, hq, dv}, c.opts);
       // the query absorbed and the tail attended to in one launch: neither depends on the other
-      check(p_xkv_absorb_q_tail(q.data_ptr(), kB.data_ptr(), c.get<void>(hi), c.get<void>(lo), b, hq, groups, w, r, kB.stride(0), 0, kB.stride(2),
+      if (!join) absorb(c, q.data_ptr(), kB, c.get<void>(hi), c.get<void>(lo), b, hq, w, r);
+      else check(p_xkv_absorb_q_tail(q.data_ptr(), kB.data_ptr(), c.get<void>(hi), c.get<void>(lo), b, hq, groups, w, r, kB.stride(0), 0, kB.stride(2),
                                 kv(kT, 0, w), kv(vT, 0, dv), Lt, S2, c.get<float>(part2), c.get<float>(lse2), scale, logit_cap, c.dt, c.stream),
             "xkv_absorb_q_tail");
       check(p_xkv_latent_stage1({c.get<void>(hi), (int)r}, c.get<void>(lo), NO_Q, kv(kA, 0, r), NO_KV, shared ? kv(kA, 0, r) : kv(vA, 0, rv),
                                 c.get<float>(part1), c.get<float>(lse1), nullptr, 0, nullptr, nullptr, b, hq, groups, L, s1.S, 0, nullptr, scale,
                                 logit_cap, c.dt, c.stream), "xkv_latent_stage1");
+      if (!join) {
+        float *pf = c.get<float>(part2), *lf = c.get<float>(lse2);
+        merge(c, c.get<float>(part1), c.get<float>(lse1), pf, hq * rows2 * dv, rows2 * dv, XKV_F32, &up, mid, s1, b, hq, L, rv, lf, hq * rows2, rows2);
+        check(p_xkv_latent_stage1({q.data_ptr(), (int)w}, nullptr, NO_Q, kv(kT, 0, w), NO_KV, kv(vT, 0, dv), pf + dv, lf + 1, nullptr, 0, nullptr,
+                                  nullptr, b, hq, groups, Lt, rows2, 32 * per, nullptr, scale, logit_cap, c.dt, c.stream), "xkv_latent_stage1");
+        merge(c, pf, lf, o.data_ptr(), hq * dv, dv, c.dt, nullptr, 0, {rows2, 0, nullptr, nullptr}, b, hq, 32 * rows2, dv);   // every row live
+        return;
+      }
       const float *rows = c.get<float>(part1), *rows_lse = c.get<float>(lse1);
       int n_rows = s1.S, len = L;
       if (first) {   // many splits: merged by the whole chip, then one row per head

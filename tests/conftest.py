@@ -34,26 +34,22 @@ def dev():
     return torch.device("cuda:0")
 
 
-@pytest.fixture(scope="session")
-def shim_lib(tmp_path_factory):
+def _build_shim(folder, name):
     import ctypes
     import subprocess
 
     from kernel_collections_amd import _lib
-    so = str(tmp_path_factory.mktemp("shim") / "liblaunch_shim.so")
-    subprocess.check_call(["g++", "-O1", "-shared", "-fPIC", "-o", so, os.path.join(ROOT, "tests", "launch_shim.cpp"), "-ldl"])
+    so = str(folder / f"lib{name}.so")
+    subprocess.check_call(["g++", "-O1", "-shared", "-fPIC", "-o", so, os.path.join(ROOT, "tests", name + ".cpp"), "-ldl"])
     lib = ctypes.CDLL(so)
     assert lib.shim_init(_lib.LIB_PATH.encode()) == 0
     return so, lib
 
 
-@pytest.fixture
-def shim(shim_lib):
-    """The native host layer over launch_shim.cpp: yields the shim, whose counters tell what a call did."""
+def _over_shim(so, lib):
     import ctypes
 
     from kernel_collections_amd import _lib
-    so, lib = shim_lib
     lib.count = lambda name: ctypes.c_int.in_dll(lib, name).value
     native = _lib.native()
     for name in ("shim_launches", "shim_stage1", "shim_locked_calls", "shim_poison", "shim_poisoned"):
@@ -63,3 +59,26 @@ def shim(shim_lib):
         yield lib
     finally:
         native.init(_lib.LIB_PATH)
+
+
+@pytest.fixture(scope="session")
+def shim_lib(tmp_path_factory):
+    return _build_shim(tmp_path_factory.mktemp("shim"), "launch_shim")
+
+
+@pytest.fixture(scope="session")
+def shim_tail_lib(tmp_path_factory):
+    return _build_shim(tmp_path_factory.mktemp("shim"), "launch_shim_tail")
+
+
+@pytest.fixture
+def shim(shim_lib):
+    """The native host layer over launch_shim.cpp: yields the shim, whose counters tell what a call did.  It has the entry points of the ABI version,
+    not those added to it since."""
+    yield from _over_shim(*shim_lib)
+
+
+@pytest.fixture
+def shim_tail(shim_tail_lib):
+    """The same over launch_shim_tail.cpp, which has them."""
+    yield from _over_shim(*shim_tail_lib)

@@ -335,3 +335,37 @@ def test_general_rope_decode_fills_the_device(dev, form, monkeypatch):
     got = fr.gqa_xKV_rope(q, A, B, A, B, torch.empty(1, 16, 128, dtype=BF, device=dev), ns, 2, 128 ** -0.5, 5e5, **kw)
     assert seen == [ops.decode_splits(1, 2, L, r, True)] and seen[0] > 64
     check_out(got, want, form)
+
+
+@pytest.mark.parametrize("over,launches", [("shim", 5), ("shim_tail", 3)])
+@pytest.mark.parametrize("Lt", [1, 97, 1500])
+def test_prefix_tail_with_and_without_the_joined_launches(dev, over, launches, Lt, request):
+    """Native over a library of the ABI version alone and over one with the entry points added since, each against float64."""
+    from kernel_collections_amd import _lib
+    shim = request.getfixturevalue(over)
+    b, hq, L, r, w = 2, 8, 700, 256, 128
+    t = lambda *s, std=1.0, n=0: gen(s, std=std, seed=n).to(dev)
+    a = q, kA, kB, vA, vB, kT, vT = t(b, hq, w, n=1), t(b, L, r, n=2), t(b, 1, r, w, std=r ** -0.5, n=3), t(b, L, r, n=4), t(b, 1, r, w, std=r ** -0.5, n=5), \
+        t(b, Lt, 1, w, n=6), t(b, Lt, 1, w, n=7)
+    got = _lib.native().prefix_tail(*a, w ** -0.5, 0.0)
+    assert got is not None and shim.count("shim_launches") == launches
+    q, kA, kB, vA, vB, kT, vT = (x.cpu().double() for x in a)
+    k, v = torch.cat((kA @ kB[:, 0], kT[:, :, 0]), 1), torch.cat((vA @ vB[:, 0], vT[:, :, 0]), 1)
+    check_out(got, (torch.softmax(q @ k.transpose(1, 2) * w ** -0.5, -1) @ v).float(), over)
+
+
+def test_two_passes_over_a_library_that_lacks_their_wider_forms(dev, shim, monkeypatch):
+    """Value rows of 192 and more than 32 heads came with the joined launches: without them one kernel, still native."""
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd.flash_recontruction.fused_attention import _fused
+    monkeypatch.setattr(_fused, "TWO_PASS_WORK_SHARED", {x: (1, 0) for x in (128, 192, 256)})
+    for hq, r in ((8, 192), (64, 256), (8, 256)):
+        t = lambda *s, std=1.0, n=0: gen(s, std=std, seed=n).to(dev)
+        q, A, B, ns = t(1, hq, 128, n=1), t(1, 500, r, n=2), t(1, 8, r, 128, std=r ** -0.5, n=3), torch.ones(1, dtype=torch.int32, device=dev)
+        call = lambda: fr.gqa_xKV_rope(q, A, B, A, B, torch.empty_like(q), ns, 1, 0.1, 5e5)
+        before = shim.count("shim_stage1")
+        got = call()
+        assert shim.count("shim_stage1") - before == (2 if hq <= 32 and r == 256 else 1)
+        with monkeypatch.context() as m:
+            m.setattr(_fused, "TWO_PASS_WORK_SHARED", {})
+            check_out(got, call(), f"{hq} heads, rank {r}")

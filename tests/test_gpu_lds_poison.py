@@ -100,3 +100,12 @@ def test_two_basis_forms(dev, form, poisoned, monkeypatch):
 
 def test_config1_shape(dev, poisoned):
     tp.test_config1_shape_factorized_rope(dev)
+
+
+def test_tail_beside_the_absorption(dev, shim_tail):
+    """The joined launch of prefix + tail decode, through the shim that has it."""
+    import test_gpu_edges as edges
+    ctypes.c_int.in_dll(shim_tail, "shim_poison").value = 1
+    edges.test_prefix_tail_in_one_merge(dev, BF, 1, 32, 700, 33, 384, 384, 512, 512, 30.0)
+    edges.test_prefix_tail_in_one_merge(dev, FP, 2, 16, 300, 31, 512, 512, 512, 512, 0.0)
+    assert shim_tail.count("shim_poisoned") == shim_tail.count("shim_stage1") == 4

@@ -242,3 +242,20 @@ def test_two_passes_where_the_callers_counts_are_taken():
     from kernel_collections_amd.flash_recontruction.fused_attention import _fused
     B = torch.zeros(1, 2, 192, 128, dtype=torch.bfloat16)
     assert _fused._two_pass(192, 7368, B, asked=True) and not _fused._two_pass(192, 7368, B) and not _fused._two_pass(192, 4095, B, asked=True)
+
+
+def test_a_library_without_the_newer_entry_points_loads(tmp_path):
+    """Of the same ABI version: prefix + tail decode has the launches of that version to take there."""
+    import ctypes
+    import subprocess
+    from kernel_collections_amd import _xkv_host
+    newer = {"xkv_absorb_q_tail", "xkv_merge_stage2_tail"}
+    src, so = tmp_path / "plain.c", tmp_path / "libplain.so"
+    src.write_text("".join(f"int {n}(void) {{ return {_lib.ABI_VERSION if n == 'xkv_abi_version' else 0}; }}\n" for n in _lib.EXPORTS if n not in newer))
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)])
+    _lib._declare(ctypes.CDLL(str(so)))
+    _lib.native()
+    try:
+        _xkv_host.init(str(so))
+    finally:
+        _xkv_host.init(_lib.LIB_PATH)
