@@ -414,7 +414,7 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, kB.stride(0)), ws = c.plan(ws_bytes);
       const float* invp = inv.data_ptr<float>();
       Splits s{0, 0, nullptr, nullptr};
-      if (may_two_pass && (scores_alone(kB, r, hq / hkv) || (rows(kB) && ring_rank(r) && hq / hkv <= 8)) && (joined() || hq <= 32) &&
+      if (may_two_pass && (scores_alone(kB, r, hq / hkv) || (ring_rank(r) && hq / hkv <= 8)) && (joined() || hq <= 32) &&
           (ring_rank(rv) || (joined() && shared && (rv == 192 || rv == 128)))) {
         // scores first, then softmax and P.v_A in one stream for all heads.  The second pass reads the
         // scores in 16-byte packets, so their rows are whole packets: at another length the kernels get the padded one as the row's

@@ -215,6 +215,24 @@ def test_two_pass_rope_decode(dev, dtype, b, hq, hkv, L, rk, rv, off, monkeypatc
     check_out(fr.gqa_xKV_rope(qd, kAd, kBd, vAd, vBd, torch.zeros_like(qd), ns, 2, 128 ** -0.5, 5e5, pos_offset=off), ref, "one kernel")
 
 
+@pytest.mark.parametrize("rk,rv,batched", [(256, 256, False), (256, 384, True), (384, 512, False), (512, 384, True)])
+def test_two_pass_rope_decode_of_any_factor(dev, shim_tail, rk, rv, batched, monkeypatch):
+    """A factor at an odd 8-byte place: scores and values apart as with any other, whatever kernel takes the scores."""
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd.flash_recontruction.fused_attention import _fused
+    monkeypatch.setattr(_fused, "TWO_PASS_MIN_TOKENS", 0)
+    b, hq, hkv, L = 2, 32, 8, 4211
+    q, kA, vA = gen((b, hq, 128), std=0.4, seed=1).to(dev), gen((b, L, rk), seed=2).to(dev), gen((b, L, rv), seed=4).to(dev)
+    kB, vB = gen((b if batched else 1, hkv, rk, 128), std=rk ** -0.5, seed=3).to(dev), gen((1, hkv, rv, 128), std=rv ** -0.5, seed=5).to(dev).expand(b, -1, -1, -1)
+    odd = torch.empty(kB.numel() + 4, dtype=BF, device=dev)[4:].view(kB.shape).copy_(kB).expand(b, -1, -1, -1)
+    kB = kB.expand(b, -1, -1, -1)
+    ns = torch.ones(b, dtype=torch.int32, device=dev)
+    call = lambda B: fr.gqa_xKV_rope(q, kA, B, vA, vB, torch.empty_like(q), ns, 1, 128 ** -0.5, 5e5)
+    got = call(odd)
+    assert shim_tail.count("shim_stage1") == 2
+    check_out(got, call(kB), "odd factor")
+
+
 @pytest.mark.parametrize("dtype", [BF, FP])
 @pytest.mark.parametrize("b,hq,hkv,L,r,shared", [
     (1, 8, 2, 2049, 192, True),          # rows of 24 lanes, two an instruction; a score row past whole packets by one
