@@ -380,8 +380,10 @@ void rope_operands(Ten q, int64_t hq, int64_t d, Ten kA, Ten kB, Ten inv) {
 bool scores_alone(Ten kB, int64_t r, int64_t G) {
   return rows(kB) && (r <= 224 ? G <= 16 : r == 384 ? G <= 4 : (r == 256 || r == 320 || r == 448) && G <= 8);
 }
+constexpr int64_t COPIED_FACTOR_WORK = 65536;   // a factor of rank 256 that is not 16-byte packets: copied for it (measured in recon_stage1.hip)
 int score_splits(const Call& c, Ten kB, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r) {
-  if (scores_alone(kB, r, G)) return balanced_splits(b, hkv, L, r <= 256 ? 64 : 32, 1, c.cus);
+  if (scores_alone(kB, r, G) || (r == 256 && G <= 8 && hkv >= 2 && b * hkv * L >= COPIED_FACTOR_WORK))
+    return balanced_splits(b, hkv, L, r <= 256 ? 64 : 32, 1, c.cus);
   const bool resident = ring_rank(r) && G <= 8;
   return balanced_splits(b, hkv, L, 32, resident || r > 256 ? 1 : r > 128 ? 2 : 3, c.cus);
 }

@@ -337,6 +337,19 @@ static int launch_recon(const ReconParams& p, int batch, hipStream_t st) {
   return launch_status();
 }
 
+constexpr int64_t COPIED_FACTOR_WORK = 65536;   // tokens x kv heads, as in host.cpp
+// kB [batch, hkv, rank, 128] of any strides but the last -> whole packets side by side
+__global__ __launch_bounds__(256) void copy_factor_kernel(const u16* __restrict__ kB, u16* __restrict__ out, int64_t sBb, int64_t sBh, int64_t sBr, int rank) {
+  typedef u16 u16x8 __attribute__((ext_vector_type(8)));
+  const int idx = blockIdx.z * 256 + threadIdx.x, row = idx >> 4, c = (idx & 15) * 8;
+  if (row >= rank) return;
+  const u16* src = kB + blockIdx.y * sBb + blockIdx.x * sBh + row * sBr + c;
+  u16x8 v;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = src[e];
+  st16(out + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * rank * 128 + row * 128 + c, v);
+}
+
 template <typename T>
 static int dispatch_recon(const ReconParams& p, int batch, bool vshared, hipStream_t st) {
   const bool so = p.scores != nullptr;
@@ -419,6 +432,14 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
     const bool here = rank == 256 ? spec : rank == 384 ? spec && hq / hkv <= 4 : true;
     if (here && recon_scores_serves(f, kB, sBb, sBh, sBr, rank))
       return launch_recon_scores(f, kB, sBb, sBh, sBr, batch, dtype, rank, st);
+    // A factor that is not 16-byte packets: at rank 256 a copy that is, in the workspace, once the call is long enough to pay for it.  us a call, the
+    // wave-specialised kernel (which packs any factor) / copy and this one, 32 heads on 8: 4096 tokens 11.6 / 11.8, 8192 13.7 / 13.0, 2 x 28611 52.4 / 37.7, 131072
+    // 95.9 / 71.3; 16 on 2, 16000 11.2 / 12.1, 32000 13.8 / 14.1; 8 on 1, 60000 13.6 / 16.9.  At rank 384 it gains 4 % of the longest and loses 1 us of the others
+    const int64_t head = (int64_t)rank * 128, copy_b = sBb == 0 ? 0 : hkv * head;
+    if (rank == 256 && spec && hkv >= 2 && (int64_t)batch * kv_len * hkv >= COPIED_FACTOR_WORK && recon_scores_serves(f, workspace, copy_b, head, 128, rank)) {
+      copy_factor_kernel<<<dim3(hkv, sBb == 0 ? 1 : batch, cdiv(rank * 16, 256)), dim3(256), 0, st>>>((const u16*)kB, (u16*)workspace, sBb, sBh, sBr, rank);
+      return launch_recon_scores(f, workspace, copy_b, head, 128, batch, dtype, rank, st);
+    }
   }
   // The wave-specialised kernel: rank 512 / 384 / 256, a basis shared by K and V (or scores that stay with it, or of a factor that is not 16-byte packets), computed
   // RoPE angles, at most 8 query heads per kv head
