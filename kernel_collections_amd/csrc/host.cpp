@@ -142,6 +142,14 @@ struct Call {
                 stream(c10::hip::getCurrentHIPStream(device).stream()), opts(q.options()) {}
   int64_t plan(int64_t bytes) { const int64_t at = used; used += (bytes + 255) & ~(int64_t)255; return at; }
   void alloc() { scratch = at::empty({used}, opts.dtype(at::kByte)); }
+  bool try_alloc() {   // false: no room for it
+    try {
+      alloc();
+    } catch (const c10::OutOfMemoryError&) {
+      return false;
+    }
+    return true;
+  }
   template <typename T> T* get(int64_t at) const { return reinterpret_cast<T*>(reinterpret_cast<char*>(scratch.data_ptr()) + at); }
 };
 inline void same(Ten q, std::initializer_list<const at::Tensor*> ts) {   // same 16-bit type, same device
@@ -421,7 +429,8 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         // scores first, then softmax and P.v_A in one stream for all heads.  The second pass reads the
         // scores in 16-byte packets, so their rows are whole packets: at another length the kernels get the padded one as the row's
         // and the true one as every sequence's (one fill, about 2 us).
-        const int64_t row = (L + 3) / 4 * 4;
+        // Where there is no room for the scores, one kernel, which needs none.
+        const int64_t row = (L + 3) / 4 * 4, one_kernel = c.used;
         at::Tensor lens;
         if (row != L) {
           lens = at::full({b}, L, c.opts.dtype(at::kInt));
@@ -430,13 +439,16 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         s.S = scan_splits(c, b, head_groups(hq), L, true);
         const int64_t sc = c.plan(b * hq * row * 4), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
         const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
-        c.alloc();
-        recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, score_splits(c, kB, b, hkv, hq / hkv, L, r), b, hq, hkv, row,
-              scale, invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes, s.lens);
-        check(p_xkv_softmax_pv_stage1(c.get<float>(sc), kv(vA, 0, rv), c.get<float>(part), c.get<float>(lse), nullptr, s.lens, b, hq, row, s.S,
-                                      0, nullptr, c.dt, c.stream), "xkv_softmax_pv_stage1");
-        merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, row, rv);
-        return;
+        if (c.try_alloc()) {
+          recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, score_splits(c, kB, b, hkv, hq / hkv, L, r), b, hq, hkv, row,
+                scale, invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes, s.lens);
+          check(p_xkv_softmax_pv_stage1(c.get<float>(sc), kv(vA, 0, rv), c.get<float>(part), c.get<float>(lse), nullptr, s.lens, b, hq, row, s.S,
+                                        0, nullptr, c.dt, c.stream), "xkv_softmax_pv_stage1");
+          merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, row, rv);
+          return;
+        }
+        c.used = one_kernel;
+        s.lens = nullptr;
       }
       s.S = decode_splits(b, hkv, L, r, shared, c.cus);
       const int64_t part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);

@@ -165,12 +165,17 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
             sin_cos = sin_cos.to(q_pe.dtype).contiguous()
     same_basis = (v_A.data_ptr() == k_A.data_ptr() and v_A.shape == k_A.shape and v_A.stride() == k_A.stride())
     asked = (lens is not None and batch > 1) or sin_cos is not None       # the caller's counts are taken
+    scores = None
     if (not same_basis and _two_pass(k_A.shape[-1], batch * kv_len, k_B, asked, rank_v) and sin_cos is None and hq // hkv <= 8 and hq <= 32
             and rank_v in (256, 384, 512) and kv_len % 4 == 0 and ops.USE_RECON_WORKSPACE):
+        try:
+            scores = torch.empty((batch, hq, kv_len), dtype=torch.float32, device=q_pe.device)
+        except torch.OutOfMemoryError:      # one kernel, which needs none
+            pass
+    if scores is not None:
         # A value basis of its own: two passes.  The scores-only form of the reconstruction kernel runs at the rate of the
         # shared-basis fused kernel (one row stream, no P.A); softmax and P.v_A then stream v_A once for all heads at HBM
         # rate.  Fused into one kernel, the second row stream costs more than the 2 x 4 bytes per score this moves.
-        scores = torch.empty((batch, hq, kv_len), dtype=torch.float32, device=q_pe.device)
         # the scores do not depend on how pass 1 cuts the range: one round of workgroups per CU
         S1 = ops.occupancy_splits(batch, hkv, kv_len, tile=64 if k_A.shape[-1] <= 256 else 32, waves=1)
         ops.recon_stage1(q3, k_A, k_B, None, None, None, scores, None, lens, batch, hq,

@@ -90,6 +90,32 @@ def test_out_of_memory_is_torchs_own_error(dev):
     assert call().shape == (b, 32, 1, L)
 
 
+@pytest.mark.parametrize("path,r,rv,shared", [("native", 192, 192, True), ("native", 256, 256, False), ("general", 256, 256, False)])
+def test_rope_decode_without_room_for_scores_takes_one_kernel(dev, path, r, rv, shared, monkeypatch):
+    """134 MB of scores where there are 32: the call needs none of them."""
+    import kernel_collections_amd.flash_recontruction as fr
+    from kernel_collections_amd.flash_recontruction.fused_attention import _fused
+    monkeypatch.setattr(_fused, "TWO_PASS_WORK_SHARED", {192: (1, 0)})
+    monkeypatch.setattr(_fused, "TWO_PASS_MIN_TOKENS", 0)
+    b, hq, L = 32, 32, 32768
+    t = lambda *s, std=1.0, n=0: gen(s, std=std, seed=n).to(dev)
+    q, A, B = t(b, hq, 128, std=0.4, n=1), t(1, L, r, n=2).expand(b, -1, -1), t(1, 8, r, 128, std=r ** -0.5, n=3).expand(b, -1, -1, -1)
+    V, vB = (A, B) if shared else (t(1, L, rv, n=4).expand(b, -1, -1), t(1, 8, rv, 128, std=rv ** -0.5, n=5).expand(b, -1, -1, -1))
+    if path == "general":
+        q = torch.empty(b, hq, 136, dtype=BF, device=dev)[..., :128].copy_(q)
+    o, ns = torch.empty(b, hq, 128, dtype=BF, device=dev), torch.ones(b, dtype=torch.int32, device=dev)
+    call = lambda: fr.gqa_xKV_rope(q, A, B, V, vB, o, ns, 1, 128 ** -0.5, 5e5)
+    want = call().clone()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    room = torch.cuda.memory_reserved() + (32 << 20)
+    try:
+        torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(dev).total_memory)
+        check_out(call(), want, "one kernel")
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
 def test_a_kernels_refusal_is_a_runtime_error(dev):
     """An error code of the C entry points keeps its text: rows wider than stage 1 serves."""
     import kernel_collections_amd.flash_recontruction as fr
