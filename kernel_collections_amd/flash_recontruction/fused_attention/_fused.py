@@ -93,16 +93,18 @@ def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_sca
 # Two passes (scores, then softmax + P.v_A) or one kernel: scores and values each run at the rate of a kernel made for them, but a third launch and
 # the scores' way through memory cost 5 - 8 us.  Where the two cross is a matter of the tokens scanned (batch x kv_len) times the kv heads, each of
 # which rebuilds them.  us of one kernel / two passes, 32 heads on 8 kv heads unless said:
-#   values of their own: rank 256 / 256, 8192 tokens 25.6 / 29.8, 16384 35.4 / 32.6 (16 on 4: 16384 27.4 / 28.2, 32768 34.3 / 31.1; 16 on 2: 32768 28.1 / 29.7,
-#   65536 39.1 / 37.3); 384 / 512, 16384 41.7 / 44.4, 32768 59.9 / 57.0 (16 on 4: 65536 63.8 / 59.8; 16 on 2: 65536 44.7 / 50.7); 512 / 512, 16384 43.3 / 47.4,
-#   32768 64.1 / 62.3; rank pairs without an 8-wave kernel, 512 / 384: 4096 31.5 / 32.0, 8192 45.6 / 37.3 (16 on 2: 16384 34.9 / 33.8)
-#   one basis: rank 192, 8192 26.4 / 28.4, 16384 34.1 / 31.8, 131072 143 / 78.7 (16 on 2: 65536 34.9 / 34.8); rank 256, 32768 36.1 / 40.0, 65536 60.0 / 56.3 (16 on 4:
-#   65536 40.3 / 42.0, 131072 59.1 / 58.0; 16 on 2: 131072 39.6 / 48.5); rank 384 and 512 one kernel up to 131072 tokens (122 / 130, 142 / 161)
+#   values of their own: rank 256 / 256, 8192 tokens 26.2 / 30.0, 12288 30.3 / 30.8, 16384 34.4 / 32.6 (16 on 2: 49152 33.6 / 33.6); 256 / 512, 12288 34.5 / 36.9, 16384 39.7 /
+#   39.2 (16 on 4: 32768 39.6 / 37.3; 16 on 2: 98304 53.7 / 56.0); 384 / 384, 16384 39.0 / 40.4, 28672 55.7 / 49.9 (16 on 4: 32768 40.8 / 40.1; 16 on 2: 98304 54.7 / 57.6); 384 /
+#   512, 16384 41.2 / 43.6, 28672 56.8 / 53.1 (16 on 4: 57344 57.0 / 54.9; 8 on 1: 200000 80.9 / 78.1); 512 / 512, 28672 58.7 / 58.9, 32768 64.3 / 63.5 (8 on 1: 200000 89.7 / 84.5);
+#   rank pairs without an 8-wave kernel, 512 / 384: 4096 31.8 / 33.2, 8192 45.5 / 38.8 (8 on 1: 98304 63.9 / 51.9)
+#   one basis: rank 128, 8192 23.5 / 25.6, 14336 28.7 / 27.4 (16 on 2: 57344 29.9 / 29.6; 8 on 1: 131072 33.2 / 32.5); rank 192, 8192 25.9 / 27.9, 14336 32.1 / 30.3, 131072 143 / 78.7
+#   (16 on 2: 57344 32.9 / 32.4; 8 on 1: 131072 36.2 / 37.8, 262144 52.9 / 55.4); rank 256, 32768 36.1 / 40.0, 51200 51.2 / 48.4 (16 on 4: 102400 51.0 / 50.3; 16 on 2: 131072
+#   39.6 / 48.5); rank 384 and 512 one kernel up to 131072 tokens (122 / 130, 142 / 161)
 TWO_PASS_KEY_RANKS = (512, 384, 256)
-TWO_PASS_MIN_TOKENS = 49152         # from here on at 8 kv heads whatever the ranks, and where a caller's counts are taken
-TWO_PASS_WORK = {(256, 256): 98304, (256, 512): 98304, (384, 384): 229376, (384, 512): 229376, (512, 512): 245760}   # pairs with an 8-wave kernel
-TWO_PASS_WORK_OTHER = 32768
-TWO_PASS_WORK_SHARED = {128: (1, 114688), 192: (1, 114688), 256: (4, 409600)}    # least kv heads, tokens x kv heads
+TWO_PASS_MIN_TOKENS = 49152         # where a caller's counts are taken, whatever the kv heads; the other lines are in thirds of it
+TWO_PASS_WORK = {(256, 256): 6, (256, 512): 8, (384, 384): 14, (384, 512): 14, (512, 512): 15}   # tokens x kv heads, pairs with an 8-wave kernel
+TWO_PASS_WORK_OTHER = 2
+TWO_PASS_WORK_SHARED = {128: (1, 114688), 192: (2, 114688), 256: (4, 409600)}    # least kv heads, tokens x kv heads
 # Key ranks up to 192 have no 8-wave kernel: two passes from this many tokens x kv heads on, and from four times as many at the ranks
 # that the generic kernel is instantiated for (key rank 64, value rank 256, 1024 tokens 17.6 / 18.9, 4096 27.8 / 24.7; 16 on 4, 2048 19.7 / 20.6, 3072 22.9 / 21.7;
 # 8 on 1, 8192 21.5 / 23.1, 12288 24.1 / 23.4; key rank 192, value rank 512, 4096 27.8 / 30.3, 8192 38.3 / 37.4, 16384 59.4 / 40.1; 16 on 4, 8192 28.5 / 30.2, 16384
@@ -121,7 +123,7 @@ def _two_pass(rank, tokens, k_B, asked=False, v_rank=512, shared=False):
         least, work = TWO_PASS_WORK_SHARED.get(rank, (1, float("inf")))
         return hkv >= least and tokens * hkv >= work
     if rank in TWO_PASS_KEY_RANKS:
-        work = min(TWO_PASS_WORK.get((rank, v_rank), TWO_PASS_WORK_OTHER), 8 * TWO_PASS_MIN_TOKENS)
+        work = TWO_PASS_WORK.get((rank, v_rank), TWO_PASS_WORK_OTHER) * TWO_PASS_MIN_TOKENS // 3
         return tokens * hkv >= work or (asked and tokens >= TWO_PASS_MIN_TOKENS)
     if rank > TWO_PASS_SMALL_RANK or not ops._row_ok(k_B):
         return False

@@ -179,6 +179,17 @@ def test_two_passes_at_small_key_ranks_where_they_are_faster(rank, hkv, tokens, 
     assert _fused._two_pass(rank, tokens, torch.zeros(1, hkv, rank, 128, dtype=torch.bfloat16)) == two
 
 
+@pytest.mark.parametrize("rank,v_rank,hkv,tokens,two", [
+    (256, 256, 8, 8192, False), (256, 256, 8, 12288, True), (256, 512, 8, 12288, False), (256, 512, 8, 16384, True), (256, 512, 2, 49152, False),
+    (384, 384, 8, 16384, False), (384, 384, 8, 28672, True), (512, 512, 8, 28672, False), (512, 512, 8, 32768, True), (512, 384, 8, 4096, True), (512, 384, 8, 2048, False),
+    (192, 0, 1, 262144, False), (192, 0, 2, 57344, True), (128, 0, 1, 131072, True), (256, 0, 2, 262144, False), (256, 0, 4, 102400, True), (384, 0, 8, 131072, False)])
+def test_two_passes_where_they_are_faster(rank, v_rank, hkv, tokens, two):
+    """Both sides as measured beside the lines; v_rank 0: one basis."""
+    from kernel_collections_amd.flash_recontruction.fused_attention import _fused
+    B = torch.zeros(1, hkv, rank, 128, dtype=torch.bfloat16)
+    assert _fused._two_pass(rank, tokens, B, v_rank=v_rank or rank, shared=not v_rank) == two
+
+
 @pytest.mark.parametrize("batch,groups,per_cu,jobs", [(1, 1, 1, 256), (32, 1, 1, 256), (128, 1, 1, 256), (129, 1, 1, 512), (64, 8, 2, 128),
                                                      (65, 8, 2, 192), (3, 300, 1, 6), (5, 512, 2, 10)])
 def test_ragged_batches_get_two_jobs_a_sequence(batch, groups, per_cu, jobs):
