@@ -243,7 +243,7 @@ def test_two_pass_rope_decode_of_any_factor(dev, shim_tail, rk, rv, batched, mon
     (3, 48, 4, 100, 192, True),          # 12 heads per kv head, groups of 24
     (1, 4, 1, 5, 128, True), (1, 8, 8, 33, 192, True),
 ])
-def test_two_pass_rope_decode_of_one_basis(dev, dtype, b, hq, hkv, L, r, shared, monkeypatch):
+def test_two_pass_rope_decode_of_one_basis(dev, shim_tail, dtype, b, hq, hkv, L, r, shared, monkeypatch):
     import kernel_collections_amd.flash_recontruction as fr
     from kernel_collections_amd.flash_recontruction.fused_attention import _fused
     monkeypatch.setattr(_fused, "TWO_PASS_MIN_TOKENS", 0)
@@ -259,7 +259,10 @@ def test_two_pass_rope_decode_of_one_basis(dev, dtype, b, hq, hkv, L, r, shared,
     call = lambda: fr.gqa_xKV_rope(qd, kAd, kBd, vAd, vBd, torch.zeros_like(qd), ns, 2, 128 ** -0.5, 5e5)
     for name, work in (("two passes", 0), ("one kernel", 1 << 40)):
         monkeypatch.setattr(_fused, "TWO_PASS_WORK_SHARED", {x: (1, work) for x in (128, 192, 256)})
+        monkeypatch.setattr(_fused, "TWO_PASS_KEY_RANKS", () if work else (512, 384, 256))
+        before = shim_tail.count("shim_stage1")
         check_out(call(), ref, name)
+        assert shim_tail.count("shim_stage1") - before == (1 if work else 2)
 
 
 @pytest.mark.parametrize("lens,floor,target", [
