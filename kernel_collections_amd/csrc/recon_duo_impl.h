@@ -1,7 +1,6 @@
 // Fused reconstruct + RoPE + softmax + P.A stage 1 with a SEPARATE value basis (a second row stream), which the
 // wave-specialised kernel (recon_spec_impl.h) is not built for: key rank 256 / 384 / 512, value rank 256 / 384 / 512, head_dim 128, computed
-// RoPE angles.  (The template also has a scores-only and a shared-basis mode; recon_scores.hip and
-// recon_spec_impl.h are the faster ones there and the dispatcher sends those shapes to them.)  Included by the recon_duo_*.hip translation units, which instantiate the shapes.
+// RoPE angles.  Included by the recon_duo_*.hip translation units, which instantiate the shapes.
 //
 // Work split.  One workgroup = one (batch, kv head, split), 8 wavefronts = two per SIMD.  The waves form a 2 x 4 grid
 // over (rank half kq, feature quarter dq): wave (kq, dq) keeps B[kh][RK/2 kq .. +RK/2][{16 dq .. +16} u {64 + 16 dq .. +16}]
@@ -37,8 +36,6 @@ typedef short s16x4d __attribute__((ext_vector_type(4)));
 typedef short s16x8d __attribute__((ext_vector_type(8)));
 typedef float f32x2d __attribute__((ext_vector_type(2)));
 
-enum { DUO_SCORES = 0, DUO_VSHARED = 1, DUO_VDISTINCT = 2 };
-
 constexpr int FT = 32;              // tokens per tile
 constexpr int NW = 8;               // wavefronts per workgroup
 constexpr int FSP_ROW = FT + 4;     // partial-score row stride (floats)
@@ -53,26 +50,24 @@ template <typename T> constexpr float lazy_rescale() { return std::is_same<T, _F
 // LDS budget: everything but the tile rings
 constexpr int DUO_TAIL = NW * 8 * FSP_ROW * 4 + 2 * 8 * 128 * 2 + 2 * 16 * FP_ROW * 2 + 32 * 4 + 16 * 4 + 32 * 2;
 
-template <int RK, int RV, int MODE>
+template <int RK, int RV>
 struct DuoShape {
-  static constexpr bool V2 = MODE == DUO_VDISTINCT;
   static constexpr int KROW = RK * 2 + 16;                 // padded key-tile row: 16 rows hit 16 distinct bank groups
   static constexpr int VROW = RV * 2 + 16;
-  static constexpr int KTILE = FT * KROW, VTILE = V2 ? FT * VROW : 0;
+  static constexpr int KTILE = FT * KROW, VTILE = FT * VROW;
   static constexpr int ROOM = 160 * 1024 - DUO_TAIL;
-  // one stream: as many slots as fit, at most 6.  Two streams: 2 value slots, and 3 key slots when they fit (else 2)
-  static constexpr int NSV = V2 ? 2 : 0;
+  // 2 value slots, and 3 key slots when they fit (else 2)
+  static constexpr int NSV = 2;
   static constexpr int NSK_FIT = (ROOM - NSV * VTILE) / KTILE;
-  static constexpr int NSK = V2 ? (NSK_FIT >= 3 ? 3 : 2) : (NSK_FIT > 6 ? 6 : NSK_FIT);
+  static constexpr int NSK = NSK_FIT >= 3 ? 3 : 2;
   static constexpr int SHM = NSK * KTILE + NSV * VTILE + DUO_TAIL;
-  static_assert(NSK >= 2 && (V2 || NSK >= 4), "ring too short");
   static_assert(SHM <= 160 * 1024, "LDS budget");
-  // key tile t + KAHEAD and (two streams) value tile t + VAHEAD are issued at the start of iteration t
-  static constexpr int KAHEAD = V2 ? NSK : NSK - 1;
+  // key tile t + KAHEAD and value tile t + VAHEAD are issued at the start of iteration t
+  static constexpr int KAHEAD = NSK;
   static constexpr int VAHEAD = NSV - 1;
-  static constexpr int LPT = V2 ? 8 : 4;                   // loads per wave and iteration
+  static constexpr int LPT = 8;                            // loads per wave and iteration
   // loads that may still be in flight where tile t+2's keys must have landed (end of I2 of iteration t) ...
-  static constexpr int WAIT_K = V2 ? 4 + 8 * (NSK - 2) : 4 * (NSK - 3);
+  static constexpr int WAIT_K = 4 + 8 * (NSK - 2);
   // ... and where tile t's values must have landed (end of I1 of iteration t)
   static constexpr int WAIT_V = 8 * VAHEAD;
   static_assert(WAIT_K < 64 && WAIT_V < 64, "vmcnt holds 6 bits");
@@ -164,16 +159,15 @@ __global__ __launch_bounds__(256) void duo_pack_b_kernel(const T* __restrict__ k
   }
 }
 
-template <typename T, int RK, int RV, int MODE>
+template <typename T, int RK, int RV>
 __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) {
   typedef typename Elem<T>::vec8 vec8;
-  typedef DuoShape<RK, RV, MODE> S;
-  constexpr bool SCORES = MODE == DUO_SCORES, V2 = MODE == DUO_VDISTINCT;
+  typedef DuoShape<RK, RV> S;
   constexpr int KROW = S::KROW, KTILE = S::KTILE, NSK = S::NSK, VROW = S::VROW, VTILE = S::VTILE, NSV = S::NSV;
   constexpr int NKS = RK / 32;        // k-steps (16 ranks each) of a wave's rank half
   constexpr int KA = NKS / 2;         // k-steps of tile t+1 that run in I1 (beside the rotation of tile t)
   constexpr int PF = 2;               // tile fragments read ahead of the MFMA that consumes them
-  constexpr int DV = V2 ? RV : RK;    // value features
+  constexpr int DV = RV;              // value features
   constexpr int NMB = DV / 128;       // 16-feature blocks of the DV / 8 value features a wave owns
   static_assert(RK % 128 == 0 && DV % 128 == 0 && KA >= 4, "shape");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -198,7 +192,7 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
 
   // ---- LDS carve-up ---------------------------------------------------------------------------------------------
   unsigned char* kring = smem;                                             // NSK * KTILE
-  unsigned char* vring = V2 ? smem + NSK * KTILE : smem;                   // NSV * VTILE (one stream: the key ring)
+  unsigned char* vring = smem + NSK * KTILE;                               // NSV * VTILE
   float* s_part = reinterpret_cast<float*>(smem + NSK * KTILE + NSV * VTILE);   // [8 waves][8 heads][FSP_ROW]
   sc_t* qhat = reinterpret_cast<sc_t*>(s_part + NW * 8 * FSP_ROW);         // [2][8 heads][128]
   T* p_lds = reinterpret_cast<T*>(qhat + 2 * 8 * 128);                                          // [2][16 head slots][FP_ROW]
@@ -213,14 +207,12 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
   // ---- async tile loads: wave w brings rows 4w .. 4w+3 of every tile ---------------------------------------------
   DuoStream<RK, KROW, NSK> ks_;
   ks_.init(reinterpret_cast<const unsigned char*>(p.kA) + b * p.sAb * 2, p.sAl, start, wave, lane, smem_lds);
-  DuoStream<V2 ? RV : RK, V2 ? VROW : KROW, V2 ? NSV : NSK> vs_;
-  if (V2) vs_.init(reinterpret_cast<const unsigned char*>(p.vA) + b * p.sVb * 2, p.sVl, start, wave, lane, smem_lds + NSK * KTILE);
+  DuoStream<RV, VROW, NSV> vs_;
+  vs_.init(reinterpret_cast<const unsigned char*>(p.vA) + b * p.sVb * 2, p.sVl, start, wave, lane, smem_lds + NSK * KTILE);
 #pragma unroll
   for (int i = 0; i < S::KAHEAD; ++i) ks_.issue(end, last, wave, lane);
-  if (V2) {
 #pragma unroll
-    for (int i = 0; i < S::VAHEAD; ++i) vs_.issue(end, last, wave, lane);
-  }
+  for (int i = 0; i < S::VAHEAD; ++i) vs_.issue(end, last, wave, lane);
 
   // ---- stationary B operands: NKS k-steps of one 32-feature block (16 low features + their 16 partners) ----------
   vec8 breg[NKS];
@@ -292,18 +284,14 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
   const sc_t* qrow = q_live ? qhat + ((lane & 7) < G ? (lane & 7) : G - 1) * 128 + (dq * 4 + g2) * 8 : qzero;
   const int qpar = q_live ? 8 * 128 : 0;   // q^ is double-buffered by tile parity, the zeros are not
   auto tr_read = [&](int t) {   // this wave's DV/8 value features of tile t, token-major
-    if (SCORES) return;
-    constexpr int VR = V2 ? VROW : KROW;
-    const unsigned char* vt = (V2 ? vring + (t % NSV) * VTILE : kring + (t % NSK) * KTILE) + (8 * g4 + (n16 >> 2)) * VR +
-                              (wave * (DV / 8) + 4 * (n16 & 3)) * 2;
+    const unsigned char* vt = vring + (t % NSV) * VTILE + (8 * g4 + (n16 >> 2)) * VROW + (wave * (DV / 8) + 4 * (n16 & 3)) * 2;
 #pragma unroll
     for (int mb = 0; mb < NMB; ++mb) {
       tr[2 * mb] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4d*)(vt + mb * 32));
-      tr[2 * mb + 1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4d*)(vt + mb * 32 + 4 * VR));
+      tr[2 * mb + 1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4d*)(vt + mb * 32 + 4 * VROW));
     }
   };
   auto pv = [&](int buf) {      // acc^T[feature, head] += V^T P^T over the tile held in tr, P and rescale factors from buffer buf
-    if (SCORES) return;
     const float al = alpha_lds[buf * 16 + n16];
     const vec8 pb = ld16<vec8>(p_lds + buf * (16 * FP_ROW) + n16 * FP_ROW + 8 * g4);
 #pragma unroll
@@ -354,7 +342,7 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
       if (ks == 2) {             // scalar address work and the load issue run under the MFMAs already in the pipe
         XKV_DUO_FENCE();
         ks_.issue(end, last, wave, lane);          // key tile t + KAHEAD, into the slot freed at the last barrier
-        if (V2) vs_.issue(end, last, wave, lane);  // value tile t + VAHEAD
+        vs_.issue(end, last, wave, lane);  // value tile t + VAHEAD
       }
       if (ks == (KA > 5 ? 5 : KA - 1)) {
         if ((n16 & 7) < G)
@@ -363,7 +351,7 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
       XKV_DUO_FENCE();
     }
     write_qhat(t + 1);       // into the buffer tile t does not read
-    if (V2) duo_wait_vmcnt<S::WAIT_V>();   // this wave's rows of value tile t have landed
+    duo_wait_vmcnt<S::WAIT_V>();   // this wave's rows of value tile t have landed
     __syncthreads();         // B1: partial scores of tile t, q^(t+1) visible; value tile t complete
     // ---- I2 ----
     // The softmax is a chain of dependent steps (LDS reads, adds, two cross-lane reductions, exponentials).  It is written
@@ -379,12 +367,9 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
         }
       }
     };
-    float al = 1.f;
-    vec8 pb;
-    if (!SCORES) {     // P and the rescale factors of tile t-1 were published before the last barrier
-      al = alpha_lds[(PAR ^ 1) * 16 + n16];
-      pb = ld16<vec8>(p_lds + (PAR ^ 1) * (16 * FP_ROW) + n16 * FP_ROW + 8 * g4);
-    }
+    // P and the rescale factors of tile t-1 were published before the last barrier
+    const float al = alpha_lds[(PAR ^ 1) * 16 + n16];
+    const vec8 pb = ld16<vec8>(p_lds + (PAR ^ 1) * (16 * FP_ROW) + n16 * FP_ROW + 8 * g4);
     f32x2d v[NW];
     {
       const float* sp = s_part + sm_row * FSP_ROW + 2 * n16;
@@ -397,57 +382,34 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
     mfmas(std::integral_constant<int, 0>());
     float s0 = ((v[0][0] + v[1][0]) + (v[2][0] + v[3][0])) + ((v[4][0] + v[5][0]) + (v[6][0] + v[7][0]));
     float s1 = ((v[0][1] + v[1][1]) + (v[2][1] + v[3][1])) + ((v[4][1] + v[5][1]) + (v[6][1] + v[7][1]));
-    float e0 = 0.f, e1 = 0.f, alpha = 1.f;
-    if (SCORES) {
-      if (sm_valid && lane < 16) {
-        const int64_t o = ((int64_t)b * p.hq + h0 + wave) * p.kv_len + tok;
-        s0 *= p.sm_scale;
-        s1 *= p.sm_scale;
-        if (p.scores_dtype == XKV_F32) {
-          float* dst = reinterpret_cast<float*>(p.scores) + o;
-          if (tok < end) dst[0] = s0;
-          if (tok + 1 < end) dst[1] = s1;
-        } else {
-          T* dst = reinterpret_cast<T*>(p.scores) + o;
-          if (tok < end) dst[0] = from_f32<T>(s0);
-          if (tok + 1 < end) dst[1] = from_f32<T>(s1);
-        }
-      }
-      XKV_DUO_FENCE();
-      mfmas(std::integral_constant<int, 1>());
-      mfmas(std::integral_constant<int, 2>());
-      mfmas(std::integral_constant<int, 3>());
-    } else {
-      s0 = s0 * p.sm_scale + (tok < end ? 0.f : NEG_INF);       // (finite) - inf = -inf: masked without a branch
-      s1 = s1 * p.sm_scale + (tok + 1 < end ? 0.f : NEG_INF);
-      XKV_DUO_FENCE();
-      // stage 1: the tile maximum of this head; the reference only moves when it exceeds it by lazy_rescale<T>()
-      mfmas(std::integral_constant<int, 1>());
-      const float mx = row_reduce<true, 16>(fmaxf(s0, s1));
-      const float m_new = mx > m_ref + lazy_rescale<T>() ? mx : m_ref;
-      XKV_DUO_FENCE();
-      // stage 2: exponentials, P and the rescale factor -> LDS (buffer t & 1; absent heads keep zeros)
-      mfmas(std::integral_constant<int, 2>());
-      alpha = __expf(m_ref - m_new);
-      m_ref = m_new;
-      e0 = __expf(s0 - m_ref);
-      e1 = __expf(s1 - m_ref);
-      T* pd = p_lds + PAR * (16 * FP_ROW) + wave * FP_ROW + 2 * n16;   // the four 16-lane groups store the same values
-      pd[0] = from_f32<T>(sm_valid ? e0 : 0.f);
-      pd[1] = from_f32<T>(sm_valid ? e1 : 0.f);
-      alpha_lds[PAR * 16 + wave] = sm_valid ? alpha : 1.f;
-      XKV_DUO_FENCE();
-      // stage 3: acc += P.A of tile t-1 from the operands in registers, then tile t's operands replace them
-      mfmas(std::integral_constant<int, 3>());
+    s0 = s0 * p.sm_scale + (tok < end ? 0.f : NEG_INF);       // (finite) - inf = -inf: masked without a branch
+    s1 = s1 * p.sm_scale + (tok + 1 < end ? 0.f : NEG_INF);
+    XKV_DUO_FENCE();
+    // stage 1: the tile maximum of this head; the reference only moves when it exceeds it by lazy_rescale<T>()
+    mfmas(std::integral_constant<int, 1>());
+    const float mx = row_reduce<true, 16>(fmaxf(s0, s1));
+    const float m_new = mx > m_ref + lazy_rescale<T>() ? mx : m_ref;
+    XKV_DUO_FENCE();
+    // stage 2: exponentials, P and the rescale factor -> LDS (buffer t & 1; absent heads keep zeros)
+    mfmas(std::integral_constant<int, 2>());
+    const float alpha = __expf(m_ref - m_new);
+    m_ref = m_new;
+    const float e0 = __expf(s0 - m_ref), e1 = __expf(s1 - m_ref);
+    T* pd = p_lds + PAR * (16 * FP_ROW) + wave * FP_ROW + 2 * n16;   // the four 16-lane groups store the same values
+    pd[0] = from_f32<T>(sm_valid ? e0 : 0.f);
+    pd[1] = from_f32<T>(sm_valid ? e1 : 0.f);
+    alpha_lds[PAR * 16 + wave] = sm_valid ? alpha : 1.f;
+    XKV_DUO_FENCE();
+    // stage 3: acc += P.A of tile t-1 from the operands in registers, then tile t's operands replace them
+    mfmas(std::integral_constant<int, 3>());
 #pragma unroll
-      for (int mb = 0; mb < NMB; ++mb) {
-        const vec8 a = __builtin_bit_cast(vec8, (s16x8d)__builtin_shufflevector(tr[2 * mb], tr[2 * mb + 1], 0, 1, 2, 3, 4, 5, 6, 7));
-        acc[mb] = Elem<T>::mfma16(a, pb, acc[mb] * al);
-      }
-      XKV_DUO_FENCE();
-      tr_read(t);
-      l_run = l_run * alpha + row_reduce<false, 16>(e0 + e1);
+    for (int mb = 0; mb < NMB; ++mb) {
+      const vec8 a = __builtin_bit_cast(vec8, (s16x8d)__builtin_shufflevector(tr[2 * mb], tr[2 * mb + 1], 0, 1, 2, 3, 4, 5, 6, 7));
+      acc[mb] = Elem<T>::mfma16(a, pb, acc[mb] * al);
     }
+    XKV_DUO_FENCE();
+    tr_read(t);
+    l_run = l_run * alpha + row_reduce<false, 16>(e0 + e1);
     XKV_DUO_FENCE();
     duo_wait_vmcnt<S::WAIT_K>();   // this wave's rows of key tile t+2 have landed
     __syncthreads();         // B2: P, rescale factors of tile t visible; key tile t+2 complete; the slots read in this
@@ -459,7 +421,6 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
   }
   pv((ntiles - 1) & 1);      // P.A of the last tile
   duo_wait_vmcnt<0>();       // the clamped look-ahead loads must land before the LDS is released
-  if (SCORES) return;
   if (sm_valid && lane == 0) { ml_lds[2 * wave] = m_ref; ml_lds[2 * wave + 1] = l_run; }
   __syncthreads();
 
@@ -475,12 +436,12 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
   }
 }
 
-template <typename T, int RK, int RV, int MODE>
+template <typename T, int RK, int RV>
 int launch_duo_t(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, hipStream_t st) {
-  typedef DuoShape<RK, RV, MODE> S;
+  typedef DuoShape<RK, RV> S;
   const int nb = sBb == 0 ? 1 : batch;   // one packed copy when the factor is shared by the batch
   duo_pack_b_kernel<T, RK><<<dim3(p.hkv, nb, 16), dim3(256), 0, st>>>((const T*)kB, (T*)p.Bp, sBb, sBh, sBr, p.hkv);
-  auto kern = recon_duo_kernel<T, RK, RV, MODE>;
+  auto kern = recon_duo_kernel<T, RK, RV>;
   static DynLds lds;
   const int e = ensure_dynamic_lds(lds, reinterpret_cast<const void*>(kern), S::SHM, true);
   if (e != XKV_OK) return e;
@@ -489,10 +450,10 @@ int launch_duo_t(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, 
   return launch_status();
 }
 
-template <int RK, int RV, int MODE>
+template <int RK, int RV>
 int launch_duo(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype, hipStream_t st) {
-  return dtype == XKV_BF16 ? launch_duo_t<__bf16, RK, RV, MODE>(p, kB, sBb, sBh, sBr, batch, st)
-                           : launch_duo_t<_Float16, RK, RV, MODE>(p, kB, sBb, sBh, sBr, batch, st);
+  return dtype == XKV_BF16 ? launch_duo_t<__bf16, RK, RV>(p, kB, sBb, sBh, sBr, batch, st)
+                           : launch_duo_t<_Float16, RK, RV>(p, kB, sBb, sBh, sBr, batch, st);
 }
 
 }  // namespace duo

@@ -18,7 +18,7 @@ struct FastParams {
 };
 
 // The wave-specialised 8-wave kernel (recon_spec_impl.h), one translation unit per key rank: the key basis reused as
-// the value basis, and scores only where a factor is not made of 16-byte packets.
+// the value basis, and the scores only that recon_scores.hip is not dispatched for (any factor, up to eight query heads per kv head).
 int launch_recon_spec_512(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
                           hipStream_t st);
 int launch_recon_spec_384(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
@@ -32,19 +32,18 @@ inline int launch_recon_spec(const FastParams& p, const void* kB, int64_t sBb, i
                        : launch_recon_spec_256(p, kB, sBb, sBh, sBr, batch, dtype, st);
 }
 
-// Scores only, up to 16 query heads per kv head (recon_scores.hip): ranks up to 256, multiples of 64 up to 512.  Reads kB as it is
+// Scores only (recon_scores.hip): ranks up to 224 with up to 16 query heads per kv head, 256, 320, 384 and 448 with up to 8.  Reads kB as it is
 // (16-byte packets of unit stride; Bp of the parameters is not used).
 bool recon_scores_serves(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int rank);
 int launch_recon_scores(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype, int rank,
                         hipStream_t st);
 
-// The 8-wave kernels (recon_duo_impl.h) for key ranks 256 / 384 / 512 with a separate value basis of rank rv (mode 2; the
-// kernel template also has a scores-only mode 0 and a shared-basis mode 1, which the kernels above now serve).  Each
-// translation unit serves the shapes it instantiates and returns DUO_NOT_MINE for the others.
+// The 8-wave kernels (recon_duo_impl.h) for key ranks 256 / 384 / 512 with a separate value basis of rank rv.  Each translation
+// unit serves the shapes it instantiates and returns DUO_NOT_MINE for the others.
 constexpr int DUO_NOT_MINE = -1000;
 int launch_recon_duo_b(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                       int mode, int rk, int rv, hipStream_t st);
+                       int rk, int rv, hipStream_t st);
 int launch_recon_duo_c(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                       int mode, int rk, int rv, hipStream_t st);
+                       int rk, int rv, hipStream_t st);
 
 }  // namespace xkv

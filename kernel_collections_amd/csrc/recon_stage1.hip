@@ -465,8 +465,8 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
     f.hq = hq; f.hkv = hkv; f.kv_len = kv_len; f.max_splits = max_splits; f.total_wg = batch * hkv * max_splits;
     f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
     f.vA = vA.ptr; f.sVb = vA.stride_b; f.sVl = vA.stride_l;
-    int rc = launch_recon_duo_b(f, kB, sBb, sBh, sBr, batch, dtype, 2, rank, vA.dim, st);
-    if (rc == DUO_NOT_MINE) rc = launch_recon_duo_c(f, kB, sBb, sBh, sBr, batch, dtype, 2, rank, vA.dim, st);
+    int rc = launch_recon_duo_b(f, kB, sBb, sBh, sBr, batch, dtype, rank, vA.dim, st);
+    if (rc == DUO_NOT_MINE) rc = launch_recon_duo_c(f, kB, sBb, sBh, sBr, batch, dtype, rank, vA.dim, st);
     if (rc != DUO_NOT_MINE) return rc;
   }
   return dtype == XKV_BF16 ? dispatch_recon<__bf16>(p, batch, vshared, st) : dispatch_recon<_Float16>(p, batch, vshared, st);
