@@ -707,7 +707,7 @@ def bench_ropedecode(args, dev):
                                % (L, rk, rv), "kv_splits": S},
         "roofline": {"bound": "mfma", "kernel": "recon_scores_kernel + latent_ring_kernel (given scores), two passes", "achieved": round(tf, 1), "peak": PEAK_BF16_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(tf / PEAK_BF16_TFLOPS, 4), "traffic": None,
-                     "note": "whole call (pack, stage 1, merge) over algorithmic FLOP", "algorithmic_flop": flops,
+                     "note": "whole call (scores, values, merge) over algorithmic FLOP", "algorithmic_flop": flops,
                      "hbm_side_GBps": round(B * L * (rk + rv) * 2 / (us * 1e-6) / 1e9, 1)},
         "uncompressed_flash_decode_us": round(comp_ms * 1e3 / args.steps, 2),
         "parity_vs_oracle": parity,

@@ -22,9 +22,9 @@
 // instructions of a tile are 1088 cycles, a block of 16 pairs takes 400 with everything else, and a group's start (barrier, q^)
 // 500 more.  A branch or a memory operation waited for on the spot costs such a wave its whole latency, so the groups are straight-line code: places
 // written whether they are needed or not, stores dropped by the resource's bounds, the output's form a template parameter.
-// us at 131072 tokens, 8 kv heads, 32 heads: rank 64 34.9, 128 45.8, 192 57.9, 256 63.8, 384 102, 512 126; the same with rows read in operand
-// order, rotation of keys by base and place, and branches 47.5, 53.7, 63.9, 77.8, 117, 141.  Two waves per SIMD with half the pairs each
-// and a barrier per step: 38.8, 50.5, 59.7, 73.7, 105, 173.
+// us at 131072 tokens, 8 kv heads, 32 heads: rank 64 34.9, 128 45.8, 192 57.9, 224 64.8, 256 63.8, 320 100, 384 102, 448 122; with rows read in operand
+// order, rotation of keys by base and place, and branches rank 64 47.5, 128 53.7, 192 63.9, 256 77.8, 384 117.  Two waves per SIMD with half the pairs each
+// and a barrier per step: 38.8, 50.5, 59.7, 73.7, 105.
 #include "recon_fast.h"
 #include "xkv_common.h"
 #include <type_traits>
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(256, 1) void recon_scores_kernel(const FastParams p
     block(i, u_c, IC<3>());
   };
   // The start of the group of steps from i on.  The barrier: every wave has written its q^ of this group and, last group, its scores;
-  // it has read those whose places are written next.
+  // it has read those whose places are written next (behind the last group a barrier of its own says so).
   auto group = [&]() {
     __syncthreads();
     if constexpr (WPT == 1) { s_out[0] = s_done[1]; s_out[1] = s_done[0]; }

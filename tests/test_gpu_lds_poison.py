@@ -4,7 +4,7 @@ pass a parity test when the previous launch left the same rows in the same place
 the same stream, by `xkv_poison_lds`, which leaves a NaN pattern in all 160 KiB of every CU: stale reads then show up as NaNs in
 the output.  Both host layers: the native one over launch_shim.cpp, which poisons before every stage-1 launch of a call, and the
 general one, launch by launch, under a poisoning binding.  The cases are the parity tests of test_gpu_parity.py themselves, one or two per kernel family that tracks its own
-loads (latent_ring, recon_spec, recon_fast, recon_duo) plus the generic kernels, called again.
+loads (latent_ring, recon_spec, recon_scores, recon_duo) plus the generic kernels, called again.
 """
 import ctypes
 
@@ -83,9 +83,9 @@ def test_ring_kernel_scores_and_decode(dev, dtype, poisoned):
 @pytest.mark.parametrize("dtype", [BF, FP])
 def test_reconstruction_kernels(dev, dtype, poisoned):
     tp.test_qab_rope(dev, dtype, 2, 32, 8, 1000, 512, 5e5)     # recon_spec, scores mode, rank 512
-    tp.test_qab_rope(dev, dtype, 2, 8, 2, 300, 384, 5e5)       # ... rank 384
-    tp.test_qab_rope(dev, dtype, 1, 8, 2, 77, 256, 1e7)        # recon_fast (4 waves), rank 256
-    tp.test_qab_rope(dev, dtype, 2, 4, 4, 40, 192, 1e7)        # generic kernel, rank 192
+    tp.test_qab_rope(dev, dtype, 2, 8, 2, 300, 384, 5e5)       # recon_scores, two waves a tile
+    tp.test_qab_rope(dev, dtype, 1, 8, 2, 77, 256, 1e7)        # recon_scores at its largest factor
+    tp.test_qab_rope(dev, dtype, 2, 4, 4, 40, 192, 1e7)        # recon_scores, rank 192
     tp.test_fused_rope(dev, dtype, 2, 32, 8, 3000, 512, 512, 4, True)    # recon_spec fused, shared basis
     tp.test_fused_rope(dev, dtype, 1, 32, 8, 1500, 256, 384, 3, False)   # a value basis of its own
 
