@@ -25,6 +25,7 @@
 #include <stdexcept>
 
 #include "../../include/xkv_hip.h"
+#include "head_rows.h"
 
 namespace {
 
@@ -513,16 +514,19 @@ PyObject* gqa(PyObject*, PyObject* const* a, Py_ssize_t n) {
       }
       // 2, 4 or 8 kv heads of 128 side by side in a token row: stage 1 serves every head of a split from one workgroup, one per CU
       const bool rows128 = (hkv == 8 || hkv == 4 || hkv == 2) && d == 128 && hq <= 32 && k.stride(2) == d && k.stride(1) >= hkv * d;
-      const bool in_row = rows128 && (fact ? ring_rank(dv) && v.stride(1) >= dv : v.stride(2) == d && v.stride(1) >= hkv * d);
+      const bool planned = lens.defined() && b > 1;   // one sequence is cut into the splits of the longest it may be
+      const bool in_row = rows128 && (fact ? ring_rank(dv) && v.stride(1) >= dv
+                                           : v.stride(2) == d && v.stride(1) >= hkv * d && xkv::head_rows_pay(hkv, hq, b, L, planned, false));
       // 512-wide token rows of other heads beside 512-wide value rows: the same form, against a block-diagonal query
       const bool wide4 = !in_row && fact && hkv * d == 512 && dv == 512 && hq <= 32 && k.stride(2) == d;
       const bool wide = in_row || wide4;
       const int per_cu = wide ? 1 : 2, groups = wide ? 1 : (int)hkv, longest_floor = wide ? floor_wide : floor_head;
       need(longest_floor > 0);
-      const int floor = std::min(longest_floor, split_floor(b, groups, L, per_cu, c.cus, fact));
+      int floor = split_floor(b, groups, L, per_cu, c.cus, fact);
+      if (in_row && !fact) floor = xkv::head_rows_floor(hkv, b * L, floor);
+      floor = std::min(longest_floor, floor);
       Ragged rg{};
       Splits s{0, 0, nullptr, nullptr};
-      const bool planned = lens.defined() && b > 1;   // one sequence is cut into the splits of the longest it may be
       if (planned) rg = ragged(c, s, b, groups, L, floor, per_cu);
       else s.S = std::min(balanced_splits(b, groups, L, 32, per_cu, c.cus), cdiv(L, floor));
       if (lens.defined()) s.lens = lens.data_ptr<int32_t>();
@@ -655,6 +659,13 @@ PyObject* py_decode_splits(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 6, [&]() -> PyObject* { return PyLong_FromLong(decode_splits(I(a[0]), I(a[1]), I(a[2]), I(a[3]), I(a[4]), I(a[5]))); });
 }
 
+// head_rows(heads, hq, batch, kv_len, ragged) -> bool and head_rows_floor(heads, tokens, floor) -> int (head_rows.h)
+PyObject* py_head_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 5, [&]() -> PyObject* { return PyBool_FromLong(xkv::head_rows_pay(I(a[0]), I(a[1]), I(a[2]), I(a[3]), I(a[4]), false)); });
+}
+PyObject* py_head_rows_floor(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 3, [&]() -> PyObject* { return PyLong_FromLong(xkv::head_rows_floor(I(a[0]), I(a[1]), I(a[2]))); });
+}
 // split_floor(batch, groups, kv_len, per_cu, cus, up) -> int
 PyObject* py_split_floor(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 6, [&]() -> PyObject* { return PyLong_FromLong(split_floor(I(a[0]), I(a[1]), I(a[2]), I(a[3]), I(a[4]), I(a[5]))); });
@@ -697,7 +708,8 @@ PyObject* init(PyObject*, PyObject* path) {
 #define XKV_FAST(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fn)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"init", init, METH_O, nullptr},       XKV_FAST("balanced_splits", py_balanced_splits), XKV_FAST("nope_decode", nope_decode), XKV_FAST("ragged_target", py_ragged_target),
-    XKV_FAST("split_floor", py_split_floor), XKV_FAST("decode_splits", py_decode_splits),
+    XKV_FAST("split_floor", py_split_floor), XKV_FAST("decode_splits", py_decode_splits), XKV_FAST("head_rows", py_head_rows),
+    XKV_FAST("head_rows_floor", py_head_rows_floor),
     XKV_FAST("nope_scores", nope_scores),  XKV_FAST("rope_decode", rope_decode),            XKV_FAST("rope_scores", rope_scores),
     XKV_FAST("gqa", gqa),                  XKV_FAST("mla", mla),                            XKV_FAST("prefix_tail", prefix_tail),
     {nullptr, nullptr, 0, nullptr}};

@@ -17,6 +17,7 @@
 
 #include "xkv_common.h"
 #include "latent_ring.h"
+#include "head_rows.h"
 
 namespace xkv {
 
@@ -447,7 +448,8 @@ extern "C" int xkv_latent_stage1(xkv_q_operand qn, const void* qn_lo, xkv_q_oper
   const int row_heads = n_kv_groups == 8 || n_kv_groups == 4 || n_kv_groups == 2 ? n_kv_groups : 0;
   if (!scores_only && !qn_lo && !dr && C.dim == 128 && row_heads && C.stride_h == 128 && C.stride_l >= row_heads * 128 &&
       hq <= 32) {
-    const bool v_heads = V.dim == 128 && V.stride_h == 128 && V.stride_l >= row_heads * 128;
+    const bool v_heads = V.dim == 128 && V.stride_h == 128 && V.stride_l >= row_heads * 128 &&
+                         head_rows_pay(row_heads, hq, batch, kv_len, kv_lens && batch > 1, split_plan != nullptr);
     const bool v_shared_row = V.stride_h == 0 && (V.dim == 256 || V.dim == 384 || V.dim == 512) && V.stride_l >= V.dim;
     if (v_heads || v_shared_row) {
       LatentParams w = p;

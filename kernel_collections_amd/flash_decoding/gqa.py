@@ -34,8 +34,11 @@ def _plan(wide, lens, splits, S, batch, groups, kv_len, device, up):
     floor, per_cu = (MAX_SPLIT_TOKENS_WIDE, 1) if wide else (MAX_SPLIT_TOKENS, 2)
     if not floor:
         return ops.as_int32_dev(splits, batch, device), 0, S, None
-    groups = 1 if wide else groups
-    floor = min(floor, ops.split_floor(batch, groups, kv_len, per_cu, up))
+    heads, groups = groups, 1 if wide else groups
+    least = ops.split_floor(batch, groups, kv_len, per_cu, up)
+    if wide and not up:
+        least = ops.head_rows_floor(heads, batch * kv_len, least)
+    floor = min(floor, least)
     if lens is not None and batch > 1:
         return ops.ragged_plan(lens, batch, groups, kv_len, floor, per_cu)
     S = min(ops.occupancy_splits(batch, groups, kv_len, tile=32, waves=per_cu), -(-kv_len // floor))
@@ -74,7 +77,8 @@ def decode_attention_fwd(q, k_buffer, v_buffer, o, num_kv_splits, max_kv_splits,
     # 2, 4 or 8 kv heads of 128 side by side in a token row: stage 1 serves every head of a split from one workgroup (whole
     # rows through its LDS ring), so there are hkv times fewer workgroups and a split may be twice as long
     wide = (hkv in (2, 4, 8) and d == 128 and hq <= 32 and k_buffer.stride(2) == d and v_buffer.stride(2) == d
-            and k_buffer.stride(1) >= hkv * d and v_buffer.stride(1) >= hkv * d)
+            and k_buffer.stride(1) >= hkv * d and v_buffer.stride(1) >= hkv * d
+            and ops.head_rows(hkv, hq, batch, kv_len, lens is not None and batch > 1))
     splits, cap, S, plan = _plan(wide, lens, num_kv_splits, S, batch, hkv, kv_len, q.device, False)
     partial, lse = ops.workspaces(batch, hq, S, dv, q.device, plan)
     ops.latent_stage1(q3, None, None,

@@ -290,6 +290,18 @@ def split_floor(batch: int, groups: int, kv_len: int, per_cu: int, up: bool) -> 
     return _xkv_host.split_floor(batch, groups, kv_len, per_cu, num_cus(), up)
 
 
+def head_rows(heads: int, hq: int, batch: int, kv_len: int, ragged: bool) -> bool:
+    """Whether plain keys and values of 2, 4 or 8 kv heads of 128 are scanned as one row per token (`csrc/head_rows.h`)."""
+    from . import _xkv_host
+    return _xkv_host.head_rows(heads, hq, batch, kv_len, ragged)
+
+
+def head_rows_floor(heads: int, tokens: int, floor: int) -> int:
+    """Shortest split of such rows, `floor` the shortest of others."""
+    from . import _xkv_host
+    return _xkv_host.head_rows_floor(heads, tokens, floor)
+
+
 def ragged_plan(lens, batch: int, groups: int, kv_len: int, floor: int, per_cu: int = 1):
     """Splits of a ragged batch: ``(None, cap, jobs, split plan on the device)``, the plan packed - or ``(None, cap, splits, None)`` for
     a batch that fits the device at the shortest splits.  The split length is planned on

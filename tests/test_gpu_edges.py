@@ -450,6 +450,24 @@ def test_value_rows_of_few_heads_far_apart(dev, stride, L):
     assert max_abs(out, ref) <= 2.0 ** -9 * 8      # as above
 
 
+@pytest.mark.parametrize("hq,hkv,b,L,ragged", [(32, 4, 1, 16384, False), (32, 4, 1, 16385, False), (12, 4, 2, 4096, False), (12, 4, 2, 4097, False), (4, 4, 3, 1, False),
+                                               (32, 4, 2, 2048, True), (32, 4, 2, 2049, True), (32, 2, 1, 8192, False), (32, 2, 1, 8193, False), (16, 2, 1, 4096, False), (16, 2, 1, 4097, False),
+                                               (16, 2, 1, 8001, False)])
+def test_few_heads_on_both_sides_of_the_lines(dev, hq, hkv, b, L, ragged):
+    """One workgroup per kv head or for all, through the native layer and the general one (a query that is not packed)."""
+    from kernel_collections_amd.flash_decoding import gqa
+    q, K, V = gen((b, hq, 128), std=0.3, seed=1), gen((b, L, hkv, 128), seed=2), gen((b, L, hkv, 128), seed=3)
+    lens = [L - 700 * i for i in range(b)] if ragged else [L] * b
+    s = torch.einsum("bkgd,blkd->bkgl", q.double().reshape(b, hkv, -1, 128), K.double())
+    s.masked_fill_(torch.arange(L) >= torch.tensor(lens)[:, None, None, None], float("-inf"))
+    ref = torch.einsum("bkgl,blkd->bkgd", torch.softmax(s, -1), V.double()).reshape(b, hq, 128).float()
+    qd, Kd, Vd, ns = q.to(dev), K.to(dev), V.to(dev), torch.full((b,), 3, dtype=torch.int32, device=dev)
+    kw = {"kv_lens": torch.tensor(lens, dtype=torch.int32, device=dev)} if ragged else {}
+    wide = torch.empty(b, hq, 136, dtype=BF, device=dev)[..., :128].copy_(qd)
+    for name, x in (("native", qd), ("general", wide)):
+        check_out(gqa.decode_attention_fwd(x, Kd, Vd, torch.empty_like(qd), ns, 3, 1.0, **kw), ref, name)
+
+
 def test_rows_of_a_tail_cost_the_prefix_scan_nothing(dev):
     """A prefix scan into a workspace with rows for a tail: workgroups without tokens would deal the others out unevenly."""
     b, hq, L, S = 16, 24, 17377, 16

@@ -270,3 +270,35 @@ def test_a_library_without_the_newer_entry_points_loads(tmp_path):
         _xkv_host.init(str(so))
     finally:
         _xkv_host.init(_lib.LIB_PATH)
+
+
+@pytest.mark.parametrize("hq,hkv,b,L,ragged,row", [
+    (32, 4, 1, 4000, False, False), (32, 4, 2, 8192, False, False), (32, 4, 2, 8193, False, True), (16, 4, 2, 4000, False, False), (16, 4, 1, 8193, False, True),
+    (32, 4, 2, 2048, True, False), (32, 4, 3, 1500, True, True), (16, 4, 3, 300, True, True), (32, 2, 1, 100, False, False), (32, 2, 1, 8193, False, True), (32, 2, 2, 100, True, True), (16, 2, 1, 100, False, True),
+    (32, 8, 1, 100, False, True)])
+def test_few_heads_are_one_row_where_that_is_faster(hq, hkv, b, L, ragged, row, monkeypatch):
+    """Both sides as measured beside the rule, and the splits of the general path for the kernel that runs."""
+    from kernel_collections_amd import _xkv_host
+    from kernel_collections_amd.flash_decoding import gqa
+
+    class Planned(Exception):
+        pass
+
+    def stop(batch, hq, S, dv, device, plan=None):
+        raise Planned(S)
+    assert ops.head_rows(hkv, hq, b, L, ragged) == row
+    monkeypatch.setattr(ops, "workspaces", stop)
+    monkeypatch.setattr(_lib, "require_gpu", lambda t: None)
+    if ragged:
+        return
+    z = lambda *s: torch.zeros(s, dtype=torch.bfloat16)
+    with pytest.raises(Planned) as e:
+        gqa.decode_attention_fwd(z(b, hq, 128), z(b, L, hkv, 128), z(b, L, hkv, 128), z(b, hq, 128), torch.ones(b, dtype=torch.int32), 1)
+    groups, per_cu = (1, 1) if row else (hkv, 2)
+    floor = ops.head_rows_floor(hkv, b * L, ops.split_floor(b, groups, L, per_cu, False))
+    assert e.value.args[0] == min(_xkv_host.balanced_splits(b, groups, L, 32, per_cu, ops.num_cus()), -(-L // floor))
+
+
+def test_rows_of_two_heads_have_no_split_of_one_tile():
+    assert [ops.head_rows_floor(h, t, 32) for h, t in ((2, 4096), (2, 4097), (2, 8000), (4, 8000), (8, 8000))] == [32, 64, 64, 32, 32]
+    assert ops.head_rows_floor(2, 9000, 128) == 128
