@@ -1,6 +1,6 @@
-// Split-K flash-decoding stage 1 for WIDE latent rows (256 .. 1024 features, optionally + 64 RoPE features):
+// Split-K flash-decoding stage 1 for WIDE latent rows (192 .. 1024 features, optionally + 64 RoPE features):
 // the bandwidth-bound scans of the path (absorbed no-PE xKV scores and decode, MLA over c_kv | k_pe, V-only
-// factorised decode with the per-head keys viewed as one 1024-wide row against a block-diagonal query).
+// factorised and plain decode with the keys of 2, 4 or 8 heads viewed as one row against a block-diagonal query).
 //
 // Same arithmetic as latent_stage1.hip; what differs is how bytes move.  A CU has to keep roughly
 // (HBM latency x its share of the HBM rate) = 60-100 KB of loads in flight to stream at full rate.  Here four extra
