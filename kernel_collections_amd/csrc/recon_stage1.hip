@@ -416,7 +416,7 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
   hipStream_t st = (hipStream_t)stream;
   const int64_t need = xkv_recon_workspace_bytes(batch, hkv, rank, sBb);
   const bool spec = rope && !sin_cos && (rank == 512 || rank == 384 || rank == 256) && hq / hkv <= 8 && workspace && need > 0 &&
-                    workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0;
+                    workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && kA.stride_l >= 0 && kA.stride_l < (1 << 25);   // 32-bit row offsets
   if (so && rope && !sin_cos) {
     FastParams f{};
     f.q = q_pe; f.kA = kA.ptr; f.sAb = kA.stride_b; f.sAl = kA.stride_l;
