@@ -26,6 +26,7 @@
 
 #include "../../include/xkv_hip.h"
 #include "head_rows.h"
+#include "recon_groups.h"
 
 namespace {
 
@@ -390,7 +391,15 @@ bool scores_alone(Ten kB, int64_t r, int64_t G) {
   return rows(kB) && (r <= 224 ? G <= 16 : r == 384 ? G <= 4 : (r == 256 || r == 320 || r == 448) && G <= 8);
 }
 constexpr int64_t COPIED_FACTOR_WORK = 65536;   // a factor of rank 256 that is not 16-byte packets: copied for it (measured in recon_stage1.hip)
+// Several kv heads a workgroup (recon_heads_impl.h) where that leaves enough workgroups: the splits, or 0
+int heads_splits(bool packets, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r, bool scores, int cus) {
+  const int nh = packets ? xkv::recon_heads(r, hkv, G, scores) : 0;
+  if (!nh || b * hkv * L < xkv::recon_heads_work(r, hkv)) return 0;
+  const int S = balanced_splits(b, hkv / nh, L, 32, 1, cus);
+  return b * (hkv / nh) * S >= xkv::RECON_HEADS_WORKGROUPS ? S : 0;
+}
 int score_splits(const Call& c, Ten kB, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r) {
+  if (const int S = heads_splits(rows(kB), b, hkv, G, L, r, true, c.cus)) return S;
   if (scores_alone(kB, r, G) || (r == 256 && G <= 8 && hkv >= 2 && b * hkv * L >= COPIED_FACTOR_WORK))
     return balanced_splits(b, hkv, L, r <= 256 ? 64 : 32, 1, c.cus);
   const bool resident = ring_rank(r) && G <= 8;
@@ -425,7 +434,9 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, kB.stride(0)), ws = c.plan(ws_bytes);
       const float* invp = inv.data_ptr<float>();
       Splits s{0, 0, nullptr, nullptr};
-      if (may_two_pass && (scores_alone(kB, r, hq / hkv) || (ring_rank(r) && hq / hkv <= 8)) && (joined() || hq <= 32) &&
+      // over one basis that kernel is ahead of two passes too (rank 256, 65536 tokens 55.5 / 45.6, 131072 87.7 / 73.0 us)
+      const int S_heads = shared ? heads_splits(rows(kB), b, hkv, hq / hkv, L, r, false, c.cus) : 0;
+      if (may_two_pass && !S_heads && (scores_alone(kB, r, hq / hkv) || (ring_rank(r) && hq / hkv <= 8)) && (joined() || hq <= 32) &&
           (ring_rank(rv) || (joined() && shared && (rv == 192 || rv == 128)))) {
         // scores first, then softmax and P.v_A in one stream for all heads.  The second pass reads the
         // scores in 16-byte packets, so their rows are whole packets: at another length the kernels get the padded one as the row's
@@ -451,7 +462,7 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         c.used = one_kernel;
         s.lens = nullptr;
       }
-      s.S = decode_splits(b, hkv, L, r, shared, c.cus);
+      s.S = S_heads ? S_heads : decode_splits(b, hkv, L, r, shared, c.cus);
       const int64_t part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
       const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
       c.alloc();

@@ -17,6 +17,8 @@ struct FastParams {
   const void* vA; int64_t sVb, sVl;             // separate value basis (recon_duo kernels only)
 };
 
+struct FactorOperand { const void* p; int64_t sb, sh, sr; };   // kB [batch, hkv, rank, 128]
+
 // The wave-specialised 8-wave kernel (recon_spec_impl.h), one translation unit per key rank: the key basis reused as
 // the value basis, and the scores only that recon_scores.hip is not dispatched for (any factor, up to eight query heads per kv head).
 int launch_recon_spec_512(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
@@ -30,6 +32,16 @@ inline int launch_recon_spec(const FastParams& p, const void* kB, int64_t sBb, i
   return rank == 512   ? launch_recon_spec_512(p, kB, sBb, sBh, sBr, batch, dtype, st)
          : rank == 384 ? launch_recon_spec_384(p, kB, sBb, sBh, sBr, batch, dtype, st)
                        : launch_recon_spec_256(p, kB, sBb, sBh, sBr, batch, dtype, st);
+}
+
+// Several kv heads per workgroup (recon_heads_impl.h): the shapes of recon_heads (recon_groups.h), factors of 16-byte packets, which it reads as they are.
+int launch_recon_heads_512(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st);
+int launch_recon_heads_384(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st);
+int launch_recon_heads_256(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st);
+inline int launch_recon_heads(const FastParams& p, const FactorOperand& kB, int batch, int dtype, int rank, hipStream_t st) {
+  return rank == 512   ? launch_recon_heads_512(p, kB, batch, dtype, st)
+         : rank == 384 ? launch_recon_heads_384(p, kB, batch, dtype, st)
+                       : launch_recon_heads_256(p, kB, batch, dtype, st);
 }
 
 // Scores only (recon_scores.hip): ranks up to 224 with up to 16 query heads per kv head, 256, 320, 384 and 448 with up to 8.  Reads kB as it is

@@ -49,8 +49,6 @@ constexpr int SEED = 16;             // steps between range-reduced base angles:
 enum { TO_F32, TO_16, TO_16_ODD };   // scores as stored: fp32, 16 bits a whole dword at a time, 16 bits each on its own (rows of odd length)
 constexpr int OUT = -1;              // lane offset that no resource reaches: the store is dropped
 
-struct FactorOperand { const void* p; int64_t sb, sh, sr; };
-
 template <int NKS, int WPT> struct ScoresShape {
   static constexpr int RK = 32 * NKS, RANK = RK * WPT;           // ranks of a wave
   static constexpr int STEP = 64 / WPT;                          // tokens

@@ -18,6 +18,7 @@
 // range-reduced sincosf every 32 tiles and advanced by a constant rotation in between.
 #include "xkv_common.h"
 #include "recon_fast.h"
+#include "recon_groups.h"
 #include <mutex>
 
 namespace xkv {
@@ -417,6 +418,18 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
   const int64_t need = xkv_recon_workspace_bytes(batch, hkv, rank, sBb);
   const bool spec = rope && !sin_cos && (rank == 512 || rank == 384 || rank == 256) && hq / hkv <= 8 && workspace && need > 0 &&
                     workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && kA.stride_l >= 0 && kA.stride_l < (1 << 25);   // 32-bit row offsets
+  // Several kv heads per workgroup, where the splits make enough of them: a factor of 16-byte packets, and whatever else the wave-specialised kernel asks for
+  const int nh = rope && !sin_cos ? recon_heads(rank, hkv, hq / hkv, so) : 0;
+  if (nh && (so || vshared) && spec && (int64_t)batch * (hkv / nh) * max_splits >= RECON_HEADS_WORKGROUPS &&
+      ((sBb | sBh | sBr) & 7) == 0 && (reinterpret_cast<uintptr_t>(kB) & 15) == 0) {
+    FastParams f{};
+    f.q = q_pe; f.kA = kA.ptr; f.sAb = kA.stride_b; f.sAl = kA.stride_l;
+    f.partial = partial; f.lse = lse; f.scores = scores_out; f.scores_dtype = scores_dtype;
+    f.num_splits = num_kv_splits; f.kv_lens = kv_lens;
+    f.hq = hq; f.hkv = hkv; f.kv_len = kv_len; f.max_splits = max_splits;
+    f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
+    return launch_recon_heads(f, FactorOperand{kB, sBb, sBh, sBr}, batch, dtype, rank, st);
+  }
   if (so && rope && !sin_cos) {
     FastParams f{};
     f.q = q_pe; f.kA = kA.ptr; f.sAb = kA.stride_b; f.sAl = kA.stride_l;

@@ -1,0 +1,104 @@
+"""recon_heads_kernel (several kv heads per workgroup) at the sizes where its periods, ring and tails end, against float64, with the LDS poisoned."""
+import pytest
+import torch
+
+from util import check_out, gen
+
+pytestmark = pytest.mark.gpu
+
+from kernel_collections_amd import _lib, ops  # noqa: E402
+
+BF, FP = torch.bfloat16, torch.float16
+NAN = 0x7FFF7FFF
+
+
+def keys_and_scores(q, A, B, off):
+    """Scores [b, hq, L] of rotated reconstructed keys, in float64 on the inputs' device."""
+    b, hkv, L, G = q.shape[0], B.shape[1], A.shape[1], q.shape[1] // B.shape[1]
+    inv = ops.rope_inv_freq(128, 5e5, torch.device("cpu")).to(q.device)
+    ang = (torch.arange(off, off + L, device=q.device).float()[:, None] * inv).double()
+    k = torch.matmul(A.double().unsqueeze(1), B.double())
+    lo, hi = k[..., :64], k[..., 64:]
+    k = torch.cat((lo * ang.cos() - hi * ang.sin(), hi * ang.cos() + lo * ang.sin()), -1)
+    s = torch.matmul(q.double().reshape(b, hkv, G, 128), k.transpose(-1, -2).contiguous())
+    return s.reshape(b, hkv * G, L)
+
+
+def operands(dev, dtype, b, hkv, G, L, r, stride):
+    q, B = gen((b, hkv * G, 128), std=0.5, dtype=dtype, seed=1).to(dev), gen((b, hkv, r, 128), std=r ** -0.5, dtype=dtype, seed=3).to(dev)
+    A = torch.full((b, L, stride), float("nan"), dtype=dtype, device=dev)[..., :r].copy_(gen((b, L, r), dtype=dtype, seed=2))
+    return q, A, B
+
+
+def poison():
+    assert _lib.lib().xkv_poison_lds(NAN, None, torch.cuda.current_stream().cuda_stream) == 0
+
+
+# S splits of n tiles each, the last one `cut` tokens short, in as many sequences as the kernel is taken for: every slot of the ring, both
+# parities, tails, seeds of the angles (every 28 tiles), head slots that stay empty
+S, WORKGROUPS = 24, 192
+SIZES = [(r, hkv, G, n, cut) for r, hkv in ((512, 2), (512, 8), (384, 4), (256, 4)) for n, cut, G in ((1, 31, 4), (2, 1, 1), (3, 0, 3), (4, 17, 4), (5, 30, 2), (33, 5, 4))]
+SIZES += [(r, 2, G, n, 9) for r in (512, 384) for n, G in ((1, 8), (6, 5), (31, 8))]
+
+
+def sequences(r, hkv):
+    return -(-WORKGROUPS * (4 if r == 256 else 2) // (hkv * S))
+
+
+@pytest.mark.parametrize("r,hkv,G,n,cut", SIZES)
+@pytest.mark.parametrize("dtype", [BF, FP])
+def test_decode(dev, dtype, r, hkv, G, n, cut):
+    b, L, hq, off = sequences(r, hkv), 32 * n * S - cut, hkv * G, 1000
+    q, A, B = operands(dev, dtype, b, hkv, G, L, r, r + 8)
+    lens = [L] + [L // 3 + 1] * (b - 1)
+    kl = torch.tensor(lens, dtype=torch.int32, device=dev)
+    part, lse = torch.full((b, hq, S, r), float("nan"), device=dev), torch.full((b, hq, S), float("nan"), device=dev)
+    poison()
+    ops.recon_stage1(q, A, B, A, part, lse, None, None, kl, b, hq, hkv, L, S, 128 ** -0.5, True, ops.rope_inv_freq(128, 5e5, q.device), off, None)
+    out = torch.empty((b, hq, r), device=dev)
+    ops.merge_stage2(part, lse, out, None, None, kl, b, hq, hq, L, S)
+    s = keys_and_scores(q, A, B, off) * 128 ** -0.5
+    for i, m in enumerate(lens):
+        ref = torch.softmax(s[i, :, :m], -1) @ A[i, :m].double()
+        check_out(out[i], ref, f"sequence {i}")
+        # P is 16 bits wide (2^-9 or 2^-11 of it), the keys and the query were in fp16 on the way
+        assert (out[i] - ref).norm() <= (4e-3 if dtype == BF else 2e-3) * ref.norm()
+
+
+@pytest.mark.parametrize("r,hkv,G,n,cut", [x for x in SIZES if x[0] != 256])
+@pytest.mark.parametrize("dtype,out", [(BF, torch.float32), (FP, FP)])
+def test_scores(dev, dtype, out, r, hkv, G, n, cut):
+    b, L, hq, off = sequences(r, hkv), 32 * n * S - cut, hkv * G, 77
+    q, A, B = operands(dev, dtype, b, hkv, G, L, r, r + 16)
+    ref = 0.25 * keys_and_scores(q, A, B, off)
+    for _ in range(3):
+        s = torch.full((b, hq, 1, L), float("nan"), dtype=out, device=dev)
+        poison()
+        ops.recon_stage1(q, A, B, None, None, None, s, None, None, b, hq, hkv, L, S, 0.25, True, ops.rope_inv_freq(128, 5e5, q.device), off, None)
+        d = s[:, :, 0].double() - ref
+        # The key and the query rounded to fp16 once each: 2.06e-4 of their size over all mantissas, together 2.9e-4; the result in fp16 as much more.  Angles in fp32
+        # up to position 25000: half a unit, 2^-10 radians, at the fastest pairs, half of that on average over tokens and 1 / 64 .. of the pairs: 1e-4.
+        assert d.norm() <= (3.5e-4 if out == torch.float32 else 4.2e-4) * ref.norm()
+        assert d.abs().max() <= 4e-3 * ref.abs().max()      # a tile read before it is there would be of the size of the scores
+
+
+@pytest.mark.parametrize("scale", [65504.0, 2.0 ** -12])
+def test_scores_of_large_and_small_queries(dev, scale):
+    """A rotated pair is up to 1.41 times as long as its larger feature, past fp16's largest number; a query below 6e-5 is subnormal there."""
+    q, A, B = operands(dev, FP, 1, 2, 4, 6144, 512, 512)
+    A *= 0.02
+    q = q.sign() * scale if scale > 1 else q * scale
+    s = torch.empty((1, 8, 1, 6144), device=dev)
+    ops.recon_stage1(q, A, B, None, None, None, s, None, None, 1, 8, 2, 6144, 192, 1.0, True, ops.rope_inv_freq(128, 5e5, q.device), 0, None)
+    ref = keys_and_scores(q, A, B, 0)
+    assert (s[:, :, 0].double() - ref).norm() <= 4e-4 * ref.norm()
+
+
+def test_splits_fill_the_device_once(dev, shim):
+    """A call past the line is cut for workgroups of several heads, a short one and one of a single kv head for one each."""
+    import kernel_collections_amd.flash_recontruction as fr
+    for hkv, L, r, groups in ((8, 12000, 512, 4), (8, 11000, 512, 8), (4, 32768, 384, 2), (4, 32700, 384, 4), (8, 32768, 256, 2), (8, 32000, 256, 8), (2, 163840, 512, 1), (2, 163800, 512, 2),
+                              (1, 200000, 512, 1)):
+        q, A, B = operands(dev, BF, 1, hkv, 4, L, r, r)
+        fr.gqa_xKV_rope(q, A, B, A, B, torch.empty_like(q), torch.ones(1, dtype=torch.int32, device=dev), 1, 0.1, 5e5)
+        assert shim.count("shim_recon_splits") == ops.occupancy_splits(1, groups, L, tile=32, waves=1)
