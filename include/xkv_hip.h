@@ -203,14 +203,14 @@ int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void* kB,
                      void* workspace, int64_t workspace_bytes,
                      int dtype, void* stream);
 
-/* Bytes of caller-owned scratch that lets xkv_recon_stage1 take its MFMA-bound fast path (kB re-packed into MFMA
- * operand order: one copy per batch entry, a single copy when stride_kB_b == 0).  0: no fast path for this rank.
+/* Bytes of caller-owned scratch that lets xkv_recon_stage1 take its MFMA-bound fast path (a copy of kB where it is not 16-byte
+ * packets: one per batch entry, a single one when stride_kB_b == 0; the other factors are read as they are).  0: no fast path for this rank.
  * Passing workspace == NULL (or too few bytes) is valid and selects the generic kernel.  No reference counterpart. */
 int64_t xkv_recon_workspace_bytes(int batch, int hkv, int rank, int64_t stride_kB_b);
 
 /* xkv_recon_stage1 for callers that cannot allocate device memory (code under HIP graph capture, serving loops or
  * harnesses that forbid hipMalloc): the same arguments without the workspace, the same kernels and results.  The scratch
- * that the fast paths need (xkv_recon_workspace_bytes(): kB re-packed into MFMA operand order) is a static device array of
+ * that the fast paths need (xkv_recon_workspace_bytes(): a copy of kB) is a static device array of
  * XKV_STATIC_SCRATCH_BYTES inside the library, one copy per GPU, held until the process ends; the call allocates and
  * frees nothing.  A shape that needs more (hkv * rank * 128 * 2 bytes per copy of kB, one copy per batch entry unless
  * stride_kB_b == 0) returns XKV_ESCRATCH and launches nothing.  Every call on a GPU uses that GPU's one array and
@@ -219,7 +219,7 @@ int64_t xkv_recon_workspace_bytes(int batch, int hkv, int rank, int64_t stride_k
  * The FIRST call on a device for a given kernel shape does host-side set-up (the array's address is looked up with
  * hipGetSymbolAddress, the kernel's dynamic LDS size is raised with hipFuncSetAttribute): make one warm-up call per device
  * and shape outside stream capture before capturing.  XKV_ESCRATCH is returned only for shapes that would take a path that
- * packs kB (generated RoPE angles, at most 8 query heads per kv head); other shapes run the generic kernel without scratch.
+ * may copy kB (generated RoPE angles, at most 8 query heads per kv head); other shapes run the generic kernel without scratch.
  * No counterpart in the reference, whose wrappers allocate with torch.empty on every call
  * (flash_recontruction/fused_attention/no_pe/v1.py:434-446). */
 #define XKV_STATIC_SCRATCH_BYTES (4 << 20)

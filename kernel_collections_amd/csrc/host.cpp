@@ -386,11 +386,8 @@ void rope_operands(Ten q, int64_t hq, int64_t d, Ten kA, Ten kB, Ten inv) {
 }
 // recon_scores_kernel: four tiles of 16 tokens a step (two beyond rank 256), one workgroup per CU; otherwise the kernels that hold a kv
 // head's factor in registers keep one, the generic kernel two or three.
-// what recon_scores_kernel runs, of the operands that this layer takes
-bool scores_alone(Ten kB, int64_t r, int64_t G) {
-  return rows(kB) && (r <= 224 ? G <= 16 : r == 384 ? G <= 4 : (r == 256 || r == 320 || r == 448) && G <= 8);
-}
-constexpr int64_t COPIED_FACTOR_WORK = 65536;   // a factor of rank 256 that is not 16-byte packets: copied for it (measured in recon_stage1.hip)
+// what recon_scores_kernel alone runs, of the operands that this layer takes
+bool scores_alone(Ten kB, int64_t r, int64_t G) { return rows(kB) && (r <= 224 ? G <= 16 : (r == 320 || r == 448) && G <= 8); }
 // Several kv heads a workgroup (recon_heads_impl.h) where that leaves enough workgroups: the splits, or 0
 int heads_splits(bool packets, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r, bool scores, int cus) {
   const int nh = packets ? xkv::recon_heads(r, hkv, G, scores) : 0;
@@ -400,7 +397,7 @@ int heads_splits(bool packets, int64_t b, int64_t hkv, int64_t G, int64_t L, int
 }
 int score_splits(const Call& c, Ten kB, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r) {
   if (const int S = heads_splits(rows(kB), b, hkv, G, L, r, true, c.cus)) return S;
-  if (scores_alone(kB, r, G) || (r == 256 && G <= 8 && hkv >= 2 && b * hkv * L >= COPIED_FACTOR_WORK))
+  if (scores_alone(kB, r, G) || xkv::recon_scores_pays(r, hkv, G, b * L))
     return balanced_splits(b, hkv, L, r <= 256 ? 64 : 32, 1, c.cus);
   const bool resident = ring_rank(r) && G <= 8;
   return balanced_splits(b, hkv, L, 32, resident || r > 256 ? 1 : r > 128 ? 2 : 3, c.cus);

@@ -3,14 +3,13 @@
 
 namespace xkv {
 
-int launch_recon_duo_b(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                       int rk, int rv, hipStream_t st) {
+int launch_recon_duo_b(const FastParams& p, const FactorOperand& kB, int batch, int dtype, int rk, int rv, hipStream_t st) {
   using namespace duo;
 #define XKV_DUO_CASE(RK, RV) \
-  if (rk == RK && rv == RV) return launch_duo<RK, RV>(p, kB, sBb, sBh, sBr, batch, dtype, st);
+  if (rk == RK && rv == RV) return launch_duo<RK, RV>(p, kB, batch, dtype, st);
   XKV_DUO_CASE(512, 512) XKV_DUO_CASE(384, 512) XKV_DUO_CASE(384, 384)
 #undef XKV_DUO_CASE
-  return DUO_NOT_MINE;
+  return XKV_EUNSUPPORTED;
 }
 
 }  // namespace xkv

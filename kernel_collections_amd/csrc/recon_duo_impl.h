@@ -27,6 +27,7 @@
 #pragma once
 #include "xkv_common.h"
 #include "recon_fast.h"
+#include "factor_rows.h"
 #include <type_traits>
 
 namespace xkv {
@@ -135,32 +136,8 @@ struct DuoStream {
   }
 };
 
-// ---------------------------------------------------------------------------------------------------------------
-// kB [hkv][RK][128] (strided) -> Bp [hkv][wave 8][ks RK/32][lane 64][8]: the 16-byte packet lane l = (n32, g2) of wave
-// (kq, dq) feeds to MFMA ks as the A operand: B[RK/2 kq + 16 ks + 8 g2 + e][feature], feature = 16 dq + n32 for the low
-// half of the block (n32 < 16) and 64 + 16 dq + n32 - 16 (the rotate-half partner) for the upper half.
-// ---------------------------------------------------------------------------------------------------------------
-template <typename T, int RK>
-__global__ __launch_bounds__(256) void duo_pack_b_kernel(const T* __restrict__ kB, T* __restrict__ Bp, int64_t sBb, int64_t sBh,
-                                                          int64_t sBr, int hkv) {
-  constexpr int NKS = RK / 32;
-  const int kh = blockIdx.x, b = blockIdx.y;
-  const T* Bh = kB + b * sBb + kh * sBh;
-  T* out = Bp + ((int64_t)b * hkv + kh) * (RK * 128);
-  for (int idx = blockIdx.z * 256 + threadIdx.x; idx < NW * NKS * 64; idx += 256 * gridDim.z) {
-    const int l = idx & 63, ks = (idx >> 6) % NKS, w = idx / (64 * NKS);
-    const int kq = w >> 2, dq = w & 3, n32 = l & 31;
-    const int col = n32 < 16 ? 16 * dq + n32 : 64 + 16 * dq + n32 - 16;
-    const int row0 = (RK / 2) * kq + 16 * ks + 8 * (l >> 5);
-    typename Elem<T>::vec8 v;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = Bh[(int64_t)(row0 + e) * sBr + col];
-    st16(out + (int64_t)idx * 8, v);
-  }
-}
-
 template <typename T, int RK, int RV>
-__global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) {
+__global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p, const FactorOperand kB) {
   typedef typename Elem<T>::vec8 vec8;
   typedef DuoShape<RK, RV> S;
   constexpr int KROW = S::KROW, KTILE = S::KTILE, NSK = S::NSK, VROW = S::VROW, VTILE = S::VTILE, NSV = S::NSV;
@@ -200,6 +177,17 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
   float* ml_lds = alpha_lds + 32;                                          // [8][2]
   sc_t* qzero = reinterpret_cast<sc_t*>(ml_lds + 16);                      // [32] zeros: the q-dot operand of masked lanes
   const unsigned smem_lds = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
+  // ---- frequencies and queries: in front of the loads that take longer
+  float freq[8];         // of this lane's pairs 16 dq + 8 (r / 4) + 4 g2 + r % 4
+#pragma unroll
+  for (int r = 0; r < 8; ++r) freq[r] = p.inv_freq[16 * dq + 8 * (r >> 2) + 4 * g2 + (r & 3)];
+  const float qinv = p.inv_freq[lane];
+  T qraw[2] = {};
+  if (wave < G) {        // head slot = wave, pair = lane
+    const T* qrow = reinterpret_cast<const T*>(p.q) + ((int64_t)b * p.hq + h0 + wave) * 128;
+    qraw[0] = qrow[lane];
+    qraw[1] = qrow[lane + 64];
+  }
   for (int i = tid; i < 2 * 16 * FP_ROW; i += 64 * NW) p_lds[i] = from_f32<T>(0.f);   // slots of absent heads stay zero
   if (tid < 32) alpha_lds[tid] = 1.f;
   if (tid < 32) qzero[tid] = from_f32<sc_t>(0.f);
@@ -214,13 +202,11 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
 #pragma unroll
   for (int i = 0; i < S::VAHEAD; ++i) vs_.issue(end, last, wave, lane);
 
-  // ---- stationary B operands: NKS k-steps of one 32-feature block (16 low features + their 16 partners) ----------
-  vec8 breg[NKS];
-  {
-    const T* bp = reinterpret_cast<const T*>(p.Bp) + b * p.sBpb + (int64_t)kh * (RK * 128) + ((int64_t)wave * (64 * NKS) + lane) * 8;
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) breg[ks] = ld16<vec8>(bp + ks * 512);
-  }
+  // ---- the factor, through the value slots that no first tile is on its way to, and the scores behind them
+  typedef FactorRows<T, RK> Factor;
+  static_assert((NSV - S::VAHEAD) * VTILE + NW * 8 * FSP_ROW * 4 >= Factor::BYTES, "room for two chunks");
+  Factor factor;
+  factor.template init<true>(reinterpret_cast<const T*>(kB.p) + b * kB.sb + kh * kB.sh, kB.sr, tid);
 
   // ---- in-tile rotation table: accumulator registers r and r + 8 of lane (token n32, g2) are the two members of pair
   // j = 16 dq + 8 (r / 4) + 4 g2 + r % 4 ---------------------------------------------------------------------------------
@@ -230,20 +216,14 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
 #pragma unroll
   for (int r = 0; r < 8; r += 2) {
     float c0, s0, c1, s1;
-    __sincosf((float)n32 * p.inv_freq[16 * dq + 8 * (r >> 2) + 4 * g2 + (r & 3)], &s0, &c0);
-    __sincosf((float)n32 * p.inv_freq[16 * dq + 8 * ((r + 1) >> 2) + 4 * g2 + ((r + 1) & 3)], &s1, &c1);
+    __sincosf((float)n32 * freq[r], &s0, &c0);
+    __sincosf((float)n32 * freq[r + 1], &s1, &c1);
     ch[r >> 1] = rot2{(_Float16)c0, (_Float16)c1};
     sh[r >> 1] = rot2{(_Float16)s0, (_Float16)s1};
   }
 
   // ---- query-side base rotation: thread -> (head slot = wave, pair j = lane) -------------------------------------------
-  float q0 = 0.f, q1 = 0.f;
-  if (wave < G) {
-    const T* qrow = reinterpret_cast<const T*>(p.q) + ((int64_t)b * p.hq + h0 + wave) * 128;
-    q0 = to_f32(qrow[lane]);
-    q1 = to_f32(qrow[lane + 64]);
-  }
-  const float qinv = p.inv_freq[lane];
+  const float q0 = to_f32(qraw[0]), q1 = to_f32(qraw[1]);
   // q^ is kept in q-dot operand order: pair j = 16 dq' + 8 o + 4 g' + e sits at [dq'][o][g'][e] (partner at e + 4), so
   // that a lane's 8 contraction values are one 16-byte read
   const int qpos = (lane >> 2) * 8 + (lane & 3);
@@ -304,8 +284,10 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
   // ---- pipeline ------------------------------------------------------------------------------------------------------------
   const f32x16 z16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   write_qhat(0);
-  duo_wait_vmcnt<0>();      // the first tiles and the B operands
-  // the compiler cannot see the direct-to-LDS loads: make it finish its own loads here, not inside the loop
+  // ---- stationary B operands: NKS k-steps of one 32-feature block (16 low features + their 16 partners), of this wave's rank half
+  vec8 breg[NKS];
+  factor.pass(reinterpret_cast<T*>(vring + S::VAHEAD * VTILE), tid, [&](int ch, const T* buf) { breg[ch] = Factor::operand(buf, 16 * kq, dq, lane); });
+  duo_wait_vmcnt<0>();      // the first tiles
 #pragma unroll
   for (int ks = 0; ks < NKS; ++ks) asm volatile("" : "+v"(breg[ks]));
   __syncthreads();
@@ -437,23 +419,20 @@ __global__ __launch_bounds__(64 * NW) void recon_duo_kernel(const FastParams p) 
 }
 
 template <typename T, int RK, int RV>
-int launch_duo_t(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, hipStream_t st) {
+int launch_duo_t(const FastParams& p, const FactorOperand& kB, int batch, hipStream_t st) {
   typedef DuoShape<RK, RV> S;
-  const int nb = sBb == 0 ? 1 : batch;   // one packed copy when the factor is shared by the batch
-  duo_pack_b_kernel<T, RK><<<dim3(p.hkv, nb, 16), dim3(256), 0, st>>>((const T*)kB, (T*)p.Bp, sBb, sBh, sBr, p.hkv);
   auto kern = recon_duo_kernel<T, RK, RV>;
   static DynLds lds;
   const int e = ensure_dynamic_lds(lds, reinterpret_cast<const void*>(kern), S::SHM, true);
   if (e != XKV_OK) return e;
   const int total = batch * p.hkv * p.max_splits;
-  kern<<<dim3(xcd_grid(total, p.hkv)), dim3(64 * NW), S::SHM, st>>>(p);
+  kern<<<dim3(xcd_grid(total, p.hkv)), dim3(64 * NW), S::SHM, st>>>(p, kB);
   return launch_status();
 }
 
 template <int RK, int RV>
-int launch_duo(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype, hipStream_t st) {
-  return dtype == XKV_BF16 ? launch_duo_t<__bf16, RK, RV>(p, kB, sBb, sBh, sBr, batch, st)
-                           : launch_duo_t<_Float16, RK, RV>(p, kB, sBb, sBh, sBr, batch, st);
+int launch_duo(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st) {
+  return dtype == XKV_BF16 ? launch_duo_t<__bf16, RK, RV>(p, kB, batch, st) : launch_duo_t<_Float16, RK, RV>(p, kB, batch, st);
 }
 
 }  // namespace duo

@@ -6,8 +6,8 @@
 namespace xkv {
 
 struct FastParams {
-  const void* q; const void* kA; const void* Bp;   // Bp: kB re-packed into MFMA operand order (caller workspace)
-  int64_t sAb, sAl, sBpb;
+  const void* q; const void* kA;
+  int64_t sAb, sAl;
   float* partial; float* lse;
   void* scores; int scores_dtype;               // scores != NULL: write [batch, hq, kv_len] scaled scores, no softmax / P.A
   const int32_t* num_splits; const int32_t* kv_lens;
@@ -17,24 +17,20 @@ struct FastParams {
   const void* vA; int64_t sVb, sVl;             // separate value basis (recon_duo kernels only)
 };
 
-struct FactorOperand { const void* p; int64_t sb, sh, sr; };   // kB [batch, hkv, rank, 128]
+struct FactorOperand { const void* p; int64_t sb, sh, sr; };   // kB [batch, hkv, rank, 128] in 16-byte packets
 
 // The wave-specialised 8-wave kernel (recon_spec_impl.h), one translation unit per key rank: the key basis reused as
-// the value basis, and the scores only that recon_scores.hip is not dispatched for (any factor, up to eight query heads per kv head).
-int launch_recon_spec_512(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                          hipStream_t st);
-int launch_recon_spec_384(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                          hipStream_t st);
-int launch_recon_spec_256(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                          hipStream_t st);
-inline int launch_recon_spec(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                             int rank, hipStream_t st) {
-  return rank == 512   ? launch_recon_spec_512(p, kB, sBb, sBh, sBr, batch, dtype, st)
-         : rank == 384 ? launch_recon_spec_384(p, kB, sBb, sBh, sBr, batch, dtype, st)
-                       : launch_recon_spec_256(p, kB, sBb, sBh, sBr, batch, dtype, st);
+// the value basis, and the scores only that recon_scores.hip is not dispatched for (up to eight query heads per kv head).
+int launch_recon_spec_512(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st);
+int launch_recon_spec_384(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st);
+int launch_recon_spec_256(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st);
+inline int launch_recon_spec(const FastParams& p, const FactorOperand& kB, int batch, int dtype, int rank, hipStream_t st) {
+  return rank == 512   ? launch_recon_spec_512(p, kB, batch, dtype, st)
+         : rank == 384 ? launch_recon_spec_384(p, kB, batch, dtype, st)
+                       : launch_recon_spec_256(p, kB, batch, dtype, st);
 }
 
-// Several kv heads per workgroup (recon_heads_impl.h): the shapes of recon_heads (recon_groups.h), factors of 16-byte packets, which it reads as they are.
+// Several kv heads per workgroup (recon_heads_impl.h): the shapes of recon_heads (recon_groups.h).
 int launch_recon_heads_512(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st);
 int launch_recon_heads_384(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st);
 int launch_recon_heads_256(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st);
@@ -45,17 +41,14 @@ inline int launch_recon_heads(const FastParams& p, const FactorOperand& kB, int 
 }
 
 // Scores only (recon_scores.hip): ranks up to 224 with up to 16 query heads per kv head, 256, 320, 384 and 448 with up to 8.  Reads kB as it is
-// (16-byte packets of unit stride; Bp of the parameters is not used).
+// (16-byte packets of unit stride).
 bool recon_scores_serves(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int rank);
 int launch_recon_scores(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype, int rank,
                         hipStream_t st);
 
-// The 8-wave kernels (recon_duo_impl.h) for key ranks 256 / 384 / 512 with a separate value basis of rank rv.  Each translation
-// unit serves the shapes it instantiates and returns DUO_NOT_MINE for the others.
-constexpr int DUO_NOT_MINE = -1000;
-int launch_recon_duo_b(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                       int rk, int rv, hipStream_t st);
-int launch_recon_duo_c(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                       int rk, int rv, hipStream_t st);
+// The 8-wave kernels (recon_duo_impl.h): key ranks 256 / 384 / 512 with a separate value basis of rank rv
+inline bool recon_duo_serves(int rk, int rv) { return rv == rk || (rv == 512 && (rk == 384 || rk == 256)); }
+int launch_recon_duo_b(const FastParams& p, const FactorOperand& kB, int batch, int dtype, int rk, int rv, hipStream_t st);   // 512 and 384
+int launch_recon_duo_c(const FastParams& p, const FactorOperand& kB, int batch, int dtype, int rk, int rv, hipStream_t st);   // 256
 
 }  // namespace xkv

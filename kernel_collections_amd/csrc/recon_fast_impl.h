@@ -1,5 +1,4 @@
-// Pieces of the reconstruction kernels that read a tile for all ranks (recon_spec_impl.h, recon_heads_impl.h): direct-to-LDS row loads, the packed factor,
-// tile constants.
+// Pieces of the reconstruction kernels that read a tile for all ranks (recon_spec_impl.h, recon_heads_impl.h): direct-to-LDS row loads, tile constants.
 #pragma once
 #include "xkv_common.h"
 #include "recon_fast.h"
@@ -50,28 +49,6 @@ template <int RK, int OFF> __device__ __forceinline__ void row_to_lds(u32x4 res,
                  : "=&v"(at) : "s"(lds), "s"(row_off), "v"(lane16), "s"(res), "n"(OFF), "s"((1ull << (RK / 8 % 64)) - 1) : "memory", "m0", "scc");
 }
 template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
-// ---------------------------------------------------------------------------------------------------------------
-// kB [hkv][RK][128] (strided) -> Bp [hkv][wave 4][ks RK/16][lane 64][8]: the 16-byte packet lane l of reconstruction wave w feeds to k-step
-// ks as the A operand: B[16 ks + 8 (l / 32) + e][64 (l % 32 / 16) + 16 w + l % 16].
-// ---------------------------------------------------------------------------------------------------------------
-template <typename T, int RK>
-__global__ __launch_bounds__(256) void pack_b_kernel(const T* __restrict__ kB, T* __restrict__ Bp, int64_t sBb, int64_t sBh,
-                                                      int64_t sBr, int hkv) {
-  const int kh = blockIdx.x, b = blockIdx.y;
-  const T* Bh = kB + b * sBb + kh * sBh;
-  constexpr int NK = RK / 16;
-  T* out = Bp + ((int64_t)b * hkv + kh) * (RK * 128);
-  for (int idx = blockIdx.z * 256 + threadIdx.x; idx < 4 * NK * 64; idx += 256 * gridDim.z) {
-    const int l = idx & 63, ks = (idx >> 6) % NK, w = idx / (64 * NK);
-    const int col = 64 * ((l >> 4) & 1) + 16 * w + (l & 15);
-    const int row0 = 16 * ks + 8 * (l >> 5);
-    typename Elem<T>::vec8 v;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = Bh[(int64_t)(row0 + e) * sBr + col];
-    st16(out + (int64_t)idx * 8, v);
-  }
-}
 
 #define XKV_FENCE() __builtin_amdgcn_sched_barrier(0)
 

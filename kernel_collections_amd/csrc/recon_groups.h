@@ -1,5 +1,5 @@
-// kv heads that a workgroup of recon_heads_kernel (recon_heads_impl.h) serves, and from which size on, for stage 1's dispatcher and the host layers that
-// choose its splits.
+// Which kernel serves a call of generated angles at ranks 512, 384 and 256, from which size on: kv heads that a workgroup of recon_heads_kernel (recon_heads_impl.h)
+// serves, and scores by recon_scores_kernel, for stage 1's dispatcher and the host layers that choose its splits.
 #pragma once
 #include <cstdint>
 
@@ -15,18 +15,25 @@ inline int recon_heads(int rank, int hkv, int G, bool scores) {
 
 // Tokens x kv heads from which on host layers plan for it: a workgroup reads two or four factors before it starts, and has a half or a quarter of the tokens
 // of one for one head.  us a call, one head a workgroup (recon_spec_kernel) / several, 32 heads on 8 kv heads unless said.
-//   rank 512: 4096 tokens 24.4 / 25.3, 8192 28.1 / 28.4, 12000 31.9 / 30.9, 24000 42.1 / 40.1; 16 on 4, 2 x 12000 31.4 / 31.0; 64 on 8, 12000 33.4 / 33.4
-//   rank 384: 8192 23.6 / 25.1, 16384 29.6 / 29.7, 24000 35.2 / 34.3; 16 on 4, 2 x 12000 26.2 / 27.5, 32768 30.8 / 30.2
-//   rank 256: 16384 24.5 / 27.5, 24000 28.9 / 30.2, 32768 33.5 / 33.4, 48000 41.7 / 40.2; 16 on 4, 32768 25.9 / 28.3, 65536 34.6 / 34.5
-//   two kv heads, one workgroup for both: nothing is left to share a row's way from memory with.  Rank 512, 66000 36.8 / 39.5, 131072 57.6 / 58.5, 262144 92.4 / 88.8; rank 384, 66000
-//   32.1 / 33.3, 131072 47.4 / 46.6, 262144 78.0 / 73.9
-//   scores alone: rank 512, 8192 15.7 / 15.6, 16384 22.8 / 21.8, 16 on 2, 66000 23.5 / 25.1, 131072 43.6 / 42.0; rank 384, 8192 13.3 / 13.2, 16384 18.9 / 18.2, 16 on 2, 66000 20.2 / 21.4
+//   rank 512: 12000 tokens 30.5 / 32.4, 20000 37.3 / 37.8, 24000 41.1 / 41.1, 32000 49.3 / 47.9; 16 on 4, 2 x 24000 40.9 / 41.4, 2 x 32768 49.1 / 48.1; 64 on 8, 24000 42.1 / 43.5
+//   rank 384: 24000 34.1 / 35.2, 32768 40.5 / 40.7, 48000 52.3 / 51.4; 16 on 4, 32768 29.7 / 31.2, 65536 41.6 / 41.0
+//   rank 256: 32768 32.6 / 34.0, 48000 41.4 / 40.8, 65536 51.8 / 47.5; 16 on 4, 65536 34.2 / 35.2, 131072 53.4 / 48.5
+//   two kv heads, one workgroup for both: nothing is left to share a row's way from memory with.  Rank 512, 262144 95.2 / 93.6, 393216 132 / 125; rank 384, 262144 78.8 / 76.4
+//   scores alone: rank 512, 16384 21.7 / 22.8, 24000 29.2 / 29.4, 48000 50.4 / 48.0, 16 on 2, 200000 61.5 / 61.7; rank 384, 64 on 8, 24000 24.6 / 25.6, 48000 41.9 / 41.4
 inline int64_t recon_heads_work(int rank, int hkv) {
-  if (hkv == 2) return 327680;
-  return rank == 512 ? 90112 : rank == 384 ? 131072 : 262144;
+  if (hkv == 2) return 458752;
+  return rank == 512 ? 229376 : rank == 384 ? 294912 : 344064;
 }
 
 // Workgroups from which on the dispatcher takes it, whoever chose the splits: the chip three quarters full
 constexpr int64_t RECON_HEADS_WORKGROUPS = 192;
+
+// Scores at ranks 256 and 384 of up to eight heads a kv head, by recon_scores_kernel or by one head a workgroup of the wave-specialised kernel, whose workgroups start
+// faster.  us a call, wave-specialised / recon_scores, 32 heads on 8 unless said: rank 256, 1000 tokens 6.5 / 8.7, 8192 9.6 / 10.8, 16384 14.0 / 13.9, 32768 23.0 / 21.3; 64 on 8,
+// 8192 10.1 / 11.5, 16384 15.5 / 15.1; 16 on 2, 16384 8.2 / 10.8, 65536 15.3 / 16.3; 12 on 3, 60000 18.8 / 17.3; 4 on 1, 60000 10.9 / 13.8.  Rank 384, 1000 7.0 / 9.1, 8192 11.7 /
+// 13.4, 32768 28.4 / 28.3; 12 on 3, 130001 43.8 / 47.7, 8 x 131072 322 / 328; 20 on 5, 4 x 30000 59.2 / 60.9; 8 on 2, 65536 19.3 / 19.5; 4 on 1, 120000 20.6 / 21.5, 262144 48.9 / 45.1
+inline bool recon_scores_pays(int rank, int hkv, int G, int64_t tokens) {
+  return rank == 256 ? G <= 8 && tokens * hkv >= 131072 : rank == 384 && hkv == 1 && G <= 4 && tokens >= 196608;
+}
 
 }  // namespace xkv

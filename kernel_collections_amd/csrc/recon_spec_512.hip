@@ -3,9 +3,8 @@
 
 namespace xkv {
 
-int launch_recon_spec_512(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                          hipStream_t st) {
-  return spec::launch_recon_spec_rank<512>(p, kB, sBb, sBh, sBr, batch, dtype, st);
+int launch_recon_spec_512(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st) {
+  return spec::launch_recon_spec_rank<512>(p, kB, batch, dtype, st);
 }
 
 }  // namespace xkv

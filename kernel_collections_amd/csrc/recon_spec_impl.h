@@ -7,7 +7,8 @@
 // over is scores, 4 KB a tile.  It also sends the tile loads, evenly spread.  (Split 2 x 2 over rank and feature halves, each operand read served two matrix
 // instructions, but 16 KB of partial keys went through the LDS and back, whose writes wait while load data arrives, and the consumers added and
 // rotated them: 521 us for 16 x 32768 tokens, 8 kv heads, rank 512, against 506; 1 x 1000 22.3 / 21.4 a call, 4096 25.5 / 24.1, 30000 on one kv head 28.3 / 26.7,
-// 130000 on three 75.5 / 72.3; rank 384, 2 x 50000 on three 51.7 / 46.8; rank 256, 64 heads on 8, 40000 47.3 / 40.2.)
+// 130000 on three 75.5 / 72.3; rank 384, 2 x 50000 on three 51.7 / 46.8; rank 256, 64 heads on 8, 40000 47.3 / 40.2.  Then without a launch in front that packed the factor:
+// 1 x 1000 19.9, 4096 22.1.)
 // Consumer waves (4..7; consumer c owns RK / 4 latent features of P.A) do the rest, each step one workgroup barrier behind the one before it:
 //   period p:  reconstruction   last k-steps of tile p-1, rotation + q-dot of tile p-1, first k-steps of tile p, loads of tile p+3 (ring of 4 slots)
 //              consumers        softmax + P.A of tile p-2 (scores summed from the four waves' parts; the softmax is computed by
@@ -20,6 +21,7 @@
 // each kv head moves for itself; where several kv heads can share them, recon_heads_impl.h takes the call.
 #pragma once
 #include "recon_fast_impl.h"
+#include "factor_rows.h"
 
 namespace xkv {
 namespace spec {
@@ -35,7 +37,7 @@ template <int RK> struct SpecShape {
   static constexpr int SP_FLOATS = 4 * 8 * FSP_ROW;   // one buffer of partial scores: [reconstruction wave 4][head 8][FSP_ROW]
   static constexpr int LATE = 4;               // k-steps of a tile that run after the barrier that ends its period
   static constexpr int EARLY = 1;              // operand reads are issued this many slots before the uniform one-per-slot rate
-  static constexpr size_t SHM = (size_t)SRING * FTILE + 2 * SP_FLOATS * 4 + 2 * 8 * 128 * 2 + 128 * 2;
+  static constexpr size_t SHM = (size_t)SRING * FTILE + 2 * SP_FLOATS * 4 + 2 * 8 * 128 * 2 + 128 * 2 + 8 * 4;
 };
 
 // The consumer's accumulation registers are managed by hand, by register number, in asm statements: a[0 .. RK/16) hold the P.A
@@ -70,7 +72,7 @@ template <int R> __device__ __forceinline__ float acc_get_at() {
 }
 // GP: head slots of a kv head rounded up to 4 or 8 (softmax lane layout).  SCORES: write the scaled scores only.
 template <typename T, bool SCORES, int RK, int GP>
-__global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p) {
+__global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p, const FactorOperand kB) {
   typedef typename Elem<T>::vec8 vec8;
   typedef SpecShape<RK> S;
   constexpr int FROW = S::FROW, FTILE = S::FTILE, NK = S::NK, NMB = S::NMB, SP_FLOATS = S::SP_FLOATS;
@@ -99,13 +101,23 @@ __global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p) {
   float* s_part = reinterpret_cast<float*>(smem + SRING * FTILE);          // [2][4 reconstruction waves][8 heads][FSP_ROW]
   sc_t* qhat = reinterpret_cast<sc_t*>(s_part + 2 * SP_FLOATS);            // [2][8 heads][128]
   sc_t* qzero = qhat + 2 * 8 * 128;                                        // [128] zeros: the q-dot operand of masked lanes
+  float* unscale = reinterpret_cast<float*>(qzero + 128);                  // [8]
   const unsigned ring_lds = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)ring;
-  if (tid < 128) qzero[tid] = from_f32<sc_t>(0.f);
+
+  // the factor, brought by all waves through the slot that no first tile is on its way to, and the scores behind it
+  typedef FactorRows<T, RK> Factor;
+  static_assert(FTILE + 2 * SP_FLOATS * 4 >= Factor::BYTES, "room for two chunks");
+  Factor factor;
+  const T* const Bh = reinterpret_cast<const T*>(kB.p) + b * kB.sb + kh * kB.sh;
+  T* const stage = reinterpret_cast<T*>(ring + (SRING - 1) * FTILE);
 
   if (wave < 4) {
     // =================================================================================================================
     // reconstruction wave
     // =================================================================================================================
+    float freq[8];         // of this lane's pairs 16 wave + 8 (r / 4) + 4 g2 + r % 4
+#pragma unroll
+    for (int r = 0; r < 8; ++r) freq[r] = p.inv_freq[16 * wave + 8 * (r >> 2) + 4 * g2 + (r & 3)];
     // ---- tile loads, straight to the LDS: rows 8 wave .. + 7 of a tile belong to this wave, one (RK * 2 bytes: lanes 0 .. RK/8 - 1) per
     // instruction.  Rows past the split's end are out of the resource's range and leave zeros; the softmax masks them.
     const int row_bytes = (int)p.sAl * 2;
@@ -129,16 +141,8 @@ __global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p) {
       next_tile();
       static_for<8>([&](auto r_c) { load_row(t_c, r_c); });
     });
-    // B operands go from memory straight into accumulation registers (no transit through the 128 ordinary registers the
-    // kernel may use): the loads are asm, and so is the wait for them.
-    vec8 breg[NK];
-    {
-      const T* bp = reinterpret_cast<const T*>(p.Bp) + b * p.sBpb + (int64_t)kh * (RK * 128) + (int64_t)wave * (64 * NK) * 8;
-#pragma unroll
-      for (int ks = 0; ks < NK; ++ks)
-        asm volatile("global_load_dwordx4 %0, %1, %2" : "=a"(breg[ks]) : "v"((unsigned)(lane * 16 + ks * 1024)), "s"(bp) : "memory");
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+    factor.template init<false>(Bh, kB.sr, tid);
+    if (tid < 128) qzero[tid] = from_f32<sc_t>(0.f);
     // in-tile rotation of this wave's 8 pairs per lane (token n32, g2): pair 16 wave + 8 (r / 4) + 4 g2 + r % 4, r = 0 .. 7.  Two tables: the
     // query-side base is that of an EVEN tile and serves the odd tile after it too, whose offsets are 32 .. 63.
     float ct[2][8], st[2][8];
@@ -146,7 +150,15 @@ __global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p) {
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int r = 0; r < 8; ++r)
-        __sincosf((float)(n32 + 32 * h) * p.inv_freq[16 * wave + 8 * (r >> 2) + 4 * g2 + (r & 3)], &st[h][r], &ct[h][r]);
+        __sincosf((float)(n32 + 32 * h) * freq[r], &st[h][r], &ct[h][r]);
+    vec8 breg[NK];
+    factor.pass(stage, tid, [&](int ch, const T* buf) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        breg[2 * ch + i] = Factor::operand(buf, 16 * i, wave, lane);
+        asm volatile("" : "+a"(breg[2 * ch + i]));
+      }
+    });
     // q-dot B operand: lanes whose token half (lane bit 4) matches their column's (lane bit 3) read q^ of head lane % 8 (absent heads: the
     // last one; their columns are not used), the others read zeros
     const bool q_live = ((lane >> 4) & 1) == ((lane >> 3) & 1);
@@ -159,7 +171,8 @@ __global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) ka[s][r] = 0.f;
     const unsigned char* fr0 = ring + n32 * FROW + 8 * g2 * 2;
-    __syncthreads();        // the consumers' prologue: tiles 0 and 1 and q^(0) are in the LDS
+    wait_vmcnt<0>();
+    __syncthreads();        // tiles 0 to 2 are in the LDS, and the consumers' q^(0)
 
     // Period pp: the last LATE k-steps of tile pp-1 (accumulator set (pp-1) % 2; their operands were read before the barrier,
     // so the matrix pipe has work while the first operands of tile pp travel from the LDS), then the first NK - LATE k-steps
@@ -269,6 +282,22 @@ __global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p) {
     }
   }
   const float qinv = p.inv_freq[lane];
+  factor.template init<false>(Bh, kB.sr, tid);
+  if constexpr (SCORES) {
+    // Multiplied by the power of two that brings the head's largest feature to 2^14 .. 2^15, and the scores by the inverse: fp16 then holds every
+    // rotated pair, and the parts of small queries are no subnormals there.  A feature that is no finite number leaves the others as they are.
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int bits = __builtin_bit_cast(int, row_reduce<true, 16>(fmaxf(fabsf(q0[i]), fabsf(q1[i]))));
+      const int top = max(max(__builtin_amdgcn_readlane(bits, 0), __builtin_amdgcn_readlane(bits, 16)),
+                          max(__builtin_amdgcn_readlane(bits, 32), __builtin_amdgcn_readlane(bits, 48)));
+      const int up = max(-1, min(14 + 127 - (top >> 23), 100));
+      const float f = __builtin_bit_cast(float, (127 + up) << 23);
+      q0[i] *= f;
+      q1[i] *= f;
+      if (lane == 0) unscale[c + 4 * i] = __builtin_bit_cast(float, (127 - up) << 23);
+    }
+  }
   // q^ is kept in q-dot operand order: pair j = 32 dq' + 8 o + 4 g' + e sits at [o][dq'][g'][e] (partner at e + 4), so that
   // a lane's 8 contraction values of chunk o are one 16-byte read
   const int qpos = ((((lane >> 3) & 3) * 2 + (lane >> 5)) * 2 + ((lane >> 2) & 1)) * 8 + (lane & 3);
@@ -289,6 +318,7 @@ __global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p) {
     qcb = cc; qsb = ss;
   };
   write_qhat(0);
+  factor.pass(stage, tid, [](int, const T*) {});
 
   // ---- softmax role: every consumer computes P of all heads; lane (n16, g4) holds head n16 % GP, tokens 8 g4 + TPL (n16 / GP) ..
   constexpr int TPL = GP / 2;   // tokens per lane
@@ -334,7 +364,7 @@ __global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p) {
     if (SCORES) {   // consumer c writes heads c and c + 4: lane -> (head c + 4 (lane / 32), token lane % 32)
       const int head = c + 4 * g2;
       const float* sp = s_part + TPAR * SP_FLOATS + (head < G ? head : G - 1) * FSP_ROW + n32;
-      const float s = ((sp[0] + sp[8 * FSP_ROW]) + (sp[2 * 8 * FSP_ROW] + sp[3 * 8 * FSP_ROW])) * p.sm_scale;
+      const float s = ((sp[0] + sp[8 * FSP_ROW]) + (sp[2 * 8 * FSP_ROW] + sp[3 * 8 * FSP_ROW])) * (p.sm_scale * unscale[head]);
       const int tok = start + t * FT + n32;
       if (head < G && tok < end) {
         const int64_t o = ((int64_t)b * p.hq + h0 + head) * p.kv_len + tok;
@@ -455,10 +485,8 @@ __global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p) {
 }
 
 template <typename T, int RK>
-int launch_recon_spec_t(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, hipStream_t st) {
+int launch_recon_spec_t(const FastParams& p, const FactorOperand& kB, int batch, hipStream_t st) {
   typedef SpecShape<RK> S;
-  const int nb = sBb == 0 ? 1 : batch;   // one packed copy when the factor is shared by the batch
-  pack_b_kernel<T, RK><<<dim3(p.hkv, nb, 32), dim3(256), 0, st>>>((const T*)kB, (T*)p.Bp, sBb, sBh, sBr, p.hkv);
   const bool gp4 = p.hq / p.hkv <= 4;
   auto kern = p.scores ? (gp4 ? recon_spec_kernel<T, true, RK, 4> : recon_spec_kernel<T, true, RK, 8>)
                        : (gp4 ? recon_spec_kernel<T, false, RK, 4> : recon_spec_kernel<T, false, RK, 8>);
@@ -466,15 +494,13 @@ int launch_recon_spec_t(const FastParams& p, const void* kB, int64_t sBb, int64_
   const int e = ensure_dynamic_lds(lds[(p.scores ? 2 : 0) + (gp4 ? 1 : 0)], reinterpret_cast<const void*>(kern), (int)S::SHM, true);
   if (e != XKV_OK) return e;
   const int total = batch * p.hkv * p.max_splits;
-  kern<<<dim3(xcd_grid(total, p.hkv)), dim3(512), S::SHM, st>>>(p);
+  kern<<<dim3(xcd_grid(total, p.hkv)), dim3(512), S::SHM, st>>>(p, kB);
   return launch_status();
 }
 
 template <int RK>
-int launch_recon_spec_rank(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype,
-                           hipStream_t st) {
-  return dtype == XKV_BF16 ? launch_recon_spec_t<__bf16, RK>(p, kB, sBb, sBh, sBr, batch, st)
-                           : launch_recon_spec_t<_Float16, RK>(p, kB, sBb, sBh, sBr, batch, st);
+int launch_recon_spec_rank(const FastParams& p, const FactorOperand& kB, int batch, int dtype, hipStream_t st) {
+  return dtype == XKV_BF16 ? launch_recon_spec_t<__bf16, RK>(p, kB, batch, st) : launch_recon_spec_t<_Float16, RK>(p, kB, batch, st);
 }
 
 }  // namespace spec

@@ -338,7 +338,6 @@ static int launch_recon(const ReconParams& p, int batch, hipStream_t st) {
   return launch_status();
 }
 
-constexpr int64_t COPIED_FACTOR_WORK = 65536;   // tokens x kv heads, as in host.cpp
 // kB [batch, hkv, rank, 128] of any strides but the last -> whole packets side by side
 __global__ __launch_bounds__(256) void copy_factor_kernel(const u16* __restrict__ kB, u16* __restrict__ out, int64_t sBb, int64_t sBh, int64_t sBr, int rank) {
   typedef u16 u16x8 __attribute__((ext_vector_type(8)));
@@ -349,6 +348,20 @@ __global__ __launch_bounds__(256) void copy_factor_kernel(const u16* __restrict_
 #pragma unroll
   for (int e = 0; e < 8; ++e) v[e] = src[e];
   st16(out + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * rank * 128 + row * 128 + c, v);
+}
+
+static void copy_factor(const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int hkv, int rank, void* out, hipStream_t st) {
+  copy_factor_kernel<<<dim3(hkv, sBb == 0 ? 1 : batch, cdiv(rank * 16, 256)), dim3(256), 0, st>>>((const u16*)kB, (u16*)out, sBb, sBh, sBr, rank);
+}
+static bool whole_packets(const void* kB, int64_t sBb, int64_t sBh, int64_t sBr) {
+  return ((sBb | sBh | sBr) & 7) == 0 && (reinterpret_cast<uintptr_t>(kB) & 15) == 0;
+}
+// The factor as the kernels that hold it in registers read it: as it is, or a copy in the workspace (one of all sequences where they share it)
+static FactorOperand packets(const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int hkv, int rank, void* workspace, hipStream_t st) {
+  if (whole_packets(kB, sBb, sBh, sBr)) return {kB, sBb, sBh, sBr};
+  copy_factor(kB, sBb, sBh, sBr, batch, hkv, rank, workspace, st);
+  const int64_t head = (int64_t)rank * 128;
+  return {workspace, sBb == 0 ? 0 : hkv * head, head, 128};
 }
 
 template <typename T>
@@ -421,7 +434,7 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
   // Several kv heads per workgroup, where the splits make enough of them: a factor of 16-byte packets, and whatever else the wave-specialised kernel asks for
   const int nh = rope && !sin_cos ? recon_heads(rank, hkv, hq / hkv, so) : 0;
   if (nh && (so || vshared) && spec && (int64_t)batch * (hkv / nh) * max_splits >= RECON_HEADS_WORKGROUPS &&
-      ((sBb | sBh | sBr) & 7) == 0 && (reinterpret_cast<uintptr_t>(kB) & 15) == 0) {
+      whole_packets(kB, sBb, sBh, sBr)) {
     FastParams f{};
     f.q = q_pe; f.kA = kA.ptr; f.sAb = kA.stride_b; f.sAl = kA.stride_l;
     f.partial = partial; f.lse = lse; f.scores = scores_out; f.scores_dtype = scores_dtype;
@@ -437,56 +450,49 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
     f.num_splits = num_kv_splits; f.kv_lens = kv_lens;
     f.hq = hq; f.hkv = hkv; f.kv_len = kv_len; f.max_splits = max_splits; f.total_wg = batch * hkv * max_splits;
     f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
-    // Scores-only shapes (us a call, this kernel / the one it replaces, 32 heads on 8 kv heads: rank 128, 5 x 7488 tokens 17.9 / 21.6; rank
-    // 192, 7 x 39246 124 / 153; rank 224, 131072 64.5 / 241; rank 256, 2 x 28611 30.9 / 41.8; rank 320, 131072 99.8 / 269; rank 384, 5 x 2903 19.8 / 21.4, 2 x
-    // 81976 135 / 146; rank 448, 131072 127 / 313).  At ranks 256 and 384 its rotated query is one fp16 value, so only where the caller's workspace asks for kernels that have
-    // that.  At rank 384 not beyond four heads per kv head: two waves' halves of the q-dot cost more there than the wave-specialised kernel's pack launch
-    // (32 on 8, 2100 10.5 / 10.6, 8 x 200001 1320 / 1342; 48 on 8, 3 x 130001 344 / 342; 64 on 8, 2500 11.3 / 10.8; 16 on 2, 9000 11.6 / 10.2)
-    const bool here = rank == 256 ? spec : rank == 384 ? spec && hq / hkv <= 4 : true;
-    if (here && recon_scores_serves(f, kB, sBb, sBh, sBr, rank))
-      return launch_recon_scores(f, kB, sBb, sBh, sBr, batch, dtype, rank, st);
-    // A factor that is not 16-byte packets: at rank 256 a copy that is, in the workspace, once the call is long enough to pay for it.  us a call, the
-    // wave-specialised kernel (which packs any factor) / copy and this one, 32 heads on 8: 4096 tokens 11.6 / 11.8, 8192 13.7 / 13.0, 2 x 28611 52.4 / 37.7, 131072
-    // 95.9 / 71.3; 16 on 2, 16000 11.2 / 12.1, 32000 13.8 / 14.1; 8 on 1, 60000 13.6 / 16.9.  At rank 384 it gains 4 % of the longest and loses 1 us of the others
-    const int64_t head = (int64_t)rank * 128, copy_b = sBb == 0 ? 0 : hkv * head;
-    if (rank == 256 && spec && hkv >= 2 && (int64_t)batch * kv_len * hkv >= COPIED_FACTOR_WORK && recon_scores_serves(f, workspace, copy_b, head, 128, rank)) {
-      copy_factor_kernel<<<dim3(hkv, sBb == 0 ? 1 : batch, cdiv(rank * 16, 256)), dim3(256), 0, st>>>((const u16*)kB, (u16*)workspace, sBb, sBh, sBr, rank);
-      return launch_recon_scores(f, workspace, copy_b, head, 128, batch, dtype, rank, st);
+    // Scores-only shapes (us a call, this kernel / the generic one, 32 heads on 8 kv heads: rank 128, 5 x 7488 tokens 17.9 / 21.6; rank
+    // 192, 7 x 39246 124 / 153; rank 224, 131072 64.5 / 241; rank 320, 131072 99.8 / 269; rank 448, 131072 127 / 313).  At ranks 256 and 384 its rotated query is one fp16
+    // value, so only where the caller's workspace asks for kernels that have that; a factor that is not 16-byte packets is copied there.
+    const bool two = rank == 256 || rank == 384;
+    if (!two || (spec && recon_scores_pays(rank, hkv, hq / hkv, (int64_t)batch * kv_len))) {
+      const int64_t head = (int64_t)rank * 128;
+      const bool copy = two && !whole_packets(kB, sBb, sBh, sBr);
+      const FactorOperand rows = copy ? FactorOperand{workspace, sBb == 0 ? 0 : hkv * head, head, 128} : FactorOperand{kB, sBb, sBh, sBr};
+      if (recon_scores_serves(f, rows.p, rows.sb, rows.sh, rows.sr, rank)) {
+        if (copy) copy_factor(kB, sBb, sBh, sBr, batch, hkv, rank, workspace, st);
+        return launch_recon_scores(f, rows.p, rows.sb, rows.sh, rows.sr, batch, dtype, rank, st);
+      }
     }
   }
-  // The wave-specialised kernel: rank 512 / 384 / 256, a basis shared by K and V (or scores that stay with it, or of a factor that is not 16-byte packets), computed
-  // RoPE angles, at most 8 query heads per kv head
+  // The wave-specialised kernel: rank 512 / 384 / 256, a basis shared by K and V or scores alone, computed RoPE angles, at most 8 query heads per kv head
   if ((so || vshared) && spec) {
-    FastParams f;
-    f.q = q_pe; f.kA = kA.ptr; f.Bp = workspace;
-    f.sAb = kA.stride_b; f.sAl = kA.stride_l; f.sBpb = sBb == 0 ? 0 : (int64_t)hkv * rank * 128;
+    FastParams f{};
+    f.q = q_pe; f.kA = kA.ptr; f.sAb = kA.stride_b; f.sAl = kA.stride_l;
     f.partial = partial; f.lse = lse; f.scores = scores_out; f.scores_dtype = scores_dtype;
     f.num_splits = num_kv_splits; f.kv_lens = kv_lens;
     f.hq = hq; f.hkv = hkv; f.kv_len = kv_len; f.max_splits = max_splits; f.total_wg = batch * hkv * max_splits;
     f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
-    return launch_recon_spec(f, kB, sBb, sBh, sBr, batch, dtype, rank, st);
+    return launch_recon_spec(f, packets(kB, sBb, sBh, sBr, batch, hkv, rank, workspace, st), batch, dtype, rank, st);
   }
   // 8-wave kernels: a value basis of its own beside key ranks 256 / 384 / 512
-  if (!so && !vshared && rope && !sin_cos && hq / hkv <= 8 && workspace && need > 0 && workspace_bytes >= need &&
+  if (!so && !vshared && recon_duo_serves(rank, vA.dim) && rope && !sin_cos && hq / hkv <= 8 && workspace && need > 0 && workspace_bytes >= need &&
       (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && (int64_t)kA.stride_l * 2 * 3 < ((int64_t)1 << 31) &&
       (int64_t)vA.stride_l * 2 * 3 < ((int64_t)1 << 31)) {
-    FastParams f;
-    f.q = q_pe; f.kA = kA.ptr; f.Bp = workspace;
-    f.sAb = kA.stride_b; f.sAl = kA.stride_l; f.sBpb = sBb == 0 ? 0 : (int64_t)hkv * rank * 128;
+    FastParams f{};
+    f.q = q_pe; f.kA = kA.ptr; f.sAb = kA.stride_b; f.sAl = kA.stride_l;
     f.partial = partial; f.lse = lse; f.scores = nullptr; f.scores_dtype = scores_dtype;
     f.num_splits = num_kv_splits; f.kv_lens = kv_lens;
     f.hq = hq; f.hkv = hkv; f.kv_len = kv_len; f.max_splits = max_splits; f.total_wg = batch * hkv * max_splits;
     f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
     f.vA = vA.ptr; f.sVb = vA.stride_b; f.sVl = vA.stride_l;
-    int rc = launch_recon_duo_b(f, kB, sBb, sBh, sBr, batch, dtype, rank, vA.dim, st);
-    if (rc == DUO_NOT_MINE) rc = launch_recon_duo_c(f, kB, sBb, sBh, sBr, batch, dtype, rank, vA.dim, st);
-    if (rc != DUO_NOT_MINE) return rc;
+    const FactorOperand rows = packets(kB, sBb, sBh, sBr, batch, hkv, rank, workspace, st);
+    return rank == 256 ? launch_recon_duo_c(f, rows, batch, dtype, rank, vA.dim, st) : launch_recon_duo_b(f, rows, batch, dtype, rank, vA.dim, st);
   }
   return dtype == XKV_BF16 ? dispatch_recon<__bf16>(p, batch, vshared, st) : dispatch_recon<_Float16>(p, batch, vshared, st);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
-// The same stage 1 for callers that cannot allocate: the packed copy of kB lives in a file-scope device array instead of
+// The same stage 1 for callers that cannot allocate: the copy of kB (where it is not 16-byte packets) lives in a file-scope device array instead of
 // a caller workspace.  Every GPU holds its own copy of the array at its own address; the address is looked up once per
 // device (first call with that device current) and kept.  The array's NAME is only a host-side handle for that lookup:
 // kernels and copies always get the looked-up pointer.

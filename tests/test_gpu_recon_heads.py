@@ -97,7 +97,7 @@ def test_scores_of_large_and_small_queries(dev, scale):
 def test_splits_fill_the_device_once(dev, shim):
     """A call past the line is cut for workgroups of several heads, a short one and one of a single kv head for one each."""
     import kernel_collections_amd.flash_recontruction as fr
-    for hkv, L, r, groups in ((8, 12000, 512, 4), (8, 11000, 512, 8), (4, 32768, 384, 2), (4, 32700, 384, 4), (8, 32768, 256, 2), (8, 32000, 256, 8), (2, 163840, 512, 1), (2, 163800, 512, 2),
+    for hkv, L, r, groups in ((8, 28672, 512, 4), (8, 28600, 512, 8), (4, 73728, 384, 2), (4, 73700, 384, 4), (8, 43008, 256, 2), (8, 43000, 256, 8), (2, 229376, 512, 1), (2, 229300, 512, 2),
                               (1, 200000, 512, 1)):
         q, A, B = operands(dev, BF, 1, hkv, 4, L, r, r)
         fr.gqa_xKV_rope(q, A, B, A, B, torch.empty_like(q), torch.ones(1, dtype=torch.int32, device=dev), 1, 0.1, 5e5)
