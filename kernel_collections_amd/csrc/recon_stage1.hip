@@ -474,10 +474,10 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
     f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
     return launch_recon_spec(f, packets(kB, sBb, sBh, sBr, batch, hkv, rank, workspace, st), batch, dtype, rank, st);
   }
-  // 8-wave kernels: a value basis of its own beside key ranks 256 / 384 / 512
+  // 8-wave kernels: a value basis of its own beside key ranks 256 / 384 / 512.  Rows that overlap (expanded ones too) would make their unsigned lane offsets negative
   if (!so && !vshared && recon_duo_serves(rank, vA.dim) && rope && !sin_cos && hq / hkv <= 8 && workspace && need > 0 && workspace_bytes >= need &&
-      (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && (int64_t)kA.stride_l * 2 * 3 < ((int64_t)1 << 31) &&
-      (int64_t)vA.stride_l * 2 * 3 < ((int64_t)1 << 31)) {
+      (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && kA.stride_l >= rank && (int64_t)kA.stride_l * 2 * 3 < ((int64_t)1 << 31) &&
+      vA.stride_l >= vA.dim && (int64_t)vA.stride_l * 2 * 3 < ((int64_t)1 << 31)) {
     FastParams f{};
     f.q = q_pe; f.kA = kA.ptr; f.sAb = kA.stride_b; f.sAl = kA.stride_l;
     f.partial = partial; f.lse = lse; f.scores = nullptr; f.scores_dtype = scores_dtype;
