@@ -26,6 +26,7 @@
 
 #include "../../include/xkv_hip.h"
 #include "head_rows.h"
+#include "merge_rule.h"
 #include "recon_groups.h"
 
 namespace {
@@ -207,12 +208,8 @@ void write_plan(const Call& c, Splits& s, const Ragged& r, int64_t batch) {
 }
 
 // ---- merge (with or without the up-projection by vB [b, hkv, dv, d_out]) ------------------------------------------------
-// Partial values a workgroup of the up-projecting merge may fold; beyond, the rows are merged first.  us of one kernel / of rows and
-// up-projection, batches of 1 .. 32 of 16 .. 64 heads, dv 256 and 512: at 32768 5.0 - 14.4 / 7.8 - 17.7, one kernel ahead everywhere; at
-// 49152 even in the narrowest case (batch 4, 48 splits of 256: 8.6 / 8.6); at 65536 behind there (10.6 / 9.9).
-constexpr int64_t MERGE_ROWS_FLOATS = 49152;
 struct Up { const void* p; int64_t sb, sh, sr; int d_out, dtype, hkv; };
-bool rows_first(int S, int64_t hq, int hkv, int64_t dv) { return S > 1 && S * (hq / hkv) * dv > MERGE_ROWS_FLOATS; }
+bool rows_first(int S, int64_t hq, const Up& up, int64_t dv, int64_t batch) { return xkv::merge_rows_first(S, hq, up.hkv, dv, batch, up.d_out); }
 int64_t rows_bytes(int64_t batch, int64_t hq, int64_t dv) { return batch * hq * (dv + 1) * 4; }
 
 void merge(const Call& c, const float* partial, const float* lse, void* out, int64_t sOb, int64_t sOh, int out_dtype, const Up* up,
@@ -223,7 +220,7 @@ void merge(const Call& c, const float* partial, const float* lse, void* out, int
                              s.plan, dv, sOb, sOh, out_dtype, lse_out, sLb, sLh, c.stream), "xkv_merge_stage2");
     return;
   }
-  if (rows_first(s.S, hq, up->hkv, dv)) {   // many splits: merge the rows first, spread over the chip, then one row per head
+  if (rows_first(s.S, hq, *up, dv, batch)) {   // many splits: merge the rows first, spread over the chip, then one row per head
     float* mid = c.get<float>(rows_at);
     float* mid_lse = lse_out ? lse_out : mid + batch * hq * dv;
     if (!lse_out) { sLb = hq; sLh = 1; }
@@ -331,7 +328,7 @@ PyObject* nope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       else s.S = scan_splits(c, b, groups, L, ring_scan(r, rv));
       if (lens.defined()) s.lens = lens.data_ptr<int32_t>();
       const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
-      const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
+      const int64_t mid = c.plan(rows_first(s.S, hq, up, rv, b) ? rows_bytes(b, hq, rv) : 0);
       c.alloc();
       if (planned) write_plan(c, s, rg, b);
       absorb(c, q.data_ptr(), kB, c.get<void>(hi), c.get<void>(lo), b, hq, d, r);
@@ -447,7 +444,7 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         }
         s.S = scan_splits(c, b, head_groups(hq), L, true);
         const int64_t sc = c.plan(b * hq * row * 4), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
-        const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
+        const int64_t mid = c.plan(rows_first(s.S, hq, up, rv, b) ? rows_bytes(b, hq, rv) : 0);
         if (c.try_alloc()) {
           recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, score_splits(c, kB, b, hkv, hq / hkv, L, r), b, hq, hkv, row,
                 scale, invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes, s.lens);
@@ -461,7 +458,7 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       }
       s.S = S_heads ? S_heads : decode_splits(b, hkv, L, r, shared, c.cus);
       const int64_t part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
-      const int64_t mid = c.plan(rows_first(s.S, hq, up.hkv, rv) ? rows_bytes(b, hq, rv) : 0);
+      const int64_t mid = c.plan(rows_first(s.S, hq, up, rv, b) ? rows_bytes(b, hq, rv) : 0);
       c.alloc();
       recon(c, q, kA, kB, &vA, c.get<float>(part), c.get<float>(lse), nullptr, 0, s.S, b, hq, hkv, L, scale, invp, pos,
             ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
@@ -539,7 +536,7 @@ PyObject* gqa(PyObject*, PyObject* const* a, Py_ssize_t n) {
       else s.S = std::min(balanced_splits(b, groups, L, 32, per_cu, c.cus), cdiv(L, floor));
       if (lens.defined()) s.lens = lens.data_ptr<int32_t>();
       const int64_t part = c.plan(s.rows(b, hq) * dv * 4), lse = c.plan(s.rows(b, hq) * 4), bd = c.plan(wide4 ? b * hq * 512 * 2 : 0);
-      const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, dv) ? rows_bytes(b, hq, dv) : 0);
+      const int64_t mid = c.plan(fact && rows_first(s.S, hq, up, dv, b) ? rows_bytes(b, hq, dv) : 0);
       c.alloc();
       if (planned) write_plan(c, s, rg, b);
       const void* qp = q.data_ptr();
@@ -583,7 +580,7 @@ PyObject* mla(PyObject*, PyObject* const* a, Py_ssize_t n) {
       Splits s{scan_splits(c, b, groups, L, e == 64 && (r == 512 || (fact && ring_rank(r)))), 0, nullptr, nullptr};
       const int64_t hi = c.plan(fact ? b * hq * r * 2 : 0), lo = c.plan(fact ? b * hq * r * 2 : 0);
       const int64_t part = c.plan(s.rows(b, hq) * r * 4), lse = c.plan(s.rows(b, hq) * 4);
-      const int64_t mid = c.plan(fact && rows_first(s.S, hq, up.hkv, r) ? rows_bytes(b, hq, r) : 0);
+      const int64_t mid = c.plan(fact && rows_first(s.S, hq, up, r, b) ? rows_bytes(b, hq, r) : 0);
       c.alloc();
       o = at::empty({b, hq, w}, c.opts);
       const void *q_hi = qn.data_ptr(), *q_lo = nullptr;
@@ -626,7 +623,7 @@ PyObject* prefix_tail(PyObject*, PyObject* const* a, Py_ssize_t n) {
       // them live; a cap states the count, because the rows are one more: row 0 is the merged, up-projected prefix with its log-sum-exp
       const bool join = joined();
       const int blocks = cdiv(Lt, 32), per = cdiv(blocks, join ? 32 : 4), S2 = cdiv(blocks, per), rows2 = S2 + (join ? 0 : 1);
-      const bool first = rows_first(s1.S, hq, up.hkv, rv);
+      const bool first = xkv::merge_tail_rows_first(s1.S, hq, up.hkv, rv);
       const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part1 = c.plan(b * hq * s1.S * rv * 4), lse1 = c.plan(b * hq * s1.S * 4);
       const int64_t mid = c.plan(first ? rows_bytes(b, hq, rv) : 0), part2 = c.plan(b * hq * rows2 * dv * 4), lse2 = c.plan(b * hq * rows2 * 4);
       c.alloc();

@@ -1,0 +1,41 @@
+// Forms of the up-projecting merge (merge_up_kernel in small_kernels.hip), for its dispatcher and for the host layers that may merge the rows in a launch of their own first.
+#pragma once
+#include <cstdint>
+
+namespace xkv {
+
+constexpr int MERGE_CB = 64;       // columns per workgroup: whole 128-byte lines of a vB row
+
+inline int64_t merge_blocks(int64_t heads, int64_t batch, int d_out) { return heads * batch * ((d_out + MERGE_CB - 1) / MERGE_CB); }
+
+// Heads of a workgroup that folds a packet's splits in one thread: those of a kv head (vB is read once for them) as far as their merged rows fit 48 KiB of LDS
+inline int merge_heads(int64_t hq, int hkv, int64_t dv, int64_t batch, int d_out) {
+  const int g = (int)(hq / hkv);
+  int hpw = g;
+  while (hpw > 1 && (g % hpw != 0 || hpw * dv * 4 > 48 * 1024)) --hpw;
+  while (hpw > 4 && hpw % 2 == 0 && merge_blocks(hq / hpw, batch, d_out) < 256) hpw /= 2;
+  return hpw;
+}
+
+// One head a workgroup, its splits dealt out among groups of threads, where that is not more than a workgroup per CU (each reads its head's part of vB again) and a head
+// has splits to deal out.  us, a graph of merges, 32 heads on 8 kv heads, d_out 128 unless said: a thread all splits / dealt out.  Batch 1, values of 256: 8 splits 4.5 / 4.9, 16 5.1 /
+// 4.9, 32 6.3 / 4.9, 64 8.7 / 5.2; of 512: 8 6.1 / 5.8, 32 7.9 / 6.5, 128 18.1 / 9.5; 64 heads, 32 of 512 7.9 / 7.0; batch 4, 16 of 512 7.5 / 6.6; batch 8, 16 of 512 7.9 / 9.3; 16 on
+// 1, d_out 512, batch 8, 32 of 256 7.0 / 9.3
+inline bool merge_spread(int64_t splits, int64_t hq, int64_t batch, int64_t dv, int d_out) {
+  return splits > 1 && splits * dv >= 4096 && merge_blocks(hq, batch, d_out) <= 256;
+}
+
+// Partial values that a workgroup may fold in every column block, one head of it (SPREAD) or all; beyond, the rows are merged first, by the whole chip.  us of one kernel
+// / rows and up-projection: dealt out, batch 1, 128 splits of 512 9.5 / 11.3, 256 of 384 11.7 / 12.1, 256 of 512 13.2 / 13.0 (16 on 1, d_out 512 13.2 / 12.1); a thread all splits, batch
+// 8, 32 of 512 (65536 values) 9.6 / 11.9, 16 on 1, d_out 512, batch 8, 32 of 256 (32768) 7.0 / 7.7, batch 16, 16 of 256 (32768) 7.2 / 9.1
+constexpr int64_t MERGE_SPREAD_FLOATS = 98304, MERGE_FLOATS = 65536;
+inline bool merge_rows_first(int64_t splits, int64_t hq, int hkv, int64_t dv, int64_t batch, int d_out) {
+  if (merge_spread(splits, hq, batch, dv, d_out)) return splits * dv > MERGE_SPREAD_FLOATS;
+  return splits > 1 && splits * merge_heads(hq, hkv, dv, batch, d_out) * dv > MERGE_FLOATS;
+}
+
+// The same with a tail's rows beside them (xkv_merge_stage2_tail), which one workgroup folds for all heads of a kv head
+constexpr int64_t MERGE_TAIL_FLOATS = 49152;
+inline bool merge_tail_rows_first(int64_t splits, int64_t hq, int hkv, int64_t dv) { return splits > 1 && splits * (hq / hkv) * dv > MERGE_TAIL_FLOATS; }
+
+}  // namespace xkv

@@ -3,6 +3,7 @@
 #include <type_traits>
 
 #include "xkv_common.h"
+#include "merge_rule.h"
 
 namespace xkv {
 
@@ -425,11 +426,10 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(
 // 20 - 21.7); 8 splits of 256, 4.7 us (7.0); 16 x 32 heads, 2 splits of 512, 8.6 us (11.6).
 //
 // MANY_LOOP: many splits on a chip that the heads fill (launch_merge): a workgroup folds once for several column blocks.  MANY_SPREAD: on
-// one that is not full: one head per workgroup, its splits dealt out among groups of threads as in merge_rows_kernel.  256 splits of 512, 32 heads, d_out 128: 12.6 us (26.4 with a thread folding all splits of its packet).
-constexpr int MERGE_CB = 64;       // columns per workgroup: whole 128-byte lines of a vB row
+// one that is not full: one head per workgroup, its splits dealt out among groups of threads as in merge_rows_kernel, the product for that head alone (with three
+// absent heads multiplied beside it 0.6 - 0.9 us more).  32 splits of 256, 32 heads, d_out 128: 4.9 us (6.3 with a thread folding all splits of its packet), 128 of 512 9.5 (18.1).
 constexpr int MERGE_UP_T = 512;
 enum { MANY_LOOP = 1, MANY_SPREAD = 2 };
-constexpr int MERGE_ROWS_FLOATS = 49152;   // partial values a workgroup folds in every column block at most; measured in host.cpp
 //
 // TAIL: the up-projected row is merged with rows that are in output space already (the plain tail beside a factorised prefix), by their
 // log-sum-exps.  Their packets are folded while the merged rows are; a kernel of its own for it was 4 - 5 us more.
@@ -443,7 +443,8 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     float* __restrict__ lse_out, int64_t sLb, int64_t sLh, int split_cap, const int32_t* __restrict__ split_plan, const MergeTail tail) {
   typedef typename Elem<TB>::vec8 vec8;
   extern __shared__ float merged[];               // [hpw][dv]; MANY_SPREAD: then a packet, a maximum and a sum of every thread
-  __shared__ float tot[4][4 * MERGE_CB];          // [quarter of the row groups][4 heads x 64 columns]
+  constexpr int HP = MANY == MANY_SPREAD ? 1 : 4; // heads of a pass
+  __shared__ float tot[4][HP * MERGE_CB];         // [quarter of the row groups][heads x 64 columns]
   const int hfirst = blockIdx.x * hpw, kh = hfirst / (hq / hkv), b = blockIdx.y;
   int c0 = blockIdx.z * MERGE_CB;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -531,15 +532,15 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
   }
   __syncthreads();
   for (;;) {                                      // this workgroup's column blocks
-    for (int g0 = 0; g0 < hpw; g0 += 4) {
-      float acc[32];                                // [4 heads][8 columns]
+    for (int g0 = 0; g0 < hpw; g0 += HP) {
+      float acc[8 * HP];                            // [heads][8 columns]
 #pragma unroll
-      for (int i = 0; i < 32; ++i) acc[i] = 0.f;
+      for (int i = 0; i < 8 * HP; ++i) acc[i] = 0.f;
 #pragma unroll
       for (int r = 0; r < RPT; ++r) {
         const int rho = grp + 64 * r;
 #pragma unroll
-        for (int gi = 0; gi < 4; ++gi) {
+        for (int gi = 0; gi < HP; ++gi) {
           const float m = g0 + gi < hpw && rho < dv ? merged[(g0 + gi) * dv + rho] : 0.f;
 #pragma unroll
           for (int e = 0; e < 8; ++e) acc[gi * 8 + e] += m * to_f32(w[r][e]);
@@ -555,16 +556,21 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
         acc[i] = keep + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give), CTRL, 0xf, 0xf, false)); \
       }                                                                                                                       \
       }
-      XKV_HALVE(16, 8, 0x140)   // row_mirror
-      XKV_HALVE(8, 4, 0x141)    // row_half_mirror
-      XKV_HALVE(4, 2, 0x1B)     // quad_perm [3,2,1,0]
-      XKV_HALVE(2, 1, 0xB1)     // quad_perm [1,0,3,2]
-#undef XKV_HALVE
-      const int idx = (lane & 8 ? 16 : 0) + (lane & 4 ? 8 : 0) + (lane & 2 ? 4 : 0) + (lane & 1 ? 2 : 0);   // this lane's two sums
+      XKV_HALVE(4 * HP, 8, 0x140)   // row_mirror
+      XKV_HALVE(2 * HP, 4, 0x141)   // row_half_mirror
+      XKV_HALVE(HP, 2, 0x1B)        // quad_perm [3,2,1,0]
+      const int idx = (lane & 8 ? 4 * HP : 0) + (lane & 4 ? 2 * HP : 0) + (lane & 2 ? HP : 0) + (lane & 1 ? HP / 2 : 0);   // this lane's sums
+      if constexpr (HP == 4) {
+        XKV_HALVE(2, 1, 0xB1)       // quad_perm [1,0,3,2]
 #pragma unroll
-      for (int i = 0; i < 2; ++i) tot[wave >> 1][((idx + i) >> 3) * MERGE_CB + cb * 8 + ((idx + i) & 7)] = acc[i];
+        for (int i = 0; i < 2; ++i) tot[wave >> 1][((idx + i) >> 3) * MERGE_CB + cb * 8 + ((idx + i) & 7)] = acc[i];
+      } else {
+        const float sum = acc[0] + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, acc[0]), 0xB1, 0xf, 0xf, false));
+        if (!(lane & 1)) tot[wave >> 1][cb * 8 + idx] = sum;
+      }
+#undef XKV_HALVE
       __syncthreads();
-      if (tid < 4 * MERGE_CB) {
+      if (tid < HP * MERGE_CB) {
         const int gi = tid / MERGE_CB, c = c0 + tid % MERGE_CB;
         if (g0 + gi < hpw && c < d_out) {
           float v = tot[0][tid] + tot[1][tid] + tot[2][tid] + tot[3][tid];
@@ -620,19 +626,15 @@ static int launch_merge(const float* partial, const float* lse, void* out, const
                                                           lse_out, sLb, sLh, split_cap, split_plan);
     return launch_status();
   }
-  // one workgroup for all heads of a kv head (vB is read once for them) as far as their merged rows fit 48 KiB of LDS
-  const int g = hq / hkv;
-  int hpw = g;
-  while (hpw > 1 && (g % hpw != 0 || (size_t)hpw * dv * sizeof(float) > 48 * 1024)) --hpw;
-  while (hpw > 4 && hpw % 2 == 0 && (int64_t)(hq / hpw) * batch * cdiv(d_out, MERGE_CB) < 256) hpw /= 2;
   // Many splits (a caller with scratch to spare merges the rows first, as the wrappers do): where the heads fill the chip a workgroup
   // folds once for several column blocks; where they do not even with a workgroup per block, a workgroup takes one head and deals
-  // its splits out among groups of threads.
+  // its splits out among groups of threads, as it does wherever that is the faster (merge_rule.h).
+  int hpw = merge_heads(hq, hkv, dv, batch, d_out);
   int z = cdiv(d_out, MERGE_CB);
-  const bool many = seq_splits > 1 && (int64_t)seq_splits * g * dv > MERGE_ROWS_FLOATS;
-  const bool spread = many && (int64_t)(hq / hpw) * batch * z < 256;
+  const bool many = tail.splits ? merge_tail_rows_first(seq_splits, hq, hkv, dv) : seq_splits > 1 && (int64_t)seq_splits * hpw * dv > MERGE_FLOATS;
+  const bool spread = !tail.splits && (merge_spread(seq_splits, hq, batch, dv, d_out) || (many && (int64_t)(hq / hpw) * batch * z < 256));
   if (spread) hpw = 1;
-  if (many) z = (int)std::min<int64_t>(z, cdiv(256, std::min<int64_t>(256, (int64_t)(hq / hpw) * batch)));
+  if (many || spread) z = (int)std::min<int64_t>(z, cdiv(256, std::min<int64_t>(256, (int64_t)(hq / hpw) * batch)));
   const dim3 grid(hq / hpw, batch, z);
   const size_t shm = ((size_t)hpw * dv + (spread ? MERGE_UP_T * 6 : 0) + (tail.splits ? hpw * (MERGE_CB + 3) : 0)) * sizeof(float);
 #define XKV_MERGE_UP_TAIL(RPT, MANY, TAIL)                                                                                           \

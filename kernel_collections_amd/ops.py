@@ -216,7 +216,19 @@ def recon_stage1(q3, kA, kB, vA, partial, lse, scores, num_kv_splits, kv_lens, b
         "xkv_recon_stage1")
 
 
-MERGE_ROWS_FLOATS = 49152   # partial values a workgroup of the up-projecting merge may fold (measured beside the same constant of csrc/host.cpp)
+def _merge_rows_first(splits, batch, hq, hkv, dv, d_out):
+    """merge_rows_first of csrc/merge_rule.h, where its lines were measured: more splits than a workgroup should fold in every column block."""
+    if splits <= 1:
+        return False
+    blocks = -(-d_out // 64)
+    if splits * dv >= 4096 and hq * batch * blocks <= 256:      # one head a workgroup
+        return splits * dv > 98304
+    hpw = g = hq // hkv
+    while hpw > 1 and (g % hpw or hpw * dv * 4 > 48 * 1024):
+        hpw -= 1
+    while hpw > 4 and hpw % 2 == 0 and hq // hpw * batch * blocks < 256:
+        hpw //= 2
+    return splits * hpw * dv > 65536
 
 
 def merge_stage2(partial, lse, out, vB, num_kv_splits, kv_lens, batch, hq, hkv, kv_len, max_splits, lse_out=None, split_cap=0,
@@ -225,10 +237,8 @@ def merge_stage2(partial, lse, out, vB, num_kv_splits, kv_lens, batch, hq, hkv, 
     of the merged range.  Up-projections wider than 512 columns run as column blocks of 512."""
     dv = partial.shape[-1]
     seq_splits = max_splits if split_plan is None or num_kv_splits is not None else _cdiv(kv_len, split_cap)
-    if vB is not None and seq_splits > 1 and seq_splits * (hq // hkv) * dv > MERGE_ROWS_FLOATS:
-        # many splits: merge the rows first, spread over the chip, then up-project one row per head.  The up-projecting kernel
-        # repeats the merge in every block of 64 columns, which costs more than a second launch once that is
-        # MERGE_ROWS_FLOATS partial values per workgroup.
+    if vB is not None and _merge_rows_first(seq_splits, batch, hq, hkv, dv, vB.shape[-1]):
+        # many splits: merge the rows first, spread over the chip, then up-project one row per head
         mid, mid_lse = torch.empty((batch, hq, dv), dtype=torch.float32, device=partial.device), lse_out
         if mid_lse is None:
             mid_lse = torch.empty((batch, hq), dtype=torch.float32, device=partial.device)
