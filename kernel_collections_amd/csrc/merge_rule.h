@@ -25,10 +25,14 @@ inline bool merge_spread(int64_t splits, int64_t hq, int64_t batch, int64_t dv, 
   return splits > 1 && splits * dv >= 4096 && merge_blocks(hq, batch, d_out) <= 256;
 }
 
+// One head a workgroup too where there is little to fold: all heads of a kv head / one, 32 on 8 heads unless said.  Batch 1, one row of 512 5.8 / 4.8, of 256 4.2 / 3.7, 4 splits of
+// 512 6.0 / 4.8; 32 on 1, d_out 512, one of 512 5.9 / 4.9; batch 4, 7 splits of 512 6.3 / 5.1; batch 5, one of 512 5.9 / 6.6, batch 16 6.2 / 11.3
+inline bool merge_one_head(int64_t hq, int64_t batch, int d_out) { return merge_blocks(hq, batch, d_out) <= 256; }
+
 // Partial values that a workgroup may fold in every column block, one head of it (SPREAD) or all; beyond, the rows are merged first, by the whole chip.  us of one kernel
-// / rows and up-projection: dealt out, batch 1, 128 splits of 512 9.5 / 11.3, 256 of 384 11.7 / 12.1, 256 of 512 13.2 / 13.0 (16 on 1, d_out 512 13.2 / 12.1); a thread all splits, batch
+// / rows and up-projection: dealt out, batch 1, 128 splits of 512 9.5 / 10.2, 256 of 256 8.6 / 9.7, 256 of 384 11.7 / 11.0, 16 on 2, 128 of 512 8.3 / 8.7; a thread all splits, batch
 // 8, 32 of 512 (65536 values) 9.6 / 11.9, 16 on 1, d_out 512, batch 8, 32 of 256 (32768) 7.0 / 7.7, batch 16, 16 of 256 (32768) 7.2 / 9.1
-constexpr int64_t MERGE_SPREAD_FLOATS = 98304, MERGE_FLOATS = 65536;
+constexpr int64_t MERGE_SPREAD_FLOATS = 65536, MERGE_FLOATS = 65536;
 inline bool merge_rows_first(int64_t splits, int64_t hq, int hkv, int64_t dv, int64_t batch, int d_out) {
   if (merge_spread(splits, hq, batch, dv, d_out)) return splits * dv > MERGE_SPREAD_FLOATS;
   return splits > 1 && splits * merge_heads(hq, hkv, dv, batch, d_out) * dv > MERGE_FLOATS;

@@ -421,15 +421,14 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(
 // With an up-projection: one workgroup per (hpw heads of one kv head, block of 64 output columns).  Thread (cb, grp): 8 columns
 // x the vB rows grp, grp + 64, ...; its vB packets are on the way before the split counts are known.  The heads' merged rows
 // meet in the LDS (every column block repeats that merge: a caller with many splits merges the rows first), then 8 FMAs per packet and head, and the 64 row groups are added by halving exchanges inside a 16-lane row (each step
-// a lane keeps half of its sums and hands the other half over) and four LDS words per total.  By trace, batch 1: one row per
-// head, dv 512, 6.4 us for 32 heads on 8 or 1 kv heads (rows + up-projection at 256 splits: 12.5 us, one kernel that did both
-// 20 - 21.7); 8 splits of 256, 4.7 us (7.0); 16 x 32 heads, 2 splits of 512, 8.6 us (11.6).
+// a lane keeps half of its sums and hands the other half over) and four LDS words per total.  Batch 1, one row per
+// head, dv 512: 4.8 us in a graph of merges for 32 heads on 8 or 1 kv heads (5.8 with four heads a workgroup); 16 x 32 heads, 2 splits of 512, 8.6 us by trace (11.6).
 //
 // MANY_LOOP: many splits on a chip that the heads fill (launch_merge): a workgroup folds once for several column blocks.  MANY_SPREAD: on
 // one that is not full: one head per workgroup, its splits dealt out among groups of threads as in merge_rows_kernel, the product for that head alone (with three
-// absent heads multiplied beside it 0.6 - 0.9 us more).  32 splits of 256, 32 heads, d_out 128: 4.9 us (6.3 with a thread folding all splits of its packet), 128 of 512 9.5 (18.1).
+// absent heads multiplied beside it 0.6 - 0.9 us more).  ONE_HEAD: the same product where there are few splits (merge_rule.h).  32 splits of 256, 32 heads, d_out 128: 4.9 us (6.3 with a thread folding all splits of its packet), 128 of 512 9.5 (18.1).
 constexpr int MERGE_UP_T = 512;
-enum { MANY_LOOP = 1, MANY_SPREAD = 2 };
+enum { ONE_PASS = 0, MANY_LOOP = 1, MANY_SPREAD = 2, ONE_HEAD = 3 };
 //
 // TAIL: the up-projected row is merged with rows that are in output space already (the plain tail beside a factorised prefix), by their
 // log-sum-exps.  Their packets are folded while the merged rows are; a kernel of its own for it was 4 - 5 us more.
@@ -443,7 +442,7 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
     float* __restrict__ lse_out, int64_t sLb, int64_t sLh, int split_cap, const int32_t* __restrict__ split_plan, const MergeTail tail) {
   typedef typename Elem<TB>::vec8 vec8;
   extern __shared__ float merged[];               // [hpw][dv]; MANY_SPREAD: then a packet, a maximum and a sum of every thread
-  constexpr int HP = MANY == MANY_SPREAD ? 1 : 4; // heads of a pass
+  constexpr int HP = MANY == MANY_SPREAD || MANY == ONE_HEAD ? 1 : 4;   // heads of a pass
   __shared__ float tot[4][HP * MERGE_CB];         // [quarter of the row groups][heads x 64 columns]
   const int hfirst = blockIdx.x * hpw, kh = hfirst / (hq / hkv), b = blockIdx.y;
   int c0 = blockIdx.z * MERGE_CB;
@@ -583,7 +582,7 @@ __global__ __launch_bounds__(MERGE_UP_T) void merge_up_kernel(
       }
       __syncthreads();            // tot is reused by the next four heads, or the next columns
     }
-    if constexpr (!MANY) return;
+    if constexpr (MANY == ONE_PASS || MANY == ONE_HEAD) return;
     c0 += gridDim.z * MERGE_CB;
     if (c0 >= d_out) return;
     load_w();
@@ -633,7 +632,8 @@ static int launch_merge(const float* partial, const float* lse, void* out, const
   int z = cdiv(d_out, MERGE_CB);
   const bool many = tail.splits ? merge_tail_rows_first(seq_splits, hq, hkv, dv) : seq_splits > 1 && (int64_t)seq_splits * hpw * dv > MERGE_FLOATS;
   const bool spread = !tail.splits && (merge_spread(seq_splits, hq, batch, dv, d_out) || (many && (int64_t)(hq / hpw) * batch * z < 256));
-  if (spread) hpw = 1;
+  const bool head = !many && !spread && merge_one_head(hq, batch, d_out);
+  if (spread || head) hpw = 1;
   if (many || spread) z = (int)std::min<int64_t>(z, cdiv(256, std::min<int64_t>(256, (int64_t)(hq / hpw) * batch)));
   const dim3 grid(hq / hpw, batch, z);
   const size_t shm = ((size_t)hpw * dv + (spread ? MERGE_UP_T * 6 : 0) + (tail.splits ? hpw * (MERGE_CB + 3) : 0)) * sizeof(float);
@@ -644,13 +644,14 @@ static int launch_merge(const float* partial, const float* lse, void* out, const
   if (tail.splits) {
     if (many) return XKV_EUNSUPPORTED;   // the caller merges the rows first
     if constexpr (std::is_same<O, TB>::value) {
-      if (dv <= 256) XKV_MERGE_UP_TAIL(4, 0, true); else XKV_MERGE_UP_TAIL(8, 0, true);
+      if (head) { if (dv <= 256) XKV_MERGE_UP_TAIL(4, ONE_HEAD, true); else XKV_MERGE_UP_TAIL(8, ONE_HEAD, true); }
+      else { if (dv <= 256) XKV_MERGE_UP_TAIL(4, ONE_PASS, true); else XKV_MERGE_UP_TAIL(8, ONE_PASS, true); }
       return launch_status();
     }
     return XKV_EDTYPE;
   }
-  if (dv <= 256) { if (spread) XKV_MERGE_UP(4, MANY_SPREAD); else if (many) XKV_MERGE_UP(4, MANY_LOOP); else XKV_MERGE_UP(4, 0); }
-  else { if (spread) XKV_MERGE_UP(8, MANY_SPREAD); else if (many) XKV_MERGE_UP(8, MANY_LOOP); else XKV_MERGE_UP(8, 0); }
+  if (dv <= 256) { if (spread) XKV_MERGE_UP(4, MANY_SPREAD); else if (many) XKV_MERGE_UP(4, MANY_LOOP); else if (head) XKV_MERGE_UP(4, ONE_HEAD); else XKV_MERGE_UP(4, ONE_PASS); }
+  else { if (spread) XKV_MERGE_UP(8, MANY_SPREAD); else if (many) XKV_MERGE_UP(8, MANY_LOOP); else if (head) XKV_MERGE_UP(8, ONE_HEAD); else XKV_MERGE_UP(8, ONE_PASS); }
 #undef XKV_MERGE_UP
 #undef XKV_MERGE_UP_TAIL
   return launch_status();

@@ -222,7 +222,7 @@ def _merge_rows_first(splits, batch, hq, hkv, dv, d_out):
         return False
     blocks = -(-d_out // 64)
     if splits * dv >= 4096 and hq * batch * blocks <= 256:      # one head a workgroup
-        return splits * dv > 98304
+        return splits * dv > 65536
     hpw = g = hq // hkv
     while hpw > 1 and (g % hpw or hpw * dv * 4 > 48 * 1024):
         hpw -= 1
