@@ -37,7 +37,7 @@ PEAK_BF16_TFLOPS = 2500.0
 TRAFFIC_TABLE = os.path.join(ROOT, "profiles", "hbm_traffic_table.txt")
 CSRC = os.path.join(ROOT, "kernel_collections_amd", "csrc")
 TRAFFIC_SOURCES = {
-    "c3": ["recon_spec_impl.h", "recon_fast_impl.h", "recon_stage1.hip"],
+    "c3": ["recon_heads_impl.h", "recon_fast_impl.h", "recon_stage1.hip"],
     "c2": ["latent_ring.hip", "latent_ring.h"], "c5": ["latent_ring.hip", "latent_ring.h"], "c4": ["latent_ring.hip", "latent_ring.h"],
 }
 
@@ -260,13 +260,14 @@ def bench_c3(args, dev):
     step(0)
     parity = {"shared_basis": require_close(o[:1], ref0, "c3, sequence 0")}
 
-    # dominant kernel alone: stage 1
-    partial, lse = ops.workspaces(B, Hq, S, r, dev)
+    # dominant kernel alone: stage 1, cut as the call cuts it, for workgroups of two kv heads
+    S1 = args.splits or ops.occupancy_splits(B, Hkv // 2, L, tile=32, waves=1)
+    partial, lse = ops.workspaces(B, Hq, S1, r, dev)
     inv = ops.rope_inv_freq(d, theta, dev)
 
     def stage1(i):
         l = i % layers
-        ops.recon_stage1(q[l], A, kB[l], A, partial, lse, None, ns, None, B, Hq, Hkv, L, S, scale, True, inv, 0, None)
+        ops.recon_stage1(q[l], A, kB[l], A, partial, lse, None, None, None, B, Hq, Hkv, L, S1, scale, True, inv, 0, None)
 
     first_ms = None
     if args.headline_first:   # diagnosis: the same loop as the first GPU work of the process
@@ -292,7 +293,7 @@ def bench_c3(args, dev):
         parity["distinct_value_basis"] = require_close(o2[:1], ref_d, "c3 with its own value basis, sequence 0")
         d_ms, d_q = time_loop(lambda i: fr.gqa_xKV_rope(q[i % layers], A, kB[i % layers], Av, vB[i % layers], o2, ns, S, scale, theta),
                               args.steps, args.warmup)
-        distinct = {"us": round(d_ms * 1e3 / args.steps, 2), "step_us": d_q, "kernel": "recon_spec_kernel (scores) + latent_ring_kernel (given scores), two passes",
+        distinct = {"us": round(d_ms * 1e3 / args.steps, 2), "step_us": d_q, "kernel": "recon_heads_kernel (scores) + latent_ring_kernel (given scores), two passes",
                     "hbm_bytes": 2 * B * L * r * 2}
         del Av
 
@@ -321,7 +322,7 @@ def bench_c3(args, dev):
         "tokens_per_s": B / (us * 1e-6), "kv_tokens_scanned_per_s": B * L / (us * 1e-6),
         "config": {"workload": "c3 fused RoPE xKV decode: batch 16, 32q/8kv heads, d128, ctx %d, rank 512, "
                                "A shared by K/V and by a 4-layer group, per layer" % L, "kv_splits": S},
-        "roofline": {"bound": "mfma", "kernel": "recon_spec_kernel", "achieved": round(achieved, 1),
+        "roofline": {"bound": "mfma", "kernel": "recon_heads_kernel", "achieved": round(achieved, 1),
                      "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": round(achieved / PEAK_BF16_TFLOPS, 4),
                      "traffic": recorded_traffic("c3") if (L == 32768 and not args.splits) else None,
                      "kernel_avg_us": round(k_avg_ms * 1e3, 2), "kernel_median_us": round(k_med_ms * 1e3, 2),
@@ -705,7 +706,7 @@ def bench_ropedecode(args, dev):
         "ms_per_step": total_ms / args.steps, "step_us": step_q,
         "config": {"workload": "fused RoPE xKV decode, separate bases: batch 1, 32q/8kv, d128, kv_len %d, K rank %d, V rank %d, bf16"
                                % (L, rk, rv), "kv_splits": S},
-        "roofline": {"bound": "mfma", "kernel": "recon_scores_kernel + latent_ring_kernel (given scores), two passes", "achieved": round(tf, 1), "peak": PEAK_BF16_TFLOPS,
+        "roofline": {"bound": "mfma", "kernel": "recon_heads_kernel (scores) + latent_ring_kernel (given scores), two passes", "achieved": round(tf, 1), "peak": PEAK_BF16_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(tf / PEAK_BF16_TFLOPS, 4), "traffic": None,
                      "note": "whole call (scores, values, merge) over algorithmic FLOP", "algorithmic_flop": flops,
                      "hbm_side_GBps": round(B * L * (rk + rv) * 2 / (us * 1e-6) / 1e9, 1)},
