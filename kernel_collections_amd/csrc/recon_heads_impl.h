@@ -170,18 +170,16 @@ __global__ __launch_bounds__(256, 1) void recon_heads_kernel(const FastParams p,
     const int s = wave + 4 * i, kv = s / GP, g = s % GP;
     q0[i] = g < G ? to_f32(qraw[i][0]) : 0.f;
     q1[i] = g < G ? to_f32(qraw[i][1]) : 0.f;
-    if constexpr (SCORES) {
-      // Multiplied by the power of two that brings the head's largest feature to 2^14 .. 2^15, and the scores by the inverse: fp16 then holds every
-      // rotated pair, and the parts of small queries are no subnormals there.  A feature that is no finite number leaves the others as they are.
-      const int bits = __builtin_bit_cast(int, row_reduce<true, 16>(fmaxf(fabsf(q0[i]), fabsf(q1[i]))));
-      const int top = max(max(__builtin_amdgcn_readlane(bits, 0), __builtin_amdgcn_readlane(bits, 16)),
-                          max(__builtin_amdgcn_readlane(bits, 32), __builtin_amdgcn_readlane(bits, 48)));
-      const int up = max(-1, min(14 + 127 - (top >> 23), 100));
-      const float f = __builtin_bit_cast(float, (127 + up) << 23);
-      q0[i] *= f;
-      q1[i] *= f;
-      if (lane == 0) unscale[kv * 8 + g] = __builtin_bit_cast(float, (127 - up) << 23);
-    }
+    // Multiplied by the power of two that brings the head's largest feature to 2^14 .. 2^15, and the scores by the inverse: fp16 then holds every
+    // rotated pair, and the parts of small queries are no subnormals there.  A feature that is no finite number leaves the others as they are.
+    const int bits = __builtin_bit_cast(int, row_reduce<true, 16>(fmaxf(fabsf(q0[i]), fabsf(q1[i]))));
+    const int top = max(max(__builtin_amdgcn_readlane(bits, 0), __builtin_amdgcn_readlane(bits, 16)),
+                        max(__builtin_amdgcn_readlane(bits, 32), __builtin_amdgcn_readlane(bits, 48)));
+    const int up = max(-1, min(14 + 127 - (top >> 23), 100));
+    const float f = __builtin_bit_cast(float, (127 + up) << 23);
+    q0[i] *= f;
+    q1[i] *= f;
+    if (lane == 0) unscale[kv * 8 + g] = __builtin_bit_cast(float, (127 - up) << 23);
   }
   // q^ is kept in q-dot operand order: pair j = 32 dq' + 8 o + 4 g' + e sits at [o][dq'][g'][e] (partner at e + 4)
   const int qpos = ((((lane >> 3) & 3) * 2 + (lane >> 5)) * 2 + ((lane >> 2) & 1)) * 8 + (lane & 3);
@@ -233,7 +231,7 @@ __global__ __launch_bounds__(256, 1) void recon_heads_kernel(const FastParams p,
   const int sm_tok = 8 * g4 + TPL * (n16 / GC);
   const float* const ssrc = s_part + ((sm_slot / GP) * 8 + (sm_g < G ? sm_g : G - 1)) * FSP_ROW + sm_tok;
   float m_ref = NEG_INF, l_run = 0.f;   // reference maximum of the lane's head (base-2 domain); this lane's share of its row sum
-  const float scale2 = p.sm_scale * 1.44269504088896f, lazy2 = lazy_rescale<T>() * 1.44269504088896f;
+  const float scale2 = p.sm_scale * unscale[(sm_slot / GP) * 8 + (sm_g < G ? sm_g : G - 1)] * 1.44269504088896f, lazy2 = lazy_rescale<T>() * 1.44269504088896f;
   f32x4 acc[NMB];
 #pragma unroll
   for (int mb = 0; mb < NMB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};

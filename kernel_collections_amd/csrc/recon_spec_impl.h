@@ -283,7 +283,7 @@ __global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p, con
   }
   const float qinv = p.inv_freq[lane];
   factor.template init<false>(Bh, kB.sr, tid);
-  if constexpr (SCORES) {
+  {
     // Multiplied by the power of two that brings the head's largest feature to 2^14 .. 2^15, and the scores by the inverse: fp16 then holds every
     // rotated pair, and the parts of small queries are no subnormals there.  A feature that is no finite number leaves the others as they are.
 #pragma unroll
@@ -326,7 +326,7 @@ __global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p, con
   const int sm_row = sm_head < G ? sm_head : G - 1;
   const int sm_tok = 8 * g4 + TPL * (n16 / GP);
   float m_ref = NEG_INF, l_run = 0.f;   // reference maximum of the lane's head (base-2 domain); this lane's share of its row sum
-  const float scale2 = p.sm_scale * 1.44269504088896f, lazy2 = lazy_rescale<T>() * 1.44269504088896f;
+  const float lazy2 = lazy_rescale<T>() * 1.44269504088896f;
   // P.A accumulators (consumer c owns latent features RK/4 c .. + RK/4; column n16 = head slot) and the transposed tile reads
   // of two tiles live in accumulation registers a[0 .. 3 RK/16), by number (see pa_mfma_at)
   constexpr int TR0 = 4 * NMB, TRSET = 4 * NMB;
@@ -336,6 +336,7 @@ __global__ __launch_bounds__(512) void recon_spec_kernel(const FastParams p, con
   else asm volatile("" ::: "a63");
 
   __syncthreads();
+  const float scale2 = p.sm_scale * unscale[sm_row] * 1.44269504088896f;
 
   // Transposed reads: a 16-lane group reads a block of 4 rows x 16 columns, lanes 4 j .. 4 j + 3 supplying row j, and lane i
   // receives column i (4 values, one per row).  Rows 2 j (first read) and 2 j + 1 (second read) of the group's 8 tokens: with

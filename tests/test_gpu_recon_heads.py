@@ -102,3 +102,37 @@ def test_splits_fill_the_device_once(dev, shim):
         q, A, B = operands(dev, BF, 1, hkv, 4, L, r, r)
         fr.gqa_xKV_rope(q, A, B, A, B, torch.empty_like(q), torch.ones(1, dtype=torch.int32, device=dev), 1, 0.1, 5e5)
         assert shim.count("shim_recon_splits") == ops.occupancy_splits(1, groups, L, tile=32, waves=1)
+
+
+@pytest.mark.parametrize("r,hkv", [(512, 2), (384, 2), (256, 4)])
+@pytest.mark.parametrize("S", [2, WORKGROUPS])                    # one kv head a workgroup, and several
+@pytest.mark.parametrize("dtype,size", [(FP, 65504.0), (BF, 2.0 ** -24), (FP, 0.0)])
+def test_decode_of_large_and_small_queries(dev, dtype, size, r, hkv, S):
+    """As of the scores alone: a rotated pair may leave fp16's range where neither of its features does, and small ones are subnormal there."""
+    L, G, off = 6144, 3, 100
+    q, A, B = operands(dev, dtype, 1, hkv, G, L, r, r)
+    q = q.sign() * size if size > 1 else q * size
+    scale = 0.25 / size if size else 1.0
+    part, lse = torch.full((1, hkv * G, S, r), float("nan"), device=dev), torch.full((1, hkv * G, S), float("nan"), device=dev)
+    poison()
+    ops.recon_stage1(q, A, B, A, part, lse, None, None, None, 1, hkv * G, hkv, L, S, scale, True, ops.rope_inv_freq(128, 5e5, q.device), off, None)
+    out, total = torch.empty((1, hkv * G, r), device=dev), torch.empty((1, hkv * G), device=dev)
+    ops.merge_stage2(part, lse, out, None, None, None, 1, hkv * G, hkv * G, L, S, total)
+    s = keys_and_scores(q, A, B, off) * scale
+    ref = torch.softmax(s, -1) @ A.double()
+    # P is 16 bits wide (2^-9 or 2^-11 of it), the keys and the query were in fp16 on the way: 2.9e-4 of a score, in a row's sum as much at most
+    assert (out - ref).norm() <= (4e-3 if dtype == BF else 2e-3) * ref.norm()
+    assert (total - torch.logsumexp(s, -1)).abs().max() <= 4e-4 * max(1.0, s.abs().max().item())
+
+
+@pytest.mark.parametrize("hq,hkv,L", [(32, 8, 52000), (24, 6, 70000)])     # calls that scores and values apart once served
+def test_long_decode_of_large_queries(dev, hq, hkv, L):
+    import kernel_collections_amd.flash_recontruction as fr
+    q, A, B = operands(dev, FP, 1, hkv, hq // hkv, L, 256, 256)
+    q = q.sign() * 65504
+    V = gen((1, hkv, 256, 128), std=1 / 16, dtype=FP, seed=5).to(dev)
+    o = fr.gqa_xKV_rope(q, A, B, A, V, torch.empty(1, hq, 128, device=dev), torch.ones(1, dtype=torch.int32, device=dev), 1, 0.25 / 65504, 5e5)
+    P = torch.softmax(keys_and_scores(q, A, B, 0) * (0.25 / 65504), -1)
+    ref = ((P @ A.double()).reshape(1, hkv, hq // hkv, 256) @ V.double()).reshape(1, hq, 128)
+    # as above; fp32 angles up to position 70000: half a unit, 2^-8 radians, at the fastest pairs, 2.5e-4 of a score beside the 2.9e-4
+    assert (o - ref).norm() <= 3e-3 * ref.norm()
