@@ -42,7 +42,8 @@ template <int RK, int NH, bool SCORES, int TPL> struct HeadsShape {
   static constexpr int AHEAD = 10 / NH;        // k-steps between the read of an operand and its use
   static constexpr int SP_FLOATS = 4 * NH * 8 * FSP_ROW;   // one buffer of partial scores: [wave 4][kv NH][head 8][FSP_ROW]
   // rotation: QU instructions per quarter (four pairs a lane) of a head
-  static constexpr int QU = SCORES ? 20 : 12, NU = QU * 2 * NH;
+  static constexpr bool FP32 = SCORES || RK == 256;   // rotation
+  static constexpr int QU = FP32 ? 20 : 12, NU = QU * 2 * NH;
   static constexpr int SU = TPL / 4 * 7 + 2;   // steps of the softmax
   static constexpr int PA = (NMB + 1) / 2;     // places of P.A at the end
   static constexpr int ROT0 = NH + 3;
@@ -64,6 +65,7 @@ __global__ __launch_bounds__(256, 1) void recon_heads_kernel(const FastParams p,
   constexpr int TPL = GC / 2;                  // tokens per lane of the softmax
   typedef HeadsShape<RK, NH, SCORES, TPL> S;
   constexpr int FROW = S::FROW, FTILE = S::FTILE, NK = S::NK, M = S::M, NMB = S::NMB, SP_FLOATS = S::SP_FLOATS, AHEAD = S::AHEAD, BAR = S::BAR, QU = S::QU;
+  constexpr bool FP32 = S::FP32;
   static_assert(GC <= 16 && GC >= 8 && (S::ROT1 - S::ROT0) > 0 && S::done(2 * NH - 1) + 2 < BAR && BAR <= S::NEXT, "places of a period");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -271,14 +273,15 @@ __global__ __launch_bounds__(256, 1) void recon_heads_kernel(const FastParams p,
       for (int ks = 0; ks < NK; ++ks) asm volatile("" : "+a"(breg[kv][ks]));
     const int t1 = pp - 1;
     const bool live = pp > 0;
-    // rotation of tile pp - 1, four pairs of a head at a time, in three stages that depend on the stage before alone.  Scores: in fp32, rounded once.  Else in
-    // packed fp16 (its error is that of the keys' rounding once more)
+    // rotation of tile pp - 1, four pairs of a head at a time, in three stages that depend on the stage before alone.  Scores, and rank 256, whose long calls
+    // took their scores apart before: in fp32, rounded once.  Else in packed fp16 (its error is that of the keys' rounding once more).  Rank 256, 65536 tokens, 32 heads on 8
+    // kv heads: 49.4 us a call in fp32, 47.7 in fp16 
     float tl[4], th[4], kl[4], kr[4];
     h2 lo2[2], hi2[2], pl[2], ph[2], kw[4];
     auto rotate = [&](auto u2_c) {
       constexpr int KV = decltype(u2_c)::value / (2 * QU), O = decltype(u2_c)::value / QU % 2, U = decltype(u2_c)::value % QU;
       const f32x16& j = k[PAR ^ 1][KV];
-      if constexpr (SCORES) {
+      if constexpr (FP32) {
         constexpr int STAGE = U / 8, R = STAGE < 2 ? U % 8 / 2 : U - 16;
         const float lo = j[4 * O + R], hi = j[8 + 4 * O + R], cc = ct[PAR ^ 1][4 * O + R], ss = st[PAR ^ 1][4 * O + R];
         if constexpr (STAGE == 0) {

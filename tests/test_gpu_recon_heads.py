@@ -136,3 +136,15 @@ def test_long_decode_of_large_queries(dev, hq, hkv, L):
     ref = ((P @ A.double()).reshape(1, hkv, hq // hkv, 256) @ V.double()).reshape(1, hq, 128)
     # as above; fp32 angles up to position 70000: half a unit, 2^-8 radians, at the fastest pairs, 2.5e-4 of a score beside the 2.9e-4
     assert (o - ref).norm() <= 3e-3 * ref.norm()
+
+
+def test_scores_of_decode_at_rank_256(dev):
+    """Peaked rows: a split's log-sum-exp is its largest score, which the call had from a pass of its own before one kernel served it."""
+    r, hkv, G, L, S, scale = 256, 4, 4, 6144, WORKGROUPS, 4.0
+    q, A, B = operands(dev, BF, 1, hkv, G, L, r, r)
+    part, lse = torch.empty((1, hkv * G, S, r), device=dev), torch.empty((1, hkv * G, S), device=dev)
+    ops.recon_stage1(q, A, B, A, part, lse, None, None, None, 1, hkv * G, hkv, L, S, scale, True, ops.rope_inv_freq(128, 5e5, q.device), 0, None)
+    s = keys_and_scores(q, A, B, 0) * scale
+    err = lse - torch.logsumexp(s.reshape(1, hkv * G, S, L // S), -1)
+    # The key and the query rounded to fp16 once each: 2.9e-4 of the scores' size (3072 rows: within 2 %); rotated in fp16 besides, with cosines of 16 bits, 3.9e-4
+    assert err.pow(2).mean().sqrt() <= 3.2e-4 * s.pow(2).mean().sqrt()
