@@ -233,7 +233,10 @@ __global__ __launch_bounds__(256, 1) void recon_heads_kernel(const FastParams p,
   const int sm_tok = 8 * g4 + TPL * (n16 / GC);
   const float* const ssrc = s_part + ((sm_slot / GP) * 8 + (sm_g < G ? sm_g : G - 1)) * FSP_ROW + sm_tok;
   float m_ref = NEG_INF, l_run = 0.f;   // reference maximum of the lane's head (base-2 domain); this lane's share of its row sum
-  const float scale2 = p.sm_scale * unscale[(sm_slot / GP) * 8 + (sm_g < G ? sm_g : G - 1)] * 1.44269504088896f, lazy2 = lazy_rescale<T>() * 1.44269504088896f;
+  // Rank 256: the running maximum itself, whose weight of 1 is exact in 16 bits, as in the pass over given scores that long calls had before.  65536 tokens, 32 heads on 8 kv heads:
+  // 50.4 us a call, 49.4 with a lazy reference, 58.8 as two passes; error of bf16 against float64 3.2e-4, 3.6e-4, 3.0e-4 over even weights, 1.1e-3, 1.7e-3, 1.1e-3 over peaked ones
+  constexpr float LAZY = RK == 256 ? 0.f : lazy_rescale<T>();
+  const float scale2 = p.sm_scale * unscale[(sm_slot / GP) * 8 + (sm_g < G ? sm_g : G - 1)] * 1.44269504088896f, lazy2 = LAZY * 1.44269504088896f;
   f32x4 acc[NMB];
 #pragma unroll
   for (int mb = 0; mb < NMB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
