@@ -671,6 +671,10 @@ PyObject* py_head_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_head_rows_floor(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 3, [&]() -> PyObject* { return PyLong_FromLong(xkv::head_rows_floor(I(a[0]), I(a[1]), I(a[2]))); });
 }
+// recon_scores_pays(rank, kv heads, heads per kv head, tokens) -> bool (recon_groups.h)
+PyObject* py_recon_scores_pays(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 4, [&]() -> PyObject* { return PyBool_FromLong(xkv::recon_scores_pays(I(a[0]), I(a[1]), I(a[2]), I(a[3]))); });
+}
 // split_floor(batch, groups, kv_len, per_cu, cus, up) -> int
 PyObject* py_split_floor(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 6, [&]() -> PyObject* { return PyLong_FromLong(split_floor(I(a[0]), I(a[1]), I(a[2]), I(a[3]), I(a[4]), I(a[5]))); });
@@ -714,7 +718,7 @@ PyObject* init(PyObject*, PyObject* path) {
 PyMethodDef methods[] = {
     {"init", init, METH_O, nullptr},       XKV_FAST("balanced_splits", py_balanced_splits), XKV_FAST("nope_decode", nope_decode), XKV_FAST("ragged_target", py_ragged_target),
     XKV_FAST("split_floor", py_split_floor), XKV_FAST("decode_splits", py_decode_splits), XKV_FAST("head_rows", py_head_rows),
-    XKV_FAST("head_rows_floor", py_head_rows_floor),
+    XKV_FAST("head_rows_floor", py_head_rows_floor), XKV_FAST("recon_scores_pays", py_recon_scores_pays),
     XKV_FAST("nope_scores", nope_scores),  XKV_FAST("rope_decode", rope_decode),            XKV_FAST("rope_scores", rope_scores),
     XKV_FAST("gqa", gqa),                  XKV_FAST("mla", mla),                            XKV_FAST("prefix_tail", prefix_tail),
     {nullptr, nullptr, 0, nullptr}};

@@ -40,7 +40,7 @@ inline int launch_recon_heads(const FastParams& p, const FactorOperand& kB, int 
                        : launch_recon_heads_256(p, kB, batch, dtype, st);
 }
 
-// Scores only (recon_scores.hip): ranks up to 224 with up to 16 query heads per kv head, 256, 320, 384 and 448 with up to 8.  Reads kB as it is
+// Scores only (recon_scores.hip): ranks up to 224 with up to 16 query heads per kv head, 256, 320 and 448 with up to 8.  Reads kB as it is
 // (16-byte packets of unit stride).
 bool recon_scores_serves(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int rank);
 int launch_recon_scores(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int batch, int dtype, int rank,

@@ -28,12 +28,13 @@ inline int64_t recon_heads_work(int rank, int hkv) {
 // Workgroups from which on the dispatcher takes it, whoever chose the splits: the chip three quarters full
 constexpr int64_t RECON_HEADS_WORKGROUPS = 192;
 
-// Scores at ranks 256 and 384 of up to eight heads a kv head, by recon_scores_kernel or by one head a workgroup of the wave-specialised kernel, whose workgroups start
-// faster.  us a call, wave-specialised / recon_scores, 32 heads on 8 unless said: rank 256, 1000 tokens 6.5 / 8.7, 8192 9.6 / 10.8, 16384 14.0 / 13.9, 32768 23.0 / 21.3; 64 on 8,
-// 8192 10.1 / 11.5, 16384 15.5 / 15.1; 16 on 2, 16384 8.2 / 10.8, 65536 15.3 / 16.3; 12 on 3, 60000 18.8 / 17.3; 4 on 1, 60000 10.9 / 13.8.  Rank 384, 1000 7.0 / 9.1, 8192 11.7 /
-// 13.4, 32768 28.4 / 28.3; 12 on 3, 130001 43.8 / 47.7, 8 x 131072 322 / 328; 20 on 5, 4 x 30000 59.2 / 60.9; 8 on 2, 65536 19.3 / 19.5; 4 on 1, 120000 20.6 / 21.5, 262144 48.9 / 45.1
+// Scores at rank 256 of up to eight heads a kv head, by recon_scores_kernel or by one head a workgroup of the wave-specialised kernel, whose workgroups start faster, the more
+// so the fewer kv heads read the same factor.  us a call, wave-specialised / recon_scores, 32 heads on 8 unless said: 1000 tokens 6.5 / 8.7, 12288 12.7 / 13.1, 16384 14.8 / 14.3, 32768
+// 22.5 / 20.0; 16 on 4, 16384 9.2 / 10.3, 32768 13.1 / 13.1, 65536 21.2 / 19.6; 12 on 3, 43000 13.4 / 14.3, 54000 17.3 / 16.3; 16 on 2, 65536 14.1 / 15.3, 98304 18.4 / 18.3, 131072 22.5 /
+// 21.4; 8 on 1, 131072 16.1 / 20.5, 524288 45.8 / 48.7, 8 x 16384 16.1 / 20.4, 2000000 229 / 230.  Rank 384 never: 32 on 8, 32768 28.4 / 28.3; 12 on 3, 130001 43.8 / 47.7; 4 on 1, 196608
+// 27.6 / 29.7, 262144 34.1 / 36.7, 524288 82.4 / 84.9
 inline bool recon_scores_pays(int rank, int hkv, int G, int64_t tokens) {
-  return rank == 256 ? G <= 8 && tokens * hkv >= 131072 : rank == 384 && hkv == 1 && G <= 4 && tokens >= 196608;
+  return rank == 256 && G <= 8 && hkv > 1 && tokens * hkv >= (hkv == 2 ? 196608 : hkv == 3 ? 143360 : 131072);
 }
 
 }  // namespace xkv

@@ -15,14 +15,14 @@
 // RoPE by angle addition: R(position) = R(first token of the step) R(place in the step).  The second factor is per-lane constants; the
 // first is moved to the query, q^ = R(step)^T q, which the workgroup needs once for all its tokens: in every group of two steps the waves
 // make the q^ of the next group (a pair per lane) and leave it in the LDS, as a high and a low fp16 part: the scores are then as exact as those
-// of an unrotated query (2.1e-4 of their size against float64, all of it the keys' rounding to fp16).  At ranks 256 and 384 it is one fp16 value
-// (2.9e-4), for callers that give a workspace and with it had the wave-specialised kernels' one value (3.8e-4 and 4.4e-4): a low part costs 4 - 8 % there.
+// of an unrotated query (2.1e-4 of their size against float64, all of it the keys' rounding to fp16).  At rank 256 it is one fp16 value
+// (2.9e-4), for callers that give a workspace and with it the wave-specialised kernel's one value: a low part costs 4 - 8 % there.
 //
 // What bounds it: one wave per SIMD that issues everything in order, an instruction in 5 cycles at best, and the LDS.  At 256 ranks the 68 matrix
 // instructions of a tile are 1088 cycles, a block of 16 pairs takes 400 with everything else, and a group's start (barrier, q^)
 // 500 more.  A branch or a memory operation waited for on the spot costs such a wave its whole latency, so the groups are straight-line code: places
 // written whether they are needed or not, stores dropped by the resource's bounds, the output's form a template parameter.
-// us at 131072 tokens, 8 kv heads, 32 heads: rank 64 34.9, 128 45.8, 192 57.9, 224 64.8, 256 63.8, 320 100, 384 102, 448 122; with rows read in operand
+// us at 131072 tokens, 8 kv heads, 32 heads: rank 64 34.9, 128 45.8, 192 57.9, 224 64.8, 256 63.8, 320 100, 448 122 (384 102, level with the wave-specialised kernel from 32768 tokens on); with rows read in operand
 // order, rotation of keys by base and place, and branches rank 64 47.5, 128 53.7, 192 63.9, 256 77.8, 384 117.  Two waves per SIMD with half the pairs each
 // and a barrier per step: 38.8, 50.5, 59.7, 73.7, 105.
 #include "recon_fast.h"
@@ -52,7 +52,7 @@ constexpr int OUT = -1;              // lane offset that no resource reaches: th
 template <int NKS, int WPT> struct ScoresShape {
   static constexpr int RK = 32 * NKS, RANK = RK * WPT;           // ranks of a wave
   static constexpr int STEP = 64 / WPT;                          // tokens
-  static constexpr bool LO = RANK != 256 && RANK != 384;         // q^ has a low part
+  static constexpr bool LO = RANK != 256;                        // q^ has a low part
   static constexpr int ROW = RK * 2, TILE = 16 * ROW, RING = SLOTS * 4 * TILE;   // [slot][wave][16 rows]
   // behind the ring: scores that wait for the other wave's [2 GROUP steps][wave][lane], q^ [2 groups][GROUP steps][parts][head][QROW words]
   static constexpr int PART = WPT == 1 ? 0 : 2 * GROUP * 4 * 64 * 16, QROW = 64 + 4;
@@ -486,7 +486,7 @@ int launch_mode(const FastParams& p, const FactorOperand& kB, int batch, int ran
     XKV_SCORES_RANK(8)
 #undef XKV_SCORES_RANK
 #define XKV_SCORES_RANK(N) case 64 * N: return launch_t<T, N, 2, MODE>(p, kB, batch, st);
-    XKV_SCORES_RANK(5) XKV_SCORES_RANK(6) XKV_SCORES_RANK(7)
+    XKV_SCORES_RANK(5) XKV_SCORES_RANK(7)
 #undef XKV_SCORES_RANK
     default: return XKV_EUNSUPPORTED;
   }
@@ -504,7 +504,7 @@ int launch(const FastParams& p, const FactorOperand& kB, int batch, int rank, hi
 bool recon_scores_serves(const FastParams& p, const void* kB, int64_t sBb, int64_t sBh, int64_t sBr, int rank) {
   if (((sBb | sBh | sBr) & 7) || (reinterpret_cast<uintptr_t>(kB) & 15)) return false;
   if (rank > 224 && p.hq / p.hkv > 8) return false;                  // the LDS
-  if (rank > 256 && (rank % 64 || rank == 512)) return false;        // two equal halves; 512 is faster elsewhere
+  if (rank > 256 && rank != 320 && rank != 448) return false;        // two equal halves; 384 and 512 are faster elsewhere
   // 32-bit lane offsets: 16 token rows, the score rows of 16 heads.  Rows that overlap would make offsets negative
   return p.sAl >= rank && p.sAl < (1 << 25) && (int64_t)(p.hq / p.hkv) * p.kv_len < (1 << 28);
 }

@@ -451,12 +451,12 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
     f.hq = hq; f.hkv = hkv; f.kv_len = kv_len; f.max_splits = max_splits; f.total_wg = batch * hkv * max_splits;
     f.sm_scale = sm_scale; f.inv_freq = inv_freq; f.pos_offset = pos_offset;
     // Scores-only shapes (us a call, this kernel / the generic one, 32 heads on 8 kv heads: rank 128, 5 x 7488 tokens 17.9 / 21.6; rank
-    // 192, 7 x 39246 124 / 153; rank 224, 131072 64.5 / 241; rank 320, 131072 99.8 / 269; rank 448, 131072 127 / 313).  At ranks 256 and 384 its rotated query is one fp16
+    // 192, 7 x 39246 124 / 153; rank 224, 131072 64.5 / 241; rank 320, 131072 99.8 / 269; rank 448, 131072 127 / 313).  At rank 256 its rotated query is one fp16
     // value, so only where the caller's workspace asks for kernels that have that; a factor that is not 16-byte packets is copied there.
-    const bool two = rank == 256 || rank == 384;
-    if (!two || (spec && recon_scores_pays(rank, hkv, hq / hkv, (int64_t)batch * kv_len))) {
+    const bool one_value = rank == 256;
+    if (!one_value || (spec && recon_scores_pays(rank, hkv, hq / hkv, (int64_t)batch * kv_len))) {
       const int64_t head = (int64_t)rank * 128;
-      const bool copy = two && !whole_packets(kB, sBb, sBh, sBr);
+      const bool copy = one_value && !whole_packets(kB, sBb, sBh, sBr);
       const FactorOperand rows = copy ? FactorOperand{workspace, sBb == 0 ? 0 : hkv * head, head, 128} : FactorOperand{kB, sBb, sBh, sBr};
       if (recon_scores_serves(f, rows.p, rows.sb, rows.sh, rows.sr, rank)) {
         if (copy) copy_factor(kB, sBb, sBh, sBr, batch, hkv, rank, workspace, st);

@@ -190,6 +190,15 @@ def test_two_passes_where_they_are_faster(rank, v_rank, hkv, tokens, two):
     assert _fused._two_pass(rank, tokens, B, v_rank=v_rank or rank, shared=not v_rank) == two
 
 
+@pytest.mark.parametrize("rank,hkv,G,tokens,pays", [
+    (256, 8, 4, 12288, False), (256, 8, 4, 16384, True), (256, 8, 9, 16384, False), (256, 4, 4, 16384, False), (256, 4, 4, 32768, True), (256, 3, 4, 43000, False), (256, 3, 8, 54000, True),
+    (256, 2, 8, 65536, False), (256, 2, 8, 131072, True), (256, 1, 8, 131072, False), (256, 1, 4, 524288, False), (384, 8, 4, 32768, False), (384, 1, 4, 262144, False)])
+def test_scores_by_independent_waves_where_they_are_faster(rank, hkv, G, tokens, pays):
+    """Both sides as measured beside the line: the fewer kv heads, the later."""
+    from kernel_collections_amd import _xkv_host
+    assert _xkv_host.recon_scores_pays(rank, hkv, G, tokens) == pays
+
+
 @pytest.mark.parametrize("batch,groups,per_cu,jobs", [(1, 1, 1, 256), (32, 1, 1, 256), (128, 1, 1, 256), (129, 1, 1, 512), (64, 8, 2, 128),
                                                      (65, 8, 2, 192), (3, 300, 1, 6), (5, 512, 2, 10)])
 def test_ragged_batches_get_two_jobs_a_sequence(batch, groups, per_cu, jobs):
