@@ -96,17 +96,20 @@ def decode_k_only(q, k_A, k_B, v_buffer, o, num_kv_splits, max_kv_splits, sm_sca
 #   values of their own: rank 256 / 256, 12288 tokens 26.4 / 27.3, 14336 29.7 / 29.7 (16 on 2: 49152 32.8 / 34.4, 65536 39.0 / 37.3); 256 / 512, 16384 35.0 / 37.1, 24576 48.9 / 43.0
 #   (16 on 4: 32768 38.9 / 38.0; 16 on 2: 98304 55.5 / 55.5); 384 / 384, 16384 37.9 / 38.1, 20480 40.5 / 39.9, 24576 45.9 / 43.1 (16 on 4: 40960 41.5 / 40.0; 16 on 2: 98304 56.6 /
 #   54.2); 384 / 512, 20480 42.3 / 42.0, 24576 49.3 / 45.9 (16 on 4: 49152 49.5 / 47.0; 16 on 2: 131072 74.7 / 70.0); 512 / 512, 24576 51.5 / 50.7, 30720 58.9 / 57.1 (16 on 2:
-#   131072 78.6 / 78.7, 163840 94.9 / 93.6); 8 on 1 never, rows read from memory: 384 / 512, 200000 80.8 / 89.7, 300000 110 / 123; 512 / 512, 300000 125 / 138;
+#   131072 78.6 / 78.7, 163840 94.9 / 93.6); 8 on 1, whose rows come from memory, 384 / 512, 200000 80.8 / 89.7, 300000 110 / 123; 512 / 512, 262144 108 / 104: those lines are where two passes
+#   were the faster once, because calls beyond them had fp32 rotation, a scaled query and weights from the running maximum, which the one kernel has not (bf16, rank 256 / 256, 131072 tokens: 1.8e-3 from
+#   float64 against 1.5e-3, peaked 2.4e-3 and 1.6e-3; queries of 65504 give NaN);
 #   rank pairs without an 8-wave kernel, 512 / 384: 4096 31.8 / 33.2, 8192 45.5 / 38.8 (8 on 1: 98304 63.9 / 51.9)
 #   one basis: rank 128, 8192 23.5 / 25.6, 14336 28.7 / 27.4 (16 on 2: 57344 29.9 / 29.6; 8 on 1: 131072 33.2 / 32.5); rank 192, 8192 25.9 / 27.9, 14336 32.1 / 30.3, 131072 143 / 78.7
 #   (16 on 2: 57344 32.9 / 32.4; 8 on 1: 131072 36.2 / 37.8, 262144 52.9 / 55.4); rank 256 with several kv heads a workgroup one kernel, which the native layer takes before it asks, else (64 on 8, 65536 50.9 / 57.6, 163840
-#   111 / 114, 262144 179 / 174; 24 on 6: 98304 58.0 / 62.9, 163840 88.1 / 88.3, 262144 140 / 129; 32 on 4: 262144 97.5 / 105; 16 on 2: 131072 39.6 / 48.5); rank 384 and 512 one kernel up to 131072 tokens (122 / 130, 142 / 161)
+#   111 / 114, 262144 179 / 174; 24 on 6: 98304 58.0 / 62.9, 163840 88.1 / 88.3, 262144 140 / 129; 32 on 4: 262144 97.5 / 105; 16 on 2: 131072 39.6 / 48.5) as exact as calls were that
+#   had no such kernel: even weights in bf16 3.8e-4 from float64 against 3.3e-4, peaked ones 2.1e-3 and 1.2e-3; rank 384 and 512 one kernel up to 131072 tokens (122 / 130, 142 / 161)
 TWO_PASS_KEY_RANKS = (512, 384, 256)
 TWO_PASS_MIN_TOKENS = 49152         # where a caller's counts are taken, whatever the kv heads; the other lines are in thirds of it
 TWO_PASS_WORK = {(256, 256): 6, (256, 512): 8, (384, 384): 10, (384, 512): 10, (512, 512): 15}   # tokens x kv heads, pairs with an 8-wave kernel
+TWO_PASS_WORK_ONE = {(384, 384): 14, (384, 512): 14}    # of one kv head, where that is another line
 TWO_PASS_WORK_OTHER = 2
 TWO_PASS_WORK_SHARED = {128: (1, 114688), 192: (2, 114688), 256: (4, 409600)}    # least kv heads, tokens x kv heads
-TWO_PASS_WORK_ALONE = 1179648       # rank 256 where no kv heads share a workgroup
 # Key ranks up to 192 have no 8-wave kernel: two passes from this many tokens x kv heads on, and from four times as many at the ranks
 # that the generic kernel is instantiated for (key rank 64, value rank 256, 1024 tokens 17.6 / 18.9, 4096 27.8 / 24.7; 16 on 4, 2048 19.7 / 20.6, 3072 22.9 / 21.7;
 # 8 on 1, 8192 21.5 / 23.1, 12288 24.1 / 23.4; key rank 192, value rank 512, 4096 27.8 / 30.3, 8192 38.3 / 37.4, 16384 59.4 / 40.1; 16 on 4, 8192 28.5 / 30.2, 16384
@@ -119,17 +122,16 @@ GENERIC_RANKS = (128, 192)
 TWO_PASS_MIN_TOKENS_ASKED = 4096
 
 
-def _two_pass(rank, tokens, k_B, asked=False, v_rank=512, shared=False, hq=0):
+def _two_pass(rank, tokens, k_B, asked=False, v_rank=512, shared=False):
     hkv = k_B.shape[1]
     if shared:
         least, work = TWO_PASS_WORK_SHARED.get(rank, (1, float("inf")))
-        if rank == 256 and work and (hkv % 4 or hq > 4 * hkv):
-            work = max(work, TWO_PASS_WORK_ALONE)
         return hkv >= least and tokens * hkv >= work
     if rank in TWO_PASS_KEY_RANKS:
-        work = TWO_PASS_WORK.get((rank, v_rank), TWO_PASS_WORK_OTHER) * TWO_PASS_MIN_TOKENS // 3
-        least = 2 if (rank, v_rank) in TWO_PASS_WORK and work else 1
-        return (hkv >= least and tokens * hkv >= work) or (asked and tokens >= TWO_PASS_MIN_TOKENS)
+        work = TWO_PASS_WORK.get((rank, v_rank), TWO_PASS_WORK_OTHER)
+        if hkv == 1:
+            work = TWO_PASS_WORK_ONE.get((rank, v_rank), work)
+        return tokens * hkv >= work * TWO_PASS_MIN_TOKENS // 3 or (asked and tokens >= TWO_PASS_MIN_TOKENS)
     if rank > TWO_PASS_SMALL_RANK or not ops._row_ok(k_B):
         return False
     if asked:
@@ -144,7 +146,7 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
     if sin_cos is None and kv_lens is None and ops.USE_RECON_WORKSPACE:
         native = _lib.native()
         shared = v_A is k_A or (v_A.data_ptr() == k_A.data_ptr() and v_A.shape == k_A.shape and v_A.stride() == k_A.stride())
-        two_pass = _two_pass(k_A.shape[-1], k_A.shape[0] * k_A.shape[1], k_B, v_rank=v_A.shape[-1], shared=shared, hq=q_pe.shape[1])
+        two_pass = _two_pass(k_A.shape[-1], k_A.shape[0] * k_A.shape[1], k_B, v_rank=v_A.shape[-1], shared=shared)
         done = native and native.rope_decode(q_pe, k_A, k_B, v_A, v_B, o, sm_scale,
                                              ops.rope_inv_freq(q_pe.shape[-1], theta, q_pe.device), pos_offset, two_pass)
         if done is not None:

@@ -125,15 +125,16 @@ def test_decode_of_large_and_small_queries(dev, dtype, size, r, hkv, S):
     assert (total - torch.logsumexp(s, -1)).abs().max() <= 4e-4 * max(1.0, s.abs().max().item())
 
 
-@pytest.mark.parametrize("hq,hkv,L", [(32, 8, 52000), (24, 6, 70000)])     # calls that scores and values apart once served
-def test_long_decode_of_large_queries(dev, hq, hkv, L):
+@pytest.mark.parametrize("hq,hkv,L,shared", [(32, 8, 52000, True), (24, 6, 70000, True), (8, 1, 98304, False)])     # calls that scores and values apart once served, or do
+def test_long_decode_of_large_queries(dev, hq, hkv, L, shared):
     import kernel_collections_amd.flash_recontruction as fr
     q, A, B = operands(dev, FP, 1, hkv, hq // hkv, L, 256, 256)
     q = q.sign() * 65504
     V = gen((1, hkv, 256, 128), std=1 / 16, dtype=FP, seed=5).to(dev)
-    o = fr.gqa_xKV_rope(q, A, B, A, V, torch.empty(1, hq, 128, device=dev), torch.ones(1, dtype=torch.int32, device=dev), 1, 0.25 / 65504, 5e5)
+    vA = A if shared else gen((1, L, 256), dtype=FP, seed=4).to(dev)
+    o = fr.gqa_xKV_rope(q, A, B, vA, V, torch.empty(1, hq, 128, device=dev), torch.ones(1, dtype=torch.int32, device=dev), 1, 0.25 / 65504, 5e5)
     P = torch.softmax(keys_and_scores(q, A, B, 0) * (0.25 / 65504), -1)
-    ref = ((P @ A.double()).reshape(1, hkv, hq // hkv, 256) @ V.double()).reshape(1, hq, 128)
+    ref = ((P @ vA.double()).reshape(1, hkv, hq // hkv, 256) @ V.double()).reshape(1, hq, 128)
     # as above; fp32 angles up to position 70000: half a unit, 2^-8 radians, at the fastest pairs, 2.5e-4 of a score beside the 2.9e-4
     assert (o - ref).norm() <= 3e-3 * ref.norm()
 

@@ -182,6 +182,9 @@ def test_two_passes_at_small_key_ranks_where_they_are_faster(rank, hkv, tokens, 
 @pytest.mark.parametrize("rank,v_rank,hkv,tokens,two", [
     (256, 256, 8, 8192, False), (256, 256, 8, 12288, True), (256, 512, 8, 12288, False), (256, 512, 8, 16384, True), (256, 512, 2, 49152, False),
     (384, 384, 8, 16384, False), (384, 384, 8, 28672, True), (512, 512, 8, 28672, False), (512, 512, 8, 32768, True), (512, 384, 8, 4096, True), (512, 384, 8, 2048, False),
+    (384, 384, 8, 20480, True), (384, 512, 8, 16384, False), (384, 512, 8, 24576, True), (384, 384, 2, 65536, False), (384, 384, 2, 98304, True),
+    (256, 256, 1, 98303, False), (256, 256, 1, 98304, True), (384, 512, 1, 200000, False), (384, 512, 1, 229376, True), (384, 384, 1, 229375, False), (512, 512, 1, 262144, True),   # one kv head
+    (256, 0, 6, 68266, False), (256, 0, 6, 68267, True), (256, 0, 8, 51200, True),     # one basis, whatever shares a workgroup
     (192, 0, 1, 262144, False), (192, 0, 2, 57344, True), (128, 0, 1, 131072, True), (256, 0, 2, 262144, False), (256, 0, 4, 102400, True), (384, 0, 8, 131072, False)])
 def test_two_passes_where_they_are_faster(rank, v_rank, hkv, tokens, two):
     """Both sides as measured beside the lines; v_rank 0: one basis."""
