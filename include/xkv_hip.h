@@ -175,7 +175,10 @@ int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, float* partial,
  *   s[b,h,l]     = sm_scale * q_pe[b,h,:] . K'[b,h/G,l,:]        (K' rounded to the operand dtype)
  *
  * then either scores_out (as above) or the split softmax with V = vA (rank-space partials
- * [batch, hq, max_splits, vA.dim]).  rope == 0 skips the rotation (pure reconstruction).
+ * [batch, hq, max_splits, vA.dim]).  rope == 0 skips the rotation (pure reconstruction); rope == XKV_ROPE_GROUPED is 1 with a hint:
+ * max_splits was chosen for workgroups of several kv heads and holds for every sequence, which are as long as kv_len says (kv_lens
+ * then ends their padding); the kernel for them runs wherever it is built for the shape.  Otherwise it runs where num_kv_splits and kv_lens are NULL
+ * and the splits make it the faster: the work that device counts and lengths leave is not known here.
  * Envelope: head_dim == 128, G = hq/hkv <= 16, rank % 32 == 0, rank <= 512, vA.dim % 64 == 0 <= 512.
  * With computed angles (sin_cos == NULL), G <= 8 and a workspace of xkv_recon_workspace_bytes() the call runs a
  * specialised kernel (kB packed once into the workspace, stationary in registers; v_mfma_f32_32x32x16; direct-to-LDS tile
@@ -191,6 +194,7 @@ int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, float* partial,
  * _qAB_fwd_precomp[grid] at qAB/v2.py:170-186 in scores_out mode; the fused form has no single
  * reference launch - it composes that reconstruction with the stage 1 of
  * fused_attention/no_pe/v1.py:227-262. */
+#define XKV_ROPE_GROUPED 3
 int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void* kB,
                      int64_t stride_kB_b, int64_t stride_kB_h, int64_t stride_kB_r,
                      xkv_kv_operand vA,

@@ -369,11 +369,11 @@ PyObject* nope_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 void recon(const Call& c, Ten q, Ten kA, Ten kB, const at::Tensor* vA, float* partial, float* lse, void* scores, int scores_dtype, int S,
-           int64_t b, int64_t hq, int64_t hkv, int64_t L, float scale, const float* inv, int64_t pos, void* ws, int64_t ws_bytes,
+           bool grouped, int64_t b, int64_t hq, int64_t hkv, int64_t L, float scale, const float* inv, int64_t pos, void* ws, int64_t ws_bytes,
            const int32_t* lens = nullptr) {
   check(p_xkv_recon_stage1(q.data_ptr(), kv(kA, 0, kA.size(2)), kB.data_ptr(), kB.stride(0), kB.stride(1), kB.stride(2),
                            vA ? kv(*vA, 0, vA->size(2)) : NO_KV, partial, lse, scores, scores_dtype, nullptr, lens, b, hq, hkv, L, S,
-                           scale, 1, inv, pos, nullptr, 0, ws, ws_bytes, c.dt, c.stream), "xkv_recon_stage1");
+                           scale, grouped ? XKV_ROPE_GROUPED : 1, inv, pos, nullptr, 0, ws, ws_bytes, c.dt, c.stream), "xkv_recon_stage1");
 }
 void rope_operands(Ten q, int64_t hq, int64_t d, Ten kA, Ten kB, Ten inv) {
   const int64_t b = q.size(0), hkv = kB.size(1), r = kA.size(2);
@@ -392,12 +392,13 @@ int heads_splits(bool packets, int64_t b, int64_t hkv, int64_t G, int64_t L, int
   const int S = balanced_splits(b, hkv / nh, L, 32, 1, cus);
   return b * (hkv / nh) * S >= xkv::RECON_HEADS_WORKGROUPS ? S : 0;
 }
-int score_splits(const Call& c, Ten kB, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r) {
-  if (const int S = heads_splits(rows(kB), b, hkv, G, L, r, true, c.cus)) return S;
+struct ReconSplits { int S; bool grouped; };   // grouped: cut for several kv heads a workgroup
+ReconSplits score_splits(const Call& c, Ten kB, int64_t b, int64_t hkv, int64_t G, int64_t L, int64_t r) {
+  if (const int S = heads_splits(rows(kB), b, hkv, G, L, r, true, c.cus)) return {S, true};
   if (scores_alone(kB, r, G) || xkv::recon_scores_pays(r, hkv, G, b * L))
-    return balanced_splits(b, hkv, L, r <= 256 ? 64 : 32, 1, c.cus);
+    return {balanced_splits(b, hkv, L, r <= 256 ? 64 : 32, 1, c.cus), false};
   const bool resident = ring_rank(r) && G <= 8;
-  return balanced_splits(b, hkv, L, 32, resident || r > 256 ? 1 : r > 128 ? 2 : 3, c.cus);
+  return {balanced_splits(b, hkv, L, 32, resident || r > 256 ? 1 : r > 128 ? 2 : 3, c.cus), false};
 }
 // Scores and P.A in one kernel: one workgroup per CU; two only where the generic kernel, instantiated for the rank, does without a value
 // tile of its own (us at one / two / three workgroups a CU, batch 1, 32 heads on 8, 9000 tokens: rank 64 32 / 42 / 50, rank 128 28 / 26 / 34,
@@ -446,8 +447,9 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t sc = c.plan(b * hq * row * 4), part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
         const int64_t mid = c.plan(rows_first(s.S, hq, up, rv, b) ? rows_bytes(b, hq, rv) : 0);
         if (c.try_alloc()) {
-          recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, score_splits(c, kB, b, hkv, hq / hkv, L, r), b, hq, hkv, row,
-                scale, invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes, s.lens);
+          const ReconSplits scores = score_splits(c, kB, b, hkv, hq / hkv, L, r);
+          recon(c, q, kA, kB, nullptr, nullptr, nullptr, c.get<void>(sc), XKV_F32, scores.S, scores.grouped, b, hq, hkv, row, scale,
+                invp, pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes, s.lens);
           check(p_xkv_softmax_pv_stage1(c.get<float>(sc), kv(vA, 0, rv), c.get<float>(part), c.get<float>(lse), nullptr, s.lens, b, hq, row, s.S,
                                         0, nullptr, c.dt, c.stream), "xkv_softmax_pv_stage1");
           merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, row, rv);
@@ -460,7 +462,7 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int64_t part = c.plan(s.rows(b, hq) * rv * 4), lse = c.plan(s.rows(b, hq) * 4);
       const int64_t mid = c.plan(rows_first(s.S, hq, up, rv, b) ? rows_bytes(b, hq, rv) : 0);
       c.alloc();
-      recon(c, q, kA, kB, &vA, c.get<float>(part), c.get<float>(lse), nullptr, 0, s.S, b, hq, hkv, L, scale, invp, pos,
+      recon(c, q, kA, kB, &vA, c.get<float>(part), c.get<float>(lse), nullptr, 0, s.S, S_heads > 0, b, hq, hkv, L, scale, invp, pos,
             ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
       merge(c, c.get<float>(part), c.get<float>(lse), o.data_ptr(), o.stride(0), o.stride(1), odt, &up, mid, s, b, hq, L, rv);
     });
@@ -485,8 +487,9 @@ PyObject* rope_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, B.stride(0)), ws = c.plan(ws_bytes);
       if (ws_bytes) c.alloc();
       out = at::empty({b, hq, 1, L}, f32 ? c.opts.dtype(at::kFloat) : c.opts);
-      recon(c, q, A, B, nullptr, nullptr, nullptr, out.data_ptr(), f32 ? XKV_F32 : c.dt, score_splits(c, B, b, hkv, hq / hkv, L, r), b, hq, hkv,
-            L, scale, inv.data_ptr<float>(), pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
+      const ReconSplits s = score_splits(c, B, b, hkv, hq / hkv, L, r);
+      recon(c, q, A, B, nullptr, nullptr, nullptr, out.data_ptr(), f32 ? XKV_F32 : c.dt, s.S, s.grouped, b, hq, hkv, L,
+            scale, inv.data_ptr<float>(), pos, ws_bytes ? c.get<void>(ws) : nullptr, ws_bytes);
     });
     return THPVariable_Wrap(out);
   });

@@ -431,10 +431,13 @@ extern "C" int xkv_recon_stage1(const void* q_pe, xkv_kv_operand kA, const void*
   const int64_t need = xkv_recon_workspace_bytes(batch, hkv, rank, sBb);
   const bool spec = rope && !sin_cos && (rank == 512 || rank == 384 || rank == 256) && hq / hkv <= 8 && workspace && need > 0 &&
                     workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && kA.stride_l >= 0 && kA.stride_l < (1 << 25);   // 32-bit row offsets
-  // Several kv heads per workgroup, where the splits make enough of them: a factor of 16-byte packets, and whatever else the wave-specialised kernel asks for
+  // Several kv heads per workgroup, where the caller planned for them or gave splits, known here, that make it the faster.  Counts and lengths on the device are not: where most
+  // of the possible splits are dead it keeps half as many CUs busy as one head a workgroup (us a call, several heads / one, 32 heads on 8: rank 512, lengths (30000, 1000), splits (31, 1)
+  // of 31 59.3 / 47.8; rank 384, (32768, 4000, 2000, 1000), 16 each, 80.0 / 54.6; where all live, 16 x 32768 of 4 each 458 / 534).  A factor of 16-byte packets, and whatever else the
+  // wave-specialised kernel asks for
   const int nh = rope && !sin_cos ? recon_heads(rank, hkv, hq / hkv, so) : 0;
-  if (nh && (so || vshared) && spec && (int64_t)batch * (hkv / nh) * max_splits >= RECON_HEADS_WORKGROUPS &&
-      whole_packets(kB, sBb, sBh, sBr)) {
+  if (nh && (so || vshared) && spec && whole_packets(kB, sBb, sBh, sBr) &&
+      (rope == XKV_ROPE_GROUPED || (!num_kv_splits && !kv_lens && recon_heads_pays(rank, hkv, nh, batch, kv_len, max_splits)))) {
     FastParams f{};
     f.q = q_pe; f.kA = kA.ptr; f.sAb = kA.stride_b; f.sAl = kA.stride_l;
     f.partial = partial; f.lse = lse; f.scores = scores_out; f.scores_dtype = scores_dtype;

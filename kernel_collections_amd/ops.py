@@ -197,6 +197,9 @@ def softmax_pv_stage1(scores, V, partial, lse, num_kv_splits, kv_lens, batch, hq
         "xkv_softmax_pv_stage1")
 
 
+ROPE_GROUPED = 3   # XKV_ROPE_GROUPED: rotation, and splits that were chosen for several kv heads a workgroup
+
+
 def recon_stage1(q3, kA, kB, vA, partial, lse, scores, num_kv_splits, kv_lens, batch, hq, hkv, kv_len, max_splits,
                  sm_scale, rope, inv_freq, pos_offset, sin_cos):
     a_op = kv_operand(kA, kA.stride(0), kA.stride(1), 0, kA.shape[-1])

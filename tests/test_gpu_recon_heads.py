@@ -54,7 +54,7 @@ def test_decode(dev, dtype, r, hkv, G, n, cut):
     kl = torch.tensor(lens, dtype=torch.int32, device=dev)
     part, lse = torch.full((b, hq, S, r), float("nan"), device=dev), torch.full((b, hq, S), float("nan"), device=dev)
     poison()
-    ops.recon_stage1(q, A, B, A, part, lse, None, None, kl, b, hq, hkv, L, S, 128 ** -0.5, True, ops.rope_inv_freq(128, 5e5, q.device), off, None)
+    ops.recon_stage1(q, A, B, A, part, lse, None, None, kl, b, hq, hkv, L, S, 128 ** -0.5, ops.ROPE_GROUPED, ops.rope_inv_freq(128, 5e5, q.device), off, None)
     out = torch.empty((b, hq, r), device=dev)
     ops.merge_stage2(part, lse, out, None, None, kl, b, hq, hq, L, S)
     s = keys_and_scores(q, A, B, off) * 128 ** -0.5
@@ -74,7 +74,7 @@ def test_scores(dev, dtype, out, r, hkv, G, n, cut):
     for _ in range(3):
         s = torch.full((b, hq, 1, L), float("nan"), dtype=out, device=dev)
         poison()
-        ops.recon_stage1(q, A, B, None, None, None, s, None, None, b, hq, hkv, L, S, 0.25, True, ops.rope_inv_freq(128, 5e5, q.device), off, None)
+        ops.recon_stage1(q, A, B, None, None, None, s, None, None, b, hq, hkv, L, S, 0.25, ops.ROPE_GROUPED, ops.rope_inv_freq(128, 5e5, q.device), off, None)
         d = s[:, :, 0].double() - ref
         # The key and the query rounded to fp16 once each: 2.06e-4 of their size over all mantissas, together 2.9e-4; the result in fp16 as much more.  Angles in fp32
         # up to position 25000: half a unit, 2^-10 radians, at the fastest pairs, half of that on average over tokens and 1 / 64 .. of the pairs: 1e-4.
@@ -89,7 +89,7 @@ def test_scores_of_large_and_small_queries(dev, scale):
     A *= 0.02
     q = q.sign() * scale if scale > 1 else q * scale
     s = torch.empty((1, 8, 1, 6144), device=dev)
-    ops.recon_stage1(q, A, B, None, None, None, s, None, None, 1, 8, 2, 6144, 192, 1.0, True, ops.rope_inv_freq(128, 5e5, q.device), 0, None)
+    ops.recon_stage1(q, A, B, None, None, None, s, None, None, 1, 8, 2, 6144, 192, 1.0, ops.ROPE_GROUPED, ops.rope_inv_freq(128, 5e5, q.device), 0, None)
     ref = keys_and_scores(q, A, B, 0)
     assert (s[:, :, 0].double() - ref).norm() <= 4e-4 * ref.norm()
 
@@ -115,7 +115,7 @@ def test_decode_of_large_and_small_queries(dev, dtype, size, r, hkv, S):
     scale = 0.25 / size if size else 1.0
     part, lse = torch.full((1, hkv * G, S, r), float("nan"), device=dev), torch.full((1, hkv * G, S), float("nan"), device=dev)
     poison()
-    ops.recon_stage1(q, A, B, A, part, lse, None, None, None, 1, hkv * G, hkv, L, S, scale, True, ops.rope_inv_freq(128, 5e5, q.device), off, None)
+    ops.recon_stage1(q, A, B, A, part, lse, None, None, None, 1, hkv * G, hkv, L, S, scale, ops.ROPE_GROUPED if S > 2 else True, ops.rope_inv_freq(128, 5e5, q.device), off, None)
     out, total = torch.empty((1, hkv * G, r), device=dev), torch.empty((1, hkv * G), device=dev)
     ops.merge_stage2(part, lse, out, None, None, None, 1, hkv * G, hkv * G, L, S, total)
     s = keys_and_scores(q, A, B, off) * scale
@@ -144,7 +144,7 @@ def test_scores_of_decode_at_rank_256(dev):
     r, hkv, G, L, S, scale = 256, 4, 4, 6144, WORKGROUPS, 4.0
     q, A, B = operands(dev, BF, 1, hkv, G, L, r, r)
     part, lse = torch.empty((1, hkv * G, S, r), device=dev), torch.empty((1, hkv * G, S), device=dev)
-    ops.recon_stage1(q, A, B, A, part, lse, None, None, None, 1, hkv * G, hkv, L, S, scale, True, ops.rope_inv_freq(128, 5e5, q.device), 0, None)
+    ops.recon_stage1(q, A, B, A, part, lse, None, None, None, 1, hkv * G, hkv, L, S, scale, ops.ROPE_GROUPED, ops.rope_inv_freq(128, 5e5, q.device), 0, None)
     s = keys_and_scores(q, A, B, 0) * scale
     err = lse - torch.logsumexp(s.reshape(1, hkv * G, S, L // S), -1)
     # The key and the query rounded to fp16 once each: 2.9e-4 of the scores' size (3072 rows: within 2 %); rotated in fp16 besides, with cosines of 16 bits, 3.9e-4
@@ -157,7 +157,7 @@ def test_the_largest_weight_at_rank_256_is_exact(dev):
     L = 32 * n * S
     q, A, B = operands(dev, BF, 1, hkv, G, L, r, r)
     part, lse = torch.empty((1, hkv * G, S, r), device=dev), torch.empty((1, hkv * G, S), device=dev)
-    ops.recon_stage1(q, A, B, A, part, lse, None, None, None, 1, hkv * G, hkv, L, S, scale, True, ops.rope_inv_freq(128, 5e5, q.device), 0, None)
+    ops.recon_stage1(q, A, B, A, part, lse, None, None, None, 1, hkv * G, hkv, L, S, scale, ops.ROPE_GROUPED, ops.rope_inv_freq(128, 5e5, q.device), 0, None)
     s = (keys_and_scores(q, A, B, 0) * scale).reshape(hkv * G, S, 32 * n)
     top = s.topk(2, -1).values
     gap = top[..., 0] - top[..., 1]
@@ -166,3 +166,25 @@ def test_the_largest_weight_at_rank_256_is_exact(dev):
     err = (part[0] - ref[:, :, 0]).norm(dim=-1) / ref[:, :, 0].norm(dim=-1)
     # the others: a few e^-8, times the error of their scores, 3e-4 of 57; a weight of 1 to 2 in bf16 would be 1e-3 off
     assert close.sum() > 500 and err[close].max() <= 2e-4
+
+
+def test_several_heads_where_the_splits_are_known(dev):
+    """Counts or lengths on the device, splits that leave a round half empty and short calls keep one kv head a workgroup, as a factor at an odd place does."""
+    r, hkv, G = 512, 8, 4
+
+    def call(L, S, odd=False, counts=None, lens=None, rope=True):
+        q, A, B = operands(dev, BF, 1, hkv, G, L, r, r)
+        if odd:
+            B = torch.empty(B.numel() + 4, dtype=BF, device=dev)[4:].view(B.shape).copy_(B)
+        part, lse = torch.zeros((1, hkv * G, S, r), device=dev), torch.zeros((1, hkv * G, S), device=dev)
+        to = lambda n: None if n is None else torch.tensor([n], dtype=torch.int32, device=dev)
+        ops.recon_stage1(q, A, B, A, part, lse, None, to(counts), to(lens), 1, hkv * G, hkv, L, S, 128 ** -0.5, rope, ops.rope_inv_freq(128, 5e5, q.device), 0, None)
+        return part
+
+    one = call(28672, 64, odd=True)      # a copy of the factor: never several heads
+    assert torch.equal(call(28672, 64, counts=64), one) and torch.equal(call(28672, 64, lens=28672), one)
+    several = call(28672, 64, rope=ops.ROPE_GROUPED)
+    assert not torch.equal(several, one) and torch.equal(call(28672, 64), several)      # one round of 256 workgroups, or two of 512
+    assert torch.equal(call(28672, 64, lens=28672, rope=ops.ROPE_GROUPED), several)
+    assert torch.equal(call(30720, 80), call(30720, 80, odd=True))                       # 320 in two rounds, or 640 in three
+    assert torch.equal(call(20480, 64), call(20480, 64, odd=True))                       # short
