@@ -628,7 +628,7 @@ PyObject* prefix_tail(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int blocks = cdiv(Lt, 32), per = cdiv(blocks, join ? 32 : 4), S2 = cdiv(blocks, per), rows2 = S2 + (join ? 0 : 1);
       const bool first = xkv::merge_tail_rows_first(s1.S, hq, up.hkv, rv);
       const int64_t hi = c.plan(b * hq * r * 2), lo = c.plan(b * hq * r * 2), part1 = c.plan(b * hq * s1.S * rv * 4), lse1 = c.plan(b * hq * s1.S * 4);
-      const int64_t mid = c.plan(first ? rows_bytes(b, hq, rv) : 0), part2 = c.plan(b * hq * rows2 * dv * 4), lse2 = c.plan(b * hq * rows2 * 4);
+      const int64_t mid = c.plan((join ? first : rows_first(s1.S, hq, up, rv, b)) ? rows_bytes(b, hq, rv) : 0), part2 = c.plan(b * hq * rows2 * dv * 4), lse2 = c.plan(b * hq * rows2 * 4);
       c.alloc();
       o = at::empty({b, hq, dv}, c.opts);
       // the query absorbed and the tail attended to in one launch: neither depends on the other
@@ -678,6 +678,10 @@ PyObject* py_head_rows_floor(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_recon_scores_pays(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 4, [&]() -> PyObject* { return PyBool_FromLong(xkv::recon_scores_pays(I(a[0]), I(a[1]), I(a[2]), I(a[3]))); });
 }
+// merge_rows_first(splits, heads, kv heads, width, batch, columns) -> bool (merge_rule.h)
+PyObject* py_merge_rows_first(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 6, [&]() -> PyObject* { return PyBool_FromLong(xkv::merge_rows_first(I(a[0]), I(a[1]), I(a[2]), I(a[3]), I(a[4]), I(a[5]))); });
+}
 // split_floor(batch, groups, kv_len, per_cu, cus, up) -> int
 PyObject* py_split_floor(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 6, [&]() -> PyObject* { return PyLong_FromLong(split_floor(I(a[0]), I(a[1]), I(a[2]), I(a[3]), I(a[4]), I(a[5]))); });
@@ -722,6 +726,7 @@ PyMethodDef methods[] = {
     {"init", init, METH_O, nullptr},       XKV_FAST("balanced_splits", py_balanced_splits), XKV_FAST("nope_decode", nope_decode), XKV_FAST("ragged_target", py_ragged_target),
     XKV_FAST("split_floor", py_split_floor), XKV_FAST("decode_splits", py_decode_splits), XKV_FAST("head_rows", py_head_rows),
     XKV_FAST("head_rows_floor", py_head_rows_floor), XKV_FAST("recon_scores_pays", py_recon_scores_pays),
+    XKV_FAST("merge_rows_first", py_merge_rows_first),
     XKV_FAST("nope_scores", nope_scores),  XKV_FAST("rope_decode", rope_decode),            XKV_FAST("rope_scores", rope_scores),
     XKV_FAST("gqa", gqa),                  XKV_FAST("mla", mla),                            XKV_FAST("prefix_tail", prefix_tail),
     {nullptr, nullptr, 0, nullptr}};

@@ -29,12 +29,12 @@ inline bool merge_spread(int64_t splits, int64_t hq, int64_t batch, int64_t dv, 
 // 512 6.0 / 4.8; 32 on 1, d_out 512, one of 512 5.9 / 4.9; batch 4, 7 splits of 512 6.3 / 5.1; batch 5, one of 512 5.9 / 6.6, batch 16 6.2 / 11.3
 inline bool merge_one_head(int64_t hq, int64_t batch, int d_out) { return merge_blocks(hq, batch, d_out) <= 256; }
 
-// Partial values that a workgroup may fold in every column block, one head of it (SPREAD) or all; beyond, the rows are merged first, by the whole chip.  us of one kernel
+// Partial values that a workgroup may fold in every column block, of one head (dealt out) or of all of its heads; beyond, the rows are merged first, by the whole chip.  us of one kernel
 // / rows and up-projection: dealt out, batch 1, 128 splits of 512 9.5 / 10.2, 256 of 256 8.6 / 9.7, 256 of 384 11.7 / 11.0, 16 on 2, 128 of 512 8.3 / 8.7; a thread all splits, batch
 // 8, 32 of 512 (65536 values) 9.6 / 11.9, 16 on 1, d_out 512, batch 8, 32 of 256 (32768) 7.0 / 7.7, batch 16, 16 of 256 (32768) 7.2 / 9.1
-constexpr int64_t MERGE_SPREAD_FLOATS = 65536, MERGE_FLOATS = 65536;
+constexpr int64_t MERGE_FLOATS = 65536;
 inline bool merge_rows_first(int64_t splits, int64_t hq, int hkv, int64_t dv, int64_t batch, int d_out) {
-  if (merge_spread(splits, hq, batch, dv, d_out)) return splits * dv > MERGE_SPREAD_FLOATS;
+  if (merge_spread(splits, hq, batch, dv, d_out)) return splits * dv > MERGE_FLOATS;
   return splits > 1 && splits * merge_heads(hq, hkv, dv, batch, d_out) * dv > MERGE_FLOATS;
 }
 

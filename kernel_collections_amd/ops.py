@@ -219,28 +219,17 @@ def recon_stage1(q3, kA, kB, vA, partial, lse, scores, num_kv_splits, kv_lens, b
         "xkv_recon_stage1")
 
 
-def _merge_rows_first(splits, batch, hq, hkv, dv, d_out):
-    """merge_rows_first of csrc/merge_rule.h, where its lines were measured: more splits than a workgroup should fold in every column block."""
-    if splits <= 1:
-        return False
-    blocks = -(-d_out // 64)
-    if splits * dv >= 4096 and hq * batch * blocks <= 256:      # one head a workgroup
-        return splits * dv > 65536
-    hpw = g = hq // hkv
-    while hpw > 1 and (g % hpw or hpw * dv * 4 > 48 * 1024):
-        hpw -= 1
-    while hpw > 4 and hpw % 2 == 0 and hq // hpw * batch * blocks < 256:
-        hpw //= 2
-    return splits * hpw * dv > 65536
-
-
 def merge_stage2(partial, lse, out, vB, num_kv_splits, kv_lens, batch, hq, hkv, kv_len, max_splits, lse_out=None, split_cap=0,
                  split_plan=None):
     """out `[b,Hq,*]` (strides honoured on the first two axes).  `lse_out` `[b,Hq]` (any strides, fp32): log-sum-exp
     of the merged range.  Up-projections wider than 512 columns run as column blocks of 512."""
     dv = partial.shape[-1]
     seq_splits = max_splits if split_plan is None or num_kv_splits is not None else _cdiv(kv_len, split_cap)
-    if vB is not None and _merge_rows_first(seq_splits, batch, hq, hkv, dv, vB.shape[-1]):
+    if vB is not None and hkv == 1 and hq > 32:   # at most 32 query heads per kv head in the up-projecting merge: the shared matrix as several heads
+        hkv = head_groups(hq)
+        vB = vB.expand(-1, hkv, -1, -1)
+    from . import _xkv_host
+    if vB is not None and _xkv_host.merge_rows_first(seq_splits, hq, hkv, dv, batch, min(vB.shape[-1], 512)):
         # many splits: merge the rows first, spread over the chip, then up-project one row per head
         mid, mid_lse = torch.empty((batch, hq, dv), dtype=torch.float32, device=partial.device), lse_out
         if mid_lse is None:
@@ -261,9 +250,6 @@ def merge_stage2(partial, lse, out, vB, num_kv_splits, kv_lens, batch, hq, hkv, 
     if vB is None:
         call(out, None, dv, (0, 0, 0), _lib.XKV_BF16, lse_out)
         return out
-    if hkv == 1 and hq > 32:   # at most 32 query heads per kv head in the up-projecting merge: the shared matrix as several heads
-        hkv = head_groups(hq)
-        vB = vB.expand(-1, hkv, -1, -1)
     vB = as_rows(vB)
     sv, vdt = (vB.stride(0), vB.stride(1), vB.stride(2)), dtype_code(vB.dtype)
     for c0 in range(0, vB.shape[-1], 512):

@@ -202,6 +202,25 @@ def test_scores_by_independent_waves_where_they_are_faster(rank, hkv, G, tokens,
     assert _xkv_host.recon_scores_pays(rank, hkv, G, tokens) == pays
 
 
+@pytest.mark.parametrize("batch,hq,hkv,S,dv,d_out,launches", [
+    (1, 32, 8, 128, 512, 128, 1), (1, 32, 8, 129, 512, 128, 2), (8, 32, 8, 32, 512, 128, 1), (8, 32, 8, 33, 512, 128, 2),
+    (1, 32, 8, 33, 512, 1024, 2),      # two blocks of 512 columns, the splits of a head dealt out in each
+    (2, 40, 1, 25, 512, 512, 1), (2, 40, 1, 26, 512, 512, 2)])      # 40 heads of one kv head: groups of 20, folded five at a time
+def test_merge_takes_rows_first_by_the_native_rule(batch, hq, hkv, S, dv, d_out, launches, monkeypatch):
+    calls = []
+
+    class Library:
+        def xkv_merge_stage2(self, *args):
+            calls.append(args)
+            return 0
+    monkeypatch.setattr(ops._lib, "lib", lambda: Library())
+    monkeypatch.setattr(ops, "stream_ptr", lambda t: None)
+    z = lambda *s: torch.zeros(s, dtype=torch.bfloat16)
+    ops.merge_stage2(torch.zeros(1).expand(batch, hq, S, dv), torch.zeros(1).expand(batch, hq, S), z(batch, hq, d_out), z(1, hkv, dv, d_out).expand(batch, -1, -1, -1), None, None, batch, hq,
+                     hkv, 32 * S, S)
+    assert len(calls) == launches
+
+
 @pytest.mark.parametrize("batch,groups,per_cu,jobs", [(1, 1, 1, 256), (32, 1, 1, 256), (128, 1, 1, 256), (129, 1, 1, 512), (64, 8, 2, 128),
                                                      (65, 8, 2, 192), (3, 300, 1, 6), (5, 512, 2, 10)])
 def test_ragged_batches_get_two_jobs_a_sequence(batch, groups, per_cu, jobs):
