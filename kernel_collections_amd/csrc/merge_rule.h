@@ -38,7 +38,9 @@ inline bool merge_rows_first(int64_t splits, int64_t hq, int hkv, int64_t dv, in
   return splits > 1 && splits * merge_heads(hq, hkv, dv, batch, d_out) * dv > MERGE_FLOATS;
 }
 
-// The same with a tail's rows beside them (xkv_merge_stage2_tail), which one workgroup folds for all heads of a kv head
+// The same with a tail's rows beside them (xkv_merge_stage2_tail), whose splits no form deals out: a thread folds all of a packet's.  The line counts all heads of a kv head also where a
+// workgroup takes one (merge_one_head), for which it lies early: us of a call, 32 heads on one matrix, batch 1, rank 512, tail 128, one kernel / rows first, 8 splits 23.5 / 26.7, 16 24.5 / 27.1,
+// 32 26.6 / 28.0, and 64, from 2048 tokens of prefix on, 30.8 / 29.4 (rank 256 22.0 / 21.0; 4 x 8 heads 26.3 / 25.0)
 constexpr int64_t MERGE_TAIL_FLOATS = 49152;
 inline bool merge_tail_rows_first(int64_t splits, int64_t hq, int hkv, int64_t dv) { return splits > 1 && splits * (hq / hkv) * dv > MERGE_TAIL_FLOATS; }
 

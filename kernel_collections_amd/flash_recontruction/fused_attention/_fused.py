@@ -186,7 +186,7 @@ def decode_rope(q_pe, k_A, k_B, v_A, v_B, o, num_kv_splits, max_kv_splits, sm_sc
         # shared-basis fused kernel (one row stream, no P.A); softmax and P.v_A then stream v_A once for all heads at HBM
         # rate.  Fused into one kernel, the second row stream costs more than the 2 x 4 bytes per score this moves.
         # the scores do not depend on how pass 1 cuts the range: one round of workgroups per CU
-        S1 = ops.occupancy_splits(batch, hkv, kv_len, tile=64 if k_A.shape[-1] <= 256 else 32, waves=1)
+        S1 = ops.occupancy_splits(batch, hkv, kv_len, tile=ops.scores_tile(k_A.shape[-1], hkv, hq // hkv, batch * kv_len), waves=1)
         ops.recon_stage1(q3, k_A, k_B, None, None, None, scores, None, lens, batch, hq,
                          hkv, kv_len, S1, float(sm_scale), True, inv, int(pos_offset), None)
         S2 = ops.latent_splits(batch, 1, kv_len, rank_v, absorbed=True)

@@ -49,12 +49,12 @@ def _scores(q, Ak, Bk, inv_freq, sin_cos, pos_offset, sm_scale, out_dtype):
     Ak = ops.as_rows(Ak)
     Bk = Bk if Bk.stride(-1) == 1 else Bk.contiguous()
     out = torch.empty((bsz, num_heads, 1, kv_len), dtype=out_dtype, device=q.device)
-    # one workgroup per CU that takes 64 tokens a step, 32 beyond rank 256; with a table, or more than eight heads per kv head beyond rank 224, or
-    # where a factor that is not 16-byte packets finds no workspace, the register-staged scores kernel, which keeps 2-3 up to rank 256
+    # one workgroup per CU, of 64 tokens a step where independent waves take the scores at ranks up to 256, of 32 otherwise; with a table, or more than eight heads per kv head beyond rank
+    # 224, or where a factor that is not 16-byte packets finds no workspace, the register-staged scores kernel, which keeps 2-3 up to rank 256
     G = num_heads // num_kv_heads
     packed = ops.USE_RECON_WORKSPACE and G <= 8 and rank in (256, 384, 512)
     if sin_cos is None and (packed or (ops._row_ok(Bk) and (rank <= 224 or (G <= 8 and rank in (320, 448))))):
-        n_splits = ops.occupancy_splits(bsz, num_kv_heads, kv_len, tile=64 if rank <= 256 else 32, waves=1)
+        n_splits = ops.occupancy_splits(bsz, num_kv_heads, kv_len, tile=ops.scores_tile(rank, num_kv_heads, G, bsz * kv_len), waves=1)
     else:
         n_splits = ops.occupancy_splits(bsz, num_kv_heads, kv_len, tile=32, waves=1 if rank > 256 else (2 if rank > 128 else 3))
     ops.recon_stage1(q3, Ak, Bk, None, None, None, out, None, None, bsz, num_heads, num_kv_heads, kv_len,

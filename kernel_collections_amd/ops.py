@@ -283,6 +283,12 @@ def decode_splits(batch: int, hkv: int, kv_len: int, rank: int, shared: bool) ->
     return _xkv_host.decode_splits(batch, hkv, kv_len, rank, shared, num_cus())
 
 
+def scores_tile(rank: int, hkv: int, G: int, tokens: int) -> int:
+    """Tokens a step of the kernel that takes the scores of rotated keys: 64 of independent waves (`csrc/recon_groups.h` at rank 256), else 32."""
+    from . import _xkv_host
+    return 64 if rank <= 224 or _xkv_host.recon_scores_pays(rank, hkv, G, tokens) else 32
+
+
 def split_floor(batch: int, groups: int, kv_len: int, per_cu: int, up: bool) -> int:
     """Shortest split in tokens (`split_floor` in csrc/host.cpp); `up`: the merged rows are up-projected."""
     from . import _xkv_host

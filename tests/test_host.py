@@ -202,6 +202,19 @@ def test_scores_by_independent_waves_where_they_are_faster(rank, hkv, G, tokens,
     assert _xkv_host.recon_scores_pays(rank, hkv, G, tokens) == pays
 
 
+@pytest.mark.parametrize("rank,hkv,L,tile", [(256, 8, 1000, 32), (256, 2, 20000, 32), (256, 4, 50000, 64), (192, 8, 1000, 64), (384, 8, 2500, 32)])
+def test_scores_of_the_general_path_are_cut_for_the_kernel_that_runs(rank, hkv, L, tile, monkeypatch):
+    from kernel_collections_amd import _xkv_host
+    import kernel_collections_amd.flash_recontruction as fr
+    given = []
+    monkeypatch.setattr(ops, "recon_stage1", lambda *args: given.append(args[13]))
+    monkeypatch.setattr(_lib, "require_gpu", lambda t: None)
+    z = lambda *s: torch.zeros(s, dtype=torch.bfloat16)
+    fr.qAB_rope_v1(z(1, 4 * hkv, 1, 128), z(1, L, rank), z(1, hkv, rank, 128), 5e5)
+    cut = lambda t: _xkv_host.balanced_splits(1, hkv, L, t, 1, ops.num_cus())
+    assert given == [cut(tile)] and cut(tile) != cut(96 - tile)
+
+
 @pytest.mark.parametrize("batch,hq,hkv,S,dv,d_out,launches", [
     (1, 32, 8, 128, 512, 128, 1), (1, 32, 8, 129, 512, 128, 2), (8, 32, 8, 32, 512, 128, 1), (8, 32, 8, 33, 512, 128, 2),
     (1, 32, 8, 33, 512, 1024, 2),      # two blocks of 512 columns, the splits of a head dealt out in each
