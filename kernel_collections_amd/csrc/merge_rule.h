@@ -30,12 +30,25 @@ inline bool merge_spread(int64_t splits, int64_t hq, int64_t batch, int64_t dv, 
 inline bool merge_one_head(int64_t hq, int64_t batch, int d_out) { return merge_blocks(hq, batch, d_out) <= 256; }
 
 // Partial values that a workgroup may fold in every column block, of one head (dealt out) or of all of its heads; beyond, the rows are merged first, by the whole chip.  us of one kernel
-// / rows and up-projection: dealt out, batch 1, 128 splits of 512 9.5 / 10.2, 256 of 256 8.6 / 9.7, 256 of 384 11.7 / 11.0, 16 on 2, 128 of 512 8.3 / 8.7; a thread all splits, batch
-// 8, 32 of 512 (65536 values) 9.6 / 11.9, 16 on 1, d_out 512, batch 8, 32 of 256 (32768) 7.0 / 7.7, batch 16, 16 of 256 (32768) 7.2 / 9.1
+// / rows and up-projection: dealt out, batch 1, 128 splits of 512 9.5 / 10.2, 256 of 256 8.6 / 9.7, 256 of 384 11.7 / 11.0, 16 on 2, 128 of 512 8.3 / 8.7
 constexpr int64_t MERGE_FLOATS = 65536;
+// Where a thread folds all splits of its packets one after another, every column block reads them again: out of the same XCD's L2 if the blocks of a head lie on one (workgroups go round-robin
+// over the 8 XCDs, heads and sequences first), else from memory.  With more than 16 splits that decides earlier, and so do, of more than two blocks, a second round of workgroups and more than 48 splits.
+// us of a whole call, one kernel / rows and up-projection, 512 columns.  On one XCD, 16 on 1, 6 sequences, 40 splits of 384 (61440 values) 30.4 / 31.8, 8, 30 of 512 (61440) 33.9 / 35.4, 4, 59 of 256
+// (60416) 27.4 / 25.9; 32 on 1, 5, 47 of 256 (48128) by 0.7, 12, 20 of 256 (40960) by 1.6 one kernel, 7, 34 of 384 (52224) 36.6 / 35.8.  Apart, 16 on 1, 9, 27 of 256 (27648) 0.1, of 384 (41472)
+// 36.2 / 34.2, 13, 19 of 384 (29184) 35.9 / 35.0, 7, 34 of 256 (34816) 26.9 / 26.3, of 384 33.0 / 31.8, 27, 9 of 512 (36864) 42.8 / 44.2, 17, 14 of 512 (57344) by 0.9 one kernel; 16 on 2, 128 columns, 9, 28 of 384 (43008) 46.9 / 46.4,
+// 17, 14 of 512 (28672) 46.9 / 48.9
+constexpr int64_t MERGE_FLOATS_APART = 28672, MERGE_FLOATS_ROUNDS = 49152;
 inline bool merge_rows_first(int64_t splits, int64_t hq, int hkv, int64_t dv, int64_t batch, int d_out) {
+  if (splits <= 1) return false;
   if (merge_spread(splits, hq, batch, dv, d_out)) return splits * dv > MERGE_FLOATS;
-  return splits > 1 && splits * merge_heads(hq, hkv, dv, batch, d_out) * dv > MERGE_FLOATS;
+  const int hpw = merge_heads(hq, hkv, dv, batch, d_out);
+  const int64_t values = splits * hpw * dv;
+  if (splits <= 16) return values > MERGE_FLOATS;
+  const bool apart = d_out > MERGE_CB && hq / hpw * batch % 8;
+  if (apart) return values > MERGE_FLOATS_APART;
+  const bool rounds = d_out > 2 * MERGE_CB && (splits > 48 || merge_blocks(hq / hpw, batch, d_out) > 256);
+  return values > (rounds ? MERGE_FLOATS_ROUNDS : MERGE_FLOATS);
 }
 
 // The same with a tail's rows beside them (xkv_merge_stage2_tail), whose splits no form deals out: a thread folds all of a packet's.  The line counts all heads of a kv head also where a

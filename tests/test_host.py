@@ -218,7 +218,9 @@ def test_scores_of_the_general_path_are_cut_for_the_kernel_that_runs(rank, hkv, 
 @pytest.mark.parametrize("batch,hq,hkv,S,dv,d_out,launches", [
     (1, 32, 8, 128, 512, 128, 1), (1, 32, 8, 129, 512, 128, 2), (8, 32, 8, 32, 512, 128, 1), (8, 32, 8, 33, 512, 128, 2),
     (1, 32, 8, 33, 512, 1024, 2),      # two blocks of 512 columns, the splits of a head dealt out in each
-    (2, 40, 1, 25, 512, 512, 1), (2, 40, 1, 26, 512, 512, 2)])      # 40 heads of one kv head: groups of 20, folded five at a time
+    (2, 40, 1, 25, 512, 512, 1), (2, 40, 1, 26, 512, 512, 2),       # 40 heads of one kv head: groups of 20, folded five at a time
+    (9, 16, 1, 27, 384, 512, 2), (8, 16, 1, 30, 512, 512, 1), (17, 16, 1, 14, 512, 512, 1), (9, 16, 1, 27, 256, 512, 1),     # column blocks of a head on two XCDs, or on one; few splits
+    (7, 32, 1, 34, 384, 512, 2), (12, 32, 1, 20, 256, 512, 1), (4, 16, 1, 59, 256, 512, 2), (9, 16, 2, 28, 384, 128, 2), (9, 32, 8, 28, 512, 128, 1)])
 def test_merge_takes_rows_first_by_the_native_rule(batch, hq, hkv, S, dv, d_out, launches, monkeypatch):
     calls = []
 
