@@ -181,14 +181,12 @@ int xkv_softmax_pv_stage1(const float* scores, xkv_kv_operand V, float* partial,
  * and the splits make it the faster: the work that device counts and lengths leave is not known here.
  * Envelope: head_dim == 128, G = hq/hkv <= 16, rank % 32 == 0, rank <= 512, vA.dim % 64 == 0 <= 512.
  * With computed angles (sin_cos == NULL), G <= 8 and a workspace of xkv_recon_workspace_bytes() the call runs a
- * specialised kernel (kB packed once into the workspace, stationary in registers; v_mfma_f32_32x32x16; direct-to-LDS tile
- * rings): at ranks 256 / 384 / 512 with vA the same tensor as kA the wave-specialised kernel (four
- * reconstruction waves in a 2 x 2 rank/feature split hand fp16 key tiles to four waves that rotate, score, soften and
- * accumulate P.A), with scores_out at rank 512 and, where G > 4, 384; at those ranks with a separate vA of rank 256 / 384 / 512 the 8-wave
- * kernel (2 x 4 split, second row stream for vA); other scores_out at ranks 256 and 384 with a factor of 16-byte packets independent waves, one or two
- * to 16 tokens, which read kB as it is.  These hold the rotated query as one fp16 value, beside the keys' rounding to fp16 (scores within 2.9e-4 .. 4.4e-4 of
- * float64 against 2.1e-4).  Without a workspace: independent waves with a query of two parts for scores_out at ranks up to 224 (G <= 16), 320 and 448
- * (G <= 8); otherwise the generic kernel, whose query is not rotated.
+ * specialised kernel (kB stationary in registers, read as it is where it is 16-byte packets, else copied into the workspace; v_mfma_f32_32x32x16; direct-to-LDS
+ * tile rings): at ranks 256 / 384 / 512 with vA the same tensor as kA, and with scores_out, several kv heads a workgroup or the wave-specialised kernel (four
+ * waves rebuild, rotate and score, four soften and accumulate P.A); at those ranks with a separate vA of rank 256 / 384 / 512 the 8-wave
+ * kernel (2 x 4 split, second row stream for vA); long scores_out at rank 256 independent waves, one to 16 tokens.  These hold the rotated query as one fp16
+ * value, beside the keys' rounding to fp16 (scores_out within 2.9e-4 of float64 against 2.1e-4).  Without a workspace: independent waves with a query of two parts for
+ * scores_out at ranks up to 224 (G <= 16), 320 and 448 (G <= 8); otherwise the generic kernel, whose query is not rotated.
  * Computed angles rotate the query in most of these kernels: one that holds an infinity or a NaN gives scores that are no numbers.
  * Replaces _qAB_fwd[grid] at flash_recontruction/qAB/v1.py:135-145 (v3.py / v4.py / ref.py twins) and
  * _qAB_fwd_precomp[grid] at qAB/v2.py:170-186 in scores_out mode; the fused form has no single
@@ -223,7 +221,8 @@ int64_t xkv_recon_workspace_bytes(int batch, int hkv, int rank, int64_t stride_k
  * The FIRST call on a device for a given kernel shape does host-side set-up (the array's address is looked up with
  * hipGetSymbolAddress, the kernel's dynamic LDS size is raised with hipFuncSetAttribute): make one warm-up call per device
  * and shape outside stream capture before capturing.  XKV_ESCRATCH is returned only for shapes that would take a path that
- * may copy kB (generated RoPE angles, at most 8 query heads per kv head); other shapes run the generic kernel without scratch.
+ * may copy kB (generated RoPE angles, at most 8 query heads per kv head), by their size, also where kB is 16-byte packets and would not be copied; other
+ * shapes run the generic kernel without scratch.
  * No counterpart in the reference, whose wrappers allocate with torch.empty on every call
  * (flash_recontruction/fused_attention/no_pe/v1.py:434-446). */
 #define XKV_STATIC_SCRATCH_BYTES (4 << 20)

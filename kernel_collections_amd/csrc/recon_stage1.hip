@@ -533,8 +533,8 @@ extern "C" int xkv_recon_stage1_static(const void* q_pe, xkv_kv_operand kA, cons
                                        int64_t sc_stride_l, int dtype, void* stream) {
   if (batch <= 0 || hkv <= 0) return XKV_EINVAL;
   int64_t need = xkv_recon_workspace_bytes(batch, hkv, kA.dim, sBb);
-  // only the MFMA-bound paths (generated angles, at most 8 query heads per kv head) pack kB; every other shape runs the
-  // generic kernel, which needs no scratch
+  // only the MFMA-bound paths (generated angles, at most 8 query heads per kv head) may copy kB; every other shape runs the
+  // generic kernel, which needs no scratch.  A shape that may is refused by its size, whether its strides ask for the copy or not
   if (!(rope && !sin_cos && hq > 0 && hq % hkv == 0 && hq / hkv <= 8)) need = 0;
   if (need > (int64_t)XKV_STATIC_SCRATCH_BYTES) return XKV_ESCRATCH;   // nothing is launched
   void* ws = nullptr;

@@ -132,10 +132,30 @@ def test_recon_scores_small_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, of
     (1, 8, 2, 640, 512, 1, None, 99999),        # whole steps only, angles seeded twice
 ])
 def test_recon_scores_large_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, off, monkeypatch):
-    if r in (384, 512):    # with a workspace the wave-specialised kernel (at rank 384 beyond four heads per kv head), without one the generic one
+    if r in (384, 512):    # with a workspace the wave-specialised kernel, as at rank 256 in calls this short, without one the generic one
         test_recon_scores_small_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, off)
         monkeypatch.setattr(ops, "USE_RECON_WORKSPACE", False)
     test_recon_scores_small_ranks(dev, dtype, out, b, hq, hkv, L, r, S, lens, off)
+
+
+@pytest.mark.parametrize("dtype,out", [(BF, torch.float32), (FP, FP), (BF, BF)])
+@pytest.mark.parametrize("G,S,L", [(1, 1, 4096), (4, 1, 4097), (5, 3, 4096), (8, 2, 4098)])
+def test_recon_scores_rank_256(dev, dtype, out, G, S, L):
+    """Ends of steps and groups where the call, by the rows it may have, is long enough for the independent waves; rows past a sequence are NaN."""
+    from kernel_collections_amd import _xkv_host
+    from test_gpu_recon_heads import keys_and_scores
+    lens, hkv, off = [1, 97, 131, 259, 64, 1123, 65, L], 4, 131072 - 4096
+    b, hq, r = len(lens), hkv * G, 256
+    assert _xkv_host.recon_scores_pays(r, hkv, G, b * L)
+    q, B = gen((b, hq, 128), std=0.5, dtype=dtype, seed=1).to(dev), gen((b, hkv, r, 128), std=r ** -0.5, dtype=dtype, seed=3).to(dev)
+    A = gen((b, L, r), dtype=dtype, seed=2).to(dev)
+    ref = 0.25 * keys_and_scores(q, A, B, off)
+    for i, n in enumerate(lens):
+        A[i, n:] = float("nan")
+    s = torch.full((b, hq, 1, L), float("nan"), dtype=out, device=dev)
+    ops.recon_stage1(q, A, B, None, None, None, s, None, torch.tensor(lens, dtype=torch.int32, device=dev), b, hq, hkv, L, S, 0.25, True, ops.rope_inv_freq(128, 5e5, q.device), off, None)
+    for i, n in enumerate(lens):
+        check_scores(s[i, ..., :n].cpu(), ref[i, :, None, :n].float().cpu(), f"{n} tokens")
 
 
 @pytest.mark.parametrize("hkv,r", [(4, 384), (1, 320), (4, 448)])

@@ -57,8 +57,37 @@ def test_decode_over_any_layout_of_the_factor(dev, rk, rv, G, dtype, how):
 
 
 @pytest.mark.parametrize("how", LAYOUTS)
+@pytest.mark.parametrize("r,hkv,G,dtype", [(512, 2, 8, BF), (384, 4, 3, FP), (256, 4, 4, BF)])
+def test_several_heads_over_any_layout_of_the_factor(dev, r, hkv, G, dtype, how):
+    """Splits cut for several kv heads a workgroup: whole packets bit-equal to the call over a contiguous factor, others by the kernel of one head a workgroup over a copy."""
+    b, S, off = 2, 8, 9
+    L, hq = 32 * 5 * S - 7, hkv * G
+    q, A = gen((b, hq, 128), std=0.5, dtype=dtype, seed=1).to(dev), gen((b, L, r), dtype=dtype, seed=2).to(dev)
+    B = gen((1 if how == LAYOUTS[1] else b, hkv, r, 128), std=r ** -0.5, dtype=dtype, seed=3).to(dev).expand(b, hkv, r, 128)
+
+    def call(factor, rope):
+        part, lse = torch.full((b, hq, S, r), float("nan"), device=dev), torch.full((b, hq, S), float("nan"), device=dev)
+        s = torch.full((b, hq, 1, L), float("nan"), device=dev)
+        for values, out in ((A, None), (None, s)):
+            assert _lib.lib().xkv_poison_lds(NAN, None, torch.cuda.current_stream().cuda_stream) == 0
+            ops.recon_stage1(q, A, factor, values, part, lse, out, None, None, b, hq, hkv, L, S, 128 ** -0.5, rope, ops.rope_inv_freq(128, 5e5, q.device), off, None)
+        return part, lse, s
+
+    part, lse, s = call(laid_out(B, how), ops.ROPE_GROUPED)
+    other = call(laid_out(B, "whole"), ops.ROPE_GROUPED if how in LAYOUTS[:3] else True)
+    assert all(torch.equal(x, y) for x, y in zip((part, lse, s), other))
+    out = torch.empty((b, hq, r), device=dev)
+    ops.merge_stage2(part, lse, out, None, None, None, b, hq, hq, L, S)
+    ref = keys_and_scores(q, A, B, off) * 128 ** -0.5
+    # the key and the query rounded to fp16 once each, 2.9e-4 of the scores' size; P is 16 bits wide (2^-9 or 2^-11 of it)
+    assert (s[:, :, 0] - ref).norm() <= 3.5e-4 * ref.norm()
+    ref = torch.softmax(ref, -1) @ A.double()
+    assert (out - ref).norm() <= (4e-3 if dtype == BF else 2e-3) * ref.norm()
+
+
+@pytest.mark.parametrize("how", LAYOUTS)
 @pytest.mark.parametrize("r,G", [(512, 5), (384, 4), (256, 8), (256, 1)])
-@pytest.mark.parametrize("L", [65, 24000])     # rank 256: on both sides of the line from which recon_scores_kernel takes it
+@pytest.mark.parametrize("L", [65, 24000])     # rank 256: on both sides of the line from which recon_scores_kernel takes it (143360 tokens x kv heads for three)
 def test_scores_over_any_layout_of_the_factor(dev, r, G, L, how):
     b, hkv = 2, 3
     q, A = gen((b, hkv * G, 1, 128), dtype=FP, seed=1).to(dev), gen((b, L, r), std=0.2, dtype=FP, seed=2).to(dev)

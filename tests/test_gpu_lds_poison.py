@@ -83,8 +83,10 @@ def test_ring_kernel_scores_and_decode(dev, dtype, poisoned):
 @pytest.mark.parametrize("dtype", [BF, FP])
 def test_reconstruction_kernels(dev, dtype, poisoned):
     tp.test_qab_rope(dev, dtype, 2, 32, 8, 1000, 512, 5e5)     # recon_spec, scores mode, rank 512
-    tp.test_qab_rope(dev, dtype, 2, 8, 2, 300, 384, 5e5)       # recon_scores, two waves a tile
-    tp.test_qab_rope(dev, dtype, 1, 8, 2, 77, 256, 1e7)        # recon_scores at its largest factor
+    tp.test_qab_rope(dev, dtype, 2, 8, 2, 300, 384, 5e5)       # ... at ranks 384 and 256
+    tp.test_qab_rope(dev, dtype, 1, 8, 2, 77, 256, 1e7)
+    tp.test_qab_rope(dev, dtype, 2, 8, 2, 300, 448, 5e5)       # recon_scores, two waves a tile
+    tp.test_qab_rope(dev, dtype, 1, 8, 4, 32769, 256, 1e7)     # recon_scores at its largest factor
     tp.test_qab_rope(dev, dtype, 2, 4, 4, 40, 192, 1e7)        # recon_scores, rank 192
     tp.test_fused_rope(dev, dtype, 2, 32, 8, 3000, 512, 512, 4, True)    # recon_spec fused, shared basis
     tp.test_fused_rope(dev, dtype, 1, 32, 8, 1500, 256, 384, 3, False)   # a value basis of its own
