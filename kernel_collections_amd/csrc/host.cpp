@@ -429,7 +429,7 @@ PyObject* rope_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const int64_t ws_bytes = p_xkv_recon_workspace_bytes(b, hkv, r, kB.stride(0)), ws = c.plan(ws_bytes);
       const float* invp = inv.data_ptr<float>();
       Splits s{0, 0, nullptr, nullptr};
-      // over one basis that kernel is ahead of two passes too (rank 256, 65536 tokens 55.5 / 45.6, 131072 87.7 / 73.0 us)
+      // over one basis that kernel is ahead of two passes too, and as exact (rank 256, 52000 tokens 51.0 / 44.7, 65536 57.5 / 50.4, 131072 90.0 / 79.1, 16 x 32768 283 / 256 us)
       const int S_heads = shared ? heads_splits(rows(kB), b, hkv, hq / hkv, L, r, false, c.cus) : 0;
       if (may_two_pass && !S_heads && (scores_alone(kB, r, hq / hkv) || (ring_rank(r) && hq / hkv <= 8)) && (joined() || hq <= 32) &&
           (ring_rank(rv) || (joined() && shared && (rv == 192 || rv == 128)))) {

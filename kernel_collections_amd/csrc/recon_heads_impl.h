@@ -17,8 +17,8 @@
 // operand reads), into the slot of the tile that the first of the two barriers has done with: they have a period to two to arrive.  The next tile's
 // operands are read behind the barrier that has waited for it (NEXT).
 //
-// 16 x 32768 tokens, 32 heads on 8 kv heads: rank 512 438 us (1.30 PFLOP/s; one head a workgroup 506), 384 348, 256 (four heads) 224; 2755 clocks a period at rank 512
-// where the matrix instructions take 2240, at 1.62 GHz under the power limit (matrix instructions alone: 1.8).  A call starts with 16000 - 20000 clocks in front of the first period:
+// 16 x 32768 tokens, 32 heads on 8 kv heads, several heads / one a workgroup: rank 512 446 / 528 us (438 / 506 at a higher clock: 1.30 PFLOP/s), 384 360 / 416, 256, four heads, 243; 2755 - 2785 clocks a
+// period at rank 512 where the matrix instructions take 2240, at 1.57 - 1.62 GHz under the power limit (matrix instructions alone: 1.8).  A call starts with 16000 - 20000 clocks in front of the first period:
 // 6000 until the first load of a cold device returns, then 256 KB of factors at the rate at which all CUs together read the L2 (33 bytes a clock each).
 #pragma once
 #include "recon_fast_impl.h"
